@@ -116,7 +116,7 @@ def lengths(case):
 def spec_of(name):
     s = get_spec(name)
     if not isinstance(s, HybridSpec):
-        return replace(s, layers=8)
+        return replace(s, layers=4)
 
     def dense(ff):
         if not isinstance(ff, RoutedFF):
