@@ -2,9 +2,9 @@
 // paged cache: where a block of keys lies comes from a KV policy.
 #pragma once
 
-#include "gridllm_common.h"
+#include "gridllm_tiles.h"
 
-#define LOG2E 1.4426950408889634f
+#include <type_traits>
 
 // Where 64 keys (aligned to 64) of a sequence's kv head start, in elements.
 // Caches of contiguous slots: [slots, Hk, Smax, D].
@@ -40,6 +40,9 @@ struct AllKeys {
     DEV_INLINE int start(int b, int seq) const { return b << 6; }
     DEV_INLINE int skip(int k0, int q0) const { return k0; }
     DEV_INLINE bool sees(int q, int key) const { return true; }
+    // whether all queries up to q see the 64 keys from `key` on, as far as
+    // they are not ahead of them
+    DEV_INLINE bool sees_tile(int q, int key) const { return true; }
 };
 
 // The last `size` keys, its own included, and the first `keep`.
@@ -58,12 +61,15 @@ struct WindowKeys {
         const int k = kept(seq);
         return (b < k ? b : window(seq) + b - k) << 6;
     }
-    // first key, from k0 on, of a tile of 32 that rows from q0 on may see
+    // first key, from k0 on, of a tile of 64 that rows from q0 on may see
     DEV_INLINE int skip(int k0, int q0) const {
-        return k0 < keep ? k0 : max(k0, max(0, q0 - size + 1) & ~31);
+        return k0 < keep ? k0 : max(k0, max(0, q0 - size + 1) & ~63);
     }
     DEV_INLINE bool sees(int q, int key) const {
         return q - key < size || key < keep;
+    }
+    DEV_INLINE bool sees_tile(int q, int key) const {
+        return q - key < size || key + 63 < keep;
     }
 };
 
@@ -476,171 +482,283 @@ k_attn_combine(bf16_t* __restrict__ out, const float* __restrict__ ws,
 }
 // ===========================================================================
 // GQA prefill attention — flash-style on MFMA (bf16), reads K/V straight
-// from the slot cache (no permuted host-side views).
+// from the cache.
 //   q:   [T, Hq, D] bf16 (roped)
-//   kc/vc: [slots, Hk, Smax, D] bf16
 //   out: [T, Hq, D] bf16
-// Workgroup = 4 waves; wave w owns 32 q-rows (q0 + w*32) of ONE q-head;
-// K/V walked in 32-row tiles with online softmax (guide App. B prefill).
+// Workgroup = 4 waves; wave w owns 32 q-rows of ONE q-head. K/V are walked in
+// tiles of 64 keys, loaded straight into LDS one tile ahead.
 //
-// Layout trick (guide §5.5 "swapped QK^T"): S^T = mfma(A=K, B=Q) puts a
-// whole q-row's scores in ONE lane (C col = lane&31 = q), so the softmax
-// row-reduce is 15 in-register fmax + one shfl_xor(32) — no LDS. P is then
-// routed to the PV MFMA's B-operand layout through a per-wave LDS scratch
-// (paired b32 writes -> b128 fragment reads, same-wave lgkmcnt wait only),
-// and O^T = mfma(A=V^T, B=P) accumulates with V staged TRANSPOSED in LDS
-// (transpose once per tile, cooperative; A-fragments then read b128-clean).
-// mfma_f32_32x32x16_bf16 maps (guide §3):
+// S^T = mfma(A=K, B=Q) puts a q-row's scores in ONE lane pair, so the softmax
+// row-reduce stays in registers; the weights become the B operand of
+// O^T = mfma(A=V^T, B=P) by one swap of lane halves, and V^T comes from LDS by
+// transposing reads. The softmax's reference moves only when a row's maximum
+// grows by more than 2^MAX_LAG (weights are at most that, sums are f32).
+//
+// 8000 tokens, 24 heads of 128 over 8: 481 us, 817 TFLOP/s of the pairs that
+// are seen (1889 us with one 32-key tile at a time, V transposed by stores into
+// LDS and K read from L2 by every wave). Matrix cores, vector unit (half of it
+// the exponentials) and LDS are each 40 % busy, one wave's phases after each
+// other; two waves share a SIMD. Tiles of 32 keys with three waves a SIMD take
+// 512 us; working on three tiles at once by software, 526 (registers).
+// mfma_f32_32x32x16_bf16:
 //   A[i][k]: lane l holds i = l&31, k = (l>>5)*8 + 0..7
 //   B[k][j]: lane l holds j = l&31, same k chunk
 //   C/D[i][j]: col j = l&31, row i = (reg&3) + 8*(reg>>2) + 4*(l>>5)
-// Constraints: D in {64, 128}; Hq % Hk == 0.
+// Constraints: D in {64, 128, 256}; Hq % Hk == 0.
 // ===========================================================================
+#define MAX_LAG 8.f
 
-// Shared body: one 128-q-row tile of one q-head for one sequence.
-// q0 = first q row of this tile; vt/plds = caller's LDS buffers.
+// LDS elements of a block: two tiles of keys and values.
+template <int D>
+constexpr int prefill_lds() { return 2 * 64 * 2 * D; }
+
+// Scheduling of N LDS reads that feed one MFMA each: AHEAD of them in flight.
+// (Left alone the compiler reads two, waits for both, and so on: the LDS
+// latency eight times in a row.)
+template <int N, int AHEAD>
+DEV_INLINE void reads_ahead() {
+    __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+#pragma unroll
+    for (int i = 0; i < N - AHEAD; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
+}
+
+// Work item of a prefill block: tiles of one head lie on one XCD (blocks go
+// round the 8 XCDs), later tiles, which see more keys, first. False: none.
+DEV_INLINE bool prefill_item(int ntiles, int Hq, int* tile, int* head) {
+    const int total = ntiles * Hq, per = (total + 7) >> 3;
+    const int at = (int)(blockIdx.x >> 3);
+    const int i = (int)(blockIdx.x & 7) * per + at;
+    if (at >= per || i >= total) return false;
+    *head = i / ntiles;
+    *tile = ntiles - 1 - i % ntiles;
+    return true;
+}
+static inline unsigned prefill_grid(long ntiles, long Hq) {
+    return (unsigned)((ntiles * Hq + 7) / 8 * 8);
+}
+
+// One tile of 128 q-rows of one q-head for one sequence. q0 = its first row;
 // row0 = row of q[0] in the epilogue's gate.
 template <int D, class KV, class Keys = AllKeys>
 __device__ __forceinline__ void
 attn_prefill_tile(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
-                  const KV& kv,
-                  int T, int Hq, int G, int slot,
+                  const KV& kv, int T, int Hq, int G, int hq, int slot,
                   int s_total, int causal_off, float scale, int q0,
-                  bf16_t* vt, bf16_t* plds_all, const HeadEpilogue& epi,
-                  int row0, const Keys keys = Keys()) {
+                  bf16_t* lds, const HeadEpilogue& epi, int row0,
+                  const Keys keys = Keys()) {
     constexpr int NS = D / 16;     // 16-wide d slices (QK^T fragments)
     constexpr int NT = D / 32;     // 32-wide d tiles (output / V^T)
-    constexpr int VST = 40;        // padded k-stride of V^T tile (16B-mult)
+    constexpr int VT = NT < 4 ? NT : 4;
+    constexpr int CPR = D / 8;     // 16-byte chunks per row
+    constexpr int LOADS = 64 * CPR / 256;    // of K, and of V, per thread
+    constexpr int TILE = 2 * 64 * D;
 
     const int lane = threadIdx.x & 63;
-    const int wid = threadIdx.x >> 6;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int hi = lane >> 5;
     const int ln = lane & 31;
-    const int hq = blockIdx.y;
     const int hk = hq / G;
     const int qw = q0 + wid * 32;
 
-    // Q fragments: lane holds Q[qw+ln][s*16 + hi*8 + 0..7] (B operand)
+    // Q fragments: lane holds Q[row][s*16 + hi*8 + 0..7] (B operand). Scores
+    // are scaled by |scale|; its sign goes into q.
     bf16x8 qf[NS];
     {
         const bf16_t* qrow =
             q + ((long)min(qw + ln, T - 1) * Hq + hq) * D + hi * 8;
 #pragma unroll
         for (int s = 0; s < NS; ++s) qf[s] = *(const bf16x8*)(qrow + s * 16);
+        if (scale < 0.f)
+#pragma unroll
+            for (int s = 0; s < NS; ++s) qf[s] = -qf[s];
     }
+    const float scale2 = fabsf(scale) * LOG2E;      // log2-domain softmax
 
-    const int q_abs = causal_off + qw + ln;   // this lane's absolute q pos
-    float m = -INFINITY, l = 0.f;
+    // A thread loads 16-byte chunks of rows trow, trow + 256 / CPR, ... K's
+    // chunks are XORed with the row's low bits: 8 rows at one column then lie
+    // in 8 different chunks. V's by 4 times those of 4 rows (D = 64, whose rows
+    // fill half the banks: of every second row), so that the 4 rows x 4 chunks
+    // of a transposing read fill the banks (with K's swizzle they shared a
+    // quarter of them: 10 % of the kernel). The low bits are the same in all of
+    // a thread's rows.
+    const int trow = threadIdx.x / CPR, tcol = threadIdx.x % CPR;
+    const int kcol = (tcol ^ (trow & 7)) * 8;
+    const int vcol = (tcol ^ (CPR > 8 ? (trow & 3) << 2 : (trow & 2) << 1)) * 8;
+    // keys from k0 on, which lie together; rows behind the last key repeat it
+    auto issue = [&](int k0, bf16_t* to) {
+        const long at = kv.off(slot, hk, k0);
+        const bf16_t *ks = kv.k + at, *vs = kv.v + at;
+        const int last = s_total - 1 - k0;
+        bf16_t* tw = to + wid * 512;
+        if (last >= 63) {
+            const u32 ko = trow * D + kcol, vo = trow * D + vcol;
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) {
+                load_lds16(ks + i * 2048 + ko, tw + i * 2048);
+                load_lds16(vs + i * 2048 + vo, tw + TILE / 2 + i * 2048);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) {
+                const u32 r = min(trow + i * (256 / CPR), last) * D;
+                load_lds16(ks + r + kcol, tw + i * 2048);
+                load_lds16(vs + r + vcol, tw + TILE / 2 + i * 2048);
+            }
+        }
+    };
+
+    // Where a lane reads, of a tile's first rows: K by the swizzle of its row
+    // (the low bits of the chunk number; the others are the slice's), V by
+    // transposing reads of rows l % 16 / 4, whose swizzle exchanges 32-wide
+    // tiles.
+    int kat[4], vat[VT];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+        kat[s] = ln * D + ((s * 2 + hi) ^ (ln & 7)) * 8;
+    const int vr = (lane & 15) >> 2;
+#pragma unroll
+    for (int t = 0; t < VT; ++t)
+        vat[t] = (hi * 8 + vr) * D + (t ^ (CPR > 8 ? vr : vr >> 1)) * 32 +
+                 (lane & 16) + (lane & 3) * 4;
+
+    const int q_abs = causal_off + qw + ln;
+    float m = -1e30f, l = 0.f;          // finite: nothing seen weighs 0
     f32x16 acc[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
 
-    // causal upper bound for the workgroup's LAST q-row
-    const int kmax = min(s_total, causal_off + q0 + 128);
-
-    const int qfirst = causal_off + q0;
-    for (int k0 = keys.skip(0, qfirst); k0 < kmax;
-         k0 = keys.skip(k0 + 32, qfirst)) {
-        const long blk = kv.off(slot, hk, k0);   // 32 keys lie together
-        const int klast = s_total - 1 - k0;
-        // ---- stage V^T tile (cooperative transpose) --------------------
-        __syncthreads();               // previous tile's vt readers done
-        {
-            constexpr int CPR = D / 8;            // b128 chunks per V row
-            for (int c = threadIdx.x; c < 32 * CPR; c += 256) {
-                const int kr = c / CPR;
-                const int d8 = (c % CPR) * 8;
-                uint4 v = *(const uint4*)(
-                    kv.v + blk + min(kr, klast) * D + d8);
-                const bf16_t* pv = (const bf16_t*)&v;
+    // One tile in LDS; MASK: some of its keys are not seen by all rows.
+    auto step = [&](const bf16_t* kt, int kc, auto MASK) {
+        constexpr bool mask = decltype(MASK)::value;
+        const bf16_t* vt = kt + TILE / 2;
+        f32x16 sv[2];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) vt[(d8 + j) * VST + kr] = pv[j];
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sv[u][r] = 0.f;
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                sv[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    *(const bf16x8*)(kt + kat[s & 3] + u * 32 * D +
+                                     (s >> 2) * 64), qf[s], sv[u], 0, 0, 0);
+        reads_ahead<2 * NS, 4>();
+        __builtin_amdgcn_sched_barrier(0);
+
+        float mx = -FLT_MAX;
+        u32 seen = 0;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if constexpr (mask) {
+                    const int key = kc + u * 32 + (r & 3) + 8 * (r >> 2) +
+                                    4 * hi;
+                    const bool ok = key < s_total && key <= q_abs &&
+                                    keys.sees(q_abs, key);
+                    seen |= (u32)ok << (u * 16 + r);
+                    mx = fmaxf(mx, ok ? sv[u][r] : -FLT_MAX);
+                } else {
+                    mx = fmaxf(mx, sv[u][r]);
+                }
             }
+        mx = max_across32(mx) * scale2;
+        if (__any(mx > m + MAX_LAG)) {
+            const float mn = mx > m + MAX_LAG ? mx : m;
+            const float alpha = fast_exp2(m - mn);
+            l *= alpha;
+            m = mn;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[t][r] *= alpha;
         }
-        __syncthreads();
-
-        // ---- S^T = K·Q^T (K fragments straight from HBM/L2) ------------
-        f32x16 s_acc;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s_acc[r] = 0.f;
-        {
-            const bf16_t* krow =
-                kv.k + blk + min(ln, klast) * D + hi * 8;
+        for (int u = 0; u < 2; ++u) {
+            float ls = 0.f;
 #pragma unroll
-            for (int s = 0; s < NS; ++s) {
-                const bf16x8 kf = *(const bf16x8*)(krow + s * 16);
-                s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                    kf, qf[s], s_acc, 0, 0, 0);
+            for (int r = 0; r < 16; ++r) {
+                float w = fast_exp2(fmaf(sv[u][r], scale2, -m));
+                if constexpr (mask)
+                    w = seen >> (u * 16 + r) & 1 ? w : 0.f;
+                sv[u][r] = w;
+                ls += w;
             }
-        }
-
-        // ---- mask + online softmax (lane owns one q-row) ---------------
-        float sv[16], tmax = -INFINITY;
-        const float scl2 = scale * 1.4426950408889634f;   // log2 domain
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int kg = k0 + (r & 3) + 8 * (r >> 2) + 4 * hi;
-            const bool ok = (kg < s_total) && (kg <= q_abs) &&
-                            keys.sees(q_abs, kg);
-            sv[r] = ok ? s_acc[r] * scl2 : -INFINITY;
-            tmax = fmaxf(tmax, sv[r]);
-        }
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
-        const float mn = fmaxf(m, tmax);
-        const float alpha = (m == -INFINITY) ? 0.f : exp2f(m - mn);
-        float p[16], psum = 0.f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            p[r] = (sv[r] == -INFINITY) ? 0.f : exp2f(sv[r] - mn);
-            psum += p[r];
-        }
-        psum += __shfl_xor(psum, 32, WAVE);
-        l = l * alpha + psum;
-        m = mn;
-
-        // ---- P -> PV B-fragment layout via per-wave LDS scratch --------
-        // (kpos, q=ln) lands where slice sidx = kpos>>4, lane
-        // lr = ln + 32*((kpos>>3)&1), word i = kpos&7 will read it; regs
-        // pair (r, r+1) = (kpos, kpos+1) -> one packed b32 write.
-        bf16_t* ps = plds_all + wid * (2 * 64 * 8);
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-            const int kpos = (r & 3) + 8 * (r >> 2) + 4 * hi;
-            const int sidx = kpos >> 4;
-            const int lr = ln + 32 * ((kpos >> 3) & 1);
-            u32 w = (u32)f2bf(p[r]) | ((u32)f2bf(p[r + 1]) << 16);
-            *(u32*)(ps + (sidx * 64 + lr) * 8 + (kpos & 7)) = w;
-        }
-        // rescale output accumulators while the P writes land
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[t][r] *= alpha;
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-
-        // ---- O^T += V^T · P --------------------------------------------
-        bf16x8 pf[2];
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-            pf[s] = *(const bf16x8*)(ps + (s * 64 + lane) * 8);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const bf16_t* vrow = vt + (t * 32 + ln) * VST + hi * 8;
+            l += ls;
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                const bf16x8 vf = *(const bf16x8*)(vrow + s * 16);
-                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                    vf, pf[s], acc[t], 0, 0, 0);
+                // lane half hi holds keys 8 g + 4 hi + 0..3; it needs
+                // 8 hi + 0..7
+                u32 w[4];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const int o = 8 * s + 2 * i;
+                    const u32x2 x = __builtin_amdgcn_permlane32_swap(
+                        pack2(sv[u][o], sv[u][o + 1]),
+                        pack2(sv[u][o + 4], sv[u][o + 5]), false, false);
+                    w[i] = x[0];
+                    w[2 + i] = x[1];
+                }
+                bf16x8 pf;
+                __builtin_memcpy(&pf, w, 16);
+                // O^T += V^T P
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    bf16x8 v;
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const bf16x4 x = read_transposed(
+                            vt + vat[t % VT] + (u * 32 + s * 16 + j * 4) * D +
+                            t / VT * VT * 32);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) v[j * 4 + i] = x[i];
+                    }
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        v, pf, acc[t], 0, 0, 0);
+                }
             }
         }
+    };
+
+    const int kmax = min(s_total, causal_off + q0 + 128);
+    const int qfirst = causal_off + q0;
+    int k0 = keys.skip(0, qfirst), buf = 0;
+    if (k0 < kmax) issue(k0, lds);
+    // all rows of the block see the whole tile
+    auto whole = [&] {
+        return k0 + 63 <= qfirst && k0 + 63 < s_total &&
+               keys.sees_tile(qfirst + 127, k0);
+    };
+    auto walk = [&](auto MASK) {
+        const int kc = k0;
+        const bf16_t* kt = lds + buf * TILE;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        lds_barrier();              // tile is there, the other one is free
+        buf ^= 1;
+        k0 = keys.skip(k0 + 64, qfirst);
+        if (k0 < kmax) issue(k0, lds + buf * TILE);
+        if (!decltype(MASK)::value || kc <= causal_off + qw + 31)
+            step(kt, kc, MASK);     // else ahead of all of the wave's rows
+    };
+    // two loops, so that sums stay in their registers
+    while (k0 < kmax) {
+        while (k0 < kmax && whole()) walk(std::false_type());
+        while (k0 < kmax && !whole()) walk(std::true_type());
     }
 
     // ---- normalize + store: lane holds O^T[*][q=ln] — one q-row --------
+    l += __shfl_xor(l, 32, WAVE);
     if (qw + ln < T) {
-        const float inv = epi.factor(row0 + qw + ln, hq, m, l);
-        bf16_t* orow = out + epi.at(qw + ln, hq, Hq, D);
+        const int r = qw + ln;
+        const float inv = epi.factor(row0 + r, hq, m, l);
+        bf16_t* orow = out + epi.at(r, hq, Hq, D);
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
 #pragma unroll
@@ -651,8 +769,8 @@ attn_prefill_tile(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
                 for (int i = 0; i < 4; ++i) f[i] = acc[t][4 * g + i] * inv;
                 if (epi.gate_el) {
                     float z[4];
-                    ld4(epi.gate + (long)(row0 + qw + ln) * epi.gate_ld +
-                        hq * D + d, z);
+                    ld4(epi.gate + (long)(row0 + r) * epi.gate_ld + hq * D + d,
+                        z);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) f[i] /= 1.f + __expf(-z[i]);
                 }

@@ -716,16 +716,18 @@ k_qknorm_kv(T* __restrict__ qkv, T* __restrict__ q_out,
 template <int D, class Keys>
 __global__ void __launch_bounds__(256, D > 128 ? 1 : 2)
 k_paged_prefill(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
-                const PagedKV<D> kv, const int* __restrict__ meta, int Hq,
-                int G, float scale, const HeadEpilogue epi, const Keys keys) {
-    __shared__ __attribute__((aligned(16))) bf16_t vt[D * 40];
-    __shared__ __attribute__((aligned(16))) bf16_t plds[4][2 * 64 * 8];
-    const int* m = meta + blockIdx.x * 8;
+                const PagedKV<D> kv, const int* __restrict__ meta, int ntiles,
+                int Hq, int G, float scale, const HeadEpilogue epi,
+                const Keys keys) {
+    __shared__ __attribute__((aligned(16))) bf16_t lds[prefill_lds<D>()];
+    int tile, hq;
+    if (!prefill_item(ntiles, Hq, &tile, &hq)) return;
+    const int* m = meta + tile * 8;
     const int q_off = m[0], len = m[1], start = m[4];
     attn_prefill_tile<D>(out + epi.at(q_off, 0, Hq, D),
-                         q + (long)q_off * Hq * D, kv, len, Hq, G, m[2],
-                         start + len, start, scale, m[3], vt, &plds[0][0],
-                         epi, q_off, keys);
+                            q + (long)q_off * Hq * D, kv, len, Hq, G, hq, m[2],
+                            start + len, start, scale, m[3], lds, epi, q_off,
+                            keys);
 }
 
 // Exact mode: one block per (row, query head), f32 cache, any position.
@@ -2505,11 +2507,11 @@ int gh_paged_prefill(void* stream, void* out, const void* q, const void* kc,
     const HeadEpilogue epi{(const float*)sink, (const bf16_t*)gate, gate_ld,
                            gate && gate_el, oscale, out_ld};
     hipStream_t st_ = (hipStream_t)stream;
-#define GO(DD, K, ...) k_paged_prefill<DD, K><<<dim3(ntiles, Hq), 256, 0, \
-        st_>>>((bf16_t*)out, (const bf16_t*)q, \
-        PagedKV<DD>{(const bf16_t*)kc, (const bf16_t*)vc, (const int*)table, \
-                    Hk, per_slot}, (const int*)meta, Hq, Hq / Hk, scale, epi, \
-        K{__VA_ARGS__})
+#define GO(DD, K, ...) k_paged_prefill<DD, K> \
+        <<<prefill_grid(ntiles, Hq), 256, 0, st_>>>((bf16_t*)out, \
+        (const bf16_t*)q, PagedKV<DD>{(const bf16_t*)kc, (const bf16_t*)vc, \
+        (const int*)table, Hk, per_slot}, (const int*)meta, ntiles, Hq, \
+        Hq / Hk, scale, epi, K{__VA_ARGS__})
 #define PICK(DD) do { if (window) GO(DD, WindowKeys, window, keep); \
         else GO(DD, AllKeys); } while (0)
     if (D == 64) PICK(64);

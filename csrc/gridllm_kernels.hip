@@ -615,18 +615,18 @@ k_attn_prefill(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
                const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
                int T, int Hq, int G, int Hk, int Smax, int slot,
                int s_total, int causal_off, float scale) {
-    constexpr int VST = 40;
-    __shared__ __attribute__((aligned(16))) bf16_t vt[D * VST];
-    __shared__ __attribute__((aligned(16))) bf16_t plds[4][2 * 64 * 8];
+    __shared__ __attribute__((aligned(16))) bf16_t lds[prefill_lds<D>()];
+    int tile, hq;
+    if (!prefill_item((T + 127) / 128, Hq, &tile, &hq)) return;
     const SlotKV<D> kv{kc, vc, Hk, Smax};
     const HeadEpilogue epi{nullptr, nullptr, 0};
-    attn_prefill_tile<D>(out, q, kv, T, Hq, G, slot, s_total, causal_off,
-                         scale, blockIdx.x * 128, vt, &plds[0][0], epi, 0);
+    attn_prefill_tile<D>(out, q, kv, T, Hq, G, hq, slot, s_total,
+                            causal_off, scale, tile * 128, lds, epi, 0);
 }
 
 // ===========================================================================
 // Varlen BATCHED prefill: one launch covers MANY fresh sequences.
-//   meta[tile] = {q_off, len, slot, q0}: tile `blockIdx.x` works on rows
+//   meta[tile] = {q_off, len, slot, q0}: a tile is rows
 //   [q0, q0+128) of the sequence packed at q_off in q/out, against KV slot
 //   `slot` with s_total = len, causal_off = 0.
 // Motivation (round-2 serving profile, lt_worker_batcher.prof): admission
@@ -639,17 +639,17 @@ __global__ void __launch_bounds__(256, 2)
 k_attn_prefill_batch(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
                      const bf16_t* __restrict__ kc,
                      const bf16_t* __restrict__ vc,
-                     const int4* __restrict__ meta, int Hq, int G, int Hk,
-                     int Smax, float scale) {
-    constexpr int VST = 40;
-    __shared__ __attribute__((aligned(16))) bf16_t vt[D * VST];
-    __shared__ __attribute__((aligned(16))) bf16_t plds[4][2 * 64 * 8];
-    const int4 m = meta[blockIdx.x];
+                     const int4* __restrict__ meta, int ntiles, int Hq, int G,
+                     int Hk, int Smax, float scale) {
+    __shared__ __attribute__((aligned(16))) bf16_t lds[prefill_lds<D>()];
+    int tile, hq;
+    if (!prefill_item(ntiles, Hq, &tile, &hq)) return;
+    const int4 m = meta[tile];
     const SlotKV<D> kv{kc, vc, Hk, Smax};
     const HeadEpilogue epi{nullptr, nullptr, 0};
     attn_prefill_tile<D>(out + (long)m.x * Hq * D, q + (long)m.x * Hq * D,
-                         kv, m.y, Hq, G, m.z, m.y, /*causal_off=*/0, scale,
-                         m.w, vt, &plds[0][0], epi, 0);
+                            kv, m.y, Hq, G, hq, m.z, m.y, /*causal_off=*/0,
+                            scale, m.w, lds, epi, 0);
 }
 
 template <int MT>
@@ -1090,7 +1090,8 @@ int gl_attn_prefill(void* stream, void* out, const void* q, const void* kc,
     hipStream_t st = (hipStream_t)stream;
     if (Hq % Hk) return -110;
     const int G = Hq / Hk;
-    dim3 grid((unsigned)((T + 127) / 128), (unsigned)Hq), blk(256);
+    if (T < 1 || s_total < 1) return -100;
+    dim3 grid(prefill_grid((T + 127) / 128, Hq)), blk(256);
     if (D == 128)
         k_attn_prefill<128><<<grid, blk, 0, st>>>(
             (bf16_t*)out, (const bf16_t*)q, (const bf16_t*)kc,
@@ -1114,15 +1115,18 @@ int gl_attn_prefill_batch(void* stream, void* out, const void* q,
     hipStream_t st = (hipStream_t)stream;
     if (Hq % Hk) return -110;
     const int G = Hq / Hk;
-    dim3 grid((unsigned)ntiles, (unsigned)Hq), blk(256);
+    if (ntiles < 1) return -100;
+    dim3 grid(prefill_grid(ntiles, Hq)), blk(256);
     if (D == 128)
         k_attn_prefill_batch<128><<<grid, blk, 0, st>>>(
             (bf16_t*)out, (const bf16_t*)q, (const bf16_t*)kc,
-            (const bf16_t*)vc, (const int4*)meta, Hq, G, Hk, Smax, scale);
+            (const bf16_t*)vc, (const int4*)meta, ntiles, Hq, G, Hk, Smax,
+            scale);
     else if (D == 64)
         k_attn_prefill_batch<64><<<grid, blk, 0, st>>>(
             (bf16_t*)out, (const bf16_t*)q, (const bf16_t*)kc,
-            (const bf16_t*)vc, (const int4*)meta, Hq, G, Hk, Smax, scale);
+            (const bf16_t*)vc, (const int4*)meta, ntiles, Hq, G, Hk, Smax,
+            scale);
     else
         return -111;
     LAUNCH_CHECK();

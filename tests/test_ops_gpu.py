@@ -227,6 +227,35 @@ def test_attn_prefill_mfma_gpu(dev, t, hq, hk, d, cau):
     assert _mx(out.cpu(), ref) < 0.03
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("t,cau,sign", [
+    (1, 0, 1), (33, 0, 1), (64, 63, 1), (65, 64, 1), (128, 1, -1),
+    (129, 191, 1), (300, 62, 1),
+])
+def test_attn_prefill_tile_edges_gpu(dev, t, cau, sign, d):
+    """Rows and keys at the edges of tiles of 128 and 64, scores that grow by
+    more than the softmax reference's lag from tile to tile, and NaN behind the
+    last key, which nothing may read. Weights and the output are rounded to
+    bf16 (2^-8 each), values are of the order of 1: 0.02 in the worst
+    element."""
+    torch.manual_seed(t + cau)
+    from gridllm_amd.ops import hip_ops
+    n, hq, hk = cau + t, 6, 2
+    q = torch.randn(t, hq, d, device=dev).to(torch.bfloat16)
+    kc = torch.randn(2, hk, 640, d, device=dev)
+    kc = (kc * torch.linspace(0.1, 4, 640, device=dev).view(1, 1, -1, 1)).to(
+        torch.bfloat16)
+    vc = torch.randn(2, hk, 640, d, device=dev).to(torch.bfloat16)
+    kc[:, :, n:], vc[:, :, n:] = float("nan"), float("nan")
+    scale = sign * d ** -0.5
+    out = hip_ops.attn_prefill_cache(q, kc, vc, 1, n, cau, scale)
+    kk = kc[1, :, :n].permute(1, 0, 2).unsqueeze(0).cpu().float()
+    vv = vc[1, :, :n].permute(1, 0, 2).unsqueeze(0).cpu().float()
+    ref = R.attn_prefill(q.unsqueeze(0).cpu().float(), kk, vv, scale,
+                         causal_offset=cau)[0]
+    assert _mx(out.cpu(), ref) < 0.02
+
+
 @pytest.mark.parametrize("m,n,k", [
     (256, 5120, 3072), (256, 3072, 8192), (128, 3072, 3072),
     (200, 16384, 3072),       # ragged M
