@@ -112,24 +112,63 @@ struct HeadEpilogue {
 // ===========================================================================
 // GQA decode attention (flash-decode style).
 //   q:   [B, Hq, D] bf16 (one new token per sequence)
-//   kc/vc: [B, Hk, Smax, D] bf16
+//   kc/vc: bf16 caches
 //   seqlen: [B] int32 (number of valid keys, including the current token)
 //   out: [B, Hq, D] bf16
-//   ws (nsplit>1): f32 [B, Hk, G, nsplit, D+2]  (unnormalized acc, m, l)
+//   ws (nsplit>1): f32 [B, Hq, nsplit, D+2]  (unnormalized acc, m, l)
 //
-// Block = 256 thr = 4 waves, one block per (b, hk, split). Each wave owns
-// key-blocks of 64 (one key per lane), keeps per-(g) online-softmax state,
-// then the 4 waves combine in LDS. G = Hq/Hk (q-heads per kv-head) so each
-// K/V row is read once and reused for all G query heads.
-// Constraints: D in {64, 128}; G <= 8; D % 8 == 0.
+// Block = 4 waves, one block per (b, hk, split). Waves take turns at steps of
+// KS = 4096 / D keys, whose K and V (8 KB each) they load into registers one
+// step ahead: K as MFMA operands (scores of all G = Hq/Hk query heads at once,
+// S = mfma(A=Q, B=K)), V row-wise, 16 bytes a lane, for f32 sums in the vector
+// unit; weights stay f32 and pass through LDS. The 4 waves combine in LDS.
+// Bound by HBM and, for few keys, by the chain load - scores - weights - sums.
+// 24 heads of 128 over 8, before (a key row per lane, f32 scores, waves waiting
+// for their own loads) and now: 24 rows of up to 6000 keys 193 -> 70 us
+// (5.1 TB/s), 256 of up to 384 99 -> 46 us (5.2 TB/s), one of 900 17 -> 9 us.
+// Loads past the caches are 5 % faster than plain ones where the keys of all
+// rows exceed them.
+// mfma_f32_16x16x32_bf16:
+//   A[i][k]: lane l holds i = l&15, k = (l>>4)*8 + 0..7
+//   B[k][j]: lane l holds j = l&15, same k chunk
+//   D[i][j]: lane l holds j = l&15, i = (l>>4)*4 + reg
+// Constraints: D in {64, 128, 256}; G <= 8.
 // ===========================================================================
 
 #define MAXG 8
+#define MAX_SPLIT 64
+
+// The softmax's reference moves only when a maximum grows by more than
+// 2^MAX_LAG: weights are at most that, their sums are f32.
+#define MAX_LAG 8.f
+
+template <int N>                       // x of the lane N further on in its 16
+DEV_INLINE float rotate16(float x) {
+    return __uint_as_float(__builtin_amdgcn_mov_dpp(
+        (int)__float_as_uint(x), 0x120 + N, 0xf, 0xf, true));
+}
+DEV_INLINE float max_of16(float x) {
+    x = fmaxf(x, rotate16<8>(x));
+    x = fmaxf(x, rotate16<4>(x));
+    x = fmaxf(x, rotate16<2>(x));
+    return fmaxf(x, rotate16<1>(x));
+}
+DEV_INLINE float sum_of16(float x) {
+    x += rotate16<8>(x);
+    x += rotate16<4>(x);
+    x += rotate16<2>(x);
+    return x + rotate16<1>(x);
+}
+
+// Steps of a row and of one of its splits: at least one for each wave.
+DEV_INLINE int split_steps(int steps, int nsplit) {
+    return max((steps + nsplit - 1) / nsplit, 4);
+}
 
 // A kv head with more than MAXG query heads is served by `ngrp` blocks of G
 // query heads each. Sequence lengths are given as seqlen + seq_add.
 template <int D, int G, class KV, class Keys>
-__global__ void __launch_bounds__(256, 3)
+__global__ void __launch_bounds__(256, 2)
 k_attn_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
               const KV kv,
               const int* __restrict__ seqlen, int seq_add,
@@ -137,6 +176,11 @@ k_attn_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
               float* __restrict__ ws,
               int ngrp, int nsplit, float scale, const HeadEpilogue epi,
               const Keys keys) {
+    constexpr int KS = 4096 / D;           // keys of a step
+    constexpr int SPB = 64 / KS;           // steps of a block of 64 keys
+    constexpr int KT = KS / 16, ND = D / 32;
+    constexpr int LV = D / 8;              // lanes of a V row
+    constexpr int R = G < 4 ? G : 4;       // heads of a lane
     const int Hg = kv.Hk * ngrp;
     const int split = blockIdx.x % nsplit;
     const int hg = (blockIdx.x / nsplit) % Hg;
@@ -144,161 +188,207 @@ k_attn_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
     const int b = blockIdx.x / (nsplit * Hg);
     const int bc = slot_map ? slot_map[b] : b;   // cache slot for this row
     const int lane = threadIdx.x & 63;
-    const int wid = threadIdx.x >> 6;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int Hq = Hg * G;
 
-    __shared__ float q_lds[G * D];
-    __shared__ float red[4][G * (D > 64 ? D : 64)];
-    __shared__ float wml[4][G][2];            // per-wave m, l
+    __shared__ __attribute__((aligned(16))) float p_lds[4][G][KS];
+    __shared__ float red[4][G * D];
+    __shared__ float wml[4][G][2];         // per-wave m, l
 
     const int seq = seqlen[b] + seq_add;
-    // split range, 64-aligned chunks
-    const int chunks = keys.blocks(seq);
-    const int per = (chunks + nsplit - 1) / nsplit;
-    const int c0 = split * per;
-    const int c1 = min(chunks, c0 + per);
-
-    // stage q (scaled) into LDS as f32
-    const int Hq = Hg * G;
-    for (int i = threadIdx.x; i < G * D; i += 256) {
-        int g = i / D, d = i % D;
-        // log2-domain softmax: fold log2(e) into the q prescale so every
-        // exp becomes a native v_exp_f32 exp2 (identical values:
-        // exp2((x-m)*log2e) == exp(x-m))
-        q_lds[i] = bf2f(q[((long)b * Hq + hg * (long)G + g) * D + d])
-                   * (scale * 1.4426950408889634f);
+    const int blocks = keys.blocks(seq);
+    const int steps = blocks <= 0 ? 0 : (blocks - 1) * SPB +
+        (seq - keys.start(blocks - 1, seq) + KS - 1) / KS;
+    const int per = split_steps(steps, nsplit);
+    const int end = min(steps, split * per + per);
+    int cur = split * per + wid;
+    if (split && split * per >= steps) {   // nothing left for this split
+        if (threadIdx.x < G) {
+            float* wsp = ws + (((long)b * Hq + hg * G + threadIdx.x) * nsplit +
+                               split) * (D + 2);
+            wsp[D] = -INFINITY;
+            wsp[D + 1] = 0.f;
+        }
+        return;
     }
-    __syncthreads();
 
-    // per-wave online softmax state.
-    // P.V layout: the wave reads RPI = 64/(D/8) V-rows per b128-load
-    // iteration — lane covers row-group rg = lane/DV and d = (lane%DV)*8
-    // + 0..7 — so a 64-key block takes 64/RPI wide-load iterations instead
-    // of 64 row-at-a-time u32 iterations (which measured as a serial
-    // L2-latency chain, 3.2 TB/s). Each lane holds PARTIAL sums over its
-    // row group; one shfl_xor ladder at the end totals them.
-    float m[G], l[G];
-    constexpr int DV = D / 8;          // lanes per V row
-    constexpr int RPI = 64 / DV;       // V rows per iteration
-    float facc[G][8];
+    const int fr = lane & 15, kg = (lane >> 4) * 8;
+    bf16x8 qf[ND];                         // head fr (or the last one)
+    {
+        const bf16_t* qr = q + ((long)b * Hq + hg * G + min(fr, G - 1)) * D +
+                           kg;
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        m[g] = -INFINITY;
-        l[g] = 0.f;
+        for (int s = 0; s < ND; ++s) qf[s] = *(const bf16x8*)(qr + s * 32);
+    }
+    const float scale2 = scale * LOG2E;    // log2-domain softmax
+
+    const int rg = lane / LV, d8 = (lane % LV) * 8;
+    bf16x8 kf[KT][ND];
+    uint4 vf[8];
+    auto first_key = [&](int st) {
+        return keys.start(st / SPB, seq) + st % SPB * KS;
+    };
+    // rows behind the last key repeat it
+    auto start_of = [&](int st) {
+        const int k0 = first_key(st);
+        return kv.off(bc, hk, k0 & ~63) + (k0 & 63) * D;
+    };
+    auto load_k = [&](int st, long at) {
+        const int last = seq - 1 - first_key(st);
+        const bf16_t* p = kv.k + at + kg;
+#pragma unroll
+        for (int t = 0; t < KT; ++t) {
+            const bf16_t* r = p + min(t * 16 + fr, last) * D;
+#pragma unroll
+            for (int s = 0; s < ND; ++s)
+                kf[t][s] = __builtin_nontemporal_load((const bf16x8*)(r + s * 32));
+        }
+    };
+    typedef __attribute__((ext_vector_type(4))) u32 u32x4;
+    auto load_v = [&](int st, long at) {
+        const int last = seq - 1 - first_key(st);
+        const bf16_t* p = kv.v + at + d8;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const u32x4 x = __builtin_nontemporal_load(
+                (const u32x4*)(p + min(rg * 8 + j, last) * D));
+            vf[j] = make_uint4(x[0], x[1], x[2], x[3]);
+        }
+    };
+
+    float m[R], l[R];                      // of heads (lane >> 4) * 4 + r
+    float facc[G][8];                      // sums over this lane's V rows
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        m[r] = -1e30f;                     // finite: nothing seen weighs 0
+        l[r] = 0.f;
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g)
 #pragma unroll
         for (int i = 0; i < 8; ++i) facc[g][i] = 0.f;
-    }
-    const int rg = lane / DV;
-    const int d8 = (lane % DV) * 8;
 
-    int cb = c0 + wid;
-    long next = cb < c1 ? kv.off(bc, hk, keys.start(cb, seq)) : 0;
-    for (; cb < c1; cb += 4) {
-        const int kb = keys.start(cb, seq);
-        const bf16_t* kblk = kv.k + next;
-        const bf16_t* vblk = kv.v + next;
-        if (cb + 4 < c1) next = kv.off(bc, hk, keys.start(cb + 4, seq));
-        const int j = kb + lane;
-        const bool valid = j < seq && keys.sees(seq - 1, j);
-        float s[G];
+    auto step = [&](int st, auto MORE) {
+        long next = 0;
+        if constexpr (decltype(MORE)::value) next = start_of(st + 4);
+        f32x4 s[KT];
 #pragma unroll
-        for (int g = 0; g < G; ++g) s[g] = 0.f;
-        if (valid) {
-            const bf16_t* krow = kblk + lane * D;
+        for (int t = 0; t < KT; ++t) {
+            s[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int dd = 0; dd < D; dd += 8) {
-                uint4 kv = *(const uint4*)(krow + dd);
-                float kf[8];
-                unpack8(kv, kf);
-#pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    float a = 0.f;
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) a += kf[i] * q_lds[g * D + dd + i];
-                    s[g] += a;
-                }
-            }
+            for (int c = 0; c < ND; ++c)
+                s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    qf[c], kf[t][c], s[t], 0, 0, 0);
         }
-        // online softmax update per g; store p into LDS (reuse red[] rows)
+        if constexpr (decltype(MORE)::value) load_k(st + 4, next);
+        const int k0 = first_key(st);
+        float mx[R];
+        bool move = false;
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            float sv = valid ? s[g] : -INFINITY;
-            float bmax = wave_reduce_max(sv);
-            float mn = fmaxf(m[g], bmax);
-            // guard: all-invalid block -> bmax=-inf, mn may stay -inf
-            float alpha = (m[g] == -INFINITY) ? 0.f : exp2f(m[g] - mn);
-            float p = (sv == -INFINITY) ? 0.f : exp2f(sv - mn);
-            l[g] = l[g] * alpha + wave_reduce_sum(p);
-            if (mn != m[g]) {          // defer-rescale: skip when max held
+        for (int r = 0; r < R; ++r) {
+            mx[r] = -FLT_MAX;
 #pragma unroll
-                for (int i = 0; i < 8; ++i) facc[g][i] *= alpha;
+            for (int t = 0; t < KT; ++t) {
+                const int key = k0 + t * 16 + fr;
+                s[t][r] = key < seq && keys.sees(seq - 1, key)
+                    ? s[t][r] * scale2 : -INFINITY;
+                mx[r] = fmaxf(mx[r], s[t][r]);
             }
-            m[g] = mn;
-            red[wid][g * 64 + lane] = p;      // per-wave scratch: p for 64 keys
+            mx[r] = max_of16(mx[r]);
+            move |= mx[r] > m[r] + MAX_LAG;
         }
-        // wave-local LDS visibility (no cross-wave traffic here)
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        // accumulate P·V: RPI rows per iteration, one b128 load per lane
-        const int jmax = min(64, seq - kb);
-        for (int jb = 0; jb < jmax; jb += RPI) {
-            const int j2 = jb + rg;
-            const uint4 vv = *(const uint4*)(
-                vblk + min(j2, jmax - 1) * D + d8);
-            float vf[8];
-            unpack8(vv, vf);
+        if (__any(move)) {
+            float alpha[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const float mn = mx[r] > m[r] + MAX_LAG ? mx[r] : m[r];
+                alpha[r] = exp2f(m[r] - mn);
+                l[r] *= alpha[r];
+                m[r] = mn;
+            }
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                const float p = (j2 < jmax) ? red[wid][g * 64 + j2] : 0.f;
+                const float a = __uint_as_float(__builtin_amdgcn_readlane(
+                    __float_as_uint(alpha[g & 3]), g >> 2 << 4));
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    facc[g][i] = fmaf(p, vf[i], facc[g][i]);
+                for (int i = 0; i < 8; ++i) facc[g][i] *= a;
             }
         }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int head = (lane >> 4) * 4 + r;
+#pragma unroll
+            for (int t = 0; t < KT; ++t) {
+                const float p = fast_exp2(s[t][r] - m[r]);
+                l[r] += p;
+                if (head < G) p_lds[wid][head][t * 16 + fr] = p;
+            }
+        }
+        // this wave's weights alone
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        float p[G][8];
+#pragma unroll
+        for (int g = 0; g < G; ++g) ld8(&p_lds[wid][g][rg * 8], p[g]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            float v[8];
+            unpack8(vf[j], v);
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    facc[g][i] = fmaf(p[g][j], v[i], facc[g][i]);
+        }
+        if constexpr (decltype(MORE)::value) load_v(st + 4, next);
+        asm volatile("" ::: "memory");     // weights are read
+    };
+    if (cur < end) {
+        const long at = start_of(cur);
+        load_k(cur, at);
+        load_v(cur, at);
+        for (; cur + 4 < end; cur += 4) step(cur, std::true_type());
+        step(cur, std::false_type());
     }
 
-    // total each lane's row-group partials: after the ladder every lane
-    // holds the full sum for its d = d8 + 0..7 slice
+    // total the lanes' V rows and keys, then the waves
 #pragma unroll
     for (int g = 0; g < G; ++g)
 #pragma unroll
         for (int i = 0; i < 8; ++i)
 #pragma unroll
-            for (int off = 32; off >= DV; off >>= 1)
+            for (int off = 32; off >= LV; off >>= 1)
                 facc[g][i] += __shfl_xor(facc[g][i], off, WAVE);
-
-    // cross-wave combine in LDS
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        wml[wid][g][0] = m[g];
-        wml[wid][g][1] = l[g];
+    for (int r = 0; r < R; ++r) {
+        const int head = (lane >> 4) * 4 + r;
+        l[r] = sum_of16(l[r]);
+        if (fr == 0 && head < G) {
+            wml[wid][head][0] = m[r];
+            wml[wid][head][1] = l[r];
+        }
     }
-    __syncthreads();
+    if (lane < LV)
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        float M = fmaxf(fmaxf(wml[0][g][0], wml[1][g][0]),
-                        fmaxf(wml[2][g][0], wml[3][g][0]));
-        float f = (m[g] == -INFINITY) ? 0.f : exp2f(m[g] - M);
-        if (lane < DV)
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-                red[wid][g * D + d8 + i] = facc[g][i] * f;
-        if (lane == g % 64) wml[wid][g][1] = l[g] * f;  // scaled l (one lane writes)
-    }
+        for (int g = 0; g < G; ++g) st8(&red[wid][g * D + d8], facc[g]);
     __syncthreads();
-
-    // final reduction over 4 waves + output
     for (int i = threadIdx.x; i < G * D; i += 256) {
         const int g = i / D, d = i % D;
-        float a = red[0][g * D + d] + red[1][g * D + d] +
-                  red[2][g * D + d] + red[3][g * D + d];
-        float L = wml[0][g][1] + wml[1][g][1] + wml[2][g][1] + wml[3][g][1];
-        float M = fmaxf(fmaxf(wml[0][g][0], wml[1][g][0]),
-                        fmaxf(wml[2][g][0], wml[3][g][0]));
+        float M = wml[0][g][0], a = 0.f, L = 0.f;
+#pragma unroll
+        for (int w = 1; w < 4; ++w) M = fmaxf(M, wml[w][g][0]);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const float f = exp2f(wml[w][g][0] - M);
+            a += red[w][i] * f;
+            L += wml[w][g][1] * f;
+        }
         if (nsplit == 1) {
             out[epi.at(b, hg * G + g, Hq, D) + d] =
                 f2bf(a * epi.factor(b, hg * G + g, M, L) *
                      epi.element(b, (hg * G + g) * D + d));
         } else {
-            float* wsp = ws + (((long)b * Hq + hg * G + g) * nsplit + split) * (D + 2);
+            float* wsp = ws + (((long)b * Hq + hg * G + g) * nsplit + split) *
+                              (D + 2);
             wsp[d] = a;
             if (d == 0) {
                 wsp[D] = M;
@@ -308,178 +398,43 @@ k_attn_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
     }
 }
 
-// ===========================================================================
-// GQA decode attention, ONE WAVE per (b, hk[, split]) — the large-batch
-// variant. At serving batches B*Hk >= ~2048 the chip holds every block
-// resident (16 waves/CU), so per-wave independence beats the 4-wave
-// cooperative block: no q-staging barrier, no cross-wave LDS combine, no
-// idle waves when seq/64 < 4. Same math as k_attn_decode; V phase reads
-// RPI rows per b128 iteration with an end shfl ladder.
-// ===========================================================================
-
-template <int D, int G, class KV, class Keys>
-__global__ void __launch_bounds__(64, 3)
-k_attn_decode1(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
-               const KV kv,
-               const int* __restrict__ seqlen, int seq_add,
-               const int* __restrict__ slot_map,
-               float* __restrict__ ws,
-               int ngrp, int nsplit, float scale, const HeadEpilogue epi,
-               const Keys keys) {
-    const int Hg = kv.Hk * ngrp;
-    const int split = blockIdx.x % nsplit;
-    const int hg = (blockIdx.x / nsplit) % Hg;
-    const int hk = hg / ngrp;
-    const int b = blockIdx.x / (nsplit * Hg);
-    const int bc = slot_map ? slot_map[b] : b;
-    const int lane = threadIdx.x;
-
-    __shared__ float q_lds[G * D];
-    __shared__ float p_lds[G * 64];
-
-    const int seq = seqlen[b] + seq_add;
-    const int chunks = keys.blocks(seq);
-    const int per = (chunks + nsplit - 1) / nsplit;
-    const int c0 = split * per;
-    const int c1 = min(chunks, c0 + per);
-
-    const int Hq = Hg * G;
-    for (int i = lane; i < G * D; i += 64)
-        q_lds[i] = bf2f(q[((long)b * Hq + hg * (long)G + i / D) * D
-                          + i % D]) * (scale * 1.4426950408889634f);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-
-    float m[G], l[G];
-    constexpr int DV = D / 8;
-    constexpr int RPI = 64 / DV;
-    float facc[G][8];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        m[g] = -INFINITY;
-        l[g] = 0.f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) facc[g][i] = 0.f;
-    }
-    const int rg = lane / DV;
-    const int d8 = (lane % DV) * 8;
-
-    long next = c0 < c1 ? kv.off(bc, hk, keys.start(c0, seq)) : 0;
-    for (int cb = c0; cb < c1; ++cb) {
-        const int kb = keys.start(cb, seq);
-        const bf16_t* kblk = kv.k + next;
-        const bf16_t* vblk = kv.v + next;
-        if (cb + 1 < c1) next = kv.off(bc, hk, keys.start(cb + 1, seq));
-        const int j = kb + lane;
-        const bool valid = j < seq && keys.sees(seq - 1, j);
-        float s[G];
-#pragma unroll
-        for (int g = 0; g < G; ++g) s[g] = 0.f;
-        if (valid) {
-            const bf16_t* krow = kblk + lane * D;
-#pragma unroll
-            for (int dd = 0; dd < D; dd += 8) {
-                uint4 kv = *(const uint4*)(krow + dd);
-                float kf[8];
-                unpack8(kv, kf);
-#pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    float a = 0.f;
-#pragma unroll
-                    for (int i = 0; i < 8; ++i)
-                        a += kf[i] * q_lds[g * D + dd + i];
-                    s[g] += a;
-                }
-            }
-        }
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            float sv = valid ? s[g] : -INFINITY;
-            float bmax = wave_reduce_max(sv);
-            float mn = fmaxf(m[g], bmax);
-            float alpha = (m[g] == -INFINITY) ? 0.f : exp2f(m[g] - mn);
-            float p = (sv == -INFINITY) ? 0.f : exp2f(sv - mn);
-            l[g] = l[g] * alpha + wave_reduce_sum(p);
-            if (mn != m[g]) {          // defer-rescale: skip when max held
-#pragma unroll
-                for (int i = 0; i < 8; ++i) facc[g][i] *= alpha;
-            }
-            m[g] = mn;
-            p_lds[g * 64 + lane] = p;
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        // P.V: RPI rows per b128 iteration; p read from same-wave LDS
-        // (an LDS hop, not shfl: it bounds how far the scheduler can
-        // interleave the K and V phases — shfl spilled 1.5 KB here)
-        const int jmax = min(64, seq - kb);
-        for (int jb = 0; jb < jmax; jb += RPI) {
-            const int j2 = jb + rg;
-            const uint4 vv = *(const uint4*)(
-                vblk + min(j2, jmax - 1) * D + d8);
-            float vf[8];
-            unpack8(vv, vf);
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const float p = (j2 < jmax) ? p_lds[g * 64 + j2] : 0.f;
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    facc[g][i] = fmaf(p, vf[i], facc[g][i]);
-            }
-        }
-    }
-
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-#pragma unroll
-            for (int off = 32; off >= DV; off >>= 1)
-                facc[g][i] += __shfl_xor(facc[g][i], off, WAVE);
-
-    if (lane < DV) {
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            if (nsplit == 1) {
-                const float f = epi.factor(b, hg * G + g, m[g], l[g]);
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    out[epi.at(b, hg * G + g, Hq, D) + d8 + i] =
-                        f2bf(facc[g][i] * f *
-                             epi.element(b, (hg * G + g) * D + d8 + i));
-            } else {
-                float* wsp = ws + (((long)b * Hq + hg * G + g) * nsplit
-                                   + split) * (D + 2);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) wsp[d8 + i] = facc[g][i];
-                if (lane == 0) {
-                    wsp[D] = m[g];
-                    wsp[D + 1] = l[g];
-                }
-            }
-        }
-    }
-}
-
-// Combine split-S partials: grid = B*Hq blocks, D threads.
-__global__ void
+// Combine split-S partials: a block of 256 per (row, head); nsplit <=
+// MAX_SPLIT. Splits that had no keys hold a maximum of -inf and no sums.
+template <int D>
+__global__ void __launch_bounds__(256)
 k_attn_combine(bf16_t* __restrict__ out, const float* __restrict__ ws,
-               int Hq, int D, int nsplit, const HeadEpilogue epi) {
+               int Hq, int nsplit, const HeadEpilogue epi) {
+    constexpr int NG = 256 / D;               // splits side by side
+    __shared__ float part[NG > 1 ? NG - 1 : 1][D];
     const long bh = blockIdx.x;               // b*Hq + hq
-    const int d = threadIdx.x;
+    const int d = threadIdx.x % D, grp = threadIdx.x / D;
+    const int lane = threadIdx.x & 63;
     const float* base = ws + bh * (long)nsplit * (D + 2);
-    float M = -INFINITY;
-    for (int s = 0; s < nsplit; ++s) M = fmaxf(M, base[s * (D + 2) + D]);
-    float num = 0.f, den = 0.f;
-    for (int s = 0; s < nsplit; ++s) {
-        const float* p = base + s * (long)(D + 2);
-        float ms = p[D];
-        float f = (ms == -INFINITY) ? 0.f : exp2f(ms - M);
-        num += f * p[d];
-        den += f * p[D + 1];
+    float ms = -INFINITY, ls = 0.f;
+    if (lane < nsplit) {
+        ms = base[lane * (D + 2) + D];
+        ls = base[lane * (D + 2) + D + 1];
+    }
+    const float M = wave_reduce_max(ms);
+    const float f = ms == -INFINITY ? 0.f : exp2f(ms - M);
+    const float den = wave_reduce_sum(ls * f);
+    const int used = __popcll(__ballot(ms != -INFINITY));   // the first ones
+    float num = 0.f;
+#pragma unroll 8
+    for (int s = grp; s < used; s += NG)
+        num = fmaf(__shfl(f, s, WAVE), base[s * (D + 2) + d], num);
+    if (NG > 1) {
+        if (grp) part[grp - 1][d] = num;
+        __syncthreads();
+        if (grp) return;
+#pragma unroll
+        for (int g = 0; g < NG - 1; ++g) num += part[g][d];
     }
     const int b = (int)(bh / Hq), h = (int)(bh % Hq);
     out[epi.at(b, h, Hq, D) + d] =
         f2bf(num * epi.factor(b, h, M, den) * epi.element(b, h * D + d));
 }
+
 // ===========================================================================
 // GQA prefill attention — flash-style on MFMA (bf16), reads K/V straight
 // from the cache.
@@ -506,8 +461,6 @@ k_attn_combine(bf16_t* __restrict__ out, const float* __restrict__ ws,
 //   C/D[i][j]: col j = l&31, row i = (reg&3) + 8*(reg>>2) + 4*(l>>5)
 // Constraints: D in {64, 128, 256}; Hq % Hk == 0.
 // ===========================================================================
-#define MAX_LAG 8.f
-
 // LDS elements of a block: two tiles of keys and values.
 template <int D>
 constexpr int prefill_lds() { return 2 * 64 * 2 * D; }

@@ -2220,14 +2220,9 @@ static void launch_paged_decode(hipStream_t st, void* out, const void* q,
                                 const HeadEpilogue& epi,
                                 const WindowKeys& keys) {
     const dim3 grid((unsigned)(B * kv.Hk * ngrp * nsplit));
-    if (nsplit == 1 && B * kv.Hk * ngrp >= 2048)
-        k_attn_decode1<D, G><<<grid, dim3(64), 0, st>>>(
-            (bf16_t*)out, (const bf16_t*)q, kv, pos, 1, slot, ws, ngrp,
-            nsplit, scale, epi, keys);
-    else
-        k_attn_decode<D, G><<<grid, dim3(256), 0, st>>>(
-            (bf16_t*)out, (const bf16_t*)q, kv, pos, 1, slot, ws, ngrp,
-            nsplit, scale, epi, keys);
+    k_attn_decode<D, G><<<grid, dim3(256), 0, st>>>(
+        (bf16_t*)out, (const bf16_t*)q, kv, pos, 1, slot, ws, ngrp, nsplit,
+        scale, epi, keys);
 }
 
 template <int D>
@@ -2252,8 +2247,8 @@ static int paged_decode(hipStream_t st, void* out, const void* q,
     }
     LAUNCH_CHECK();
     if (nsplit > 1) {
-        k_attn_combine<<<dim3((unsigned)(B * Hq)), dim3(D), 0, st>>>(
-            (bf16_t*)out, ws, Hq, D, nsplit, epi);
+        k_attn_combine<D><<<dim3((unsigned)(B * Hq)), dim3(256), 0, st>>>(
+            (bf16_t*)out, ws, Hq, nsplit, epi);
         LAUNCH_CHECK();
     }
     return 0;
@@ -2480,7 +2475,9 @@ int gh_paged_decode(void* stream, void* out, const void* q, const void* kc,
                     int Hq, int Hk, int D, int nsplit, float scale,
                     int window, int keep, const void* sink, const void* gate,
                     int gate_ld, int gate_el, float oscale, int out_ld) {
-    if (B < 1 || Hq % Hk || nsplit < 1 || window < 0 || keep < 0) return -100;
+    if (B < 1 || Hq % Hk || nsplit < 1 || nsplit > MAX_SPLIT || window < 0 ||
+        keep < 0)
+        return -100;
     const HeadEpilogue epi{(const float*)sink, (const bf16_t*)gate, gate_ld,
                            gate && gate_el, oscale, out_ld};
     const WindowKeys keys{window ? window : 1 << 30, keep};

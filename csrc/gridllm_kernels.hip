@@ -12,9 +12,8 @@
 //  * memory-bound ops target the HBM3E roofline (~6.3 TB/s achievable);
 //    the M<=512 decode projections are per-CU load-path/latency-bound, so
 //    gemm_proj pipelines both operands through LDS by global_load_lds.
-//  * attention decode: 4-wave cooperative workgroup per (batch, kv_head,
-//    split) for small batches (LDS combine, split-S partials), one-wave
-//    workgroups once B*Hk alone fills the chip.
+//  * attention decode: 4-wave workgroup per (batch, kv_head, split), K and V
+//    streamed through registers; split-S partials where B*Hk is small.
 //  * exported as extern "C" with an explicit hipStream_t so launches are
 //    capturable in hipGraphs from the Python host layer (ctypes binding —
 //    no torch C++ ABI dependency, no hipify, no CUDA shims).
@@ -739,18 +738,11 @@ static int launch_attn_decode(hipStream_t st, bf16_t* out, const bf16_t* q,
                               float* ws, int B, int Hk, int G, int Smax,
                               int nsplit, float scale) {
     dim3 grid((unsigned)(B * Hk * nsplit));
-    // one-wave variant only on the unsplit path (the auto-nsplit rule
-    // yields nsplit==1 whenever B*Hk >= 512, so this is the common case;
-    // explicit nsplit>1 calls keep the 4-wave cooperative kernel)
-    const bool onewave = nsplit == 1 && (B * Hk) >= 2048;
     const SlotKV<D> kv{kc, vc, Hk, Smax};
     const HeadEpilogue epi{nullptr, nullptr, 0};
     switch (G) {   // compile-time G keeps softmax state in registers
 #define CASE_G(GG) \
-        case GG: if (onewave) k_attn_decode1<D, GG><<<grid, dim3(64), 0, st>>>( \
-                out, q, kv, seqlen, 0, slot_map, ws, 1, nsplit, scale, epi, \
-                AllKeys()); \
-            else k_attn_decode<D, GG><<<grid, dim3(256), 0, st>>>( \
+        case GG: k_attn_decode<D, GG><<<grid, dim3(256), 0, st>>>( \
                 out, q, kv, seqlen, 0, slot_map, ws, 1, nsplit, scale, epi, \
                 AllKeys()); \
             break;
@@ -758,6 +750,12 @@ static int launch_attn_decode(hipStream_t st, bf16_t* out, const bf16_t* q,
         CASE_G(5) CASE_G(6) CASE_G(7) CASE_G(8)
 #undef CASE_G
         default: return -102;
+    }
+    LAUNCH_CHECK();
+    if (nsplit > 1) {
+        k_attn_combine<D><<<dim3((unsigned)(B * Hk * G)), dim3(256), 0, st>>>(
+            out, ws, Hk * G, nsplit, epi);
+        LAUNCH_CHECK();
     }
     return 0;
 }
@@ -829,7 +827,8 @@ int gl_attn_decode(void* stream, void* out, const void* q, const void* kc,
                    void* ws, int B, int Hq,
                    int Hk, int D, int Smax, int nsplit, float scale) {
     const int G = Hq / Hk;
-    if (Hq % Hk != 0 || G > MAXG || nsplit < 1) return -100;
+    if (Hq % Hk != 0 || G > MAXG || nsplit < 1 || nsplit > MAX_SPLIT)
+        return -100;
     hipStream_t st = (hipStream_t)stream;
     int rc;
     if (D == 128) {
@@ -845,15 +844,7 @@ int gl_attn_decode(void* stream, void* out, const void* q, const void* kc,
     } else {
         return -101;
     }
-    if (rc != 0) return rc;
-    LAUNCH_CHECK();
-    if (nsplit > 1) {
-        k_attn_combine<<<dim3((unsigned)(B * Hq)), dim3(D), 0, st>>>(
-            (bf16_t*)out, (const float*)ws, Hq, D, nsplit,
-            HeadEpilogue{nullptr, nullptr, 0});
-        LAUNCH_CHECK();
-    }
-    return 0;
+    return rc;
 }
 
 int gl_gemm_skinny(void* stream, void* out, void* ws, const void* x,

@@ -19,7 +19,7 @@ import torch.nn.functional as F
 
 from gridllm_amd.ops.build import lib_path
 from gridllm_amd.ops.hip_ops import (HipExtensionMissing, _check,
-                                     _check_range)
+                                     _check_range, decode_splits)
 from gridllm_amd.ops.reference import Glu
 from gridllm_amd.ops.reference_hybrid import (ALL_KEYS, Choice, Keys, StepMeta,
                                               Talk)
@@ -378,8 +378,7 @@ def paged_attn(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor,
         return out
     if st.nd:
         groups = h // max(d for d in range(1, 9) if (h // g) % d == 0)
-        nsplit = max(1, min(512 // max(1, st.nd * groups),
-                            (keys.most(st.max_len) + 255) // 256, 32))
+        nsplit = decode_splits(st.nd * groups, keys.most(st.max_len))
         ws = torch.empty(st.nd * h * nsplit * (p + 2), dtype=torch.float32,
                          device=q.device) if nsplit > 1 else None
         _call("gh_paged_decode", out, q, kc, vc, st.table, per, st.pos,

@@ -177,6 +177,22 @@ def kv_append(kcache: torch.Tensor, vcache: torch.Tensor, k_new: torch.Tensor,
                             _ptr(v_new), _ptr(slot), n, hk, d, smax), "kv_append")
 
 
+_MAX_SPLIT = 64                # what the combining kernel takes
+
+
+def decode_splits(blocks: int, keys: int) -> int:
+    """Into how many parts decode attention splits rows of up to `keys` keys,
+    `blocks` of them counting their kv heads: up to six workgroups a CU, none
+    for less than 128 keys. A row of fewer keys takes as many as it needs; the
+    others end at once, at 7 ns each, and the combining kernel takes longer.
+    Measured in us, 8 kv heads of 128: one row of 8000 keys 26 in 6 parts, 18
+    in 12, 15 in 32, 20 in 64; 24 rows of up to 6000 92 in one, 74 in 5, 70 in
+    8 and 12, 83 in 32; 64 rows of up to 2000 63 in one, 69 in 2, 62 in 3 to 6,
+    87 in 16; 256 rows of up to 384 47 in one, 62 in 2."""
+    return max(1, min(1536 // max(1, blocks), (keys + 127) // 128,
+                      32 if blocks <= 16 else 16))
+
+
 def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
                 seqlen: torch.Tensor, scale: float, nsplit: int = 0,
                 slot_map: Optional[torch.Tensor] = None,
@@ -189,9 +205,8 @@ def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
     b, hq, d = q.shape
     hk, smax = kcache.shape[1], kcache.shape[2]
     if nsplit <= 0:
-        # fill the chip: >=512 workgroups, but never splits smaller than 256 keys
-        max_useful = max(1, (smax + 255) // 256)
-        nsplit = max(1, min(512 // max(1, b * hk), max_useful, 32))
+        nsplit = decode_splits(b * hk, smax)
+    nsplit = min(nsplit, _MAX_SPLIT)
     _check_range("attn_decode.seqlen", seqlen, smax + 1)
     if slot_map is not None:
         _check_range("attn_decode.slot_map", slot_map, kcache.shape[0])

@@ -227,6 +227,34 @@ def test_attn_prefill_mfma_gpu(dev, t, hq, hk, d, cau):
     assert _mx(out.cpu(), ref) < 0.03
 
 
+@pytest.mark.parametrize("hq,hk,d", [(6, 2, 64), (8, 1, 128), (5, 1, 128)])
+@pytest.mark.parametrize("nsplit", [0, 1, 3, 64, 100])
+def test_attn_decode_step_edges_gpu(dev, hq, hk, d, nsplit):
+    """Lengths at the edges of steps of 32 and 64 keys and of splits, scores
+    that grow by more than the softmax reference's lag, NaN behind the last
+    key. Only q, k, v (as given) and the output are bf16: half a unit of 2^-8
+    of values up to 4."""
+    torch.manual_seed(hq + nsplit)
+    from gridllm_amd.ops import hip_ops
+    seqs = [1, 15, 16, 17, 31, 32, 33, 64, 65, 127, 128, 129, 257, 640]
+    b, smax = len(seqs), 640
+    q = torch.randn(b, hq, d, device=dev).to(torch.bfloat16)
+    kc = torch.randn(b, hk, smax, d, device=dev)
+    kc = (kc * torch.linspace(0.1, 4, smax, device=dev).view(1, 1, -1, 1)).to(
+        torch.bfloat16)
+    vc = torch.randn(b, hk, smax, d, device=dev).to(torch.bfloat16)
+    for i, n in enumerate(seqs):
+        kc[i, :, n:], vc[i, :, n:] = float("nan"), float("nan")
+    seqlen = torch.tensor(seqs, dtype=torch.int32, device=dev)
+    out = hip_ops.attn_decode(q, kc, vc, seqlen, -d ** -0.5, nsplit=nsplit)
+    for i, n in enumerate(seqs):
+        ref = R.attn_decode(
+            q[i:i + 1].cpu().float(), kc[i:i + 1, :, :n].cpu().float(),
+            vc[i:i + 1, :, :n].cpu().float(), seqlen[i:i + 1].cpu(),
+            -d ** -0.5)
+        assert _mx(out[i:i + 1].cpu(), ref) < 0.01, n
+
+
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("t,cau,sign", [
     (1, 0, 1), (33, 0, 1), (64, 63, 1), (65, 64, 1), (128, 1, -1),
