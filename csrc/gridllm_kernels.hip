@@ -349,6 +349,125 @@ k_gemm_skinny(bf16_t* __restrict__ out, float* __restrict__ ws,
 }
 
 // ===========================================================================
+// Few-row GEMM: out[M,N] = x[M,K] @ W[N,K]^T (bf16 I/O, f32 sums), M <= 16.
+//
+// Bound by streaming W, and for weights of a few MB by how soon all of it is on
+// its way: a block takes 16 columns over all of K, its 8 waves a part of K
+// each, whose loads (of W past the caches, of x from L2) start a batch of U
+// chunks ahead, straight into MFMA operands. The waves' sums meet in LDS, so
+// there is no second kernel and no workspace. One row, against k_gemm_skinny
+// and k_gemm_combine at their best split (a launch in a graph is 3.5 us):
+// 3072 x 3072 10.7 -> 6.9 us, 5120 x 3072 12.1 -> 11.3, 3072 x 8192
+// 18.3 -> 14.9; gate/up 16384 x 3072 (k_gemm_proj) 25.0 -> 24.7 us. Every block
+// reads all of x, which for 16 rows costs as much as W.
+// mfma_f32_16x16x32_bf16: A = x rows, B = W rows (k-contiguous both).
+// GLU: W rows in groups of 64 gate | 64 up; a block takes 16 of each and
+// stores the gated unit [M, N / 2].
+// Constraints: N % 16 == 0 (GLU: N % 128 == 0), K % 32 == 0.
+// ===========================================================================
+template <int GLU>
+__global__ void __launch_bounds__(512, 2)
+k_gemm_rows(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
+            const bf16_t* __restrict__ w, int M, int N, int K,
+            const GluParams glu) {
+    constexpr int WAVES = 8, U = 4, NC = GLU ? 2 : 1;
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int fr = lane & 15, kg = (lane >> 4) * 8;
+    const int n0 = GLU ? (blockIdx.x >> 2) * 128 + (blockIdx.x & 3) * 16
+                       : blockIdx.x * 16;
+    const int chunks = K >> 5;
+    const int per = (chunks + WAVES - 1) / WAVES;
+    const int c0 = wid * per, c1 = min(chunks, c0 + per);
+
+    const bf16_t* wp[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+        wp[i] = w + (long)(n0 + i * 64 + fr) * K + kg;
+    const bf16_t* xp = x + (long)min(fr, M - 1) * K + kg;
+
+    f32x4 acc[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) acc[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    bf16x8 a0[U], b0[U][NC], a1[U], b1[U][NC];
+    // chunks behind the last repeat it, and are not added
+    auto load = [&](bf16x8 (&a)[U], bf16x8 (&b)[U][NC], int c) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int at = min(c + u, c1 - 1) * 32;
+#pragma unroll
+            for (int i = 0; i < NC; ++i)
+                b[u][i] = __builtin_nontemporal_load(
+                    (const bf16x8*)(wp[i] + at));
+            a[u] = *(const bf16x8*)(xp + at);
+        }
+    };
+    auto add = [&](bf16x8 (&a)[U], bf16x8 (&b)[U][NC]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < NC; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    a[u], b[u][i], acc[i], 0, 0, 0);
+    };
+    // (Guards in `add` itself, and a last batch inside the loop, made the
+    // compiler overwrite operands that were still to be used.)
+    auto add_some = [&](bf16x8 (&a)[U], bf16x8 (&b)[U][NC], int n) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (u >= n) break;
+#pragma unroll
+            for (int i = 0; i < NC; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    a[u], b[u][i], acc[i], 0, 0, 0);
+        }
+    };
+    int c = c0, left = c1 - c0;
+    if (left > 0) {
+        load(a0, b0, c);
+        while (left > 2 * U) {
+            load(a1, b1, c + U);
+            add(a0, b0);
+            load(a0, b0, c + 2 * U);
+            add(a1, b1);
+            c += 2 * U;
+            left -= 2 * U;
+        }
+        if (left > U) {
+            load(a1, b1, c + U);
+            add(a0, b0);
+            add_some(a1, b1, left - U);
+        } else {
+            add_some(a0, b0, left);
+        }
+    }
+
+    // the waves' sums; lane holds row (l >> 4) * 4 + r, column l & 15
+    __shared__ f32x4 red[WAVES][NC][64];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) red[wid][i][lane] = acc[i];
+    __syncthreads();
+    if (wid) return;
+    f32x4 s[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        s[i] = red[0][i][lane];
+#pragma unroll
+        for (int v = 1; v < WAVES; ++v) s[i] += red[v][i][lane];
+    }
+    const int col = GLU ? (blockIdx.x >> 2) * 64 + (blockIdx.x & 3) * 16 + fr
+                        : n0 + fr;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int m = (lane >> 4) * 4 + r;
+        if (m < M)
+            out[(long)m * (GLU ? N >> 1 : N) + col] =
+                f2bf(GLU ? glu_act(s[0][r], s[NC - 1][r], glu) : s[0][r]);
+    }
+}
+
+// ===========================================================================
 // Projection GEMM for decode batches M in [65..512]:
 //   out[M,N] = x[M,K] @ W[N,K]^T (bf16 I/O, f32 accum)
 //
@@ -870,6 +989,23 @@ int gl_gemm_skinny(void* stream, void* out, void* ws, const void* x,
             (bf16_t*)out, (const float*)ws, mn, splitk);
         LAUNCH_CHECK();
     }
+    return 0;
+}
+
+int gl_gemm_rows(void* stream, void* out, const void* x, const void* w, int M,
+                 int N, int K, int fuse_glu, float alpha, float limit,
+                 float shift, float cubic) {
+    if (M < 1 || M > 16 || K < 32 || K % 32 || N % (fuse_glu ? 128 : 16))
+        return -100;
+    const GluParams glu{alpha, limit, shift, cubic};
+    hipStream_t st = (hipStream_t)stream;
+    if (fuse_glu)
+        k_gemm_rows<1><<<dim3((unsigned)(N / 32)), dim3(512), 0, st>>>(
+            (bf16_t*)out, (const bf16_t*)x, (const bf16_t*)w, M, N, K, glu);
+    else
+        k_gemm_rows<0><<<dim3((unsigned)(N / 16)), dim3(512), 0, st>>>(
+            (bf16_t*)out, (const bf16_t*)x, (const bf16_t*)w, M, N, K, glu);
+    LAUNCH_CHECK();
     return 0;
 }
 

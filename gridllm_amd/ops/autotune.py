@@ -168,7 +168,11 @@ def tune_gateup(m: int, n: int, k: int, device) -> tuple[str, int]:
 def linear_gateup(x: torch.Tensor, w_il: torch.Tensor,
                   glu: Glu = SWIGLU) -> torch.Tensor:
     """Fused gate/up projection + gated linear unit on an INTERLEAVED weight:
-    returns [M, F] activated. Dispatches through the tuned table."""
+    returns [M, F] activated. Few rows go to gemm_rows, others through the
+    tuned table."""
+    if x.dim() == 2 and x.shape[0] <= 16 and \
+            hip_ops.gemm_rows_wanted(x, w_il, fuse_swiglu=True):
+        return hip_ops.gemm_rows(x, w_il, fuse_swiglu=True, glu=glu)
     c = _CHOICE_GU.get((x.shape[0], w_il.shape[0], w_il.shape[1]))
     if c is not None and c[0] == "proj":
         return hip_ops.gemm_proj(x, w_il, splitk=c[1], fuse_swiglu=True,
@@ -184,8 +188,13 @@ def choice(m: int, n: int, k: int) -> Optional[tuple[str, int]]:
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """Dispatch x @ w.T through the tuned table (GPU bf16 2-D x only)."""
+    """Dispatch x @ w.T (GPU bf16 2-D x only): few rows to gemm_rows, others
+    through the tuned table."""
     if x.dim() == 2 and x.is_cuda and x.dtype == torch.bfloat16:
+        if x.shape[0] <= 16 and hip_ops.gemm_rows_wanted(x, w) and not (
+                torch.is_grad_enabled()
+                and (x.requires_grad or w.requires_grad)):
+            return hip_ops.gemm_rows(x, w)
         c = _CHOICE.get((x.shape[0], w.shape[0], w.shape[1]))
         if c is not None:
             if c[0] == "ours":

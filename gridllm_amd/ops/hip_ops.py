@@ -53,6 +53,8 @@ def _load() -> ctypes.CDLL:
     lib.gl_gemm_skinny.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp,
                                    c_i, c_i, c_i, c_i, c_i]
     lib.gl_gemm_skinny.restype = c_i
+    lib.gl_gemm_rows.argtypes = [c_vp] * 4 + [c_i] * 4 + [c_f] * 4
+    lib.gl_gemm_rows.restype = c_i
     lib.gl_gemm_proj.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp,
                                  c_i, c_i, c_i, c_i, c_i, c_i, c_i, c_i,
                                  c_f, c_f, c_f, c_f]
@@ -296,6 +298,43 @@ def gemm_skinny(x: torch.Tensor, w: torch.Tensor,
         ws = torch.empty(splitk * m * n, dtype=torch.float32, device=x.device)
     _check(lib.gl_gemm_skinny(_stream(), _ptr(out), _ptr(ws), _ptr(x), _ptr(w),
                               m, n, k, splitk, kslice), "gemm_skinny")
+    return out
+
+
+def gemm_rows_wanted(x: torch.Tensor, w: torch.Tensor,
+                     fuse_swiglu: bool = False) -> bool:
+    """Whether gemm_rows is the kernel for x [M, K] @ w [N, K]^T. For up to 4
+    rows it is the fastest here for every w but a vocabulary's (one row: 6.9 us
+    against 10.7 of the best split of gemm_skinny for 3072 x 3072, 11.3 against
+    12.1 for 5120 x 3072, 14.9 against 18.3 for 3072 x 8192; 128256 x 3072: 157
+    against 144 of the library's). Up to 16 rows it stays so for w of up to
+    20 MB, where a second launch costs more than every block's reading of x
+    (16 rows: 9.8 against 11.6, but 17.1 against 13.4 for 5120 x 3072). A
+    gate/up projection with its unit: 24.9 us against 25.3 of gemm_proj at 4
+    rows, 25.9 against 24.6 at 8."""
+    m, k = x.shape
+    n = w.shape[0]
+    return (0 < m <= (16 if n * k <= 10_000_000 and not fuse_swiglu else 4)
+            and n < 65536 and k % 32 == 0
+            and n % (128 if fuse_swiglu else 16) == 0
+            and x.is_contiguous() and w.is_contiguous()
+            and w.dtype == torch.bfloat16
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+
+
+def gemm_rows(x: torch.Tensor, w: torch.Tensor,
+              out: Optional[torch.Tensor] = None, fuse_swiglu: bool = False,
+              glu: Glu = SWIGLU) -> torch.Tensor:
+    """out[M,N] = x[M,K] @ w[N,K]^T, bf16, M <= 16: blocks of 16 columns over
+    all of K, without a workspace. fuse_swiglu: as in gemm_proj."""
+    lib = _load()
+    m, k = x.shape
+    n = w.shape[0]
+    if out is None:
+        out = torch.empty(m, n // 2 if fuse_swiglu else n,
+                          dtype=x.dtype, device=x.device)
+    _check(lib.gl_gemm_rows(_stream(), _ptr(out), _ptr(x), _ptr(w), m, n, k,
+                            1 if fuse_swiglu else 0, *glu), "gemm_rows")
     return out
 
 

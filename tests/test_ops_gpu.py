@@ -192,6 +192,32 @@ def test_gemm_skinny_gpu(dev, m, n, k):
     assert err < 0.02 * ref.abs().max().item(), err
 
 
+@pytest.mark.parametrize("m", [1, 2, 15, 16])
+@pytest.mark.parametrize("n,k", [
+    (128, 32), (1152, 896), (256, 224), (128, 4864), (2048, 2048),
+    (128, 8192), (384, 1056), (128, 2304),
+])
+def test_gemm_rows_gpu(dev, m, n, k):
+    """Rows, parts of K per wave (none, less than a batch, one and a part, two
+    and a part, several) and columns at their edges. bf16 operands as given,
+    f32 sums over K, one rounding of the result: 2^-9 of it and K 2^-24 of the
+    sum of magnitudes."""
+    torch.manual_seed(m + k)
+    from gridllm_amd.ops import hip_ops
+    x = torch.randn(m, k, device=dev).to(torch.bfloat16)
+    w = torch.randn(n, k, device=dev).to(torch.bfloat16)
+    ref = (x.cpu().double() @ w.cpu().double().t())
+    bound = ref.abs() * 2 ** -8 + k * 2 ** -24 * (
+        x.cpu().double().abs() @ w.cpu().double().abs().t())
+    out = hip_ops.gemm_rows(x, w)
+    assert ((out.cpu().double() - ref).abs() <= bound).all()
+    w = w * k ** -0.5
+    out = hip_ops.gemm_rows(x, w, fuse_swiglu=True)
+    v = (x.cpu().double() @ w.cpu().double().t()).view(m, n // 128, 2, 64)
+    g, u = v[:, :, 0].reshape(m, -1), v[:, :, 1].reshape(m, -1)
+    assert _mx(out.cpu().double(), g * torch.sigmoid(g) * u) < 0.05
+
+
 def test_gemm_skinny_splitk_consistent(dev):
     torch.manual_seed(10)
     from gridllm_amd.ops import hip_ops
