@@ -438,13 +438,13 @@ class SlotSampler:
         if all(s.greedy for s in states):
             return logits.argmax(dim=-1)
         need_filter = any(s.need_filter for s in states)
-        temps = self.temps[slot_ids].unsqueeze(1)
         if (logits.is_cuda and not need_filter
                 and os.environ.get("GRIDLLM_FUSED_SAMPLER", "1") != "0"):
             from gridllm_amd.ops import hip_ops
-            return hip_ops.sample_gumbel(
-                logits.contiguous(), self._keys(slot_ids).contiguous(),
-                temps.view(-1).contiguous())
+            return hip_ops.sample_gumbel_slots(
+                logits.contiguous(), slot_ids.long().contiguous(), self.temps,
+                self.seeds, self.draws, self.nongreedy)
+        temps = self.temps[slot_ids].unsqueeze(1)
         x = logits / temps
         v = logits.shape[1]
         if need_filter:

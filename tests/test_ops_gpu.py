@@ -388,6 +388,58 @@ def test_gemm_proj_wide_gpu(dev, m, n, k):
     assert (o1.float() - o4.float()).abs().max().item() < 0.05
 
 
+@pytest.mark.parametrize("b,v", [(1, 1), (3, 63), (2, 2047), (5, 4099),
+                                 (1, 128256), (64, 8192), (1100, 515)])
+def test_sample_gumbel_segments(dev, b, v):
+    """Rows of one and of several segments, of odd lengths, with -inf, +inf,
+    NaN, ties and close seconds, against the same formulas in 64-bit torch: the
+    picked value has to be the largest to f32's accuracy, by slot with the keys
+    of SlotSampler as with given keys."""
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator().manual_seed(b * v)
+    x = torch.randn(b, v, generator=g) * 3
+    x[:, ::3] = x[:, ::3].round()
+    x[0, v // 2:] = float("-inf")
+    if v > 8:
+        x[-1, 5] = float("nan")
+    if b > 2:
+        x[1] = float("-inf")
+        x[2, v - 1] = float("inf")
+    seeds = torch.randint(0, 2 ** 62, (b,), generator=g)
+    draws = torch.randint(0, 1000, (b,), generator=g)
+    live = (torch.arange(b) % 4 != 3).long()
+    temps = torch.rand(b, generator=g) + 0.3
+    keys = (seeds * 6364136223846793005
+            + (draws + 1) * 1442695040888963407) & ((1 << 63) - 1)
+    keys = keys * live
+    z = (torch.arange(v).unsqueeze(0) ^ keys.unsqueeze(1)) \
+        * -7046029254386353131
+    z = z ^ (z >> 29)
+    z = z * -4658895280553007687
+    z = z ^ (z >> 32)
+    u = (((z >> 38) & 0xFFFFFF).float() / (1 << 24)).clamp(1e-6, 1 - 1e-6)
+    val = x.double() / temps.double().unsqueeze(1) \
+        - torch.log(-torch.log(u.double())) * live.unsqueeze(1)
+    val = val.nan_to_num(nan=float("-inf"), posinf=1e30)
+    slots = torch.randperm(b, generator=g)
+    by = [torch.empty_like(t).index_copy(0, slots, t).to(dev)
+          for t in (temps, seeds, draws, live)]
+    got = hip_ops.sample_gumbel(x.to(dev), keys.to(dev), temps.to(dev))
+    got2 = hip_ops.sample_gumbel_slots(x.to(dev), slots.to(dev), *by)
+    assert torch.equal(got, got2)
+    assert torch.equal(by[2].cpu()[slots], draws + 1)
+    for r in range(b):
+        best = val[r].max()
+        if best == float("-inf"):
+            assert got[r] == 0
+        elif not live[r]:                     # no noise: the first of ties
+            assert got[r] == (x[r] / temps[r]).nan_to_num(
+                nan=float("-inf"), posinf=1e30).argmax()
+        else:                                 # a logarithm of 1 - 1e-6 is good
+            at = val[r, int(got[r])]          # to 2^-24 / 1e-6 in f32
+            assert at >= best - 1e-5 * abs(best) - 1e-4
+
+
 @pytest.mark.skipif(os.environ.get("GRIDLLM_FUSED_SAMPLER") == "0",
                     reason="fused sampler explicitly disabled")
 def test_sample_gumbel_matches_eager(dev):
