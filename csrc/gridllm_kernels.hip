@@ -27,61 +27,114 @@
 //   if res_in:  z = x + res_in; res_out = z  else z = x
 //   y = z * rsqrt(mean(z^2) + eps) * w
 // x,y,w,res: bf16. One workgroup (256 thr) per row; H % 8 == 0.
+// A row stays in registers between the two passes (NV chunks a thread, or
+// NV = 0: rows of any length, read twice): 8000 rows of 3072 with a residual 38
+// -> 33 us, 6 TB/s.
 // ===========================================================================
 
+template <int NV>
+DEV_INLINE void rmsnorm_row(bf16_t* yr, const bf16_t* xr, const bf16_t* w,
+                            const bf16_t* rr, bf16_t* ro, int H, float eps,
+                            float* red) {
+    const int nchunk = H >> 3;  // uint4 chunks
+    uint4 z[NV ? NV : 1];       // of this thread, rounded as they are stored
+    float ss = 0.f;
+    auto first = [&](int c) {
+        uint4 v = ((const uint4*)xr)[c];
+        float f[8];
+        unpack8(v, f);
+        if (rr) {
+            float g[8];
+            unpack8(((const uint4*)rr)[c], g);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f[i] += g[i];
+            v = pack8(f);
+            ((uint4*)ro)[c] = v;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ss += f[i] * f[i];
+        return v;
+    };
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            const int c = threadIdx.x + k * 256;
+            if (c < nchunk) z[k] = first(c);
+        }
+    } else {
+        for (int c = threadIdx.x; c < nchunk; c += 256) first(c);
+    }
+    const float scale = rsqrtf(block_sum(ss, red) / (float)H + eps);
+    auto second = [&](int c, const uint4 zv) {
+        float f[8], g[8];
+        unpack8(zv, f);
+        unpack8(((const uint4*)w)[c], g);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] = f[i] * scale * g[i];
+        ((uint4*)yr)[c] = pack8(f);
+    };
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            const int c = threadIdx.x + k * 256;
+            if (c < nchunk) second(c, z[k]);
+        }
+    } else {
+        const bf16_t* zr = rr ? ro : xr;
+        for (int c = threadIdx.x; c < nchunk; c += 256)
+            second(c, ((const uint4*)zr)[c]);
+    }
+}
+
+template <int NV>
 __global__ void __launch_bounds__(256)
 k_rmsnorm(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
           const bf16_t* __restrict__ w, const bf16_t* __restrict__ res_in,
           bf16_t* __restrict__ res_out, int H, float eps) {
-    const long row = blockIdx.x;
-    const bf16_t* xr = x + row * (long)H;
-    const bf16_t* rr = res_in ? res_in + row * (long)H : nullptr;
-    bf16_t* ro = res_out ? res_out + row * (long)H : nullptr;
-    bf16_t* yr = y + row * (long)H;
+    __shared__ float red[4];
+    const long at = blockIdx.x * (long)H;
+    rmsnorm_row<NV>(y + at, x + at, w, res_in ? res_in + at : nullptr,
+                    res_out ? res_out + at : nullptr, H, eps, red);
+}
 
-    __shared__ float s_red[4];
-    __shared__ float s_scale;
-
-    float ss = 0.f;
-    const int nchunk = H >> 3;  // uint4 chunks
-    for (int c = threadIdx.x; c < nchunk; c += 256) {
-        uint4 xv = ((const uint4*)xr)[c];
-        float f[8];
-        unpack8(xv, f);
-        if (rr) {
-            uint4 rv = ((const uint4*)rr)[c];
-            float g[8];
-            unpack8(rv, g);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) f[i] += g[i];
-            ((uint4*)ro)[c] = pack8(f);
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) ss += f[i] * f[i];
-    }
-    ss = wave_reduce_sum(ss);
-    const int wid = threadIdx.x >> 6;
-    const int lane = threadIdx.x & 63;
-    if (lane == 0) s_red[wid] = ss;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float t = s_red[0] + s_red[1] + s_red[2] + s_red[3];
-        s_scale = rsqrtf(t / (float)H + eps);
+// ===========================================================================
+// Start of a decode step: see gl_decode_positions. One block: its two passes
+// stand for the dozen index kernels of 4 us each that a step started with.
+// ===========================================================================
+__global__ void __launch_bounds__(1024)
+k_decode_positions(int* __restrict__ pos, int* __restrict__ slot_t,
+                   int* __restrict__ pos_rope, int* __restrict__ attn_seq,
+                   int* seq_lens, const int* __restrict__ rope_off,
+                   const int* __restrict__ slot_map, int B, int Smax) {
+    for (int i = threadIdx.x; i < B; i += 1024) {
+        const int s = slot_map[i], p = seq_lens[s];
+        pos[i] = p;
+        if (slot_t) slot_t[i] = s * Smax + p;
+        if (attn_seq) attn_seq[i] = p + 1;
+        if (pos_rope) pos_rope[i] = p + rope_off[s];
     }
     __syncthreads();
-    const float scale = s_scale;
+    for (int i = threadIdx.x; i < B; i += 1024)
+        atomicAdd(seq_lens + slot_map[i], 1);
+}
 
-    const bf16_t* zr = rr ? ro : xr;  // fused path re-reads the written residual (L1/L2 hot)
-    for (int c = threadIdx.x; c < nchunk; c += 256) {
-        uint4 zv = ((const uint4*)zr)[c];
-        uint4 wv = ((const uint4*)w)[c];
-        float f[8], g[8];
-        unpack8(zv, f);
-        unpack8(wv, g);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) f[i] = f[i] * scale * g[i];
-        ((uint4*)yr)[c] = pack8(f);
-    }
+// x = emb[token], y = rmsnorm(x) * w: one block per row. Tokens count from the
+// end if negative and are held to the table.
+template <int NV>
+__global__ void __launch_bounds__(256)
+k_embed_norm(bf16_t* __restrict__ x, bf16_t* __restrict__ y,
+             const bf16_t* __restrict__ emb,
+             const long long* __restrict__ tokens,
+             const bf16_t* __restrict__ w, int H, int vocab, float eps) {
+    __shared__ float red[4];
+    long long t = tokens[blockIdx.x];
+    if (t < 0) t += vocab;
+    t = t < 0 ? 0 : t < vocab ? t : vocab - 1;
+    const long at = blockIdx.x * (long)H;
+    const bf16_t* row = emb + t * H;
+    for (int c = threadIdx.x; c < H >> 3; c += 256)
+        ((uint4*)(x + at))[c] = ((const uint4*)row)[c];
+    rmsnorm_row<NV>(y + at, row, w, nullptr, nullptr, H, eps, red);
 }
 
 // ===========================================================================
@@ -200,6 +253,54 @@ k_rope_kv(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ q_out,
         dst[i] = f2bf(a * c - b * s);
         dst[i + half] = f2bf(a * s + b * c);
     }
+}
+
+// The same, 8 pairs a lane: half / 8 lanes turn a q or k head (two 16-byte
+// loads and stores), as many copy a v head; heads of all tokens lie one after
+// the other over the lanes. D % 16 == 0 and rows at 16 bytes. 8000 tokens of
+// 24 + 8 + 8 heads of 128: 83 us (2 TB/s) with a wave per head and 2-byte
+// accesses, 31 us (5.2 TB/s) now.
+__global__ void __launch_bounds__(256)
+k_rope_kv8(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ q_out,
+           bf16_t* __restrict__ kc, bf16_t* __restrict__ vc,
+           const float* __restrict__ cost, const float* __restrict__ sint,
+           const int* __restrict__ pos, const int* __restrict__ slot,
+           int N, int Hq, int Hk, int D, int Smax) {
+    const int half = D >> 1, lanes = half >> 3, heads = Hq + 2 * Hk;
+    const long i = blockIdx.x * 256L + threadIdx.x;
+    const long item = i / lanes;
+    if (item >= (long)N * heads) return;
+    const int c = (int)(i % lanes) * 8;
+    const int n = (int)(item / heads), h = (int)(item % heads);
+    const bf16_t* src = qkv + item * D + c;
+    uint4 lo = *(const uint4*)src, hi = *(const uint4*)(src + half);
+    if (h < Hq + Hk) {
+        const long at = (long)pos[n] * half + c;
+        float a[8], b[8], co[8], si[8];
+        ld8(cost + at, co);
+        ld8(sint + at, si);
+        unpack8(lo, a);
+        unpack8(hi, b);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const float u = a[k], v = b[k];
+            a[k] = u * co[k] - v * si[k];
+            b[k] = u * si[k] + v * co[k];
+        }
+        lo = pack8(a);
+        hi = pack8(b);
+    }
+    bf16_t* dst;
+    if (h < Hq) {
+        dst = q_out + ((long)n * Hq + h) * D + c;
+    } else {
+        const int s = slot[n], b = s / Smax, p = s - b * Smax;
+        const int hk = h < Hq + Hk ? h - Hq : h - Hq - Hk;
+        dst = (h < Hq + Hk ? kc : vc) + (((long)b * Hk + hk) * Smax + p) * D +
+              c;
+    }
+    *(uint4*)dst = lo;
+    *(uint4*)(dst + half) = hi;
 }
 
 // ===========================================================================
@@ -962,9 +1063,48 @@ extern "C" {
 int gl_rmsnorm(void* stream, void* y, const void* x, const void* w,
                const void* res_in, void* res_out, long n, int h, float eps) {
     if (h % 8 != 0) return -100;
-    k_rmsnorm<<<dim3((unsigned)n), dim3(256), 0, (hipStream_t)stream>>>(
-        (bf16_t*)y, (const bf16_t*)x, (const bf16_t*)w,
-        (const bf16_t*)res_in, (bf16_t*)res_out, h, eps);
+#define GO(NV) k_rmsnorm<NV> \
+        <<<dim3((unsigned)n), dim3(256), 0, (hipStream_t)stream>>>( \
+        (bf16_t*)y, (const bf16_t*)x, (const bf16_t*)w, \
+        (const bf16_t*)res_in, (bf16_t*)res_out, h, eps)
+    if (h <= 2048) GO(1);
+    else if (h <= 4096) GO(2);
+    else if (h <= 8192) GO(4);
+    else GO(0);
+#undef GO
+    LAUNCH_CHECK();
+    return 0;
+}
+
+// What a decode step starts with. Per batch row: position, place in the cache,
+// rotary position and number of keys of its slot, whose length goes up by one
+// (all rows read before any counts: rows may share a slot). slot_t, pos_rope,
+// attn_seq and rope_off may be null.
+int gl_decode_positions(void* stream, void* pos, void* slot_t, void* pos_rope,
+                        void* attn_seq, void* seq_lens, const void* rope_off,
+                        const void* slot_map, int B, int Smax) {
+    if (B < 1) return 0;
+    k_decode_positions<<<dim3(1), dim3(1024), 0, (hipStream_t)stream>>>(
+        (int*)pos, (int*)slot_t, (int*)pos_rope, (int*)attn_seq,
+        (int*)seq_lens, (const int*)rope_off, (const int*)slot_map, B, Smax);
+    LAUNCH_CHECK();
+    return 0;
+}
+
+int gl_embed_norm(void* stream, void* x, void* y, const void* emb,
+                  const void* tokens, const void* w, long n, int h, int vocab,
+                  float eps) {
+    if (h % 8 != 0 || vocab < 1) return -100;
+    if (n < 1) return 0;
+#define GO(NV) k_embed_norm<NV> \
+        <<<dim3((unsigned)n), dim3(256), 0, (hipStream_t)stream>>>( \
+        (bf16_t*)x, (bf16_t*)y, (const bf16_t*)emb, \
+        (const long long*)tokens, (const bf16_t*)w, h, vocab, eps)
+    if (h <= 2048) GO(1);
+    else if (h <= 4096) GO(2);
+    else if (h <= 8192) GO(4);
+    else GO(0);
+#undef GO
     LAUNCH_CHECK();
     return 0;
 }
@@ -1010,6 +1150,19 @@ int gl_rope_kv(void* stream, const void* qkv, void* q_out, void* kc, void* vc,
                const void* cost, const void* sint, const void* pos,
                const void* slot, int N, int Hq, int Hk, int D, int Smax) {
     if (D % 4 != 0 || N == 0) return (D % 4) ? -100 : 0;
+    const unsigned long ptrs = (unsigned long)qkv | (unsigned long)q_out |
+        (unsigned long)kc | (unsigned long)vc | (unsigned long)cost |
+        (unsigned long)sint;
+    if (D % 16 == 0 && ptrs % 16 == 0) {
+        const long items = (long)N * (Hq + 2 * Hk) * (D / 16);
+        k_rope_kv8<<<dim3((unsigned)((items + 255) / 256)), dim3(256), 0,
+                     (hipStream_t)stream>>>(
+            (const bf16_t*)qkv, (bf16_t*)q_out, (bf16_t*)kc, (bf16_t*)vc,
+            (const float*)cost, (const float*)sint, (const int*)pos,
+            (const int*)slot, N, Hq, Hk, D, Smax);
+        LAUNCH_CHECK();
+        return 0;
+    }
     k_rope_kv<<<dim3((unsigned)(N * (Hq + Hk))), dim3(64), 0,
                 (hipStream_t)stream>>>(
         (const bf16_t*)qkv, (bf16_t*)q_out, (bf16_t*)kc, (bf16_t*)vc,

@@ -982,11 +982,9 @@ class HybridModel:
         """One decode step of a batch, from device tensors alone (capturable):
         tokens [B] int64, slot_map [B] int32 -> logits f32 [B, vocab]. The
         cache must have been prepared for the slots (prepare_decode)."""
-        slots = slot_map.long()
-        st = StepMeta(nd=tokens.shape[0], pos=self.cache.seq_lens[slots],
-                      slot=slot_map, table=self.cache.table,
-                      max_len=self.max_seq, absorbed=tokens.shape[0])
+        pos = hops.decode_lengths(self.cache.seq_lens, slot_map)
+        st = StepMeta(nd=tokens.shape[0], pos=pos, slot=slot_map,
+                      table=self.cache.table, max_len=self.max_seq,
+                      absorbed=tokens.shape[0])
         x = self._run(tokens, st)
-        self.cache.seq_lens.index_add_(
-            0, slots, torch.ones_like(slot_map))
         return self._head(x, None)

@@ -479,14 +479,12 @@ class LlamaModel:
         Fully tensor-driven -> hipGraph-capturable."""
         s = self.spec
         b = tokens.shape[0]
-        pos = self.cache.seq_lens[slot_map.long()]          # [B] int32
-        slot_t = slot_map * self.cache.max_seq + pos
-        attn_seq = pos + 1
         # rope at the ABSOLUTE position (shifted slots have rope_off > 0)
-        pos_rope = pos + self.cache.rope_off[slot_map.long()]
-        x = self.embed[tokens]
-        resid = x
-        normed, _ = ops.rmsnorm(x, self.layers[0].attn_norm, s.norm_eps)
+        slot_t, pos_rope, attn_seq = ops.decode_positions(
+            self.cache.seq_lens, slot_map, self.cache.rope_off,
+            self.cache.max_seq)
+        resid, normed = ops.embed_norm(tokens, self.embed,
+                                       self.layers[0].attn_norm, s.norm_eps)
         for li, lw in enumerate(self.layers):
             qkv = _linear(normed, lw.wqkv)
             if lw.bqkv is not None:
@@ -507,8 +505,4 @@ class LlamaModel:
                          if li + 1 < len(self.layers) else self.final_norm)
             normed, resid = ops.rmsnorm(mlp_out, next_norm, s.norm_eps,
                                         residual=resid)
-        self.cache.seq_lens.index_add_(
-            0, slot_map.long(),
-            torch.ones(b, dtype=torch.int32, device=self.device))
-        logits = _linear(normed, self.lm_head).float()
-        return logits
+        return _linear(normed, self.lm_head).float()

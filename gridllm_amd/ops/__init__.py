@@ -38,6 +38,28 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float,
     return reference.rmsnorm(x, weight, eps, residual)
 
 
+def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
+                     rope_off: torch.Tensor, smax: int
+                     ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """Start of a decode step: cache places, rotary positions and key counts
+    of slots slot_map [B], whose lengths advance by one."""
+    if _on_gpu(seq_lens):
+        from gridllm_amd.ops import hip_ops
+        return hip_ops.decode_positions(
+            seq_lens, slot_map.int().contiguous(), rope_off, smax)
+    return reference.decode_positions(seq_lens, slot_map, rope_off, smax)
+
+
+def embed_norm(tokens: torch.Tensor, emb: torch.Tensor, weight: torch.Tensor,
+               eps: float) -> Tuple[torch.Tensor, torch.Tensor]:
+    """emb[tokens] and its rmsnorm."""
+    if _on_gpu(emb) and emb.dtype == torch.bfloat16:
+        from gridllm_amd.ops import hip_ops
+        return hip_ops.embed_norm(tokens.long().contiguous(), emb, weight, eps)
+    x = emb[tokens]
+    return x, rmsnorm(x, weight, eps)[0]
+
+
 def rope(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor,
          sin: torch.Tensor, pos: torch.Tensor
          ) -> Tuple[torch.Tensor, torch.Tensor]:

@@ -17,6 +17,7 @@ from typing import Callable, Optional, Union
 import torch
 import torch.nn.functional as F
 
+from gridllm_amd.ops import hip_ops
 from gridllm_amd.ops.build import lib_path
 from gridllm_amd.ops.hip_ops import (HipExtensionMissing, _check,
                                      _check_range, decode_splits)
@@ -120,6 +121,12 @@ def _dense(*ts: Optional[torch.Tensor]) -> None:
     for t in ts:
         if t is not None and not t.is_contiguous():
             raise ValueError("kernel operand is not contiguous")
+
+
+def decode_lengths(seq_lens: torch.Tensor,
+                   slot_map: torch.Tensor) -> torch.Tensor:
+    """The lengths of slots slot_map [B] int32, which then advance by one."""
+    return hip_ops.decode_lengths(seq_lens, slot_map.int().contiguous())
 
 
 def embed(tok: torch.Tensor, pos: torch.Tensor, emb: torch.Tensor,

@@ -38,6 +38,10 @@ def _load() -> ctypes.CDLL:
     c_vp, c_i, c_l, c_f = ctypes.c_void_p, ctypes.c_int, ctypes.c_long, ctypes.c_float
     lib.gl_rmsnorm.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_l, c_i, c_f]
     lib.gl_rmsnorm.restype = c_i
+    lib.gl_decode_positions.argtypes = [c_vp] * 8 + [c_i, c_i]
+    lib.gl_decode_positions.restype = c_i
+    lib.gl_embed_norm.argtypes = [c_vp] * 6 + [c_l, c_i, c_i, c_f]
+    lib.gl_embed_norm.restype = c_i
     lib.gl_rope.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i, c_i, c_i, c_i]
     lib.gl_rope.restype = c_i
     lib.gl_swiglu.argtypes = [c_vp, c_vp, c_vp, c_l, c_i, c_f, c_f, c_f, c_f]
@@ -124,6 +128,47 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float,
                           _ptr(residual), _ptr(residual_out), n, h,
                           ctypes.c_float(eps)), "rmsnorm")
     return out
+
+
+def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
+                     rope_off: torch.Tensor, smax: int
+                     ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """Start of a decode step over slots slot_map [B] int32 of seq_lens: cache
+    places slot * smax + length, rotary positions length + rope_off[slot], and
+    key counts length + 1, all int32 [B]. Advances the slots' lengths."""
+    b = slot_map.shape[0]
+    _check_range("decode_positions.slot_map", slot_map, seq_lens.shape[0])
+    out = torch.empty(4, b, dtype=torch.int32, device=seq_lens.device)
+    _check(_load().gl_decode_positions(
+        _stream(), _ptr(out[0]), _ptr(out[1]), _ptr(out[2]), _ptr(out[3]),
+        _ptr(seq_lens), _ptr(rope_off), _ptr(slot_map), b, smax),
+        "decode_positions")
+    return out[1], out[2], out[3]
+
+
+def decode_lengths(seq_lens: torch.Tensor,
+                   slot_map: torch.Tensor) -> torch.Tensor:
+    """The lengths of slots slot_map [B] int32, which then advance by one."""
+    b = slot_map.shape[0]
+    _check_range("decode_lengths.slot_map", slot_map, seq_lens.shape[0])
+    pos = torch.empty(b, dtype=torch.int32, device=seq_lens.device)
+    _check(_load().gl_decode_positions(
+        _stream(), _ptr(pos), None, None, None, _ptr(seq_lens), None,
+        _ptr(slot_map), b, 0), "decode_lengths")
+    return pos
+
+
+def embed_norm(tokens: torch.Tensor, emb: torch.Tensor, weight: torch.Tensor,
+               eps: float) -> tuple[torch.Tensor, torch.Tensor]:
+    """x = emb[tokens] [n, H] and rmsnorm(x) * weight; tokens [n] int64."""
+    n, h = tokens.shape[0], emb.shape[1]
+    _check_range("embed_norm.tokens", tokens, emb.shape[0])
+    x = torch.empty(n, h, dtype=emb.dtype, device=emb.device)
+    y = torch.empty_like(x)
+    _check(_load().gl_embed_norm(
+        _stream(), _ptr(x), _ptr(y), _ptr(emb), _ptr(tokens), _ptr(weight), n,
+        h, emb.shape[0], ctypes.c_float(eps)), "embed_norm")
+    return x, y
 
 
 def rope(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor,

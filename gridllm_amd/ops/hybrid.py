@@ -21,6 +21,7 @@ def _dispatch(name: str):
     return op
 
 
+decode_lengths = _dispatch("decode_lengths")
 embed = _dispatch("embed")
 post_norm = _dispatch("post_norm")
 sum_norm = _dispatch("sum_norm")

@@ -48,6 +48,18 @@ def rope_tables(head_dim: int, max_seq: int, theta: float = 500000.0,
     return freqs.cos().contiguous(), freqs.sin().contiguous()
 
 
+def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
+                     rope_off: torch.Tensor, smax: int
+                     ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """(slot * smax + length, length + rope_off[slot], length + 1) of slots
+    slot_map [B]; their lengths advance by one."""
+    slots = slot_map.long()
+    pos = seq_lens[slots]
+    out = slot_map * smax + pos, pos + rope_off[slots], pos + 1
+    seq_lens.index_add_(0, slots, torch.ones_like(pos))
+    return out
+
+
 def rope(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor,
          sin: torch.Tensor, pos: torch.Tensor
          ) -> Tuple[torch.Tensor, torch.Tensor]:

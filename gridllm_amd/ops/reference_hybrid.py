@@ -146,6 +146,13 @@ class DepthAverage:
     store: bool = True
 
 
+def decode_lengths(seq_lens, slot_map):
+    slots = slot_map.long()
+    pos = seq_lens[slots]
+    seq_lens.index_add_(0, slots, torch.ones_like(pos))
+    return pos
+
+
 def embed(tok, pos, emb, ptab, w=None, w_off=0.0, width=0, eps=0.0, out=None):
     x = emb[tok].float()
     if ptab is not None:

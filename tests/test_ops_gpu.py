@@ -153,7 +153,44 @@ def test_attn_decode_slot_map_gpu(dev):
     assert _mx(out.cpu(), ref) < 0.03
 
 
-@pytest.mark.parametrize("n,hq,hk,d", [(5, 24, 8, 128), (16, 32, 8, 64)])
+@pytest.mark.parametrize("b", [1, 63, 1024, 1500])
+def test_decode_positions_gpu(dev, b):
+    """Rows of one and several turns of the block, several rows on one slot."""
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator().manual_seed(b)
+    lens = torch.randint(0, 1000, (b + 1,), generator=g, dtype=torch.int32)
+    off = torch.randint(0, 1000, (b + 1,), generator=g, dtype=torch.int32)
+    slots = torch.randperm(b + 1, generator=g)[:b].int()
+    slots[b // 2:] = b
+    want = lens.clone()
+    ref = R.decode_positions(want, slots, off, 2048)
+    got = lens.to(dev)
+    out = hip_ops.decode_positions(got, slots.to(dev), off.to(dev), 2048)
+    for x, y in zip(out, ref):
+        assert torch.equal(x.cpu(), y)
+    assert torch.equal(got.cpu(), want)
+    assert torch.equal(hip_ops.decode_lengths(got, slots.to(dev)).cpu(),
+                       want[slots.long()])
+
+
+@pytest.mark.parametrize("n,h", [(1, 8), (5, 896), (3, 2056), (2, 8192),
+                                 (2, 8200)])
+def test_embed_norm_gpu(dev, n, h):
+    """Rows in registers and beyond: the bits of a lookup and of rmsnorm."""
+    from gridllm_amd.ops import hip_ops
+    emb = torch.randn(50, h, device=dev).to(torch.bfloat16)
+    w = torch.randn(h, device=dev).to(torch.bfloat16)
+    tok = torch.tensor([49, 0, -1, 7, 7][:n], device=dev)
+    x, y = hip_ops.embed_norm(tok, emb, w, 1e-5)
+    assert torch.equal(x, emb[tok])
+    assert torch.equal(y, hip_ops.rmsnorm(emb[tok], w, 1e-5))
+    ref, _ = R.rmsnorm(emb[tok].cpu().float(), w.cpu().float(), 1e-5)
+    # one rounding to bf16 of values up to 16
+    assert _mx(y.cpu(), ref) < 0.04
+
+
+@pytest.mark.parametrize("n,hq,hk,d", [(5, 24, 8, 128), (16, 32, 8, 64),
+                                       (7, 4, 2, 20), (1, 3, 1, 16)])
 def test_rope_kv_fused_gpu(dev, n, hq, hk, d):
     """Fused rope+kv-write vs the composed reference (strided qkv input)."""
     torch.manual_seed(8)
