@@ -118,6 +118,23 @@ k_decode_positions(int* __restrict__ pos, int* __restrict__ slot_t,
         atomicAdd(seq_lens + slot_map[i], 1);
 }
 
+// A prompt's positions start .. start + T - 1 and places in its slot, whose
+// length and rotary offset (if it starts anew) are set: one launch for six.
+__global__ void __launch_bounds__(256)
+k_prompt_positions(int* __restrict__ pos, int* __restrict__ slot_t,
+                   int* __restrict__ seq_lens, int* __restrict__ rope_off,
+                   int slot, int start, int T, int Smax) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < T) {
+        pos[i] = start + i;
+        slot_t[i] = slot * Smax + start + i;
+    }
+    if (i == 0) {
+        seq_lens[slot] = start + T;
+        if (start == 0) rope_off[slot] = 0;
+    }
+}
+
 // x = emb[token], y = rmsnorm(x) * w: one block per row. Tokens count from the
 // end if negative and are held to the table.
 template <int NV>
@@ -1087,6 +1104,17 @@ int gl_decode_positions(void* stream, void* pos, void* slot_t, void* pos_rope,
     k_decode_positions<<<dim3(1), dim3(1024), 0, (hipStream_t)stream>>>(
         (int*)pos, (int*)slot_t, (int*)pos_rope, (int*)attn_seq,
         (int*)seq_lens, (const int*)rope_off, (const int*)slot_map, B, Smax);
+    LAUNCH_CHECK();
+    return 0;
+}
+
+int gl_prompt_positions(void* stream, void* pos, void* slot_t, void* seq_lens,
+                        void* rope_off, int slot, int start, int T, int Smax) {
+    if (T < 1 || slot < 0 || start < 0) return -100;
+    k_prompt_positions<<<dim3((T + 255) / 256), dim3(256), 0,
+                         (hipStream_t)stream>>>(
+        (int*)pos, (int*)slot_t, (int*)seq_lens, (int*)rope_off, slot, start,
+        T, Smax);
     LAUNCH_CHECK();
     return 0;
 }

@@ -349,13 +349,12 @@ class LlamaModel:
         return_hidden, returns (logits, mean-pooled final hidden [H] f32)."""
         s = self.spec
         t = tokens.shape[0]
-        pos = torch.arange(start_pos, start_pos + t, dtype=torch.int32,
-                           device=self.device)
-        slot_t = torch.full((t,), slot * self.cache.max_seq, dtype=torch.int32,
-                            device=self.device) + pos
-        x = self.embed[tokens]                              # [T, H]
-        resid = x
-        normed, _ = ops.rmsnorm(x, self.layers[0].attn_norm, s.norm_eps)
+        # (a fresh slot's shift offset is reset: alloc is host-only)
+        pos, slot_t = ops.prompt_positions(
+            t, slot, start_pos, self.cache.seq_lens, self.cache.rope_off,
+            self.cache.max_seq)
+        resid, normed = ops.embed_norm(tokens, self.embed,
+                                       self.layers[0].attn_norm, s.norm_eps)
         for li, lw in enumerate(self.layers):
             qkv = _linear(normed, lw.wqkv)
             if lw.bqkv is not None:
@@ -377,10 +376,6 @@ class LlamaModel:
                          if li + 1 < len(self.layers) else self.final_norm)
             normed, resid = ops.rmsnorm(mlp_out, next_norm, s.norm_eps,
                                         residual=resid)
-        self.cache.seq_lens[slot] = start_pos + t
-        if start_pos == 0:
-            # fresh slot: reset the shift offset (alloc is host-only)
-            self.cache.rope_off[slot] = 0
         logits = _linear(normed[-1:], self.lm_head).float()
         if return_hidden:
             return logits[0], normed.float().mean(dim=0)
@@ -422,9 +417,8 @@ class LlamaModel:
                     for i, (ln, sl) in enumerate(zip(lens, slots))
                     for q0 in range(0, ln, 128)]
             meta = self.up.upload(np.asarray(rows, dtype=np.int32))
-        x = self.embed[tokens]
-        resid = x
-        normed, _ = ops.rmsnorm(x, self.layers[0].attn_norm, s.norm_eps)
+        resid, normed = ops.embed_norm(tokens, self.embed,
+                                       self.layers[0].attn_norm, s.norm_eps)
         for li, lw in enumerate(self.layers):
             qkv = _linear(normed, lw.wqkv)
             if lw.bqkv is not None:

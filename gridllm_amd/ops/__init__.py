@@ -50,6 +50,18 @@ def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
     return reference.decode_positions(seq_lens, slot_map, rope_off, smax)
 
 
+def prompt_positions(t: int, slot: int, start: int, seq_lens: torch.Tensor,
+                     rope_off: torch.Tensor, smax: int
+                     ) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Positions and cache places of t tokens from `start` on; sets the slot's
+    length, and its rope_off to 0 if start is 0."""
+    if _on_gpu(seq_lens):
+        from gridllm_amd.ops import hip_ops
+        return hip_ops.prompt_positions(t, slot, start, seq_lens, rope_off,
+                                        smax)
+    return reference.prompt_positions(t, slot, start, seq_lens, rope_off, smax)
+
+
 def embed_norm(tokens: torch.Tensor, emb: torch.Tensor, weight: torch.Tensor,
                eps: float) -> Tuple[torch.Tensor, torch.Tensor]:
     """emb[tokens] and its rmsnorm."""

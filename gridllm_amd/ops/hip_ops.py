@@ -40,6 +40,8 @@ def _load() -> ctypes.CDLL:
     lib.gl_rmsnorm.restype = c_i
     lib.gl_decode_positions.argtypes = [c_vp] * 8 + [c_i, c_i]
     lib.gl_decode_positions.restype = c_i
+    lib.gl_prompt_positions.argtypes = [c_vp] * 5 + [c_i] * 4
+    lib.gl_prompt_positions.restype = c_i
     lib.gl_embed_norm.argtypes = [c_vp] * 6 + [c_l, c_i, c_i, c_f]
     lib.gl_embed_norm.restype = c_i
     lib.gl_rope.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i, c_i, c_i, c_i]
@@ -84,8 +86,8 @@ def available() -> bool:
     return os.path.exists(_LIB_PATH)
 
 
-def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+def _stream() -> int:
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _check(rc: int, op: str) -> None:
@@ -93,8 +95,11 @@ def _check(rc: int, op: str) -> None:
         raise RuntimeError(f"HIP kernel {op} failed with code {rc}")
 
 
-def _ptr(t: Optional[torch.Tensor]) -> ctypes.c_void_p:
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+# Addresses stay plain numbers, which the declared signatures convert: a prompt
+# of a few layers and tokens is bound by what its launches cost the host (4 us
+# each less than with ctypes objects and torch's Stream object).
+def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
+    return None if t is None else t.data_ptr()
 
 
 # Debug validation (the sanitizer analog for a ctypes-bound kernel layer,
@@ -126,7 +131,7 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float,
         out = torch.empty_like(x)
     _check(lib.gl_rmsnorm(_stream(), _ptr(out), _ptr(x), _ptr(weight),
                           _ptr(residual), _ptr(residual_out), n, h,
-                          ctypes.c_float(eps)), "rmsnorm")
+                          eps), "rmsnorm")
     return out
 
 
@@ -144,6 +149,20 @@ def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
         _ptr(seq_lens), _ptr(rope_off), _ptr(slot_map), b, smax),
         "decode_positions")
     return out[1], out[2], out[3]
+
+
+def prompt_positions(t: int, slot: int, start: int, seq_lens: torch.Tensor,
+                     rope_off: torch.Tensor, smax: int
+                     ) -> tuple[torch.Tensor, torch.Tensor]:
+    """Positions start .. start + t - 1 and cache places slot * smax + those,
+    int32 [t]. Sets the slot's length, and its rope_off to 0 if start is 0."""
+    if not (0 <= slot < seq_lens.shape[0]):
+        raise IndexError(f"slot {slot} of {seq_lens.shape[0]}")
+    out = torch.empty(2, t, dtype=torch.int32, device=seq_lens.device)
+    _check(_load().gl_prompt_positions(
+        _stream(), _ptr(out[0]), _ptr(out[1]), _ptr(seq_lens), _ptr(rope_off),
+        slot, start, t, smax), "prompt_positions")
+    return out[0], out[1]
 
 
 def decode_lengths(seq_lens: torch.Tensor,
@@ -167,7 +186,7 @@ def embed_norm(tokens: torch.Tensor, emb: torch.Tensor, weight: torch.Tensor,
     y = torch.empty_like(x)
     _check(_load().gl_embed_norm(
         _stream(), _ptr(x), _ptr(y), _ptr(emb), _ptr(tokens), _ptr(weight), n,
-        h, emb.shape[0], ctypes.c_float(eps)), "embed_norm")
+        h, emb.shape[0], eps), "embed_norm")
     return x, y
 
 
@@ -267,7 +286,7 @@ def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
     _check(lib.gl_attn_decode(_stream(), _ptr(out), _ptr(q), _ptr(kcache),
                               _ptr(vcache), _ptr(seqlen), _ptr(slot_map),
                               _ptr(ws), b, hq, hk, d, smax, nsplit,
-                              ctypes.c_float(scale)), "attn_decode")
+                              scale), "attn_decode")
     return out
 
 
@@ -286,7 +305,7 @@ def attn_prefill_cache(q: torch.Tensor, kcache: torch.Tensor,
     _check(lib.gl_attn_prefill(_stream(), _ptr(out), _ptr(q), _ptr(kcache),
                                _ptr(vcache), t, hq, hk, d, smax, slot,
                                s_total, causal_offset,
-                               ctypes.c_float(scale)), "attn_prefill")
+                               scale), "attn_prefill")
     return out
 
 
@@ -312,7 +331,7 @@ def attn_prefill_cache_batch(q: torch.Tensor, kcache: torch.Tensor,
     _check(lib.gl_attn_prefill_batch(_stream(), _ptr(out), _ptr(q),
                                      _ptr(kcache), _ptr(vcache), _ptr(meta),
                                      ntiles, hq, hk, d, smax,
-                                     ctypes.c_float(scale)),
+                                     scale),
            "attn_prefill_batch")
     return out
 
@@ -493,7 +512,7 @@ def swiglu_il(gu: torch.Tensor, out: Optional[torch.Tensor] = None,
     if out is None:
         out = torch.empty(*gu.shape[:-1], f, dtype=gu.dtype, device=gu.device)
     _check(lib.gl_swiglu_il(_stream(), _ptr(out), _ptr(gu),
-                            ctypes.c_long(n), f, *glu), "swiglu_il")
+                            n, f, *glu), "swiglu_il")
     return out
 
 

@@ -48,6 +48,19 @@ def rope_tables(head_dim: int, max_seq: int, theta: float = 500000.0,
     return freqs.cos().contiguous(), freqs.sin().contiguous()
 
 
+def prompt_positions(t: int, slot: int, start: int, seq_lens: torch.Tensor,
+                     rope_off: torch.Tensor, smax: int
+                     ) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Positions start .. start + t - 1 and slot * smax + those; sets the
+    slot's length, and its rope_off to 0 if start is 0."""
+    pos = torch.arange(start, start + t, dtype=torch.int32,
+                       device=seq_lens.device)
+    seq_lens[slot] = start + t
+    if start == 0:
+        rope_off[slot] = 0
+    return pos, pos + slot * smax
+
+
 def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
                      rope_off: torch.Tensor, smax: int
                      ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
