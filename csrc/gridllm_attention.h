@@ -126,8 +126,8 @@ struct HeadEpilogue {
 // 24 heads of 128 over 8, before (a key row per lane, f32 scores, waves waiting
 // for their own loads) and now: 24 rows of up to 6000 keys 193 -> 70 us
 // (5.1 TB/s), 256 of up to 384 99 -> 46 us (5.2 TB/s), one of 900 17 -> 9 us.
-// Loads past the caches are 5 % faster than plain ones where the keys of all
-// rows exceed them.
+// V's loads go past the caches; K's, of half a cache line each, do not (both
+// halves would fetch it: 24 rows 73 us).
 // mfma_f32_16x16x32_bf16:
 //   A[i][k]: lane l holds i = l&15, k = (l>>4)*8 + 0..7
 //   B[k][j]: lane l holds j = l&15, same k chunk
@@ -241,7 +241,7 @@ k_attn_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
             const bf16_t* r = p + min(t * 16 + fr, last) * D;
 #pragma unroll
             for (int s = 0; s < ND; ++s)
-                kf[t][s] = __builtin_nontemporal_load((const bf16x8*)(r + s * 32));
+                kf[t][s] = *(const bf16x8*)(r + s * 32);
         }
     };
     typedef __attribute__((ext_vector_type(4))) u32 u32x4;

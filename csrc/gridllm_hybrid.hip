@@ -2119,20 +2119,21 @@ k_moe_gemm_few(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
 #pragma unroll
     for (int t = 0; t < NW; ++t) acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
     const int steps = K >> 5;
-    for (int s0 = wid; s0 < steps; s0 += 4 * U) {
+    for (int s0 = 0; s0 < steps; s0 += 4 * U) {
+        // a wave takes two neighbouring steps, whose loads share cache lines
+        auto step = [&](int u) { return s0 + ((u >> 1) * 4 + wid) * 2 + (u & 1); };
         bf16x8 a[U], b[U][NW];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int s = min(s0 + u * 4, steps - 1);
+            const int s = min(step(u), steps - 1);
 #pragma unroll
             for (int t = 0; t < NW; ++t)
-                b[u][t] = __builtin_nontemporal_load(
-                    (const bf16x8*)(wr + (long)t * 16 * K + s * 32));
+                b[u][t] = *(const bf16x8*)(wr + (long)t * 16 * K + s * 32);
             a[u] = *(const bf16x8*)(xr + s * 32);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (s0 + u * 4 < steps)
+            if (step(u) < steps)
 #pragma unroll
                 for (int t = 0; t < NW; ++t)
                     acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(

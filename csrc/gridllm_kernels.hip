@@ -349,7 +349,7 @@ k_kv_append(bf16_t* __restrict__ kc, bf16_t* __restrict__ vc,
 // The decode-path projection GEMMs (M = batch <= 256, W = torch linear
 // weight, row-major [N,K]) are HBM-bound on W. hipBLASLt reaches only ~40%
 // of the roofline on these shapes (profiles/r01_decode_profile.md), so this
-// kernel streams W once with non-temporal loads straight into MFMA B
+// kernel streams W once, straight into MFMA B
 // fragments — both operands are k-contiguous, so fragments load directly
 // from HBM/L2 with no LDS staging (guide: "GEMV / M<=16 decode weights:
 // load straight to VGPRs"; generalized to M<=256 via 16-row MFMA tiles).
@@ -373,7 +373,8 @@ k_gemm_skinny(bf16_t* __restrict__ out, float* __restrict__ ws,
     // kslice a small multiple of 256, so 2-8 blocks share each CU and TLP
     // hides the weight-stream latency (one wave per SIMD cannot — measured).
     // Per 256-k sub-slice the body is straight-line: issue all 8 B chunks
-    // (nt, 16 B/lane, k-contiguous), stage the x panel into LDS coalesced
+    // (16 B/lane, k-contiguous; not nontemporal: a load takes half a cache
+    // line, 24 rows of 9216 x 3072 in 8 parts 22.2 -> 19.6 us), stage the x panel into LDS coalesced
     // (XOR-swizzled), barrier, 8 x MT MFMAs off ds_read_b128 fragments.
     const int lane = threadIdx.x & 63;
     const int wid = threadIdx.x >> 6;
@@ -403,8 +404,7 @@ k_gemm_skinny(bf16_t* __restrict__ out, float* __restrict__ ws,
         bf16x8 bb[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u)
-            bb[u] = __builtin_nontemporal_load(
-                (const bf16x8*)(wrow + min(kp + u * 32, kcl)));
+            bb[u] = *(const bf16x8*)(wrow + min(kp + u * 32, kcl));
         // stage x[*, kp:kp+KS] -> LDS: thread c covers (row=c/32, kc=c%32);
         // 32 lanes read one row's 512 B contiguously; swizzled ds_write_b128
         if (kp > k0) __syncthreads();           // previous panel fully read
@@ -471,13 +471,15 @@ k_gemm_skinny(bf16_t* __restrict__ out, float* __restrict__ ws,
 //
 // Bound by streaming W, and for weights of a few MB by how soon all of it is on
 // its way: a block takes 16 columns over all of K, its 8 waves a part of K
-// each, whose loads (of W past the caches, of x from L2) start a batch of U
-// chunks ahead, straight into MFMA operands. The waves' sums meet in LDS, so
-// there is no second kernel and no workspace. One row, against k_gemm_skinny
-// and k_gemm_combine at their best split (a launch in a graph is 3.5 us):
-// 3072 x 3072 10.7 -> 6.9 us, 5120 x 3072 12.1 -> 11.3, 3072 x 8192
-// 18.3 -> 14.9; gate/up 16384 x 3072 (k_gemm_proj) 25.0 -> 24.7 us. Every block
-// reads all of x, which for 16 rows costs as much as W.
+// each, whose loads start a batch of U chunks ahead, straight into MFMA
+// operands. The waves' sums meet in LDS, so there is no second kernel and no
+// workspace. One row, against k_gemm_skinny and k_gemm_combine at their best
+// split (a launch in a graph is 3.5 us): 3072 x 3072 10.7 -> 7.2 us,
+// 5120 x 3072 12.1 -> 10.5, 3072 x 8192 18.3 -> 14.9; gate/up 16384 x 3072
+// (k_gemm_proj) 25.0 -> 21.5 us. Every block reads all of x, which for 16 rows
+// costs as much as W. W's loads are plain: each takes half a cache line of a
+// row, and past the caches (nontemporal) both halves fetch it: 8.0, 11.1, 16.6
+// and 24.3 us.
 // mfma_f32_16x16x32_bf16: A = x rows, B = W rows (k-contiguous both).
 // GLU: W rows in groups of 64 gate | 64 up; a block takes 16 of each and
 // stores the gated unit [M, N / 2].
@@ -516,8 +518,7 @@ k_gemm_rows(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
             const int at = min(c + u, c1 - 1) * 32;
 #pragma unroll
             for (int i = 0; i < NC; ++i)
-                b[u][i] = __builtin_nontemporal_load(
-                    (const bf16x8*)(wp[i] + at));
+                b[u][i] = *(const bf16x8*)(wp[i] + at);
             a[u] = *(const bf16x8*)(xp + at);
         }
     };

@@ -344,7 +344,7 @@ def gemm_skinny(x: torch.Tensor, w: torch.Tensor,
                 out: Optional[torch.Tensor] = None,
                 splitk: int = 0) -> torch.Tensor:
     """out[M,N] = x[M,K] @ w[N,K]^T, bf16, M<=256 (decode projections).
-    Streams w once (nt loads) into MFMA fragments; split-K sized to fill
+    Streams w once into MFMA fragments; split-K sized to fill
     256 CUs with f32 partial slabs + combine."""
     lib = _load()
     m, k = x.shape
@@ -369,14 +369,14 @@ def gemm_skinny(x: torch.Tensor, w: torch.Tensor,
 def gemm_rows_wanted(x: torch.Tensor, w: torch.Tensor,
                      fuse_swiglu: bool = False) -> bool:
     """Whether gemm_rows is the kernel for x [M, K] @ w [N, K]^T. For up to 4
-    rows it is the fastest here for every w but a vocabulary's (one row: 6.9 us
-    against 10.7 of the best split of gemm_skinny for 3072 x 3072, 11.3 against
-    12.1 for 5120 x 3072, 14.9 against 18.3 for 3072 x 8192; 128256 x 3072: 157
+    rows it is the fastest here for every w but a vocabulary's (one row: 7.2 us
+    against 10.7 of the best split of gemm_skinny for 3072 x 3072, 10.5 against
+    12.1 for 5120 x 3072, 14.9 against 16.6 for 3072 x 8192; 128256 x 3072: 157
     against 144 of the library's). Up to 16 rows it stays so for w of up to
     20 MB, where a second launch costs more than every block's reading of x
-    (16 rows: 9.8 against 11.6, but 17.1 against 13.4 for 5120 x 3072). A
-    gate/up projection with its unit: 24.9 us against 25.3 of gemm_proj at 4
-    rows, 25.9 against 24.6 at 8."""
+    (16 rows: 9.8 us against 11.2, but 16.5 against 12 for 5120 x 3072). A
+    gate/up projection with its unit: 23.4 us against 25.3 of gemm_proj at 4
+    rows, 27.7 against 24.7 at 16."""
     m, k = x.shape
     n = w.shape[0]
     return (0 < m <= (16 if n * k <= 10_000_000 and not fuse_swiglu else 4)
