@@ -117,23 +117,107 @@ DEV_INLINE float from_8_lanes_on(float x) {
 // keys a query at position p sees: from here on, up to p
 DEV_INLINE int first_seen(int p, int chunk) { return p / chunk * chunk; }
 
-// tiles of 32 keys of a split
-DEV_INLINE void split_tiles(int p, int chunk, int nsplit, int split, int* t0,
-                            int* t1) {
-    const int a = first_seen(p, chunk) >> 5, b = (p >> 5) + 1;
-    const int per = (b - a + nsplit - 1) / nsplit;
-    *t0 = a + split * per;
-    *t1 = min(b, *t0 + per);
+// 16-byte pieces of a tile's row are swapped by this: 8 rows' same piece lies in
+// 8 places, and so do 4 rows' pairs of pieces, which a transposed read takes.
+DEV_INLINE int twist(int row) { return (row & 3) << 1 | (row >> 2 & 1); }
+
+// Tiles of 32 keys that a row at position p sees, and the first of them.
+DEV_INLINE int seen_tiles(int p, int chunk, int* first) {
+    *first = first_seen(p, chunk) >> 5;
+    return (p >> 5) + 1 - *first;
+}
+
+// (x + c - 1) / c, exact up to 2^20, and no more than 255
+DEV_INLINE int parts_of(int x, float c) {
+    return min((int)((x + c - 0.5f) * __frcp_rn(c)), 255);
+}
+
+// Row and part of a block: each row's tiles in parts of about c, where c is the
+// smallest of some sizes that all rows' parts are `blocks` at most with, so that
+// all run at once; no row in parts if none is. N <= 256 rows; all lanes of a wave
+// find the same. Returns false for a block that is left over.
+struct Part { int n, split, parts, block0; };
+DEV_INLINE bool find_part(int b, int blocks, const int* pos, int last, int N,
+                          int chunk, Part* x) {
+    const int lane = threadIdx.x & 63;
+    int len[4], total = 0, first;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int n = lane * 4 + i;
+        const int p = min(pos[min(n, N - 1)], last);
+        len[i] = n < N ? seen_tiles(p, chunk, &first) : 0;
+        total += len[i];
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1)
+        total += __shfl_xor(total, off, WAVE);
+    // sizes from all rows' share of a block on to 8 times that
+    const int c0 = max(2, (total + blocks - 1) / blocks);
+    auto size = [&](int k) {
+        return (float)(int)(c0 * fast_exp2(k * 0.2f) + 0.5f);
+    };
+    u32 sums[8];                       // of two sizes each
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        sums[k] = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            sums[k] += parts_of(len[i], size(2 * k)) |
+                       parts_of(len[i], size(2 * k + 1)) << 16;
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) sums[k] += __shfl_xor(sums[k], off, WAVE);
+    int best = 16;
+#pragma unroll
+    for (int k = 7; k >= 0; --k) {
+        if ((int)(sums[k] >> 16) <= blocks) best = 2 * k + 1;
+        if ((int)(sums[k] & 0xffff) <= blocks) best = 2 * k;
+    }
+    const float c = best < 16 ? size(best) : 1e6f;
+    int cnt[4], ahead = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ahead += cnt[i] = parts_of(len[i], c);
+    const int mine = ahead;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(ahead, off, WAVE);
+        ahead += lane >= off ? y : 0;
+    }
+    const int all = __builtin_amdgcn_readlane(ahead, 63);
+    if (b >= all) return false;
+    ahead -= mine;
+    const int at = __popcll(__ballot(ahead <= b && mine > 0)) - 1;
+    int s = b - __builtin_amdgcn_readlane(ahead, at), n = at * 4;
+    x->parts = __builtin_amdgcn_readlane(cnt[0], at);
+#pragma unroll
+    for (int i = 1; i < 4; ++i) {
+        if (n == at * 4 + i - 1 && s >= x->parts) {
+            s -= x->parts;
+            x->parts = __builtin_amdgcn_readlane(cnt[i], at);
+            ++n;
+        }
+    }
+    x->n = n;
+    x->split = s;
+    x->block0 = b - s;
+    return true;
 }
 
 // ===========================================================================
-// Decode. Block: a row and a split of its keys; tiles of 32 keys of all G value
+// Decode. Block: a row (ws == null) or a part of a row's keys; tiles of 32 keys of all G value
 // heads go through LDS (16-byte pieces XOR-swizzled by the row), the next one
 // in flight. Scores: up to 16 heads of one value head against 16 keys are one
 // item, and a wave has one or two of the same heads; the weights meet in LDS,
 // and a wave then has all heads' weights against CW columns of one value head.
-//   ws (nsplit > 1): sums [N][nsplit][G][H][P], and behind them the weights'
-//   sums [N][nsplit][H]
+//   ws: sums [blocks][G][H][P], the weights' sums [blocks][H], and of each row
+//   the first block and the number of its parts, int [N][2]
+// Bound by the tiles' way to LDS: a block fits a CU once (24 heads, 8 values of
+// 128) and takes 3.4 us for a tile of 64 KB, 4.9 TB/s if all CUs have a block.
+// With a block per row, 160 rows of up to 1000 keys took 105 us, the longest
+// row's time, on 160 of 256 CUs; in parts they take 75, the combining kernel's 7
+// included, and rows of 1000 keys all, which are left whole, 114 (112).
 // ===========================================================================
 template <int P, int GP, int HB, int R>
 struct DecodeShape {
@@ -160,7 +244,7 @@ k_talk_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
               const int* __restrict__ pos, const int* __restrict__ slot,
               float* __restrict__ ws, const float* __restrict__ kw,
               const float* __restrict__ talk, const Rotation rot, int N,
-              int H, int G, int chunk, int nsplit, const Cap cap) {
+              int H, int G, int chunk, const Cap cap) {
     typedef DecodeShape<P, GP, HB, R> Sh;
     constexpr int WAVES = Sh::WAVES, CW = Sh::CW, CH = P / 8;
     constexpr int NS = P / 32, RS = R / 32, NT = CW / 16, PLD = Sh::PLD;
@@ -170,15 +254,23 @@ k_talk_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
     float* const ls = (float*)(smem + Sh::ELEMS);   // [2][HB * 16]
     float* const ivs = ls + HB * 32;                // [2][GP][32]
     float* const tabs = ivs + GP * 64;              // cos, sin [32][R / 2]
-    const int n = blockIdx.x / nsplit, split = blockIdx.x % nsplit;
     const int lane = threadIdx.x & 63, wv = wave_number();
     const int fr = lane & 15, gq = lane >> 4;
     const int rep = H / G, rbn = (rep + 15) >> 4, items = 2 * G * rbn;
     const int per = (items + WAVES - 1) / WAVES;    // 1 or 2
+    Part own{(int)blockIdx.x, 0, 1, 0};
+    if (ws && !find_part(blockIdx.x, gridDim.x, pos, per_slot * PAGE - 1, N,
+                         chunk, &own)) return;
+    const int n = own.n;
     const int p = min(pos[n], per_slot * PAGE - 1);
     const int lo = first_seen(p, chunk);
-    int t0, t1;
-    split_tiles(p, chunk, nsplit, split, &t0, &t1);
+    int t0;
+    const int tiles = seen_tiles(p, chunk, &t0);
+    const int share = (tiles + own.parts - 1) / own.parts;
+    const int live = (tiles + share - 1) / share, end = t0 + tiles;
+    t0 += own.split * share;
+    const int t1 = min(t0 + share, end);
+    if (t0 >= t1) return;
     const int* tab = table + (long)slot[n] * per_slot;
 
     auto issue = [&](int t, long page) {
@@ -190,7 +282,7 @@ k_talk_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
             const int kv = pc / (32 * CH), row = pc / CH % 32, c = pc % CH;
             if (kv < G)                            // the same for a wave
                 load_lds16(src + ((long)kv * PAGE + row) * P +
-                               (c ^ (row & 7)) * 8,
+                               (c ^ twist(row)) * 8,
                            dst + (i * WAVES + wv) * 512);
         }
         const int kv = wv * 8 + (lane >> 3);       // 8 value heads a wave
@@ -215,12 +307,9 @@ k_talk_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
                            (bf16_t*)(tabs + w * 256));
         }
     };
-    int page = tab[min(t0, t1 - 1) >> 1];
-    if (t0 < t1) {
-        issue(t0, page);
-        issue_rotation(t0);
-        page = tab[min(t0 + 1, t1 - 1) >> 1];
-    }
+    issue(t0, tab[t0 >> 1]);
+    issue_rotation(t0);
+    int page = tab[min(t0 + 1, t1 - 1) >> 1];
     // this wave's scores: up to 16 heads of one value head, 16 or 32 keys.
     // Behind the rotated part the keys' weights go into the queries.
     const int sg = min(wv * per >> 1, G * rbn - 1), kv = sg / rbn;
@@ -242,7 +331,6 @@ k_talk_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
     const bool few = rep <= 8;
     for (int i = threadIdx.x; i < HB * 16 * PLD / 2; i += WAVES * 64)
         ((u32*)pb)[i] = 0;
-    if (threadIdx.x < HB * 32) ls[threadIdx.x] = 0.f;
 
     const int vh = wv * CW / P, part = wv * CW % P;   // value head, column
     float l[2] = {0.f, 0.f};
@@ -266,7 +354,7 @@ k_talk_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
 #pragma unroll
             for (int s = 0; s < NS; ++s)
                 kf[s] = *(const bf16x8*)(tile + (kv * 32 + row) * P +
-                                         ((s * 4 + gq) ^ (row & 7)) * 8);
+                                         ((s * 4 + gq) ^ twist(row)) * 8);
 #pragma unroll
             for (int s = 0; s < RS; ++s) {
                 const int c = s * 32 + gq * 8;
@@ -337,7 +425,7 @@ k_talk_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
             for (int j = 0; j < 2; ++j) {
                 const int row = gq * 8 + (fr >> 2) + j * 4;
                 const bf16x4 x = read_transposed(
-                    tile + (vh * 32 + row) * P + ((d >> 3) ^ (row & 7)) * 8 +
+                    tile + (vh * 32 + row) * P + ((d >> 3) ^ twist(row)) * 8 +
                     (d & 7));
 #pragma unroll
                 for (int i = 0; i < 4; ++i) v[j * 4 + i] = x[i];
@@ -348,8 +436,7 @@ k_talk_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
                     pf[b], v, acc[b][c], 0, 0, 0);
         }
     }
-    lds_barrier();                  // ls is cleared, also without a tile
-    if (mine > 0) {
+    if (mine > 0) {                 // (each head's two sums have a writer)
         float s[2] = {l[0], l[1]};
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -363,12 +450,15 @@ k_talk_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
         }
     }
     __syncthreads();
-    if (nsplit > 1) {
-        const long at = (long)n * nsplit + split;
-        float* wl = ws + (long)N * nsplit * G * H * P + at * H;
+    if (ws && own.split == 0 && threadIdx.x == 0)
+        *(int2*)(ws + (long)gridDim.x * (G * H * P + H) + n * 2) =
+            make_int2(own.block0, live);
+    if (live > 1) {
+        const long at = blockIdx.x;
+        float* wl = ws + (long)gridDim.x * G * H * P + at * H;
         for (int h = threadIdx.x; h < H; h += WAVES * 64)
             wl[h] = ls[h] + ls[HB * 16 + h];
-        if (vh >= G || t0 >= t1) return;
+        if (vh >= G) return;
         float* wo = ws + (at * G + vh) * H * P + part + fr;
 #pragma unroll
         for (int b = 0; b < HB; ++b)
@@ -415,81 +505,82 @@ k_talk_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
     }
 }
 
-// Splits of a row added up, normalised and mixed. Block: a row, a value head,
-// 32 columns; 256 threads are 32 score heads by 8 x 4 columns. H <= 64.
+// Parts of a row added up, normalised and mixed. Block: a row, a value head, COLS
+// columns: threads are 16-byte pieces of these by STEP score heads, and each has
+// KM of the up to HB * 16. Bound by latency, the parts being in the caches. Of
+// blocks of 128 columns there are few enough to run at once with many rows: 160
+// rows, of which 80 are in parts, take 75 us in all with these and 81 with blocks
+// of 32 columns (8 values of 128, 24 heads); 32 rows take 36 and 32, one row of
+// 1000 keys 32 and 19, as more of a row's parts are loaded at once.
+template <int HB, int COLS>
 __global__ void __launch_bounds__(256)
 k_talk_combine(bf16_t* __restrict__ out, const float* __restrict__ ws,
-               const float* __restrict__ talk, const int* __restrict__ pos,
-               int per_slot, int N, int H, int G, int P, int chunk,
-               int nsplit, float rho) {
-    __shared__ __attribute__((aligned(16))) float red[4][4][32];
+               const float* __restrict__ talk, int H, int G, int P, int blocks,
+               float rho) {
+    constexpr int PIECES = COLS / 4, STEP = 256 / PIECES;
+    constexpr int KM = (HB * 16 + STEP - 1) / STEP;
+    __shared__ __attribute__((aligned(16))) float red[4][4][COLS];
     __shared__ float nrm[64];
-    const int n = blockIdx.x, kv = blockIdx.y, rep = H / G;
-    const int c0 = blockIdx.z * 32, tid = threadIdx.x;
-    const int c = c0 + (tid & 7) * 4, g0 = tid >> 3;
-    const int p = min(pos[n], per_slot * PAGE - 1);
-    int t0, t1, live = 0;              // splits that have keys come first
-    for (; live < nsplit; ++live) {
-        split_tiles(p, chunk, nsplit, live, &t0, &t1);
-        if (t0 >= t1) break;
-    }
-    constexpr int U = 8;               // rows in flight
-    const float* wl = ws + (long)N * nsplit * G * H * P + (long)n * nsplit * H;
-    if (tid < H) {
-        float l = exp2f(-rho);
-        for (int s0 = 0; s0 < live; s0 += U) {
-            float f[U];
+    const int n = blockIdx.x, kv = blockIdx.y, rep = H / G, tid = threadIdx.x;
+    const int c0 = blockIdx.z * COLS, cl = tid % PIECES * 4, g0 = tid / PIECES;
+    const float* wl = ws + (long)blocks * G * H * P + min(tid, H - 1);
+    const int2 own = *(const int2*)(ws + (long)blocks * (G * H * P + H) + n * 2);
+    const int live = own.y;
+    if (live == 1) return;             // its block has stored the result
+    const long b0 = own.x;
+    float l = exp2f(-rho), o[KM][4] = {};
+    auto add = [&](auto U, int s) {    // U parts in flight
+        float f[U][KM][4], x[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-                f[u] = wl[min(s0 + u, live - 1) * H + tid];
+        for (int u = 0; u < U; ++u) {
+            x[u] = wl[(b0 + s + u) * H];
 #pragma unroll
-            for (int u = 0; u < U; ++u) l += s0 + u < live ? f[u] : 0.f;
+            for (int k = 0; k < KM; ++k)
+                ld4(ws + (((b0 + s + u) * G + kv) * H +
+                          min(g0 + k * STEP, H - 1)) * P + c0 + cl, f[u][k]);
         }
-        nrm[tid] = 1.f / l;
-    }
-    float o[2][4] = {};
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const int g = g0 + k * 32;
-        if (g >= H) break;
-        const float* src = ws + (((long)n * nsplit * G + kv) * H + g) * P + c;
-        for (int s0 = 0; s0 < live; s0 += U) {
-            float f[U][4];
+        for (int u = 0; u < U; ++u) {
+            l += x[u];
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-                ld4(src + (long)min(s0 + u, live - 1) * G * H * P, f[u]);
+            for (int k = 0; k < KM; ++k)
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (s0 + u < live)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) o[k][j] += f[u][j];
+                for (int j = 0; j < 4; ++j) o[k][j] += f[u][k][j];
         }
-    }
+    };
+    constexpr int U = KM > 4 ? 2 : KM > 2 ? 4 : 8;
+    int s = 0;
+    for (; s + U <= live; s += U) add(std::integral_constant<int, U>(), s);
+    for (; s < live; ++s) add(std::integral_constant<int, 1>(), s);
+    if (tid < H) nrm[tid] = 1.f / l;
     for (int i0 = 0; i0 < rep; i0 += 4) {
         __syncthreads();               // nrm is there, red is free
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
+            const float* row = talk + (kv * rep + min(i0 + i, rep - 1)) * H;
             float a[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                const int g = g0 + k * 32;
-                if (g >= H || i0 + i >= rep) continue;
-                const float x = talk[(kv * rep + i0 + i) * H + g] * nrm[g];
+            for (int k = 0; k < KM; ++k) {
+                const int g = g0 + k * STEP;
+                const float x = g < H ? row[min(g, H - 1)] * nrm[min(g, H - 1)]
+                                      : 0.f;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) a[j] += x * o[k][j];
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int off = 8; off < 64; off <<= 1)
+                for (int off = PIECES; off < 64; off <<= 1)
                     a[j] += __shfl_xor(a[j], off, WAVE);
-            if ((tid & 63) < 8) st4(&red[tid >> 6][i][(tid & 7) * 4], a);
+            if ((tid & 63) < PIECES) st4(&red[tid >> 6][i][cl], a);
         }
         __syncthreads();
-        const int i = tid >> 5, d = tid & 31;
-        if (i < 4 && i0 + i < rep)
-            out[((long)n * H + kv * rep + i0 + i) * P + c0 + d] =
-                f2bf(red[0][i][d] + red[1][i][d] + red[2][i][d] + red[3][i][d]);
+        for (int at = tid; at < 4 * COLS; at += 256) {
+            const int i = at / COLS, d = at % COLS;
+            if (i0 + i < rep)
+                out[((long)n * H + kv * rep + i0 + i) * P + c0 + d] = f2bf(
+                    red[0][i][d] + red[1][i][d] + red[2][i][d] + red[3][i][d]);
+        }
     }
 }
 
@@ -979,19 +1070,24 @@ static int go_decode(hipStream_t st, bf16_t* out, const bf16_t* q,
                      const bf16_t* vc, const float* inv, const int* table,
                      int per_slot, const int* pos, const int* slot, float* ws,
                      const float* kw, const float* talk, const Rotation rot,
-                     int N, int H, int G, int chunk, int nsplit,
+                     int N, int H, int G, int chunk, int blocks,
                      const Cap cap) {
     typedef DecodeShape<P, GP, HB, R> Sh;
     if (Sh::BYTES > 160 * 1024) return -102;
     const int e = allow_lds<k_talk_decode<P, GP, HB, R>>(Sh::BYTES);
     if (e) return e;
-    k_talk_decode<P, GP, HB, R><<<N * nsplit, Sh::WAVES * 64, Sh::BYTES, st>>>(
+    k_talk_decode<P, GP, HB, R><<<ws ? blocks : N, Sh::WAVES * 64, Sh::BYTES,
+                                  st>>>(
         out, q, vc, inv, table, per_slot, pos, slot, ws, kw, talk, rot, N, H,
-        G, chunk, nsplit, cap);
+        G, chunk, cap);
     LAUNCH_CHECK();
-    if (nsplit > 1) {
-        k_talk_combine<<<dim3(N, G, P / 32), 256, 0, st>>>(
-            out, ws, talk, pos, per_slot, N, H, G, P, chunk, nsplit, cap.rho);
+    if (ws) {
+        if (P >= 128 && N >= 96)
+            k_talk_combine<HB, 128><<<dim3(N, G, P / 128), 256, 0, st>>>(
+                out, ws, talk, H, G, P, blocks, cap.rho);
+        else
+            k_talk_combine<HB, 32><<<dim3(N, G, P / 32), 256, 0, st>>>(
+                out, ws, talk, H, G, P, blocks, cap.rho);
         LAUNCH_CHECK();
     }
     return 0;
@@ -1023,19 +1119,18 @@ int gt_talk_decode(void* stream, void* out, const void* q, const void* vc,
                    const void* pos, const void* slot, void* ws,
                    const void* kw, const void* talk, const void* cos_,
                    const void* sin_, int nrot, int N, int H, int G, int P,
-                   int R, int chunk, int nsplit, float rate, float top,
+                   int R, int chunk, int blocks, float rate, float top,
                    float rho) {
-    if (N < 1 || !sizes_ok(H, G, P, R, nrot, chunk) || nsplit < 1 ||
-        nsplit > 64 || H > 64 || G * P > 1024 ||
-        nrot < per_slot * PAGE ||
-        (nsplit > 1 && !ws)) return -100;
+    if (N < 1 || !sizes_ok(H, G, P, R, nrot, chunk) || H > 64 ||
+        G * P > 1024 || nrot < per_slot * PAGE ||
+        (ws && (N > 256 || blocks < 1))) return -100;
     const Rotation rot = rotation(cos_, sin_, R, nrot);
     const Cap cap{rate, top, rho};
 #define GO(A, B, C, D) return go_decode<A, B, C, D>((hipStream_t)stream, \
         (bf16_t*)out, (const bf16_t*)q, (const bf16_t*)vc, \
         (const float*)inv, (const int*)table, per_slot, (const int*)pos, \
         (const int*)slot, (float*)ws, (const float*)kw, (const float*)talk, \
-        rot, N, H, G, chunk, nsplit, cap)
+        rot, N, H, G, chunk, blocks, cap)
 #define HEADS(A, B, D) do { if (H <= 16) GO(A, B, 1, D); \
         else if (H <= 32) GO(A, B, 2, D); else GO(A, B, 4, D); } while (0)
 #define VALUES(A, D) do { if (G == 1) HEADS(A, 1, D); \

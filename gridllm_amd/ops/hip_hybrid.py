@@ -653,10 +653,15 @@ def _talk_sizes(tk: Talk, g: int, p: int) -> tuple[bool, bool]:
     return one, one and nh <= 4 and nh * p <= 512
 
 
-def _talk_splits(rows: int, heads: int, seen: int) -> int:
-    """Into how many parts a decode row's keys are split. (A part's sums are as
-    large as the values of 2 * heads keys.)"""
-    return max(1, min(256 // rows, -(-seen // max(128, 8 * heads)), 32))
+def _talk_blocks(rows: int, g: int, p: int, seen: int) -> int:
+    """Blocks that a step's rows are cut into parts for, by the lengths that the
+    kernel finds; 0: each row is a block's, which fill the chip or have little to
+    cut. (A block's LDS is two tiles of 32 keys' values, so that a CU has one
+    block, or two where values are small.)"""
+    if rows > 224 or seen <= 64:
+        return 0
+    tiles = rows * (-(-seen // 32) + 1)
+    return min(256 if g * p > 256 else 512, -(-tiles // 2))
 
 
 def talk_attn(q: torch.Tensor, vc: torch.Tensor, inv: torch.Tensor,
@@ -680,12 +685,12 @@ def talk_attn(q: torch.Tensor, vc: torch.Tensor, inv: torch.Tensor,
     portions = st.talk.get(tk.chunk) if tiled else None
     na = n if portions is None else st.absorbed
     if na:
-        nsplit = _talk_splits(na, h, min(st.max_len, tk.chunk))
-        ws = torch.empty(na * nsplit * (g * h * p + h), dtype=torch.float32,
-                         device=dev) if nsplit > 1 else None
+        blocks = _talk_blocks(na, g, p, min(st.max_len, tk.chunk))
+        ws = torch.empty(blocks * (g * h * p + h) + 2 * na,
+                         dtype=torch.float32, device=dev) if blocks else None
         _call("gt_talk_decode", out, q, vc, inv, st.table, per, st.pos,
               st.slot, ws, tk.knorm, tk.talk, *tk.rot, nrot, na, h, g, p, r,
-              tk.chunk, nsplit, *cap)
+              tk.chunk, blocks, *cap)
     if portions is not None:
         kx = torch.empty(2, portions.pages, g, PAGE * p, dtype=q.dtype,
                          device=dev)

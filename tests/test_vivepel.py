@@ -326,6 +326,46 @@ def test_rotation_far_out(run):
         (2e-5 if run[1] == "fp32" else 0.03)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 7, 60, 224])
+@pytest.mark.parametrize("sizes", [(24, 8, 128, 4096, 64), (9, 3, 20, 70, 6),
+                                   (40, 1, 64, 333, 64)])
+def test_decode_in_parts(n, sizes, monkeypatch):
+    """Rows in parts, as many as there are blocks for, against blocks of one row
+    each and against the exact mode."""
+    from gridllm_amd.ops import hip_hybrid
+    heads, groups, dim, chunk, rot = sizes
+    cfg = config((attn(heads, groups, dim, chunk, rot, 1e4, dim ** -0.5, 30.0),
+                  None))
+    m = build(cfg, ("cuda", "bf16"), slots=3, max_seq=900)
+    c, tk = m.cache, m.layers[0].talk
+    g = torch.Generator().manual_seed(n)
+    for slot in [c.alloc(900) for _ in range(3)]:
+        c.extend([slot], [900])
+    c.v[0].copy_(torch.randn(c.v[0].shape, generator=g))
+    c.inv[0].copy_(torch.rand(c.inv[0].shape, generator=g) + 0.5)
+    pos = torch.randint(0, 900, (n,), generator=g)
+    edges = torch.tensor([899, 0, 31, 32, 63, 64, 332, 333])[:n]
+    pos[torch.randperm(n, generator=g)[:len(edges)]] = edges
+    st = hops.StepMeta(nd=n, pos=pos.to("cuda", torch.int32),
+                       slot=torch.randint(0, 3, (n,), generator=g).to(
+                           "cuda", torch.int32),
+                       table=c.table, max_len=900)
+    st.absorbed = n
+    p = c.v[0].shape[-1]
+    q = torch.randn(n, heads, p, generator=g).to("cuda", torch.bfloat16)
+    got = hops.talk_attn(q, c.v[0], c.inv[0], st, tk)
+    assert hip_hybrid._talk_blocks(n, groups, p, min(900, chunk)) > 0
+    exact = hops.talk_attn(q.float(), c.v[0].float(), c.inv[0], st, tk)
+    monkeypatch.setattr(hip_hybrid, "_talk_blocks", lambda *a: 0)
+    alone = hops.talk_attn(q, c.v[0], c.inv[0], st, tk)
+    # the same products, added up in f32 in another order: one rounding apart
+    d = (got.float() - alone.float()).abs()
+    assert bool((d <= 2 ** -7 * alone.float().abs() + 1e-4).all())
+    assert float((got.float() - exact).abs().max()) < \
+        0.05 + 0.01 * math.sqrt(heads)
+
+
 # ----------------------------------------------- cuts, batches, pages, slots
 
 @pytest.mark.parametrize("run", RUNS)
