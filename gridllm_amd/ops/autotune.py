@@ -1,11 +1,11 @@
 """Per-shape GEMM dispatch autotuner.
 
 For each decode projection shape (M, N, K) the engine will hit, measure
-hipBLASLt (torch F.linear) against the in-house skinny GEMM at several
-split-K choices, and cache the winner. ops.linear() then dispatches through
-the table — never slower than the library, faster where the hand-written
-weight-streaming kernel wins. (PyTorch TunableOp only tunes WITHIN
-hipBLASLt; measured +2% on these shapes — profiles/r01_decode_profile.md.)
+hipBLASLt (torch F.linear) against the in-house GEMMs at several tilings, and
+cache the winner. ops.linear() then dispatches through the table — never slower
+than the library, faster where a hand-written kernel wins; shapes that were not
+timed go by rule. (PyTorch TunableOp only tunes WITHIN hipBLASLt; measured +2%
+on these shapes — profiles/r01_decode_profile.md.)
 """
 
 from __future__ import annotations
@@ -22,165 +22,132 @@ from gridllm_amd.utils.logging import get_logger
 
 log = get_logger("autotune")
 
-# (m, n, k) -> ("blas", 0) | ("ours", splitk)
-_CHOICE: dict[tuple[int, int, int], tuple[str, int]] = {}
+# (m, n, k) -> ("blas",) | ("rows",) | ("ours", splitk) |
+# ("tile", rows, cols, splitk)
+_CHOICE: dict[tuple[int, int, int], tuple] = {}
 # gate/up projection with fused SwiGLU (n = 2F interleaved rows):
-# (m, n, k) -> ("blas", 0) | ("proj", splitk)
-_CHOICE_GU: dict[tuple[int, int, int], tuple[str, int]] = {}
+# (m, n, k) -> ("blas",) | ("rows",) | ("tile", rows, cols, splitk)
+_CHOICE_GU: dict[tuple[int, int, int], tuple] = {}
+_ITERS = 24                     # calls of a timing
 _SPLITK_CANDIDATES = (0, 2, 4, 6, 8, 12, 16, 24, 32)
 
 
-def _time_fn(fn, ws, iters: int = 24) -> float:
+def _weights(n: int, k: int, device) -> list[torch.Tensor]:
+    """Copies of a weight, so that each call of a timing (or, where two of them
+    are more than the Infinity Cache holds, each other one) reads its own."""
+    copies = min(_ITERS, max(2, (640 << 20) // max(1, n * k * 2)))
+    w = torch.randn(n, k, device=device).to(torch.bfloat16) * 0.1
+    return [w] + [w.clone() for _ in range(copies - 1)]
+
+
+def _time_fn(fn, ws) -> float:
     """Time fn(w) cycling over weight copies so W streams from HBM, not the
     256 MB Infinity Cache — an L3-warm measurement picks kernels that lose
-    in-situ (decode reads 6+ GB of weights per step; nothing stays in L3)."""
-    for i in range(4):
-        fn(ws[i % len(ws)])
+    in-situ (decode reads 6+ GB of weights per step; nothing stays in L3). The
+    calls are captured, as a decode step is: launched one by one from here, a
+    kernel of less than 10 us takes as long as its launch."""
+    fn(ws[0])
+    flush = torch.empty(512 << 20, dtype=torch.uint8, device=ws[0].device)
     torch.cuda.synchronize()
-    t0 = time.monotonic()
-    for i in range(iters):
-        fn(ws[i % len(ws)])
-    torch.cuda.synchronize()
-    return (time.monotonic() - t0) / iters
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for i in range(_ITERS):
+            fn(ws[i % len(ws)])
+    best = float("inf")
+    for _ in range(3):
+        flush.fill_(1)
+        torch.cuda.synchronize()
+        t0 = time.monotonic()
+        graph.replay()
+        torch.cuda.synchronize()
+        best = min(best, time.monotonic() - t0)
+    return best / _ITERS
 
 
-def tune_shape(m: int, n: int, k: int, device) -> tuple[str, int]:
-    key = (m, n, k)
-    if key in _CHOICE:
-        return _CHOICE[key]
-    x = torch.randn(m, k, device=device).to(torch.bfloat16) * 0.1
-    wbytes = n * k * 2
-    ncopies = min(6, max(2, (320 << 20) // max(1, wbytes)))
-    ws = [torch.randn(n, k, device=device).to(torch.bfloat16) * 0.1
-          for _ in range(ncopies)]
-    best = ("blas", 0)
-    t_best = _time_fn(lambda w: F.linear(x, w), ws)
-    if hip_ops.gemm_skinny_supported(m, n, k):
-        seen = set()
-        for sk in _SPLITK_CANDIDATES:
-            if sk > max(1, k // 256):
-                continue
-            if sk in seen:
-                continue
-            seen.add(sk)
-            try:
-                t = _time_fn(lambda w: hip_ops.gemm_skinny(x, w, splitk=sk), ws)
-            except RuntimeError:
-                continue
-            if t < t_best * 0.97:           # require a real margin
-                t_best = t
-                best = ("ours", sk)
-    if hip_ops.gemm_proj_supported(m, n, k):
-        # latency-bound regime: (N/64)*splitk ~ 0.5-1x the 256 CUs
-        rule = max(1, min(k // 256, 256 // max(1, n // 64)))
-        for sk in sorted({1, rule, rule * 2, max(1, rule // 2)}):
-            if sk > max(1, k // 64):
-                continue
-            try:
-                t = _time_fn(lambda w: hip_ops.gemm_proj(x, w, splitk=sk), ws)
-            except RuntimeError:
-                continue
-            if t < t_best * 0.97:
-                t_best = t
-                best = ("proj", sk)
-    if 64 < m <= 2048 and n % 128 == 0 and k % 64 == 0:
-        # m-tiled decomposition (grid.y m-tiles, W slice re-read from XCD
-        # L2): candidate mtiles keep 64..256 rows per tile; splitk
-        # composes when the grid is still thin. Covers serving buckets
-        # ABOVE the plain-proj 512 cap too (768/1024 fell back to
-        # hipBLASLt at 0.7-1.6 TB/s — r02j b768 trace).
-        for mt in (2, 3, 4, 6, 8, 12, 16):
-            rpt = (m + mt - 1) // mt
-            if rpt > 256 or (rpt < 64 and not (mt == 2 and m > 64)):
-                continue
-            rule = max(1, min(k // 256,
-                              256 // max(1, (n // 128) * mt)))
-            for sk in sorted({1, rule}):
-                try:
-                    t = _time_fn(lambda w: hip_ops.gemm_proj(
-                        x, w, splitk=sk, mtiles=mt), ws)
-                except RuntimeError:
-                    continue
-                if t < t_best * 0.97:
-                    t_best = t
-                    best = ("projm", sk, mt)
-    if hip_ops.gemm_proj_wide_supported(m, n, k):
-        rule = max(1, min(k // 256, 256 // max(1, n // 256)))
-        for sk in sorted({1, rule, rule * 2}):
-            if sk > max(1, k // 64):
-                continue
-            try:
-                t = _time_fn(lambda w: hip_ops.gemm_proj_wide(x, w, splitk=sk),
-                             ws)
-            except RuntimeError:
-                continue
-            if t < t_best * 0.97:
-                t_best = t
-                best = ("projw", sk)
-    del ws
-    _CHOICE[key] = best
+def _run(c: tuple, x: torch.Tensor, w: torch.Tensor,
+         glu: Optional[Glu] = None) -> torch.Tensor:
+    """x @ w.T by a choice; with glu, of an interleaved gate/up weight and its
+    gated unit."""
+    fuse = glu is not None
+    unit = glu or SWIGLU
+    if c[0] == "rows":
+        return hip_ops.gemm_rows(x, w, fuse_swiglu=fuse, glu=unit)
+    if c[0] == "tile":
+        return hip_ops.gemm_tile(x, w, *c[1:], fuse_swiglu=fuse, glu=unit)
+    if c[0] == "ours":
+        return hip_ops.gemm_skinny(x, w, splitk=c[1])
+    out = F.linear(x, w)
+    return hip_ops.swiglu_il(out, glu=unit) if fuse else out
+
+
+def _by_rule(x: torch.Tensor, w: torch.Tensor, fuse: bool = False) -> tuple:
+    """The choice for a shape that was not timed. gemm_rows has no second kernel,
+    but every block reads all of x: it is the faster one for w of up to 20 MB
+    with up to 4 rows and up to 14 MB with 16 (against gemm_tile: 3072 x 2048, 16
+    rows: 7.2 us, 7.4; 3072 x 3072: one row 7.2, 7.9, 16 rows 9.8, 8.0; 5120 x
+    3072, one row 10.8, 10.0; gate/up 16384 x 3072, one row: 21.7, 19.8)."""
+    m, size = x.shape[0], w.numel()
+    if m <= 16 and hip_ops.gemm_rows_supported(x, w, fuse):
+        if size <= (10_000_000 if m <= 4 else 7_000_000):
+            return ("rows",)
+    if m <= 256 and x.is_contiguous() and w.is_contiguous() and \
+            w.dtype == torch.bfloat16 and \
+            (x.data_ptr() | w.data_ptr()) % 16 == 0:
+        tiling = hip_ops.gemm_tiling(m, *w.shape, fuse)
+        if tiling is not None:
+            return ("tile", *tiling)
+    if m <= 4 and hip_ops.gemm_rows_supported(x, w, fuse):
+        return ("rows",)
+    return ("blas",)
+
+
+def _tune(x: torch.Tensor, n: int, glu: Optional[Glu] = None) -> tuple:
+    """The fastest for x and a weight of n rows."""
+    m, k = x.shape
+    ws = _weights(n, k, x.device)
+    best: tuple = ("blas",)
+    t_best = _time_fn(lambda w: _run(best, x, w, glu), ws)
+    tried: list[tuple] = [("tile", *t) for t in hip_ops.gemm_tilings(
+        m, n, k, glu is not None)]
+    if hip_ops.gemm_rows_supported(x, ws[0], glu is not None):
+        tried.append(("rows",))
+    if not tried and glu is None and hip_ops.gemm_skinny_supported(m, n, k):
+        tried = [("ours", sk) for sk in _SPLITK_CANDIDATES
+                 if sk <= max(1, k // 256)]
+    for c in tried:
+        t = _time_fn(lambda w: _run(c, x, w, glu), ws)
+        if t < t_best * 0.97:               # require a real margin
+            t_best = t
+            best = c
     return best
 
 
-def tune_gateup(m: int, n: int, k: int, device) -> tuple[str, int]:
+def tune_shape(m: int, n: int, k: int, device) -> tuple:
+    key = (m, n, k)
+    if key not in _CHOICE:
+        x = torch.randn(m, k, device=device).to(torch.bfloat16) * 0.1
+        _CHOICE[key] = _tune(x, n)
+    return _CHOICE[key]
+
+
+def tune_gateup(m: int, n: int, k: int, device) -> tuple:
     """Tune the interleaved gate/up projection (n = 2F rows): library GEMM
-    + interleaved-SwiGLU pass vs the fused-epilogue projection kernel."""
+    + interleaved-SwiGLU pass vs the fused-epilogue kernels."""
     key = (m, n, k)
-    if key in _CHOICE_GU:
-        return _CHOICE_GU[key]
-    x = torch.randn(m, k, device=device).to(torch.bfloat16) * 0.1
-    wbytes = n * k * 2
-    ncopies = min(6, max(2, (320 << 20) // max(1, wbytes)))
-    ws = [torch.randn(n, k, device=device).to(torch.bfloat16) * 0.1
-          for _ in range(ncopies)]
-    best = ("blas", 0)
-    t_best = _time_fn(lambda w: hip_ops.swiglu_il(F.linear(x, w)), ws)
-    if m <= 2048 and n % 128 == 0 and k % 64 == 0:
-        rule = max(1, min(k // 256, 256 // max(1, n // 128)))
-        for sk in sorted({1, rule, rule * 2, max(1, rule // 2)}):
-            if sk > max(1, k // 64):
-                continue
-            try:
-                t = _time_fn(lambda w: hip_ops.gemm_proj(
-                    x, w, splitk=sk, fuse_swiglu=True), ws)
-            except RuntimeError:
-                continue
-            if t < t_best * 0.97:
-                t_best = t
-                best = ("proj", sk)
-        for mt in (2, 3, 4, 6, 8, 12, 16):   # m-tiled + fused epilogue
-            rpt = (m + mt - 1) // mt
-            if rpt > 256 or (rpt < 64 and not (mt == 2 and m > 64)):
-                continue
-            try:
-                t = _time_fn(lambda w: hip_ops.gemm_proj(
-                    x, w, splitk=1, fuse_swiglu=True, mtiles=mt), ws)
-            except RuntimeError:
-                continue
-            if t < t_best * 0.97:
-                t_best = t
-                best = ("projm", 1, mt)
-    del ws
-    _CHOICE_GU[key] = best
-    return best
+    if key not in _CHOICE_GU:
+        x = torch.randn(m, k, device=device).to(torch.bfloat16) * 0.1
+        _CHOICE_GU[key] = _tune(x, n, SWIGLU)
+    return _CHOICE_GU[key]
 
 
 def linear_gateup(x: torch.Tensor, w_il: torch.Tensor,
                   glu: Glu = SWIGLU) -> torch.Tensor:
     """Fused gate/up projection + gated linear unit on an INTERLEAVED weight:
-    returns [M, F] activated. Few rows go to gemm_rows, others through the
-    tuned table."""
-    if x.dim() == 2 and x.shape[0] <= 16 and \
-            hip_ops.gemm_rows_wanted(x, w_il, fuse_swiglu=True):
-        return hip_ops.gemm_rows(x, w_il, fuse_swiglu=True, glu=glu)
+    returns [M, F] activated, through the tuned table or by rule."""
     c = _CHOICE_GU.get((x.shape[0], w_il.shape[0], w_il.shape[1]))
-    if c is not None and c[0] == "proj":
-        return hip_ops.gemm_proj(x, w_il, splitk=c[1], fuse_swiglu=True,
-                                 glu=glu)
-    if c is not None and c[0] == "projm":
-        return hip_ops.gemm_proj(x, w_il, splitk=c[1], fuse_swiglu=True,
-                                 mtiles=c[2], glu=glu)
-    return hip_ops.swiglu_il(F.linear(x, w_il), glu=glu)
+    if c is None:
+        c = _by_rule(x, w_il, True) if x.dim() == 2 else ("blas",)
+    return _run(c, x, w_il, glu)
 
 
 def choice(m: int, n: int, k: int) -> Optional[tuple[str, int]]:
@@ -188,23 +155,15 @@ def choice(m: int, n: int, k: int) -> Optional[tuple[str, int]]:
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """Dispatch x @ w.T (GPU bf16 2-D x only): few rows to gemm_rows, others
-    through the tuned table."""
+    """Dispatch x @ w.T (GPU bf16 2-D x only) through the tuned table or by
+    rule."""
     if x.dim() == 2 and x.is_cuda and x.dtype == torch.bfloat16:
-        if x.shape[0] <= 16 and hip_ops.gemm_rows_wanted(x, w) and not (
-                torch.is_grad_enabled()
-                and (x.requires_grad or w.requires_grad)):
-            return hip_ops.gemm_rows(x, w)
         c = _CHOICE.get((x.shape[0], w.shape[0], w.shape[1]))
+        if c is None and not (torch.is_grad_enabled() and
+                              (x.requires_grad or w.requires_grad)):
+            c = _by_rule(x, w)
         if c is not None:
-            if c[0] == "ours":
-                return hip_ops.gemm_skinny(x, w, splitk=c[1])
-            if c[0] == "proj":
-                return hip_ops.gemm_proj(x, w, splitk=c[1])
-            if c[0] == "projm":
-                return hip_ops.gemm_proj(x, w, splitk=c[1], mtiles=c[2])
-            if c[0] == "projw":
-                return hip_ops.gemm_proj_wide(x, w, splitk=c[1])
+            return _run(c, x, w)
     return F.linear(x, w)
 
 
@@ -221,6 +180,6 @@ def tune_model_shapes(model, buckets) -> None:
                 tune_gateup(m, n, k, model.device)
             else:
                 tune_shape(m, n, k, model.device)
-    picked = sum(1 for v in _CHOICE.values() if v[0] == "ours")
+    picked = sum(1 for v in _CHOICE.values() if v[0] != "blas")
     log.performance("gemm autotune done", shapes=len(_CHOICE),
                     ours=picked, ms=int((time.monotonic() - t0) * 1000))

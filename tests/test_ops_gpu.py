@@ -575,6 +575,62 @@ def test_prefill_batch_engine_parity(dev):
         assert dk < 1.6e-2, (i, dk)
 
 
+@pytest.mark.parametrize("fuse", [False, True])
+@pytest.mark.parametrize("m,n,k,sk", [
+    (17, 384, 64, 1),          # one tile of K
+    (33, 384, 512, 1),         # as many as buffers, or one more or less
+    (1, 128, 576, 3),          # parts of fewer tiles than buffers
+    (95, 1152, 896, 4),        # the last part shorter
+    (160, 2176, 1088, 1),      # a number of blocks that 8 does not divide
+    (161, 640, 3072, 5), (257, 256, 1024, 2), (700, 384, 640, 1),
+])
+def test_gemm_tile(dev, m, n, k, sk, fuse):
+    """Every tile size against f32, at edges of rows, of K's parts and of the
+    ring of tiles in LDS."""
+    from gridllm_amd.ops import hip_ops
+    n = n // 128 * 128 if fuse else n
+    g = torch.Generator().manual_seed(m + k)
+    x = torch.randn(m, k, generator=g).to(dev, torch.bfloat16)
+    w = torch.randn(n, k, generator=g).to(dev, torch.bfloat16)
+    ref = x.float() @ w.float().t()
+    # bf16 result: 2^-9 of its size; K products' sums: k eps of their sizes' sum
+    tol = 2 ** -8 * ref.abs() + k * 2 ** -24 * (x.float().abs() @
+                                                w.float().abs().t()) + 1e-6
+    if fuse:
+        gate, up = ref.view(m, -1, 2, 64).unbind(2)
+        ref = (gate * torch.sigmoid(gate) * up).reshape(m, -1)
+        # (the unit's exponential is the hardware's)
+        gt, ut = tol.view(m, -1, 2, 64).unbind(2)
+        tol = (2 ** -8 * (gate * up).abs() + 1.2 * gt * up.abs() +
+               gate.abs() * ut).reshape(m, -1) + 1e-4
+    out = torch.empty_like(ref, dtype=torch.bfloat16)
+    for rows in (32, 64, 96, 128, 160, 192, 256):
+        for cols in (64, 128) if fuse else (64, 96, 128):
+            if n % cols == 0:
+                hip_ops.gemm_tile(x, w, rows, cols, sk, out.fill_(9e9), fuse)
+                assert bool(((out.float() - ref).abs() <= tol).all()), \
+                    (rows, cols)
+
+
+def test_gemm_tilings():
+    """What the tuner tries is what the kernel takes."""
+    from gridllm_amd.ops import hip_ops
+    for m in (1, 16, 17, 64, 129, 160, 256, 300, 1024, 2048):
+        for n, k in ((64, 64), (192, 896), (3072, 8192), (128256, 3072),
+                     (100, 64), (128, 96)):
+            for fuse in (False, True):
+                for rows, cols, sk in hip_ops.gemm_tilings(m, n, k, fuse):
+                    assert n % cols == 0 and k % 64 == 0 and sk >= 1
+                    assert rows in (32, 64, 96, 128, 160, 192, 256)
+                    assert sk == 1 or (sk * -(-m // rows) * n // cols <= 256
+                                       and k // sk >= 64)
+                rule = hip_ops.gemm_tiling(m, n, k, fuse)
+                assert rule is None or (rule[0] in (
+                    32, 64, 96, 128, 160, 192, 256) and n % rule[1] == 0
+                    and k % 64 == 0 and k // rule[2] >= 64)
+                assert not (rule and fuse and (n % 128 or rule[1] == 96))
+
+
 @pytest.mark.parametrize("m,n,k,mt,sk", [
     (256, 5120, 3072, 2, 1),   # qkv m-tiled
     (256, 5120, 3072, 2, 3),   # + splitk compose
