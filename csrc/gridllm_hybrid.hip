@@ -1416,23 +1416,31 @@ k_mlstm_chunk_out(float* __restrict__ o, const float* __restrict__ dS,
 // without the normaliser row.
 // ===========================================================================
 
-// b of one chunk for 256 channels: z = W2 u + bias with w = W2^T, f32 [R][C].
-// The first items are U each of the first nd tokens, chunks of their own; then
-// come the chunks ({first token, length, ..}).
+// b of one chunk for 64 channels: z = W2 u + bias with w = W2^T, f32 [R][C]. A
+// wave has U tokens, whose sums meet in LDS. The first items are 4 U each of the
+// first nd tokens, chunks of their own; then come the chunks ({first token,
+// length, ..}). Bound by the logarithms and their latency: with one thread for
+// a channel's 64 tokens (3050 tokens, 1536 channels: 1.2 waves a SIMD) it took 45
+// us, so 31.
 template <int U>
 __global__ void __launch_bounds__(256)
 k_gla_decay(float* __restrict__ b, const float* __restrict__ u,
             const float* __restrict__ w, const float* __restrict__ bias,
             const int4* __restrict__ chunks, int nd, int R, int C,
             float inv_tau) {
-    const int it = blockIdx.x, singles = (nd + U - 1) / U;
-    int4 ch = make_int4(it * U, min(U, nd - it * U), 0, 0);
-    if (it >= singles) ch = chunks[it - singles];
-    const int c = blockIdx.y * 256 + threadIdx.x;
-    if (c >= C) return;
+    __shared__ float sums[4][64];
+    const int it = blockIdx.x, singles = (nd + 4 * U - 1) / (4 * U);
+    const bool single = it < singles;
+    int4 ch = make_int4(it * 4 * U, min(4 * U, nd - it * 4 * U), 0, 0);
+    if (!single) ch = chunks[it - singles];
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = min((int)blockIdx.y * 64 + lane, C - 1);
+    const bool own = (int)blockIdx.y * 64 + lane < C;
     const float b0 = bias[c];
-    float sum = 0.f;
-    for (int t0 = 0; t0 < ch.y; t0 += U) {
+    float ahead = 0.f;                 // of the steps of 4 U tokens before
+    for (int s0 = 0; s0 < ch.y; s0 += 4 * U) {
+        const int t0 = s0 + wid * U;
         float z[U];
         const float* ur[U];
 #pragma unroll
@@ -1451,14 +1459,31 @@ k_gla_decay(float* __restrict__ b, const float* __restrict__ u,
 #pragma unroll
                     for (int i = 0; i < U; ++i) z[i] += ur[i][rb + k] * wv[k];
         }
+        float sum = 0.f;
 #pragma unroll
         for (int i = 0; i < U; ++i) {
-            if (t0 + i >= ch.y) break;
             const float la =
                 (fminf(z[i], 0.f) - log1pf(expf(-fabsf(z[i])))) * inv_tau;
-            sum = it < singles ? la : sum + la;
-            b[(long)(ch.x + t0 + i) * C + c] = sum;
+            sum = single || t0 + i >= ch.y ? la : sum + la;
+            z[i] = sum;
         }
+        if (!single) {
+            sums[wid][lane] = sum;
+            __syncthreads();
+            float all = ahead;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                if (v == wid) ahead = all;
+                all += sums[v][lane];
+            }
+#pragma unroll
+            for (int i = 0; i < U; ++i) z[i] += ahead;
+            ahead = all;
+            __syncthreads();
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+            if (own && t0 + i < ch.y) b[(long)(ch.x + t0 + i) * C + c] = z[i];
     }
 }
 
@@ -1610,32 +1635,186 @@ DEV_INLINE f32x4 mfma_split(bf16x8 ah, bf16x8 al, bf16x8 bh, bf16x8 bl,
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, c, 0, 0, 0);
 }
 
-// Block = (chunk, head, every gridDim.z-th 128 value columns); wave w owns
-// tokens 16 w .. 16 w + 15. Scores refer to b at the end of the 16 tokens
-// before: queries then decay by exp(b_t - ref) and older keys by
-// exp(ref - b_s), both at most 1. Keys of the same 16 tokens grow by
-// exp(ref - b_s) instead, unless a channel loses so much in 16 tokens that
-// this could overflow; then these scores are taken pair by pair.
+// Places in LDS of 16-byte pieces c, swapped by the row so that 16 lanes' rows
+// do not meet in a bank: of 64 f32, of 64 bf16, and of `cols` bf16 that are read
+// transposed, where 4 rows' pairs of pieces have to lie apart.
+DEV_INLINE int at_f32(int row, int c) { return row * 64 + (c ^ (row & 15)) * 4; }
+DEV_INLINE int at_bf16(int row, int c) { return row * 64 + (c ^ (row & 7)) * 8; }
+DEV_INLINE int at_cols(int row, int c, int cols) {
+    return row * cols + (c ^ ((row & 3) << 1 | (row >> 2 & 1))) * 8;
+}
+
+// 64 tokens' values, up to 256 columns of them, on their way to LDS
+DEV_INLINE void load_values(bf16_t* vs, const bf16_t* v, long ld_, int last,
+                            int cols) {
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int i = 0; i < cols / 32; ++i) {
+        const int pc = i * 256 + threadIdx.x, row = pc / (cols / 8);
+        const int c = at_cols(row, pc % (cols / 8), cols) / 8 -
+                      row * (cols / 8);
+        load_lds16(v + min(row, last) * ld_ + c * 8,
+                   vs + (i * 256 + wid * 64) * 8);
+    }
+}
+
+// Values (16 columns from `col` on, as the products' rows) of 32 tokens.
+DEV_INLINE bf16x8 value_piece(const bf16_t* vs, int ks, int col, int cols) {
+    const int lane = threadIdx.x & 63, fr = lane & 15, gq = lane >> 4;
+    const int d = col + (fr & 3) * 4;
+    bf16x8 v;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int row = ks * 32 + gq * 8 + (fr >> 2) + j * 4;
+        const bf16x4 x =
+            read_transposed(vs + at_cols(row, d >> 3, cols) + (d & 7));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[j * 4 + i] = x[i];
+    }
+    return v;
+}
+
+// Output gates of a chunk, for lane = 4 columns c * 64 + wid * 16 + gq * 4 + r of
+// tokens rt * 16 + fr: on their way ahead of the last products.
+DEV_INLINE void load_gates(uint2 (&z)[4][4], const bf16_t* gate, long ld_,
+                           int last, int DV) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (c * 64 < DV)
+                z[c][rt] = *(const uint2*)(
+                    gate + min(rt * 16 + (lane & 15), last) * ld_ + c * 64 +
+                    wid * 16 + (lane >> 4) * 4);
+}
+
+// A chunk's outputs, laid out as its gates, with all of the head's columns in the
+// block: unit RMS, times norm, times the gate's sigmoid (SILU: and the gate).
+// red: f32 [4][64] in LDS.
+template <bool SILU>
+DEV_INLINE void store_normed(bf16_t* out, const f32x4 (&acc)[4][4],
+                             float* red, const uint2 (&gates)[4][4],
+                             long out_ld, const float* norm, int len, int DV,
+                             int dvtrue, float eps) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int fr = lane & 15, gq = lane >> 4, col0 = wid * 16 + gq * 4;
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+        float ss = 0.f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (c * 64 < DV)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) ss += acc[c][rt][r] * acc[c][rt][r];
+        ss += __shfl_xor(ss, 16, WAVE);
+        ss += __shfl_xor(ss, 32, WAVE);
+        if (gq == 0) red[wid * 64 + rt * 16 + fr] = ss;
+    }
+    float w[4][4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        if (c * 64 < DV) ld4(norm + c * 64 + col0, w[c]);
+    __syncthreads();
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+        const int t = rt * 16 + fr;
+        const float ss = red[t] + red[64 + t] + red[128 + t] + red[192 + t];
+        const float rs = 1.f / sqrtf(ss / (float)dvtrue + eps);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (c * 64 >= DV) continue;
+            float z[4];
+            ld4((const bf16_t*)&gates[c][rt], z);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                z[r] = acc[c][rt][r] * rs * w[c][r] *
+                       __builtin_amdgcn_rcpf(1.f + __expf(-z[r])) *
+                       (SILU ? z[r] : 1.f);
+            if (t < len) st4(out + t * out_ld + c * 64 + col0, z);
+        }
+    }
+}
+
+// Block = (chunk, head, 256 value columns). Scores: wave w owns tokens 16 w ..
+// 16 w + 15. They refer to b at the end of the 16 tokens before: queries then
+// decay by exp(b_t - ref) and older keys by exp(ref - b_s), both at most 1. Keys
+// of the same 16 tokens grow by exp(ref - b_s) instead, unless a channel loses
+// so much in 16 tokens that this could overflow; then these scores are taken
+// pair by pair. Outputs: a wave owns every fourth 16 columns for all 64 tokens,
+// so that the state is read once; decayed queries and scores meet in LDS. With
+// all of a head's columns here (out), the head's norm and gate follow at once.
+// Bound by reading the state (128 KB a head and chunk of 128 x 256) and the
+// latencies between its few steps. 590 blocks of it: 78 us with tokens split
+// over the waves, each reading the whole state, and 22 of the norm behind it;
+// now 61, of which the gates take 18 and the scores' decays 11. (The gate's
+// sigmoid is the hardware's, 1e-6, ahead of a bf16 result.)
 #define GLA_SPAN 60.f
 __global__ void __launch_bounds__(256, 2)
-k_gla_chunk_out(float* __restrict__ o, const float* __restrict__ dS,
-                const bf16_t* __restrict__ qkv, const float* __restrict__ b,
-                const int4* __restrict__ chunks, int H, int DK, int DV,
-                int ld_, float qscale) {
-    __shared__ __attribute__((aligned(16))) bf16_t vt[128 * MLD];
-    __shared__ __attribute__((aligned(16))) bf16_t ph[64 * MLD];
-    __shared__ __attribute__((aligned(16))) bf16_t pl[64 * MLD];
+k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
+                const float* __restrict__ dS, const bf16_t* __restrict__ qkv,
+                const float* __restrict__ b, const int4* __restrict__ chunks,
+                const float* __restrict__ norm, int H, int DK, int DV,
+                int ld_, float qscale, int dvtrue, float eps) {
+    __shared__ __attribute__((aligned(16))) bf16_t vs[64 * 256];
+    __shared__ __attribute__((aligned(16))) float bs[64 * 64];
+    __shared__ __attribute__((aligned(16))) bf16_t ks_[64 * 64];
+    __shared__ __attribute__((aligned(16))) bf16_t qs[2][64 * 64];
     const int4 ch = chunks[blockIdx.x];
-    const int h = blockIdx.y;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int fr = lane & 15, kg = (lane >> 4) * 8, r0 = wid * 16;
+    const int h = blockIdx.y, v0 = blockIdx.z * 256, nv = min(256, DV - v0);
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int fr = lane & 15, gq = lane >> 4, kg = gq * 8, r0 = wid * 16;
     const long C = (long)H * DK;
     const int last = ch.y - 1;
     const float* bh = b + (long)ch.x * C + h * DK;     // row t at t * C
     const bf16_t* qh = qkv + (long)ch.x * ld_ + h * DK;
     const bf16_t* kh = qh + C;
-    const int tq = min(r0 + fr, last);
-    const float* ref = r0 ? bh + min(r0 - 1, last) * C : nullptr;
+    const int tq = min(r0 + fr, last), tr = min(r0 - 1, last);
+    const float* ref = r0 ? bh + tr * C : nullptr;
+    const u32* Sb = (const u32*)dS + ((long)blockIdx.x * H + h) * DV * DK +
+                    (long)(v0 + wid * 16 + fr) * DK + kg;
+
+    auto issue = [&](int k0) {         // b and keys of 64 channels
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int pc = i * 256 + threadIdx.x, row = pc >> 4;
+            load_lds16((const bf16_t*)(bh + min(row, last) * C + k0 +
+                                       ((pc & 15) ^ (row & 15)) * 4),
+                       (bf16_t*)(bs + (i * 256 + wid * 64) * 4));
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int pc = i * 256 + threadIdx.x, row = pc >> 3;
+            load_lds16(kh + (long)min(row, last) * ld_ + k0 +
+                           ((pc & 7) ^ (row & 7)) * 8,
+                       ks_ + (i * 256 + wid * 64) * 8);
+        }
+    };
+    uint4 st[2][4][2], qown[2], qall[2];
+    const int tall = threadIdx.x >> 2;
+    auto load_state = [&](int k0, int ks, int c) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            st[ks][c][i] = *(const uint4*)(Sb + (long)c * 64 * DK + k0 +
+                                           ks * 32 + i * 4);
+    };
+    auto load_queries = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            qown[i] = *(const uint4*)(qh + (long)tq * ld_ + k0 + i * 32 + kg);
+            qall[i] = *(const uint4*)(qh + (long)min(tall, last) * ld_ + k0 +
+                                      (threadIdx.x & 3) * 16 + i * 8);
+        }
+    };
+    issue(0);
+    load_queries(0);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (c * 64 < nv) load_state(0, ks, c);
+    load_values(vs, qkv + (long)ch.x * ld_ + 2 * C + h * DV + v0, ld_, last,
+                nv);
 
     // ---- does a channel lose too much within these 16 tokens?
     float span = 0.f;
@@ -1644,32 +1823,84 @@ k_gla_chunk_out(float* __restrict__ o, const float* __restrict__ dS,
                                bh[min(r0 + 15, last) * C + c]);
     const bool pairwise = wave_reduce_max(span) > GLA_SPAN;
 
-    // ---- scores
-    f32x4 sc[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) sc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    // scores, and what the entering state gives
     const int jmax = pairwise ? wid - 1 : wid;
-    for (int k0 = 0; k0 < DK; k0 += 32) {
-        const int c = k0 + kg;
-        float rf[8], e[8];
+    f32x4 sc[4], acc[4][4];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) rf[i] = 0.f;
-        if (ref) ld8(ref + c, rf);
-        ld8(bh + tq * C + c, e);
+    for (int j = 0; j < 4; ++j) {
+        sc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 8; ++i) e[i] -= rf[i];
-        bf16x8 ah, al;
-        decayed8(qh + (long)tq * ld_ + c, e, ah, al);
+        for (int c = 0; c < 4; ++c) acc[j][c] = sc[j];
+    }
+    for (int k0 = 0; k0 < DK; k0 += 64) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        lds_barrier();
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (j > jmax) continue;
-            const int s = min(j * 16 + fr, last);
-            ld8(bh + s * C + c, e);
+        for (int i = 0; i < 2; ++i) {              // queries for the state
+            const int c = (threadIdx.x & 3) * 2 + i;
+            float e[8];
+            ld4(bs + at_f32(tall, c * 2), e);
+            ld4(bs + at_f32(tall, c * 2 + 1), e + 4);
+            bf16x8 hi, lo;
+            decayed8((const bf16_t*)&qall[i], e, hi, lo);
+            *(bf16x8*)(qs[0] + at_bf16(tall, c)) = hi;
+            *(bf16x8*)(qs[1] + at_bf16(tall, c)) = lo;
+        }
 #pragma unroll
-            for (int i = 0; i < 8; ++i) e[i] = rf[i] - e[i];
-            bf16x8 th, tl;
-            decayed8(kh + (long)s * ld_ + c, e, th, tl);
-            sc[j] = mfma_split(ah, al, th, tl, sc[j]);
+        for (int ks = 0; ks < 2; ++ks) {
+            const int c = ks * 4 + gq;
+            float rf[8], e[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) rf[i] = 0.f;
+            if (r0) {
+                ld4(bs + at_f32(tr, c * 2), rf);
+                ld4(bs + at_f32(tr, c * 2 + 1), rf + 4);
+            }
+            ld4(bs + at_f32(tq, c * 2), e);
+            ld4(bs + at_f32(tq, c * 2 + 1), e + 4);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) e[i] -= rf[i];
+            bf16x8 ah, al;
+            decayed8((const bf16_t*)&qown[ks], e, ah, al);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (j > jmax) continue;
+                const int s = j * 16 + fr;
+                ld4(bs + at_f32(s, c * 2), e);
+                ld4(bs + at_f32(s, c * 2 + 1), e + 4);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) e[i] = rf[i] - e[i];
+                bf16x8 th, tl;
+                decayed8(ks_ + at_bf16(s, c), e, th, tl);
+                sc[j] = mfma_split(ah, al, th, tl, sc[j]);
+            }
+        }
+        lds_barrier();
+        if (k0 + 64 < DK) {
+            issue(k0 + 64);
+            load_queries(k0 + 64);
+        }
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            bf16x8 hi[4], lo[4];
+#pragma unroll
+            for (int rt = 0; rt < 4; ++rt) {
+                hi[rt] = *(const bf16x8*)(
+                    qs[0] + at_bf16(rt * 16 + fr, ks * 4 + gq));
+                lo[rt] = *(const bf16x8*)(
+                    qs[1] + at_bf16(rt * 16 + fr, ks * 4 + gq));
+            }
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                if (c * 64 >= nv) continue;
+                bf16x8 sh, sl;
+                split8((const u32*)st[ks][c], sh, sl);
+                if (k0 + 64 < DK) load_state(k0 + 64, ks, c);
+#pragma unroll
+                for (int rt = 0; rt < 4; ++rt)
+                    acc[c][rt] = mfma_split(sh, sl, hi[rt], lo[rt],
+                                            acc[c][rt]);
+            }
         }
     }
     if (pairwise) {
@@ -1696,78 +1927,72 @@ k_gla_chunk_out(float* __restrict__ o, const float* __restrict__ dS,
         for (int j = 0; j < 4; ++j)
             if (j == wid) sc[j] = d;
     }
+    uint2 gates[4][4];
+    if (out)
+        load_gates(gates, qkv + (long)ch.x * ld_ + 2 * C + (long)H * DV + h * DV,
+                   ld_, last, DV);
+    // (the b of all waves' scores is no longer needed)
+    bf16_t* const ph = (bf16_t*)bs;
+    bf16_t* const pl = ph + 64 * 64;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         if (j > (wid | 1)) continue;
         const int key = j * 16 + fr;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int row = r0 + (lane >> 4) * 4 + r;
+            const int row = r0 + gq * 4 + r;
             const float p = key <= row && key <= last ? sc[j][r] * qscale : 0.f;
-            split_bf16(p, ph[row * MLD + key], pl[row * MLD + key]);
+            const int at = at_bf16(row, key >> 3) + (key & 7);
+            split_bf16(p, ph[at], pl[at]);
         }
     }
-    // (rows of ph and pl are read by the wave that wrote them)
-
-    const u32* Sb = (const u32*)dS + ((long)blockIdx.x * H + h) * DV * DK;
-    for (int v0 = blockIdx.z * 128; v0 < DV; v0 += gridDim.z * 128) {
-        const int nv = min(128, DV - v0);
-        __syncthreads();                 // readers of the last columns are done
-        for (int i = threadIdx.x; i < 64 * (nv / 8); i += 256) {
-            const int t = i & 63, c8 = (i >> 6) * 8;
-            const uint4 vv = *(const uint4*)(
-                qkv + (long)(ch.x + min(t, last)) * ld_ + 2 * C + h * DV + v0 +
-                c8);
-            const bf16_t* pv = (const bf16_t*)&vv;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) vt[(c8 + j) * MLD + t] = pv[j];
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[c][rt][r] *= qscale;
+    __syncthreads();
+    // the chunk's own values
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        bf16x8 hi[4], lo[4];
+#pragma unroll
+        for (int rt = ks * 2; rt < 4; ++rt) {
+            hi[rt] =
+                *(const bf16x8*)(ph + at_bf16(rt * 16 + fr, ks * 4 + gq));
+            lo[rt] =
+                *(const bf16x8*)(pl + at_bf16(rt * 16 + fr, ks * 4 + gq));
         }
-        __syncthreads();
-        // ---- what the entering state gives, then the chunk's own values
-        f32x4 acc[8];
 #pragma unroll
-        for (int c = 0; c < 8; ++c) acc[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        for (int k0 = 0; k0 < DK; k0 += 32) {
-            float e[8];
-            ld8(bh + tq * C + k0 + kg, e);
-            bf16x8 ah, al;
-            decayed8(qh + (long)tq * ld_ + k0 + kg, e, ah, al);
+        for (int c = 0; c < 4; ++c) {
+            if (c * 64 >= nv) continue;
+            const bf16x8 v = value_piece(vs, ks, c * 64 + wid * 16, nv);
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                if (c * 16 >= nv) continue;
-                bf16x8 hi, lo;
-                split8(Sb + (long)(v0 + c * 16 + fr) * DK + k0 + kg, hi, lo);
-                acc[c] = mfma_split(ah, al, hi, lo, acc[c]);
+            for (int rt = ks * 2; rt < 4; ++rt) {
+                acc[c][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    v, hi[rt], acc[c][rt], 0, 0, 0);
+                acc[c][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    v, lo[rt], acc[c][rt], 0, 0, 0);
             }
         }
+    }
+    if (out) {
+        store_normed<true>(
+            out + ((long)ch.x * H + h) * DV, acc, (float*)qs, gates,
+            (long)H * DV, norm + h * DV, ch.y, DV, dvtrue, eps);
+        return;
+    }
 #pragma unroll
-        for (int c = 0; c < 8; ++c)
+    for (int rt = 0; rt < 4; ++rt) {
+        const int t = rt * 16 + fr;
+        if (t > last) continue;
+        float* ob = o + ((long)(ch.x + t) * H + h) * (DV + 4) + v0 + r0 +
+                    gq * 4;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[c][r] *= qscale;
-        for (int ks = 0; ks <= (wid >> 1); ++ks) {
-            const int at = (r0 + fr) * MLD + ks * 32 + kg;
-            const bf16x8 ah = *(const bf16x8*)(ph + at);
-            const bf16x8 al = *(const bf16x8*)(pl + at);
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                if (c * 16 >= nv) continue;
-                const bf16x8 v =
-                    *(const bf16x8*)(vt + (c * 16 + fr) * MLD + ks * 32 + kg);
-                acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    ah, v, acc[c], 0, 0, 0);
-                acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    al, v, acc[c], 0, 0, 0);
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = r0 + (lane >> 4) * 4 + r;
-            if (row > last) continue;
-            float* ob = o + ((long)(ch.x + row) * H + h) * (DV + 4) + v0 + fr;
-#pragma unroll
-            for (int c = 0; c < 8; ++c)
-                if (c * 16 < nv) ob[c * 16] = acc[c][r];
-        }
+        for (int c = 0; c < 4; ++c)
+            if (c * 64 < nv)
+                *(f32x4*)(ob + c * 64) = acc[c][rt];
     }
 }
 
@@ -2648,24 +2873,26 @@ int gh_gla_decay(void* stream, void* b, const void* u, const void* w,
                  const void* bias, const void* chunks, int nd, int nchunks,
                  int R, int C, float inv_tau) {
     if (nd + nchunks < 1 || R < 1 || C < 1) return -100;
-#define GO(U) k_gla_decay<U><<<dim3((nd + U - 1) / U + nchunks, \
-        (C + 255) / 256), 256, 0, (hipStream_t)stream>>>((float*)b, \
+#define GO(U) k_gla_decay<U><<<dim3((nd + 4 * U - 1) / (4 * U) + nchunks, \
+        (C + 63) / 64), 256, 0, (hipStream_t)stream>>>((float*)b, \
         (const float*)u, (const float*)w, (const float*)bias, \
         (const int4*)chunks, nd, R, C, inv_tau)
-    if (nchunks) GO(16); else GO(4);
+    if (nchunks) GO(16); else GO(1);
 #undef GO
     LAUNCH_CHECK();
     return 0;
 }
 
-int gh_gla_chunks(void* stream, void* o, void* S, void* dS, const void* qkv,
-                  const void* b, const void* chunks, const void* segs,
-                  int nchunks, int nseg, int H, int DK, int DV, int ld_,
-                  float qscale) {
-    if (nchunks < 1 || nseg < 1 || DK % 64 || DV % 64) return -100;
+int gh_gla_chunks(void* stream, void* o, void* out, void* S, void* dS,
+                  const void* qkv, const void* b, const void* chunks,
+                  const void* segs, const void* norm, int nchunks, int nseg,
+                  int H, int DK, int DV, int ld_, float qscale, int dvtrue,
+                  float eps) {
+    if (nchunks < 1 || nseg < 1 || DK % 64 || DV % 64 || (out && DV > 256))
+        return -100;
     hipStream_t st_ = (hipStream_t)stream;
     // few chunks: value columns in blocks of their own, though each then takes
-    // the decays or scores again
+    // the decays again
     const bool many = nchunks * H >= 512;
     k_gla_chunk_state<<<dim3(nchunks, H, DK / 64 * (many ? 1 : DV / 64)), 256,
                         0, st_>>>((float*)dS, (const bf16_t*)qkv,
@@ -2676,10 +2903,10 @@ int gh_gla_chunks(void* stream, void* o, void* S, void* dS, const void* qkv,
                        st_>>>((float*)dS, (float*)S, (const float*)b,
         (const int4*)chunks, (const int4*)segs, H, DK, DV);
     LAUNCH_CHECK();
-    k_gla_chunk_out<<<dim3(nchunks, H, many ? 1 : (DV + 127) / 128), 256, 0,
-                      st_>>>((float*)o,
-        (const float*)dS, (const bf16_t*)qkv, (const float*)b,
-        (const int4*)chunks, H, DK, DV, ld_, qscale);
+    k_gla_chunk_out<<<dim3(nchunks, H, (DV + 255) / 256), 256, 0, st_>>>(
+        (float*)o, (bf16_t*)out, (const float*)dS, (const bf16_t*)qkv,
+        (const float*)b, (const int4*)chunks, (const float*)norm, H, DK, DV,
+        ld_, qscale, dvtrue, eps);
     LAUNCH_CHECK();
     return 0;
 }

@@ -53,7 +53,7 @@ _SIGS = {
     "gh_rec_out": "iipppppppppiiiiiiiiff",
     "gh_mlstm_chunks": "ipppppppppiiiiiiff",
     "gh_gla_decay": "pppppiiiif",
-    "gh_gla_chunks": "pppppppiiiiiif",
+    "gh_gla_chunks": "pppppppppiiiiiifif",
     "gh_moe_route": "pppppppippiiiiiiffiii",
     "gh_moe_gemm": "iipppppiiiiiffffp",
     "gn_latent_rows": "ippppippppppiiiiiiiif",
@@ -610,19 +610,23 @@ def gla(rows: torch.Tensor, u: torch.Tensor, wa2: torch.Tensor,
     _call("gh_gla_decay", b, u, wa2, ba2, st.chunks if nch else None,
           st.nd if nch else n, nch, wa2.shape[0], h * dk, 1.0 / tau)
     o = torch.empty(n, h, dv + 4, dtype=torch.float32, device=dev)
+    out = torch.empty(n, h * dv, dtype=rows.dtype, device=dev)
     segs, nseg = (st.segs, st.segs.shape[0]) if f and st.segs is not None \
         else (None, st.nd)
     if nseg:
         rpb = 128 if nseg * h * dv >= 128 * 2048 else 32
         _call("gh_rec_step", f, _CHANNELS, o, S, None, rows, b, segs, st.pos,
               st.slot, nseg, h, dk, dv, ld, qscale, 0.0, rpb)
+    whole = nch and dv <= 256          # chunks' blocks have all of a head
     if nch:
         ds = torch.empty(nch, h, dv, dk, dtype=torch.float32, device=dev)
-        _call("gh_gla_chunks", o, S, ds, rows, b, st.chunks, st.chunk_segs,
-              nch, st.chunk_segs.shape[0], h, dk, dv, ld, qscale)
-    out = torch.empty(n, h * dv, dtype=rows.dtype, device=dev)
-    _call("gh_rec_out", f, 1, out, o, None, rows, None, None, st.pos, st.slot,
-          norm, 0, 0, n, h, dk, dv, ld, vdim, 0.0, eps)
+        _call("gh_gla_chunks", o, out if whole else None, S, ds, rows, b,
+              st.chunks, st.chunk_segs, norm, nch, st.chunk_segs.shape[0], h,
+              dk, dv, ld, qscale, vdim, eps)
+    plain = st.nd if whole else n
+    if plain:
+        _call("gh_rec_out", f, 1, out, o, None, rows, None, None, st.pos,
+              st.slot, norm, 0, 0, plain, h, dk, dv, ld, vdim, 0.0, eps)
     return out
 
 

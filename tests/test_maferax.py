@@ -752,3 +752,56 @@ def test_trace_replay(checkpoint, tmp_path, run):
     for k, w in want.items():
         got = np.fromfile(os.path.join(out, f"{k}.f32"), dtype="<f4")
         close(torch.from_numpy(got).view(w.shape), w, run, coarse=0.1, odd=0.5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dk,dv", [(64, 64), (128, 256), (64, 192), (192, 128),
+                                   (64, 320)])
+def test_gla_chunk_sizes(dk, dv):
+    """Decode rows and portions of whole and cut chunks in one step, for heads
+    whose columns a block has all of (up to 256) or not."""
+    from gridllm_amd.ops import reference_hybrid
+    h, nd, lens = 2, 2, (1, 64, 130)
+    g = torch.Generator().manual_seed(dk + dv)
+    n = nd + sum(lens)
+    entries, chunks, segs = [(0, 1, 0, 7), (1, 1, 1, 3)], [], []
+    at = nd
+    for i, ln in enumerate(lens):
+        start = 0 if i == 2 else 5
+        entries.append((at, ln, nd + i, start))
+        segs.append((nd + i, start, len(chunks), -(-ln // 64)))
+        chunks += [(at + c, min(64, ln - c), i, 0) for c in range(0, ln, 64)]
+        at += ln
+    pos = torch.cat([torch.arange(e[3], e[3] + e[1]) for e in entries])
+    slot = torch.cat([torch.full((e[1],), e[2]) for e in entries])
+
+    def t(rows):
+        return torch.tensor(rows, dtype=torch.int32)
+    meta = dict(nd=nd, pos=pos.int(), slot=slot.int(),
+                table=torch.zeros(5, 1, dtype=torch.int32), max_len=200)
+    rows = torch.randn(n, h * 2 * (dk + dv), generator=g).to(torch.bfloat16)
+    u = torch.randn(n, 8, generator=g)
+    wa, ba = torch.randn(8, h * dk, generator=g), torch.randn(h * dk,
+                                                              generator=g)
+    S = torch.randn(5, h, dv, dk, generator=g)
+    norm = torch.rand(h * dv, generator=g) + 0.5
+    S0 = S.clone()
+    want = reference_hybrid.gla(rows.float(), u, wa, ba, S0, norm,
+                                hops.StepMeta(segs=t(entries), **meta), dk, dv,
+                                16.0, 1e-5)
+    dev = "cuda"
+    S1 = S.to(dev)
+    st = hops.StepMeta(chunks=t(chunks).to(dev), chunk_segs=t(segs).to(dev),
+                       segs=t(entries).to(dev),
+                       **{k: v.to(dev) if torch.is_tensor(v) else v
+                          for k, v in meta.items()})
+    got = hops.gla(rows.to(dev), u.to(dev), wa.to(dev), ba.to(dev), S1,
+                   norm.to(dev), st, dk, dv, 16.0, 1e-5).cpu().float()
+    # bf16 result; sums of products of (hi, lo) pairs, 2^-16 each, that a unit
+    # RMS row of cancelling terms makes up to 16 times as large
+    gate = torch.nn.functional.silu(rows[:, -h * dv:].float()).abs() * norm
+    assert bool(((got - want).abs() <= 2 ** -8 * want.abs() +
+                 2 ** -11 * gate + 1e-6).all())
+    used = [e[2] for e in entries]
+    assert float((S1.cpu()[used] - S0[used]).abs().max()) < \
+        2 ** -11 * float(S0.abs().max())
