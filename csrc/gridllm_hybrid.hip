@@ -1249,23 +1249,173 @@ DEV_INLINE void split8(const u32* p, bf16x8& hi, bf16x8& lo) {
     lo = *(bf16x8*)&b;
 }
 
-// Block = (chunk, head, 128 value columns); a wave owns 16 tokens.
+// Places in LDS of 16-byte pieces c, swapped by the row so that 16 lanes' rows
+// do not meet in a bank: of 64 f32, of 64 bf16, and of `cols` bf16 that are read
+// transposed, where 4 rows' pairs of pieces have to lie apart.
+DEV_INLINE int at_f32(int row, int c) { return row * 64 + (c ^ (row & 15)) * 4; }
+DEV_INLINE int at_bf16(int row, int c) { return row * 64 + (c ^ (row & 7)) * 8; }
+DEV_INLINE int at_cols(int row, int c, int cols) {
+    return row * cols + (c ^ ((row & 3) << 1 | (row >> 2 & 1))) * 8;
+}
+
+// 64 tokens' values, up to 256 columns of them, on their way to LDS
+DEV_INLINE void load_values(bf16_t* vs, const bf16_t* v, long ld_, int last,
+                            int cols) {
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int i = 0; i < cols / 32; ++i) {
+        const int pc = i * 256 + threadIdx.x, row = pc / (cols / 8);
+        const int c = at_cols(row, pc % (cols / 8), cols) / 8 -
+                      row * (cols / 8);
+        load_lds16(v + min(row, last) * ld_ + c * 8,
+                   vs + (i * 256 + wid * 64) * 8);
+    }
+}
+
+// Values (16 columns from `col` on, as the products' rows) of 32 tokens.
+DEV_INLINE bf16x8 value_piece(const bf16_t* vs, int ks, int col, int cols) {
+    const int lane = threadIdx.x & 63, fr = lane & 15, gq = lane >> 4;
+    const int d = col + (fr & 3) * 4;
+    bf16x8 v;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int row = ks * 32 + gq * 8 + (fr >> 2) + j * 4;
+        const bf16x4 x =
+            read_transposed(vs + at_cols(row, d >> 3, cols) + (d & 7));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[j * 4 + i] = x[i];
+    }
+    return v;
+}
+
+// Output gates of a chunk, for lane = 4 columns c * 64 + wid * 16 + gq * 4 + r of
+// tokens rt * 16 + fr: on their way ahead of the last products.
+DEV_INLINE void load_gates(uint2 (&z)[4][4], const bf16_t* gate, long ld_,
+                           int last, int DV) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (c * 64 < DV)
+                z[c][rt] = *(const uint2*)(
+                    gate + min(rt * 16 + (lane & 15), last) * ld_ + c * 64 +
+                    wid * 16 + (lane >> 4) * 4);
+}
+
+// A chunk's outputs, laid out as its gates, with all of the head's columns in the
+// block: unit RMS, times norm, times the gate's sigmoid (SILU: and the gate).
+// red: f32 [4][64] in LDS.
+template <bool SILU>
+DEV_INLINE void store_normed(bf16_t* out, const f32x4 (&acc)[4][4],
+                             float* red, const uint2 (&gates)[4][4],
+                             long out_ld, const float* norm, int len, int DV,
+                             int dvtrue, float eps) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int fr = lane & 15, gq = lane >> 4, col0 = wid * 16 + gq * 4;
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+        float ss = 0.f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (c * 64 < DV)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) ss += acc[c][rt][r] * acc[c][rt][r];
+        ss += __shfl_xor(ss, 16, WAVE);
+        ss += __shfl_xor(ss, 32, WAVE);
+        if (gq == 0) red[wid * 64 + rt * 16 + fr] = ss;
+    }
+    float w[4][4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        if (c * 64 < DV) ld4(norm + c * 64 + col0, w[c]);
+    __syncthreads();
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+        const int t = rt * 16 + fr;
+        const float ss = red[t] + red[64 + t] + red[128 + t] + red[192 + t];
+        const float rs = 1.f / sqrtf(ss / (float)dvtrue + eps);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (c * 64 >= DV) continue;
+            float z[4];
+            ld4((const bf16_t*)&gates[c][rt], z);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                z[r] = acc[c][rt][r] * rs * w[c][r] *
+                       __builtin_amdgcn_rcpf(1.f + __expf(-z[r])) *
+                       (SILU ? z[r] : 1.f);
+            if (t < len) st4(out + t * out_ld + c * 64 + col0, z);
+        }
+    }
+}
+
+// Block = (chunk, head, 256 value columns). Scores: a wave owns 16 tokens;
+// outputs: every fourth 16 columns for all 64, so that the state is read once.
+// Queries and keys come through LDS, 64 channels ahead of their use. With all of a
+// head's columns here (out), the head's norm and gate follow at once; out and
+// CONST exclude each other. Bound by reading the state and the few steps'
+// latencies: 3500 tokens, 12 heads of 128 x 256: 92 us with tokens split over
+// the waves and 128 columns a block, and 28 of the norm behind it, now 57.
 template <bool CONST>
 __global__ void __launch_bounds__(256, 2)
-k_mlstm_chunk_out(float* __restrict__ o, const float* __restrict__ dS,
+k_mlstm_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
+                  const float* __restrict__ dS,
                   const float* __restrict__ scal,
                   const bf16_t* __restrict__ qkv,
                   const float* __restrict__ gr,
-                  const int4* __restrict__ chunks, int H, int DK, int DV,
-                  int ld_, float qscale, float cap) {
-    __shared__ __attribute__((aligned(16))) bf16_t vt[128 * MLD];
-    __shared__ __attribute__((aligned(16))) bf16_t ps[64 * MLD];
-    __shared__ __attribute__((aligned(16))) bf16_t pl[CONST ? 64 * MLD : 8];
-    __shared__ float sa[MCH], sM[MCH], sm[MCH], sin_[MCH], snq[MCH];
+                  const int4* __restrict__ chunks,
+                  const float* __restrict__ norm, int H, int DK, int DV,
+                  int ld_, float qscale, float cap, int dvtrue, float eps) {
+    __shared__ __attribute__((aligned(16))) bf16_t vs[64 * 256];
+    __shared__ __attribute__((aligned(16))) bf16_t qk[2][2][64 * 64];
+    __shared__ float sa[MCH], sM[MCH], sm[MCH], sin_[MCH], snq[MCH], sden[MCH];
     const int4 ch = chunks[blockIdx.x];
-    const int h = blockIdx.y, v0 = blockIdx.z * 128;
-    const int nv = min(128, DV - v0);
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int h = blockIdx.y, v0 = blockIdx.z * 256, nv = min(256, DV - v0);
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int fr = lane & 15, gq = lane >> 4, r0 = wid * 16, last = ch.y - 1;
+    const u32* Sb = (const u32*)dS +
+                    ((long)blockIdx.x * H + h) * (CONST ? DV : DV + 1) * DK;
+    const u32* nb = Sb + (long)DV * DK + gq * 8;       // the normaliser's row
+    Sb += (long)(v0 + r0 + fr) * DK + gq * 8;
+    const bf16_t* qh = qkv + (long)ch.x * ld_ + h * DK;
+
+    auto issue = [&](int buf, int k0) {    // queries and keys of 64 channels
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int pc = i * 256 + threadIdx.x, row = pc >> 3;
+            const bf16_t* src = qh + (long)min(row, last) * ld_ + k0 +
+                                ((pc & 7) ^ (row & 7)) * 8;
+            load_lds16(src, qk[buf][0] + (i * 256 + wid * 64) * 8);
+            load_lds16(src + (long)H * DK,
+                       qk[buf][1] + (i * 256 + wid * 64) * 8);
+        }
+    };
+    uint4 st[2][4][2];
+    auto load_state = [&](int k0, int ks, int c) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            st[ks][c][i] = *(const uint4*)(Sb + (long)c * 64 * DK + k0 +
+                                           ks * 32 + i * 4);
+    };
+    uint4 nw[2][2];
+    auto load_norm = [&](int k0) {
+        if (CONST) return;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                nw[ks][i] = *(const uint4*)(nb + k0 + ks * 32 + i * 4);
+    };
+    issue(0, 0);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (c * 64 < nv) load_state(0, ks, c);
+    load_norm(0);
+    load_values(vs, qkv + (long)ch.x * ld_ + 2l * H * DK + h * DV + v0, ld_,
+                last, nv);
     if (wid == 0) {
         float F, a, amax;
         chunk_scan<CONST>(gr, ch.x, ch.y, h, H, cap, F, a, amax);
@@ -1276,56 +1426,79 @@ k_mlstm_chunk_out(float* __restrict__ o, const float* __restrict__ dS,
         sm[lane] = F + M;
         sin_[lane] = expf(m_in - M);
     }
-    for (int i = threadIdx.x; i < 64 * (nv / 8); i += 256) {
-        const int t = i & 63, c8 = (i >> 6) * 8;
-        const uint4 vv = *(const uint4*)(
-            qkv + (long)(ch.x + min(t, ch.y - 1)) * ld_ + 2 * H * DK + h * DV +
-            v0 + c8);
-        const bf16_t* pv = (const bf16_t*)&vv;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) vt[(c8 + j) * MLD + t] = pv[j];
-    }
-    __syncthreads();
-    const int fr = lane & 15, kg = (lane >> 4) * 8, r0 = wid * 16;
-    const u32* Sb = (const u32*)dS +
-                    ((long)blockIdx.x * H + h) * (CONST ? DV : DV + 1) * DK;
-    const bf16_t* qr = qkv + (long)(ch.x + min(r0 + fr, ch.y - 1)) * ld_ +
-                       h * DK + kg;
 
-    // ---- scores of this wave's tokens against the chunk's keys, and n . q
-    f32x4 sc[4];
-    const bf16_t* kr[4];
+    // ---- scores of this wave's tokens against the chunk's keys, n . q, and
+    // what the entering state gives
+    f32x4 sc[4], acc[4][4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         sc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        kr[j] = qkv + (long)(ch.x + min(j * 16 + fr, ch.y - 1)) * ld_ +
-                (H + h) * DK + kg;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[j][c] = sc[j];
     }
     float nq = 0.f;
-    for (int k0 = 0; k0 < DK; k0 += 32) {
-        const bf16x8 a = *(const bf16x8*)(qr + k0);
-        if (!CONST) {
-            float qf[8];
-            unpack8(*(const uint4*)&a, qf);
-            const u32* np = Sb + (long)DV * DK + k0 + kg;
+    int buf = 0;
+    for (int k0 = 0; k0 < DK; k0 += 64, buf ^= 1) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        lds_barrier();                 // they are there, the others are free
+        const bool more = k0 + 64 < DK;
+        if (more) issue(buf ^ 1, k0 + 64);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const u32 w = np[i];
-                nq += qf[i] * (__uint_as_float(w << 16) +
-                               __uint_as_float(w & 0xffff0000u));
+        for (int ks = 0; ks < 2; ++ks) {
+            const int c8 = ks * 4 + gq;
+            bf16x8 q[4];
+#pragma unroll
+            for (int rt = 0; rt < 4; ++rt)
+                q[rt] = *(const bf16x8*)(
+                    qk[buf][0] + at_bf16(rt * 16 + fr, c8));
+            const bf16x8 own =
+                *(const bf16x8*)(qk[buf][0] + at_bf16(r0 + fr, c8));
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (j <= wid)
+                    sc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        own,
+                        *(const bf16x8*)(qk[buf][1] +
+                                         at_bf16(j * 16 + fr, c8)),
+                        sc[j], 0, 0, 0);
+            if (!CONST) {
+                float qf[8];
+                unpack8(*(const uint4*)&own, qf);
+                const u32* np = (const u32*)nw[ks];
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    nq += qf[i] * (__uint_as_float(np[i] << 16) +
+                                   __uint_as_float(np[i] & 0xffff0000u));
+            }
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                if (c * 64 >= nv) continue;
+                bf16x8 sh, sl;
+                split8((const u32*)st[ks][c], sh, sl);
+                if (more) load_state(k0 + 64, ks, c);
+#pragma unroll
+                for (int rt = 0; rt < 4; ++rt) {
+                    acc[c][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        sh, q[rt], acc[c][rt], 0, 0, 0);
+                    acc[c][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        sl, q[rt], acc[c][rt], 0, 0, 0);
+                }
             }
         }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (j <= wid)
-                sc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    a, *(const bf16x8*)(kr[j] + k0), sc[j], 0, 0, 0);
+        if (more) load_norm(k0 + 64);
     }
+    uint2 gates[4][4];
+    if (out)
+        load_gates(gates, qkv + (long)ch.x * ld_ + 2l * H * DK + (long)H * DV +
+                              h * DV, ld_, last, DV);
     if (!CONST) {
         nq += __shfl_xor(nq, 16, WAVE);
         nq += __shfl_xor(nq, 32, WAVE);
         if (lane < 16) snq[r0 + lane] = nq;
     }
+    lds_barrier();                     // queries and keys have been read
+    bf16_t* const ps = qk[0][0];
+    bf16_t* const pl = qk[0][1];
     float den[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -1334,77 +1507,83 @@ k_mlstm_chunk_out(float* __restrict__ o, const float* __restrict__ dS,
         const float ak = sa[key];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int row = r0 + (lane >> 4) * 4 + r;
+            const int row = r0 + gq * 4 + r;
             const float p = (key <= row && key < ch.y)
                 ? sc[j][r] * qscale * expf(ak - sM[row]) : 0.f;
             den[r] += p;
-            ps[row * MLD + key] = f2bf(p);
-            if (CONST)
-                pl[row * MLD + key] = f2bf(p - bf2f(f2bf(p)));
+            const int at = at_bf16(row, key >> 3) + (key & 7);
+            ps[at] = f2bf(p);
+            if (CONST) pl[at] = f2bf(p - bf2f(f2bf(p)));
         }
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int r = 0; r < 4; ++r) {
 #pragma unroll
         for (int off = 8; off > 0; off >>= 1)
             den[r] += __shfl_xor(den[r], off, WAVE);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // own rows only
-
-    // ---- what the entering state gives, then the chunk's own values
-    f32x4 acc[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) acc[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < DK; k0 += 32) {
-        const bf16x8 a = *(const bf16x8*)(qr + k0);
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            if (c * 16 >= nv) continue;
-            bf16x8 hi, lo;
-            split8(Sb + (long)(v0 + c * 16 + fr) * DK + k0 + kg, hi, lo);
-            acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, hi, acc[c],
-                                                             0, 0, 0);
-            acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, lo, acc[c],
-                                                             0, 0, 0);
-        }
+        if (fr == 0) sden[r0 + gq * 4 + r] = den[r];
     }
+    lds_barrier();
     float inv[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int row = r0 + (lane >> 4) * 4 + r;
-        const float in = sin_[row] * qscale;
-        inv[r] = 1.f;
+    for (int rt = 0; rt < 4; ++rt) {
+        const int t = rt * 16 + fr;
+        const float in = sin_[t] * qscale;
+        inv[rt] = 1.f;
         if (!CONST) {
-            const float d = den[r] + in * snq[row];
-            inv[r] = 1.f / (fmaxf(fabsf(d), expf(-sm[row])) + 1e-6f);
+            const float d = sden[t] + in * snq[t];
+            inv[rt] = 1.f / (fmaxf(fabsf(d), expf(-sm[t])) + 1e-6f);
         }
 #pragma unroll
-        for (int c = 0; c < 8; ++c) acc[c][r] *= in;
-    }
-    for (int ks = 0; ks <= (wid >> 1); ++ks) {
-        const int at = (r0 + fr) * MLD + ks * 32 + kg;
-        const bf16x8 a = *(const bf16x8*)(ps + at);
-        bf16x8 al;
-        if (CONST) al = *(const bf16x8*)(pl + at);
+        for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            if (c * 16 >= nv) continue;
-            const bf16x8 v =
-                *(const bf16x8*)(vt + (c * 16 + fr) * MLD + ks * 32 + kg);
-            acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, v, acc[c],
-                                                             0, 0, 0);
-            if (CONST)
-                acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    al, v, acc[c], 0, 0, 0);
+            for (int r = 0; r < 4; ++r) acc[c][rt][r] *= in;
+    }
+    // ---- the chunk's own values
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        bf16x8 hi[4], lo[4];
+#pragma unroll
+        for (int rt = ks * 2; rt < 4; ++rt) {
+            const int at = at_bf16(rt * 16 + fr, ks * 4 + gq);
+            hi[rt] = *(const bf16x8*)(ps + at);
+            if (CONST) lo[rt] = *(const bf16x8*)(pl + at);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (c * 64 >= nv) continue;
+            const bf16x8 v = value_piece(vs, ks, c * 64 + r0, nv);
+#pragma unroll
+            for (int rt = ks * 2; rt < 4; ++rt) {
+                acc[c][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    v, hi[rt], acc[c][rt], 0, 0, 0);
+                if (CONST)
+                    acc[c][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        v, lo[rt], acc[c][rt], 0, 0, 0);
+            }
         }
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int row = r0 + (lane >> 4) * 4 + r;
-        if (row >= ch.y) continue;
-        float* ob = o + ((long)(ch.x + row) * H + h) * (DV + 4) + v0 + fr;
+    for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int c = 0; c < 8; ++c)
-            if (c * 16 < nv) ob[c * 16] = acc[c][r] * inv[r];
+        for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[c][rt][r] *= inv[rt];
+    if (out) {
+        store_normed<false>(
+            out + ((long)ch.x * H + h) * DV, acc, (float*)qk[1][0], gates,
+            (long)H * DV, norm + h * DV, ch.y, DV, dvtrue, eps);
+        return;
+    }
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+        const int t = rt * 16 + fr;
+        if (t > last) continue;
+        float* ob = o + ((long)(ch.x + t) * H + h) * (DV + 4) + v0 + r0 +
+                    gq * 4;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (c * 64 < nv) *(f32x4*)(ob + c * 64) = acc[c][rt];
     }
 }
 
@@ -1633,106 +1812,6 @@ DEV_INLINE f32x4 mfma_split(bf16x8 ah, bf16x8 al, bf16x8 bh, bf16x8 bl,
     c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh, c, 0, 0, 0);
     c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl, c, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, c, 0, 0, 0);
-}
-
-// Places in LDS of 16-byte pieces c, swapped by the row so that 16 lanes' rows
-// do not meet in a bank: of 64 f32, of 64 bf16, and of `cols` bf16 that are read
-// transposed, where 4 rows' pairs of pieces have to lie apart.
-DEV_INLINE int at_f32(int row, int c) { return row * 64 + (c ^ (row & 15)) * 4; }
-DEV_INLINE int at_bf16(int row, int c) { return row * 64 + (c ^ (row & 7)) * 8; }
-DEV_INLINE int at_cols(int row, int c, int cols) {
-    return row * cols + (c ^ ((row & 3) << 1 | (row >> 2 & 1))) * 8;
-}
-
-// 64 tokens' values, up to 256 columns of them, on their way to LDS
-DEV_INLINE void load_values(bf16_t* vs, const bf16_t* v, long ld_, int last,
-                            int cols) {
-    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    for (int i = 0; i < cols / 32; ++i) {
-        const int pc = i * 256 + threadIdx.x, row = pc / (cols / 8);
-        const int c = at_cols(row, pc % (cols / 8), cols) / 8 -
-                      row * (cols / 8);
-        load_lds16(v + min(row, last) * ld_ + c * 8,
-                   vs + (i * 256 + wid * 64) * 8);
-    }
-}
-
-// Values (16 columns from `col` on, as the products' rows) of 32 tokens.
-DEV_INLINE bf16x8 value_piece(const bf16_t* vs, int ks, int col, int cols) {
-    const int lane = threadIdx.x & 63, fr = lane & 15, gq = lane >> 4;
-    const int d = col + (fr & 3) * 4;
-    bf16x8 v;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int row = ks * 32 + gq * 8 + (fr >> 2) + j * 4;
-        const bf16x4 x =
-            read_transposed(vs + at_cols(row, d >> 3, cols) + (d & 7));
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[j * 4 + i] = x[i];
-    }
-    return v;
-}
-
-// Output gates of a chunk, for lane = 4 columns c * 64 + wid * 16 + gq * 4 + r of
-// tokens rt * 16 + fr: on their way ahead of the last products.
-DEV_INLINE void load_gates(uint2 (&z)[4][4], const bf16_t* gate, long ld_,
-                           int last, int DV) {
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (c * 64 < DV)
-                z[c][rt] = *(const uint2*)(
-                    gate + min(rt * 16 + (lane & 15), last) * ld_ + c * 64 +
-                    wid * 16 + (lane >> 4) * 4);
-}
-
-// A chunk's outputs, laid out as its gates, with all of the head's columns in the
-// block: unit RMS, times norm, times the gate's sigmoid (SILU: and the gate).
-// red: f32 [4][64] in LDS.
-template <bool SILU>
-DEV_INLINE void store_normed(bf16_t* out, const f32x4 (&acc)[4][4],
-                             float* red, const uint2 (&gates)[4][4],
-                             long out_ld, const float* norm, int len, int DV,
-                             int dvtrue, float eps) {
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int fr = lane & 15, gq = lane >> 4, col0 = wid * 16 + gq * 4;
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-        float ss = 0.f;
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (c * 64 < DV)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) ss += acc[c][rt][r] * acc[c][rt][r];
-        ss += __shfl_xor(ss, 16, WAVE);
-        ss += __shfl_xor(ss, 32, WAVE);
-        if (gq == 0) red[wid * 64 + rt * 16 + fr] = ss;
-    }
-    float w[4][4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-        if (c * 64 < DV) ld4(norm + c * 64 + col0, w[c]);
-    __syncthreads();
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-        const int t = rt * 16 + fr;
-        const float ss = red[t] + red[64 + t] + red[128 + t] + red[192 + t];
-        const float rs = 1.f / sqrtf(ss / (float)dvtrue + eps);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            if (c * 64 >= DV) continue;
-            float z[4];
-            ld4((const bf16_t*)&gates[c][rt], z);
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                z[r] = acc[c][rt][r] * rs * w[c][r] *
-                       __builtin_amdgcn_rcpf(1.f + __expf(-z[r])) *
-                       (SILU ? z[r] : 1.f);
-            if (t < len) st4(out + t * out_ld + c * 64 + col0, z);
-        }
-    }
 }
 
 // Block = (chunk, head, 256 value columns). Scores: wave w owns tokens 16 w ..
@@ -2840,12 +2919,14 @@ int gh_rec_row_out(void* stream, int f32, void* out, const void* o,
 }
 
 // constant: lightning attention (gr: log decay by head; mst unused)
-int gh_mlstm_chunks(void* stream, int constant, void* o, void* S, void* mst,
-                    void* dS, void* scal, const void* qkv, const void* gr,
-                    const void* chunks, const void* segs, int nchunks,
-                    int nseg, int H, int DK, int DV, int ld_, float qscale,
-                    float cap) {
-    if (nchunks < 1 || nseg < 1 || DK % 64 || DV % 64 || (!constant && !mst))
+int gh_mlstm_chunks(void* stream, int constant, void* o, void* out, void* S,
+                    void* mst, void* dS, void* scal, const void* qkv,
+                    const void* gr, const void* chunks, const void* segs,
+                    const void* norm, int nchunks, int nseg, int H, int DK,
+                    int DV, int ld_, float qscale, float cap, int dvtrue,
+                    float eps) {
+    if (nchunks < 1 || nseg < 1 || DK % 64 || DV % 64 || (!constant && !mst) ||
+        (out && (constant || DV > 256)))
         return -100;
     hipStream_t st_ = (hipStream_t)stream;
     const long quads = (long)(DV + !constant) * DK / 4;
@@ -2859,10 +2940,11 @@ int gh_mlstm_chunks(void* stream, int constant, void* o, void* S, void* mst,
         256, 0, st_>>>((float*)dS, (float*)scal, (float*)S, (float*)mst, \
         (const int4*)segs, H, DK, DV); \
     LAUNCH_CHECK(); \
-    k_mlstm_chunk_out<C><<<dim3(nchunks, H, (DV + 127) / 128), 256, 0, \
-        st_>>>((float*)o, (const float*)dS, (const float*)scal, \
-        (const bf16_t*)qkv, (const float*)gr, (const int4*)chunks, H, DK, DV, \
-        ld_, qscale, cap); \
+    k_mlstm_chunk_out<C><<<dim3(nchunks, H, (DV + 255) / 256), 256, 0, \
+        st_>>>((float*)o, (bf16_t*)out, (const float*)dS, \
+        (const float*)scal, (const bf16_t*)qkv, (const float*)gr, \
+        (const int4*)chunks, (const float*)norm, H, DK, DV, ld_, qscale, cap, \
+        dvtrue, eps); \
     LAUNCH_CHECK(); } while (0)
     if (constant) GO(true); else GO(false);
 #undef GO

@@ -51,7 +51,7 @@ _SIGS = {
     "gh_rec_step": "iippppppppiiiiiffi",
     "gh_rec_row_out": "ippppiiiiiif",
     "gh_rec_out": "iipppppppppiiiiiiiiff",
-    "gh_mlstm_chunks": "ipppppppppiiiiiiff",
+    "gh_mlstm_chunks": "ipppppppppppiiiiiiffif",
     "gh_gla_decay": "pppppiiiif",
     "gh_gla_chunks": "pppppppppiiiiiifif",
     "gh_moe_route": "pppppppippiiiiiiffiii",
@@ -417,19 +417,21 @@ def mlstm(qkv: torch.Tensor, gates: torch.Tensor, S: torch.Tensor,
         rpb = 128 if nseg * h * (dv + 1) >= 128 * 2048 else 32
         _call("gh_rec_step", f, _MLSTM, o, S, m, qkv, gates, segs, st.pos,
               st.slot, nseg, h, dk, dv, ld, qscale, cap, rpb)
+    out = torch.empty(n, h * dv, dtype=qkv.dtype, device=qkv.device)
     nplain = 0
     if not f and st.chunks is not None:
-        nplain = n - st.nd
+        whole = dv <= 256              # chunks' blocks have all of a head
+        nplain = 0 if whole else n - st.nd
         nch = st.chunks.shape[0]
         ds = torch.empty(nch, h, dv + 1, dk, dtype=torch.float32,
                          device=qkv.device)
         scal = torch.empty(nch, h, 4, dtype=torch.float32, device=qkv.device)
-        _call("gh_mlstm_chunks", 0, o, S, m, ds, scal, qkv, gates, st.chunks,
-              st.chunk_segs, nch, st.chunk_segs.shape[0], h, dk, dv, ld,
-              qscale, cap)
-    out = torch.empty(n, h * dv, dtype=qkv.dtype, device=qkv.device)
-    _call("gh_rec_out", f, 0, out, o, m, qkv, gates, segs, st.pos, st.slot,
-          norm, nseg, st.nd, nplain, h, dk, dv, ld, vdim, cap, eps)
+        _call("gh_mlstm_chunks", 0, o, out if whole else None, S, m, ds, scal,
+              qkv, gates, st.chunks, st.chunk_segs, norm, nch,
+              st.chunk_segs.shape[0], h, dk, dv, ld, qscale, cap, vdim, eps)
+    if nseg + nplain:
+        _call("gh_rec_out", f, 0, out, o, m, qkv, gates, segs, st.pos, st.slot,
+              norm, nseg, st.nd, nplain, h, dk, dv, ld, vdim, cap, eps)
     return out
 
 
@@ -461,9 +463,9 @@ def lightning(rows: torch.Tensor, S: torch.Tensor, decay: torch.Tensor,
         nch = st.chunks.shape[0]
         ds = torch.empty(nch, h, dv, dk, dtype=torch.float32, device=dev)
         scal = torch.empty(nch, h, 4, dtype=torch.float32, device=dev)
-        _call("gh_mlstm_chunks", 1, o, S, None, ds, scal, rows, decay[1],
-              st.chunks, st.chunk_segs, nch, st.chunk_segs.shape[0], h, dk, dv,
-              ld, 1.0, 0.0)
+        _call("gh_mlstm_chunks", 1, o, None, S, None, ds, scal, rows, decay[1],
+              st.chunks, st.chunk_segs, None, nch, st.chunk_segs.shape[0], h,
+              dk, dv, ld, 1.0, 0.0, 0, 0.0)
     at = h * (2 * dk + dv)
     _call("gh_rec_row_out", f, out, o, rows[:, at:], norm, n, h, dv, ld,
           out.stride(0), h * vdim, eps)

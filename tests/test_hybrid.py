@@ -685,3 +685,57 @@ def test_trace_program(checkpoint, tmp_path):
     assert [x for x in r.stdout.splitlines() if x.startswith("done")] == [
         f"done {i}" for i in range(4)]
     check_trace(out, want, ("cpu", "fp32"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dk,dv", [(64, 64), (128, 256), (64, 192), (192, 128),
+                                   (64, 320)])
+def test_mlstm_chunk_sizes(dk, dv):
+    """Decode rows and portions of whole and cut chunks in one step, for heads
+    whose columns a block has all of (up to 256) or not."""
+    from gridllm_amd.ops import reference_hybrid
+    h, nd, lens = 2, 2, (1, 64, 130)
+    g = torch.Generator().manual_seed(dk + dv)
+    n = nd + sum(lens)
+    entries, chunks, segs = [(0, 1, 0, 7), (1, 1, 1, 3)], [], []
+    at = nd
+    for i, ln in enumerate(lens):
+        start = 0 if i == 2 else 5
+        entries.append((at, ln, nd + i, start))
+        segs.append((nd + i, start, len(chunks), -(-ln // 64)))
+        chunks += [(at + c, min(64, ln - c), i, 0) for c in range(0, ln, 64)]
+        at += ln
+    pos = torch.cat([torch.arange(e[3], e[3] + e[1]) for e in entries])
+    slot = torch.cat([torch.full((e[1],), e[2]) for e in entries])
+
+    def t(rows):
+        return torch.tensor(rows, dtype=torch.int32)
+    meta = dict(nd=nd, pos=pos.int(), slot=slot.int(),
+                table=torch.zeros(5, 1, dtype=torch.int32), max_len=200)
+    rows = torch.randn(n, h * 2 * (dk + dv), generator=g).to(torch.bfloat16)
+    gates = torch.randn(n, 2 * h, generator=g) * 3
+    S = torch.randn(5, h, dv + 1, dk, generator=g)
+    # normalisers that no query makes small: every denominator is its own
+    S[:, :, dv] = 0.0
+    m, norm = torch.rand(5, h, generator=g), torch.rand(h * dv,
+                                                        generator=g) + 0.5
+    S0, m0 = S.clone(), m.clone()
+    want = reference_hybrid.mlstm(rows.float(), gates, S0, m0, norm,
+                                  hops.StepMeta(segs=t(entries), **meta), dk,
+                                  dv, 15.0, 1e-5)
+    dev = "cuda"
+    S1, m1 = S.to(dev), m.to(dev)
+    st = hops.StepMeta(chunks=t(chunks).to(dev), chunk_segs=t(segs).to(dev),
+                       segs=t(entries).to(dev),
+                       **{k: v.to(dev) if torch.is_tensor(v) else v
+                          for k, v in meta.items()})
+    got = hops.mlstm(rows.to(dev), gates.to(dev), S1, m1, norm.to(dev), st, dk,
+                     dv, 15.0, 1e-5).cpu().float()
+    # bf16 result of a unit RMS row; bf16 weights of a chunk's values, 2^-9 each
+    gate = torch.sigmoid(rows[:, -h * dv:].float()) * norm
+    assert bool(((got - want).abs() <= 2 ** -8 * want.abs() +
+                 2 ** -6 * gate + 1e-6).all())
+    used = [e[2] for e in entries]
+    assert float((S1.cpu()[used] - S0[used]).abs().max()) < \
+        2 ** -11 * float(S0.abs().max())
+    assert float((m1.cpu()[used] - m0[used]).abs().max()) < 1e-4
