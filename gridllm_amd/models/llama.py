@@ -29,6 +29,7 @@ import torch.nn.functional as F  # noqa: F401
 
 from gridllm_amd.ops.autotune import linear as _linear
 from gridllm_amd.ops.autotune import linear_gateup as _linear_gateup
+from gridllm_amd.ops.autotune import linear_rmsnorm as _linear_rmsnorm
 
 from gridllm_amd import ops
 from gridllm_amd.models.registry import ModelSpec
@@ -214,6 +215,15 @@ class LlamaModel:
             lw.wgateup = lw.wgateup[perm].contiguous()
         self.gateup_il = True
 
+    def _joined(self, x: torch.Tensor, w: torch.Tensor, norm: torch.Tensor,
+                resid: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+        """A sublayer's last projection, added to the residual, and its norm."""
+        if self.tp.size == 1:
+            return _linear_rmsnorm(x, w, norm, self.spec.norm_eps, resid)
+        out = _linear(x, w)
+        self.tp.all_reduce(out)
+        return ops.rmsnorm(out, norm, self.spec.norm_eps, residual=resid)
+
     def _mlp_act(self, normed: torch.Tensor, lw: LayerWeights) -> torch.Tensor:
         if self.gateup_il:
             return _linear_gateup(normed, lw.wgateup)
@@ -365,17 +375,12 @@ class LlamaModel:
             attn = ops.attn_prefill_cache(
                 q, self.cache.k[li], self.cache.v[li], slot, start_pos + t,
                 start_pos, self.scale)                           # [T,Hq_l,D]
-            attn_out = _linear(attn.reshape(t, -1), lw.wo)
-            self.tp.all_reduce(attn_out)
-            normed, resid = ops.rmsnorm(attn_out, lw.mlp_norm, s.norm_eps,
-                                        residual=resid)
+            normed, resid = self._joined(attn.reshape(t, -1), lw.wo,
+                                         lw.mlp_norm, resid)
             act = self._mlp_act(normed, lw)
-            mlp_out = _linear(act, lw.wdown)
-            self.tp.all_reduce(mlp_out)
             next_norm = (self.layers[li + 1].attn_norm
                          if li + 1 < len(self.layers) else self.final_norm)
-            normed, resid = ops.rmsnorm(mlp_out, next_norm, s.norm_eps,
-                                        residual=resid)
+            normed, resid = self._joined(act, lw.wdown, next_norm, resid)
         logits = _linear(normed[-1:], self.lm_head).float()
         if return_hidden:
             return logits[0], normed.float().mean(dim=0)
@@ -435,17 +440,12 @@ class LlamaModel:
                     attn[bounds[i]:bounds[i + 1]] = ops.attn_prefill_cache(
                         q[bounds[i]:bounds[i + 1]], self.cache.k[li],
                         self.cache.v[li], sl, lens[i], 0, self.scale)
-            attn_out = _linear(attn.reshape(bounds[-1], -1), lw.wo)
-            self.tp.all_reduce(attn_out)
-            normed, resid = ops.rmsnorm(attn_out, lw.mlp_norm, s.norm_eps,
-                                        residual=resid)
+            normed, resid = self._joined(attn.reshape(bounds[-1], -1), lw.wo,
+                                         lw.mlp_norm, resid)
             act = self._mlp_act(normed, lw)
-            mlp_out = _linear(act, lw.wdown)
-            self.tp.all_reduce(mlp_out)
             next_norm = (self.layers[li + 1].attn_norm
                          if li + 1 < len(self.layers) else self.final_norm)
-            normed, resid = ops.rmsnorm(mlp_out, next_norm, s.norm_eps,
-                                        residual=resid)
+            normed, resid = self._joined(act, lw.wdown, next_norm, resid)
         # ONE scatter instead of k per-sequence device writes (each is a
         # serialized H2D launch — 15 ms of host time per admission batch
         # in the round-2 serving profile)
@@ -488,15 +488,10 @@ class LlamaModel:
                             self.hq_l, self.hkv_l, self.spec.head_dim)
             attn = ops.attn_decode(q, self.cache.k[li], self.cache.v[li],
                                    attn_seq, self.scale, slot_map=slot_map)
-            attn_out = _linear(attn.reshape(b, -1), lw.wo)
-            self.tp.all_reduce(attn_out)
-            normed, resid = ops.rmsnorm(attn_out, lw.mlp_norm, s.norm_eps,
-                                        residual=resid)
+            normed, resid = self._joined(attn.reshape(b, -1), lw.wo,
+                                         lw.mlp_norm, resid)
             act = self._mlp_act(normed, lw)
-            mlp_out = _linear(act, lw.wdown)
-            self.tp.all_reduce(mlp_out)
             next_norm = (self.layers[li + 1].attn_norm
                          if li + 1 < len(self.layers) else self.final_norm)
-            normed, resid = ops.rmsnorm(mlp_out, next_norm, s.norm_eps,
-                                        residual=resid)
+            normed, resid = self._joined(act, lw.wdown, next_norm, resid)
         return _linear(normed, self.lm_head).float()

@@ -16,6 +16,7 @@ from typing import Optional
 import torch
 import torch.nn.functional as F
 
+from gridllm_amd import ops
 from gridllm_amd.ops import hip_ops
 from gridllm_amd.ops.reference import SWIGLU, Glu
 from gridllm_amd.utils.logging import get_logger
@@ -154,17 +155,37 @@ def choice(m: int, n: int, k: int) -> Optional[tuple[str, int]]:
     return _CHOICE.get((m, n, k))
 
 
+def _choose(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple]:
+    """Choice for x @ w.T, None for what is not a GPU product of bf16 rows."""
+    if x.dim() != 2 or not x.is_cuda or x.dtype != torch.bfloat16:
+        return None
+    c = _CHOICE.get((x.shape[0], w.shape[0], w.shape[1]))
+    if c is None and not (torch.is_grad_enabled() and
+                          (x.requires_grad or w.requires_grad)):
+        c = _by_rule(x, w)
+    return c
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """Dispatch x @ w.T (GPU bf16 2-D x only) through the tuned table or by
     rule."""
-    if x.dim() == 2 and x.is_cuda and x.dtype == torch.bfloat16:
-        c = _CHOICE.get((x.shape[0], w.shape[0], w.shape[1]))
-        if c is None and not (torch.is_grad_enabled() and
-                              (x.requires_grad or w.requires_grad)):
-            c = _by_rule(x, w)
-        if c is not None:
-            return _run(c, x, w)
-    return F.linear(x, w)
+    c = _choose(x, w)
+    return F.linear(x, w) if c is None else _run(c, x, w)
+
+
+def linear_rmsnorm(x: torch.Tensor, w: torch.Tensor, weight: torch.Tensor,
+                   eps: float, residual: torch.Tensor
+                   ) -> tuple[torch.Tensor, torch.Tensor]:
+    """(rmsnorm(y) * weight, y) of y = x @ w.T + residual. A product with its K
+    in parts leaves adding them up to the norm."""
+    c = _choose(x, w)
+    if c is not None and c[0] == "tile" and c[3] > 1 and \
+            w.shape[1] > 64 and w.shape[0] % 8 == 0 and \
+            residual.dtype == weight.dtype == torch.bfloat16 and \
+            residual.is_contiguous() and weight.is_contiguous():
+        return hip_ops.gemm_tile_rmsnorm(x, w, *c[1:], weight, eps, residual)
+    y = F.linear(x, w) if c is None else _run(c, x, w)
+    return ops.rmsnorm(y, weight, eps, residual=residual)
 
 
 def tune_model_shapes(model, buckets) -> None:

@@ -39,6 +39,9 @@ def _load() -> ctypes.CDLL:
     c_vp, c_i, c_l, c_f = ctypes.c_void_p, ctypes.c_int, ctypes.c_long, ctypes.c_float
     lib.gl_rmsnorm.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_l, c_i, c_f]
     lib.gl_rmsnorm.restype = c_i
+    lib.gl_rmsnorm_parts.argtypes = [c_vp] * 3 + [c_i] + [c_vp] * 3 + [
+        c_i, c_i, c_f]
+    lib.gl_rmsnorm_parts.restype = c_i
     lib.gl_decode_positions.argtypes = [c_vp] * 8 + [c_i, c_i]
     lib.gl_decode_positions.restype = c_i
     lib.gl_prompt_positions.argtypes = [c_vp] * 5 + [c_i] * 4
@@ -487,6 +490,30 @@ def gemm_tile(x: torch.Tensor, w: torch.Tensor, rows: int, cols: int,
                             m, n, k, splitk, kslice, rows, cols,
                             1 if fuse_swiglu else 0, *glu), "gemm_tile")
     return out
+
+
+def gemm_tile_rmsnorm(x: torch.Tensor, w: torch.Tensor, rows: int, cols: int,
+                      splitk: int, weight: torch.Tensor, eps: float,
+                      residual: torch.Tensor
+                      ) -> tuple[torch.Tensor, torch.Tensor]:
+    """gemm_tile with K in parts and the rmsnorm behind it, which adds them up:
+    (rmsnorm(y) * weight, y) of y = x @ w^T + residual [M, N]."""
+    lib = _load()
+    m, k = x.shape
+    n = w.shape[0]
+    kslice = ((k + splitk - 1) // splitk + 63) // 64 * 64
+    splitk = (k + kslice - 1) // kslice
+    assert splitk > 1 and residual.shape == (m, n) and weight.shape == (n,)
+    assert residual.is_contiguous() and weight.is_contiguous()
+    ws = torch.empty(splitk, m, n, dtype=torch.float32, device=x.device)
+    _check(lib.gl_gemm_tile(_stream(), None, _ptr(ws), _ptr(x), _ptr(w), m, n,
+                            k, splitk, kslice, rows, cols, 0, *SWIGLU),
+           "gemm_tile")
+    y, total = torch.empty_like(residual), torch.empty_like(residual)
+    _check(lib.gl_rmsnorm_parts(_stream(), _ptr(y), _ptr(ws), splitk,
+                                _ptr(weight), _ptr(residual), _ptr(total), m,
+                                n, eps), "rmsnorm_parts")
+    return y, total
 
 
 def gemm_proj_supported(m: int, n: int, k: int) -> bool:

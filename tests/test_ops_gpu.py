@@ -612,6 +612,28 @@ def test_gemm_tile(dev, m, n, k, sk, fuse):
                     (rows, cols)
 
 
+@pytest.mark.parametrize("m,n,k,sk", [(1, 64, 128, 2), (24, 3072, 1024, 5),
+                                      (70, 2112, 576, 9), (3, 8256, 256, 2)])
+def test_gemm_tile_rmsnorm(dev, m, n, k, sk):
+    """Partial sums that the norm adds up: what the two steps give, to a rounding
+    of the sum where the parts' sum is taken in another order."""
+    from gridllm_amd import ops
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator().manual_seed(n)
+    x, w, r = (torch.randn(*s, generator=g).to(dev, torch.bfloat16)
+               for s in ((m, k), (n, k), (m, n)))
+    weight = (torch.rand(n, generator=g) + 0.5).to(dev, torch.bfloat16)
+    y, total = hip_ops.gemm_tile_rmsnorm(x, w, 64, 64, sk, weight, 1e-5, r)
+    want, res = ops.rmsnorm(hip_ops.gemm_tile(x, w, 64, 64, sk), weight, 1e-5,
+                            residual=r)
+    # (product, then its sum with the residual: one bf16 step, 2^-8, each)
+    size = res.float().abs() + x.float().norm(dim=1, keepdim=True) * 8
+    assert bool(((total.float() - res.float()).abs() <= 2 ** -7 * size).all())
+    assert float((total != res).float().mean()) < 0.01
+    assert bool(((y.float() - want.float()).abs() <=
+                 2 ** -6 * want.float().abs() + 2 ** -6).all())
+
+
 def test_gemm_tilings():
     """What the tuner tries is what the kernel takes."""
     from gridllm_amd.ops import hip_ops
