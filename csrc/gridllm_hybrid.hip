@@ -1069,7 +1069,6 @@ k_rec_row_out(T* __restrict__ out, const float* __restrict__ o,
 // m of the slot before the step, m_in}.
 // ---------------------------------------------------------------------------
 #define MCH 64
-#define MLD 72      // padded row of 64 tokens in LDS
 
 // Lightning attention (CONST) is the case i = 0, f the same for every token: m
 // then stays 0. It has no normaliser and no head norm; gr is f by head, f32
@@ -1104,6 +1103,112 @@ DEV_INLINE void chunk_scan(const float* gr, int tok0, int clen, int h, int H,
     }
 }
 
+// Places in LDS of 16-byte pieces c, swapped by the row so that 16 lanes' rows
+// do not meet in a bank: of 64 f32, of 64 bf16, and of `cols` bf16 that are read
+// transposed, where 4 rows' pairs of pieces have to lie apart.
+DEV_INLINE int at_f32(int row, int c) { return row * 64 + (c ^ (row & 15)) * 4; }
+DEV_INLINE int at_bf16(int row, int c) { return row * 64 + (c ^ (row & 7)) * 8; }
+DEV_INLINE int at_cols(int row, int c, int cols) {
+    return row * cols + (c ^ ((row & 3) << 1 | (row >> 2 & 1))) * 8;
+}
+
+// 64 tokens' values, up to 256 columns of them, on their way to LDS
+DEV_INLINE void load_values(bf16_t* vs, const bf16_t* v, long ld_, int last,
+                            int cols) {
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int i = 0; i < cols / 32; ++i) {
+        const int pc = i * 256 + threadIdx.x, row = pc / (cols / 8);
+        const int c = at_cols(row, pc % (cols / 8), cols) / 8 -
+                      row * (cols / 8);
+        load_lds16(v + min(row, last) * ld_ + c * 8,
+                   vs + (i * 256 + wid * 64) * 8);
+    }
+}
+
+// Values (16 columns from `col` on, as the products' rows) of 32 tokens.
+DEV_INLINE bf16x8 value_piece(const bf16_t* vs, int ks, int col, int cols) {
+    const int lane = threadIdx.x & 63, fr = lane & 15, gq = lane >> 4;
+    const int d = col + (fr & 3) * 4;
+    bf16x8 v;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int row = ks * 32 + gq * 8 + (fr >> 2) + j * 4;
+        const bf16x4 x =
+            read_transposed(vs + at_cols(row, d >> 3, cols) + (d & 7));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[j * 4 + i] = x[i];
+    }
+    return v;
+}
+
+// 16 weighted keys of a thread's token (tid / 4) as (hi, lo) pairs of bf16, in LDS
+// as load_values lays out 64 columns; w: their weights
+DEV_INLINE void store_keys(bf16_t* kh, bf16_t* kl, const bf16_t* k,
+                           const float* w) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        float f[8];
+        ld8(k + i * 8, f);
+        bf16x8 hi, lo;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float x = f[j] * w[i * 8 + j];
+            hi[j] = (__bf16)x;
+            lo[j] = (__bf16)(x - (float)hi[j]);
+        }
+        const int at = at_cols(threadIdx.x >> 2, (threadIdx.x & 3) * 2 + i, 64);
+        *(bf16x8*)(kh + at) = hi;
+        *(bf16x8*)(kl + at) = lo;
+    }
+}
+
+// Sum over 64 tokens of values times weighted keys, for 64 key channels and up
+// to 256 value columns, of which a wave has every fourth 16: D, f32 rows of DK.
+DEV_INLINE void store_state(float* D, const bf16_t* vs, const bf16_t* kh,
+                            const bf16_t* kl, int nv, int DK) {
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) acc[c][d] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        bf16x8 hi[4], lo[4];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            hi[d] = value_piece(kh, ks, d * 16, 64);
+            lo[d] = value_piece(kl, ks, d * 16, 64);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (c * 64 >= nv) continue;
+            const bf16x8 v = value_piece(vs, ks, c * 64 + wid * 16, nv);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                acc[c][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    hi[d], v, acc[c][d], 0, 0, 0);
+                acc[c][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    lo[d], v, acc[c][d], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        if (c * 64 >= nv) continue;
+        float* row = D + (long)(c * 64 + wid * 16 + (lane & 15)) * DK +
+                     (lane >> 4) * 4;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) *(f32x4*)(row + d * 16) = acc[c][d];
+    }
+}
+
+// A chunk's own contribution to the state. Block = (chunk, head, 64 key channels
+// and `cols` value columns, up to 256). Bound by writing it, 128 KB a head and
+// chunk of 128 x 256: 3500 tokens, 12 heads: 43 us with 64 columns a block,
+// operands transposed by 2-byte stores to LDS and results stored by 4 bytes,
+// now 35.
 template <bool CONST>
 __global__ void __launch_bounds__(256)
 k_mlstm_chunk_state(float* __restrict__ dS, float* __restrict__ scal,
@@ -1112,16 +1217,22 @@ k_mlstm_chunk_state(float* __restrict__ dS, float* __restrict__ scal,
                     const float* __restrict__ gr,
                     const int4* __restrict__ chunks,
                     const int4* __restrict__ segs, int H, int DK, int DV,
-                    int ld_, float cap) {
-    __shared__ __attribute__((aligned(16))) bf16_t vt[64 * MLD];
-    __shared__ __attribute__((aligned(16))) bf16_t kh[64 * MLD];
-    __shared__ __attribute__((aligned(16))) bf16_t kl[64 * MLD];
+                    int ld_, float cap, int cols) {
+    __shared__ __attribute__((aligned(16))) bf16_t vs[64 * 256];
+    __shared__ __attribute__((aligned(16))) bf16_t kh[64 * 64];
+    __shared__ __attribute__((aligned(16))) bf16_t kl[64 * 64];
     __shared__ float wgt[MCH];
     const int4 ch = chunks[blockIdx.x];
     const int h = blockIdx.y;
     const int nd = DK / 64;
-    const int d0 = (blockIdx.z % nd) * 64, v0 = (blockIdx.z / nd) * 64;
+    const int d0 = (blockIdx.z % nd) * 64, v0 = (blockIdx.z / nd) * cols;
+    const int nv = min(cols, DV - v0), last = ch.y - 1;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int t = threadIdx.x >> 2, c16 = (threadIdx.x & 3) * 16;
+    const bf16_t* row = qkv + (long)ch.x * ld_;
+    load_values(vs, row + 2l * H * DK + h * DV + v0, ld_, last, nv);
+    const bf16_t* kp = row + (long)min(t, last) * ld_ + (H + h) * DK + d0 + c16;
+    const uint4 kv[2] = {((const uint4*)kp)[0], ((const uint4*)kp)[1]};
     if (wid == 0) {
         float F, a, amax;
         chunk_scan<CONST>(gr, ch.x, ch.y, h, H, cap, F, a, amax);
@@ -1136,54 +1247,22 @@ k_mlstm_chunk_state(float* __restrict__ dS, float* __restrict__ scal,
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < 512; i += 256) {
-        const int t = i & 63, c8 = (i >> 6) * 8;   // a wave spans 64 tokens
-        const bf16_t* row = qkv + (long)(ch.x + min(t, ch.y - 1)) * ld_;
-        float f[8];
-        ld8(row + (H + h) * DK + d0 + c8, f);
-        const uint4 vv = *(const uint4*)(row + 2 * H * DK + h * DV + v0 + c8);
-        const bf16_t* pv = (const bf16_t*)&vv;
-        const float w = wgt[t];
+    float w[16];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float x = f[j] * w;
-            const bf16_t hi = f2bf(x);
-            kh[(c8 + j) * MLD + t] = hi;
-            kl[(c8 + j) * MLD + t] = f2bf(x - bf2f(hi));
-            vt[(c8 + j) * MLD + t] = pv[j];
-        }
-    }
-    __syncthreads();
+    for (int i = 0; i < 16; ++i) w[i] = wgt[t];
+    store_keys(kh, kl, (const bf16_t*)kv, w);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
     const int R = CONST ? DV : DV + 1;
-    float* Db = dS + ((long)blockIdx.x * H + h) * R * DK;
-    const int fr = lane & 15, kg = (lane >> 4) * 8;
-    f32x4 acc[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) acc[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-        const bf16x8 a =
-            *(const bf16x8*)(vt + (wid * 16 + fr) * MLD + ks * 32 + kg);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int at = (c * 16 + fr) * MLD + ks * 32 + kg;
-            acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                a, *(const bf16x8*)(kh + at), acc[c], 0, 0, 0);
-            acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                a, *(const bf16x8*)(kl + at), acc[c], 0, 0, 0);
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            Db[(long)(v0 + wid * 16 + (lane >> 4) * 4 + r) * DK + d0 + c * 16 +
-               fr] = acc[c][r];
+    float* Db = dS + ((long)blockIdx.x * H + h) * R * DK + d0;
+    store_state(Db + (long)v0 * DK, vs, kh, kl, nv, DK);
     if (!CONST && v0 == 0 && threadIdx.x < 64) {
         float s = 0.f;
-        for (int t = 0; t < MCH; ++t)
-            s += bf2f(kh[lane * MLD + t]) + bf2f(kl[lane * MLD + t]);
-        Db[(long)DV * DK + d0 + lane] = s;
+        for (int i = 0; i < MCH; ++i) {
+            const int at = at_cols(i, lane >> 3, 64) + (lane & 7);
+            s += bf2f(kh[at]) + bf2f(kl[at]);
+        }
+        Db[(long)DV * DK + lane] = s;
     }
 }
 
@@ -1247,44 +1326,6 @@ DEV_INLINE void split8(const u32* p, bf16x8& hi, bf16x8& lo) {
     a.w = (y.z & 0xffffu) | (y.w << 16);  b.w = (y.z >> 16) | (y.w & 0xffff0000u);
     hi = *(bf16x8*)&a;
     lo = *(bf16x8*)&b;
-}
-
-// Places in LDS of 16-byte pieces c, swapped by the row so that 16 lanes' rows
-// do not meet in a bank: of 64 f32, of 64 bf16, and of `cols` bf16 that are read
-// transposed, where 4 rows' pairs of pieces have to lie apart.
-DEV_INLINE int at_f32(int row, int c) { return row * 64 + (c ^ (row & 15)) * 4; }
-DEV_INLINE int at_bf16(int row, int c) { return row * 64 + (c ^ (row & 7)) * 8; }
-DEV_INLINE int at_cols(int row, int c, int cols) {
-    return row * cols + (c ^ ((row & 3) << 1 | (row >> 2 & 1))) * 8;
-}
-
-// 64 tokens' values, up to 256 columns of them, on their way to LDS
-DEV_INLINE void load_values(bf16_t* vs, const bf16_t* v, long ld_, int last,
-                            int cols) {
-    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    for (int i = 0; i < cols / 32; ++i) {
-        const int pc = i * 256 + threadIdx.x, row = pc / (cols / 8);
-        const int c = at_cols(row, pc % (cols / 8), cols) / 8 -
-                      row * (cols / 8);
-        load_lds16(v + min(row, last) * ld_ + c * 8,
-                   vs + (i * 256 + wid * 64) * 8);
-    }
-}
-
-// Values (16 columns from `col` on, as the products' rows) of 32 tokens.
-DEV_INLINE bf16x8 value_piece(const bf16_t* vs, int ks, int col, int cols) {
-    const int lane = threadIdx.x & 63, fr = lane & 15, gq = lane >> 4;
-    const int d = col + (fr & 3) * 4;
-    bf16x8 v;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int row = ks * 32 + gq * 8 + (fr >> 2) + j * 4;
-        const bf16x4 x =
-            read_transposed(vs + at_cols(row, d >> 3, cols) + (d & 7));
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[j * 4 + i] = x[i];
-    }
-    return v;
 }
 
 // Output gates of a chunk, for lane = 4 columns c * 64 + wid * 16 + gq * 4 + r of
@@ -1676,72 +1717,40 @@ DEV_INLINE void split_bf16(float x, bf16_t& hi, bf16_t& lo) {
     lo = f2bf(x - bf2f(hi));
 }
 
-// A chunk's own contribution to the state. Block = (chunk, head, 64 key
-// channels and every so many-th 64 value columns).
+// A chunk's own contribution to the state, in blocks as mLSTM's. (3050 tokens, 12
+// heads of 128 x 256: 33 us before, now 28.)
 __global__ void __launch_bounds__(256)
 k_gla_chunk_state(float* __restrict__ dS, const bf16_t* __restrict__ qkv,
                   const float* __restrict__ b, const int4* __restrict__ chunks,
-                  int H, int DK, int DV, int ld_) {
-    __shared__ __attribute__((aligned(16))) bf16_t vt[64 * MLD];
-    __shared__ __attribute__((aligned(16))) bf16_t kh[64 * MLD];
-    __shared__ __attribute__((aligned(16))) bf16_t kl[64 * MLD];
+                  int H, int DK, int DV, int ld_, int cols) {
+    __shared__ __attribute__((aligned(16))) bf16_t vs[64 * 256];
+    __shared__ __attribute__((aligned(16))) bf16_t kh[64 * 64];
+    __shared__ __attribute__((aligned(16))) bf16_t kl[64 * 64];
     const int4 ch = chunks[blockIdx.x];
-    const int h = blockIdx.y;
-    const int nd = DK / 64, nv = gridDim.z / nd;
-    const int d0 = (blockIdx.z % nd) * 64;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const float* bl = b + (long)(ch.x + ch.y - 1) * H * DK + h * DK + d0;
-    for (int i = threadIdx.x; i < 512; i += 256) {
-        const int t = i & 63, c8 = (i >> 6) * 8;   // a wave spans 64 tokens
-        const long n = ch.x + min(t, ch.y - 1);
-        const bf16_t* row = qkv + n * ld_;
-        float f[8], bt[8], bT[8];
-        ld8(row + (H + h) * DK + d0 + c8, f);
-        ld8(b + n * H * DK + h * DK + d0 + c8, bt);
-        ld8(bl + c8, bT);
+    const int h = blockIdx.y, nd = DK / 64, last = ch.y - 1;
+    const int d0 = (blockIdx.z % nd) * 64, v0 = (blockIdx.z / nd) * cols;
+    const int nv = min(cols, DV - v0);
+    const int t = threadIdx.x >> 2, c16 = (threadIdx.x & 3) * 16;
+    const bf16_t* row = qkv + (long)ch.x * ld_;
+    const long n = min(t, last);
+    const float* bt = b + (ch.x + n) * H * DK + h * DK + d0 + c16;
+    const float* bT = bt + (last - n) * H * DK;
+    float e[16], w[16];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float x = t < ch.y ? f[j] * __expf(bT[j] - bt[j]) : 0.f;
-            split_bf16(x, kh[(c8 + j) * MLD + t], kl[(c8 + j) * MLD + t]);
-        }
+    for (int i = 0; i < 16; i += 8) {
+        ld8(bt + i, e + i);
+        ld8(bT + i, w + i);
     }
-    float* Db = dS + ((long)blockIdx.x * H + h) * DV * DK;
-    const int fr = lane & 15, kg = (lane >> 4) * 8;
-    for (int v0 = blockIdx.z / nd * 64; v0 < DV; v0 += nv * 64) {
-        __syncthreads();                 // readers of the last columns are done
-        for (int i = threadIdx.x; i < 512; i += 256) {
-            const int t = i & 63, c8 = (i >> 6) * 8;
-            const uint4 vv = *(const uint4*)(
-                qkv + (long)(ch.x + min(t, ch.y - 1)) * ld_ + 2 * H * DK +
-                h * DV + v0 + c8);
-            const bf16_t* pv = (const bf16_t*)&vv;
+    const bf16_t* kp = row + n * ld_ + (H + h) * DK + d0 + c16;
+    const uint4 kv[2] = {((const uint4*)kp)[0], ((const uint4*)kp)[1]};
+    load_values(vs, row + 2l * H * DK + h * DV + v0, ld_, last, nv);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) vt[(c8 + j) * MLD + t] = pv[j];
-        }
-        __syncthreads();
-        f32x4 acc[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const bf16x8 a =
-                *(const bf16x8*)(vt + (wid * 16 + fr) * MLD + ks * 32 + kg);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int at = (c * 16 + fr) * MLD + ks * 32 + kg;
-                acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    a, *(const bf16x8*)(kh + at), acc[c], 0, 0, 0);
-                acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    a, *(const bf16x8*)(kl + at), acc[c], 0, 0, 0);
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                Db[(long)(v0 + wid * 16 + (lane >> 4) * 4 + r) * DK + d0 +
-                   c * 16 + fr] = acc[c][r];
-    }
+    for (int i = 0; i < 16; ++i) w[i] = t <= last ? __expf(w[i] - e[i]) : 0.f;
+    store_keys(kh, kl, (const bf16_t*)kv, w);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    store_state(dS + (((long)blockIdx.x * H + h) * DV + v0) * DK + d0, vs, kh,
+                kl, nv, DK);
 }
 
 // The state that enters each chunk, left in dS as (hi | lo << 16) bf16 pairs;
@@ -2918,6 +2927,10 @@ int gh_rec_row_out(void* stream, int f32, void* out, const void* o,
     return 0;
 }
 
+// Value columns of a block of a chunk's state. Few chunks: 64, so that there are
+// more blocks, though each takes the keys' weights again.
+static int state_columns(int items) { return items >= 256 ? 256 : 64; }
+
 // constant: lightning attention (gr: log decay by head; mst unused)
 int gh_mlstm_chunks(void* stream, int constant, void* o, void* out, void* S,
                     void* mst, void* dS, void* scal, const void* qkv,
@@ -2930,11 +2943,12 @@ int gh_mlstm_chunks(void* stream, int constant, void* o, void* out, void* S,
         return -100;
     hipStream_t st_ = (hipStream_t)stream;
     const long quads = (long)(DV + !constant) * DK / 4;
+    const int cols = state_columns(nchunks * H);
 #define GO(C) do { \
-    k_mlstm_chunk_state<C><<<dim3(nchunks, H, (DK / 64) * (DV / 64)), 256, 0, \
-        st_>>>((float*)dS, (float*)scal, (const float*)mst, \
+    k_mlstm_chunk_state<C><<<dim3(nchunks, H, \
+        DK / 64 * ((DV + cols - 1) / cols)), 256, 0, st_>>>((float*)dS, (float*)scal, (const float*)mst, \
         (const bf16_t*)qkv, (const float*)gr, (const int4*)chunks, \
-        (const int4*)segs, H, DK, DV, ld_, cap); \
+        (const int4*)segs, H, DK, DV, ld_, cap, cols); \
     LAUNCH_CHECK(); \
     k_mlstm_chunk_scan<C><<<dim3(nseg, H, (unsigned)((quads + 255) / 256)), \
         256, 0, st_>>>((float*)dS, (float*)scal, (float*)S, (float*)mst, \
@@ -2973,12 +2987,10 @@ int gh_gla_chunks(void* stream, void* o, void* out, void* S, void* dS,
     if (nchunks < 1 || nseg < 1 || DK % 64 || DV % 64 || (out && DV > 256))
         return -100;
     hipStream_t st_ = (hipStream_t)stream;
-    // few chunks: value columns in blocks of their own, though each then takes
-    // the decays again
-    const bool many = nchunks * H >= 512;
-    k_gla_chunk_state<<<dim3(nchunks, H, DK / 64 * (many ? 1 : DV / 64)), 256,
-                        0, st_>>>((float*)dS, (const bf16_t*)qkv,
-        (const float*)b, (const int4*)chunks, H, DK, DV, ld_);
+    const int cols = state_columns(nchunks * H);
+    k_gla_chunk_state<<<dim3(nchunks, H, DK / 64 * ((DV + cols - 1) / cols)),
+                        256, 0, st_>>>((float*)dS, (const bf16_t*)qkv,
+        (const float*)b, (const int4*)chunks, H, DK, DV, ld_, cols);
     LAUNCH_CHECK();
     const long quads = (long)DV * DK / 4;
     k_gla_chunk_scan<<<dim3(nseg, H, (unsigned)((quads + 255) / 256)), 256, 0,
