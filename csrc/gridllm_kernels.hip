@@ -639,7 +639,9 @@ k_gemm_rows(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
 // lines in its L2; those of other rows and the same columns follow each other.
 //   EPI 1: W rows in groups of 64 gate | 64 up; a block takes CT * 8 of each and
 //   stores the gated unit [M, N / 2].
-//   splitk > 1: f32 partials [splitk][M][N] in ws.
+//   splitk > 1: f32 partials [splitk][M][N] in ws. out == null otherwise: the
+//   result, rounded to bf16, as f32 in ws (a vocabulary's scores: 256 rows of
+//   128256 took 30 us to be widened behind it).
 // Constraints: N % (16 CT) == 0 (128 for EPI 1), K % 64 == 0, kslice % 64 == 0.
 //
 // Bound by a CU's loads: those of x, which hit in L2, and of W queue up behind
@@ -821,8 +823,9 @@ k_gemm_tile(bf16_t* __restrict__ out, float* __restrict__ ws,
             const int n = w_row(col_tile(b) * 16) + gq * 4;
             float f[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) f[r] = acc[a][b][r];
-            if (splitk == 1) st4(out + (long)m * N + n, f);
+            for (int r = 0; r < 4; ++r)
+                f[r] = splitk == 1 ? bf2f(f2bf(acc[a][b][r])) : acc[a][b][r];
+            if (splitk == 1 && out) st4(out + (long)m * N + n, f);
             else st4(ws + ((long)ks * M + m) * N + n, f);
         }
     }
@@ -1376,7 +1379,7 @@ int gl_gemm_tile(void* stream, void* out, void* ws, const void* x,
     if (M < 1 || K < 1 || K % 64 || kslice < 64 || kslice % 64 || N < 1 ||
         cols < 1 || N % cols || (fuse_swiglu && N % 128) || splitk < 1 ||
         (long)(splitk - 1) * kslice >= K || (long)splitk * kslice < K ||
-        (splitk > 1 && !ws) || (splitk == 1 && !out)) return -100;
+        (splitk > 1 && !ws) || (!out && (!ws || fuse_swiglu))) return -100;
     hipStream_t st = (hipStream_t)stream;
     int e = -103;
 #define GO(RT, CT, EPI) \
@@ -1388,7 +1391,7 @@ int gl_gemm_tile(void* stream, void* out, void* ws, const void* x,
     COLS(2); COLS(4); COLS(6); COLS(8); COLS(10); COLS(12); COLS(16);
 #undef COLS
 #undef GO
-    if (e || splitk == 1 || !out) return e;    // (no out: partials are wanted)
+    if (e || splitk == 1 || !out) return e;    // (no out: ws is wanted)
     const long quads = (long)M * (fuse_swiglu ? N >> 3 : N >> 2);
     const int grid = (int)min((quads + 255) / 256, (long)2048);
     if (fuse_swiglu)

@@ -36,6 +36,7 @@ from gridllm_amd.models.registry import (AttentionMixer, DenseFF, GlaMixer,
                                          Rotary, RoutedFF, TalkingMixer)
 from gridllm_amd.ops import hybrid as hops
 from gridllm_amd.ops.autotune import linear as _linear
+from gridllm_amd.ops.autotune import linear_f32 as _linear_f32
 from gridllm_amd.ops.autotune import linear_gateup as _linear_gateup
 from gridllm_amd.ops.hybrid import (ChunkPortions, Choice, DepthAverage, Keys,
                                     StepMeta, Talk)
@@ -813,8 +814,7 @@ class HybridModel:
 
     def _head(self, x: torch.Tensor, rows: Optional[torch.Tensor]
               ) -> torch.Tensor:
-        return _linear(self._normed(x, rows, self.head_norm),
-                       self.head).float()
+        return _linear_f32(self._normed(x, rows, self.head_norm), self.head)
 
     # -- steps -------------------------------------------------------------
 

@@ -28,6 +28,7 @@ import torch
 import torch.nn.functional as F  # noqa: F401
 
 from gridllm_amd.ops.autotune import linear as _linear
+from gridllm_amd.ops.autotune import linear_f32 as _linear_f32
 from gridllm_amd.ops.autotune import linear_gateup as _linear_gateup
 from gridllm_amd.ops.autotune import linear_rmsnorm as _linear_rmsnorm
 
@@ -381,7 +382,7 @@ class LlamaModel:
             next_norm = (self.layers[li + 1].attn_norm
                          if li + 1 < len(self.layers) else self.final_norm)
             normed, resid = self._joined(act, lw.wdown, next_norm, resid)
-        logits = _linear(normed[-1:], self.lm_head).float()
+        logits = _linear_f32(normed[-1:], self.lm_head)
         if return_hidden:
             return logits[0], normed.float().mean(dim=0)
         return logits[0]
@@ -457,7 +458,7 @@ class LlamaModel:
         # fresh slots start unshifted (alloc no longer touches the device)
         self.cache.rope_off.index_fill_(0, dev3[0], 0)
         lasts = dev3[2]
-        logits = _linear(normed[lasts], self.lm_head).float()
+        logits = _linear_f32(normed[lasts], self.lm_head)
         if return_hidden:
             hidden = torch.stack([
                 normed[bounds[i]:bounds[i + 1]].float().mean(dim=0)
@@ -494,4 +495,4 @@ class LlamaModel:
             next_norm = (self.layers[li + 1].attn_norm
                          if li + 1 < len(self.layers) else self.final_norm)
             normed, resid = self._joined(act, lw.wdown, next_norm, resid)
-        return _linear(normed, self.lm_head).float()
+        return _linear_f32(normed, self.lm_head)

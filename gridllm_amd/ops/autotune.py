@@ -81,6 +81,12 @@ def _run(c: tuple, x: torch.Tensor, w: torch.Tensor,
     return hip_ops.swiglu_il(out, glu=unit) if fuse else out
 
 
+def _run_f32(c: tuple, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    if c[0] == "tile" and c[3] == 1:
+        return hip_ops.gemm_tile_f32(x, w, *c[1:3])
+    return _run(c, x, w).float()
+
+
 def _by_rule(x: torch.Tensor, w: torch.Tensor, fuse: bool = False) -> tuple:
     """The choice for a shape that was not timed. gemm_rows has no second kernel,
     but every block reads all of x: it is the faster one for w of up to 20 MB
@@ -102,12 +108,17 @@ def _by_rule(x: torch.Tensor, w: torch.Tensor, fuse: bool = False) -> tuple:
     return ("blas",)
 
 
-def _tune(x: torch.Tensor, n: int, glu: Optional[Glu] = None) -> tuple:
-    """The fastest for x and a weight of n rows."""
+def _tune(x: torch.Tensor, n: int, glu: Optional[Glu] = None,
+          f32: bool = False) -> tuple:
+    """The fastest for x and a weight of n rows; f32: with a result of that."""
     m, k = x.shape
     ws = _weights(n, k, x.device)
+
+    def time_of(c: tuple) -> float:
+        return _time_fn(lambda w: _run_f32(c, x, w) if f32 else
+                        _run(c, x, w, glu), ws)
     best: tuple = ("blas",)
-    t_best = _time_fn(lambda w: _run(best, x, w, glu), ws)
+    t_best = time_of(best)
     tried: list[tuple] = [("tile", *t) for t in hip_ops.gemm_tilings(
         m, n, k, glu is not None)]
     if hip_ops.gemm_rows_supported(x, ws[0], glu is not None):
@@ -116,18 +127,18 @@ def _tune(x: torch.Tensor, n: int, glu: Optional[Glu] = None) -> tuple:
         tried = [("ours", sk) for sk in _SPLITK_CANDIDATES
                  if sk <= max(1, k // 256)]
     for c in tried:
-        t = _time_fn(lambda w: _run(c, x, w, glu), ws)
+        t = time_of(c)
         if t < t_best * 0.97:               # require a real margin
             t_best = t
             best = c
     return best
 
 
-def tune_shape(m: int, n: int, k: int, device) -> tuple:
+def tune_shape(m: int, n: int, k: int, device, f32: bool = False) -> tuple:
     key = (m, n, k)
     if key not in _CHOICE:
         x = torch.randn(m, k, device=device).to(torch.bfloat16) * 0.1
-        _CHOICE[key] = _tune(x, n)
+        _CHOICE[key] = _tune(x, n, f32=f32)
     return _CHOICE[key]
 
 
@@ -173,6 +184,12 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return F.linear(x, w) if c is None else _run(c, x, w)
 
 
+def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """linear(x, w).float(): a vocabulary's scores."""
+    c = _choose(x, w)
+    return F.linear(x, w).float() if c is None else _run_f32(c, x, w)
+
+
 def linear_rmsnorm(x: torch.Tensor, w: torch.Tensor, weight: torch.Tensor,
                    eps: float, residual: torch.Tensor
                    ) -> tuple[torch.Tensor, torch.Tensor]:
@@ -194,8 +211,8 @@ def tune_model_shapes(model, buckets) -> None:
     shapes, gu_shapes = model.gemm_shapes()
     t0 = time.monotonic()
     for m in buckets:
-        for n, k in shapes:
-            tune_shape(m, n, k, model.device)
+        for n, k in shapes:             # (the vocabulary's scores are f32)
+            tune_shape(m, n, k, model.device, n == model.spec.vocab)
         for n, k in gu_shapes:
             if getattr(model, "gateup_il", False):
                 tune_gateup(m, n, k, model.device)

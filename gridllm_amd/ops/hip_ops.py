@@ -492,6 +492,19 @@ def gemm_tile(x: torch.Tensor, w: torch.Tensor, rows: int, cols: int,
     return out
 
 
+def gemm_tile_f32(x: torch.Tensor, w: torch.Tensor, rows: int,
+                  cols: int) -> torch.Tensor:
+    """gemm_tile(...).float(), K in one part, without the bf16 copy."""
+    lib = _load()
+    m, k = x.shape
+    n = w.shape[0]
+    out = torch.empty(m, n, dtype=torch.float32, device=x.device)
+    _check(lib.gl_gemm_tile(_stream(), None, _ptr(out), _ptr(x), _ptr(w), m, n,
+                            k, 1, (k + 63) // 64 * 64, rows, cols, 0,
+                            *SWIGLU), "gemm_tile")
+    return out
+
+
 def gemm_tile_rmsnorm(x: torch.Tensor, w: torch.Tensor, rows: int, cols: int,
                       splitk: int, weight: torch.Tensor, eps: float,
                       residual: torch.Tensor

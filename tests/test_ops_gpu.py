@@ -612,6 +612,20 @@ def test_gemm_tile(dev, m, n, k, sk, fuse):
                     (rows, cols)
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 64, 64), (33, 192, 576),
+                                   (257, 8256, 128)])
+def test_gemm_tile_f32(dev, m, n, k):
+    """The result as f32 is that of bf16, widened, to the bit."""
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator().manual_seed(n)
+    x, w = (torch.randn(*s, generator=g).to(dev, torch.bfloat16)
+            for s in ((m, k), (n, k)))
+    for cols in (64, 96):
+        if n % cols == 0:
+            assert torch.equal(hip_ops.gemm_tile_f32(x, w, 64, cols),
+                               hip_ops.gemm_tile(x, w, 64, cols).float())
+
+
 @pytest.mark.parametrize("m,n,k,sk", [(1, 64, 128, 2), (24, 3072, 1024, 5),
                                       (70, 2112, 576, 9), (3, 8256, 256, 2)])
 def test_gemm_tile_rmsnorm(dev, m, n, k, sk):
