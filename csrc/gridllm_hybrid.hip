@@ -101,10 +101,31 @@ DEV_INLINE void sublayer8(const T* y, const float* wt, int top, long n, int W,
     }
 }
 
-template <class T, bool MOE>
+// 8 columns of a sublayer's output that is still f32 partial sums [parts][N][W]
+// of its last product (K in parts): added up, and rounded as the product's result
+// would be. Spares that product's second launch.
+DEV_INLINE void summed8(const float* y, int parts, long n, long N, int W, int c,
+                        float* v) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = 0.f;
+#pragma unroll 4
+    for (int k = 0; k < parts; ++k) {
+        float f[8];
+        ld8(y + (k * N + n) * W + c, f);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] += f[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = bf2f(f2bf(v[i]));
+}
+
+// What y is: a sublayer's output, a row per (token, expert), or partial sums
+enum { PLAIN, PAIRS, PARTS };
+
+template <class T, int KIND>
 __global__ void __launch_bounds__(256)
 k_post_norm(float* __restrict__ x, T* __restrict__ xb,
-            const T* __restrict__ y, const float* __restrict__ wt, int top,
+            const void* __restrict__ y, const float* __restrict__ wt, int top,
             const float* __restrict__ w, float w_off, int W, int Wtrue,
             float eps) {
     __shared__ float red[4];
@@ -115,7 +136,11 @@ k_post_norm(float* __restrict__ x, T* __restrict__ xb,
     for (int j = 0; j < 4; ++j) {
         const int c = (j * 256 + threadIdx.x) * 8;
         if (c < W) {
-            sublayer8<T, MOE>(y, wt, top, n, W, c, v[j]);
+            if (KIND == PARTS)
+                summed8((const float*)y, top, n, gridDim.x, W, c, v[j]);
+            else
+                sublayer8<T, KIND == PAIRS>((const T*)y, wt, top, n, W, c,
+                                            v[j]);
 #pragma unroll
             for (int i = 0; i < 8; ++i) ss += v[j][i] * v[j][i];
         }
@@ -285,10 +310,12 @@ DEV_INLINE void scale_groups(float* f, const float* rs, int c,
     }
 }
 
+// parts > 0: y is f32 partial sums
 template <class T, bool ADD, int GR>
 __global__ void __launch_bounds__(256)
 k_group_norm(T* __restrict__ out, float* __restrict__ x,
-             const T* __restrict__ y, const int* __restrict__ rows,
+             const void* __restrict__ y, int parts,
+             const int* __restrict__ rows,
              const float* __restrict__ wy, const float* __restrict__ w, int W,
              const Groups gp, float eps) {
     extern __shared__ float part[];        // W / GR, then a factor per group
@@ -300,7 +327,12 @@ k_group_norm(T* __restrict__ out, float* __restrict__ x,
         const int c = (j * 256 + threadIdx.x) * 8;
         if (c < W) {
             ld8(x + n * W + c, a[j]);
-            if (ADD) ld8(y + n * W + c, v[j]);
+            if (ADD) {
+                if (parts)
+                    summed8((const float*)y, parts, n, gridDim.x, W, c, v[j]);
+                else
+                    ld8((const T*)y + n * W + c, v[j]);
+            }
         }
     }
     if (ADD) {
@@ -2608,11 +2640,23 @@ int gh_post_norm(void* stream, int f32, void* x, void* xb, const void* y,
                  int W, int Wtrue, float eps) {
     if (W % 64 || W > 8192 || N < 1) return -100;
     hipStream_t st_ = (hipStream_t)stream;
-#define GO(T, M) k_post_norm<T, M><<<N, 256, 0, st_>>>((float*)x, (T*)xb, \
-        (const T*)y, (const float*)wt, top, (const float*)w, w_off, W, Wtrue, \
-        eps)
-    if (f32) { if (wt) GO(float, true); else GO(float, false); }
-    else { if (wt) GO(bf16_t, true); else GO(bf16_t, false); }
+#define GO(T, M) k_post_norm<T, M><<<N, 256, 0, st_>>>((float*)x, (T*)xb, y, \
+        (const float*)wt, top, (const float*)w, w_off, W, Wtrue, eps)
+    if (f32) { if (wt) GO(float, PAIRS); else GO(float, PLAIN); }
+    else { if (wt) GO(bf16_t, PAIRS); else GO(bf16_t, PLAIN); }
+    LAUNCH_CHECK();
+    return 0;
+}
+
+// y: f32 partial sums [parts][N][W]
+int gh_post_norm_parts(void* stream, void* x, void* xb, const void* y,
+                       int parts, const void* w, float w_off, int N, int W,
+                       int Wtrue, float eps) {
+    if (W % 64 || W > 8192 || N < 1 || parts < 1) return -100;
+    hipStream_t st_ = (hipStream_t)stream;
+    const void* wt = nullptr;
+    const int top = parts;
+    GO(bf16_t, PARTS);
 #undef GO
     LAUNCH_CHECK();
     return 0;
@@ -2634,16 +2678,16 @@ int gh_norm_rows(void* stream, int f32, void* out, const void* x,
 }
 
 int gh_group_norm(void* stream, int f32, void* out, void* x, const void* y,
-                  const void* rows, const void* wy, const void* w, int N,
-                  int W, int groups, int size, float eps) {
-    if (N < 1 || W % 8 || W > 8192 || groups < 1 || size < 1 ||
+                  int parts, const void* rows, const void* wy, const void* w,
+                  int N, int W, int groups, int size, float eps) {
+    if (parts < 0 || (parts && (f32 || !y)) || N < 1 || W % 8 || W > 8192 || groups < 1 || size < 1 ||
         (long)groups * size > W || (!y && !out) || (y && rows)) return -100;
     const int gr = size % 8 == 0 ? 8 : size % 4 == 0 ? 4 : size % 2 ? 1 : 2;
     const int lds = (W / gr + groups) * 4;
     if (lds > 64 * 1024) return -100;
     const Groups gp{groups, size};
 #define GO(T, A, B) k_group_norm<T, A, B><<<N, 256, lds, \
-        (hipStream_t)stream>>>((T*)out, (float*)x, (const T*)y, \
+        (hipStream_t)stream>>>((T*)out, (float*)x, y, parts, \
         (const int*)rows, (const float*)wy, (const float*)w, W, gp, eps)
 #define PICK(T, A) do { if (gr == 8) GO(T, A, 8); else if (gr == 4) \
         GO(T, A, 4); else if (gr == 2) GO(T, A, 2); else GO(T, A, 1); \

@@ -38,6 +38,7 @@ from gridllm_amd.ops import hybrid as hops
 from gridllm_amd.ops.autotune import linear as _linear
 from gridllm_amd.ops.autotune import linear_f32 as _linear_f32
 from gridllm_amd.ops.autotune import linear_gateup as _linear_gateup
+from gridllm_amd.ops.autotune import linear_parts as _linear_parts
 from gridllm_amd.ops.hybrid import (ChunkPortions, Choice, DepthAverage, Keys,
                                     StepMeta, Talk)
 from gridllm_amd.ops.reference import SWIGLU, Glu
@@ -607,6 +608,13 @@ class HybridModel:
 
     # -- layers ------------------------------------------------------------
 
+    def _joined(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+        """A sublayer's last projection: its partial sums, where the norm behind
+        it is a kernel that adds them up."""
+        s = self.spec
+        adds = s.pre_norms or (not s.streams and s.post_alpha is None)
+        return (_linear_parts if adds else _linear)(x, w)
+
     def _mix(self, i: int, w: BlockWeights, mx, xb: torch.Tensor,
              st: StepMeta) -> torch.Tensor:
         c, eps = self.cache, self.spec.norm_eps
@@ -647,7 +655,7 @@ class HybridModel:
             gates = hops.proj_f32(xb, w.wgates, w.bgates)
             o = hops.mlstm(rows, gates, c.S[i], c.m[i], w.mnorm, st, mx.dim,
                            mx.vdim, mx.gate_cap, eps)
-        return _linear(o, w.wo)
+        return self._joined(o, w.wo)
 
     def _attend(self, i: int, w: BlockWeights, mx: AttentionMixer,
                 rows: torch.Tensor, st: StepMeta, out: torch.Tensor,
@@ -683,11 +691,11 @@ class HybridModel:
         expert), the pairs' weights and those of identity experts; with weighted
         inputs the rows just add up."""
         if isinstance(ff, DenseFF):
-            return _linear(self._gated(w, ff, xb), w.down), None, None
+            return self._joined(self._gated(w, ff, xb), w.down), None, None
         if isinstance(ff, PolyFF):
             z = hops.poly_norm(_linear(xb, w.up), w.act, ff.ff,
                                self.spec.norm_eps)
-            return _linear(z, w.down), None, None
+            return self._joined(z, w.down), None, None
         assert isinstance(ff, RoutedFF)
         return hops.moe(xb, hops.proj_f32(xb, w.router), w.up, w.down,
                         self._choice(w, ff))

@@ -190,6 +190,15 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return F.linear(x, w).float() if c is None else _run_f32(c, x, w)
 
 
+def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """linear(x, w), or its f32 partial sums [parts, M, N] if K is in parts, for
+    post_norm and join_norm."""
+    c = _choose(x, w)
+    if c is not None and c[0] == "tile" and c[3] > 1 and w.shape[1] > 64:
+        return hip_ops.gemm_tile_parts(x, w, *c[1:])
+    return F.linear(x, w) if c is None else _run(c, x, w)
+
+
 def linear_rmsnorm(x: torch.Tensor, w: torch.Tensor, weight: torch.Tensor,
                    eps: float, residual: torch.Tensor
                    ) -> tuple[torch.Tensor, torch.Tensor]:

@@ -35,9 +35,10 @@ LOG2E = 1.4426950408889634
 _SIGS = {
     "gh_embed": "ipppppppfiiifii",
     "gh_post_norm": "ippppipfiiif",
+    "gh_post_norm_parts": "pppipfiiif",
     "gh_sum_norm": "ipppppippffppiiiiif",
     "gh_norm_rows": "ippppfiiif",
-    "gh_group_norm": "ippppppiiiif",
+    "gh_group_norm": "ipppipppiiiif",
     "gh_poly_norm": "ipppiiif",
     "gh_glu_f32": "ppliffff",
     "gh_proj_f32": "ppppiii",
@@ -153,8 +154,16 @@ def post_norm(x: torch.Tensor, xb: torch.Tensor, y: torch.Tensor,
               w: torch.Tensor, w_off: float, width: int, eps: float,
               pair_w: Optional[torch.Tensor] = None) -> None:
     """x += norm(y), in place, and xb = x in its type. With pair_w [n, top],
-    y [n * top, W] is first summed over a token's pairs by these weights."""
+    y [n * top, W] is first summed over a token's pairs by these weights; f32 y
+    [parts, n, W] over the parts."""
     n, wp = x.shape
+    if y.dim() == 3:
+        _dense(x, xb, y, w)
+        assert y.shape[1:] == x.shape and w.shape == (wp,) and not _f32(xb)
+        assert pair_w is None and _f32(y)
+        _call("gh_post_norm_parts", x, xb, y, y.shape[0], w, w_off, n, wp,
+              width, eps)
+        return
     top = 0 if pair_w is None else pair_w.shape[1]
     _dense(x, xb, y, w, pair_w)
     assert y.shape == (n * max(1, top), wp) and w.shape == (wp,)
@@ -212,7 +221,7 @@ def group_norm(x: torch.Tensor, rows: Optional[torch.Tensor], w: torch.Tensor,
     if rows is not None:
         _check_range("group_norm.rows", rows, x.shape[0])
     out = torch.empty(m, x.shape[1], dtype=dtype, device=x.device)
-    _call("gh_group_norm", _f32(out), out, x, None, rows, None, w, m,
+    _call("gh_group_norm", _f32(out), out, x, None, 0, rows, None, w, m,
           x.shape[1], groups, width // groups, eps)
     return out
 
@@ -221,13 +230,18 @@ def join_norm(x: torch.Tensor, y: torch.Tensor, wy: torch.Tensor,
               w: Optional[torch.Tensor], groups: int, width: int,
               eps: float) -> Optional[torch.Tensor]:
     """x += norm(y) * wy, in place; then norm(x) * w in y's type, if there is a
-    w. Norms as in group_norm."""
+    w. Norms as in group_norm. f32 y [parts, n, W] is a bf16 product's partial
+    sums."""
     n, wp = x.shape
+    parts = y.shape[0] if y.dim() == 3 else 0
     _dense(x, y, wy, w)
-    assert y.shape == x.shape and wy.shape == (wp,) and width % groups == 0
-    out = None if w is None else torch.empty_like(y)
-    _call("gh_group_norm", _f32(y), out, x, y, None, wy, w, n, wp, groups,
-          width // groups, eps)
+    assert y.shape[-2:] == x.shape and wy.shape == (wp,) and \
+        width % groups == 0 and (not parts or _f32(y))
+    dtype = torch.bfloat16 if parts else y.dtype
+    out = None if w is None else torch.empty(n, wp, dtype=dtype,
+                                             device=y.device)
+    _call("gh_group_norm", dtype == torch.float32, out, x, y, parts, None, wy,
+          w, n, wp, groups, width // groups, eps)
     return out
 
 

@@ -505,27 +505,37 @@ def gemm_tile_f32(x: torch.Tensor, w: torch.Tensor, rows: int,
     return out
 
 
+def gemm_tile_parts(x: torch.Tensor, w: torch.Tensor, rows: int, cols: int,
+                    splitk: int) -> torch.Tensor:
+    """gemm_tile's partial sums, f32 [parts, M, N], for a kernel that adds them
+    up itself (and rounds their sum to bf16)."""
+    lib = _load()
+    m, k = x.shape
+    n = w.shape[0]
+    kslice = ((k + splitk - 1) // splitk + 63) // 64 * 64
+    splitk = (k + kslice - 1) // kslice
+    assert splitk > 1
+    ws = torch.empty(splitk, m, n, dtype=torch.float32, device=x.device)
+    _check(lib.gl_gemm_tile(_stream(), None, _ptr(ws), _ptr(x), _ptr(w), m, n,
+                            k, splitk, kslice, rows, cols, 0, *SWIGLU),
+           "gemm_tile")
+    return ws
+
+
 def gemm_tile_rmsnorm(x: torch.Tensor, w: torch.Tensor, rows: int, cols: int,
                       splitk: int, weight: torch.Tensor, eps: float,
                       residual: torch.Tensor
                       ) -> tuple[torch.Tensor, torch.Tensor]:
     """gemm_tile with K in parts and the rmsnorm behind it, which adds them up:
     (rmsnorm(y) * weight, y) of y = x @ w^T + residual [M, N]."""
-    lib = _load()
-    m, k = x.shape
-    n = w.shape[0]
-    kslice = ((k + splitk - 1) // splitk + 63) // 64 * 64
-    splitk = (k + kslice - 1) // kslice
-    assert splitk > 1 and residual.shape == (m, n) and weight.shape == (n,)
+    m, n = x.shape[0], w.shape[0]
+    assert residual.shape == (m, n) and weight.shape == (n,)
     assert residual.is_contiguous() and weight.is_contiguous()
-    ws = torch.empty(splitk, m, n, dtype=torch.float32, device=x.device)
-    _check(lib.gl_gemm_tile(_stream(), None, _ptr(ws), _ptr(x), _ptr(w), m, n,
-                            k, splitk, kslice, rows, cols, 0, *SWIGLU),
-           "gemm_tile")
+    ws = gemm_tile_parts(x, w, rows, cols, splitk)
     y, total = torch.empty_like(residual), torch.empty_like(residual)
-    _check(lib.gl_rmsnorm_parts(_stream(), _ptr(y), _ptr(ws), splitk,
-                                _ptr(weight), _ptr(residual), _ptr(total), m,
-                                n, eps), "rmsnorm_parts")
+    _check(_load().gl_rmsnorm_parts(
+        _stream(), _ptr(y), _ptr(ws), ws.shape[0], _ptr(weight),
+        _ptr(residual), _ptr(total), m, n, eps), "rmsnorm_parts")
     return y, total
 
 

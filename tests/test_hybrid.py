@@ -739,3 +739,28 @@ def test_mlstm_chunk_sizes(dk, dv):
     assert float((S1.cpu()[used] - S0[used]).abs().max()) < \
         2 ** -11 * float(S0.abs().max())
     assert float((m1.cpu()[used] - m0[used]).abs().max()) < 1e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,w,parts,size", [(1, 64, 2, 8), (24, 3072, 5, 384),
+                                            (3, 1088, 9, 4)])
+def test_norms_add_parts(n, w, parts, size):
+    """Partial sums against the sum that a product would have stored."""
+    g = torch.Generator().manual_seed(w)
+    y = torch.randn(parts, n, w, generator=g).cuda()
+    whole = torch.zeros_like(y[0])
+    for part in y:                     # in the kernels' order
+        whole = whole + part
+    whole = whole.to(torch.bfloat16)
+    x = torch.randn(n, w, generator=g).cuda()
+    a, b = (torch.rand(w, generator=g).cuda() for _ in range(2))
+    x0, x1 = x.clone(), x.clone()
+    b0, b1 = (torch.empty(n, w, dtype=torch.bfloat16, device="cuda")
+              for _ in range(2))
+    hops.post_norm(x0, b0, whole, a, 1.0, w, 1e-5)
+    hops.post_norm(x1, b1, y, a, 1.0, w, 1e-5)
+    assert torch.equal(x0, x1) and torch.equal(b0, b1)
+    x0, x1 = x.clone(), x.clone()
+    h0 = hops.join_norm(x0, whole, a, b, w // size, w, 1e-5)
+    h1 = hops.join_norm(x1, y, a, b, w // size, w, 1e-5)
+    assert torch.equal(x0, x1) and torch.equal(h0, h1)
