@@ -951,10 +951,9 @@ k_attn_prefill(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
 //   meta[tile] = {q_off, len, slot, q0}: a tile is rows
 //   [q0, q0+128) of the sequence packed at q_off in q/out, against KV slot
 //   `slot` with s_total = len, causal_off = 0.
-// Motivation (round-2 serving profile, lt_worker_batcher.prof): admission
-// batches ran attention per-sequence per-layer from Python — 52k host
-// launches, 36 ms per 32-prompt admission. One meta-driven launch per
-// layer removes the Python loop and fills the chip (ntiles * Hq blocks).
+// Motivation: admission batches ran attention per sequence and layer from
+// Python — 52k host launches, 36 ms per 32-prompt admission. One meta-driven
+// launch per layer removes the loop and fills the chip (ntiles * Hq blocks).
 // ===========================================================================
 template <int D>
 __global__ void __launch_bounds__(256, 2)

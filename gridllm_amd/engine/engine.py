@@ -215,7 +215,7 @@ class InferenceEngine:
         g = torch.cuda.CUDAGraph()
         # ONE shared memory pool for every bucket graph: private per-graph
         # pools totalled 49.7 GB at max_batch 1536 (23 buckets) and OOM'd
-        # the 288 GB card (gpurun_out/r02n_serving_c1536.log). Sharing is
+        # the 288 GB card. Sharing is
         # safe under the capture-largest-first discipline (engine init
         # captures descending; a replay never outgrows the pool's high-
         # water mark set by the largest capture).

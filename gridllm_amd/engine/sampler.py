@@ -275,8 +275,7 @@ def sample_batch_vectorized(logits: torch.Tensor,
             logits[ii, tt] = vals
     if (logits.is_cuda and not plan.need_filter
             and os.environ.get("GRIDLLM_FUSED_SAMPLER", "1") != "0"):
-        # DEFAULT ON (hardware-validated round 2: test green on MI355X,
-        # serving +6% — gpurun_out/r02_lt_c192_fused.log): one HIP launch
+        # DEFAULT ON (serving +6% on MI355X): one HIP launch
         # replacing the ~15-op eager chain below; same RNG contract
         # (csrc k_sample_gumbel docstring). Greedy rows ride along with
         # key==0. GRIDLLM_FUSED_SAMPLER=0 restores the eager chain.

@@ -20,7 +20,7 @@ def _pseudo_word(tid: int) -> str:
     tokenizers decode every non-special id to text; mapping the synthetic
     vocab's unassigned ids (258..V) to "" made 99.8% of sampled tokens
     invisible on a random-init model — streaming looked silent and TTFT
-    was unmeasurable (gpurun_out/r02ab traces). Memoized: this runs on
+    was unmeasurable. Memoized: this runs on
     the batcher thread once per generated token."""
     w = _PSEUDO_CACHE.get(tid)
     if w is None:

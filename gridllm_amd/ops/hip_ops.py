@@ -104,11 +104,10 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
-# Debug validation (the sanitizer analog for a ctypes-bound kernel layer,
-# SURVEY.md §5.2): GRIDLLM_VALIDATE=1 makes every wrapper range-check its
-# index tensors BEFORE launching — a device sync per call, debug only.
-# (A slot_t overflow of exactly the kind this catches cost a GPU box:
-# the bucket>=max_seq graph-warmup fault.)
+# Debug validation (the sanitizer analog for a ctypes-bound kernel layer):
+# GRIDLLM_VALIDATE=1 makes every wrapper range-check its index tensors BEFORE
+# launching — a device sync per call, debug only. (It catches a slot_t that
+# overflows, as a graph's warm-up at bucket >= max_seq once did.)
 _VALIDATE = os.environ.get("GRIDLLM_VALIDATE", "") == "1"
 
 

@@ -108,8 +108,7 @@ class WorkerAgent:
         # live by then. The reverse order LOST whole assignment bursts:
         # a respawned worker with a queued backlog was re-registered and
         # immediately assigned 16 jobs into the subscription gap — they
-        # sat "active" on a live idle worker until the job timeout
-        # (chaos repro: gpurun_out/lt_server_ready.log 10:46:29).
+        # sat "active" on a live idle worker until the job timeout.
         await self.bus.subscribe(Channels.worker_job(self.worker_id),
                                  self._h_job_msg)
         await self.bus.subscribe(Channels.worker_reregister(self.worker_id),
