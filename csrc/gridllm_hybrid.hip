@@ -1415,8 +1415,7 @@ DEV_INLINE void store_normed(bf16_t* out, const f32x4 (&acc)[4][4],
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 z[r] = acc[c][rt][r] * rs * w[c][r] *
-                       __builtin_amdgcn_rcpf(1.f + __expf(-z[r])) *
-                       (SILU ? z[r] : 1.f);
+                       (sigmoidf_(z[r]) * (SILU ? z[r] : 1.f));
             if (t < len) st4(out + t * out_ld + c * 64 + col0, z);
         }
     }
@@ -1866,8 +1865,7 @@ DEV_INLINE f32x4 mfma_split(bf16x8 ah, bf16x8 al, bf16x8 bh, bf16x8 bl,
 // Bound by reading the state (128 KB a head and chunk of 128 x 256) and the
 // latencies between its few steps. 590 blocks of it: 78 us with tokens split
 // over the waves, each reading the whole state, and 22 of the norm behind it;
-// now 61, of which the gates take 18 and the scores' decays 11. (The gate's
-// sigmoid is the hardware's, 1e-6, ahead of a bf16 result.)
+// now 61, of which the gates take 18 and the scores' decays 11.
 #define GLA_SPAN 60.f
 __global__ void __launch_bounds__(256, 2)
 k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,

@@ -764,3 +764,49 @@ def test_norms_add_parts(n, w, parts, size):
     h0 = hops.join_norm(x0, whole, a, b, w // size, w, 1e-5)
     h1 = hops.join_norm(x1, y, a, b, w // size, w, 1e-5)
     assert torch.equal(x0, x1) and torch.equal(h0, h1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["mlstm", "gla"])
+def test_prompt_gates(kind):
+    """A prompt's output gate, far from 0 where the exponential's argument is
+    large, is as exact as a decode row's. Tokens are chunks of their own with
+    values of +-1, so that the normed sums are +-1 and the result is the norm's
+    weight times the gate."""
+    h, dk, dv, n = 4, 64, 256, 130
+    g = torch.Generator().manual_seed(11)
+    sign = torch.randint(0, 2, (n, h * dv), generator=g) * 2.0 - 1
+    z = (-16 - 64 * torch.rand(n, h * dv, generator=g)).to(torch.bfloat16)
+    rows = torch.cat([torch.ones(n, 2 * h * dk), sign, z.float()],
+                     1).to("cuda", torch.bfloat16)
+    norm = torch.rand(h * dv, generator=g) + 0.5
+
+    def t(*columns):
+        return torch.tensor([[i if c is None else c for c in columns]
+                             for i in range(n)], dtype=torch.int32).cuda()
+    st = hops.StepMeta(chunks=t(None, 1, None, 0), segs=t(None, 1, None, 0),
+                       chunk_segs=t(None, 0, None, 1), nd=0, max_len=200,
+                       pos=t(0).view(-1), slot=t(None).view(-1),
+                       table=torch.zeros(n, 1, dtype=torch.int32).cuda())
+    if kind == "mlstm":
+        got = hops.mlstm(rows, torch.zeros(n, 2 * h).cuda(),
+                         torch.zeros(n, h, dv + 1, dk).cuda(),
+                         torch.zeros(n, h).cuda(), norm.cuda(), st, dk, dv,
+                         15.0, 1e-30)
+    else:
+        got = hops.gla(rows, torch.zeros(n, 8).cuda(),
+                       torch.zeros(8, h * dk).cuda(),
+                       torch.zeros(h * dk).cuda(),
+                       torch.zeros(n, h, dv, dk).cuda(), norm.cuda(), st, dk,
+                       dv, 16.0, 1e-30)
+    zd = z.double()
+    want = sign.double() * norm.double() * torch.sigmoid(zd)
+    if kind == "gla":
+        want = want * zd
+    # f32: an exponential within 2^-23, the norm's 16 sums of a lane at 2^-25
+    # each (under a root) and ten further roundings of 2^-24: below 1.5e-6. So
+    # results that far from the middle of two bf16 are rounded as the exact ones.
+    mant = torch.frexp(want.abs())[0] * 256
+    clear = ((mant % 1) - 0.5).abs() > 1.5e-6 * mant
+    assert bool(clear.float().mean() > 0.99)
+    assert torch.equal(got.cpu()[clear], want.to(torch.bfloat16)[clear])
