@@ -10,11 +10,13 @@ on these shapes — profiles/r01_decode_profile.md.)
 
 from __future__ import annotations
 
+import functools
 import time
 from typing import Optional
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from gridllm_amd import ops
 from gridllm_amd.ops import hip_ops
@@ -29,6 +31,7 @@ _CHOICE: dict[tuple[int, int, int], tuple] = {}
 # gate/up projection with fused SwiGLU (n = 2F interleaved rows):
 # (m, n, k) -> ("blas",) | ("rows",) | ("tile", rows, cols, splitk)
 _CHOICE_GU: dict[tuple[int, int, int], tuple] = {}
+_BF16, _transformed = torch.bfloat16, torch._C._are_functorch_transforms_active
 _ITERS = 24                     # calls of a timing
 _SPLITK_CANDIDATES = (0, 2, 4, 6, 8, 12, 16, 24, 32)
 
@@ -87,25 +90,35 @@ def _run_f32(c: tuple, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return _run(c, x, w).float()
 
 
-def _by_rule(x: torch.Tensor, w: torch.Tensor, fuse: bool = False) -> tuple:
-    """The choice for a shape that was not timed. gemm_rows has no second kernel,
+def _fit(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple[int, int, int]]:
+    """(M, N, K) of x [M, K] @ w [N, K]^T if the kernels here read both as
+    F.linear would: bf16 matrices that fit each other, dense and aligned, without
+    a forward-mode tangent or a torch.func transform, which pass a kernel by."""
+    if x.dtype is not _BF16 or w.dtype is not _BF16 or _transformed() or \
+            forward_ad._current_level >= 0 or x.device != w.device:
+        return None
+    xs, ws = x.shape, w.shape
+    if len(xs) != 2 or len(ws) != 2 or xs[1] != ws[1] or not ws[0] or \
+            not ws[1] or (x.data_ptr() | w.data_ptr()) & 15 or \
+            not x.is_contiguous() or not w.is_contiguous():
+        return None
+    return xs[0], ws[0], ws[1]
+
+
+@functools.lru_cache(maxsize=4096)
+def _rule(m: int, n: int, k: int, fuse: bool = False) -> tuple:
+    """The choice for sizes that were not timed. gemm_rows has no second kernel,
     but every block reads all of x: it is the faster one for w of up to 20 MB
     with up to 4 rows and up to 14 MB with 16 (against gemm_tile: 3072 x 2048, 16
     rows: 7.2 us, 7.4; 3072 x 3072: one row 7.2, 7.9, 16 rows 9.8, 8.0; 5120 x
     3072, one row 10.8, 10.0; gate/up 16384 x 3072, one row: 21.7, 19.8)."""
-    m, size = x.shape[0], w.numel()
-    if m <= 16 and hip_ops.gemm_rows_supported(x, w, fuse):
-        if size <= (10_000_000 if m <= 4 else 7_000_000):
-            return ("rows",)
-    if m <= 256 and x.is_contiguous() and w.is_contiguous() and \
-            w.dtype == torch.bfloat16 and \
-            (x.data_ptr() | w.data_ptr()) % 16 == 0:
-        tiling = hip_ops.gemm_tiling(m, *w.shape, fuse)
-        if tiling is not None:
-            return ("tile", *tiling)
-    if m <= 4 and hip_ops.gemm_rows_supported(x, w, fuse):
+    rows = hip_ops.gemm_rows_fits(m, n, k, fuse)
+    if rows and n * k <= (10_000_000 if m <= 4 else 7_000_000):
         return ("rows",)
-    return ("blas",)
+    tiling = hip_ops.gemm_tiling(m, n, k, fuse)
+    if tiling is not None:
+        return ("tile", *tiling)
+    return ("rows",) if rows and m <= 4 else ("blas",)
 
 
 def _tune(x: torch.Tensor, n: int, glu: Optional[Glu] = None,
@@ -156,9 +169,8 @@ def linear_gateup(x: torch.Tensor, w_il: torch.Tensor,
                   glu: Glu = SWIGLU) -> torch.Tensor:
     """Fused gate/up projection + gated linear unit on an INTERLEAVED weight:
     returns [M, F] activated, through the tuned table or by rule."""
-    c = _CHOICE_GU.get((x.shape[0], w_il.shape[0], w_il.shape[1]))
-    if c is None:
-        c = _by_rule(x, w_il, True) if x.dim() == 2 else ("blas",)
+    fit = _fit(x, w_il)
+    c = ("blas",) if fit is None else _CHOICE_GU.get(fit) or _rule(*fit, True)
     return _run(c, x, w_il, glu)
 
 
@@ -168,13 +180,11 @@ def choice(m: int, n: int, k: int) -> Optional[tuple[str, int]]:
 
 def _choose(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple]:
     """Choice for x @ w.T, None for what is not a GPU product of bf16 rows."""
-    if x.dim() != 2 or not x.is_cuda or x.dtype != torch.bfloat16:
+    if not x.is_cuda or (torch.is_grad_enabled() and
+                         (x.requires_grad or w.requires_grad)):
         return None
-    c = _CHOICE.get((x.shape[0], w.shape[0], w.shape[1]))
-    if c is None and not (torch.is_grad_enabled() and
-                          (x.requires_grad or w.requires_grad)):
-        c = _by_rule(x, w)
-    return c
+    fit = _fit(x, w)
+    return None if fit is None else _CHOICE.get(fit) or _rule(*fit)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

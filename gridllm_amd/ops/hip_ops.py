@@ -367,15 +367,19 @@ def gemm_skinny(x: torch.Tensor, w: torch.Tensor,
     return out
 
 
+def gemm_rows_fits(m: int, n: int, k: int, fuse_swiglu: bool = False) -> bool:
+    """Whether gemm_rows has these sizes."""
+    return (0 < m <= 16 and 0 < n < 65536 and k > 0 and k % 32 == 0
+            and n % (128 if fuse_swiglu else 16) == 0)
+
+
 def gemm_rows_supported(x: torch.Tensor, w: torch.Tensor,
                         fuse_swiglu: bool = False) -> bool:
     """Whether gemm_rows takes x [M, K] @ w [N, K]^T."""
-    m, k = x.shape
-    n = w.shape[0]
-    return (0 < m <= 16 and n < 65536 and k % 32 == 0
-            and n % (128 if fuse_swiglu else 16) == 0
+    return (x.shape[1] == w.shape[1]
+            and gemm_rows_fits(x.shape[0], *w.shape, fuse_swiglu)
             and x.is_contiguous() and w.is_contiguous()
-            and w.dtype == torch.bfloat16
+            and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
@@ -446,7 +450,7 @@ def gemm_tiling(m: int, n: int, k: int,
     library product's sizes (17920 x 1536: 22.9 us, 22.2), but for the gated
     unit that it would need a second kernel for, and so are about 4 M weights
     with more than 128 rows (2048 x 2048: 10.4, 9.2; 896 x 4864: 11.0, 10.3)."""
-    if not 0 < m <= 256 or k % 64 or (fuse_swiglu and n % 128) or \
+    if not 0 < m <= 256 or n < 1 or k < 1 or k % 64 or (fuse_swiglu and n % 128) or \
             (m > 128 and 3_000_000 < n * k < 5_000_000):
         return None
     if m <= 64:

@@ -120,3 +120,50 @@ def test_attn_prefill_with_cached_prefix():
     full = R.attn_prefill(q, k, v, scale)
     part = R.attn_prefill(q[:, tpre:], k, v, scale, causal_offset=tpre)
     assert torch.allclose(full[:, tpre:], part, atol=1e-5)
+
+
+def _mat(*shape, dtype=torch.bfloat16):
+    return torch.zeros(*shape, dtype=dtype)
+
+
+@pytest.mark.parametrize("m", [1, 16, 200])
+def test_linear_takes_what_fits(m, monkeypatch):
+    """Products whose operands F.linear refuses, or reads in a way of its own,
+    are left to it."""
+    from torch.autograd import forward_ad
+
+    from gridllm_amd.ops import autotune
+    ran = []
+    monkeypatch.setattr(autotune, "_run", lambda c, x, *rest: ran.append(c))
+
+    def choice(x, w):
+        ran.clear()
+        autotune.linear_gateup(x, w)
+        return ran[0]
+    x, w, blas = _mat(m, 256), _mat(512, 256), ("blas",)
+    assert choice(x, w) != blas
+    for bad in (_mat(m, 192), _mat(m, 320), _mat(m, 256, dtype=torch.float32),
+                _mat(m, 256, dtype=torch.float16), _mat(256),
+                _mat(m, 2, 256), _mat(m, 512)[:, ::2],
+                _mat(m * 256 + 1)[1:].view(m, 256),
+                torch.zeros(m, 256, dtype=torch.bfloat16, device="meta")):
+        assert choice(bad, w) == blas
+    for bad in (_mat(512, 128), _mat(512, 256, dtype=torch.float32),
+                _mat(256, 512).t(), _mat(0, 256)):
+        assert choice(x, bad) == blas
+    assert choice(_mat(m, 0), _mat(512, 0)) == blas
+    assert choice(_mat(0, 256), w) == blas
+    # the same of sizes that were timed
+    monkeypatch.setitem(autotune._CHOICE_GU, (m, 512, 256), ("rows",))
+    assert choice(x, w) == ("rows",)
+    assert choice(_mat(m, 192), w) == choice(_mat(m, 512)[:, ::2], w) == blas
+    seen = []
+
+    def look(a):
+        seen.append(choice(a, w))
+        return a
+    torch.func.vmap(look)(_mat(2, m, 256))
+    torch.func.jvp(look, (x,), (x,))
+    with forward_ad.dual_level():
+        look(forward_ad.make_dual(x, x))
+    assert seen == [blas] * 3
