@@ -174,7 +174,8 @@ k_prompt_positions(int* __restrict__ pos, int* __restrict__ slot_t,
 }
 
 // x = emb[token], y = rmsnorm(x) * w: one block per row. Tokens count from the
-// end if negative and are held to the table.
+// end if negative; others than the table has end the program, as an index does
+// that a lookup by torch finds out of bounds.
 template <int NV>
 __global__ void __launch_bounds__(256)
 k_embed_norm(bf16_t* __restrict__ x, bf16_t* __restrict__ y,
@@ -184,7 +185,7 @@ k_embed_norm(bf16_t* __restrict__ x, bf16_t* __restrict__ y,
     __shared__ float red[4];
     long long t = tokens[blockIdx.x];
     if (t < 0) t += vocab;
-    t = t < 0 ? 0 : t < vocab ? t : vocab - 1;
+    if (t < 0 || t >= vocab) __builtin_trap();
     const long at = blockIdx.x * (long)H;
     const bf16_t* row = emb + t * H;
     for (int c = threadIdx.x; c < H >> 3; c += 256)

@@ -64,8 +64,13 @@ def prompt_positions(t: int, slot: int, start: int, seq_lens: torch.Tensor,
 
 def embed_norm(tokens: torch.Tensor, emb: torch.Tensor, weight: torch.Tensor,
                eps: float) -> Tuple[torch.Tensor, torch.Tensor]:
-    """emb[tokens] and its rmsnorm."""
-    if _on_gpu(emb) and emb.dtype == torch.bfloat16:
+    """emb[tokens] and its rmsnorm. The fused kernel has token numbers on emb's
+    device and dense rows; other indices and layouts are indexed as they are."""
+    if (_on_gpu(emb) and emb.dtype == weight.dtype == torch.bfloat16
+            and tokens.device == emb.device and tokens.dim() == 1
+            and tokens.dtype in (torch.int64, torch.int32)
+            and emb.is_contiguous() and weight.is_contiguous()
+            and (emb.data_ptr() | weight.data_ptr()) % 16 == 0):
         from gridllm_amd.ops import hip_ops
         return hip_ops.embed_norm(tokens.long().contiguous(), emb, weight, eps)
     x = emb[tokens]

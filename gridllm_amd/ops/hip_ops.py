@@ -180,8 +180,14 @@ def decode_lengths(seq_lens: torch.Tensor,
 
 def embed_norm(tokens: torch.Tensor, emb: torch.Tensor, weight: torch.Tensor,
                eps: float) -> tuple[torch.Tensor, torch.Tensor]:
-    """x = emb[tokens] [n, H] and rmsnorm(x) * weight; tokens [n] int64."""
+    """x = emb[tokens] [n, H] and rmsnorm(x) * weight; tokens [n] int64, counted
+    from the end if negative. Others than the table has end the program, as they
+    do in torch's lookup."""
     n, h = tokens.shape[0], emb.shape[1]
+    if not (tokens.is_cuda and tokens.device == emb.device == weight.device and
+            tokens.dtype == torch.int64 and weight.shape == (h,)):
+        raise ValueError("embed_norm: tokens [n] int64, emb [vocab, H] and "
+                         "weight [H] on one GPU")
     _check_range("embed_norm.tokens", tokens, emb.shape[0])
     x = torch.empty(n, h, dtype=emb.dtype, device=emb.device)
     y = torch.empty_like(x)

@@ -167,3 +167,44 @@ def test_linear_takes_what_fits(m, monkeypatch):
     with forward_ad.dual_level():
         look(forward_ad.make_dual(x, x))
     assert seen == [blas] * 3
+
+
+def test_embed_norm_by_kernel_or_index(monkeypatch):
+    """Indices and layouts that the fused kernel does not read are looked up by
+    torch, which takes host indices of a table elsewhere, masks and strides."""
+    from gridllm_amd import ops
+    from gridllm_amd.ops import hip_ops
+    fused = []
+
+    def kernel(tokens, emb, weight, eps):
+        fused.append(tokens)
+        return emb[tokens], R.rmsnorm(emb[tokens], weight, eps)[0]
+    monkeypatch.setattr(ops, "_on_gpu", lambda t: True)
+    monkeypatch.setattr(hip_ops, "embed_norm", kernel)
+    monkeypatch.setattr(ops, "rmsnorm", R.rmsnorm)
+    g = torch.Generator().manual_seed(3)
+    emb = torch.randn(10, 64, generator=g).to(torch.bfloat16)
+    w, tok = torch.ones(64, dtype=torch.bfloat16), torch.tensor([3, -1, 0])
+    off = torch.zeros(10 * 64 + 1, dtype=torch.bfloat16)[1:].view(10, 64)
+    off.copy_(emb)
+    for t, e, by_kernel in ((tok, emb, True), (tok.int(), emb, True),
+                            (tok[[0, 0, 1, 1, 2, 2]][::2], emb, True),
+                            (tok, emb.t().contiguous().t(), False),
+                            (tok, off, False), (tok.view(3, 1), emb, False),
+                            (torch.arange(10) % 3 == 0, emb, False)):
+        fused.clear()
+        x, y = ops.embed_norm(t, e, w, 1e-5)
+        assert bool(fused) == by_kernel
+        assert torch.equal(x, emb[t])
+        assert torch.equal(y, R.rmsnorm(emb[t], w, 1e-5)[0])
+    fused.clear()
+    assert ops.embed_norm(tok, emb.to("meta"), w.to("meta"),
+                          1e-5)[0].shape == (3, 64) and not fused
+
+
+def test_embed_norm_refuses():
+    from gridllm_amd.ops import hip_ops
+    emb, w = _mat(10, 64), _mat(64)
+    for tok in (torch.tensor([3]), torch.tensor([3], dtype=torch.int32)):
+        with pytest.raises(ValueError):
+            hip_ops.embed_norm(tok, emb, w, 1e-5)

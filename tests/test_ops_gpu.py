@@ -189,6 +189,20 @@ def test_embed_norm_gpu(dev, n, h):
     assert _mx(y.cpu(), ref) < 0.04
 
 
+def test_embed_norm_other_indices_gpu(dev):
+    """Host indices and other layouts, as torch's lookup takes them."""
+    from gridllm_amd import ops
+    from gridllm_amd.ops import hip_ops
+    emb = torch.randn(50, 96, device=dev).to(torch.bfloat16)
+    w = torch.randn(96, device=dev).to(torch.bfloat16)
+    tok = torch.tensor([49, 0, -1, 7, 7])
+    for t, e in ((tok, emb), (tok.to(dev).int(), emb),
+                 (tok.to(dev), emb.t().contiguous().t())):
+        x, y = ops.embed_norm(t, e, w, 1e-5)
+        assert torch.equal(x, emb[tok])
+        assert torch.equal(y, hip_ops.rmsnorm(emb[tok], w, 1e-5))
+
+
 @pytest.mark.parametrize("n,hq,hk,d", [(5, 24, 8, 128), (16, 32, 8, 64),
                                        (7, 4, 2, 20), (1, 3, 1, 16)])
 def test_rope_kv_fused_gpu(dev, n, hq, hk, d):
