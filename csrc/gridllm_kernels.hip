@@ -137,15 +137,20 @@ k_rmsnorm_parts(bf16_t* __restrict__ y, const float* __restrict__ ws, int parts,
 
 // ===========================================================================
 // Start of a decode step: see gl_decode_positions. One block: its two passes
-// stand for the dozen index kernels of 4 us each that a step started with.
+// stand for the dozen index kernels of 4 us each that a step started with. A slot
+// that there is not ends the program, as an index does that torch finds out of
+// bounds, before anything is read or counted by it.
 // ===========================================================================
 __global__ void __launch_bounds__(1024)
 k_decode_positions(int* __restrict__ pos, int* __restrict__ slot_t,
                    int* __restrict__ pos_rope, int* __restrict__ attn_seq,
                    int* seq_lens, const int* __restrict__ rope_off,
-                   const int* __restrict__ slot_map, int B, int Smax) {
+                   const int* __restrict__ slot_map, int B, int slots,
+                   int Smax) {
     for (int i = threadIdx.x; i < B; i += 1024) {
-        const int s = slot_map[i], p = seq_lens[s];
+        const int s = slot_map[i];
+        if ((unsigned)s >= (unsigned)slots) __builtin_trap();
+        const int p = seq_lens[s];
         pos[i] = p;
         if (slot_t) slot_t[i] = s * Smax + p;
         if (attn_seq) attn_seq[i] = p + 1;
@@ -1198,15 +1203,17 @@ int gl_rmsnorm_parts(void* stream, void* y, const void* ws, int parts,
 
 // What a decode step starts with. Per batch row: position, place in the cache,
 // rotary position and number of keys of its slot, whose length goes up by one
-// (all rows read before any counts: rows may share a slot). slot_t, pos_rope,
-// attn_seq and rope_off may be null.
+// (all rows read before any counts: rows may share a slot). slots: of seq_lens
+// and rope_off. slot_t, pos_rope, attn_seq and rope_off may be null.
 int gl_decode_positions(void* stream, void* pos, void* slot_t, void* pos_rope,
                         void* attn_seq, void* seq_lens, const void* rope_off,
-                        const void* slot_map, int B, int Smax) {
+                        const void* slot_map, int B, int slots, int Smax) {
+    if (slots < 1 || (pos_rope && !rope_off)) return -100;
     if (B < 1) return 0;
     k_decode_positions<<<dim3(1), dim3(1024), 0, (hipStream_t)stream>>>(
         (int*)pos, (int*)slot_t, (int*)pos_rope, (int*)attn_seq,
-        (int*)seq_lens, (const int*)rope_off, (const int*)slot_map, B, Smax);
+        (int*)seq_lens, (const int*)rope_off, (const int*)slot_map, B, slots,
+        Smax);
     LAUNCH_CHECK();
     return 0;
 }

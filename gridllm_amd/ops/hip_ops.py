@@ -42,7 +42,7 @@ def _load() -> ctypes.CDLL:
     lib.gl_rmsnorm_parts.argtypes = [c_vp] * 3 + [c_i] + [c_vp] * 3 + [
         c_i, c_i, c_f]
     lib.gl_rmsnorm_parts.restype = c_i
-    lib.gl_decode_positions.argtypes = [c_vp] * 8 + [c_i, c_i]
+    lib.gl_decode_positions.argtypes = [c_vp] * 8 + [c_i] * 3
     lib.gl_decode_positions.restype = c_i
     lib.gl_prompt_positions.argtypes = [c_vp] * 5 + [c_i] * 4
     lib.gl_prompt_positions.restype = c_i
@@ -136,6 +136,19 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float,
     return out
 
 
+def _check_ints(op: str, slot_map: torch.Tensor, *by_slot: torch.Tensor
+                ) -> None:
+    """Dense int32 vectors on one GPU, those by slot of one length. (A slot that
+    they have not ends the program, as an index out of bounds does in torch.)"""
+    slots = by_slot[0].shape[0]
+    for t in (slot_map, *by_slot):
+        if not (t.is_cuda and t.device == slot_map.device and t.dim() == 1
+                and t.dtype == torch.int32 and t.is_contiguous()):
+            raise ValueError(f"{op}: int32 vectors on one GPU")
+    if any(t.shape[0] != slots for t in by_slot):
+        raise ValueError(f"{op}: lengths by slot differ")
+
+
 def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
                      rope_off: torch.Tensor, smax: int
                      ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -143,12 +156,13 @@ def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
     places slot * smax + length, rotary positions length + rope_off[slot], and
     key counts length + 1, all int32 [B]. Advances the slots' lengths."""
     b = slot_map.shape[0]
+    _check_ints("decode_positions", slot_map, seq_lens, rope_off)
     _check_range("decode_positions.slot_map", slot_map, seq_lens.shape[0])
     out = torch.empty(4, b, dtype=torch.int32, device=seq_lens.device)
     _check(_load().gl_decode_positions(
         _stream(), _ptr(out[0]), _ptr(out[1]), _ptr(out[2]), _ptr(out[3]),
-        _ptr(seq_lens), _ptr(rope_off), _ptr(slot_map), b, smax),
-        "decode_positions")
+        _ptr(seq_lens), _ptr(rope_off), _ptr(slot_map), b, seq_lens.shape[0],
+        smax), "decode_positions")
     return out[1], out[2], out[3]
 
 
@@ -170,11 +184,12 @@ def decode_lengths(seq_lens: torch.Tensor,
                    slot_map: torch.Tensor) -> torch.Tensor:
     """The lengths of slots slot_map [B] int32, which then advance by one."""
     b = slot_map.shape[0]
+    _check_ints("decode_lengths", slot_map, seq_lens)
     _check_range("decode_lengths.slot_map", slot_map, seq_lens.shape[0])
     pos = torch.empty(b, dtype=torch.int32, device=seq_lens.device)
     _check(_load().gl_decode_positions(
         _stream(), _ptr(pos), None, None, None, _ptr(seq_lens), None,
-        _ptr(slot_map), b, 0), "decode_lengths")
+        _ptr(slot_map), b, seq_lens.shape[0], 0), "decode_lengths")
     return pos
 
 

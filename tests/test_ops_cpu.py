@@ -208,3 +208,21 @@ def test_embed_norm_refuses():
     for tok in (torch.tensor([3]), torch.tensor([3], dtype=torch.int32)):
         with pytest.raises(ValueError):
             hip_ops.embed_norm(tok, emb, w, 1e-5)
+
+
+def test_decode_positions_refuse():
+    """Host tensors, other types and tables of other lengths are an error ahead of
+    the launch; so is a step over no slots."""
+    from gridllm_amd.ops import hip_ops
+    i32 = torch.zeros(4, dtype=torch.int32)
+    with pytest.raises(ValueError):
+        hip_ops.decode_positions(i32, i32, i32, 64)
+    with pytest.raises(ValueError):
+        hip_ops.decode_lengths(i32, i32)
+    meta = torch.zeros(4, dtype=torch.int32, device="meta")
+    for bad in (meta.long(), meta[::2], meta.view(2, 2)):
+        with pytest.raises(ValueError):
+            hip_ops.decode_lengths(meta, bad)
+    if hip_ops.available():
+        assert hip_ops._load().gl_decode_positions(
+            *(None,) * 8, 1, 0, 64) == -100
