@@ -273,13 +273,19 @@ def decode_splits(blocks: int, keys: int) -> int:
     """Into how many parts decode attention splits rows of up to `keys` keys,
     `blocks` of them counting their kv heads: up to six workgroups a CU, none
     for less than 128 keys. A row of fewer keys takes as many as it needs; the
-    others end at once, at 7 ns each, and the combining kernel takes longer.
-    Measured in us, 8 kv heads of 128: one row of 8000 keys 26 in 6 parts, 18
-    in 12, 15 in 32, 20 in 64; 24 rows of up to 6000 92 in one, 74 in 5, 70 in
-    8 and 12, 83 in 32; 64 rows of up to 2000 63 in one, 69 in 2, 62 in 3 to 6,
-    87 in 16; 256 rows of up to 384 47 in one, 62 in 2."""
-    return max(1, min(1536 // max(1, blocks), (keys + 127) // 128,
-                      32 if blocks <= 16 else 16))
+    others end at once, and the combining kernel takes longer. The number is odd:
+    workgroups go round the XCDs and their shader engines, which are powers of
+    two, and with an even one the first parts of all rows, all that short rows
+    have, would meet on some of them.
+    Measured in us, 8 kv heads of 128, in a cache of 8192: one row of 8000 keys 26
+    in 6 parts, 18 in 12, 15 in 32, 20 in 64; 24 rows of 50 to 300 9 in one, 13 in
+    7 and 9, 20 in 8, of 1000 to 6000 84 in one, 78 in 8 and 9; 64 rows of 50 to
+    300 12 in one, 16 in 3, 24 in 4, of 500 to 2000 59 in one, 60 in 3; 96 rows of
+    50 to 300 17 in one, 23 in 2 and 3, of 100 to 8000 323 in one, 292 in 2, 270 in
+    3; 256 rows of up to 384 47 in one, 62 in 2."""
+    parts = min(1536 // max(1, blocks) | 1, 31 if blocks <= 16 else 15,
+                (keys + 127) // 128)
+    return max(1, parts - 1 | 1)
 
 
 def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,

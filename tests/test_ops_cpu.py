@@ -226,3 +226,17 @@ def test_decode_positions_refuse():
     if hip_ops.available():
         assert hip_ops._load().gl_decode_positions(
             *(None,) * 8, 1, 0, 64) == -100
+
+
+def test_decode_splits():
+    """Odd numbers, which spread the first parts of all rows over the chip's
+    engines; none of less than 128 keys; no more than the combining kernel has."""
+    from gridllm_amd.ops.hip_ops import _MAX_SPLIT, decode_splits
+    for blocks in range(0, 3100):
+        for keys in (0, 1, 128, 129, 300, 513, 100_000):
+            parts = decode_splits(blocks, keys)
+            assert parts % 2 == 1 and parts <= _MAX_SPLIT
+            assert parts == 1 or (parts - 1) * 128 < keys
+            assert parts * blocks <= 1536 + blocks
+    assert [decode_splits(b, 8192) for b in (8, 24, 192, 256, 512, 768, 1537)
+            ] == [31, 15, 9, 7, 3, 3, 1]
