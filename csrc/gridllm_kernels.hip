@@ -136,46 +136,56 @@ k_rmsnorm_parts(bf16_t* __restrict__ y, const float* __restrict__ ws, int parts,
 }
 
 // ===========================================================================
-// Start of a decode step: see gl_decode_positions. One block: its two passes
-// stand for the dozen index kernels of 4 us each that a step started with. A slot
-// that there is not ends the program, as an index does that torch finds out of
-// bounds, before anything is read or counted by it.
+// Start and end of a decode step: see gl_decode_positions and
+// gl_advance_lengths, which stand for the dozen index kernels of 4 us each that
+// a step had. A slot that there is not ends the program, as an index does that
+// torch finds out of bounds, before anything is read or counted by it.
 // ===========================================================================
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(256)
 k_decode_positions(int* __restrict__ pos, int* __restrict__ slot_t,
                    int* __restrict__ pos_rope, int* __restrict__ attn_seq,
-                   int* seq_lens, const int* __restrict__ rope_off,
+                   const int* __restrict__ seq_lens,
+                   const int* __restrict__ rope_off,
                    const int* __restrict__ slot_map, int B, int slots,
                    int Smax) {
-    for (int i = threadIdx.x; i < B; i += 1024) {
-        const int s = slot_map[i];
-        if ((unsigned)s >= (unsigned)slots) __builtin_trap();
-        const int p = seq_lens[s];
-        pos[i] = p;
-        if (slot_t) slot_t[i] = s * Smax + p;
-        if (attn_seq) attn_seq[i] = p + 1;
-        if (pos_rope) pos_rope[i] = p + rope_off[s];
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < B; i += 1024)
-        atomicAdd(seq_lens + slot_map[i], 1);
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= B) return;
+    const int s = slot_map[i];
+    if ((unsigned)s >= (unsigned)slots) __builtin_trap();
+    const int p = seq_lens[s];
+    pos[i] = p;
+    if (slot_t) slot_t[i] = s * Smax + p;
+    if (attn_seq) attn_seq[i] = p + 1;
+    if (pos_rope) pos_rope[i] = p + rope_off[s];
 }
 
-// A prompt's positions start .. start + T - 1 and places in its slot, whose
-// length and rotary offset (if it starts anew) are set: one launch for six.
 __global__ void __launch_bounds__(256)
-k_prompt_positions(int* __restrict__ pos, int* __restrict__ slot_t,
-                   int* __restrict__ seq_lens, int* __restrict__ rope_off,
-                   int slot, int start, int T, int Smax) {
+k_advance_lengths(int* __restrict__ seq_lens, const int* __restrict__ slot_map,
+                  int B, int slots) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= B) return;
+    const int s = slot_map[i];
+    if ((unsigned)s >= (unsigned)slots) __builtin_trap();
+    atomicAdd(seq_lens + s, 1);
+}
+
+// A prompt's positions start .. start + T - 1 and places in its slot; and, when
+// it has been run, the slot's length and (if it started anew) rotary offset.
+__global__ void __launch_bounds__(256)
+k_prompt_positions(int* __restrict__ pos, int* __restrict__ slot_t, int slot,
+                   int start, int T, int Smax) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i < T) {
         pos[i] = start + i;
         slot_t[i] = slot * Smax + start + i;
     }
-    if (i == 0) {
-        seq_lens[slot] = start + T;
-        if (start == 0) rope_off[slot] = 0;
-    }
+}
+
+__global__ void k_prompt_end(int* __restrict__ seq_lens,
+                             int* __restrict__ rope_off, int slot, int start,
+                             int T) {
+    seq_lens[slot] = start + T;
+    if (start == 0) rope_off[slot] = 0;
 }
 
 // x = emb[token], y = rmsnorm(x) * w: one block per row. Tokens count from the
@@ -1202,29 +1212,50 @@ int gl_rmsnorm_parts(void* stream, void* y, const void* ws, int parts,
 }
 
 // What a decode step starts with. Per batch row: position, place in the cache,
-// rotary position and number of keys of its slot, whose length goes up by one
-// (all rows read before any counts: rows may share a slot). slots: of seq_lens
-// and rope_off. slot_t, pos_rope, attn_seq and rope_off may be null.
+// rotary position and number of keys of its slot. slots: of seq_lens and
+// rope_off. slot_t, pos_rope, attn_seq and rope_off may be null.
 int gl_decode_positions(void* stream, void* pos, void* slot_t, void* pos_rope,
-                        void* attn_seq, void* seq_lens, const void* rope_off,
-                        const void* slot_map, int B, int slots, int Smax) {
+                        void* attn_seq, const void* seq_lens,
+                        const void* rope_off, const void* slot_map, int B,
+                        int slots, int Smax) {
     if (slots < 1 || (pos_rope && !rope_off)) return -100;
     if (B < 1) return 0;
-    k_decode_positions<<<dim3(1), dim3(1024), 0, (hipStream_t)stream>>>(
+    k_decode_positions<<<dim3((B + 255) / 256), dim3(256), 0,
+                         (hipStream_t)stream>>>(
         (int*)pos, (int*)slot_t, (int*)pos_rope, (int*)attn_seq,
-        (int*)seq_lens, (const int*)rope_off, (const int*)slot_map, B, slots,
-        Smax);
+        (const int*)seq_lens, (const int*)rope_off, (const int*)slot_map, B,
+        slots, Smax);
     LAUNCH_CHECK();
     return 0;
 }
 
-int gl_prompt_positions(void* stream, void* pos, void* slot_t, void* seq_lens,
-                        void* rope_off, int slot, int start, int T, int Smax) {
+// What it ends with: the rows' slots are one longer (rows may share a slot).
+int gl_advance_lengths(void* stream, void* seq_lens, const void* slot_map,
+                       int B, int slots) {
+    if (slots < 1) return -100;
+    if (B < 1) return 0;
+    k_advance_lengths<<<dim3((B + 255) / 256), dim3(256), 0,
+                        (hipStream_t)stream>>>(
+        (int*)seq_lens, (const int*)slot_map, B, slots);
+    LAUNCH_CHECK();
+    return 0;
+}
+
+int gl_prompt_positions(void* stream, void* pos, void* slot_t, int slot,
+                        int start, int T, int Smax) {
     if (T < 1 || slot < 0 || start < 0) return -100;
     k_prompt_positions<<<dim3((T + 255) / 256), dim3(256), 0,
                          (hipStream_t)stream>>>(
-        (int*)pos, (int*)slot_t, (int*)seq_lens, (int*)rope_off, slot, start,
-        T, Smax);
+        (int*)pos, (int*)slot_t, slot, start, T, Smax);
+    LAUNCH_CHECK();
+    return 0;
+}
+
+int gl_prompt_end(void* stream, void* seq_lens, void* rope_off, int slot,
+                  int start, int T) {
+    if (slot < 0 || start < 0) return -100;
+    k_prompt_end<<<dim3(1), dim3(1), 0, (hipStream_t)stream>>>(
+        (int*)seq_lens, (int*)rope_off, slot, start, T);
     LAUNCH_CHECK();
     return 0;
 }

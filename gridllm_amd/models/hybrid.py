@@ -28,6 +28,7 @@ from typing import Callable, Optional, Sequence
 import numpy as np
 import torch
 
+from gridllm_amd import ops
 from gridllm_amd.models.paged import (PAGE, PagedCache, head_pad, latent_pad,
                                       pad64, rotated_pad)
 from gridllm_amd.models.registry import (AttentionMixer, DenseFF, GlaMixer,
@@ -995,4 +996,5 @@ class HybridModel:
                       table=self.cache.table, max_len=self.max_seq,
                       absorbed=tokens.shape[0])
         x = self._run(tokens, st)
+        ops.advance_lengths(self.cache.seq_lens, slot_map)
         return self._head(x, None)

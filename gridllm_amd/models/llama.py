@@ -360,10 +360,8 @@ class LlamaModel:
         return_hidden, returns (logits, mean-pooled final hidden [H] f32)."""
         s = self.spec
         t = tokens.shape[0]
-        # (a fresh slot's shift offset is reset: alloc is host-only)
-        pos, slot_t = ops.prompt_positions(
-            t, slot, start_pos, self.cache.seq_lens, self.cache.rope_off,
-            self.cache.max_seq)
+        pos, slot_t = ops.prompt_positions(t, slot, start_pos,
+                                           self.cache.max_seq, self.device)
         resid, normed = ops.embed_norm(tokens, self.embed,
                                        self.layers[0].attn_norm, s.norm_eps)
         for li, lw in enumerate(self.layers):
@@ -382,6 +380,9 @@ class LlamaModel:
             next_norm = (self.layers[li + 1].attn_norm
                          if li + 1 < len(self.layers) else self.final_norm)
             normed, resid = self._joined(act, lw.wdown, next_norm, resid)
+        # (a fresh slot's shift offset is reset: alloc is host-only)
+        ops.prompt_end(t, slot, start_pos, self.cache.seq_lens,
+                       self.cache.rope_off)
         logits = _linear_f32(normed[-1:], self.lm_head)
         if return_hidden:
             return logits[0], normed.float().mean(dim=0)
@@ -495,4 +496,5 @@ class LlamaModel:
             next_norm = (self.layers[li + 1].attn_norm
                          if li + 1 < len(self.layers) else self.final_norm)
             normed, resid = self._joined(act, lw.wdown, next_norm, resid)
+        ops.advance_lengths(self.cache.seq_lens, slot_map)
         return _linear_f32(normed, self.lm_head)

@@ -42,7 +42,7 @@ def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
                      rope_off: torch.Tensor, smax: int
                      ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Start of a decode step: cache places, rotary positions and key counts
-    of slots slot_map [B], whose lengths advance by one."""
+    of slots slot_map [B]."""
     if _on_gpu(seq_lens):
         from gridllm_amd.ops import hip_ops
         return hip_ops.decode_positions(
@@ -50,16 +50,30 @@ def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
     return reference.decode_positions(seq_lens, slot_map, rope_off, smax)
 
 
-def prompt_positions(t: int, slot: int, start: int, seq_lens: torch.Tensor,
-                     rope_off: torch.Tensor, smax: int
-                     ) -> Tuple[torch.Tensor, torch.Tensor]:
-    """Positions and cache places of t tokens from `start` on; sets the slot's
-    length, and its rope_off to 0 if start is 0."""
+def advance_lengths(seq_lens: torch.Tensor, slot_map: torch.Tensor) -> None:
+    """End of a decode step: slots slot_map [B] are one longer, by each row."""
     if _on_gpu(seq_lens):
         from gridllm_amd.ops import hip_ops
-        return hip_ops.prompt_positions(t, slot, start, seq_lens, rope_off,
-                                        smax)
-    return reference.prompt_positions(t, slot, start, seq_lens, rope_off, smax)
+        return hip_ops.advance_lengths(seq_lens, slot_map.int().contiguous())
+    reference.advance_lengths(seq_lens, slot_map)
+
+
+def prompt_positions(t: int, slot: int, start: int, smax: int, device
+                     ) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Positions and cache places of t tokens from `start` on."""
+    if torch.device(device).type == "cuda":
+        from gridllm_amd.ops import hip_ops
+        return hip_ops.prompt_positions(t, slot, start, smax, device)
+    return reference.prompt_positions(t, slot, start, smax, device)
+
+
+def prompt_end(t: int, slot: int, start: int, seq_lens: torch.Tensor,
+               rope_off: torch.Tensor) -> None:
+    """Sets the slot's length, and its rope_off to 0 if start is 0."""
+    if _on_gpu(seq_lens):
+        from gridllm_amd.ops import hip_ops
+        return hip_ops.prompt_end(t, slot, start, seq_lens, rope_off)
+    reference.prompt_end(t, slot, start, seq_lens, rope_off)
 
 
 def embed_norm(tokens: torch.Tensor, emb: torch.Tensor, weight: torch.Tensor,

@@ -126,7 +126,7 @@ def _dense(*ts: Optional[torch.Tensor]) -> None:
 
 def decode_lengths(seq_lens: torch.Tensor,
                    slot_map: torch.Tensor) -> torch.Tensor:
-    """The lengths of slots slot_map [B] int32, which then advance by one."""
+    """The lengths of slots slot_map [B] int32."""
     return hip_ops.decode_lengths(seq_lens, slot_map.int().contiguous())
 
 

@@ -44,8 +44,12 @@ def _load() -> ctypes.CDLL:
     lib.gl_rmsnorm_parts.restype = c_i
     lib.gl_decode_positions.argtypes = [c_vp] * 8 + [c_i] * 3
     lib.gl_decode_positions.restype = c_i
-    lib.gl_prompt_positions.argtypes = [c_vp] * 5 + [c_i] * 4
+    lib.gl_advance_lengths.argtypes = [c_vp] * 3 + [c_i] * 2
+    lib.gl_advance_lengths.restype = c_i
+    lib.gl_prompt_positions.argtypes = [c_vp] * 3 + [c_i] * 4
     lib.gl_prompt_positions.restype = c_i
+    lib.gl_prompt_end.argtypes = [c_vp] * 3 + [c_i] * 3
+    lib.gl_prompt_end.restype = c_i
     lib.gl_embed_norm.argtypes = [c_vp] * 6 + [c_l, c_i, c_i, c_f]
     lib.gl_embed_norm.restype = c_i
     lib.gl_rope.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i, c_i, c_i, c_i]
@@ -154,7 +158,7 @@ def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
                      ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Start of a decode step over slots slot_map [B] int32 of seq_lens: cache
     places slot * smax + length, rotary positions length + rope_off[slot], and
-    key counts length + 1, all int32 [B]. Advances the slots' lengths."""
+    key counts length + 1, all int32 [B]."""
     b = slot_map.shape[0]
     _check_ints("decode_positions", slot_map, seq_lens, rope_off)
     _check_range("decode_positions.slot_map", slot_map, seq_lens.shape[0])
@@ -166,23 +170,40 @@ def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
     return out[1], out[2], out[3]
 
 
-def prompt_positions(t: int, slot: int, start: int, seq_lens: torch.Tensor,
-                     rope_off: torch.Tensor, smax: int
+def advance_lengths(seq_lens: torch.Tensor, slot_map: torch.Tensor) -> None:
+    """End of a decode step: the lengths of slots slot_map [B] int32, one or more
+    rows each, go up by one a row."""
+    _check_ints("advance_lengths", slot_map, seq_lens)
+    _check_range("advance_lengths.slot_map", slot_map, seq_lens.shape[0])
+    _check(_load().gl_advance_lengths(
+        _stream(), _ptr(seq_lens), _ptr(slot_map), slot_map.shape[0],
+        seq_lens.shape[0]), "advance_lengths")
+
+
+def prompt_positions(t: int, slot: int, start: int, smax: int, device
                      ) -> tuple[torch.Tensor, torch.Tensor]:
     """Positions start .. start + t - 1 and cache places slot * smax + those,
-    int32 [t]. Sets the slot's length, and its rope_off to 0 if start is 0."""
-    if not (0 <= slot < seq_lens.shape[0]):
-        raise IndexError(f"slot {slot} of {seq_lens.shape[0]}")
-    out = torch.empty(2, t, dtype=torch.int32, device=seq_lens.device)
+    int32 [t]."""
+    out = torch.empty(2, t, dtype=torch.int32, device=device)
     _check(_load().gl_prompt_positions(
-        _stream(), _ptr(out[0]), _ptr(out[1]), _ptr(seq_lens), _ptr(rope_off),
-        slot, start, t, smax), "prompt_positions")
+        _stream(), _ptr(out[0]), _ptr(out[1]), slot, start, t, smax),
+        "prompt_positions")
     return out[0], out[1]
+
+
+def prompt_end(t: int, slot: int, start: int, seq_lens: torch.Tensor,
+               rope_off: torch.Tensor) -> None:
+    """Sets the slot's length to start + t, and its rope_off to 0 if start is
+    0."""
+    if not (0 <= slot < min(seq_lens.shape[0], rope_off.shape[0])):
+        raise IndexError(f"slot {slot} of {seq_lens.shape[0]}")
+    _check(_load().gl_prompt_end(_stream(), _ptr(seq_lens), _ptr(rope_off),
+                                 slot, start, t), "prompt_end")
 
 
 def decode_lengths(seq_lens: torch.Tensor,
                    slot_map: torch.Tensor) -> torch.Tensor:
-    """The lengths of slots slot_map [B] int32, which then advance by one."""
+    """The lengths of slots slot_map [B] int32."""
     b = slot_map.shape[0]
     _check_ints("decode_lengths", slot_map, seq_lens)
     _check_range("decode_lengths.slot_map", slot_map, seq_lens.shape[0])

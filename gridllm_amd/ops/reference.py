@@ -48,29 +48,34 @@ def rope_tables(head_dim: int, max_seq: int, theta: float = 500000.0,
     return freqs.cos().contiguous(), freqs.sin().contiguous()
 
 
-def prompt_positions(t: int, slot: int, start: int, seq_lens: torch.Tensor,
-                     rope_off: torch.Tensor, smax: int
+def prompt_positions(t: int, slot: int, start: int, smax: int, device=None
                      ) -> Tuple[torch.Tensor, torch.Tensor]:
-    """Positions start .. start + t - 1 and slot * smax + those; sets the
-    slot's length, and its rope_off to 0 if start is 0."""
-    pos = torch.arange(start, start + t, dtype=torch.int32,
-                       device=seq_lens.device)
+    """Positions start .. start + t - 1 and slot * smax + those."""
+    pos = torch.arange(start, start + t, dtype=torch.int32, device=device)
+    return pos, pos + slot * smax
+
+
+def prompt_end(t: int, slot: int, start: int, seq_lens: torch.Tensor,
+               rope_off: torch.Tensor) -> None:
+    """Sets the slot's length, and its rope_off to 0 if start is 0."""
     seq_lens[slot] = start + t
     if start == 0:
         rope_off[slot] = 0
-    return pos, pos + slot * smax
 
 
 def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
                      rope_off: torch.Tensor, smax: int
                      ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """(slot * smax + length, length + rope_off[slot], length + 1) of slots
-    slot_map [B]; their lengths advance by one."""
+    slot_map [B]."""
     slots = slot_map.long()
     pos = seq_lens[slots]
-    out = slot_map * smax + pos, pos + rope_off[slots], pos + 1
-    seq_lens.index_add_(0, slots, torch.ones_like(pos))
-    return out
+    return slot_map * smax + pos, pos + rope_off[slots], pos + 1
+
+
+def advance_lengths(seq_lens: torch.Tensor, slot_map: torch.Tensor) -> None:
+    seq_lens.index_add_(0, slot_map.long(),
+                        torch.ones_like(slot_map, dtype=seq_lens.dtype))
 
 
 def rope(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor,

@@ -147,10 +147,7 @@ class DepthAverage:
 
 
 def decode_lengths(seq_lens, slot_map):
-    slots = slot_map.long()
-    pos = seq_lens[slots]
-    seq_lens.index_add_(0, slots, torch.ones_like(pos))
-    return pos
+    return seq_lens[slot_map.long()]
 
 
 def embed(tok, pos, emb, ptab, w=None, w_off=0.0, width=0, eps=0.0, out=None):

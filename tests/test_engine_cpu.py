@@ -551,3 +551,43 @@ def test_async_admission_then_sync_fallback_flushes():
                                                       "num_predict": 6})
     assert r1.token_ids == ref1.token_ids
     assert r2.eval_count == 6
+
+
+@pytest.mark.parametrize("step", ["prompt", "decode", "paged decode"])
+def test_a_step_that_raises_can_be_repeated(step, monkeypatch):
+    """Lengths count what has been run: a step that ends early leaves them."""
+    from gridllm_amd import ops
+    from gridllm_amd.models.hybrid import HybridModel
+    from gridllm_amd.models.llama import LlamaModel
+    from gridllm_amd.models.registry import get_spec
+    from gridllm_amd.ops import hybrid as hops
+
+    kind = HybridModel if step == "paged decode" else LlamaModel
+    m = kind(get_spec("tiny-birepel" if kind is HybridModel else "tiny"),
+             device="cpu", dtype="fp32", kv_slots=3, max_seq=64)
+    slot = m.cache.alloc()
+    m.forward_prefill(torch.tensor([5, 6, 7]), slot)
+    tok, sl = torch.tensor([9]), torch.tensor([slot], dtype=torch.int32)
+
+    def run():
+        if step == "prompt":
+            return m.forward_prefill(torch.tensor([8, 9]), slot, 3)
+        if step == "paged decode":
+            m.cache.prepare_decode([slot])
+        return m.forward_decode(tok, sl)
+    where, name = (hops, "post_norm") if kind is HybridModel else \
+        (ops, "rmsnorm")
+    whole = getattr(where, name)
+
+    def ends(*a, **kw):
+        raise MemoryError
+    monkeypatch.setattr(where, name, ends)
+    before = m.cache.seq_lens.clone()
+    with pytest.raises(MemoryError):
+        run()
+    assert torch.equal(m.cache.seq_lens, before)
+    monkeypatch.setattr(where, name, whole)
+    run()
+    after = before.clone()
+    after[slot] += 2 if step == "prompt" else 1
+    assert torch.equal(m.cache.seq_lens, after)

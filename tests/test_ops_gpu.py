@@ -173,6 +173,36 @@ def test_decode_positions_gpu(dev, b):
                        want[slots.long()])
 
 
+@pytest.mark.parametrize("b", [1, 256, 257, 1500])
+def test_advance_lengths_gpu(dev, b):
+    """Rows of one and several blocks, several rows on one slot."""
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator().manual_seed(b)
+    want = torch.randint(0, 1000, (b + 1,), generator=g, dtype=torch.int32)
+    slots = torch.randperm(b + 1, generator=g)[:b].int()
+    slots[b // 2:] = b
+    got = want.to(dev)
+    R.advance_lengths(want, slots)
+    hip_ops.advance_lengths(got, slots.to(dev))
+    assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("t", [1, 256, 257])
+@pytest.mark.parametrize("start", [0, 5])
+def test_prompt_positions_gpu(dev, t, start):
+    from gridllm_amd.ops import hip_ops
+    for x, y in zip(hip_ops.prompt_positions(t, 2, start, 1024, dev),
+                    R.prompt_positions(t, 2, start, 1024)):
+        assert torch.equal(x.cpu(), y)
+    a, b = (torch.full((4,), 7, dtype=torch.int32) for _ in range(2))
+    x, y = a.to(dev), b.to(dev)
+    hip_ops.prompt_end(t, 2, start, x, y)
+    R.prompt_end(t, 2, start, a, b)
+    assert torch.equal(x.cpu(), a) and torch.equal(y.cpu(), b)
+    with pytest.raises(IndexError):
+        hip_ops.prompt_end(t, 4, start, x, y)
+
+
 @pytest.mark.parametrize("n,h", [(1, 8), (5, 896), (3, 2056), (2, 8192),
                                  (2, 8200)])
 def test_embed_norm_gpu(dev, n, h):
