@@ -1042,6 +1042,7 @@ struct SampleKeys {
     const long long* seeds;
     long long* draws;
     const long long* nongreedy;
+    unsigned long long count;      // of slots
     DEV_INLINE unsigned long long key(int row) const {
         if (!slots) return (unsigned long long)keys[row];
         const long long s = slots[row];
@@ -1071,6 +1072,8 @@ k_sample_gumbel(Pick* __restrict__ ws, const float* __restrict__ logits,
                 const SampleKeys how, int v, int segments) {
     constexpr int E = 4;               // elements of a lane at a time
     const int row = blockIdx.x / segments, seg = blockIdx.x % segments;
+    if (how.slots && (unsigned long long)how.slots[row] >= how.count)
+        __builtin_trap();
     const float* x = logits + (long)row * v;
     const unsigned long long key = how.key(row);
     const float t = how.temp(row), rt = 1.f / t;
@@ -1443,16 +1446,19 @@ int gl_gemm_tile(void* stream, void* out, void* ws, const void* x,
 }
 
 // keys [b] and temps [b]; or, with slots [b], temps, seeds, draws and nongreedy
-// by slot, of which draws are advanced. ws: 8 bytes per row and segment.
+// by slot (`count` of them), of which draws are advanced. ws: 8 bytes per row and
+// segment.
 int gl_sample_gumbel(void* stream, void* out, void* ws, const void* logits,
                      const void* keys, const void* temps, const void* slots,
                      const void* seeds, void* draws, const void* nongreedy,
-                     int b, int v, int segments) {
+                     int b, int v, int segments, int count) {
+    if (segments < 1 || (slots ? count < 1 || !seeds || !draws || !nongreedy
+                               : !keys)) return -100;
     if (b <= 0) return 0;
-    if (segments < 1) return -100;
     const SampleKeys how{(const long long*)keys, (const float*)temps,
                          (const long long*)slots, (const long long*)seeds,
-                         (long long*)draws, (const long long*)nongreedy};
+                         (long long*)draws, (const long long*)nongreedy,
+                         (unsigned long long)count};
     hipStream_t st = (hipStream_t)stream;
     k_sample_gumbel<<<dim3((unsigned)(b * segments)), dim3(256), 0, st>>>(
         (Pick*)ws, (const float*)logits, how, v, segments);

@@ -441,8 +441,9 @@ class SlotSampler:
                 and os.environ.get("GRIDLLM_FUSED_SAMPLER", "1") != "0"):
             from gridllm_amd.ops import hip_ops
             return hip_ops.sample_gumbel_slots(
-                logits.contiguous(), slot_ids.long().contiguous(), self.temps,
-                self.seeds, self.draws, self.nongreedy)
+                logits.contiguous(),
+                slot_ids.to(logits.device, torch.int64).contiguous(),
+                self.temps, self.seeds, self.draws, self.nongreedy)
         temps = self.temps[slot_ids].unsqueeze(1)
         x = logits / temps
         v = logits.shape[1]

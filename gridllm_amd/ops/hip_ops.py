@@ -79,7 +79,7 @@ def _load() -> ctypes.CDLL:
     lib.gl_attn_prefill_batch.restype = c_i
     lib.gl_swiglu_il.argtypes = [c_vp, c_vp, c_vp, c_l, c_i,
                                  c_f, c_f, c_f, c_f]
-    lib.gl_sample_gumbel.argtypes = [c_vp] * 10 + [c_i] * 3
+    lib.gl_sample_gumbel.argtypes = [c_vp] * 10 + [c_i] * 4
     lib.gl_sample_gumbel.restype = c_i
     lib.gl_swiglu_il.restype = c_i
     lib.gl_device_sync.argtypes = []
@@ -662,23 +662,40 @@ def sample_gumbel_slots(logits: torch.Tensor, slots: torch.Tensor,
                         ) -> torch.Tensor:
     """sample_gumbel with the rows' parameters by slot (slots [B] i64, all
     different; temps f32, seeds, draws, nongreedy i64): the keys are made in the
-    kernel, and the slots' draws advance by one."""
+    kernel, and the slots' draws advance by one. A slot that there is not ends the
+    program, as an index out of bounds does in torch."""
     return _sample(logits, None, temps, slots, seeds, draws, nongreedy)
 
 
-def _sample(logits, keys, temps, *by_slot) -> torch.Tensor:
+def _sample(logits, keys, temps, slots=None, seeds=None, draws=None,
+            nongreedy=None) -> torch.Tensor:
     lib = _load()
     b, v = logits.shape
+    per_row = keys if slots is None else slots
+    n, dev = temps.numel(), logits.get_device()
+    ok = (dev >= 0 and logits.dtype == torch.float32 and logits.is_contiguous()
+          and temps.dtype == torch.float32 and per_row.numel() == b
+          and (slots is not None or n == b))
+    for t in (temps, per_row) if slots is None else \
+            (temps, per_row, seeds, draws, nongreedy):
+        ok = (ok and t.get_device() == dev and t.is_contiguous()
+              and t.dim() == 1 and (t is temps or t.dtype == torch.int64)
+              and (t is per_row or t.numel() == n))
+    if not ok:
+        raise ValueError("sample_gumbel: f32 logits [B, V] and temps, int64 "
+                         "keys [B], or slots [B] and vectors by slot of one "
+                         "length, dense and on one GPU")
+    if slots is not None:
+        _check_range("sample_gumbel.slots", slots, n)
     # four blocks a CU, of 2048 elements or more: 64 rows of 128256 take 21 us
     # in 16 segments, 190 in one (with exact logarithms)
     segments = max(1, min(1024 // max(1, b), v // 2048, 64))
     out = torch.empty(b, dtype=torch.int32, device=logits.device)
     ws = torch.empty(b * segments, dtype=torch.int64, device=logits.device)
-    slots, seeds, draws, nongreedy = by_slot or (None,) * 4
     _check(lib.gl_sample_gumbel(
         _stream(), _ptr(out), _ptr(ws), _ptr(logits), _ptr(keys), _ptr(temps),
         _ptr(slots), _ptr(seeds), _ptr(draws), _ptr(nongreedy), b, v,
-        segments), "sample_gumbel")
+        segments, n), "sample_gumbel")
     return out
 
 

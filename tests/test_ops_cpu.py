@@ -240,3 +240,17 @@ def test_decode_splits():
             assert parts * blocks <= 1536 + blocks
     assert [decode_splits(b, 8192) for b in (8, 24, 192, 256, 512, 768, 1537)
             ] == [31, 15, 9, 7, 3, 3, 1]
+
+
+def test_sampling_refuses():
+    from gridllm_amd.ops import hip_ops
+    if not hip_ops.available():
+        pytest.skip("the HIP library is not built")
+    x, k = torch.zeros(3, 64), torch.zeros(3, dtype=torch.int64)
+    with pytest.raises(ValueError):                     # on the host
+        hip_ops.sample_gumbel(x, k, torch.ones(3))
+    with pytest.raises(ValueError):
+        hip_ops.sample_gumbel_slots(x, k, torch.ones(3), k, k, k)
+    call = hip_ops._load().gl_sample_gumbel
+    assert call(*(None,) * 10, 1, 64, 1, 1) == -100     # neither keys nor slots
+    assert call(*(None,) * 6, 1, 1, 1, 1, 1, 64, 1, 0) == -100

@@ -754,3 +754,46 @@ def test_gemm_proj_mtiled_fused_swiglu(dev):
                                 mtiles=mt)
         err = (out.float() - ref).abs().max().item()
         assert err < 0.03 * ref.abs().max().item() + 1e-5, (mt, err)
+
+
+def test_slot_sampler_takes_host_slots(dev):
+    """Slot numbers on the host, as torch's indexing takes them."""
+    from gridllm_amd.engine.sampler import SlotSampler
+    x = torch.randn(3, 5000, device=dev)
+
+    class Row:
+        class state:
+            greedy = need_filter = False
+    out = []
+    for slots in (torch.tensor([4, 0, 2]), torch.tensor([4, 0, 2]).to(dev)):
+        sm = SlotSampler(5, dev)
+        sm.temps.fill_(0.7)
+        sm.nongreedy.fill_(1)
+        sm.seeds.copy_(torch.arange(5) + 3)
+        out.append(sm.sample_ids(x, [Row] * 3, slots).tolist())
+        assert sm.draws.tolist() == [1, 0, 1, 0, 1]
+    assert out[0] == out[1]
+
+
+def test_sampling_refuses_gpu(dev):
+    """What the kernel would read beside its operands is an error ahead of the
+    launch: host tensors, other types, vectors of other lengths."""
+    from gridllm_amd.ops import hip_ops
+
+    def i64(n):
+        return torch.zeros(n, dtype=torch.int64, device=dev)
+
+    def f32(*shape):
+        return torch.ones(*shape, device=dev)
+    good = (f32(3, 64), i64(3), f32(5), i64(5), i64(5), i64(5))
+    assert hip_ops.sample_gumbel_slots(*good).tolist() == [0, 0, 0]
+    for at, bad in ((0, good[0].cpu()), (0, good[0].double()),
+                    (0, f32(3, 128)[:, ::2]), (1, i64(2)), (1, i64(3).int()),
+                    (1, i64(3).cpu()), (2, f32(4)), (3, i64(4)),
+                    (4, i64(10)[::2]), (5, f32(5))):
+        with pytest.raises(ValueError):
+            hip_ops.sample_gumbel_slots(*good[:at], bad, *good[at + 1:])
+    for keys, temps in ((i64(2), f32(3)), (i64(3), f32(2)),
+                        (i64(3).int(), f32(3)), (i64(3), f32(3).cpu())):
+        with pytest.raises(ValueError):
+            hip_ops.sample_gumbel(good[0], keys, temps)
