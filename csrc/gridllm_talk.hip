@@ -1123,7 +1123,7 @@ int gt_talk_decode(void* stream, void* out, const void* q, const void* vc,
                    float rho) {
     if (N < 1 || !sizes_ok(H, G, P, R, nrot, chunk) || H > 64 ||
         G * P > 1024 || nrot < per_slot * PAGE ||
-        (ws && (N > 256 || blocks < 1))) return -100;
+        (ws && (N > 256 || blocks < N))) return -100;   // (a row has one)
     const Rotation rot = rotation(cos_, sin_, R, nrot);
     const Cap cap{rate, top, rho};
 #define GO(A, B, C, D) return go_decode<A, B, C, D>((hipStream_t)stream, \

@@ -709,3 +709,18 @@ def test_trace_replay(checkpoint, tmp_path, run):
     for k, w in want.items():
         got = np.fromfile(os.path.join(out, f"{k}.f32"), dtype="<f4")
         close(torch.from_numpy(got).view(w.shape), w, run)
+
+
+def test_decode_blocks_for_each_row():
+    """A step of more rows than blocks would leave rows without a result."""
+    import os
+
+    from gridllm_amd.ops import hip_hybrid
+    from gridllm_amd.ops.build import lib_path
+    if not os.path.exists(lib_path("talk")):
+        pytest.skip("the HIP library is not built")
+    call = hip_hybrid._load("gt").gt_talk_decode
+    none = [None] * 4
+    for rows, blocks in ((2, 1), (200, 199), (257, 300), (1, 0)):
+        assert call(None, *none, None, 1, None, None, 1, *none, 64, rows, 9, 3,
+                    64, 64, 130, blocks, 1.0, 1.0, 0.0) == -100
