@@ -211,8 +211,8 @@ DEV_INLINE bool find_part(int b, int blocks, const int* pos, int last, int N,
 // in flight. Scores: up to 16 heads of one value head against 16 keys are one
 // item, and a wave has one or two of the same heads; the weights meet in LDS,
 // and a wave then has all heads' weights against CW columns of one value head.
-//   ws: sums [blocks][G][H][P], the weights' sums [blocks][H], and of each row
-//   the first block and the number of its parts, int [N][2]
+//   ws: sums [blocks][G][H][P], of each row the first block and the number of
+//   its parts, int [N][2] (at 8 bytes there), and the weights' sums [blocks][H]
 // Bound by the tiles' way to LDS: a block fits a CU once (24 heads, 8 values of
 // 128) and takes 3.4 us for a tile of 64 KB, 4.9 TB/s if all CUs have a block.
 // With a block per row, 160 rows of up to 1000 keys took 105 us, the longest
@@ -451,11 +451,11 @@ k_talk_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
     }
     __syncthreads();
     if (ws && own.split == 0 && threadIdx.x == 0)
-        *(int2*)(ws + (long)gridDim.x * (G * H * P + H) + n * 2) =
+        ((int2*)(ws + (long)gridDim.x * G * H * P))[n] =
             make_int2(own.block0, live);
     if (live > 1) {
         const long at = blockIdx.x;
-        float* wl = ws + (long)gridDim.x * G * H * P + at * H;
+        float* wl = ws + (long)gridDim.x * G * H * P + 2 * N + at * H;
         for (int h = threadIdx.x; h < H; h += WAVES * 64)
             wl[h] = ls[h] + ls[HB * 16 + h];
         if (vh >= G) return;
@@ -523,8 +523,9 @@ k_talk_combine(bf16_t* __restrict__ out, const float* __restrict__ ws,
     __shared__ float nrm[64];
     const int n = blockIdx.x, kv = blockIdx.y, rep = H / G, tid = threadIdx.x;
     const int c0 = blockIdx.z * COLS, cl = tid % PIECES * 4, g0 = tid / PIECES;
-    const float* wl = ws + (long)blocks * G * H * P + min(tid, H - 1);
-    const int2 own = *(const int2*)(ws + (long)blocks * (G * H * P + H) + n * 2);
+    const float* of_rows = ws + (long)blocks * G * H * P;
+    const int2 own = ((const int2*)of_rows)[n];
+    const float* wl = of_rows + 2 * gridDim.x + min(tid, H - 1);
     const int live = own.y;
     if (live == 1) return;             // its block has stored the result
     const long b0 = own.x;

@@ -329,7 +329,7 @@ def test_rotation_far_out(run):
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 7, 60, 224])
 @pytest.mark.parametrize("sizes", [(24, 8, 128, 4096, 64), (9, 3, 20, 70, 6),
-                                   (40, 1, 64, 333, 64)])
+                                   (9, 3, 20, 130, 6), (40, 1, 64, 333, 64)])
 def test_decode_in_parts(n, sizes, monkeypatch):
     """Rows in parts, as many as there are blocks for, against blocks of one row
     each and against the exact mode."""
