@@ -254,3 +254,26 @@ def test_sampling_refuses():
     call = hip_ops._load().gl_sample_gumbel
     assert call(*(None,) * 10, 1, 64, 1, 1) == -100     # neither keys nor slots
     assert call(*(None,) * 6, 1, 1, 1, 1, 1, 64, 1, 0) == -100
+
+
+def test_tuner_skips_what_cannot_run(monkeypatch):
+    """A candidate that fails is left out; the library is always there."""
+    from gridllm_amd.ops import autotune
+    took = {"blas": 3.0, "rows": 2.0, "tile": 1.0}
+    tried = []
+
+    def run(c, x, w, glu=None):
+        tried.append(c)
+        if c[0] == "tile":
+            raise RuntimeError("no such tile")
+
+    def timed(fn, ws, *rest):
+        fn(ws[0])
+        return took[tried[-1][0]]
+    monkeypatch.setattr(autotune, "_run", run)
+    monkeypatch.setattr(autotune, "_time_fn", timed)
+    x = _mat(4, 256)
+    assert autotune._tune(x, 512) == ("rows",)
+    assert {c[0] for c in tried} == {"blas", "rows", "tile"}
+    took["rows"] = 4.0
+    assert autotune._tune(x, 512) == ("blas",)
