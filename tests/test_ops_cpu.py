@@ -277,3 +277,21 @@ def test_tuner_skips_what_cannot_run(monkeypatch):
     assert {c[0] for c in tried} == {"blas", "rows", "tile"}
     took["rows"] = 4.0
     assert autotune._tune(x, 512) == ("blas",)
+
+
+def test_scripts_call_what_there_is():
+    """Every function that a script takes from the kernel layer is there."""
+    import ast
+    import pathlib
+
+    from gridllm_amd.ops import autotune, hip_hybrid, hip_ops
+    mods = {"hip_ops": hip_ops, "hip_hybrid": hip_hybrid, "autotune": autotune}
+    seen = 0
+    for path in sorted(pathlib.Path(__file__).parents[1].glob("scripts/*.py")):
+        for node in ast.walk(ast.parse(path.read_text())):
+            if isinstance(node, ast.Attribute) and \
+                    isinstance(node.value, ast.Name) and node.value.id in mods:
+                assert hasattr(mods[node.value.id], node.attr), \
+                    (path.name, node.attr)
+                seen += 1
+    assert seen > 5
