@@ -1488,7 +1488,7 @@ int gl_attn_prefill(void* stream, void* out, const void* q, const void* kc,
     hipStream_t st = (hipStream_t)stream;
     if (Hq % Hk) return -110;
     const int G = Hq / Hk;
-    if (T < 1 || s_total < 1) return -100;
+    if (T < 1) return -100;
     dim3 grid(prefill_grid((T + 127) / 128, Hq)), blk(256);
     if (D == 128)
         k_attn_prefill<128><<<grid, blk, 0, st>>>(

@@ -797,3 +797,12 @@ def test_sampling_refuses_gpu(dev):
                         (i64(3).int(), f32(3)), (i64(3), f32(3).cpu())):
         with pytest.raises(ValueError):
             hip_ops.sample_gumbel(good[0], keys, temps)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_attn_prefill_without_keys(dev, d):
+    """Queries that see nothing get nothing."""
+    from gridllm_amd.ops import hip_ops
+    q, kc, vc = (torch.randn(*s, device=dev).to(torch.bfloat16)
+                 for s in ((130, 4, d), (2, 2, 64, d), (2, 2, 64, d)))
+    assert not hip_ops.attn_prefill_cache(q, kc, vc, 1, 0, 0, 0.1).any()
