@@ -118,12 +118,14 @@ def _fit(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple[int, int, int]]:
 @functools.lru_cache(maxsize=4096)
 def _rule(m: int, n: int, k: int, fuse: bool = False) -> tuple:
     """The choice for sizes that were not timed. gemm_rows has no second kernel,
-    but every block reads all of x: it is the faster one for w of up to 20 MB
-    with up to 4 rows and up to 14 MB with 16 (against gemm_tile: 3072 x 2048, 16
-    rows: 7.2 us, 7.4; 3072 x 3072: one row 7.2, 7.9, 16 rows 9.8, 8.0; 5120 x
-    3072, one row 10.8, 10.0; gate/up 16384 x 3072, one row: 21.7, 19.8)."""
+    but every block reads all of x, and takes all of K by itself: it is the faster
+    one for w of up to 20 MB with up to 4 rows and up to 14 MB with 16 (against
+    gemm_tile: 3072 x 2048, 16 rows: 7.2 us, 7.4; 3072 x 3072: one row 7.2, 7.9, 16
+    rows 9.8, 8.0; 5120 x 3072, one row 10.8, 10.0; gate/up 16384 x 3072, one row:
+    21.7, 19.8), if K is 4096 or less (1024 x 6144, 16 rows 18.6 us, 10.3, the
+    library 13.1; 1024 x 8192, 4 rows 15.5, 10.6, 13.6)."""
     rows = hip_ops.gemm_rows_fits(m, n, k, fuse)
-    if rows and n * k <= (10_000_000 if m <= 4 else 7_000_000):
+    if rows and k <= 4096 and n * k <= (10_000_000 if m <= 4 else 7_000_000):
         return ("rows",)
     tiling = hip_ops.gemm_tiling(m, n, k, fuse)
     if tiling is not None:

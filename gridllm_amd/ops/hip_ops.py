@@ -491,15 +491,17 @@ def gemm_tiling(m: int, n: int, k: int,
     CU or less, K in parts for the others unless it is short (45 rows, the
     library's time behind it: 2048 x 8192 12.2 us, 14.5; 1536 x 8960 11.8, 22.0;
     896 x 4864 9.2, 13.3; 128256 x 3072 144, 171).
-    Up to 256: as many blocks as there are CUs or a little less, of rows before
-    parts of K, which cost a second kernel, unless K is long (160 rows: 3072 x
-    3072 15.4 us, 16.5; 5120 x 3072 16.0, 23.5; 3072 x 8192 21.7, 28.0; 256 rows:
-    17.3, 17.9; 19.8, 32.1; 26.2, 33.8). More columns than that, or rows, are a
-    library product's sizes (17920 x 1536: 22.9 us, 22.2), but for the gated
-    unit that it would need a second kernel for, and so are about 4 M weights
-    with more than 128 rows (2048 x 2048: 10.4, 9.2; 896 x 4864: 11.0, 10.3)."""
-    if not 0 < m <= 256 or n < 1 or k < 1 or k % 64 or (fuse_swiglu and n % 128) or \
-            (m > 128 and 3_000_000 < n * k < 5_000_000):
+    Up to 256: what _tile_us says of a block a CU or less, with K whole, in the
+    parts that then fill the CUs, or in half as many (160 rows: 3072 x 3072 16.6
+    us, 18.4; 5120 x 3072 16.0, 23.5; 3072 x 8192 21.7, 28.0; 1024 x 4096 11.1,
+    13.9; 256 rows: 19.4, 19.9; 19.8, 32.1; 26.2, 33.8; 13.1, 13.8). Over 51 sizes
+    of 0.3 to 50 M weights and 10 numbers of rows it takes 0.73 of the library's
+    time, 1.06 at most (2048 x 4096, 256 rows), and 1.01 of the best tiling's.
+    More blocks than CUs are a library product's sizes (17920 x 1536, 256 rows:
+    22.9 us, 22.2), but for the gated unit that it would need a second kernel
+    for."""
+    if not 0 < m <= 256 or n < 1 or k < 1 or k % 64 or (
+            fuse_swiglu and n % 128):
         return None
     if m <= 64:
         cols = 128 if n // 64 > 256 and n % 128 == 0 else 64
@@ -507,16 +509,30 @@ def gemm_tiling(m: int, n: int, k: int,
             return None
         parts = max(1, min(256 // (n // cols), k // (128 if k > 2048 else 512)))
         return 32 if m <= 32 else 64, cols, parts
-    best, most = None, 0
+    best, least = None, float("inf")
     for rows, cols, tiles in _tile_grid(m, n, k, fuse_swiglu):
-        parts = max(1, min(256 // tiles, k // 1024)) if k > 4096 else 1
-        # (ties: more tiles, fewer parts)
-        if tiles <= 256 and (tiles * parts > most or (
-                tiles * parts == most and parts < best[2])):
-            best, most = (rows, cols, parts), tiles * parts
+        if tiles > 256:
+            continue
+        most = max(1, min(256 // tiles, k // 384))
+        for parts in sorted({1, (most + 1) // 2, most}):
+            us = _tile_us(m, n, k, rows, cols, tiles, parts)
+            if us < least:
+                best, least = (rows, cols, parts), us
     if best is None and fuse_swiglu:
         return 128 if m <= 128 else 256, 128, 1
     return best
+
+
+def _tile_us(m: int, n: int, k: int, rows: int, cols: int, tiles: int,
+             parts: int) -> float:
+    """What a tiling takes of gemm_tile's time, in us, beside 6 that all have: a
+    CU's loads of its share of K, one block after the other, and with K in parts
+    the second kernel, which reads the partial sums. (Fitted to 18000 timings of 65
+    to 256 rows, 7 % off in the mean.)"""
+    kslice = -(-(-(-k // parts)) // 64) * 64
+    parts = -(-k // kslice)
+    us = -(-tiles * parts // 256) * kslice * (rows + cols - 37) * 3.9e-5
+    return us if parts == 1 else us + 1.2 + parts * m * n * 2.5e-6
 
 
 def gemm_tile(x: torch.Tensor, w: torch.Tensor, rows: int, cols: int,

@@ -295,3 +295,31 @@ def test_scripts_call_what_there_is():
                     (path.name, node.attr)
                 seen += 1
     assert seen > 5
+
+
+def test_tilings_by_rule():
+    """Each is one that the kernel has; neighbouring sizes of weights are not left
+    to another path than those around them; few columns have their K in parts."""
+    from gridllm_amd.ops import hip_ops
+    from gridllm_amd.ops.autotune import _rule
+    for m in (1, 16, 17, 33, 64, 65, 96, 129, 160, 256):
+        for n in (64, 128, 192, 896, 1024, 2048, 3072, 4096, 128256):
+            for k in (64, 192, 896, 1024, 2048, 4096, 12288):
+                for fuse in (False, True):
+                    t = hip_ops.gemm_tiling(m, n, k, fuse)
+                    if t is None:
+                        continue
+                    rows, cols, parts = t
+                    assert rows in hip_ops._TILE_ROWS and n % cols == 0
+                    assert cols in ((64, 128) if fuse else (64, 96, 128))
+                    assert 1 <= parts <= max(1, k // 64)
+    for fuse in (False, True):
+        for m in (129, 160, 256):
+            assert all(hip_ops.gemm_tiling(m, n, k, fuse)
+                       for n in range(512, 4097, 128)
+                       for k in range(512, 4097, 128))
+    for m in (96, 160, 256):
+        for n, k in ((256, 4096), (1024, 3072), (1024, 4096), (2048, 4096)):
+            assert hip_ops.gemm_tiling(m, n, k)[2] > 1
+    assert _rule(16, 1024, 6144)[0] == _rule(4, 1024, 8192)[0] == "tile"
+    assert _rule(4, 1024, 4096)[0] == "rows"
