@@ -32,6 +32,7 @@ _CHOICE: dict[tuple[int, int, int], tuple] = {}
 # (m, n, k) -> ("blas",) | ("rows",) | ("tile", rows, cols, splitk)
 _CHOICE_GU: dict[tuple[int, int, int], tuple] = {}
 _BF16, _transformed = torch.bfloat16, torch._C._are_functorch_transforms_active
+_most_rows = 256                # of a choice by rule or timing
 _ITERS = 24                     # calls of a timing, at most
 _SPLITK_CANDIDATES = (0, 2, 4, 6, 8, 12, 16, 24, 32)
 
@@ -104,11 +105,14 @@ def _fit(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple[int, int, int]]:
     """(M, N, K) of x [M, K] @ w [N, K]^T if the kernels here read both as
     F.linear would: bf16 matrices that fit each other, dense and aligned, without
     a forward-mode tangent or a torch.func transform, which pass a kernel by."""
+    xs = x.shape
+    if len(xs) != 2 or xs[0] > _most_rows:      # (early: prompts' products)
+        return None
     if x.dtype is not _BF16 or w.dtype is not _BF16 or _transformed() or \
             forward_ad._current_level >= 0 or x.device != w.device:
         return None
-    xs, ws = x.shape, w.shape
-    if len(xs) != 2 or len(ws) != 2 or xs[1] != ws[1] or not ws[0] or \
+    ws = w.shape
+    if len(ws) != 2 or xs[1] != ws[1] or not ws[0] or \
             not ws[1] or (x.data_ptr() | w.data_ptr()) & 15 or \
             not x.is_contiguous() or not w.is_contiguous():
         return None
@@ -136,7 +140,9 @@ def _rule(m: int, n: int, k: int, fuse: bool = False) -> tuple:
 def _tune(x: torch.Tensor, n: int, glu: Optional[Glu] = None,
           f32: bool = False) -> tuple:
     """The fastest for x and a weight of n rows; f32: with a result of that."""
+    global _most_rows
     m, k = x.shape
+    _most_rows = max(_most_rows, m)
     ws = _weights(n, k, x.device)
 
     def time_of(c: tuple, limit: float = float("inf")) -> float:

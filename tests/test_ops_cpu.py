@@ -277,6 +277,12 @@ def test_tuner_skips_what_cannot_run(monkeypatch):
     assert {c[0] for c in tried} == {"blas", "rows", "tile"}
     took["rows"] = 4.0
     assert autotune._tune(x, 512) == ("blas",)
+    # sizes beyond the rules' are looked up once they have been timed
+    monkeypatch.setattr(autotune, "_most_rows", 256)
+    big, w = _mat(300, 256), _mat(512, 256)
+    assert autotune._fit(big, w) is None
+    autotune._tune(big, 512)
+    assert autotune._fit(big, w) == (300, 512, 256)
 
 
 def test_scripts_call_what_there_is():
