@@ -2642,6 +2642,7 @@ int gh_post_norm(void* stream, int f32, void* x, void* xb, const void* y,
         (const float*)wt, top, (const float*)w, w_off, W, Wtrue, eps)
     if (f32) { if (wt) GO(float, PAIRS); else GO(float, PLAIN); }
     else { if (wt) GO(bf16_t, PAIRS); else GO(bf16_t, PLAIN); }
+#undef GO
     LAUNCH_CHECK();
     return 0;
 }
@@ -2651,11 +2652,9 @@ int gh_post_norm_parts(void* stream, void* x, void* xb, const void* y,
                        int parts, const void* w, float w_off, int N, int W,
                        int Wtrue, float eps) {
     if (W % 64 || W > 8192 || N < 1 || parts < 1) return -100;
-    hipStream_t st_ = (hipStream_t)stream;
-    const void* wt = nullptr;
-    const int top = parts;
-    GO(bf16_t, PARTS);
-#undef GO
+    k_post_norm<bf16_t, PARTS><<<N, 256, 0, (hipStream_t)stream>>>(
+        (float*)x, (bf16_t*)xb, y, nullptr, parts, (const float*)w, w_off, W,
+        Wtrue, eps);
     LAUNCH_CHECK();
     return 0;
 }
@@ -2678,7 +2677,8 @@ int gh_norm_rows(void* stream, int f32, void* out, const void* x,
 int gh_group_norm(void* stream, int f32, void* out, void* x, const void* y,
                   int parts, const void* rows, const void* wy, const void* w,
                   int N, int W, int groups, int size, float eps) {
-    if (parts < 0 || (parts && (f32 || !y)) || N < 1 || W % 8 || W > 8192 || groups < 1 || size < 1 ||
+    if (parts < 0 || (parts && (f32 || !y)) || N < 1 || W % 8 || W > 8192 ||
+        groups < 1 || size < 1 ||
         (long)groups * size > W || (!y && !out) || (y && rows)) return -100;
     const int gr = size % 8 == 0 ? 8 : size % 4 == 0 ? 4 : size % 2 ? 1 : 2;
     const int lds = (W / gr + groups) * 4;
@@ -2988,7 +2988,8 @@ int gh_mlstm_chunks(void* stream, int constant, void* o, void* out, void* S,
     const int cols = state_columns(nchunks * H);
 #define GO(C) do { \
     k_mlstm_chunk_state<C><<<dim3(nchunks, H, \
-        DK / 64 * ((DV + cols - 1) / cols)), 256, 0, st_>>>((float*)dS, (float*)scal, (const float*)mst, \
+        DK / 64 * ((DV + cols - 1) / cols)), 256, 0, st_>>>((float*)dS, \
+        (float*)scal, (const float*)mst, \
         (const bf16_t*)qkv, (const float*)gr, (const int4*)chunks, \
         (const int4*)segs, H, DK, DV, ld_, cap, cols); \
     LAUNCH_CHECK(); \

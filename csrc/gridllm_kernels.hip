@@ -5,13 +5,14 @@
 // (reference: client/src/services/OllamaService.ts — an HTTP adapter; the
 // compute it delegated lives here instead).
 //
-// Design notes (see /opt/skills guides):
+// Design notes:
 //  * wave64; all bf16 I/O is loaded vectorized (uint4 = 16 B = 8 bf16),
 //    compute in f32; MFMA (mfma_f32_16x16x32/32x32x16_bf16) for the
 //    matmul-shaped kernels (prefill attention, projection GEMMs).
 //  * memory-bound ops target the HBM3E roofline (~6.3 TB/s achievable);
-//    the M<=512 decode projections are per-CU load-path/latency-bound, so
-//    gemm_proj pipelines both operands through LDS by global_load_lds.
+//    decode projections are bound by streaming W, or a CU's loads of x and W:
+//    k_gemm_rows loads straight into MFMA operands, k_gemm_tile moves both
+//    through a ring of tiles in LDS.
 //  * attention decode: 4-wave workgroup per (batch, kv_head, split), K and V
 //    streamed through registers; split-S partials where B*Hk is small.
 //  * exported as extern "C" with an explicit hipStream_t so launches are
@@ -428,7 +429,8 @@ k_gemm_skinny(bf16_t* __restrict__ out, float* __restrict__ ws,
     // hides the weight-stream latency (one wave per SIMD cannot — measured).
     // Per 256-k sub-slice the body is straight-line: issue all 8 B chunks
     // (16 B/lane, k-contiguous; not nontemporal: a load takes half a cache
-    // line, 24 rows of 9216 x 3072 in 8 parts 22.2 -> 19.6 us), stage the x panel into LDS coalesced
+    // line, 24 rows of 9216 x 3072 in 8 parts 22.2 -> 19.6 us), stage the x
+    // panel into LDS coalesced
     // (XOR-swizzled), barrier, 8 x MT MFMAs off ds_read_b128 fragments.
     const int lane = threadIdx.x & 63;
     const int wid = threadIdx.x >> 6;
@@ -584,8 +586,7 @@ k_gemm_rows(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
                 acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                     a[u], b[u][i], acc[i], 0, 0, 0);
     };
-    // (Guards in `add` itself, and a last batch inside the loop, made the
-    // compiler overwrite operands that were still to be used.)
+    // the last batch, the only one that may be short: the loop has no guards
     auto add_some = [&](bf16x8 (&a)[U], bf16x8 (&b)[U][NC], int n) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {

@@ -206,11 +206,12 @@ DEV_INLINE bool find_part(int b, int blocks, const int* pos, int last, int N,
 }
 
 // ===========================================================================
-// Decode. Block: a row (ws == null) or a part of a row's keys; tiles of 32 keys of all G value
-// heads go through LDS (16-byte pieces XOR-swizzled by the row), the next one
-// in flight. Scores: up to 16 heads of one value head against 16 keys are one
-// item, and a wave has one or two of the same heads; the weights meet in LDS,
-// and a wave then has all heads' weights against CW columns of one value head.
+// Decode. Block: a row (ws == null) or a part of a row's keys; tiles of 32 keys
+// of all G value heads go through LDS (16-byte pieces XOR-swizzled by the row),
+// the next one in flight. Scores: up to 16 heads of one value head against 16
+// keys are one item, and a wave has one or two of the same heads; the weights
+// meet in LDS, and a wave then has all heads' weights against CW columns of one
+// value head.
 //   ws: sums [blocks][G][H][P], of each row the first block and the number of
 //   its parts, int [N][2] (at 8 bytes there), and the weights' sums [blocks][H]
 // Bound by the tiles' way to LDS: a block fits a CU once (24 heads, 8 values of

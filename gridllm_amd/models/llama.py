@@ -201,9 +201,9 @@ class LlamaModel:
 
     def interleave_gateup(self) -> None:
         """Reorder each wgateup's rows into 128-row groups [64 gate |
-        64 up] so the fused-SwiGLU projection kernel (ops.gemm_proj with
-        fuse_swiglu) finds matching gate/up column pairs in every BN=128
-        block. GPU-only layout change; forward dispatches accordingly."""
+        64 up] so that a block of a fused-SwiGLU product (gemm_tile,
+        gemm_rows) has matching gate and up columns. GPU-only layout change;
+        forward dispatches accordingly."""
         if self.gateup_il or self.f_l % 64 != 0:
             return
         f = self.f_l

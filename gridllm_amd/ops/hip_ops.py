@@ -435,7 +435,7 @@ def gemm_rows(x: torch.Tensor, w: torch.Tensor,
               out: Optional[torch.Tensor] = None, fuse_swiglu: bool = False,
               glu: Glu = SWIGLU) -> torch.Tensor:
     """out[M,N] = x[M,K] @ w[N,K]^T, bf16, M <= 16: blocks of 16 columns over
-    all of K, without a workspace. fuse_swiglu: as in gemm_proj."""
+    all of K, without a workspace. fuse_swiglu: as in gemm_tile."""
     lib = _load()
     m, k = x.shape
     n = w.shape[0]
