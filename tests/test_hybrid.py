@@ -688,11 +688,13 @@ def test_trace_program(checkpoint, tmp_path):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("entering", [False, True])
 @pytest.mark.parametrize("dk,dv", [(64, 64), (128, 256), (64, 192), (192, 128),
                                    (64, 320)])
-def test_mlstm_chunk_sizes(dk, dv):
+def test_mlstm_chunk_sizes(dk, dv, entering):
     """Decode rows and portions of whole and cut chunks in one step, for heads
-    whose columns a block has all of (up to 256) or not."""
+    whose columns a block has all of (up to 256) or not; with normalisers that
+    enter a portion's first chunk, and without."""
     from gridllm_amd.ops import reference_hybrid
     h, nd, lens = 2, 2, (1, 64, 130)
     g = torch.Generator().manual_seed(dk + dv)
@@ -715,14 +717,20 @@ def test_mlstm_chunk_sizes(dk, dv):
     rows = torch.randn(n, h * 2 * (dk + dv), generator=g).to(torch.bfloat16)
     gates = torch.randn(n, 2 * h, generator=g) * 3
     S = torch.randn(5, h, dv + 1, dk, generator=g)
-    # normalisers that no query makes small: every denominator is its own
-    S[:, :, dv] = 0.0
+    # denominators that no query makes small: sums of what is not negative (which
+    # the norm behind them only shows with an eps of its size), or the chunk's own
+    eps = 1.0 if entering else 1e-5
+    if entering:
+        rows[:, :2 * h * dk] = rows[:, :2 * h * dk].abs()
+        S[:, :, dv] = S[:, :, dv].abs()
+    else:
+        S[:, :, dv] = 0.0
     m, norm = torch.rand(5, h, generator=g), torch.rand(h * dv,
                                                         generator=g) + 0.5
     S0, m0 = S.clone(), m.clone()
     want = reference_hybrid.mlstm(rows.float(), gates, S0, m0, norm,
                                   hops.StepMeta(segs=t(entries), **meta), dk,
-                                  dv, 15.0, 1e-5)
+                                  dv, 15.0, eps)
     dev = "cuda"
     S1, m1 = S.to(dev), m.to(dev)
     st = hops.StepMeta(chunks=t(chunks).to(dev), chunk_segs=t(segs).to(dev),
@@ -730,7 +738,7 @@ def test_mlstm_chunk_sizes(dk, dv):
                        **{k: v.to(dev) if torch.is_tensor(v) else v
                           for k, v in meta.items()})
     got = hops.mlstm(rows.to(dev), gates.to(dev), S1, m1, norm.to(dev), st, dk,
-                     dv, 15.0, 1e-5).cpu().float()
+                     dv, 15.0, eps).cpu().float()
     # bf16 result of a unit RMS row; bf16 weights of a chunk's values, 2^-9 each
     gate = torch.sigmoid(rows[:, -h * dv:].float()) * norm
     assert bool(((got - want).abs() <= 2 ** -8 * want.abs() +
