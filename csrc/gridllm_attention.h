@@ -125,7 +125,8 @@ struct HeadEpilogue {
 // Bound by HBM and, for few keys, by the chain load - scores - weights - sums.
 // 24 heads of 128 over 8, before (a key row per lane, f32 scores, waves waiting
 // for their own loads) and now: 24 rows of up to 6000 keys 193 -> 70 us
-// (5.1 TB/s), 256 of up to 384 99 -> 46 us (5.2 TB/s), one of 900 17 -> 9 us.
+// (5.1 TB/s), 256 of up to 384 99 -> 41 us (5.9 TB/s), one of 900 17 -> 9 us, in
+// a loop; among a step's other kernels the first two take 66 and 5, and 53.
 // V's loads go past the caches; K's, of half a cache line each, do not (both
 // halves would fetch it: 24 rows 73 us).
 // mfma_f32_16x16x32_bf16:

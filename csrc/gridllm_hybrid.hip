@@ -1427,7 +1427,9 @@ DEV_INLINE void store_normed(bf16_t* out, const f32x4 (&acc)[4][4],
 // head's columns here (out), the head's norm and gate follow at once; out and
 // CONST exclude each other. Bound by reading the state and the few steps'
 // latencies: 3500 tokens, 12 heads of 128 x 256: 92 us with tokens split over
-// the waves and 128 columns a block, and 28 of the norm behind it, now 57.
+// the waves and 128 columns a block, and 28 of the norm behind it, now 66 (8 of
+// it the gates' exponentials and divisions, which are not the hardware's: those
+// are off by 6e-8 |z|).
 template <bool CONST>
 __global__ void __launch_bounds__(256, 2)
 k_mlstm_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
@@ -1865,7 +1867,7 @@ DEV_INLINE f32x4 mfma_split(bf16x8 ah, bf16x8 al, bf16x8 bh, bf16x8 bl,
 // Bound by reading the state (128 KB a head and chunk of 128 x 256) and the
 // latencies between its few steps. 590 blocks of it: 78 us with tokens split
 // over the waves, each reading the whole state, and 22 of the norm behind it;
-// now 61, of which the gates take 18 and the scores' decays 11.
+// now 64, of which the gates take 21 and the scores' decays 11.
 #define GLA_SPAN 60.f
 __global__ void __launch_bounds__(256, 2)
 k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,

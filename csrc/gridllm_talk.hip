@@ -217,8 +217,9 @@ DEV_INLINE bool find_part(int b, int blocks, const int* pos, int last, int N,
 // Bound by the tiles' way to LDS: a block fits a CU once (24 heads, 8 values of
 // 128) and takes 3.4 us for a tile of 64 KB, 4.9 TB/s if all CUs have a block.
 // With a block per row, 160 rows of up to 1000 keys took 105 us, the longest
-// row's time, on 160 of 256 CUs; in parts they take 75, the combining kernel's 7
-// included, and rows of 1000 keys all, which are left whole, 114 (112).
+// row's time, on 160 of 256 CUs; in parts they take 75 with the combining kernel,
+// and rows of 1000 keys all, which are left whole, 114 (112). (One behind the
+// other in a loop; among a step's other kernels 74 and 8.)
 // ===========================================================================
 template <int P, int GP, int HB, int R>
 struct DecodeShape {
