@@ -440,10 +440,11 @@ class SlotSampler:
         if (logits.is_cuda and not need_filter
                 and os.environ.get("GRIDLLM_FUSED_SAMPLER", "1") != "0"):
             from gridllm_amd.ops import hip_ops
+            if slot_ids.dtype != torch.int64 or not slot_ids.is_cuda:
+                slot_ids = slot_ids.to(logits.device, torch.int64)
             return hip_ops.sample_gumbel_slots(
-                logits.contiguous(),
-                slot_ids.to(logits.device, torch.int64).contiguous(),
-                self.temps, self.seeds, self.draws, self.nongreedy)
+                logits.contiguous(), slot_ids.contiguous(), self.temps,
+                self.seeds, self.draws, self.nongreedy)
         temps = self.temps[slot_ids].unsqueeze(1)
         x = logits / temps
         v = logits.shape[1]

@@ -687,31 +687,40 @@ def _sample(logits, keys, temps, slots=None, seeds=None, draws=None,
             nongreedy=None) -> torch.Tensor:
     lib = _load()
     b, v = logits.shape
-    per_row = keys if slots is None else slots
-    n, dev = temps.numel(), logits.get_device()
-    ok = (dev >= 0 and logits.dtype == torch.float32 and logits.is_contiguous()
-          and temps.dtype == torch.float32 and per_row.numel() == b
-          and (slots is not None or n == b))
-    for t in (temps, per_row) if slots is None else \
-            (temps, per_row, seeds, draws, nongreedy):
-        ok = (ok and t.get_device() == dev and t.is_contiguous()
-              and t.dim() == 1 and (t is temps or t.dtype == torch.int64)
-              and (t is per_row or t.numel() == n))
-    if not ok:
+    f32, i64, dev, n = torch.float32, torch.int64, logits.get_device(), \
+        temps.shape
+    if slots is None:
+        ok = (keys.dtype is i64 and keys.shape == n == (b,)
+              and dev == keys.get_device() and keys.is_contiguous())
+    else:
+        ok = (slots.dtype is i64 and seeds.dtype is i64 and draws.dtype is i64
+              and nongreedy.dtype is i64 and slots.shape == (b,)
+              and len(n) == 1 and seeds.shape == n and draws.shape == n
+              and nongreedy.shape == n and dev == slots.get_device()
+              == seeds.get_device() == draws.get_device()
+              == nongreedy.get_device() and slots.is_contiguous()
+              and seeds.is_contiguous() and draws.is_contiguous()
+              and nongreedy.is_contiguous())
+    if not (ok and logits.dtype is f32 and temps.dtype is f32 and dev >= 0
+            and dev == temps.get_device() and logits.is_contiguous()
+            and temps.is_contiguous()):
         raise ValueError("sample_gumbel: f32 logits [B, V] and temps, int64 "
                          "keys [B], or slots [B] and vectors by slot of one "
                          "length, dense and on one GPU")
     if slots is not None:
-        _check_range("sample_gumbel.slots", slots, n)
+        _check_range("sample_gumbel.slots", slots, n[0])
     # four blocks a CU, of 2048 elements or more: 64 rows of 128256 take 21 us
     # in 16 segments, 190 in one (with exact logarithms)
     segments = max(1, min(1024 // max(1, b), v // 2048, 64))
     out = torch.empty(b, dtype=torch.int32, device=logits.device)
-    ws = torch.empty(b * segments, dtype=torch.int64, device=logits.device)
+    ws = torch.empty(b * segments, dtype=i64, device=logits.device)
+    at = (keys.data_ptr(), temps.data_ptr(), None, None, None, None) \
+        if slots is None else (
+            None, temps.data_ptr(), slots.data_ptr(), seeds.data_ptr(),
+            draws.data_ptr(), nongreedy.data_ptr())
     _check(lib.gl_sample_gumbel(
-        _stream(), _ptr(out), _ptr(ws), _ptr(logits), _ptr(keys), _ptr(temps),
-        _ptr(slots), _ptr(seeds), _ptr(draws), _ptr(nongreedy), b, v,
-        segments, n), "sample_gumbel")
+        _stream(), out.data_ptr(), ws.data_ptr(), logits.data_ptr(), *at, b, v,
+        segments, n[0]), "sample_gumbel")
     return out
 
 
