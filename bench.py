@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Flagship serving benchmark — the BASELINE.json headline metric.
+"""Flagship serving benchmark — the reference's headline metric.
 
 Default mode times the FULL serving path: HTTP /api/generate streaming
 through gateway -> scheduler -> bus -> worker -> engine -> direct stream

@@ -212,7 +212,7 @@ k_embed_norm(bf16_t* __restrict__ x, bf16_t* __restrict__ y,
 // ===========================================================================
 // RoPE (neox/llama split-half layout), in-place on q and k.
 //   q: [T, Hq, D]  k: [T, Hk, D]  (bf16)
-//   cos/sin: [max_seq, D/2] (f32, host-precomputed table — guide App. B)
+//   cos/sin: [max_seq, D/2] (f32, host-precomputed table)
 //   pos: [T] int32 absolute positions
 // Pair (t, h, i): (a,b) = (x[i], x[i+D/2]) -> (a*c - b*s, a*s + b*c)
 // Thread handles 2 consecutive pairs (4 B loads both halves).
@@ -406,13 +406,12 @@ k_kv_append(bf16_t* __restrict__ kc, bf16_t* __restrict__ vc,
 // of the roofline on these shapes (profiles/r01_decode_profile.md), so this
 // kernel streams W once, straight into MFMA B
 // fragments — both operands are k-contiguous, so fragments load directly
-// from HBM/L2 with no LDS staging (guide: "GEMV / M<=16 decode weights:
-// load straight to VGPRs"; generalized to M<=256 via 16-row MFMA tiles).
+// from HBM/L2 with no LDS staging (M <= 256 by 16-row MFMA tiles).
 //
 // mfma_f32_16x16x32_bf16 lane mapping used here:
 //   A[i][k]: lane l holds rows i = l&15, k = (l>>4)*8 + 0..7  (8 bf16 = 16 B)
 //   B[k][j]: lane l holds col  j = l&15, same k chunk
-//   D[i][j]: col j = l&15, row i = (l>>4)*4 + reg   (guide §3)
+//   D[i][j]: col j = l&15, row i = (l>>4)*4 + reg
 // Block = 4 waves; each wave owns 16 output columns (BN = 64 per block);
 // grid = (N/64) * splitk, k-slices 32-aligned; splitk > 1 accumulates f32
 // partials in ws, combined by k_gemm_combine.

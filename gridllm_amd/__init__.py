@@ -6,7 +6,7 @@ registry + Ollama/OpenAI-compatible gateway, with the inference engine
 implemented in-process on PyTorch-ROCm + hand-written CDNA4 (gfx950)
 HIP kernels instead of delegating to an external Ollama daemon.
 
-Layers (see SURVEY.md §1):
+Layers:
   L5 gateway     gridllm_amd.server.routes   (Ollama + OpenAI + native API)
   L4 orchestration gridllm_amd.server        (JobScheduler, WorkerRegistry)
   L3 message bus gridllm_amd.bus             (asyncio TCP pub/sub + KV; the

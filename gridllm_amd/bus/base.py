@@ -1,7 +1,7 @@
 """Control-plane message bus interface.
 
 The reference's entire inter-process protocol is Redis pub/sub + KV
-(SURVEY.md §2.3; reference: server/src/services/RedisService.ts,
+(reference: server/src/services/RedisService.ts,
 client/src/services/RedisConnectionManager.ts). This image ships no Redis,
 so the rebuild provides its own bus with the same semantics:
 

@@ -2,7 +2,7 @@
 
 Lets the whole stack (scheduler, N workers, gateway) run in one asyncio
 loop for tests — the reference had no such harness (its only test needed a
-live Redis + Ollama, SURVEY.md §4).
+live Redis + Ollama).
 """
 
 from __future__ import annotations

@@ -338,7 +338,7 @@ class TcpBus(Bus):
 
     async def publish(self, channel: str, payload: dict) -> None:
         """Fire-and-forget, like Redis pub/sub (at-most-once; the control
-        plane compensates with orphan-requeue — SURVEY.md §2.3). Awaiting a
+        plane compensates with orphan-requeue). Awaiting a
         per-message ack round-trip capped token streaming at ~2.6k msg/s."""
         if self._writer is None or self.closed:
             raise ConnectionError("bus not connected")

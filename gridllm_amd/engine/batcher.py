@@ -297,7 +297,7 @@ class Batcher:
                         except Exception as e:  # noqa: BLE001
                             log.logger.exception("decode step failed")
                             # retire the rows or their KV slots leak
-                            # permanently and admission wedges (ADVICE r1)
+                            # permanently and admission wedges
                             fail_live(e)
                         prune()
             elif inflight is not None:

@@ -3,7 +3,7 @@
 The reference's Ollama path flattens chat to "role: content" text
 (reference: server/src/routes/ollama.ts:366-370) while its OpenAI path does
 real chat (openai.ts:651-654). We template properly on BOTH paths
-(SURVEY.md §7 hard-part 6 recommendation) while keeping wire shapes intact.
+while keeping wire shapes intact.
 Families: Llama-3 header style (default) and ChatML (Qwen2.5 — the
 reference's CI model family)."""
 

@@ -5,7 +5,7 @@ The reference worker shells out to an external Ollama daemon over HTTP
 in-process: Llama-family models on PyTorch-ROCm with hand-written CDNA4
 kernels (gridllm_amd.ops), a slot-based KV cache in HBM3E, hipGraph-captured
 decode steps (bucketed batch sizes), and a full sampler. Tokens stream to a
-callback — no per-token HTTP/JSON hop (SURVEY.md §3.3 hot-loop fix).
+callback — no per-token HTTP/JSON hop.
 """
 
 from __future__ import annotations
@@ -176,7 +176,7 @@ class InferenceEngine:
             return False
         if self.tp.size == 1:
             return True
-        # TP decode is hipGraph-captured too (round-1 verdict weak 3): the
+        # TP decode is hipGraph-captured too: the
         # per-layer RCCL all-reduces are captured with the step. Needs the
         # nccl(=RCCL) backend — gloo collectives are host ops and cannot
         # be captured (the tp2-on-one-GPU CI configuration).
@@ -524,7 +524,7 @@ class InferenceEngine:
     def start_rows_async(self, items: list[tuple]) -> list["_Row"]:
         """Pipelined admission: prefill + first-token sampling LAUNCH but
         never sync — the admission's GPU wait stalled the decode pipeline
-        ~10% at c1024 (round-2 profile: 124 admission syncs x ~20 ms).
+        ~10% at c1024 (124 admission syncs x ~20 ms).
         First tokens are emitted by the NEXT collect_step (the submit
         that follows attaches this batch). Caller guarantees no
         constraint/penalty rows and a running pipeline (batcher checks)."""
@@ -601,8 +601,8 @@ class InferenceEngine:
                 if extra_stops:
                     stops += extra_stops
                 # Ollama default (num_predict -1/unset): generate until EOS
-                # or the context fills — NOT a fixed cap (round-1 verdict
-                # gap 4: a generate without num_predict must not truncate
+                # or the context fills — NOT a fixed cap (a generate
+                # without num_predict must not truncate
                 # where the reference stack would not)
                 max_new = opts.num_predict \
                     if opts.num_predict and opts.num_predict > 0 \
@@ -675,7 +675,7 @@ class InferenceEngine:
                 np.asarray(slots, dtype=np.int64))
         except Exception:
             # prefill failure: release every slot this batch allocated
-            # or capacity leaks permanently (ADVICE r1, medium)
+            # or capacity leaks permanently
             self.abort_rows(rows, locked=True)
             raise
         return rows, logits, slots_t
@@ -958,7 +958,7 @@ class InferenceEngine:
 
     def _sync_cancel(self, rows: Sequence[_Row]) -> None:
         """Under TP every rank must retire the same rows at the same step, or
-        the next collective deadlocks (SURVEY.md §7 hard-part 5). Rank 0 owns
+        the next collective deadlocks. Rank 0 owns
         the cancel events; the decision is broadcast and applied via
         force_cancel on all ranks (including rank 0 — its own event could
         flip between broadcast and emit otherwise)."""

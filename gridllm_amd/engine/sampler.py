@@ -156,8 +156,7 @@ class BatchPlan:
         # ONE packed H2D per composition change instead of ~8 per-field
         # tensor() calls; the per-step key math runs fully ON DEVICE
         # (draws_dev += 1 after each draw) — the per-step host->device key
-        # upload measured 1.7 ms/step of GPU-sync stalls at c192 (round-2
-        # GPU profile, lt_worker_batcher.prof)
+        # upload measured 1.7 ms/step of GPU-sync stalls at c192
         host = np.zeros((6, b), dtype=np.float64)
         g = np.zeros(b, dtype=bool)
         seeds = np.zeros(b, dtype=np.int64)
@@ -354,7 +353,7 @@ class SlotSampler:
     The BatchPlan cache keyed on batch composition still rebuilt (a
     per-row Python loop + H2D uploads) nearly EVERY step under serving
     churn — at c=192 each step retires and admits rows, so the
-    composition never repeats (round-2 GPU profile: plan refresh 1.5 s of
+    composition never repeats (measured: plan refresh 1.5 s of
     an 11 s decode-thread window). Here every per-row constant lives in a
     device array indexed by the row's KV slot:
       * admission writes the new rows' parameters once (one packed H2D +

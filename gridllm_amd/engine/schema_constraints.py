@@ -211,8 +211,8 @@ class _Str:
         self.done = False
         # surrogate-pair escapes: a \uD800-\uDBFF escape counts ONE code
         # point together with the \uDC00-\uDFFF escape that MUST follow
-        # (pairs were counted as 2 and a lone
-        # high surrogate could be force-closed into invalid text)
+        # (counted as 2, a lone high surrogate could be force-closed into
+        # invalid text)
         self.pending_high = False      # inside a pair, low half owed
         self.hex0 = 0                  # first hex digit of current escape
         self.is_high = False           # current escape is a high surrogate

@@ -82,7 +82,7 @@ class KVCache:
         """HOST-ONLY bookkeeping: seq_lens/rope_off for the slot are
         (re)initialized by the next prefill's batched scatter — a per-slot
         scalar device write here measured ~0.5 ms of stream-sync stall per
-        call under serving load (round-2 GPU profile)."""
+        call under serving load."""
         if not self._free:
             raise RuntimeError("KV cache: no free slots")
         return self._free.pop()
@@ -234,7 +234,7 @@ class LlamaModel:
         """Load HF-layout llama weights (model.safetensors or sharded
         model-*-of-*.safetensors in `path`) into the fused TP-sharded
         layout. Each rank reads only its shard slice. Returns the number
-        of tensors consumed. (the engine-side analog of
+        of tensors consumed. (The engine-side analog of
         checkpoint/resume — the reference had none, weights lived inside
         Ollama.)"""
         import glob as _glob
@@ -415,8 +415,8 @@ class LlamaModel:
         idx = self.up.upload(np.stack([pos_np, slot_np]))
         pos, slot_t = idx[0], idx[1]
         # varlen batched attention (one meta-driven kernel launch per layer
-        # instead of a per-sequence Python loop — the round-2 profile's
-        # 36 ms-per-admission hot spot); meta rows: {q_off, len, slot, q0}
+        # instead of a per-sequence Python loop of 36 ms per admission);
+        # meta rows: {q_off, len, slot, q0}
         meta = None
         if (tokens.is_cuda and self.dtype == torch.bfloat16
                 and s.head_dim in (64, 128)):
@@ -449,8 +449,7 @@ class LlamaModel:
                          if li + 1 < len(self.layers) else self.final_norm)
             normed, resid = self._joined(act, lw.wdown, next_norm, resid)
         # ONE scatter instead of k per-sequence device writes (each is a
-        # serialized H2D launch — 15 ms of host time per admission batch
-        # in the round-2 serving profile)
+        # serialized H2D launch — 15 ms of host time per admission batch)
         import numpy as _np
         host = _np.asarray([[sl for sl in slots], lens,
                             [b - 1 for b in bounds[1:]]], dtype=_np.int64)

@@ -2,7 +2,7 @@
 
 The reference has no model definitions at all (compute lived in Ollama);
 these specs reproduce the Llama-family architectures its deployments serve
-via Ollama model tags (BASELINE.json configs: llama3.2:1b, llama3.2:3b,
+via Ollama model tags (llama3.2:1b, llama3.2:3b,
 llama3:70b).
 """
 

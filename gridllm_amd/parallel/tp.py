@@ -1,10 +1,10 @@
 """Tensor-parallel context: RCCL process groups over xGMI.
 
 One process per GPU; `torch.distributed` backend "nccl" IS RCCL on ROCm.
-The TP group fronts the registry as a single worker (SURVEY.md §5.8):
+The TP group fronts the registry as a single worker:
 rank 0 talks to the control plane, all ranks join every collective.
 
-The reference has no collectives at all (SURVEY.md §2.4) — this module is
+The reference has no collectives at all — this module is
 the xGMI data plane the rebuild adds. Decode all-reduce messages are small
 (hidden*batch*2B, tens of kB), so latency dominates and we leave algorithm
 choice to RCCL per-size; bucket tuning happens in bench, not here.
@@ -90,8 +90,7 @@ def init_tp_from_env(backend: str = "") -> TPContext:
     if not dist.is_initialized():
         if not backend:
             backend = "nccl" if torch.cuda.is_available() else "gloo"
-        # bounded collectives make TP-group failure ATOMIC (SURVEY.md §7
-        # hard-part 5): if any rank dies, the others' collectives time out
+        # bounded collectives make TP-group failure ATOMIC: if any rank dies, the others' collectives time out
         # and abort the whole process -> the registry removes the worker
         # and in-flight jobs orphan-requeue, instead of hanging forever.
         # (RCCL honors this via the process-group watchdog.)

@@ -1,11 +1,11 @@
 """Prometheus metrics for the gateway/scheduler.
 
 The reference parsed METRICS_ENABLED but never implemented metrics
-(client/src/config/index.ts:47, unused — SURVEY.md §5.5). Here /metrics is
+(client/src/config/index.ts:47, unused). Here /metrics is
 real: job lifecycle counters off the scheduler's event emitter, queue /
 fleet gauges off live stats, a TTFT histogram observed at the gateway's
 streaming path, and a generated-token counter (the two halves of the
-headline metric, BASELINE.md)."""
+headline metric)."""
 
 from __future__ import annotations
 

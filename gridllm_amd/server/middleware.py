@@ -2,7 +2,7 @@
 
 The reference shipped a fixed-window in-memory limiter with X-RateLimit
 headers but never mounted it (client/src/middleware/rateLimiter.ts:63-130,
-unmounted per SURVEY.md §2.2 C9). Here it is mounted on the gateway,
+unmounted). Here it is mounted on the gateway,
 disabled by default (limit 0) and enabled via RATE_LIMIT_MAX_REQUESTS /
 RATE_LIMIT_WINDOW_MS, matching the reference's env knob names.
 """

@@ -9,7 +9,7 @@ Reimplements the semantics of the reference's WorkerRegistry
   * re-registration request on unknown heartbeat (:261-323, :496-515)
   * busy/online flip at max_concurrent_jobs (:421-454)
 Differences: tier/resource data is actually populated by workers
-(reference gap), and the bus itself announces dropped
+(a gap of the reference), and the bus itself announces dropped
 worker connections.
 """
 

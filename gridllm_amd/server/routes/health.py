@@ -2,7 +2,7 @@
 
 /health (:16-28), /health/live (:31-39), /health/ready (:42-73),
 /health/system (:76-111), /health/workers (:114-139), /health/jobs (:142-169)
-— extended with per-worker GPU telemetry (reference had none, SURVEY §5.5).
+— extended with per-worker GPU telemetry (reference had none).
 """
 
 from __future__ import annotations

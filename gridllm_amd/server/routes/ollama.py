@@ -134,9 +134,8 @@ def _stream_ndjson(scheduler: JobScheduler, req: InferenceRequest,
             task.cancel()
             if not task.done():
                 # client disconnected mid-stream: abort the job on the
-                # worker too, or it keeps generating to completion (the
-                # SSE path got this in round 1 but
-                # the NDJSON path did not)
+                # worker too, or it keeps generating to completion, as on
+                # the SSE path
                 try:
                     await scheduler.cancel_job(req.id)
                 except Exception:  # noqa: BLE001
@@ -315,7 +314,7 @@ def build_router(scheduler: JobScheduler, registry: WorkerRegistry) -> APIRouter
 
     # ------------------------------------------------- version / show / ps
     # (beyond reference parity: the reference proxied only
-    # generate/chat/tags/embed — SURVEY.md §2.2-S5 — but Ollama SDKs probe
+    # generate/chat/tags/embed, but Ollama SDKs probe
     # these on connect, so a drop-in gateway should answer them)
 
     @r.get("/api/version")

@@ -68,7 +68,7 @@ def _usage(res: dict) -> dict:
 
 def _usage_n(results: list) -> dict:
     """Usage across n samples of ONE prompt: the shared prompt counts once;
-    completion tokens sum (OpenAI semantics — round-1 advisor finding)."""
+    completion tokens sum (OpenAI semantics)."""
     p = int((results[0].get("timings") or {}).get("prompt_eval_count", 0))
     c = sum(int((r.get("timings") or {}).get("eval_count", 0))
             for r in results)
@@ -176,7 +176,6 @@ def build_router(scheduler: JobScheduler, registry: WorkerRegistry) -> APIRouter
                 if not task.done():
                     # client disconnected mid-stream: abort the job on the
                     # worker too, or it keeps generating to completion
-                    #
                     try:
                         await scheduler.cancel_job(req.id)
                     except Exception:  # noqa: BLE001
@@ -377,7 +376,7 @@ def build_router(scheduler: JobScheduler, registry: WorkerRegistry) -> APIRouter
     @r.post("/v1/embeddings")
     async def embeddings(request: Request):
         # Ollama's OpenAI compat exposes this; the reference proxied only
-        # completions/chat/models (SURVEY.md §2.2-S6) — drop-in value-add
+        # completions/chat/models — drop-in value-add
         body = await request.json()
         model = body.get("model", "")
         _validate(model)

@@ -230,7 +230,7 @@ class StreamChunk:
 
 @dataclass
 class GPUStats:
-    """Per-GPU telemetry a worker reports (reference had none — SURVEY §2.2 C10)."""
+    """Per-GPU telemetry a worker reports (reference had none)."""
 
     device: int = -1
     name: str = "cpu"
@@ -287,7 +287,7 @@ class JobAssignment:
 
 
 # ---------------------------------------------------------------------------
-# Bus channel / key naming — the wire protocol of SURVEY.md §2.3, preserved.
+# Bus channel / key naming — the reference's wire protocol, preserved.
 # ---------------------------------------------------------------------------
 
 class Channels:

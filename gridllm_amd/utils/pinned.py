@@ -2,7 +2,7 @@
 
 A pageable `.to(device)` both enqueues BEHIND everything already on the
 stream and blocks the host until the copy lands — ~1.5 ms per call
-against a busy decode stream (round-2 serving profiles). Staging through
+against a busy decode stream. Staging through
 a reusable pinned buffer with non_blocking=True enqueues without a host
 stall. Buffers are pooled per rounded capacity in a ring of 4, each with the
 event of its last copy: a buffer is rewritten only when that copy is done, so

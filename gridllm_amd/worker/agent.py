@@ -190,7 +190,7 @@ class WorkerAgent:
             await asyncio.sleep(interval)
 
     def _check_wedge(self) -> None:
-        """TP group failover must be atomic (SURVEY §7 hard-part 5): a
+        """TP group failover must be atomic: a
         collective that hangs (peer rank dead/stuck) blocks the batcher
         thread while THIS loop keeps heartbeating, so the scheduler would
         keep routing jobs to a wedged group forever. When the batcher has
@@ -246,8 +246,8 @@ class WorkerAgent:
 
     async def _h_control(self, _ch: str, payload: dict) -> None:
         """Maintenance verbs (pause/resume/drain) — adopted from the
-        reference's dead broker path (BrokerClientService.ts:568-657,
-        SURVEY.md §2.2-C6) onto the live worker."""
+        reference's dead broker path (BrokerClientService.ts:568-657)
+        onto the live worker."""
         verb = payload.get("type")
         if verb == "pause":
             self.paused = True
@@ -325,7 +325,7 @@ class WorkerAgent:
                 done_ev.set()
 
         # thinking mode (Ollama `think: true`, reference forwards it at
-        # server/src/routes/ollama.ts:216-239 — round-1 verdict gap 3:
+        # server/src/routes/ollama.ts:216-239;
         # executed here, not silently ignored)
         think = bool((req.metadata or {}).get("think"))
         stream = None

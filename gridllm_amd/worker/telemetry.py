@@ -15,8 +15,7 @@ from gridllm_amd.types import GPUStats
 
 # TTL cache: gpu_stats runs on EVERY worker status publish (2x per job)
 # and hipMemGetInfo measured ~1.3 ms against a busy device — 2.2 s of
-# the worker loop thread at a 1024-deep admission ramp (round-2 GPU
-# profile, lt_worker_loop.prof). Telemetry freshness of 2 s is plenty
+# the worker loop thread at a 1024-deep admission ramp. Telemetry freshness of 2 s is plenty
 # for tier routing and /health.
 _CACHE: dict[int, tuple[float, GPUStats]] = {}
 _TTL_S = 2.0

@@ -7,14 +7,14 @@ batching loop: one small control broadcast per decode iteration (gloo side
 channel, parallel/tp.py) carries that iteration's admissions, then every
 rank executes the identical start_rows/step_rows sequence so all RCCL
 collectives line up. Rows join and leave the live batch in lockstep —
-a long generation no longer blocks new arrivals (
-the old design broadcast whole run-to-completion waves).
+a long generation no longer blocks new arrivals (as
+broadcasting whole run-to-completion waves would).
 
 The decode step itself is hipGraph-captured per batch bucket INCLUDING
 the per-layer all-reduces (engine._graph_ok allows tp>1 on nccl).
 
 No reference analog (the reference had zero parallelism beyond request
-sharding — SURVEY.md §2.4); design per SURVEY.md §5.8 / §7 step 6.
+sharding).
 
 Determinism across ranks:
   * logits are bitwise-identical on every rank (all-reduced activations,
@@ -74,7 +74,7 @@ class TPBatcher(Batcher):
             # checks it): a hung collective blocks THIS thread while the
             # asyncio loop keeps heartbeating — without the stamp the
             # scheduler would keep routing jobs to a wedged group
-            # (SURVEY §7 hard-part 5: group failover must be atomic)
+            # (group failover must be atomic)
             self.last_progress = _time.monotonic()
             self.busy = bool(live)
             arrivals: list[_Pending] = []

@@ -3,7 +3,7 @@
 continuous traffic while random faults fire — SIGKILL+respawn a worker,
 pause/resume via the control channel. Asserts NO request is lost: every
 submitted request must complete (orphan requeue + retries make worker
-death invisible to the client, SURVEY.md §3.5 / §5.3 — the reference had
+death invisible to the client; the reference had
 the recovery path but no injection tooling to exercise it).
 
 Usage: python scripts/chaos.py [--duration 30] [--workers 2]
@@ -71,8 +71,8 @@ async def drive(base: str, args, stats: dict, stop: asyncio.Event):
             # fixed arrival rate on a slow host built an unbounded
             # semaphore backlog that could not drain inside the post-run
             # wait and showed up as FALSE "lost" requests (the server
-            # side had completed everything it was given — box repro:
-            # gpurun_out/r02t_chaos_cpu.log vs /inference/queue stats)
+            # side had completed everything it was given, by
+            # /inference/queue stats)
             if len(tasks) < args.concurrency * 2:
                 t = asyncio.ensure_future(one(i))
                 tasks.add(t)

@@ -1,6 +1,6 @@
 #!/usr/bin/env python3
 """Serving-path load test: real server process + real worker process, driven
-through HTTP /api/generate streaming — measures the BASELINE metric on the
+through HTTP /api/generate streaming — measures the headline metric on the
 FULL path (gateway -> scheduler -> bus -> worker -> engine -> stream back),
 not just the engine loop.
 
@@ -243,7 +243,7 @@ def main():
                     help="DP workers; worker i pins cuda:i")
     ap.add_argument("--same-device", action="store_true",
                     help="all DP workers share --device (single-GPU DP "
-                         "validation, BASELINE config 3 on one lease)")
+                         "validation)")
     args = ap.parse_args()
 
     import torch

@@ -1,6 +1,5 @@
 #!/usr/bin/env python3
-"""Mixed-fleet routing validation on ONE GPU (single
-lease): a server + two workers serving DIFFERENT models (llama3.2:3b and
+"""Mixed-fleet routing validation on ONE GPU: a server + two workers serving DIFFERENT models (llama3.2:3b and
 llama3.2:1b) on the same device. Drives both models concurrently over
 /api/generate, asserts model-aware routing (each job lands on the worker
 advertising the model), then SIGKILLs the 1b worker mid-load and asserts

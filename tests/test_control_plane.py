@@ -1,6 +1,6 @@
 """Scheduler + registry semantics on the in-memory bus (fast timers).
 
-Covers the riskiest logic the reference left untested (SURVEY.md §4):
+Covers the riskiest logic the reference left untested:
 priority ordering, least-loaded selection, retries, orphan requeue-at-front,
 heartbeat-timeout removal, cancellation, streaming channels, crash-resume.
 """
@@ -324,7 +324,7 @@ async def test_registry_rehydration():
 
 @pytest.mark.asyncio
 async def test_mixed_fleet_model_aware_routing():
-    """Heterogeneous fleet (BASELINE config #5): workers advertising
+    """Heterogeneous fleet: workers advertising
     different models; each request lands only on a worker holding its
     model, and a multi-model worker serves both."""
     core = MemoryBusCore()

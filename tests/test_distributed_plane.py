@@ -1,10 +1,9 @@
-"""Round-2 control/data-plane split:
+"""Control/data-plane split:
 
 * standalone durable bus (`python -m gridllm_amd.bus`) — kill -9 the
   SERVER process mid-load, restart it against the surviving bus, and the
   queued jobs still complete (the reference's external-Redis guarantee,
-  docker-compose.yml:12-30 + JobScheduler.ts:82-126
-  missing item 2);
+  docker-compose.yml:12-30 + JobScheduler.ts:82-126);
 * detached gateway replicas (`python -m gridllm_amd.gateway`) — a
   replica serves the full API against a remote scheduler over the bus,
   with token chunks arriving on its own direct stream plane;
@@ -549,8 +548,8 @@ def test_gateway_replica_survives_bus_restart(tmp_path):
 
 def test_ndjson_client_disconnect_cancels_job(durable_stack):
     """Abruptly close the TCP connection mid-/api/generate NDJSON
-    stream: the gateway must cancel the job on the worker (SSE got this
-    in round 1; the NDJSON path kept generating to completion). The
+    stream: the gateway must cancel the job on the worker, as on the
+    SSE path. The
     fixture worker decodes at 0.25 s/step, so an uncancelled job holds
     active_jobs for minutes."""
     import socket as _socket

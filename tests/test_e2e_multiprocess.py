@@ -1,10 +1,10 @@
 """Full multi-process end-to-end: real server process (TCP bus + uvicorn
 HTTP) + 2 real worker processes (tiny CPU engines), driven over HTTP.
 
-This is the reference's CI scenario (SURVEY.md §4: redis+server+client
+This is the reference's CI scenario (redis+server+client
 full-stack) but self-contained, plus the chaos test the reference never had:
 SIGKILL a busy worker and assert the orphaned request completes on the
-survivor (SURVEY.md §3.5 semantics).
+survivor.
 """
 
 import json
@@ -213,7 +213,7 @@ def test_chaos_sigkill_busy_worker_orphan_requeue(cluster):
 def test_chaos_sigkill_during_streaming(cluster):
     """SIGKILL a worker mid-STREAM: the orphaned job requeues and the
     ORIGINAL streaming HTTP response keeps going until a final done record
-    arrives from the survivor (SURVEY.md §3.5: the job:result subscriber
+    arrives from the survivor (the job:result subscriber
     survives the worker)."""
     # w-a was killed by the previous test on some orderings; use whatever
     # workers remain and spawn a fresh disposable one to kill

@@ -316,7 +316,7 @@ def test_format_json_constrained_output():
 def test_no_slot_leak_on_prefill_failure(engine):
     """A prefill (or first-sample) failure must release every slot the
     batch allocated — otherwise transient faults permanently shrink
-    worker capacity (round-1 advisor finding, medium)."""
+    worker capacity."""
     free0 = engine.model.cache.n_free
     orig = engine.model.forward_prefill_batch
 

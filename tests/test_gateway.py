@@ -613,7 +613,7 @@ def test_think_splitter_units():
 
 
 def test_think_generate_and_chat(client):
-    """think:true is EXECUTED (round-1 verdict gap 3): generation starts
+    """think:true is EXECUTED: generation starts
     in a think block and the response carries a thinking field."""
     r = client.post("/api/generate", json={
         "model": "tiny", "prompt": "why?", "think": True, "stream": False,
@@ -655,7 +655,7 @@ def test_think_streaming_chunks(client):
 
 def test_default_num_predict_is_ctx_bounded(client):
     """Without num_predict, generation runs until EOS or the context
-    fills (Ollama default) — not a fixed 128 cap (verdict gap 4)."""
+    fills (Ollama default) — not a fixed 128 cap."""
     r = client.post("/api/generate", json={
         "model": "tiny", "prompt": "long", "stream": False,
         "options": {"temperature": 0.0}})

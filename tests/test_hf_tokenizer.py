@@ -1,7 +1,7 @@
 """HF (multi-byte BPE) tokenizer support: byte-exact token_bytes mapping
 and token-level format="json" enforcement over the byte automaton
-(engine/constraints.py::mask_logits_token_level) — closes the round-1
-limitation where the json flag was only enforced for the byte tokenizer."""
+(engine/constraints.py::mask_logits_token_level) (not for
+the byte tokenizer alone)."""
 
 import json
 

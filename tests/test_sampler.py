@@ -131,8 +131,8 @@ def test_vectorized_penalties_match_single_row():
 
 def test_batched_distribution_matches_softmax():
     """Empirical distribution of the counter-hash Gumbel sampler matches
-    softmax(logits) (locks in the RNG quality that was verified manually
-    in round 1: splitmix64-hash noise, max dev ~0.002 at N=8000)."""
+    softmax(logits) (locks in the RNG quality that was verified manually:
+    splitmix64-hash noise, max dev ~0.002 at N=8000)."""
     from gridllm_amd.engine.sampler import sample_batch_vectorized
     torch.manual_seed(0)
     lg = torch.randn(16)

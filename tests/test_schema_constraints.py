@@ -252,7 +252,7 @@ def test_string_length_bounds():
 
 def test_surrogate_pair_escapes():
     """\\uXXXX surrogate-pair escapes count ONE code point; lone
-    surrogates are unreachable (round-1 advisor finding)."""
+    surrogates are unreachable."""
     sch = {"type": "string", "maxLength": 1}
     # an astral char written as a surrogate-pair escape fits maxLength 1
     pair = b'"\\ud83d\\ude00"'

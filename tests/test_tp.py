@@ -244,8 +244,8 @@ def _tp_interleave_worker(rank: int, world: int, port: int, q):
 
 def test_tp_continuous_batching_interleaves():
     """A short request submitted while a long one is mid-decode under TP
-    must JOIN the live batch and finish first (
-    the old TP path ran whole waves to completion)."""
+    must JOIN the live batch and finish first,
+    not wait for whole waves to complete."""
     ctx = mp.get_context("spawn")
     q = ctx.SimpleQueue()
     procs = [ctx.Process(target=_tp_interleave_worker,
@@ -318,8 +318,7 @@ def test_tp2_gpu_logits_match_tp1():
     """TP=2 on ONE MI355X (2 procs, gloo collectives, shared cuda:0):
     per-step logits of a forced-token decode must match the TP=1 engine
     within bf16 all-reduce tolerance — the TP shard math runs the REAL
-    HIP kernels on both ranks (TP had only ever
-    run on CPU). Top-1 id must agree wherever the TP=1 margin is clear."""
+    HIP kernels on both ranks. Top-1 id must agree wherever the TP=1 margin is clear."""
     import torch as _t
     if not _t.cuda.is_available():
         pytest.skip("GPU required")
