@@ -360,8 +360,8 @@ class LlamaModel:
         return_hidden, returns (logits, mean-pooled final hidden [H] f32)."""
         s = self.spec
         t = tokens.shape[0]
-        pos, slot_t = ops.prompt_positions(t, slot, start_pos,
-                                           self.cache.max_seq, self.device)
+        pos, slot_t = ops.prompt_positions(
+            t, slot, start_pos, self.cache.seq_lens, self.cache.max_seq)
         resid, normed = ops.embed_norm(tokens, self.embed,
                                        self.layers[0].attn_norm, s.norm_eps)
         for li, lw in enumerate(self.layers):

@@ -58,13 +58,14 @@ def advance_lengths(seq_lens: torch.Tensor, slot_map: torch.Tensor) -> None:
     reference.advance_lengths(seq_lens, slot_map)
 
 
-def prompt_positions(t: int, slot: int, start: int, smax: int, device
-                     ) -> Tuple[torch.Tensor, torch.Tensor]:
-    """Positions and cache places of t tokens from `start` on."""
-    if torch.device(device).type == "cuda":
+def prompt_positions(t: int, slot: int, start: int, seq_lens: torch.Tensor,
+                     smax: int) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Positions and cache places of t tokens from `start` on, of a slot of
+    seq_lens."""
+    if _on_gpu(seq_lens):
         from gridllm_amd.ops import hip_ops
-        return hip_ops.prompt_positions(t, slot, start, smax, device)
-    return reference.prompt_positions(t, slot, start, smax, device)
+        return hip_ops.prompt_positions(t, slot, start, seq_lens, smax)
+    return reference.prompt_positions(t, slot, start, seq_lens, smax)
 
 
 def prompt_end(t: int, slot: int, start: int, seq_lens: torch.Tensor,

@@ -180,11 +180,13 @@ def advance_lengths(seq_lens: torch.Tensor, slot_map: torch.Tensor) -> None:
         seq_lens.shape[0]), "advance_lengths")
 
 
-def prompt_positions(t: int, slot: int, start: int, smax: int, device
-                     ) -> tuple[torch.Tensor, torch.Tensor]:
+def prompt_positions(t: int, slot: int, start: int, seq_lens: torch.Tensor,
+                     smax: int) -> tuple[torch.Tensor, torch.Tensor]:
     """Positions start .. start + t - 1 and cache places slot * smax + those,
-    int32 [t]."""
-    out = torch.empty(2, t, dtype=torch.int32, device=device)
+    int32 [t], of a slot of seq_lens."""
+    if not (0 <= slot < seq_lens.shape[0]):
+        raise IndexError(f"slot {slot} of {seq_lens.shape[0]}")
+    out = torch.empty(2, t, dtype=torch.int32, device=seq_lens.device)
     _check(_load().gl_prompt_positions(
         _stream(), _ptr(out[0]), _ptr(out[1]), slot, start, t, smax),
         "prompt_positions")

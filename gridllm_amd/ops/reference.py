@@ -48,10 +48,14 @@ def rope_tables(head_dim: int, max_seq: int, theta: float = 500000.0,
     return freqs.cos().contiguous(), freqs.sin().contiguous()
 
 
-def prompt_positions(t: int, slot: int, start: int, smax: int, device=None
-                     ) -> Tuple[torch.Tensor, torch.Tensor]:
-    """Positions start .. start + t - 1 and slot * smax + those."""
-    pos = torch.arange(start, start + t, dtype=torch.int32, device=device)
+def prompt_positions(t: int, slot: int, start: int, seq_lens: torch.Tensor,
+                     smax: int) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Positions start .. start + t - 1 and slot * smax + those, of a slot of
+    seq_lens."""
+    if not (0 <= slot < seq_lens.shape[0]):
+        raise IndexError(f"slot {slot} of {seq_lens.shape[0]}")
+    pos = torch.arange(start, start + t, dtype=torch.int32,
+                       device=seq_lens.device)
     return pos, pos + slot * smax
 
 

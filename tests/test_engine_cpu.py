@@ -591,3 +591,16 @@ def test_a_step_that_raises_can_be_repeated(step, monkeypatch):
     after = before.clone()
     after[slot] += 2 if step == "prompt" else 1
     assert torch.equal(m.cache.seq_lens, after)
+
+
+def test_a_prompt_for_no_slot_writes_nothing(monkeypatch):
+    """A slot that the cache has not is refused ahead of the first layer."""
+    from gridllm_amd import ops
+    from gridllm_amd.models.llama import LlamaModel
+    from gridllm_amd.models.registry import get_spec
+    m = LlamaModel(get_spec("tiny"), device="cpu", dtype="fp32", kv_slots=3,
+                   max_seq=64)
+    monkeypatch.setattr(ops, "rope_kv", None)       # not reached
+    for slot in (m.cache.seq_lens.shape[0], -1):
+        with pytest.raises(IndexError):
+            m.forward_prefill(torch.tensor([5, 6]), slot)

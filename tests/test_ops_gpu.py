@@ -191,16 +191,19 @@ def test_advance_lengths_gpu(dev, b):
 @pytest.mark.parametrize("start", [0, 5])
 def test_prompt_positions_gpu(dev, t, start):
     from gridllm_amd.ops import hip_ops
-    for x, y in zip(hip_ops.prompt_positions(t, 2, start, 1024, dev),
-                    R.prompt_positions(t, 2, start, 1024)):
-        assert torch.equal(x.cpu(), y)
     a, b = (torch.full((4,), 7, dtype=torch.int32) for _ in range(2))
     x, y = a.to(dev), b.to(dev)
+    for i, j in zip(hip_ops.prompt_positions(t, 2, start, x, 1024),
+                    R.prompt_positions(t, 2, start, a, 1024)):
+        assert torch.equal(i.cpu(), j)
     hip_ops.prompt_end(t, 2, start, x, y)
     R.prompt_end(t, 2, start, a, b)
     assert torch.equal(x.cpu(), a) and torch.equal(y.cpu(), b)
-    with pytest.raises(IndexError):
-        hip_ops.prompt_end(t, 4, start, x, y)
+    for slot in (4, -1):
+        with pytest.raises(IndexError):
+            hip_ops.prompt_positions(t, slot, start, x, 1024)
+        with pytest.raises(IndexError):
+            hip_ops.prompt_end(t, slot, start, x, y)
 
 
 @pytest.mark.parametrize("n,h", [(1, 8), (5, 896), (3, 2056), (2, 8192),
