@@ -116,7 +116,8 @@ def rope_kv(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
     k = qkv[:, hq * d:(hq + hk) * d].reshape(n, hk, d)
     v = qkv[:, (hq + hk) * d:].reshape(n, hk, d).contiguous()
     q, k = rope(q.contiguous(), k.contiguous(), cos, sin, pos)
-    kv_append(kcache, vcache, k, v, slot)
+    if hk:
+        kv_append(kcache, vcache, k, v, slot)
     return q
 
 

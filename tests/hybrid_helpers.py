@@ -128,3 +128,27 @@ class Bytes:
             def push(self, i):
                 return tok.decode([i])
         return D()
+
+
+def check_wanted_rows_alone(build, tokens, run):
+    """A step that wants few of its rows, whose last layer stops at the mixer for
+    the others, leaves the caches of one that wants all, and the same logits."""
+    long, short, none = tokens(150, seed=1), tokens(21, seed=2), tokens(9, seed=3)
+    few = [(long, [149]), (short, [20, 3, 3]), (none, [])]
+
+    def step(wanted):
+        m = build()
+        out = m.forward_step([(m.cache.alloc(0), ids, w) for ids, w in wanted])
+        c = m.cache
+        return out.cpu(), [t[1:] if t is not c.S[i] else t for i in range(len(
+            m.layers)) for t in (c.k[i], c.v[i], c.lat[i], c.S[i])
+            if t is not None]
+
+    want, left = step([(ids, list(range(len(ids)))) for ids, _ in few])
+    got, mine = step(few)
+    close(got, want[[149, 170, 153, 153]], run, exact=1e-4, coarse=0.1,
+          odd=0.25)
+    out, quiet = step([(ids, []) for ids, _ in few])
+    assert out.shape == (0, want.shape[1])
+    for a, b, c in zip(left, mine, quiet):
+        assert torch.equal(a, b) and torch.equal(a, c)

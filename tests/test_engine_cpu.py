@@ -254,6 +254,35 @@ def test_context_shift_matches_fresh_prefill():
             (la - lb).abs().max().item()
 
 
+def test_last_layer_of_wanted_rows_alone():
+    """A long prompt's last layer runs for its last token alone: logits and
+    caches are those of the pass that runs it for all (which hidden states
+    need), for a prompt, one that continues, and a batch."""
+    import torch as T
+    from gridllm_amd.models.llama import LlamaModel
+    from gridllm_amd.models.registry import get_spec
+
+    spec = get_spec("tiny", 1024)
+    models = [LlamaModel(spec, device="cpu", dtype="fp32", kv_slots=6,
+                         max_seq=1024) for _ in range(2)]
+    T.manual_seed(1)
+    a, b, c = (T.randint(0, spec.vocab, (n,)) for n in (300, 260, 7))
+    got, want = [], []
+    for m, out, hidden in zip(models, (got, want), (False, True)):
+        for run in (lambda: m.forward_prefill(a, 2, 0, hidden),
+                    lambda: m.forward_prefill(b, 2, 300, hidden),
+                    lambda: m.forward_prefill_batch([c, a, b], [1, 4, 3],
+                                                    hidden)):
+            r = run()
+            out.append(r[0] if hidden else r)
+    for x, y in zip(got, want):
+        assert x.shape == y.shape and (x - y).abs().max().item() < 1e-4
+    for x, y in zip(models[0].cache.k + models[0].cache.v,
+                    models[1].cache.k + models[1].cache.v):
+        assert (x - y).abs().max().item() < 1e-5
+    assert T.equal(models[0].cache.seq_lens, models[1].cache.seq_lens)
+
+
 def test_batched_prefill_matches_sequential():
     """forward_prefill_batch (one concatenated pass, per-sequence
     attention) must produce the same first-token logits as per-sequence

@@ -14,8 +14,9 @@ import torch
 
 sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
 import hybrid_oracle as oracle  # noqa: E402
-from hybrid_helpers import (EXACT, REPO, RUNS, Bytes, close,  # noqa: E402
-                            errors, feed, meta_for, one_thread,  # noqa: F401
+from hybrid_helpers import (EXACT, REPO, RUNS, Bytes,  # noqa: E402
+                            check_wanted_rows_alone, close, errors, feed,
+                            meta_for, one_thread,  # noqa: F401
                             portions, whole)
 
 from gridllm_amd.config import EngineConfig  # noqa: E402
@@ -305,6 +306,11 @@ def test_cuts_do_not_matter(sizes, run):
     want, _ = oracle.forward(FULL, weights_of(FULL), ids)
     slot = m.cache.alloc(0)
     close(feed(m, slot, ids, sizes), want, run, coarse=0.1, odd=0.1)
+
+
+@pytest.mark.parametrize("run", RUNS)
+def test_wanted_rows_alone(run):
+    check_wanted_rows_alone(lambda: build(FULL, run), tokens, run)
 
 
 @pytest.mark.parametrize("run", RUNS)

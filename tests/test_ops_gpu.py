@@ -622,6 +622,37 @@ def test_prefill_batch_engine_parity(dev):
         assert dk < 1.6e-2, (i, dk)
 
 
+@pytest.mark.parametrize("name", ["llama3.2:1b", "qwen2.5:0.5b"])
+def test_last_layer_of_wanted_rows_alone(dev, name):
+    """Logits and caches of prompts whose last layer runs for their last tokens
+    alone, against passes that run it for all (with biases and without)."""
+    from dataclasses import replace
+    from gridllm_amd.models.llama import LlamaModel
+    from gridllm_amd.models.registry import get_spec
+    spec = replace(get_spec(name, 1024), layers=2)
+    torch.manual_seed(3)
+    a, b, c = (torch.randint(0, spec.vocab, (n,), device=dev)
+               for n in (257, 300, 7))
+    got, want = [], []
+    models = [LlamaModel(spec, device=str(dev), dtype="bf16", kv_slots=6,
+                         max_seq=1024, seed=1) for _ in range(2)]
+    for m, out, hidden in zip(models, (got, want), (False, True)):
+        m.interleave_gateup()
+        for r in (m.forward_prefill(a, 2, 0, hidden),
+                  m.forward_prefill(b, 2, 257, hidden),
+                  m.forward_prefill_batch([c, a, b], [1, 4, 3], hidden)):
+            out.append(r[0] if hidden else r)
+    # products of other row counts: two bf16 roundings a sublayer, 2^-9 each
+    for x, y in zip(got, want):
+        assert x.shape == y.shape
+        assert ((x - y).norm() / y.norm()).item() < 0.02
+    for x, y in zip(models[0].cache.k + models[0].cache.v,
+                    models[1].cache.k + models[1].cache.v):
+        for s, n in ((2, 557), (1, 7), (4, 257), (3, 300)):
+            d = (x[s, :, :n].float() - y[s, :, :n].float()).norm()
+            assert d.item() <= 0.01 * y[s, :, :n].float().norm().item()
+
+
 @pytest.mark.parametrize("fuse", [False, True])
 @pytest.mark.parametrize("m,n,k,sk", [
     (17, 384, 64, 1),          # one tile of K

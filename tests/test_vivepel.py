@@ -14,7 +14,8 @@ import torch
 
 sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
 import vivepel_oracle as oracle  # noqa: E402
-from hybrid_helpers import (EXACT, RUNS, Bytes, close, errors,  # noqa: E402
+from hybrid_helpers import (EXACT, RUNS, Bytes,  # noqa: E402
+                            check_wanted_rows_alone, close, errors,
                             feed, meta_for, one_thread, portions,  # noqa: F401
                             whole)
 
@@ -377,6 +378,11 @@ def test_cuts_do_not_matter(sizes, run):
     want, _ = oracle.forward(FULL, weights_of(FULL), ids)
     slot = m.cache.alloc(0)
     close(feed(m, slot, ids, sizes), want, run)
+
+
+@pytest.mark.parametrize("run", RUNS)
+def test_wanted_rows_alone(run):
+    check_wanted_rows_alone(lambda: build(FULL, run), tokens, run)
 
 
 @pytest.mark.parametrize("run", RUNS)
