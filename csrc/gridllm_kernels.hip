@@ -22,6 +22,7 @@
 // Build: hipcc --offload-arch=gfx950 -O3 -shared -fPIC
 
 #include "gridllm_attention.h"
+#include "gridllm_wide.h"
 
 // ===========================================================================
 // RMSNorm (optionally fused residual add):
@@ -673,10 +674,6 @@ k_gemm_rows(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
 //   12288x3072  33.8 -> 20.6  35.7 -> 30.5  37.3 -> 33.1
 //   3072x12288  34.3 -> 21.2  35.4 -> 29.1  37.6 -> 35.3
 // ===========================================================================
-#define WAIT_LOADS(n) do { \
-        __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | 0xf70); \
-        asm volatile("" ::: "memory"); } while (0)
-
 template <int RT, int CT>
 struct GemmTile {
     static constexpr int R = RT * 16, BN = CT * 16;
@@ -871,6 +868,20 @@ static int launch_gemm_tile(hipStream_t st, bf16_t* out, float* ws,
     k_gemm_tile<RT, CT, EPI><<<(unsigned)((total + 7) / 8 * 8), 256, bytes,
                                st>>>(out, ws, x, w, M, N, K, splitk, kslice,
                                      rblocks, glu);
+    LAUNCH_CHECK();
+    return 0;
+}
+
+template <class S, class S2, int EPI>
+static int launch_gemm_wide(hipStream_t st, const WideArgs& p, int full) {
+    constexpr int bytes = S::BYTES > S2::BYTES ? S::BYTES : S2::BYTES;
+    const int e = allow_lds<k_gemm_wide<S, S2, EPI>>(bytes);
+    if (e) return e;
+    const int total = (p.M + S::R - 1) / S::R * ((p.N + S::C - 1) / S::C);
+    full = S2::R ? min(full, total) : total;
+    const int most = max(full, (total - full) * 2);     // blocks' tiles
+    k_gemm_wide<S, S2, EPI><<<8 * min((most + 7) / 8, 32), 512, bytes, st>>>(
+        p, full);
     LAUNCH_CHECK();
     return 0;
 }
@@ -1443,6 +1454,100 @@ int gl_gemm_tile(void* stream, void* out, void* ws, const void* x,
         k_gemm_combine<<<dim3(grid), dim3(256), 0, st>>>(
             (bf16_t*)out, (const float*)ws, (long)M * N, splitk);
     LAUNCH_CHECK();
+    return 0;
+}
+
+// shape: one of kWide; full: of its tiles, the others are halved (shape 0). epi: as
+// in gridllm_wide.h.
+int gl_gemm_wide(void* stream, void* out, const void* x, const void* w, int M,
+                 int N, int K, int shape, int full, int epi, float alpha,
+                 float limit, float shift, float cubic) {
+    const unsigned long ptrs = (unsigned long)out | (unsigned long)x |
+        (unsigned long)w;
+    if (epi < 0 || epi > 2 || full < 0 || ptrs % 16 ||
+        !wide_fits(M, N, K, epi, shape)) return -100;
+    const WideArgs p{out, (const bf16_t*)x, (const bf16_t*)w, M, N, K,
+                     GluParams{alpha, limit, shift, cubic}};
+    hipStream_t st = (hipStream_t)stream;
+    typedef WideShape<6, 4, 2> Wide192;
+    switch (shape * 3 + epi) {
+        case 0: return launch_gemm_wide<Wide256, WideHalf, 0>(st, p, full);
+        case 1: return launch_gemm_wide<Wide256, WideHalf, 1>(st, p, full);
+        case 2: return launch_gemm_wide<Wide256, WideHalf, 2>(st, p, full);
+        case 3: return launch_gemm_wide<WideShape<6, 3, 3>, NoShape, 0>(
+                st, p, full);
+        case 6: return launch_gemm_wide<WideShape<8, 3, 2>, NoShape, 0>(
+                st, p, full);
+        case 9: return launch_gemm_wide<WideShape<6, 2, 4>, NoShape, 0>(
+                st, p, full);
+        case 13: return launch_gemm_wide<Wide192, NoShape, 1>(st, p, full);
+        case 14: return launch_gemm_wide<Wide192, NoShape, 2>(st, p, full);
+    }
+    return -103;
+}
+
+// What to run a product of more than 256 rows by: plan[0] 0 the library, 1
+// gl_gemm_tile by rows plan[1], columns plan[2], parts plan[3], 2 gl_gemm_wide by
+// shape plan[1] and full plan[2]. The times are those of wide_best and of _tile_us
+// in hip_ops.py, which holds up to 1200 rows too (0.2 % off in the mean, 10 %
+// standard deviation, 600 timings).
+//   Gated units are always done here: the library's needs another pass (0.82 of
+//   its time over 100 sizes, 1.09 at most; 2731 x 16384 x 3072 338 -> 220 us).
+//   K from 4096 on with up to 1200 rows: tiles with K in parts (0.82, 0.98 at most;
+//   300 x 2048 x 8192 36.7 -> 25.9).
+//   20 us and less: what a call to the library costs the host, and twice what one
+//   here does (four layers of 0.5b, 260 tokens, are bound by that).
+//   192 x 192 and 192 x 128 tiles, which it seems not to have, where they nearly
+//   fill one or two rounds of CUs (0.93 over 17, 1.0 at most; 2731 x 3072 x 3072 56.7
+//   -> 48.4).
+//   K up to 4096 and 256 x 256 tiles that fill whole rounds and up to 0.6 of one,
+//   the library's worst sizes (0.93 over 40, 1.07 at most; 8000 x 5120 x 3072 284 ->
+//   196). Elsewhere it is 5 to 10 % faster than the kernel here.
+int gl_gemm_plan(int M, int N, int K, int fuse_glu, int* plan) {
+    plan[0] = plan[1] = plan[2] = plan[3] = 0;
+    int shape = 0, full = 0, way = 0;
+    float best = wide_best(M, N, K, fuse_glu ? 1 : 0, &shape, &full);
+    if (best < INFINITY) {
+        way = 2;
+        plan[1] = shape;
+        plan[2] = full;
+    }
+    const int heights[] = {96, 128, 160, 192, 256};
+    const int widths[] = {64, 96, 128};
+    if (M > 0 && M <= 1200 && N > 0 && K > 0 && K % 64 == 0 &&
+        !(fuse_glu && N % 128)) {
+        for (int rows : heights) for (int cols : widths) {
+            if (N % cols || (fuse_glu && cols == 96)) continue;
+            const long tiles = (long)((M + rows - 1) / rows) * (N / cols);
+            if (tiles > 512) continue;
+            const int most = max(1, min((int)(256 / tiles), K / 384));
+            for (int parts : {1, (most + 1) / 2, most}) {
+                const int slice = ((K + parts - 1) / parts + 63) / 64 * 64;
+                const int n = (K + slice - 1) / slice;
+                float us = 6.f + (tiles * n + 255) / 256 * slice *
+                    (float)(rows + cols - 37) * 3.9e-5f;
+                if (n > 1) us += 1.2f + (float)n * M * N * 2.5e-6f;
+                if (us >= best) continue;
+                best = us;
+                way = 1;
+                plan[1] = rows;
+                plan[2] = cols;
+                plan[3] = n;
+            }
+        }
+    }
+    bool here = fuse_glu || best <= 20.f || (way == 1 && K >= 4096);
+    if (way == 2) {
+        const WideTimes& t = kWide[plan[1]];
+        const long tiles = (long)((M + t.rows - 1) / t.rows) *
+                           ((N + t.cols - 1) / t.cols);
+        const long some = tiles % 256;
+        if (plan[1] == 0)
+            here |= K <= 4096 && tiles > 256 && some > 0 && some <= 154;
+        else if (plan[1] != 2)
+            here |= tiles <= 512 && (some == 0 || some >= 218);
+    }
+    plan[0] = here ? way : 0;
     return 0;
 }
 

@@ -1,0 +1,334 @@
+// Many-row GEMM: out[M,N] = x[M,K] @ W[N,K]^T (bf16 I/O, f32 sums), for prompts
+// and the largest decode batches.
+//
+// Block: 8 waves, 2 by 4, one block a CU; a wave has A by B MFMA tiles of 16 x 16.
+// Stages of 64 k of x and W come by loads into LDS, whose 16-byte pieces are
+// XOR-swizzled by their rows through the addresses (no bank conflicts), into rings
+// of NB stages. A wave takes its pieces of a half of a stage at once, ahead of the
+// products of the half before. So a stage's buffer is free after the first quarter
+// of its products, and filled again in the other three: a load has 1.25 to 1.5
+// stages' time (NB = 2) to arrive, and they are issued at the rate at which the CU
+// takes them; two barriers a stage. Measured at 8192^3, 256 x 256: 797 us with one
+// barrier, all of a stage's loads at once behind it and a block for each tile, 744
+// now (1477 TFLOP/s; the library 695 to 720). What bounds it is power: cycles are
+// the same without the loads (81 % of them with an MFMA in each SIMD), and the clock
+// goes from 2.25 to 1.65 GHz with them. With the library's 32 x 32 products: 5 %
+// slower, more ring for x alone: no change.
+//
+// Blocks stay for several tiles: the ring runs on from one to the next, under the
+// stores (16 bytes a lane: W's rows are laid into LDS in an order that gives a lane
+// 8 columns that follow each other). Tiles of an XCD are neighbours, in groups of 4
+// rows of tiles, so that what its 32 CUs read at a time fits in its L2: 8000 x 16384
+// x 3072 617 us in groups of 8, 600 of 4.
+//
+// A number of tiles that leaves the last round of CUs half empty costs a whole one:
+// the first `full` tiles are of shape S, the others of the half as large S2
+// (2731 x 8192 x 2048: 92 us in 2 rounds of 256 x 256, 80 with the rest halved).
+//
+// EPI 1: W rows in groups of 64 gate | 64 up; stores the gated unit [M, N / 2].
+// EPI 2: the result, rounded to bf16, as f32 (a vocabulary's scores).
+// Rows past M and N are read as zeros by the buffer descriptors' bounds, and so are
+// the stages past the last tile: a wave's offset is the end of the matrix at most,
+// and a lane's is added to it.
+// Constraints: N % 8 == 0 (EPI 1: 128), K % 64 == 0, K >= 256, x and W of less than
+// WIDE_BYTES.
+#pragma once
+
+#include "gridllm_tiles.h"
+
+// Waits until no more than n loads or stores of the wave are under way.
+#define WAIT_LOADS(n) do { \
+        __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | 0xf70); \
+        asm volatile("" ::: "memory"); } while (0)
+
+#define WIDE_BYTES 0xe0000000L         // (so that offsets fit into 32 bits)
+
+struct WideArgs {
+    void* out;
+    const bf16_t *x, *w;
+    int M, N, K;
+    GluParams glu;
+};
+
+template <int A_, int B_, int NB_>
+struct WideShape {
+    static constexpr int A = A_, B = B_, NB = NB_, R = A * 32, C = B * 64;
+    static constexpr int BYTES = NB * (R + C) * 128;
+};
+struct NoShape {
+    static constexpr int R = 0, BYTES = 0;
+};
+
+// Tiles item, item + stride, ... < last, whose first rows and columns are place's.
+template <class S, int EPI, class Place>
+DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
+                           int stride, Place place) {
+#ifdef __HIP_DEVICE_COMPILE__          // (the host has no buffer descriptors)
+    constexpr int A = S::A, B = S::B, NB = S::NB, R = S::R, C = S::C;
+    constexpr int BUF = (R + C) * 64, G = (R + C) / 64;  // loads of a wave, stage
+    constexpr int STORES = EPI == 1 ? A * B / 4 : EPI == 2 ? A * B
+                                                : A * ((B + 1) / 2);
+    constexpr int L1 = G / 4, L2 = 2 * L1;      // loads behind quarters 2 and 3
+    static_assert(A % 2 == 0 && (EPI != 1 || B % 4 == 0) &&
+                  (EPI != 2 || B % 2 == 0), "halves");
+    static_assert((NB - 2) * G + L2 + STORES < 64, "that can be counted");
+    if (item >= last) return;
+    const int M = p.M, N = p.N, K = p.K, nt = K >> 6;
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int fr = lane & 15, gq = lane >> 4, wr = wid >> 2, wc = wid & 3;
+    const auto xr = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)p.x, 0, (int)((u32)M * K * 2), 0x00020000);
+    const auto wrs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)p.w, 0, (int)((u32)N * K * 2), 0x00020000);
+
+    // A load takes 8 rows of the stage to LDS in the order of lanes. Row j of W's
+    // tile b is column 8 (j / 4) + j % 4, + 4 for an odd b, of the two tiles' 32 (a
+    // last, single tile: j), or of two tiles of gates, and of ups.
+    const int lr = lane >> 3, at = ((lane & 7) ^ lr) * 16;
+    int vx, vw;                                 // a lane's offsets, with k
+    u32 so[G];                                  // the wave's, of its rows
+    auto tile_of = [&](int i) {                 // W's tile in a wave's load i
+        return ((i * 8 + wid) * 8 - R) % (B * 16) >> 4;
+    };
+    auto aim = [&](int it) {
+        int m0, n0;
+        place(it, &m0, &n0);
+        vx = lr * K * 2 + at;
+        vw = ((lr >> 2) * 8 + (lr & 3)) * K * 2 + at;
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+            const int row = (i * 8 + wid) * 8;
+            int r = min(m0 + row, M);
+            if (i * 64 >= R) {
+                const int v = (row - R) / (B * 16), b = tile_of(i), j = row & 15;
+                const int c = B % 2 && b == B - 1 ? j
+                                                  : (j >> 2) * 8 + (b & 1) * 4;
+                r = n0 + v * B * 16 + (b >> 1) * 32 + c;
+                if (EPI == 1) {
+                    const int o = (n0 >> 1) + v * B * 8 +
+                                  (b % (B / 2) >> 1) * 32 + c;
+                    r = (o >> 6) * 128 + (o & 63) + (b >= B / 2 ? 64 : 0);
+                }
+                r = min(r, N);
+            }
+            so[i] = (u32)r * K * 2;             // (the end, at most)
+        }
+    };
+    auto issue = [&](int buf, int i) {
+        const bool of_x = i * 64 < R;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            of_x ? xr : wrs,
+            (__attribute__((address_space(3))) unsigned int*)(
+                lds + buf * BUF + (i * 8 + wid) * 512),
+            16, of_x || (B % 2 && tile_of(i) == B - 1) ? vx : vw, so[i], 0, 0);
+        if (i + 1 == G) {
+            vx += 128;
+            vw += 128;
+        }
+    };
+
+    f32x4 acc[A][B];
+    bf16x8 xf[2][A], wf[2][B];
+    auto read = [&](int buf, int c, int i) {    // piece i of half c of a stage
+        const bf16_t* t = lds + buf * BUF + ((c * 4 + gq) ^ (fr & 7)) * 8 +
+                          fr * 64;
+        if (i < B)
+            wf[c][i] = *(const bf16x8*)(t + (R + (wc * B + i) * 16) * 64);
+        else
+            xf[c][i - B] = *(const bf16x8*)(t + (wr * A + i - B) * 1024);
+    };
+    // Products of half c and half of its rows of tiles, from a0 on, between them
+    // the pieces of half rc of rbuf (ahead of the last products) and loads l0 ..
+    // l1 - 1 into lbuf.
+    auto quarter = [&](int c, int a0, int rbuf, int rc, bool reads, int lbuf,
+                       int l0, int l1) {
+        constexpr int Q = A / 2, PER = (A + B + Q - 2) / (Q - 1);
+        const int each = (l1 - l0 + Q - 1) / Q;
+#pragma unroll
+        for (int j = 0; j < Q; ++j) {
+#pragma unroll
+            for (int i = j * PER; i < (j + 1) * PER; ++i)
+                if (reads && i < A + B) read(rbuf, rc, i);
+#pragma unroll
+            for (int i = l0 + j * each; i < l0 + (j + 1) * each; ++i)
+                if (i < l1) issue(lbuf, i);
+#pragma unroll
+            for (int b = 0; b < B; ++b)
+                acc[a0 + j][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    wf[c][b], xf[c][a0 + j], acc[a0 + j][b], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    int buf = 0;
+    // fresh: the next stage's loads are older than the stores of the tile before
+    auto stage = [&](bool fresh, auto reads) {
+        const int next = buf + 1 == NB ? 0 : buf + 1;
+        quarter(0, 0, buf, 1, true, 0, 0, 0);
+        lds_barrier();                          // all have this stage
+        quarter(0, A / 2, 0, 0, false, buf, 0, L1);
+        quarter(1, 0, 0, 0, false, buf, L1, L2);
+        if (fresh) WAIT_LOADS((NB - 2) * G + L2 + STORES);
+        else WAIT_LOADS((NB - 2) * G + L2);
+        lds_barrier();                          // the next one is there
+        quarter(1, A / 2, next, 0, decltype(reads)::value, buf, L2, G);
+        buf = next;
+    };
+
+    aim(item);
+#pragma unroll
+    for (int u = 0; u < NB; ++u)
+#pragma unroll
+        for (int i = 0; i < G; ++i) issue(u, i);
+    WAIT_LOADS(G * (NB - 1));
+    lds_barrier();
+    bool stored = false;                        // all of the tile before
+    for (; item < last; item += stride) {
+        int m0, n0;
+        place(item, &m0, &n0);
+#pragma unroll
+        for (int i = 0; i < A + B; ++i) read(buf, 0, i);
+#pragma unroll
+        for (int a = 0; a < A; ++a)
+#pragma unroll
+            for (int b = 0; b < B; ++b) acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int kt = 0; kt < nt - 1; ++kt) {
+            if (kt == nt - NB) {                // loads go on to the next tile
+                if (item + stride < last) aim(item + stride);
+                else
+#pragma unroll
+                    for (int i = 0; i < G; ++i)
+                        so[i] = (u32)(i * 64 < R ? M : N) * K * 2;
+            }
+            stage(kt < NB - 1 && stored, std::true_type());
+        }
+        stage(false, std::false_type());
+        // lane holds row fr and columns gq * 4 + 0 .. 3 of each tile
+#pragma unroll
+        for (int a = 0; a < A; ++a) {
+            const int m = m0 + (wr * A + a) * 16 + fr;
+            if (m >= M) continue;
+            const int ld = EPI == 1 ? N >> 1 : N;
+            const int nw = EPI == 1 ? (n0 >> 1) + wc * B * 8 : n0 + wc * B * 16;
+#pragma unroll
+            for (int b = 0; b + 1 < (EPI == 1 ? B / 2 : B); b += 2) {
+                const int n = nw + b * 16 + gq * 8;
+                if (n >= ld) continue;
+                float f[8];
+#pragma unroll
+                for (int r = 0; r < 8; ++r) {
+                    const float v = acc[a][b + (r >> 2)][r & 3];
+                    f[r] = EPI == 1 ? glu_act(
+                        v, acc[a][b + (r >> 2) + B / 2][r & 3], p.glu) : v;
+                }
+                const bf16x8 v = to_bf16x8(f);
+                if (EPI == 2) {
+                    unpack8(__builtin_bit_cast(uint4, v), f);
+                    st8((float*)p.out + (long)m * ld + n, f);
+                } else {
+                    *(bf16x8*)((bf16_t*)p.out + (long)m * ld + n) = v;
+                }
+            }
+            if constexpr (B % 2 && EPI == 0) {
+                const int n = nw + (B - 1) * 16 + gq * 4;
+                if (n >= ld) continue;
+                bf16x4 v;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = (__bf16)acc[a][B - 1][r];
+                *(bf16x4*)((bf16_t*)p.out + (long)m * ld + n) = v;
+            }
+        }
+        stored = m0 + R <= M && n0 + C <= N;
+    }
+    WAIT_LOADS(0);                              // (of nothing, into LDS)
+    lds_barrier();
+#endif
+}
+
+template <class S, class S2, int EPI>
+__global__ void __launch_bounds__(512, 2)
+k_gemm_wide(const WideArgs p, int full) {
+    extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
+    const int rb = (p.M + S::R - 1) / S::R, cb = (p.N + S::C - 1) / S::C;
+    const int xcd = blockIdx.x & 7, at = (int)(blockIdx.x >> 3);
+    const int stride = (int)(gridDim.x >> 3);
+    auto place = [&](int it, int* m0, int* n0) {
+        const int group = it / (4 * cb), in = it - group * 4 * cb;
+        const int rows = min(4, rb - group * 4);
+        *m0 = (group * 4 + in % rows) * S::R;
+        *n0 = in / rows * S::C;
+    };
+    const int each = (full + 7) >> 3;           // tiles of an XCD
+    wide_tiles<S, EPI>(p, lds, xcd * each + at, min(full, (xcd + 1) * each),
+                       stride, place);
+    if constexpr (S2::R > 0) {
+        static_assert(S2::R * 2 == S::R && S2::C == S::C, "halves");
+        const int rest = (rb * cb - full) * 2, each = (rest + 7) >> 3;
+        wide_tiles<S2, EPI>(
+            p, lds, xcd * each + at, min(rest, (xcd + 1) * each), stride,
+            [&](int it, int* m0, int* n0) {
+                place(full + (it >> 1), m0, n0);
+                *m0 += (it & 1) * S2::R;
+            });
+    }
+}
+
+// Shapes by number, their sizes, and what they take, in us: a stage (`idle` of it
+// with one tile on the chip, as a whole round takes), a tile beside it (`glu` more
+// for the unit), a launch. Fitted to 270 to 590 timings each over the products of
+// the models here and 257 to 8000 rows, 3 to 6 % off in the mean.
+struct WideTimes {
+    int rows, cols;
+    float stage, idle, tile, glu, launch;
+};
+static constexpr WideTimes kWide[] = {
+    {256, 256, 1.367f, .724f, 5.34f, 2.74f, 2.3f},      // rest in halves
+    {192, 192, .846f, .772f, 3.99f, 0.f, 2.5f},
+    {256, 192, 1.108f, .786f, 3.86f, 0.f, 2.8f},
+    {192, 128, .639f, .817f, 1.79f, 0.f, 3.1f},
+    {192, 256, 1.167f, .777f, 1.14f, 3.33f, 3.4f},      // gated units, f32
+};
+static constexpr WideTimes kWideHalf = {128, 256, .841f, .768f, 1.07f, 2.14f,
+                                        1.f};
+static constexpr int kWideShapes = 5;
+typedef WideShape<8, 4, 2> Wide256;
+typedef WideShape<4, 4, 3> WideHalf;
+
+static bool wide_fits(int M, int N, int K, int epi, int shape) {
+    if (shape < 0 || shape >= kWideShapes || M < 1 || N < 1 || K < 256) return false;
+    if (K % 64 || N % (epi == 1 ? 128 : 8)) return false;
+    if ((long)M * K * 2 > WIDE_BYTES || (long)N * K * 2 > WIDE_BYTES ||
+        K > 1 << 20) return false;
+    return epi == 0 ? shape < 4 : shape == 0 || shape == 4;
+}
+
+static float wide_rounds(const WideTimes& t, int K, int epi, int tiles) {
+    const int whole = tiles / 256, some = tiles % 256, nt = K / 64;
+    const float over = t.tile + (epi == 1 ? t.glu : 0.f);
+    return whole * (nt * t.stage + over) +
+           (some ? nt * t.stage * (t.idle + (1 - t.idle) * some / 256.f) + over
+                 : 0.f);
+}
+
+// The fastest shape for a product by these times, and of how many whole tiles.
+static float wide_best(int M, int N, int K, int epi, int* shape, int* full) {
+    float best = INFINITY;
+    for (int s = 0; s < kWideShapes; ++s) {
+        if (!wide_fits(M, N, K, epi, s)) continue;
+        const WideTimes& t = kWide[s];
+        const long tiles = (long)((M + t.rows - 1) / t.rows) *
+                           ((N + t.cols - 1) / t.cols);
+        if (tiles > 1 << 24) continue;
+        const int total = (int)tiles;
+        const float us = t.launch + wide_rounds(t, K, epi, total);
+        if (us < best) { best = us; *shape = s; *full = total; }
+        if (s != 0 || total % 256 == 0) continue;
+        const int head = total / 256 * 256;
+        const float mixed = t.launch + wide_rounds(t, K, epi, head) +
+                            kWideHalf.launch +
+                            wide_rounds(kWideHalf, K, epi, (total - head) * 2);
+        if (mixed < best) { best = mixed; *shape = s; *full = head; }
+    }
+    return best;
+}

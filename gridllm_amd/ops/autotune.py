@@ -26,13 +26,14 @@ from gridllm_amd.utils.logging import get_logger
 log = get_logger("autotune")
 
 # (m, n, k) -> ("blas",) | ("rows",) | ("ours", splitk) |
-# ("tile", rows, cols, splitk)
+# ("tile", rows, cols, splitk) | ("wide", shape, whole tiles)
 _CHOICE: dict[tuple[int, int, int], tuple] = {}
 # gate/up projection with fused SwiGLU (n = 2F interleaved rows):
-# (m, n, k) -> ("blas",) | ("rows",) | ("tile", rows, cols, splitk)
+# (m, n, k) -> ("blas",) | ("rows",) | ("tile", rows, cols, splitk) |
+# ("wide", shape, whole tiles)
 _CHOICE_GU: dict[tuple[int, int, int], tuple] = {}
 _BF16, _transformed = torch.bfloat16, torch._C._are_functorch_transforms_active
-_most_rows = 256                # of a choice by rule or timing
+_most_rows = 1 << 24            # of a choice by rule or timing
 _ITERS = 24                     # calls of a timing, at most
 _SPLITK_CANDIDATES = (0, 2, 4, 6, 8, 12, 16, 24, 32)
 
@@ -89,6 +90,8 @@ def _run(c: tuple, x: torch.Tensor, w: torch.Tensor,
         return hip_ops.gemm_rows(x, w, fuse_swiglu=fuse, glu=unit)
     if c[0] == "tile":
         return hip_ops.gemm_tile(x, w, *c[1:], fuse_swiglu=fuse, glu=unit)
+    if c[0] == "wide":
+        return hip_ops.gemm_wide(x, w, *c[1:], fuse_swiglu=fuse, glu=unit)
     if c[0] == "ours":
         return hip_ops.gemm_skinny(x, w, splitk=c[1])
     out = F.linear(x, w)
@@ -98,6 +101,8 @@ def _run(c: tuple, x: torch.Tensor, w: torch.Tensor,
 def _run_f32(c: tuple, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if c[0] == "tile" and c[3] == 1:
         return hip_ops.gemm_tile_f32(x, w, *c[1:3])
+    if c[0] == "wide":
+        return hip_ops.gemm_wide(x, w, *c[1:], f32=True)
     return _run(c, x, w).float()
 
 
@@ -106,7 +111,7 @@ def _fit(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple[int, int, int]]:
     F.linear would: bf16 matrices that fit each other, dense and aligned, without
     a forward-mode tangent or a torch.func transform, which pass a kernel by."""
     xs = x.shape
-    if len(xs) != 2 or xs[0] > _most_rows:      # (early: prompts' products)
+    if len(xs) != 2 or xs[0] > _most_rows:
         return None
     if x.dtype is not _BF16 or w.dtype is not _BF16 or _transformed() or \
             forward_ad._current_level >= 0 or x.device != w.device:
@@ -128,6 +133,8 @@ def _rule(m: int, n: int, k: int, fuse: bool = False) -> tuple:
     rows 9.8, 8.0; 5120 x 3072, one row 10.8, 10.0; gate/up 16384 x 3072, one row:
     21.7, 19.8), if K is 4096 or less (1024 x 6144, 16 rows 18.6 us, 10.3, the
     library 13.1; 1024 x 8192, 4 rows 15.5, 10.6, 13.6)."""
+    if m > 256:
+        return hip_ops.gemm_plan(m, n, k, fuse) or ("blas",)
     rows = hip_ops.gemm_rows_fits(m, n, k, fuse)
     if rows and k <= 4096 and n * k <= (10_000_000 if m <= 4 else 7_000_000):
         return ("rows",)
@@ -152,6 +159,9 @@ def _tune(x: torch.Tensor, n: int, glu: Optional[Glu] = None,
     t_best = time_of(best)
     tried: list[tuple] = [("tile", *t) for t in hip_ops.gemm_tilings(
         m, n, k, glu is not None)]
+    if m > 256 or (f32 and m > 128):
+        tried += [("wide", *t) for t in hip_ops.gemm_wide_tilings(
+            m, n, k, glu is not None, f32)]
     if hip_ops.gemm_rows_supported(x, ws[0], glu is not None):
         tried.append(("rows",))
     if not tried and glu is None and hip_ops.gemm_skinny_supported(m, n, k):

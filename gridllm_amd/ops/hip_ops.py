@@ -71,6 +71,10 @@ def _load() -> ctypes.CDLL:
     lib.gl_gemm_rows.restype = c_i
     lib.gl_gemm_tile.argtypes = [c_vp] * 5 + [c_i] * 8 + [c_f] * 4
     lib.gl_gemm_tile.restype = c_i
+    lib.gl_gemm_wide.argtypes = [c_vp] * 4 + [c_i] * 6 + [c_f] * 4
+    lib.gl_gemm_wide.restype = c_i
+    lib.gl_gemm_plan.argtypes = [c_i] * 4 + [c_vp]
+    lib.gl_gemm_plan.restype = c_i
     lib.gl_attn_prefill.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_i, c_i,
                                     c_i, c_i, c_i, c_i, c_i, c_i, c_f]
     lib.gl_attn_prefill.restype = c_i
@@ -606,6 +610,60 @@ def gemm_tile_rmsnorm(x: torch.Tensor, w: torch.Tensor, rows: int, cols: int,
         _stream(), _ptr(y), _ptr(ws), ws.shape[0], _ptr(weight),
         _ptr(residual), _ptr(total), m, n, eps), "rmsnorm_parts")
     return y, total
+
+
+WIDE_SHAPES = ((256, 256), (192, 192), (256, 192), (192, 128), (192, 256))
+
+
+def gemm_wide_tilings(m: int, n: int, k: int, fuse_swiglu: bool = False,
+                      f32: bool = False) -> list[tuple[int, int]]:
+    """(shape, whole tiles) worth trying for gemm_wide: those that give 64 CUs a
+    tile, with the last round of CUs whole or in halves."""
+    if k % 64 or k < 256 or n % (128 if fuse_swiglu else 8) or \
+            max(m, n) * k * 2 > 0xe0000000:
+        return []
+    out = []
+    for i, (rows, cols) in enumerate(WIDE_SHAPES):
+        if (0 < i < 4) if fuse_swiglu or f32 else i == 4:
+            continue
+        tiles = -(-m // rows) * -(-n // cols)
+        if 64 <= tiles < 1 << 24:
+            out += [(i, t) for t in sorted({tiles, tiles // 256 * 256}
+                                           if i == 0 else {tiles})]
+    return out
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_plan(m: int, n: int, k: int, fuse_swiglu: bool = False
+              ) -> Optional[tuple]:
+    """("tile", rows, columns, parts) or ("wide", shape, whole tiles) for a
+    product of more than 256 rows that was not timed, None if it is better left
+    to the library (see gl_gemm_plan)."""
+    if not (0 < m < 1 << 24 and 0 < n < 1 << 24 and 0 < k < 1 << 20):
+        return None
+    plan = (ctypes.c_int * 4)()
+    _check(_load().gl_gemm_plan(m, n, k, fuse_swiglu, ctypes.addressof(plan)),
+           "gemm_plan")
+    if plan[0] == 1:
+        return ("tile", *plan[1:4])
+    return ("wide", plan[1], plan[2]) if plan[0] else None
+
+
+def gemm_wide(x: torch.Tensor, w: torch.Tensor, shape: int, full: int,
+              fuse_swiglu: bool = False, glu: Glu = SWIGLU,
+              f32: bool = False) -> torch.Tensor:
+    """out[M,N] = x[M,K] @ w[N,K]^T, bf16, by tiles of WIDE_SHAPES[shape] that
+    blocks of one a CU take in turn; behind the first `full` of them (shape 0)
+    tiles of half the rows. fuse_swiglu: as in gemm_tile. f32: the result, rounded
+    to bf16, as f32."""
+    m, k = x.shape
+    n = w.shape[0]
+    out = torch.empty(m, n // 2 if fuse_swiglu else n, device=x.device,
+                      dtype=torch.float32 if f32 else x.dtype)
+    _check(_load().gl_gemm_wide(
+        _stream(), out.data_ptr(), x.data_ptr(), w.data_ptr(), m, n, k, shape,
+        full, 1 if fuse_swiglu else 2 if f32 else 0, *glu), "gemm_wide")
+    return out
 
 
 def gemm_proj_supported(m: int, n: int, k: int) -> bool:

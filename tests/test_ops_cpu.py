@@ -329,3 +329,38 @@ def test_tilings_by_rule():
             assert hip_ops.gemm_tiling(m, n, k)[2] > 1
     assert _rule(16, 1024, 6144)[0] == _rule(4, 1024, 8192)[0] == "tile"
     assert _rule(4, 1024, 4096)[0] == "rows"
+
+
+def test_plans_of_many_rows():
+    """Each is one that a kernel takes; gated units are not left to the library
+    and another pass; what no kernel has is the library's."""
+    from gridllm_amd.ops import hip_ops
+    from gridllm_amd.ops.autotune import _rule
+    kinds = set()
+    for m in (257, 300, 512, 1000, 1200, 1201, 2731, 5000, 8000, 100000):
+        for n in (8, 64, 100, 896, 1152, 3072, 5120, 16384, 128256):
+            for k in (64, 100, 192, 256, 896, 3072, 4864, 8192):
+                for fuse in (False, True):
+                    plan = hip_ops.gemm_plan(m, n, k, fuse)
+                    kinds.add(plan and plan[0])
+                    if plan is None:
+                        assert not fuse or n % 128 or k % 64 or k < 256
+                        assert _rule(m, n, k, fuse) == ("blas",)
+                    elif plan[0] == "tile":
+                        rows, cols, parts = plan[1:]
+                        assert rows in hip_ops._TILE_ROWS and n % cols == 0
+                        assert cols in ((64, 128) if fuse else (64, 96, 128))
+                        assert 1 <= parts <= k // 64 and k % 64 == 0
+                    else:
+                        shape, whole = plan[1:]
+                        assert k % 64 == 0 and k >= 256
+                        assert n % (128 if fuse else 8) == 0
+                        assert shape in ((0, 4) if fuse else (0, 1, 2, 3))
+                        rows, cols = hip_ops.WIDE_SHAPES[shape]
+                        tiles = -(-m // rows) * -(-n // cols)
+                        assert whole == tiles or (shape == 0 and
+                                                  whole == tiles // 256 * 256)
+    assert kinds == {None, "tile", "wide"}
+    for bad in ((0, 256, 256), (300, 0, 256), (300, 256, 0), (-1, 256, 256),
+                (1 << 40, 256, 256), (300, 256, 1 << 40)):
+        assert hip_ops.gemm_plan(*bad) is None

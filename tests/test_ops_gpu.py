@@ -745,6 +745,88 @@ def test_gemm_tilings():
                 assert not (rule and fuse and (n % 128 or rule[1] == 96))
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (1, 8, 256),               # one row and 8 columns of a tile; 4 stages
+    (255, 256, 256), (257, 264, 320), (384, 1032, 576),
+    (192, 512, 832),           # whole tiles, then one row more
+    (193, 576, 832),
+    (1000, 17 * 256, 256),     # more tiles than an XCD's CUs, 8 divides not
+    (2100, 9 * 1024 + 128, 384),       # several tiles a block
+])
+def test_gemm_wide(dev, m, n, k):
+    """Every shape and way to halve the last tiles against f32: edges of rows and
+    columns, the least K, blocks of one and of several tiles."""
+    from gridllm_amd.ops import hip_ops
+    from gridllm_amd.ops.reference import Glu
+    g = torch.Generator().manual_seed(m + k)
+    x = torch.randn(m, k, generator=g).to(dev, torch.bfloat16)
+    w = torch.randn(n, k, generator=g).to(dev, torch.bfloat16)
+    ref = x.float() @ w.float().t()
+    # bf16 rounding, and f32 sums of k products in another order
+    room = 2 ** -8 * ref.abs() + k * 2e-7 * (k ** 0.5)
+    tiles = -(-m // 256) * -(-n // 256)
+    for shape, whole in [(0, 0), (0, 1), (0, tiles // 2), (0, tiles), (1, 0),
+                         (2, 0), (3, 0)]:
+        out = hip_ops.gemm_wide(x, w, shape, whole)
+        assert bool(((out.float() - ref).abs() <= room).all()), (shape, whole)
+    plain = hip_ops.gemm_wide(x, w, 0, tiles)
+    for shape, whole in ((0, tiles // 2), (4, 0)):
+        out = hip_ops.gemm_wide(x, w, shape, whole, f32=True)
+        assert out.dtype == torch.float32 and torch.equal(out, plain.float())
+    if n % 128:
+        return
+    glu = Glu(1.3, 2.0, 0.5, 0.1)
+    a, b = ref.view(m, -1, 2, 64).unbind(2)
+    a, b = a.clamp(max=2.0), b.clamp(-2.0, 2.0)
+    act = (a * torch.sigmoid(1.3 * a * (1 + 0.1 * a * a))
+           * (b + 0.5)).reshape(m, -1)
+    for shape, whole in ((0, 0), (0, tiles), (0, tiles // 2), (4, 0)):
+        out = hip_ops.gemm_wide(x, w, shape, whole, fuse_swiglu=True, glu=glu)
+        # 2 + 1.5 from an error of either input, and 8 bits of the result
+        assert bool(((out.float() - act).abs() <= 2 ** -8 * act.abs() +
+                     4 * k * 2e-7 * (k ** 0.5)).all()), (shape, whole)
+
+
+def test_gemm_wide_refuses(dev):
+    """Sizes and shapes that the kernel has not, ahead of a launch."""
+    from gridllm_amd.ops import hip_ops
+
+    def t(*s):
+        return torch.zeros(*s, dtype=torch.bfloat16, device=dev)
+    for m, n, k, shape, kw in ((256, 256, 192, 0, {}), (256, 256, 288, 0, {}),
+                               (256, 252, 256, 0, {}), (256, 256, 256, 5, {}),
+                               (256, 256, 256, 4, {}), (256, 256, 256, -1, {}),
+                               (256, 192, 256, 0, dict(fuse_swiglu=True)),
+                               (256, 256, 256, 1, dict(f32=True))):
+        with pytest.raises(RuntimeError):
+            hip_ops.gemm_wide(t(m, k), t(n, k), shape, 1, **kw)
+    with pytest.raises(RuntimeError):
+        hip_ops.gemm_wide(t(256 * 256 + 1)[1:].view(256, 256), t(256, 256), 0, 1)
+
+
+def test_linear_of_many_rows(dev):
+    """What the rule runs products of more than 256 rows by, against F.linear."""
+    import torch.nn.functional as F
+    from gridllm_amd.ops import autotune
+    g = torch.Generator().manual_seed(2)
+    took = set()
+    for m, n, k in ((257, 1152, 896), (300, 2048, 8192), (700, 896, 4864),
+                    (1201, 1152, 896), (1500, 17920, 384), (3000, 512, 3072)):
+        x = torch.randn(m, k, generator=g).to(dev, torch.bfloat16)
+        w = torch.randn(n, k, generator=g).to(dev, torch.bfloat16)
+        for fuse in (False, True):
+            took.add(autotune._rule(m, n, k, fuse)[0])
+            got = autotune.linear_gateup(x, w) if fuse else autotune.linear(x, w)
+            want = F.linear(x, w)
+            if fuse:
+                a, b = want.float().view(m, -1, 2, 64).unbind(2)
+                want = (F.silu(a) * b).reshape(m, -1)
+            # two roundings of the products, up to two bf16 steps each
+            err = (got.float() - want.float()).norm() / want.float().norm()
+            assert err.item() < 2 ** -7, (m, n, k, fuse)
+    assert took == {"blas", "tile", "wide"}
+
+
 @pytest.mark.parametrize("m,n,k,mt,sk", [
     (256, 5120, 3072, 2, 1),   # qkv m-tiled
     (256, 5120, 3072, 2, 3),   # + splitk compose
