@@ -1195,7 +1195,7 @@ extern "C" {
 
 int gl_rmsnorm(void* stream, void* y, const void* x, const void* w,
                const void* res_in, void* res_out, long n, int h, float eps) {
-    if (h % 8 != 0) return -100;
+    if (h % 8 != 0 || (res_in && !res_out)) return -100;
 #define GO(NV) k_rmsnorm<NV> \
         <<<dim3((unsigned)n), dim3(256), 0, (hipStream_t)stream>>>( \
         (bf16_t*)y, (const bf16_t*)x, (const bf16_t*)w, \

@@ -364,3 +364,12 @@ def test_plans_of_many_rows():
     for bad in ((0, 256, 256), (300, 0, 256), (300, 256, 0), (-1, 256, 256),
                 (1 << 40, 256, 256), (300, 256, 1 << 40)):
         assert hip_ops.gemm_plan(*bad) is None
+
+
+def test_rmsnorm_of_a_residual_needs_a_place_for_the_sum():
+    """(refused on the host: the kernel would store to address 0)"""
+    from gridllm_amd.ops import hip_ops
+    x = torch.zeros(2, 64, dtype=torch.bfloat16)
+    lib = hip_ops._load()
+    assert lib.gl_rmsnorm(None, x.data_ptr(), x.data_ptr(), x.data_ptr(),
+                          x.data_ptr(), None, 2, 64, 1e-5) == -100
