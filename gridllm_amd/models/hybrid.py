@@ -1006,14 +1006,14 @@ class HybridModel:
         if start_pos != self.cache.lens[slot]:
             raise ValueError(f"slot {slot} holds {self.cache.lens[slot]} "
                              f"tokens, not {start_pos}")
-        ids = tokens.tolist()
+        ids = tokens.long().cpu().numpy()   # (a list: 130 us more for 3500)
         out = self.forward_step([(slot, ids, [len(ids) - 1])], return_hidden)
         return (out[0][0], out[1][0]) if return_hidden else out[0]
 
     def forward_prefill_batch(self, token_lists: list, slots: list,
                               return_hidden: bool = False):
         """Several fresh sequences in one step; logits of each last token."""
-        lists = [t.tolist() for t in token_lists]
+        lists = [t.long().cpu().numpy() for t in token_lists]
         return self.forward_step(
             [(sl, ids, [len(ids) - 1]) for sl, ids in zip(slots, lists)],
             return_hidden)
