@@ -1021,12 +1021,15 @@ static void launch_gemm_skinny(hipStream_t st, bf16_t* out, float* ws,
 // Ties pick the lowest index (torch.argmax first-max rule).
 //
 // A row is cut into S segments of a block each, so that few rows fill the chip
-// too, and a second kernel picks among the segments. Bound by the hash (seven
-// 32-bit products an element); the two logarithms are taken by the hardware's
-// instruction first, and exactly only for elements that come near the best so
-// far of the wave: the picked element is among them. 64 rows of 128256:
-// 190 us with one block a row and exact logarithms throughout, 21 us now (1.6
-// TB/s), and 4 us for the pick instead of 53 us of small kernels for the keys.
+// too, and a second kernel picks among the segments. Bound by the vector unit: the
+// hash's second product (three of 32 bits: its upper half is what is used; the
+// first one is a sum, see noise_of) and two logarithms an element. These are taken
+// by the hardware's instruction first, and exactly only for elements that come
+// near the best so far of the wave: the picked element is among them. Rows of
+// 128256: 64 take 190 us with one block a row and exact logarithms throughout, 21
+// with seven 32-bit products and a branch an element and maxima through LDS, 16.5
+// now; 512 (with the pick) 115 and 82, 3.2 TB/s. The pick takes 4 us instead of 53
+// us of small kernels for the keys.
 // ===========================================================================
 struct Pick {
     float val;
@@ -1069,70 +1072,96 @@ struct SampleKeys {
     }
 };
 
-DEV_INLINE float sample_uniform(int i, unsigned long long key) {
-    unsigned long long z =
-        ((unsigned long long)i ^ key) * 0x9E3779B97F4A7C15ull;
+// u of candidate i from (i ^ key) * NOISE. With the bits of i in two parts that is
+// a sum of two products, one of which all of a wave's lanes have, and the other
+// one all chunks of 256.
+#define NOISE 0x9E3779B97F4A7C15ull
+DEV_INLINE float noise_of(unsigned long long z) {
     z ^= (unsigned long long)((long long)z >> 29);  // arithmetic >>
-    z *= 0xBF58476D1CE4E5B9ull;
-    z ^= (unsigned long long)((long long)z >> 32);
-    const float u = (float)((z >> 38) & 0xFFFFFFull) * (1.0f / 16777216.0f);
+    // z *= 0xBF58476D1CE4E5B9; z ^= z >> 32: their upper half
+    const u32 lo = (u32)z, top = (u32)(z >> 32);
+    u32 h = __umulhi(lo, 0x1CE4E5B9u) + lo * 0xBF58476Du + top * 0x1CE4E5B9u;
+    h ^= (u32)((int)h >> 31);
+    const float u = (float)(h >> 6 & 0xFFFFFFu) * (1.0f / 16777216.0f);
     return fminf(fmaxf(u, 1e-6f), (float)(1.0 - 1e-6));  // rounded like torch
 }
 
+// Candidates of a lane: 4 that follow each other in each of two chunks of 256.
 __global__ void __launch_bounds__(256)
 k_sample_gumbel(Pick* __restrict__ ws, const float* __restrict__ logits,
                 const SampleKeys how, int v, int segments) {
-    constexpr int E = 4;               // elements of a lane at a time
+    constexpr int E = 8;
     const int row = blockIdx.x / segments, seg = blockIdx.x % segments;
     if (how.slots && (unsigned long long)how.slots[row] >= how.count)
         __builtin_trap();
     const float* x = logits + (long)row * v;
     const unsigned long long key = how.key(row);
     const float t = how.temp(row), rt = 1.f / t;
-    const int per = ((v + segments - 1) / segments + 3) & ~3;
+    const int per = ((v + segments - 1) / segments + 255) & ~255;
     const int i0 = seg * per, i1 = min(v, i0 + per);
     const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool wide = (v & 3) == 0;    // rows start at 16 bytes
+    unsigned long long low[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        low[e] = ((lane * 4 + e) ^ (key & 255)) * NOISE;
     Pick best{-INFINITY, 2147483647};
-    for (int base = i0 + (threadIdx.x >> 6) * 64 * E; base < i1;
-         base += 256 * E) {
-        const int i = base + lane * E;
-        float f[E], u[E], a[E];
-        const int n = min(E, i1 - i);
-        if (wide && n == E) {
-            ld4(x + i, f);
+    auto load = [&](int base, float* f) {
+#pragma unroll
+        for (int c = 0; c < E; c += 4) {
+            const int i = base + c * 64 + lane * 4;
+            if (wide && i + 4 <= i1) {
+                ld4(x + i, f + c);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    f[c + e] = i + e < i1 ? x[i + e] : -INFINITY;
+            }
+        }
+    };
+    float f[E], ahead[E];
+    load(i0 + wid * 512, ahead);
+    for (int base = i0 + wid * 512; base < i1; base += 2048) {
+        float u[E], a[E];
+        auto at = [&](int e) { return base + (e >> 2) * 256 + lane * 4 + (e & 3); };
+#pragma unroll
+        for (int e = 0; e < E; ++e) f[e] = ahead[e];
+        load(base + 2048, ahead);
+        float lim = best.val;
+        if (key != 0ull) {             // (around the elements: they overlap)
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const unsigned long long chunk = base + (e >> 2) * 256;
+                u[e] = noise_of((chunk ^ (key & ~255ull)) * NOISE + low[e & 3]);
+                // log2 by the hardware: good to 1e-3 here, below u = 0.999
+                a[e] = f[e] * rt - 0.6931472f * __builtin_amdgcn_logf(
+                    -0.6931472f * __builtin_amdgcn_logf(u[e]));
+                lim = fmaxf(lim, u[e] <= 0.999f ? a[e] : -INFINITY);
+            }
         } else {
 #pragma unroll
-            for (int e = 0; e < E; ++e) f[e] = e < n ? x[i + e] : -INFINITY;
-        }
-        float lim = best.val;
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            a[e] = f[e] * rt;
-            u[e] = 0.f;
-            if (key != 0ull) {
-                u[e] = sample_uniform(i + e, key);
-                // log2 by the hardware: good to 1e-3 here, below u = 0.999
-                a[e] -= 0.6931472f * __builtin_amdgcn_logf(
-                    -0.6931472f * __builtin_amdgcn_logf(u[e]));
+            for (int e = 0; e < E; ++e) {
+                u[e] = 0.f;
+                a[e] = f[e] * rt;
+                lim = fmaxf(lim, a[e]);
             }
-            if (u[e] <= 0.999f) lim = fmaxf(lim, a[e]);
         }
-        lim = wave_reduce_max(lim);
+        lim = max_across16(max_of16(lim));
         lim -= 0.05f + 1e-5f * fabsf(lim);
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             // (written so that NaN and infinities take the exact way)
-            if (e < n && !(a[e] < lim && u[e] <= 0.999f)) {
+            if (at(e) < i1 && !(a[e] < lim && u[e] <= 0.999f)) {
                 float val = f[e] / t;
                 if (key != 0ull) val += -logf(-logf(u[e]));
-                if (better(val, i + e, best)) best = Pick{val, i + e};
+                if (better(val, at(e), best)) best = Pick{val, at(e)};
             }
         }
     }
     best = wave_pick(best);
     __shared__ Pick part[4];
-    if (lane == 0) part[threadIdx.x >> 6] = best;
+    if (lane == 0) part[wid] = best;
     __syncthreads();
     if (threadIdx.x == 0) {
         for (int w = 1; w < 4; ++w)

@@ -524,6 +524,15 @@ def test_sample_gumbel_segments(dev, b, v):
             assert at >= best - 1e-5 * abs(best) - 1e-4
 
 
+@pytest.mark.parametrize("b,v", [(7, 256), (5, 257), (3, 511), (4, 512), (2, 2049),
+                                 (3, 4096), (2, 6400), (1, 133000), (600, 4352)])
+def test_sample_gumbel_chunks(dev, b, v):
+    """The same at the edges of chunks of 256, of a wave's pair of them, and of
+    segments, the last of which has nothing where they are rounded up to chunks;
+    and behind 2^17 candidates."""
+    test_sample_gumbel_segments(dev, b, v)
+
+
 @pytest.mark.skipif(os.environ.get("GRIDLLM_FUSED_SAMPLER") == "0",
                     reason="fused sampler explicitly disabled")
 def test_sample_gumbel_matches_eager(dev):
