@@ -662,6 +662,14 @@ k_gemm_rows(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
 //   128256 took 30 us to be widened behind it).
 // Constraints: N % (16 CT) == 0 (128 for EPI 1), K % 64 == 0, kslice % 64 == 0.
 //
+// Where W's rows are a multiple of 4096 bytes long, what all blocks read at a time,
+// a piece of 128 bytes at the same place of each row, is in few of the memory's
+// channels (800 MB in rows of 16384 bytes 4.0 TB/s, of 6144 5.7). Blocks of
+// neighbouring columns then start one tile of K further on and wrap (6.05): 45 rows
+// of 128256 x 2048 134.7 -> 121.2 us, of 16384 x 2048 gated 20.1 -> 18.3, 64 of 3072
+// x 12288 in parts 24.2 -> 23.1. Other rows are read as fast in order (24 rows of
+// 5120 x 3072 12.8 us, 13.1; 16384 x 3072 22.8, 23.0).
+//
 // Bound by a CU's loads: those of x, which hit in L2, and of W queue up behind
 // one another (12288 x 3072, 160 rows: x alone 9 us, W alone 13, both 27, with
 // rings of any depth), so the tile is as large as the accumulators allow and all
@@ -711,11 +719,13 @@ k_gemm_tile(bf16_t* __restrict__ out, float* __restrict__ ws,
         const int c = (n0 >> 1) + r % (BN / 2);
         return (c >> 6) * 128 + (c & 63) + (r >= BN / 2 ? 64 : 0);
     };
+    const int turn = K % 2048 ? 0 : item / rblocks % cols % nt;
+    int left = nt - turn;                      // tiles up to the end of K's part
     const bf16_t* src[G];
 #pragma unroll
     for (int i = 0; i < G; ++i) {
         const int row = (i * 4 + wid) * 8 + (lane >> 3);
-        const int at = ((lane & 7) ^ (row & 7)) * 8 + k0;
+        const int at = ((lane & 7) ^ (row & 7)) * 8 + k0 + turn * 64;
         src[i] = (i * 4 + wid) * 8 < R
                      ? x + (long)min(m0 + row, M - 1) * K + at
                      : w + (long)w_row(row - R) * K + at;
@@ -726,6 +736,9 @@ k_gemm_tile(bf16_t* __restrict__ out, float* __restrict__ ws,
             load_lds16(src[i], lds + buf * BUF + (i * 4 + wid) * 512);
             src[i] += 64;
         }
+        if (--left == 0)
+#pragma unroll
+            for (int i = 0; i < G; ++i) src[i] -= nt * 64;
     };
     // a wave's columns; with gates, the second half of its tiles are the ups
     auto col_tile = [&](int b) {

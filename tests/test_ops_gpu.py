@@ -699,6 +699,19 @@ def test_gemm_tile(dev, m, n, k, sk, fuse):
                     (rows, cols)
 
 
+@pytest.mark.parametrize("fuse", [False, True])
+@pytest.mark.parametrize("m,n,k,sk", [
+    (1, 2304, 2048, 1),        # blocks start at every place of K but the last ones
+    (33, 4480, 2048, 1),       # at every one, some twice
+    (40, 1152, 4096, 9),       # parts of K, the last one shorter
+    (257, 384, 2048, 31),      # of fewer tiles than buffers
+])
+def test_gemm_tile_long_rows(dev, m, n, k, sk, fuse):
+    """The same where rows are a multiple of 4096 bytes: blocks start at different
+    places of K, and wrap."""
+    test_gemm_tile(dev, m, n, k, sk, fuse)
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 64, 64), (33, 192, 576),
                                    (257, 8256, 128)])
 def test_gemm_tile_f32(dev, m, n, k):
