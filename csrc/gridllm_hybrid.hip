@@ -2135,24 +2135,76 @@ k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
 // or k_streams_join.
 // ===========================================================================
 //
+// Pairs in the order of their experts, and the list of tiles: by block `part` of
+// those of THREADS that share the pairs, from the counts of E experts that have
+// weights.
+template <int THREADS, int MAX>
+DEV_INLINE void moe_order(int part, int* sorted, int4* tiles, const int* idx,
+                          const int* rank, const int* counts, int pairs, int E,
+                          int bm, int max_tiles) {
+    __shared__ int off[MAX + 1], toff[MAX + 1];
+    for (int e = threadIdx.x; e < E; e += THREADS) off[e + 1] = counts[e];
+    if (threadIdx.x == 0) off[0] = toff[0] = 0;
+    __syncthreads();
+    if (threadIdx.x < 64) {            // one wave scans, 64 experts a turn
+        int base = 0, tbase = 0;
+        for (int e0 = 0; e0 < E; e0 += 64) {
+            const int e = e0 + threadIdx.x;
+            int c = e < E ? off[e + 1] : 0;
+            int t = (c + bm - 1) / bm;
+#pragma unroll
+            for (int s = 1; s < 64; s <<= 1) {
+                const int a = __shfl_up(c, s, WAVE);
+                const int b = __shfl_up(t, s, WAVE);
+                if ((int)threadIdx.x >= s) { c += a; t += b; }
+            }
+            if (e < E) { off[e + 1] = base + c; toff[e + 1] = tbase + t; }
+            base += __shfl(c, 63, WAVE);
+            tbase += __shfl(t, 63, WAVE);
+        }
+    }
+    __syncthreads();
+    const int i = part * THREADS + threadIdx.x;
+    if (i < pairs && idx[i] < E) {
+        const int at = off[idx[i]] + rank[i];
+        if (at >= 0 && at < pairs) sorted[at] = i;
+    }
+    if (part == 0) {
+        for (int e = threadIdx.x; e < E; e += THREADS) {
+            const int n = off[e + 1] - off[e];
+            for (int t = 0; t * bm < n; ++t)
+                if (toff[e] + t < max_tiles)
+                    tiles[toff[e] + t] = make_int4(e, off[e] + t * bm,
+                                                   min(bm, n - t * bm), 0);
+        }
+        if (threadIdx.x == 0)
+            tiles[max_tiles] = make_int4(min(toff[E], max_tiles), 0, 0, 0);
+    }
+}
+
 // A wave routes `tpw` tokens, one expert per lane and VPL experts deep. The
 // place of an expert among a token's logits is the number of larger ones, so
 // the chosen fall out of one pass over the lanes. Counts are gathered per
 // block in LDS and added up once per block and expert.
-template <int VPL>
-__global__ void __launch_bounds__(256)
+// ALONE: one block of 16 waves has all tokens, and orders the pairs too, so that
+// few rows, which launches bound, need no zeros and no second kernel (1 row of 64
+// experts, 8 of them chosen, with the products 34.4 -> 31.5 us).
+template <int VPL, bool ALONE>
+__global__ void __launch_bounds__(ALONE ? 1024 : 256)
 k_moe_route(int* __restrict__ idx, float* __restrict__ wt,
             int* __restrict__ rank, int* __restrict__ counts,
             const float* __restrict__ z, int ldz,
             const float* __restrict__ corr, float* __restrict__ ident, int N,
             int E, int experts, int top, int groups, int keep, float eps,
-            float scale, int sigmoid, int tpw) {
+            float scale, int sigmoid, int tpw, int* __restrict__ sorted,
+            int4* __restrict__ tiles, int bm, int max_tiles) {
+    constexpr int WAVES = ALONE ? 16 : 4, THREADS = WAVES * 64;
     __shared__ int cnt[VPL * 64], base[VPL * 64];
-    __shared__ float cs[4][VPL * 64], gm[4][VPL * 64];
-    for (int e = threadIdx.x; e < VPL * 64; e += 256) cnt[e] = 0;
+    __shared__ float cs[WAVES][VPL * 64], gm[WAVES][VPL * 64];
+    for (int e = threadIdx.x; e < VPL * 64; e += THREADS) cnt[e] = 0;
     __syncthreads();
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int n0 = (blockIdx.x * 4 + wid) * tpw;
+    const int n0 = (blockIdx.x * WAVES + wid) * tpw;
     for (int n = n0; n < min(N, n0 + tpw); ++n) {
         float v[VPL], s[VPL];          // choice score, score
         int place[VPL];
@@ -2248,6 +2300,11 @@ k_moe_route(int* __restrict__ idx, float* __restrict__ wt,
         }
     }
     __syncthreads();
+    if constexpr (ALONE) {
+        moe_order<THREADS, VPL * 64>(0, sorted, tiles, idx, rank, cnt, N * top,
+                                     experts, bm, max_tiles);
+        return;
+    }
     for (int e = threadIdx.x; e < E; e += 256)
         base[e] = cnt[e] ? atomicAdd(counts + e, cnt[e]) : 0;
     __syncthreads();
@@ -2261,45 +2318,9 @@ __global__ void __launch_bounds__(256)
 k_moe_scatter(int* __restrict__ sorted, int4* __restrict__ tiles,
               const int* __restrict__ idx, const int* __restrict__ rank,
               const int* __restrict__ counts, int pairs, int E, int bm,
-              int max_tiles) {          // E: experts that have weights
-    __shared__ int off[1025], toff[1025];
-    for (int e = threadIdx.x; e < E; e += 256) off[e + 1] = counts[e];
-    if (threadIdx.x == 0) off[0] = toff[0] = 0;
-    __syncthreads();
-    if (threadIdx.x < 64) {            // one wave scans, 64 experts a turn
-        int base = 0, tbase = 0;
-        for (int e0 = 0; e0 < E; e0 += 64) {
-            const int e = e0 + threadIdx.x;
-            int c = e < E ? off[e + 1] : 0;
-            int t = (c + bm - 1) / bm;
-#pragma unroll
-            for (int s = 1; s < 64; s <<= 1) {
-                const int a = __shfl_up(c, s, WAVE);
-                const int b = __shfl_up(t, s, WAVE);
-                if ((int)threadIdx.x >= s) { c += a; t += b; }
-            }
-            if (e < E) { off[e + 1] = base + c; toff[e + 1] = tbase + t; }
-            base += __shfl(c, 63, WAVE);
-            tbase += __shfl(t, 63, WAVE);
-        }
-    }
-    __syncthreads();
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < pairs && idx[i] < E) {
-        const int at = off[idx[i]] + rank[i];
-        if (at >= 0 && at < pairs) sorted[at] = i;
-    }
-    if (blockIdx.x == 0) {
-        for (int e = threadIdx.x; e < E; e += 256) {
-            const int n = off[e + 1] - off[e];
-            for (int t = 0; t * bm < n; ++t)
-                if (toff[e] + t < max_tiles)
-                    tiles[toff[e] + t] = make_int4(e, off[e] + t * bm,
-                                                   min(bm, n - t * bm), 0);
-        }
-        if (threadIdx.x == 0)
-            tiles[max_tiles] = make_int4(min(toff[E], max_tiles), 0, 0, 0);
-    }
+              int max_tiles) {
+    moe_order<256, 1024>(blockIdx.x, sorted, tiles, idx, rank, counts, pairs, E,
+                         bm, max_tiles);
 }
 
 DEV_INLINE float sq_relu(float v) {
@@ -2323,10 +2344,12 @@ DEV_INLINE bool moe_work(const int4* tiles, int max_tiles, int ntn, int4& tl,
     return true;
 }
 
-// 128 rows x 128 columns per block, 4 waves of 64 x 64, both
+// R rows x 128 columns per block, 4 waves of R / 2 x 64, both
 // operands through LDS by global_load_lds (source addresses pre-swizzled so
 // that the lane-linear image reads back without bank conflicts), NB buffers.
-// With few rows per expert the same pipeline streams the weights.
+// With few rows per expert the same pipeline streams the weights, in tiles of 32
+// rows with 3 buffers: 48 rows in all, 64 experts, 160 -> 155 us; 12 rows gated 199 ->
+// 168 (a CU's loads queue up, and of 128 rows as many are x's as W's).
 // ACT != 0 (up projection): row r of the tile is token sorted[row0 + r] / top,
 // output in sorted order through squared ReLU (1) or, with weight rows in turns
 // of 16 gate | 16 up, the gated unit `glu` in N / 2 columns (2); pw (nullable):
@@ -2334,13 +2357,14 @@ DEV_INLINE bool moe_work(const int4* tiles, int max_tiles, int ntn, int4& tl,
 // its output goes to pair order. The MFMA computes W x^T, so a lane ends up with
 // 4 neighbouring columns of one row.
 // K % 64 == 0, N % 64 == 0 (ACT 2: N % 128 == 0).
-template <int ACT, int NB>
+template <int ACT, int NB, int R>
 __global__ void __launch_bounds__(256, 2)
 k_moe_gemm(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
            const bf16_t* __restrict__ w, const int4* __restrict__ tiles,
            const int* __restrict__ sorted, int top, int N, int K, int ntn,
            int max_tiles, const GluParams glu, const float* __restrict__ pw) {
-    constexpr int BK = 64, TB = 256 * BK, GL = 8;
+    constexpr int BK = 64, TB = (R + 128) * BK, GL = (R + 128) / 32;
+    constexpr int A = R / 32;
     constexpr bool UP = ACT != 0;
     const int NO = ACT == 2 ? N / 2 : N;
     __shared__ __attribute__((aligned(16))) bf16_t lds[NB * TB];
@@ -2348,16 +2372,16 @@ k_moe_gemm(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
     int nti;
     if (!moe_work(tiles, max_tiles, ntn, tl, nti)) return;
     const int n0 = nti * 128;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int fr = lane & 15, kg = (lane >> 4) * 8;
     const int lrow = lane >> 3, lkb = (lane & 7) * 16;
     const char* src[GL];
 #pragma unroll
-    for (int i = 0; i < GL; ++i) {     // pieces of 8 rows: 16 of x, 16 of w
-        const int piece = (i < 4 ? wid * 4 + i : 16 + wid * 4 + i - 4);
-        const int row = (piece & 15) * 8 + lrow;
+    for (int i = 0; i < GL; ++i) {     // pieces of 8 rows: A of x, 4 of w
+        const int row = (i < A ? wid * A + i : wid * 4 + i - A) * 8 + lrow;
         const bf16_t* p;
-        if (piece < 16) {
+        if (i < A) {
             const int r = tl.y + min(row, tl.z - 1);
             p = x + (long)(UP ? sorted[r] / top : r) * K;
         } else {
@@ -2368,7 +2392,7 @@ k_moe_gemm(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
     auto issue = [&](int buf, int kt) {
 #pragma unroll
         for (int i = 0; i < GL; ++i) {
-            const int piece = (i < 4 ? wid * 4 + i : 16 + wid * 4 + i - 4);
+            const int piece = i < A ? wid * A + i : 4 * A + wid * 4 + i - A;
             __builtin_amdgcn_global_load_lds(
                 (const __attribute__((address_space(1))) unsigned int*)
                     (src[i] + (long)kt * BK * 2),
@@ -2376,13 +2400,13 @@ k_moe_gemm(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
                     (lds + buf * TB + piece * 512), 16, 0, 0);
         }
     };
-    f32x4 acc[4][4];
+    f32x4 acc[A][4];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < A; ++a)
 #pragma unroll
         for (int b = 0; b < 4; ++b) acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
     const int nt = K / BK;
-    const int wr = (wid >> 1) * 64, wc = (wid & 1) * 64;
+    const int wr = (wid >> 1) * (R / 2), wc = (wid & 1) * 64;
 #pragma unroll
     for (int u = 0; u < NB - 1; ++u)
         if (u < nt) issue(u, u);
@@ -2394,7 +2418,7 @@ k_moe_gemm(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
         __builtin_amdgcn_s_barrier();
         if (kt + NB - 1 < nt) issue((kt + NB - 1) % NB, kt + NB - 1);
         const char* xb = (const char*)(lds + (kt % NB) * TB);
-        const char* wb = xb + 128 * BK * 2;
+        const char* wb = xb + R * BK * 2;
 #pragma unroll
         for (int kc = 0; kc < 2; ++kc) {
             bf16x8 b[4];
@@ -2405,7 +2429,7 @@ k_moe_gemm(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
                     (((kc * 32 + kg) * 2) ^ ((row & 7) << 4)));
             }
 #pragma unroll
-            for (int a = 0; a < 4; ++a) {
+            for (int a = 0; a < A; ++a) {
                 const int row = wr + a * 16 + fr;
                 const bf16x8 av = *(const bf16x8*)(xb + row * 128 +
                     (((kc * 32 + kg) * 2) ^ ((row & 7) << 4)));
@@ -2417,7 +2441,7 @@ k_moe_gemm(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
         }
     }
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
+    for (int a = 0; a < A; ++a) {
         const int m = wr + a * 16 + fr;
         if (m >= tl.z) continue;
         bf16_t* orow = out + (UP ? (long)tl.y + m : sorted[tl.y + m]) *
@@ -3064,18 +3088,23 @@ int gh_moe_route(void* stream, void* idx, void* wt, void* rank, void* counts,
         top > E / groups * keep)
         return -100;
     hipStream_t st_ = (hipStream_t)stream;
-#define GO(V) k_moe_route<V><<<(N + 4 * tpw - 1) / (4 * tpw), 256, 0, st_>>>((int*)idx, \
-        (float*)wt, (int*)rank, (int*)counts, (const float*)z, \
+    const long pairs = (long)N * top;
+    const bool alone = !counts;
+    if (alone && (pairs > 1024 || E > 256)) return -100;
+    const int tpw = alone ? (N + 15) / 16 : min(max(N / 2048, 1), 16);
+    const unsigned blocks = alone ? 1 : (N + 4 * tpw - 1) / (4 * tpw);
+#define GO(V, A) k_moe_route<V, A><<<blocks, A ? 1024 : 256, 0, st_>>>( \
+        (int*)idx, (float*)wt, (int*)rank, (int*)counts, (const float*)z, \
         ldz, (const float*)corr, (float*)ident, N, E, experts, top, groups, \
-        keep, eps, scale, sigmoid, tpw)
-    const int tpw = min(max(N / 2048, 1), 16);
-    if (E <= 64) GO(1);
-    else if (E <= 128) GO(2);
-    else if (E <= 256) GO(4);
-    else GO(16);
+        keep, eps, scale, sigmoid, tpw, (int*)sorted, (int4*)tiles, bm, \
+        max_tiles)
+    if (E <= 64) { if (alone) GO(1, true); else GO(1, false); }
+    else if (E <= 128) { if (alone) GO(2, true); else GO(2, false); }
+    else if (E <= 256) { if (alone) GO(4, true); else GO(4, false); }
+    else GO(16, false);
 #undef GO
     LAUNCH_CHECK();
-    const long pairs = (long)N * top;
+    if (alone) return 0;
     k_moe_scatter<<<(unsigned)((pairs + 255) / 256), 256, 0, st_>>>(
         (int*)sorted, (int4*)tiles, (const int*)idx, (const int*)rank,
         (const int*)counts, (int)pairs, experts, bm, max_tiles);
@@ -3085,8 +3114,8 @@ int gh_moe_route(void* stream, void* idx, void* wt, void* rank, void* counts,
 
 // act: 0 down, 1 up with squared ReLU, 2 gate and up (N weight rows, in turns
 // of 16 | 16) with the gated unit's constants; pw (nullable): weights of the
-// pairs on its input. bm: rows per tile of the list: 16 (few pairs; the exact mode) or
-// 128
+// pairs on its input. bm: rows per tile of the list: 16 (few pairs; the exact
+// mode), 32 or 128
 int gh_moe_gemm(void* stream, int f32, int act, void* out, const void* x,
                 const void* w, const void* tiles, const void* sorted,
                 int top, int N, int K, int bm, int max_tiles, float alpha,
@@ -3111,12 +3140,16 @@ int gh_moe_gemm(void* stream, int f32, int act, void* out, const void* x,
 #define ARGS (bf16_t*)out, (const bf16_t*)x, (const bf16_t*)w, \
         (const int4*)tiles, (const int*)sorted, top, N, K, ntn, max_tiles, \
         glu, (const float*)pw
-    if (bm == 128) {
+    if (bm == 32 || bm == 128) {
         const int ntn = (N + 127) / 128;
         const unsigned grid = (unsigned)((max_tiles * ntn + 7) / 8 * 8);
-        if (act == 2) k_moe_gemm<2, 2><<<grid, 256, 0, st_>>>(ARGS);
-        else if (act) k_moe_gemm<1, 2><<<grid, 256, 0, st_>>>(ARGS);
-        else k_moe_gemm<0, 2><<<grid, 256, 0, st_>>>(ARGS);
+#define GO(NB, R) do { \
+            if (act == 2) k_moe_gemm<2, NB, R><<<grid, 256, 0, st_>>>(ARGS); \
+            else if (act) k_moe_gemm<1, NB, R><<<grid, 256, 0, st_>>>(ARGS); \
+            else k_moe_gemm<0, NB, R><<<grid, 256, 0, st_>>>(ARGS); } while (0)
+        if (bm == 32) GO(3, 32);
+        else GO(2, 128);
+#undef GO
     } else if (bm == 16) {
         const int ntn = N / (act == 2 ? 32 : 16);
         const unsigned grid = (unsigned)((max_tiles * ntn + 7) / 8 * 8);

@@ -486,9 +486,23 @@ def lightning(rows: torch.Tensor, S: torch.Tensor, decay: torch.Tensor,
     return out
 
 
-# up to this many (token, expert) pairs, mostly of different experts, the
-# 16-row kernel fills the chip better than 128 x 128 tiles do
-_FEW_PAIRS = 64
+def _expert_rows(pairs: int, experts: int) -> int:
+    """Rows of an expert's tiles. 16, by the kernel that splits K over a block's
+    waves, while the pairs are mostly of different experts; 32 while most experts
+    have no more, whose blocks load less beside the weights; else 128. In us with
+    16, 32 and 128, 64 experts, of which 8 are chosen: 1 row 35, 42, 60; 8 111, 115,
+    119; 16 142, 140, 147; 48 183, 155, 160; 128 275, 158, 167; 192 -, 180, 170;
+    and gated, of which 7 are: 2 65, 60, 78; 6 137, 145, 173; 12 178, 168, 199; 24
+    223, 204, 216; 128 340, 223, 233; 192 -, 228, 237; 256 -, 248, 244. (64 rows are
+    at best 2 % faster than the better of 32 and 128.)"""
+    return 16 if pairs <= 64 else 32 if pairs <= 18 * experts else 128
+
+
+def _routes_alone(n: int, pairs: int, outs: int) -> bool:
+    """Whether one block routes and orders all: a wave takes 3 us for a token, as
+    long as the two launches that it spares (8 rows 111 -> 107 us in all, 16 137.8
+    -> 137.1, 32 150.0 -> 151.4), and more of them each."""
+    return n <= 16 and pairs <= 1024 and outs <= 256
 
 
 def moe(x: torch.Tensor, logits: torch.Tensor, up: torch.Tensor,
@@ -512,11 +526,12 @@ def moe(x: torch.Tensor, logits: torch.Tensor, up: torch.Tensor,
     assert outs >= e and (how.corr is None or how.corr.shape == (outs,))
     dev, f = x.device, _f32(x)
     pairs = n * top
-    bm = 16 if f or pairs <= _FEW_PAIRS else 128
+    bm = 16 if f else _expert_rows(pairs, e)
     max_tiles = min(pairs, e + pairs // bm)
     ints = torch.empty(3 * pairs, dtype=torch.int32, device=dev)
     idx, rank, order = ints[:pairs], ints[pairs:2 * pairs], ints[2 * pairs:]
-    counts = torch.zeros(outs, dtype=torch.int32, device=dev)
+    counts = None if _routes_alone(n, pairs, outs) else \
+        torch.zeros(outs, dtype=torch.int32, device=dev)
     tiles = torch.empty(max_tiles + 1, 4, dtype=torch.int32, device=dev)
     wt = torch.empty(n, top, dtype=torch.float32, device=dev)
     ident = torch.empty(n, dtype=torch.float32, device=dev) \

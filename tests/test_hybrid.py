@@ -161,6 +161,17 @@ def test_experts_at_every_batch_size(batch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("batch", [1, 16, 17, 32, 33, 54, 55, 64])
+def test_experts_at_the_edges_of_tiles(batch):
+    """The same where one block routes and where several do, and with tiles of 16,
+    32 and 128 rows."""
+    from gridllm_amd.ops import hip_hybrid
+    test_experts_at_every_batch_size(batch)
+    assert [hip_hybrid._expert_rows(2 * n, 6) for n in (32, 33, 54, 55)] == \
+        [16, 32, 32, 128]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m", [1, 64, 100, 300])
 def test_fused_gate_projection_takes_the_constants(m):
     """Every gated-unit path with a limit that cuts: the plain op, the

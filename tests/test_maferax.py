@@ -192,6 +192,38 @@ def test_routing(experts, identity, groups, keep, top, dev):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("experts,identity,groups,keep,top", [
+    (14, 2, 4, 2, 3), (60, 8, 2, 1, 8), (70, 0, 1, 1, 64), (200, 40, 12, 3, 8),
+    (1, 1, 1, 1, 2)])
+@pytest.mark.parametrize("n", [1, 15, 16])
+def test_routing_by_one_block(n, experts, identity, groups, keep, top,
+                              monkeypatch):
+    """What the kernels for more rows give, to the bit, in pair order (two tokens
+    alike, and one of NaN)."""
+    from gridllm_amd.ops import hip_hybrid
+    dev, w, f, outs = "cuda:0", 64, 64, experts + identity
+    g = torch.Generator().manual_seed(outs + n)
+    z = torch.randn(n, outs, generator=g)
+    z[n // 2] = z[0]
+    if n > 2:
+        z[2] = float("nan")
+    x = torch.randn(n, w, generator=g).to(dev, torch.bfloat16)
+    up, dn = (torch.randn(*s, generator=g).to(dev, torch.bfloat16) * 0.1
+              for s in ((experts, 2 * f, w), (experts, w, f)))
+    how = hops.Choice(top, torch.randn(outs, generator=g).to(dev), groups, keep,
+                      1e-20, 2.5)
+    assert hip_hybrid._routes_alone(n, n * top, outs)
+    got = hops.moe(x, z.to(dev), up, dn, how)
+    monkeypatch.setattr(hip_hybrid, "_routes_alone", lambda *a: False)
+    want = hops.moe(x, z.to(dev), up, dn, how)
+    real = (want[1] > 0).view(-1)
+    assert torch.equal(got[1].nan_to_num(7), want[1].nan_to_num(7))
+    assert torch.equal(got[0][real], want[0][real])
+    assert identity == 0 or torch.equal(got[2].nan_to_num(7),
+                                        want[2].nan_to_num(7))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("batch", [3, 40, 130, 600])
 def test_gated_experts_at_every_batch_size(batch):
     e, ident, w, f, top = 6, 2, 128, 192, 3
