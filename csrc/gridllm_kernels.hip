@@ -280,7 +280,8 @@ k_swiglu(bf16_t* __restrict__ out, const bf16_t* __restrict__ gateup,
 
 // ===========================================================================
 // Fused RoPE + KV-cache write (the per-layer attention prologue).
-//   qkv: [N, (Hq+2*Hk)*D] bf16 — the raw fused-QKV GEMM output (row-dense);
+//   qkv: [N, (Hq+2*Hk)*D] bf16 — the raw fused-QKV GEMM output (row-dense),
+//   bias: [(Hq+2*Hk)*D] bf16, added to it (rounded, as a sum of its own), or null;
 //   q_out: [N, Hq, D] roped q; k is roped and written straight into kcache,
 //   v copied into vcache (slot[n] = cache_slot*Smax + pos).
 // Replaces {2x contiguous-copy, rope, kv_append} = 4 kernels + one HBM
@@ -292,7 +293,7 @@ k_rope_kv(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ q_out,
           bf16_t* __restrict__ kc, bf16_t* __restrict__ vc,
           const float* __restrict__ cost, const float* __restrict__ sint,
           const int* __restrict__ pos, const int* __restrict__ slot,
-          int Hq, int Hk, int D, int Smax) {
+          const bf16_t* __restrict__ bias, int Hq, int Hk, int D, int Smax) {
     const int nh = Hq + Hk;
     const int n = blockIdx.x / nh;
     const int h = blockIdx.x % nh;
@@ -303,6 +304,9 @@ k_rope_kv(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ q_out,
     const float* srow = sint + (long)p * half;
 
     const bf16_t* src;
+    auto biased = [&](bf16_t v, int at) {
+        return bias ? f2bf(bf2f(v) + bf2f(bias[at])) : v;
+    };
     bf16_t* dst;
     if (h < Hq) {
         src = qkv + (long)n * W + h * D;
@@ -316,12 +320,12 @@ k_rope_kv(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ q_out,
         // copy v row (no rope)
         const bf16_t* vsrc = qkv + (long)n * W + (Hq + Hk + hk) * D;
         bf16_t* vdst = vc + (((b * Hk + hk) * Smax) + pp) * D;
-        for (int i = threadIdx.x; i < (D >> 1); i += 64)
-            ((u32*)vdst)[i] = ((const u32*)vsrc)[i];
+        for (int i = threadIdx.x; i < D; i += 64)
+            vdst[i] = biased(vsrc[i], (Hq + Hk + hk) * D + i);
     }
     for (int i = threadIdx.x; i < half; i += 64) {
-        float a = bf2f(src[i]);
-        float b = bf2f(src[i + half]);
+        float a = bf2f(biased(src[i], h * D + i));
+        float b = bf2f(biased(src[i + half], h * D + i + half));
         float c = crow[i], s = srow[i];
         dst[i] = f2bf(a * c - b * s);
         dst[i + half] = f2bf(a * s + b * c);
@@ -338,7 +342,8 @@ k_rope_kv8(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ q_out,
            bf16_t* __restrict__ kc, bf16_t* __restrict__ vc,
            const float* __restrict__ cost, const float* __restrict__ sint,
            const int* __restrict__ pos, const int* __restrict__ slot,
-           int N, int Hq, int Hk, int D, int Smax) {
+           const bf16_t* __restrict__ bias, int N, int Hq, int Hk, int D,
+           int Smax) {
     const int half = D >> 1, lanes = half >> 3, heads = Hq + 2 * Hk;
     const long i = blockIdx.x * 256L + threadIdx.x;
     const long item = i / lanes;
@@ -347,6 +352,19 @@ k_rope_kv8(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ q_out,
     const int n = (int)(item / heads), h = (int)(item % heads);
     const bf16_t* src = qkv + item * D + c;
     uint4 lo = *(const uint4*)src, hi = *(const uint4*)(src + half);
+    if (bias) {
+        float a[8], b[8];
+        unpack8(lo, a);
+        ld8(bias + h * D + c, b);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) a[k] += b[k];
+        lo = pack8(a);
+        unpack8(hi, a);
+        ld8(bias + h * D + c + half, b);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) a[k] += b[k];
+        hi = pack8(a);
+    }
     if (h < Hq + Hk) {
         const long at = (long)pos[n] * half + c;
         float a[8], b[8], co[8], si[8];
@@ -1374,18 +1392,19 @@ int gl_kv_append(void* stream, void* kc, void* vc, const void* kn,
 
 int gl_rope_kv(void* stream, const void* qkv, void* q_out, void* kc, void* vc,
                const void* cost, const void* sint, const void* pos,
-               const void* slot, int N, int Hq, int Hk, int D, int Smax) {
+               const void* slot, const void* bias, int N, int Hq, int Hk, int D,
+               int Smax) {
     if (D % 4 != 0 || N == 0) return (D % 4) ? -100 : 0;
     const unsigned long ptrs = (unsigned long)qkv | (unsigned long)q_out |
         (unsigned long)kc | (unsigned long)vc | (unsigned long)cost |
-        (unsigned long)sint;
+        (unsigned long)sint | (unsigned long)bias;
     if (D % 16 == 0 && ptrs % 16 == 0) {
         const long items = (long)N * (Hq + 2 * Hk) * (D / 16);
         k_rope_kv8<<<dim3((unsigned)((items + 255) / 256)), dim3(256), 0,
                      (hipStream_t)stream>>>(
             (const bf16_t*)qkv, (bf16_t*)q_out, (bf16_t*)kc, (bf16_t*)vc,
             (const float*)cost, (const float*)sint, (const int*)pos,
-            (const int*)slot, N, Hq, Hk, D, Smax);
+            (const int*)slot, (const bf16_t*)bias, N, Hq, Hk, D, Smax);
         LAUNCH_CHECK();
         return 0;
     }
@@ -1393,7 +1412,7 @@ int gl_rope_kv(void* stream, const void* qkv, void* q_out, void* kc, void* vc,
                 (hipStream_t)stream>>>(
         (const bf16_t*)qkv, (bf16_t*)q_out, (bf16_t*)kc, (bf16_t*)vc,
         (const float*)cost, (const float*)sint, (const int*)pos,
-        (const int*)slot, Hq, Hk, D, Smax);
+        (const int*)slot, (const bf16_t*)bias, Hq, Hk, D, Smax);
     LAUNCH_CHECK();
     return 0;
 }
@@ -1677,6 +1696,79 @@ int gl_attn_prefill_batch(void* stream, void* out, const void* q,
         return -111;
     LAUNCH_CHECK();
     return 0;
+}
+
+// A prompt's layer (Llama family): its launches one behind the other, 4 us of the
+// host each, where calls from Python take 7 to 13 with their tensors and checks
+// (four layers of llama3.2:1b, 45 tokens, were bound by that).
+struct LayerProduct {
+    long long kind, a, b, c;       // 0 k_gemm_rows; 1 k_gemm_tile: rows, columns, parts;
+};                                 // 2 k_gemm_wide: shape, whole tiles
+struct PromptLayer {
+    // normed rows and residuals [T, H] in and out, and behind the attention
+    void *normed, *resid, *mid_normed, *mid_resid;
+    void *qkv, *q, *attn, *act, *y, *ws;       // working space; ws: f32 parts
+    const void *wqkv, *bqkv, *wo, *wgateup, *wdown, *mlp_norm, *next_norm;
+    void *kc, *vc;
+    const void *cost, *sint, *pos, *places, *meta;     // meta: of several prompts
+    long long T, H, Hq, Hk, D, F, Smax, slot, start, tiles;
+    LayerProduct p_qkv, p_o, p_gateup, p_down;
+};
+
+static int layer_product(void* st, const LayerProduct& p, void* out, void* ws,
+                         const void* x, const void* w, int M, int N, int K,
+                         int glu) {
+    const GluParams u{1.f, INFINITY, 0.f, 0.f};
+    if (p.kind == 0)
+        return gl_gemm_rows(st, out, x, w, M, N, K, glu, u.alpha, u.limit,
+                            u.shift, u.cubic);
+    if (p.kind == 1) {
+        if (p.c < 1) return -100;
+        const int slice = ((K + (int)p.c - 1) / (int)p.c + 63) / 64 * 64;
+        return gl_gemm_tile(st, out, ws, x, w, M, N, K, (K + slice - 1) / slice,
+                            slice, (int)p.a, (int)p.b, glu, u.alpha, u.limit,
+                            u.shift, u.cubic);
+    }
+    return gl_gemm_wide(st, out, x, w, M, N, K, (int)p.a, (int)p.b, glu, u.alpha,
+                        u.limit, u.shift, u.cubic);
+}
+
+// (rmsnorm(y) * weight, y) of y = x w^T + resid
+static int layer_joined(void* st, const LayerProduct& p, const PromptLayer& l,
+                        const void* x, const void* w, int K, const void* weight,
+                        const void* resid, void* normed, void* sum, float eps) {
+    const int T = (int)l.T, H = (int)l.H;
+    const bool parts = p.kind == 1 && p.c > 1 && K > 64 && H % 8 == 0;
+    const int e = layer_product(st, p, parts ? nullptr : l.y, l.ws, x, w, T, H, K,
+                                0);
+    if (e) return e;
+    if (!parts)
+        return gl_rmsnorm(st, normed, l.y, weight, resid, sum, T, H, eps);
+    const int slice = ((K + (int)p.c - 1) / (int)p.c + 63) / 64 * 64;
+    return gl_rmsnorm_parts(st, normed, l.ws, (K + slice - 1) / slice, weight,
+                            resid, sum, T, H, eps);
+}
+
+int gl_prompt_layer(void* st, const void* layer, float scale, float eps) {
+    const PromptLayer& l = *(const PromptLayer*)layer;
+    const int T = (int)l.T, H = (int)l.H, Hq = (int)l.Hq, Hk = (int)l.Hk;
+    const int D = (int)l.D, Smax = (int)l.Smax;
+    int e = layer_product(st, l.p_qkv, l.qkv, l.ws, l.normed, l.wqkv, T,
+                          (Hq + 2 * Hk) * D, H, 0);
+    if (!e) e = gl_rope_kv(st, l.qkv, l.q, l.kc, l.vc, l.cost, l.sint, l.pos,
+                           l.places, l.bqkv, T, Hq, Hk, D, Smax);
+    if (!e) e = l.meta
+        ? gl_attn_prefill_batch(st, l.attn, l.q, l.kc, l.vc, l.meta,
+                                (int)l.tiles, Hq, Hk, D, Smax, scale)
+        : gl_attn_prefill(st, l.attn, l.q, l.kc, l.vc, T, Hq, Hk, D, Smax,
+                          (int)l.slot, (int)l.start + T, (int)l.start, scale);
+    if (!e) e = layer_joined(st, l.p_o, l, l.attn, l.wo, Hq * D, l.mlp_norm,
+                             l.resid, l.mid_normed, l.mid_resid, eps);
+    if (!e) e = layer_product(st, l.p_gateup, l.act, l.ws, l.mid_normed,
+                              l.wgateup, T, 2 * (int)l.F, H, 1);
+    if (!e) e = layer_joined(st, l.p_down, l, l.act, l.wdown, (int)l.F,
+                             l.next_norm, l.mid_resid, l.normed, l.resid, eps);
+    return e;
 }
 
 int gl_device_sync() { return (int)hipDeviceSynchronize(); }

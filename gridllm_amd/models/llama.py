@@ -28,6 +28,7 @@ import numpy as np
 import torch
 import torch.nn.functional as F  # noqa: F401
 
+from gridllm_amd.ops.autotune import choice_of as _choice_of
 from gridllm_amd.ops.autotune import linear as _linear
 from gridllm_amd.ops.autotune import linear_f32 as _linear_f32
 from gridllm_amd.ops.autotune import linear_gateup as _linear_gateup
@@ -375,12 +376,12 @@ class LlamaModel:
         lw, kc, vc = self.layers[-1], self.cache.k[-1], self.cache.v[-1]
         d, at = self.spec.head_dim, self.hq_l * self.spec.head_dim
         kv, q = _linear(normed, lw.wqkv[at:]), _linear(x, lw.wqkv[:at])
-        if lw.bqkv is not None:
-            kv, q = kv + lw.bqkv[at:], q + lw.bqkv[:at]
+        q_bias, kv_bias = (None, None) if lw.bqkv is None else (
+            lw.bqkv[:at], lw.bqkv[at:])
         ops.rope_kv(kv, kc, vc, self.cos, self.sin, pos, slot_t, 0,
-                    self.hkv_l, d)
+                    self.hkv_l, d, kv_bias)
         q = ops.rope_kv(q, kc, vc, self.cos, self.sin, x_pos, slot_t,
-                        self.hq_l, 0, d)
+                        self.hq_l, 0, d, q_bias)
         if not torch.is_tensor(slots):
             kc, vc, slots = kc[slots:slots + 1], vc[slots:slots + 1], None
         attn = ops.attn_decode(q, kc, vc, keys, self.scale, slot_map=slots)
@@ -388,6 +389,70 @@ class LlamaModel:
                                 resid)
         return self._joined(self._mlp_act(x, lw), lw.wdown, self.final_norm,
                             resid)[0]
+
+    def _layers_by_call(self, normed: torch.Tensor, resid: torch.Tensor,
+                        layers: int, pos: torch.Tensor, places: torch.Tensor,
+                        slot: int, start: int, meta: Optional[torch.Tensor]
+                        ) -> int:
+        """The first `layers` layers of a prompt (meta: of several) by one native
+        call each, on its normed rows and residuals, in place. How many have been
+        run: none where a layer takes another way than the kernels'. Small models'
+        short prompts were bound by what launches cost the host (four layers of 1b,
+        45 tokens: 383 us of the host, 190 now, 344 -> 323 us in all; of
+        qwen2.5:0.5b, 60: 371 -> 253)."""
+        s, d, t = self.spec, self.spec.head_dim, normed.shape[0]
+        if (self.device.type == "cpu" or self.dtype != torch.bfloat16
+                or self.tp.size > 1 or not self.gateup_il or d not in (64, 128)
+                or self.hq_l % self.hkv_l or t < 1):
+            return 0
+        from gridllm_amd.ops import hip_ops
+        if hip_ops._VALIDATE:
+            return 0
+        n, f, h = (self.hq_l + 2 * self.hkv_l) * d, self.f_l, s.hidden
+        at, bf16 = self.hq_l * d, torch.bfloat16
+        first = self.layers[0]
+        how = [_choice_of(t, w, w is first.wgateup) for w in (
+            first.wqkv, first.wo, first.wgateup, first.wdown)]
+        if None in how:
+            return 0
+        sizes = ((n, h), (h, at), (2 * f, h), (h, f))
+        norms = [lw.attn_norm for lw in self.layers] + [self.final_norm]
+        for lw in self.layers[:layers]:
+            for w, size in zip((lw.wqkv, lw.wo, lw.wgateup, lw.wdown), sizes):
+                if w.shape != size or w.dtype is not bf16 or \
+                        w.data_ptr() & 15 or not w.is_contiguous():
+                    return 0
+            if not lw.mlp_norm.is_contiguous():
+                return 0
+        # a layer's rows, one behind the other, from 16 bytes on each
+        dev, parts = self.device, 0
+        rows = torch.empty(n + 2 * at + f + 3 * h, t, dtype=bf16, device=dev)
+        for c, (cols, _) in zip(how, sizes):
+            if c[0] == "tile" and c[3] > 1:
+                parts = max(parts, c[3] * t * cols)
+        ws = torch.empty(parts, dtype=torch.float32, device=dev) if parts else None
+        spots, base = [], rows.data_ptr()
+        for cols in (n, at, at, f, h, h, h):
+            spots.append(base)
+            base += cols * t * 2
+        qkv, q, attn, act, y, mid, mid_resid = spots
+        tail = [self.cos.data_ptr(), self.sin.data_ptr(), pos.data_ptr(),
+                places.data_ptr(), 0 if meta is None else meta.data_ptr(), t, h,
+                self.hq_l, self.hkv_l, d, f, self.cache.max_seq, slot, start,
+                0 if meta is None else meta.shape[0]]
+        for c in how:
+            tail += hip_ops.layer_choice(c)
+        head = [normed.data_ptr(), resid.data_ptr(), mid, mid_resid, qkv, q, attn,
+                act, y, 0 if ws is None else ws.data_ptr()]
+        for li, lw in enumerate(self.layers[:layers]):
+            hip_ops.prompt_layer(head + [
+                lw.wqkv.data_ptr(),
+                0 if lw.bqkv is None else lw.bqkv.data_ptr(), lw.wo.data_ptr(),
+                lw.wgateup.data_ptr(), lw.wdown.data_ptr(),
+                lw.mlp_norm.data_ptr(), norms[li + 1].data_ptr(),
+                self.cache.k[li].data_ptr(), self.cache.v[li].data_ptr()] + tail,
+                self.scale, s.norm_eps)
+        return layers
 
     @torch.no_grad()
     def forward_prefill(self, tokens: torch.Tensor, slot: int,
@@ -404,18 +469,19 @@ class LlamaModel:
         pos, slot_t = counts[:t], slot_t[:t]    # (the next: the number of keys)
         resid, normed = ops.embed_norm(tokens, self.embed,
                                        self.layers[0].attn_norm, s.norm_eps)
+        run = self._layers_by_call(normed, resid, len(self.layers) - trim, pos,
+                                   slot_t, slot, start_pos, None)
         for li, lw in enumerate(self.layers):
+            if li < run:
+                continue
             if trim and li + 1 == len(self.layers):
                 normed = self._last_layer(
                     normed, pos, slot_t, normed[-1:], resid[-1:], pos[-1:],
                     counts[t:], slot)
                 break
-            qkv = _linear(normed, lw.wqkv)
-            if lw.bqkv is not None:
-                qkv = qkv + lw.bqkv
-            q = ops.rope_kv(qkv, self.cache.k[li], self.cache.v[li],
-                            self.cos, self.sin, pos, slot_t,
-                            self.hq_l, self.hkv_l, self.spec.head_dim)
+            q = ops.rope_kv(_linear(normed, lw.wqkv), self.cache.k[li],
+                            self.cache.v[li], self.cos, self.sin, pos, slot_t,
+                            self.hq_l, self.hkv_l, self.spec.head_dim, lw.bqkv)
             attn = ops.attn_prefill_cache(
                 q, self.cache.k[li], self.cache.v[li], slot, start_pos + t,
                 start_pos, self.scale)                           # [T,Hq_l,D]
@@ -476,18 +542,19 @@ class LlamaModel:
             meta = self.up.upload(np.asarray(rows, dtype=np.int32))
         resid, normed = ops.embed_norm(tokens, self.embed,
                                        self.layers[0].attn_norm, s.norm_eps)
+        run = 0 if meta is None else self._layers_by_call(
+            normed, resid, len(self.layers) - trim, pos, slot_t, 0, 0, meta)
         for li, lw in enumerate(self.layers):
+            if li < run:
+                continue
             if trim and li + 1 == len(self.layers):
                 normed = self._last_layer(
                     normed, pos, slot_t, normed[ends[3]], resid[ends[3]],
                     ends[0], ends[1], ends[2])
                 break
-            qkv = _linear(normed, lw.wqkv)
-            if lw.bqkv is not None:
-                qkv = qkv + lw.bqkv
-            q = ops.rope_kv(qkv, self.cache.k[li], self.cache.v[li],
-                            self.cos, self.sin, pos, slot_t,
-                            self.hq_l, self.hkv_l, self.spec.head_dim)
+            q = ops.rope_kv(_linear(normed, lw.wqkv), self.cache.k[li],
+                            self.cache.v[li], self.cos, self.sin, pos, slot_t,
+                            self.hq_l, self.hkv_l, self.spec.head_dim, lw.bqkv)
             if meta is not None:
                 attn = ops.attn_prefill_cache_batch(
                     q, self.cache.k[li], self.cache.v[li], meta, self.scale)
@@ -535,12 +602,10 @@ class LlamaModel:
         resid, normed = ops.embed_norm(tokens, self.embed,
                                        self.layers[0].attn_norm, s.norm_eps)
         for li, lw in enumerate(self.layers):
-            qkv = _linear(normed, lw.wqkv)
-            if lw.bqkv is not None:
-                qkv = qkv + lw.bqkv
-            q = ops.rope_kv(qkv, self.cache.k[li], self.cache.v[li],
-                            self.cos, self.sin, pos_rope, slot_t,
-                            self.hq_l, self.hkv_l, self.spec.head_dim)
+            q = ops.rope_kv(_linear(normed, lw.wqkv), self.cache.k[li],
+                            self.cache.v[li], self.cos, self.sin, pos_rope,
+                            slot_t, self.hq_l, self.hkv_l, self.spec.head_dim,
+                            lw.bqkv)
             attn = ops.attn_decode(q, self.cache.k[li], self.cache.v[li],
                                    attn_seq, self.scale, slot_map=slot_map)
             normed, resid = self._joined(attn.reshape(b, -1), lw.wo,

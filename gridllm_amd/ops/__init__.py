@@ -104,13 +104,14 @@ def rope(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor,
 
 def rope_kv(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
             cos: torch.Tensor, sin: torch.Tensor, pos: torch.Tensor,
-            slot: torch.Tensor, hq: int, hk: int, d: int) -> torch.Tensor:
+            slot: torch.Tensor, hq: int, hk: int, d: int,
+            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     if _on_gpu(qkv):
         from gridllm_amd.ops import hip_ops
         return hip_ops.rope_kv(qkv, kcache, vcache, cos, sin, pos, slot,
-                               hq, hk, d)
+                               hq, hk, d, bias)
     return reference.rope_kv(qkv, kcache, vcache, cos, sin, pos, slot,
-                             hq, hk, d)
+                             hq, hk, d, bias)
 
 
 def swiglu(gateup: torch.Tensor, glu: Glu = SWIGLU) -> torch.Tensor:

@@ -220,6 +220,18 @@ def _choose(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple]:
     return None if fit is None else _CHOICE.get(fit) or _rule(*fit)
 
 
+def choice_of(m: int, w: torch.Tensor, fuse: bool = False) -> Optional[tuple]:
+    """What linear (fuse: linear_gateup) runs dense aligned bf16 rows [m, K] and w
+    by, if that is one of the kernels here."""
+    if m > _most_rows or w.dtype is not _BF16 or _transformed() or \
+            forward_ad._current_level >= 0 or w.dim() != 2 or \
+            not w.is_contiguous() or w.data_ptr() & 15 or not w.numel():
+        return None
+    key = (m, *w.shape)
+    c = (_CHOICE_GU if fuse else _CHOICE).get(key) or _rule(*key, fuse)
+    return c if c[0] in ("rows", "tile", "wide") else None
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """Dispatch x @ w.T (GPU bf16 2-D x only) through the tuned table or by
     rule."""

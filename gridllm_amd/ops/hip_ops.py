@@ -8,6 +8,7 @@ silent eager fallback on the GPU path.
 
 from __future__ import annotations
 
+import array
 import ctypes
 import functools
 import os
@@ -57,8 +58,10 @@ def _load() -> ctypes.CDLL:
     lib.gl_swiglu.argtypes = [c_vp, c_vp, c_vp, c_l, c_i, c_f, c_f, c_f, c_f]
     lib.gl_swiglu.restype = c_i
     lib.gl_rope_kv.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp,
-                               c_vp, c_i, c_i, c_i, c_i, c_i]
+                               c_vp, c_vp, c_i, c_i, c_i, c_i, c_i]
     lib.gl_rope_kv.restype = c_i
+    lib.gl_prompt_layer.argtypes = [c_vp, c_vp, c_f, c_f]
+    lib.gl_prompt_layer.restype = c_i
     lib.gl_kv_append.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i, c_i, c_i, c_i]
     lib.gl_kv_append.restype = c_i
     lib.gl_attn_decode.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp,
@@ -252,9 +255,11 @@ def rope(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor,
 
 def rope_kv(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
             cos: torch.Tensor, sin: torch.Tensor, pos: torch.Tensor,
-            slot: torch.Tensor, hq: int, hk: int, d: int) -> torch.Tensor:
+            slot: torch.Tensor, hq: int, hk: int, d: int,
+            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Fused RoPE + KV write from the raw QKV GEMM output.
-    qkv: [N, (hq+2*hk)*d] bf16 (row-dense); returns roped q [N, hq, d]."""
+    qkv: [N, (hq+2*hk)*d] bf16 (row-dense), bias: [(hq+2*hk)*d] bf16, added to
+    it; returns roped q [N, hq, d]."""
     lib = _load()
     n = qkv.shape[0]
     smax = kcache.shape[2]
@@ -263,7 +268,8 @@ def rope_kv(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
     q_out = torch.empty(n, hq, d, dtype=qkv.dtype, device=qkv.device)
     _check(lib.gl_rope_kv(_stream(), _ptr(qkv), _ptr(q_out), _ptr(kcache),
                           _ptr(vcache), _ptr(cos), _ptr(sin), _ptr(pos),
-                          _ptr(slot), n, hq, hk, d, smax), "rope_kv")
+                          _ptr(slot), _ptr(bias), n, hq, hk, d, smax),
+           "rope_kv")
     return q_out
 
 
@@ -782,6 +788,23 @@ def _sample(logits, keys, temps, slots=None, seeds=None, draws=None,
         _stream(), out.data_ptr(), ws.data_ptr(), logits.data_ptr(), *at, b, v,
         segments, n[0]), "sample_gumbel")
     return out
+
+
+_LAYER_KINDS = {"rows": 0, "tile": 1, "wide": 2}
+
+
+def layer_choice(c: tuple) -> tuple[int, int, int, int]:
+    """A product's choice for prompt_layer."""
+    return (_LAYER_KINDS[c[0]], *c[1:], *(0,) * (4 - len(c)))
+
+
+def prompt_layer(fields: list, scale: float, eps: float) -> None:
+    """A prompt's layer by one call (the fields of PromptLayer, addresses and
+    numbers, in their order)."""
+    data = array.array("q", fields)
+    assert len(fields) == 50
+    _check(_load().gl_prompt_layer(_stream(), data.buffer_info()[0], scale, eps),
+           "prompt_layer")
 
 
 def device_sync() -> None:

@@ -108,10 +108,13 @@ def swiglu(gateup: torch.Tensor, glu: Glu = SWIGLU) -> torch.Tensor:
 
 def rope_kv(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
             cos: torch.Tensor, sin: torch.Tensor, pos: torch.Tensor,
-            slot: torch.Tensor, hq: int, hk: int, d: int) -> torch.Tensor:
+            slot: torch.Tensor, hq: int, hk: int, d: int,
+            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Reference of the fused RoPE+KV-write: slice the QKV GEMM output,
     rope q/k, append k/v to the caches. Returns roped q [N, hq, d]."""
     n = qkv.shape[0]
+    if bias is not None:
+        qkv = qkv + bias
     q = qkv[:, :hq * d].reshape(n, hq, d)
     k = qkv[:, hq * d:(hq + hk) * d].reshape(n, hk, d)
     v = qkv[:, (hq + hk) * d:].reshape(n, hk, d).contiguous()

@@ -597,6 +597,64 @@ def test_attn_prefill_batch_varlen(dev):
         assert err < 1e-3, (i, err)
 
 
+@pytest.mark.parametrize("name", ["qwen2.5:0.5b", "llama3.2:3b"])
+def test_prompt_layers_by_call(dev, name, monkeypatch):
+    """A prompt's layers by native calls give what their launches from Python
+    give, to the bit: rows for each kind of product, with and without a bias, new
+    and continued sequences, one and several. A layer that a kernel does not read
+    is left to Python."""
+    from dataclasses import replace
+    from gridllm_amd.models import llama
+    from gridllm_amd.models.registry import get_spec
+    spec = replace(get_spec(name), layers=3, vocab=1024)
+    m = llama.LlamaModel(spec, device=str(dev), dtype="bf16", seed=3, kv_slots=4,
+                         max_seq=1024)
+    m.interleave_gateup()
+    calls, kinds = [], set()
+    native = llama.LlamaModel._layers_by_call
+    choice = llama._choice_of
+
+    def counted(self, *args):
+        calls.append(native(self, *args))
+        return calls[-1]
+
+    def seen(*args):
+        c = choice(*args)
+        kinds.add(c and c[0])
+        return c
+    monkeypatch.setattr(llama, "_choice_of", seen)
+
+    def run():
+        g = torch.Generator().manual_seed(1)
+        out = []
+        for t in (1, 4, 16, 17, 64, 65, 257, 300):
+            ids = torch.randint(0, 1024, (t,), generator=g).to(dev)
+            more = torch.randint(0, 1024, (33,), generator=g).to(dev)
+            slot = m.cache.alloc(t + 33)
+            out.append(m.forward_prefill(ids, slot))
+            out.append(m.forward_prefill(more, slot, start_pos=t))
+            m.cache.free(slot)
+        slots = [m.cache.alloc(40) for _ in range(3)]
+        out.append(m.forward_prefill_batch(
+            [torch.arange(n, device=dev) for n in (40, 1, 17)], slots))
+        for sl in reversed(slots):
+            m.cache.free(sl)
+        return out + [t.clone() for t in m.cache.k + m.cache.v]
+    monkeypatch.setattr(llama.LlamaModel, "_layers_by_call", counted)
+    got = run()
+    assert len(calls) == 17 and all(calls[:12]) and set(calls) <= {0, 2, 3}
+    assert {"tile", "rows"} <= kinds
+    monkeypatch.setattr(llama.LlamaModel, "_layers_by_call", lambda *a: 0)
+    for a, b in zip(got, run()):
+        assert torch.equal(a, b)
+    monkeypatch.setattr(llama.LlamaModel, "_layers_by_call", counted)
+    lw = m.layers[1]
+    lw.wo = lw.wo.t().contiguous().t()
+    calls.clear()
+    m.forward_prefill(torch.arange(20, device=dev), m.cache.alloc(20))
+    assert calls == [0]
+
+
 def test_prefill_batch_engine_parity(dev):
     """forward_prefill_batch (varlen kernel path) vs sequential
     forward_prefill on the GPU engine: same logits, same KV."""
