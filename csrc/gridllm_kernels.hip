@@ -38,13 +38,13 @@
 // product whose K is in parts, rounded as its result would be.
 struct StoredRow {
     const bf16_t* x;
-    DEV_INLINE uint4 operator()(int c) const { return ((const uint4*)x)[c]; }
+    DEV_INLINE uint4 operator()(long c) const { return ((const uint4*)x)[c]; }
 };
 struct SummedRow {
     const float* ws;
     long stride;
     int parts;
-    DEV_INLINE uint4 operator()(int c) const {
+    DEV_INLINE uint4 operator()(long c) const {
         float f[8] = {};
 #pragma unroll 4
         for (int k = 0; k < parts; ++k) {
@@ -336,9 +336,12 @@ k_rope_kv(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ q_out,
 // loads and stores), as many copy a v head; heads of all tokens lie one after
 // the other over the lanes. D % 16 == 0 and rows at 16 bytes. 8000 tokens of
 // 24 + 8 + 8 heads of 128: 83 us (2 TB/s) with a wave per head and 2-byte
-// accesses, 31 us (5.2 TB/s) now.
+// accesses, 31 us (5.2 TB/s) now. Rows may be a product's partial sums (SummedRow),
+// which spares the kernel that adds them up (four layers of llama3.2:1b, 45
+// tokens 323 -> 316 us).
+template <class Row>
 __global__ void __launch_bounds__(256)
-k_rope_kv8(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ q_out,
+k_rope_kv8(const Row rows, bf16_t* __restrict__ q_out,
            bf16_t* __restrict__ kc, bf16_t* __restrict__ vc,
            const float* __restrict__ cost, const float* __restrict__ sint,
            const int* __restrict__ pos, const int* __restrict__ slot,
@@ -350,8 +353,8 @@ k_rope_kv8(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ q_out,
     if (item >= (long)N * heads) return;
     const int c = (int)(i % lanes) * 8;
     const int n = (int)(item / heads), h = (int)(item % heads);
-    const bf16_t* src = qkv + item * D + c;
-    uint4 lo = *(const uint4*)src, hi = *(const uint4*)(src + half);
+    const long src = (item * D + c) >> 3;
+    uint4 lo = rows(src), hi = rows(src + (half >> 3));
     if (bias) {
         float a[8], b[8];
         unpack8(lo, a);
@@ -1390,8 +1393,10 @@ int gl_kv_append(void* stream, void* kc, void* vc, const void* kn,
     return 0;
 }
 
-int gl_rope_kv(void* stream, const void* qkv, void* q_out, void* kc, void* vc,
-               const void* cost, const void* sint, const void* pos,
+// parts > 0: qkv is f32 sums [parts, N, (Hq + 2 Hk) D] (D % 16 == 0, all at 16
+// bytes).
+int gl_rope_kv(void* stream, const void* qkv, int parts, void* q_out, void* kc,
+               void* vc, const void* cost, const void* sint, const void* pos,
                const void* slot, const void* bias, int N, int Hq, int Hk, int D,
                int Smax) {
     if (D % 4 != 0 || N == 0) return (D % 4) ? -100 : 0;
@@ -1399,15 +1404,20 @@ int gl_rope_kv(void* stream, const void* qkv, void* q_out, void* kc, void* vc,
         (unsigned long)kc | (unsigned long)vc | (unsigned long)cost |
         (unsigned long)sint | (unsigned long)bias;
     if (D % 16 == 0 && ptrs % 16 == 0) {
-        const long items = (long)N * (Hq + 2 * Hk) * (D / 16);
-        k_rope_kv8<<<dim3((unsigned)((items + 255) / 256)), dim3(256), 0,
-                     (hipStream_t)stream>>>(
-            (const bf16_t*)qkv, (bf16_t*)q_out, (bf16_t*)kc, (bf16_t*)vc,
-            (const float*)cost, (const float*)sint, (const int*)pos,
-            (const int*)slot, (const bf16_t*)bias, N, Hq, Hk, D, Smax);
+        const long heads = Hq + 2 * Hk, items = N * heads * (D / 16);
+        const SummedRow sums{(const float*)qkv, N * heads * D, parts};
+#define GO(rows) k_rope_kv8<<<dim3((unsigned)((items + 255) / 256)), \
+            dim3(256), 0, (hipStream_t)stream>>>( \
+            rows, (bf16_t*)q_out, (bf16_t*)kc, (bf16_t*)vc, \
+            (const float*)cost, (const float*)sint, (const int*)pos, \
+            (const int*)slot, (const bf16_t*)bias, N, Hq, Hk, D, Smax)
+        if (parts > 0) GO(sums);
+        else GO(StoredRow{(const bf16_t*)qkv});
+#undef GO
         LAUNCH_CHECK();
         return 0;
     }
+    if (parts > 0) return -100;
     k_rope_kv<<<dim3((unsigned)(N * (Hq + Hk))), dim3(64), 0,
                 (hipStream_t)stream>>>(
         (const bf16_t*)qkv, (bf16_t*)q_out, (bf16_t*)kc, (bf16_t*)vc,
@@ -1733,30 +1743,38 @@ static int layer_product(void* st, const LayerProduct& p, void* out, void* ws,
                         u.limit, u.shift, u.cubic);
 }
 
+// A product's parts of K that what follows adds up; 0: none, or one.
+static int layer_parts(const LayerProduct& p, int K) {
+    if (p.kind != 1 || p.c < 2 || K <= 64) return 0;
+    const int slice = ((K + (int)p.c - 1) / (int)p.c + 63) / 64 * 64;
+    return (K + slice - 1) / slice;
+}
+
 // (rmsnorm(y) * weight, y) of y = x w^T + resid
 static int layer_joined(void* st, const LayerProduct& p, const PromptLayer& l,
                         const void* x, const void* w, int K, const void* weight,
                         const void* resid, void* normed, void* sum, float eps) {
     const int T = (int)l.T, H = (int)l.H;
-    const bool parts = p.kind == 1 && p.c > 1 && K > 64 && H % 8 == 0;
+    const int parts = H % 8 ? 0 : layer_parts(p, K);
     const int e = layer_product(st, p, parts ? nullptr : l.y, l.ws, x, w, T, H, K,
                                 0);
     if (e) return e;
     if (!parts)
         return gl_rmsnorm(st, normed, l.y, weight, resid, sum, T, H, eps);
-    const int slice = ((K + (int)p.c - 1) / (int)p.c + 63) / 64 * 64;
-    return gl_rmsnorm_parts(st, normed, l.ws, (K + slice - 1) / slice, weight,
-                            resid, sum, T, H, eps);
+    return gl_rmsnorm_parts(st, normed, l.ws, parts, weight, resid, sum, T, H,
+                            eps);
 }
 
 int gl_prompt_layer(void* st, const void* layer, float scale, float eps) {
     const PromptLayer& l = *(const PromptLayer*)layer;
     const int T = (int)l.T, H = (int)l.H, Hq = (int)l.Hq, Hk = (int)l.Hk;
     const int D = (int)l.D, Smax = (int)l.Smax;
-    int e = layer_product(st, l.p_qkv, l.qkv, l.ws, l.normed, l.wqkv, T,
-                          (Hq + 2 * Hk) * D, H, 0);
-    if (!e) e = gl_rope_kv(st, l.qkv, l.q, l.kc, l.vc, l.cost, l.sint, l.pos,
-                           l.places, l.bqkv, T, Hq, Hk, D, Smax);
+    const int parts = layer_parts(l.p_qkv, H);
+    int e = layer_product(st, l.p_qkv, parts ? nullptr : l.qkv, l.ws, l.normed,
+                          l.wqkv, T, (Hq + 2 * Hk) * D, H, 0);
+    if (!e) e = gl_rope_kv(st, parts ? l.ws : l.qkv, parts, l.q, l.kc, l.vc,
+                           l.cost, l.sint, l.pos, l.places, l.bqkv, T, Hq, Hk, D,
+                           Smax);
     if (!e) e = l.meta
         ? gl_attn_prefill_batch(st, l.attn, l.q, l.kc, l.vc, l.meta,
                                 (int)l.tiles, Hq, Hk, D, Smax, scale)

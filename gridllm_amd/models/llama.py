@@ -32,6 +32,7 @@ from gridllm_amd.ops.autotune import choice_of as _choice_of
 from gridllm_amd.ops.autotune import linear as _linear
 from gridllm_amd.ops.autotune import linear_f32 as _linear_f32
 from gridllm_amd.ops.autotune import linear_gateup as _linear_gateup
+from gridllm_amd.ops.autotune import linear_parts as _linear_parts
 from gridllm_amd.ops.autotune import linear_rmsnorm as _linear_rmsnorm
 
 from gridllm_amd import ops
@@ -227,6 +228,11 @@ class LlamaModel:
         self.tp.all_reduce(out)
         return ops.rmsnorm(out, norm, self.spec.norm_eps, residual=resid)
 
+    def _qkv(self, normed: torch.Tensor, lw: LayerWeights) -> torch.Tensor:
+        """Queries, keys and values, or their partial sums, for rope_kv."""
+        return (_linear if self.spec.head_dim % 16 else _linear_parts)(
+            normed, lw.wqkv)
+
     def _mlp_act(self, normed: torch.Tensor, lw: LayerWeights) -> torch.Tensor:
         if self.gateup_il:
             return _linear_gateup(normed, lw.wgateup)
@@ -417,12 +423,15 @@ class LlamaModel:
             return 0
         sizes = ((n, h), (h, at), (2 * f, h), (h, f))
         norms = [lw.attn_norm for lw in self.layers] + [self.final_norm]
-        for lw in self.layers[:layers]:
+        if not self.final_norm.is_contiguous():
+            return 0
+        for lw in self.layers:
             for w, size in zip((lw.wqkv, lw.wo, lw.wgateup, lw.wdown), sizes):
                 if w.shape != size or w.dtype is not bf16 or \
                         w.data_ptr() & 15 or not w.is_contiguous():
                     return 0
-            if not lw.mlp_norm.is_contiguous():
+            if not (lw.mlp_norm.is_contiguous() and lw.attn_norm.is_contiguous()
+                    and (lw.bqkv is None or lw.bqkv.is_contiguous())):
                 return 0
         # a layer's rows, one behind the other, from 16 bytes on each
         dev, parts = self.device, 0
@@ -479,7 +488,7 @@ class LlamaModel:
                     normed, pos, slot_t, normed[-1:], resid[-1:], pos[-1:],
                     counts[t:], slot)
                 break
-            q = ops.rope_kv(_linear(normed, lw.wqkv), self.cache.k[li],
+            q = ops.rope_kv(self._qkv(normed, lw), self.cache.k[li],
                             self.cache.v[li], self.cos, self.sin, pos, slot_t,
                             self.hq_l, self.hkv_l, self.spec.head_dim, lw.bqkv)
             attn = ops.attn_prefill_cache(
@@ -552,7 +561,7 @@ class LlamaModel:
                     normed, pos, slot_t, normed[ends[3]], resid[ends[3]],
                     ends[0], ends[1], ends[2])
                 break
-            q = ops.rope_kv(_linear(normed, lw.wqkv), self.cache.k[li],
+            q = ops.rope_kv(self._qkv(normed, lw), self.cache.k[li],
                             self.cache.v[li], self.cos, self.sin, pos, slot_t,
                             self.hq_l, self.hkv_l, self.spec.head_dim, lw.bqkv)
             if meta is not None:
@@ -602,7 +611,7 @@ class LlamaModel:
         resid, normed = ops.embed_norm(tokens, self.embed,
                                        self.layers[0].attn_norm, s.norm_eps)
         for li, lw in enumerate(self.layers):
-            q = ops.rope_kv(_linear(normed, lw.wqkv), self.cache.k[li],
+            q = ops.rope_kv(self._qkv(normed, lw), self.cache.k[li],
                             self.cache.v[li], self.cos, self.sin, pos_rope,
                             slot_t, self.hq_l, self.hkv_l, self.spec.head_dim,
                             lw.bqkv)

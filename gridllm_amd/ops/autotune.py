@@ -247,7 +247,7 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """linear(x, w), or its f32 partial sums [parts, M, N] if K is in parts, for
-    post_norm and join_norm."""
+    post_norm, join_norm and rope_kv."""
     c = _choose(x, w)
     if c is not None and c[0] == "tile" and c[3] > 1 and w.shape[1] > 64:
         return hip_ops.gemm_tile_parts(x, w, *c[1:])

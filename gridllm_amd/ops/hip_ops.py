@@ -57,8 +57,7 @@ def _load() -> ctypes.CDLL:
     lib.gl_rope.restype = c_i
     lib.gl_swiglu.argtypes = [c_vp, c_vp, c_vp, c_l, c_i, c_f, c_f, c_f, c_f]
     lib.gl_swiglu.restype = c_i
-    lib.gl_rope_kv.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp,
-                               c_vp, c_vp, c_i, c_i, c_i, c_i, c_i]
+    lib.gl_rope_kv.argtypes = [c_vp, c_vp, c_i] + [c_vp] * 8 + [c_i] * 5
     lib.gl_rope_kv.restype = c_i
     lib.gl_prompt_layer.argtypes = [c_vp, c_vp, c_f, c_f]
     lib.gl_prompt_layer.restype = c_i
@@ -258,17 +257,25 @@ def rope_kv(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
             slot: torch.Tensor, hq: int, hk: int, d: int,
             bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Fused RoPE + KV write from the raw QKV GEMM output.
-    qkv: [N, (hq+2*hk)*d] bf16 (row-dense), bias: [(hq+2*hk)*d] bf16, added to
-    it; returns roped q [N, hq, d]."""
+    qkv: [N, (hq+2*hk)*d] bf16 (row-dense), or f32 partial sums of it [parts, N,
+    ..] (d % 16 == 0); bias: [(hq+2*hk)*d] bf16, added to it; returns roped q [N,
+    hq, d]."""
     lib = _load()
-    n = qkv.shape[0]
+    n, width = qkv.shape[-2:]
+    parts = qkv.shape[0] if qkv.dim() == 3 else 0
+    if qkv.dtype != (torch.float32 if parts else torch.bfloat16) or (
+            bias is not None and (bias.dtype != torch.bfloat16 or
+                                  bias.shape != (width,)
+                                  or not bias.is_contiguous())):
+        raise ValueError("rope_kv: bf16 rows, or their f32 parts, and a dense "
+                         "bf16 bias")
     smax = kcache.shape[2]
     _check_range("rope_kv.slot", slot, kcache.shape[0] * smax)
     _check_range("rope_kv.pos", pos, cos.shape[0])
-    q_out = torch.empty(n, hq, d, dtype=qkv.dtype, device=qkv.device)
-    _check(lib.gl_rope_kv(_stream(), _ptr(qkv), _ptr(q_out), _ptr(kcache),
-                          _ptr(vcache), _ptr(cos), _ptr(sin), _ptr(pos),
-                          _ptr(slot), _ptr(bias), n, hq, hk, d, smax),
+    q_out = torch.empty(n, hq, d, dtype=torch.bfloat16, device=qkv.device)
+    _check(lib.gl_rope_kv(_stream(), _ptr(qkv), parts, _ptr(q_out),
+                          _ptr(kcache), _ptr(vcache), _ptr(cos), _ptr(sin),
+                          _ptr(pos), _ptr(slot), _ptr(bias), n, hq, hk, d, smax),
            "rope_kv")
     return q_out
 

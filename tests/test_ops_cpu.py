@@ -373,3 +373,24 @@ def test_rmsnorm_of_a_residual_needs_a_place_for_the_sum():
     lib = hip_ops._load()
     assert lib.gl_rmsnorm(None, x.data_ptr(), x.data_ptr(), x.data_ptr(),
                           x.data_ptr(), None, 2, 64, 1e-5) == -100
+
+
+def test_rope_kv_refuses():
+    """Rows of other types, and a bias of another type, size or stride, ahead of
+    the launch."""
+    from gridllm_amd.ops import hip_ops
+    bf16 = torch.bfloat16
+    kc = torch.zeros(1, 1, 8, 16, dtype=bf16)
+    cos, sin = R.rope_tables(16, 8)
+    at = torch.zeros(2, dtype=torch.int32)
+
+    def call(rows, bias=None):
+        hip_ops.rope_kv(rows, kc, kc, cos, sin, at, at, 2, 1, 16, bias)
+    rows = torch.zeros(2, 64, dtype=bf16)
+    for bad in (rows.float(), rows.half(), rows.expand(3, 2, 64)):
+        with pytest.raises(ValueError):
+            call(bad)
+    for bias in (torch.zeros(64), torch.zeros(32, dtype=bf16),
+                 torch.zeros(128, dtype=bf16)[::2]):
+        with pytest.raises(ValueError):
+            call(rows, bias)

@@ -260,6 +260,31 @@ def test_rope_kv_fused_gpu(dev, n, hq, hk, d):
     assert _mx(vc.cpu(), vc_ref) < 1e-6
 
 
+@pytest.mark.parametrize("n,hq,hk,d,parts,bias", [
+    (1, 3, 1, 16, 1, False), (45, 32, 8, 64, 4, True), (7, 24, 8, 128, 9, False)])
+def test_rope_kv_of_parts_gpu(dev, n, hq, hk, d, parts, bias):
+    """A product's partial sums and its bias: to the bit what its sum (by the
+    first part's order, rounded) and the bias' addition by torch give."""
+    torch.manual_seed(n)
+    from gridllm_amd.ops import hip_ops
+    ws = torch.randn(parts, n, (hq + 2 * hk) * d, device=dev)
+    qkv = torch.zeros_like(ws[0])
+    for x in ws:
+        qkv += x
+    qkv = qkv.to(torch.bfloat16)
+    add = torch.randn_like(qkv[0]) if bias else None
+    kc = torch.zeros(2, hk, 64, d, device=dev, dtype=torch.bfloat16)
+    caches = [kc, kc.clone(), kc.clone(), kc.clone()]
+    cos, sin = R.rope_tables(d, 128, device=dev)
+    pos = torch.randint(0, 120, (n,), dtype=torch.int32, device=dev)
+    slot = torch.randperm(128)[:n].int().to(dev)
+    got = hip_ops.rope_kv(ws, *caches[:2], cos, sin, pos, slot, hq, hk, d, add)
+    want = hip_ops.rope_kv(qkv if add is None else qkv + add, *caches[2:], cos,
+                           sin, pos, slot, hq, hk, d)
+    assert torch.equal(got, want) and torch.equal(caches[0], caches[2])
+    assert torch.equal(caches[1], caches[3])
+
+
 @pytest.mark.parametrize("m,n,k", [
     (1, 3072, 3072), (13, 5120, 3072), (64, 16384, 3072),
     (64, 3072, 8192), (127, 3072, 3072), (256, 128256, 3072),
