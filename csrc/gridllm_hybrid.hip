@@ -19,6 +19,7 @@
 
 #include "gridllm_attention.h"
 #include "gridllm_tiles.h"
+#include "gridllm_wide.h"
 
 // ===========================================================================
 // x = embed[token], f32, plus pos_table[position] if there is one, then its
@@ -2462,6 +2463,37 @@ k_moe_gemm(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
     }
 }
 
+// Many rows per expert: by k_gemm_wide's tiles, S::R rows of the list's by S::C
+// columns, blocks of one a CU that take them in turn. 4096 tokens, 64 experts of 3072
+// x 1024, 8 of them chosen 621 -> 493 us for both products (840 TFLOP/s; the tile
+// lists' last tiles are half empty), gated, 7 762 -> 575; bound as k_gemm_wide.
+struct ExpertRows {
+    static constexpr bool GATHER = true;
+    const int* sorted;
+    const float* pw;
+    int top;                       // up: x's rows are tokens'; 0: down
+    DEV_INLINE int from(int m) const { return top ? sorted[m] / top : m; }
+    DEV_INLINE long to(int m) const { return top ? m : sorted[m]; }
+    DEV_INLINE float weight(int m) const { return pw ? pw[sorted[m]] : 1.f; }
+};
+
+template <class S, int ACT>
+__global__ void __launch_bounds__(512, 2)
+k_moe_wide(const WideArgs p, const int4* __restrict__ tiles,
+           const int* __restrict__ sorted, int top, int experts, int max_tiles,
+           const float* __restrict__ pw) {
+    extern __shared__ __attribute__((aligned(16))) bf16_t wide_lds[];
+    const int cb = (p.N + S::C - 1) / S::C, items = tiles[max_tiles].x * cb;
+    const int xcd = blockIdx.x & 7, at = (int)(blockIdx.x >> 3);
+    const int each = (items + 7) >> 3;          // tiles of an XCD
+    wide_tiles<S, ACT == 2 ? 4 : ACT ? 3 : 0>(
+        p, wide_lds, xcd * each + at, min(items, (xcd + 1) * each),
+        (int)(gridDim.x >> 3), [&](int it) {
+            const int4 tl = tiles[it / cb];
+            return WideTile{tl.y, tl.y + tl.z, it % cb * S::C, tl.x * p.N};
+        }, experts * p.N, ExpertRows{sorted, pw, ACT ? top : 0});
+}
+
 // A few rows: up to 16 against 16 columns per block, K split over the 4 waves,
 // so that a handful of experts still fills the chip. (16 output columns: 32
 // weight rows if gated.)
@@ -2582,6 +2614,26 @@ k_moe_gemm_f32(float* __restrict__ out, const float* __restrict__ x,
 // ===========================================================================
 // Entry points. f32 != 0 selects the exact mode. 0 = success.
 // ===========================================================================
+typedef WideShape<4, 4, 3> Moe128;
+typedef WideShape<6, 4, 2> Moe192;
+typedef WideShape<8, 4, 2> Moe256;
+
+template <class S, int ACT>
+static int go_moe_wide(hipStream_t st, const WideArgs& p, const void* tiles,
+                       const void* sorted, int top, int experts, int max_tiles,
+                       const void* pw) {
+    static const hipError_t e = hipFuncSetAttribute(
+        (const void*)k_moe_wide<S, ACT>,
+        hipFuncAttributeMaxDynamicSharedMemorySize, S::BYTES);
+    if (e) return (int)e;
+    const long most = (long)max_tiles * ((p.N + S::C - 1) / S::C);
+    k_moe_wide<S, ACT><<<(unsigned)(8 * min((most + 7) / 8, 32l)), 512, S::BYTES,
+                         st>>>(p, (const int4*)tiles, (const int*)sorted, top,
+                               experts, max_tiles, (const float*)pw);
+    LAUNCH_CHECK();
+    return 0;
+}
+
 template <int D, int G>
 static void launch_paged_decode(hipStream_t st, void* out, const void* q,
                                 const PagedKV<D>& kv, const int* pos,
@@ -3115,11 +3167,12 @@ int gh_moe_route(void* stream, void* idx, void* wt, void* rank, void* counts,
 // act: 0 down, 1 up with squared ReLU, 2 gate and up (N weight rows, in turns
 // of 16 | 16) with the gated unit's constants; pw (nullable): weights of the
 // pairs on its input. bm: rows per tile of the list: 16 (few pairs; the exact
-// mode), 32 or 128
+// mode), 32 or 128; or, wide, 128, 192 or 256, with `rows` of x and as many experts
 int gh_moe_gemm(void* stream, int f32, int act, void* out, const void* x,
                 const void* w, const void* tiles, const void* sorted,
-                int top, int N, int K, int bm, int max_tiles, float alpha,
-                float limit, float shift, float cubic, const void* pw) {
+                int top, int N, int K, int bm, int max_tiles, int wide,
+                int rows, int experts, float alpha, float limit, float shift, float cubic,
+                const void* pw) {
     if (N % (act == 2 ? 128 : 64) || K % 64 || max_tiles < 1 || act < 0 ||
         act > 2)
         return -100;
@@ -3140,7 +3193,20 @@ int gh_moe_gemm(void* stream, int f32, int act, void* out, const void* x,
 #define ARGS (bf16_t*)out, (const bf16_t*)x, (const bf16_t*)w, \
         (const int4*)tiles, (const int*)sorted, top, N, K, ntn, max_tiles, \
         glu, (const float*)pw
-    if (bm == 32 || bm == 128) {
+    if (wide) {
+        if (bm != 128 && bm != 192 && bm != 256) return -103;
+        if ((long)experts * N * K * 2 > WIDE_BYTES || K < 256 || experts < 1 ||
+            (long)rows * K * 2 > 1l << 30) return -100;
+        const WideArgs p{out, (const bf16_t*)x, (const bf16_t*)w, rows, N, K, glu};
+#define GO(S) return act == 2 ? go_moe_wide<S, 2>(st_, p, tiles, sorted, top, \
+            experts, max_tiles, pw) : act ? go_moe_wide<S, 1>(st_, p, tiles, \
+            sorted, top, experts, max_tiles, pw) : go_moe_wide<S, 0>(st_, p, \
+            tiles, sorted, top, experts, max_tiles, pw)
+        if (bm == 128) GO(Moe128);
+        if (bm == 192) GO(Moe192);
+        GO(Moe256);
+#undef GO
+    } else if (bm == 32 || bm == 128) {
         const int ntn = (N + 127) / 128;
         const unsigned grid = (unsigned)((max_tiles * ntn + 7) / 8 * 8);
 #define GO(NB, R) do { \

@@ -27,6 +27,7 @@
 //
 // EPI 1: W rows in groups of 64 gate | 64 up; stores the gated unit [M, N / 2].
 // EPI 2: the result, rounded to bf16, as f32 (a vocabulary's scores).
+// EPI 3: squared ReLU. EPI 4: W rows in turns of 16 gate | 16 up, [M, N / 2].
 // Rows past M and N are read as zeros by the buffer descriptors' bounds, and so are
 // the stages past the last tile: a wave's offset is the end of the matrix at most,
 // and a lane's is added to it.
@@ -50,6 +51,20 @@ struct WideArgs {
     GluParams glu;
 };
 
+// A tile: its first row, the row behind its last one, its first column, and the row
+// of W where its matrix starts.
+struct WideTile {
+    int m0, end, n0, w0;
+};
+
+// Where rows come from and go to. GATHER: x's rows are looked up one by one.
+struct DenseRows {
+    static constexpr bool GATHER = false;
+    DEV_INLINE int from(int m) const { return m; }
+    DEV_INLINE long to(int m) const { return m; }
+    DEV_INLINE float weight(int m) const { return 1.f; }
+};
+
 template <int A_, int B_, int NB_>
 struct WideShape {
     static constexpr int A = A_, B = B_, NB = NB_, R = A * 32, C = B * 64;
@@ -59,18 +74,21 @@ struct NoShape {
     static constexpr int R = 0, BYTES = 0;
 };
 
-// Tiles item, item + stride, ... < last, whose first rows and columns are place's.
-template <class S, int EPI, class Place>
+// Tiles item, item + stride, ... < last, as place says; wrows: of W.
+template <class S, int EPI, class Place, class Rows = DenseRows>
 DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
-                           int stride, Place place) {
+                           int stride, Place place, int wrows,
+                           const Rows rows = Rows()) {
 #ifdef __HIP_DEVICE_COMPILE__          // (the host has no buffer descriptors)
     constexpr int A = S::A, B = S::B, NB = S::NB, R = S::R, C = S::C;
     constexpr int BUF = (R + C) * 64, G = (R + C) / 64;  // loads of a wave, stage
+    constexpr bool PLAIN = EPI == 4;            // W's rows are in order
     constexpr int STORES = EPI == 1 ? A * B / 4 : EPI == 2 ? A * B
-                                                : A * ((B + 1) / 2);
+                           : PLAIN ? A * B / 2 : A * ((B + 1) / 2);
+    constexpr int GX = Rows::GATHER ? R / 64 : 1;
     constexpr int L1 = G / 4, L2 = 2 * L1;      // loads behind quarters 2 and 3
     static_assert(A % 2 == 0 && (EPI != 1 || B % 4 == 0) &&
-                  (EPI != 2 || B % 2 == 0), "halves");
+                  ((EPI != 2 && !PLAIN) || B % 2 == 0), "halves");
     static_assert((NB - 2) * G + L2 + STORES < 64, "that can be counted");
     if (item >= last) return;
     const int M = p.M, N = p.N, K = p.K, nt = K >> 6;
@@ -80,37 +98,42 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
     const auto xr = __builtin_amdgcn_make_buffer_rsrc(
         (void*)p.x, 0, (int)((u32)M * K * 2), 0x00020000);
     const auto wrs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)p.w, 0, (int)((u32)N * K * 2), 0x00020000);
+        (void*)p.w, 0, (int)((u32)wrows * K * 2), 0x00020000);
 
     // A load takes 8 rows of the stage to LDS in the order of lanes. Row j of W's
     // tile b is column 8 (j / 4) + j % 4, + 4 for an odd b, of the two tiles' 32 (a
     // last, single tile: j), or of two tiles of gates, and of ups.
     const int lr = lane >> 3, at = ((lane & 7) ^ lr) * 16;
-    int vx, vw;                                 // a lane's offsets, with k
+    int vx[GX], vw;                             // a lane's offsets, with k
     u32 so[G];                                  // the wave's, of its rows
     auto tile_of = [&](int i) {                 // W's tile in a wave's load i
         return ((i * 8 + wid) * 8 - R) % (B * 16) >> 4;
     };
     auto aim = [&](int it) {
-        int m0, n0;
-        place(it, &m0, &n0);
-        vx = lr * K * 2 + at;
-        vw = ((lr >> 2) * 8 + (lr & 3)) * K * 2 + at;
+        const WideTile t = place(it);
+        const int m0 = t.m0, n0 = t.n0;
+        if constexpr (!Rows::GATHER) vx[0] = lr * K * 2 + at;
+        vw = (PLAIN ? lr : (lr >> 2) * 8 + (lr & 3)) * K * 2 + at;
 #pragma unroll
         for (int i = 0; i < G; ++i) {
             const int row = (i * 8 + wid) * 8;
             int r = min(m0 + row, M);
+            if (Rows::GATHER && i * 64 < R) {
+                vx[i % GX] = (u32)rows.from(min(m0 + row + lr, t.end - 1)) * K *
+                                 2 + at;
+                r = 0;
+            }
             if (i * 64 >= R) {
                 const int v = (row - R) / (B * 16), b = tile_of(i), j = row & 15;
                 const int c = B % 2 && b == B - 1 ? j
                                                   : (j >> 2) * 8 + (b & 1) * 4;
-                r = n0 + v * B * 16 + (b >> 1) * 32 + c;
+                r = n0 + (PLAIN ? row - R : v * B * 16 + (b >> 1) * 32 + c);
                 if (EPI == 1) {
                     const int o = (n0 >> 1) + v * B * 8 +
                                   (b % (B / 2) >> 1) * 32 + c;
                     r = (o >> 6) * 128 + (o & 63) + (b >= B / 2 ? 64 : 0);
                 }
-                r = min(r, N);
+                r = min(t.w0 + r, wrows);
             }
             so[i] = (u32)r * K * 2;             // (the end, at most)
         }
@@ -121,9 +144,12 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
             of_x ? xr : wrs,
             (__attribute__((address_space(3))) unsigned int*)(
                 lds + buf * BUF + (i * 8 + wid) * 512),
-            16, of_x || (B % 2 && tile_of(i) == B - 1) ? vx : vw, so[i], 0, 0);
+            16, of_x ? vx[i % GX]
+                : !Rows::GATHER && B % 2 && tile_of(i) == B - 1 ? vx[0] : vw,
+            so[i], 0, 0);
         if (i + 1 == G) {
-            vx += 128;
+#pragma unroll
+            for (int k = 0; k < GX; ++k) vx[k] += 128;
             vw += 128;
         }
     };
@@ -184,8 +210,8 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
     lds_barrier();
     bool stored = false;                        // all of the tile before
     for (; item < last; item += stride) {
-        int m0, n0;
-        place(item, &m0, &n0);
+        const WideTile t = place(item);
+        const int m0 = t.m0, n0 = t.n0;
 #pragma unroll
         for (int i = 0; i < A + B; ++i) read(buf, 0, i);
 #pragma unroll
@@ -199,7 +225,7 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
                 else
 #pragma unroll
                     for (int i = 0; i < G; ++i)
-                        so[i] = (u32)(i * 64 < R ? M : N) * K * 2;
+                        so[i] = (u32)(i * 64 < R ? M : wrows) * K * 2;
             }
             stage(kt < NB - 1 && stored, std::true_type());
         }
@@ -208,9 +234,26 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
 #pragma unroll
         for (int a = 0; a < A; ++a) {
             const int m = m0 + (wr * A + a) * 16 + fr;
-            if (m >= M) continue;
-            const int ld = EPI == 1 ? N >> 1 : N;
-            const int nw = EPI == 1 ? (n0 >> 1) + wc * B * 8 : n0 + wc * B * 16;
+            if (m >= t.end) continue;
+            const int ld = EPI == 1 || EPI == 4 ? N >> 1 : N;
+            const long at = rows.to(m) * ld;
+            const int nw = EPI == 1 ? (n0 >> 1) + wc * B * 8
+                : EPI == 4 ? (n0 >> 1) + wc * B * 8 : n0 + wc * B * 16;
+            if constexpr (PLAIN) {
+                const float wi = rows.weight(m);
+#pragma unroll
+                for (int b = 0; b < B; b += 2) {
+                    const int n = nw + b * 8 + gq * 4;
+                    if (n >= ld) continue;
+                    float f[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        f[r] = glu_act(wi * acc[a][b][r],
+                                       wi * acc[a][(b + 1) % B][r], p.glu);
+                    st4((bf16_t*)p.out + at + n, f);
+                }
+                continue;
+            }
 #pragma unroll
             for (int b = 0; b + 1 < (EPI == 1 ? B / 2 : B); b += 2) {
                 const int n = nw + b * 16 + gq * 8;
@@ -220,14 +263,15 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
                 for (int r = 0; r < 8; ++r) {
                     const float v = acc[a][b + (r >> 2)][r & 3];
                     f[r] = EPI == 1 ? glu_act(
-                        v, acc[a][b + (r >> 2) + B / 2][r & 3], p.glu) : v;
+                        v, acc[a][b + (r >> 2) + B / 2][r & 3], p.glu)
+                        : EPI == 3 ? fmaxf(v, 0.f) * fmaxf(v, 0.f) : v;
                 }
                 const bf16x8 v = to_bf16x8(f);
                 if (EPI == 2) {
                     unpack8(__builtin_bit_cast(uint4, v), f);
-                    st8((float*)p.out + (long)m * ld + n, f);
+                    st8((float*)p.out + at + n, f);
                 } else {
-                    *(bf16x8*)((bf16_t*)p.out + (long)m * ld + n) = v;
+                    *(bf16x8*)((bf16_t*)p.out + at + n) = v;
                 }
             }
             if constexpr (B % 2 && EPI == 0) {
@@ -236,10 +280,10 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
                 bf16x4 v;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) v[r] = (__bf16)acc[a][B - 1][r];
-                *(bf16x4*)((bf16_t*)p.out + (long)m * ld + n) = v;
+                *(bf16x4*)((bf16_t*)p.out + at + n) = v;
             }
         }
-        stored = m0 + R <= M && n0 + C <= N;
+        stored = m0 + R <= t.end && n0 + C <= N;
     }
     WAIT_LOADS(0);                              // (of nothing, into LDS)
     lds_barrier();
@@ -253,24 +297,24 @@ k_gemm_wide(const WideArgs p, int full) {
     const int rb = (p.M + S::R - 1) / S::R, cb = (p.N + S::C - 1) / S::C;
     const int xcd = blockIdx.x & 7, at = (int)(blockIdx.x >> 3);
     const int stride = (int)(gridDim.x >> 3);
-    auto place = [&](int it, int* m0, int* n0) {
+    auto place = [&](int it) {
         const int group = it / (4 * cb), in = it - group * 4 * cb;
         const int rows = min(4, rb - group * 4);
-        *m0 = (group * 4 + in % rows) * S::R;
-        *n0 = in / rows * S::C;
+        return WideTile{(group * 4 + in % rows) * S::R, p.M, in / rows * S::C, 0};
     };
     const int each = (full + 7) >> 3;           // tiles of an XCD
     wide_tiles<S, EPI>(p, lds, xcd * each + at, min(full, (xcd + 1) * each),
-                       stride, place);
+                       stride, place, p.N);
     if constexpr (S2::R > 0) {
         static_assert(S2::R * 2 == S::R && S2::C == S::C, "halves");
         const int rest = (rb * cb - full) * 2, each = (rest + 7) >> 3;
         wide_tiles<S2, EPI>(
             p, lds, xcd * each + at, min(rest, (xcd + 1) * each), stride,
-            [&](int it, int* m0, int* n0) {
-                place(full + (it >> 1), m0, n0);
-                *m0 += (it & 1) * S2::R;
-            });
+            [&](int it) {
+                WideTile t = place(full + (it >> 1));
+                t.m0 += (it & 1) * S2::R;
+                return t;
+            }, p.N);
     }
 }
 

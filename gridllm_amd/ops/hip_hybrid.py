@@ -11,6 +11,8 @@ reference_hybrid; ops.hybrid picks one by device.
 from __future__ import annotations
 
 import ctypes
+import functools
+import math
 import os
 from typing import Callable, Optional, Union
 
@@ -56,7 +58,7 @@ _SIGS = {
     "gh_gla_decay": "pppppiiiif",
     "gh_gla_chunks": "pppppppppiiiiiifif",
     "gh_moe_route": "pppppppippiiiiiiffiii",
-    "gh_moe_gemm": "iipppppiiiiiffffp",
+    "gh_moe_gemm": "iipppppiiiiiiiiffffp",
     "gn_latent_rows": "ippppippppppiiiiiiiif",
     "gn_head_gemm": "ippppiiiiili",
     "gn_latent_decode": "pppppipppppiiiiiiif",
@@ -486,7 +488,8 @@ def lightning(rows: torch.Tensor, S: torch.Tensor, decay: torch.Tensor,
     return out
 
 
-def _expert_rows(pairs: int, experts: int) -> int:
+@functools.lru_cache(maxsize=4096)
+def _expert_rows(pairs: int, experts: int, wide: tuple = ()) -> int:
     """Rows of an expert's tiles. 16, by the kernel that splits K over a block's
     waves, while the pairs are mostly of different experts; 32 while most experts
     have no more, whose blocks load less beside the weights; else 128. In us with
@@ -494,8 +497,41 @@ def _expert_rows(pairs: int, experts: int) -> int:
     119; 16 142, 140, 147; 48 183, 155, 160; 128 275, 158, 167; 192 -, 180, 170;
     and gated, of which 7 are: 2 65, 60, 78; 6 137, 145, 173; 12 178, 168, 199; 24
     223, 204, 216; 128 340, 223, 233; 192 -, 228, 237; 256 -, 248, 244. (64 rows are
-    at best 2 % faster than the better of 32 and 128.)"""
-    return 16 if pairs <= 64 else 32 if pairs <= 18 * experts else 128
+    at best 2 % faster than the better of 32 and 128.)
+    wide: ((N, K), ..) of the products if k_moe_wide takes them. Its tiles are of 256
+    columns, and of the rows that the rounds of CUs take least with, times a tile's
+    time (kWide's), were the pairs spread by chance: a few experts with a tile more
+    are a round more. 128, 192 and 256 rows: 512 tokens 189, 203, 207 us, 768 249, 214,
+    219, 1536 269, 317, 239, 4096 545, 493, 501 (the kernel for 128 x 128: 197, 257,
+    307, 621); gated 1024 325, 294, 304, 2048 398, 506, 346, 4096 659, 693, 575 (344,
+    447, 762)."""
+    if pairs <= 64:
+        return 16
+    if pairs <= 18 * experts:
+        return 32
+    mean = pairs / experts
+    spread = math.sqrt(mean * (1 - 1 / experts)) + 1e-9
+    best, least = 128, math.inf
+    for rows, us in ((128, .841), (192, 1.167), (256, 1.367)) if wide else ():
+        tiles = experts * sum(
+            0.5 * math.erfc((k * rows - mean) / spread / math.sqrt(2))
+            for k in range(int((mean + 6 * spread) / rows) + 1))
+        cost = sum(math.ceil(math.ceil(tiles - .005) * -(-n // 256) / 256) * us * k
+                   for n, k in wide)
+        if cost < least:
+            best, least = rows, cost
+    return best
+
+
+def _experts_wide(up: torch.Tensor, down: torch.Tensor, n: int, pairs: int
+                  ) -> tuple:
+    """(N, K) of the products if k_moe_wide takes them: rows and weights within a
+    buffer's offsets, and K of a ring of stages at least."""
+    sizes = tuple(up.shape[1:]), tuple(down.shape[1:])
+    fit = min(k for _, k in sizes) >= 256 and \
+        max(up.numel(), down.numel()) * 2 <= 0xe0000000 and \
+        max(n * sizes[0][1], pairs * sizes[1][1]) * 2 <= 1 << 30
+    return sizes if fit else ()
 
 
 def _routes_alone(n: int, pairs: int, outs: int) -> bool:
@@ -526,7 +562,9 @@ def moe(x: torch.Tensor, logits: torch.Tensor, up: torch.Tensor,
     assert outs >= e and (how.corr is None or how.corr.shape == (outs,))
     dev, f = x.device, _f32(x)
     pairs = n * top
-    bm = 16 if f else _expert_rows(pairs, e)
+    wide = () if f else _experts_wide(up, down, n, pairs)
+    bm = 16 if f else _expert_rows(pairs, e, wide)
+    wide = bool(wide) and bm >= 128
     max_tiles = min(pairs, e + pairs // bm)
     ints = torch.empty(3 * pairs, dtype=torch.int32, device=dev)
     idx, rank, order = ints[:pairs], ints[pairs:2 * pairs], ints[2 * pairs:]
@@ -541,10 +579,10 @@ def moe(x: torch.Tensor, logits: torch.Tensor, up: torch.Tensor,
           how.keep, how.eps, how.scale, int(how.sigmoid), bm, max_tiles)
     act = torch.empty(pairs, ff, dtype=x.dtype, device=dev)
     _call("gh_moe_gemm", f, rows // ff, act, x, up, tiles, order, top, rows, w,
-          bm, max_tiles, *how.glu, wt if how.weigh_input else None)
+          bm, max_tiles, wide, n, e, *how.glu, wt if how.weigh_input else None)
     ye = torch.empty(pairs, w, dtype=x.dtype, device=dev)
     _call("gh_moe_gemm", f, 0, ye, act, down, tiles, order, top, w, ff, bm,
-          max_tiles, *how.glu, None)
+          max_tiles, wide, pairs, e, *how.glu, None)
     return ye, wt, ident
 
 

@@ -172,6 +172,39 @@ def test_experts_at_the_edges_of_tiles(batch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("act", ["squared", "gated", "weighed"])
+@pytest.mark.parametrize("batch,rows", [(70, 128), (200, 192), (333, 256),
+                                        (700, 128)])
+def test_experts_by_wide_tiles(batch, rows, act, monkeypatch):
+    """What tiles of 128 x 128 give, to the bit: columns that the tiles do not
+    divide, behind which the next expert's weights lie, an expert without rows, one
+    with most of them, and K of few stages and of many."""
+    from gridllm_amd.ops import hip_hybrid
+    e, w, f, top = 7, 1088, 320, 2
+    g = torch.Generator().manual_seed(batch)
+    x, up, dn = (torch.randn(*s, generator=g).bfloat16().cuda() for s in (
+        (batch, w), (e, f if act == "squared" else 2 * f, w), (e, w, f)))
+    z = torch.randn(batch, e, generator=g)
+    z[:, 3] -= 50.0
+    z[:, 5] += 2.0
+    how = hops.Choice(top, sigmoid=act == "weighed",
+                      weigh_input=act == "weighed")
+    wide = hip_hybrid._experts_wide
+    seen = hip_hybrid._expert_rows
+    monkeypatch.setattr(hip_hybrid, "_expert_rows", lambda *a: rows)
+    got = hops.moe(x, z.cuda(), up * 0.1, dn, how)
+    assert wide(up, dn, batch, batch * top) == (up.shape[1:], dn.shape[1:])
+    monkeypatch.setattr(hip_hybrid, "_experts_wide", lambda *a: ())
+    monkeypatch.setattr(hip_hybrid, "_expert_rows", lambda *a: 128)
+    want = hops.moe(x, z.cuda(), up * 0.1, dn, how)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    sizes = ((1024, 3072), (3072, 1024))
+    assert [seen(8 * n, 64, sizes) for n in (512, 768, 1536)] == [128, 192, 256]
+    assert not wide(up[..., :192], dn, batch, batch * top)
+    assert not wide(up, dn, 1 << 20, 1 << 21)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m", [1, 64, 100, 300])
 def test_fused_gate_projection_takes_the_constants(m):
     """Every gated-unit path with a limit that cuts: the plain op, the
