@@ -687,9 +687,10 @@ k_gemm_rows(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
 // a piece of 128 bytes at the same place of each row, is in few of the memory's
 // channels (800 MB in rows of 16384 bytes 4.0 TB/s, of 6144 5.7). Blocks of
 // neighbouring columns then start one tile of K further on and wrap (6.05): 45 rows
-// of 128256 x 2048 134.7 -> 121.2 us, of 16384 x 2048 gated 20.1 -> 18.3, 64 of 3072
-// x 12288 in parts 24.2 -> 23.1. Other rows are read as fast in order (24 rows of
-// 5120 x 3072 12.8 us, 13.1; 16384 x 3072 22.8, 23.0).
+// of 128256 x 2048 134.7 -> 121.2 us, of 16384 x 2048 gated 20.1 -> 18.3. Parts of K
+// are at different places anyway (24 rows of 3072 x 8192 in 5 parts 16.2 either way,
+// 64 of 3072 x 12288 24.2, 23.1), and other rows are read as fast in order (24 rows
+// of 5120 x 3072 12.8 us, 13.1; 16384 x 3072 22.8, 23.0).
 //
 // Bound by a CU's loads: those of x, which hit in L2, and of W queue up behind
 // one another (12288 x 3072, 160 rows: x alone 9 us, W alone 13, both 27, with
@@ -740,7 +741,7 @@ k_gemm_tile(bf16_t* __restrict__ out, float* __restrict__ ws,
         const int c = (n0 >> 1) + r % (BN / 2);
         return (c >> 6) * 128 + (c & 63) + (r >= BN / 2 ? 64 : 0);
     };
-    const int turn = K % 2048 ? 0 : item / rblocks % cols % nt;
+    const int turn = K % 2048 || splitk > 1 ? 0 : item / rblocks % cols % nt;
     int left = nt - turn;                      // tiles up to the end of K's part
     const bf16_t* src[G];
 #pragma unroll
@@ -1574,7 +1575,11 @@ int gl_gemm_wide(void* stream, void* out, const void* x, const void* w, int M,
 //   K up to 4096 and 256 x 256 tiles that fill whole rounds and up to 0.6 of one,
 //   the library's worst sizes (0.93 over 40, 1.07 at most; 8000 x 5120 x 3072 284 ->
 //   196). Elsewhere it is 5 to 10 % faster than the kernel here.
-int gl_gemm_plan(int M, int N, int K, int fuse_glu, int* plan) {
+//   whole: not in parts of K, and gated units by k_gemm_wide, so that results are the
+// library's to the bit. Where a model makes much of a rounding (a sequence's first
+// token has one key, and a head's norm behind it leaves the sign of q . k alone),
+// they then don't depend on what runs them.
+int gl_gemm_plan(int M, int N, int K, int fuse_glu, int whole, int* plan) {
     plan[0] = plan[1] = plan[2] = plan[3] = 0;
     int shape = 0, full = 0, way = 0;
     float best = wide_best(M, N, K, fuse_glu ? 1 : 0, &shape, &full);
@@ -1585,7 +1590,7 @@ int gl_gemm_plan(int M, int N, int K, int fuse_glu, int* plan) {
     }
     const int heights[] = {96, 128, 160, 192, 256};
     const int widths[] = {64, 96, 128};
-    if (M > 0 && M <= 1200 && N > 0 && K > 0 && K % 64 == 0 &&
+    if (!whole && M > 0 && M <= 1200 && N > 0 && K > 0 && K % 64 == 0 &&
         !(fuse_glu && N % 128)) {
         for (int rows : heights) for (int cols : widths) {
             if (N % cols || (fuse_glu && cols == 96)) continue;

@@ -25,7 +25,9 @@
 // the first `full` tiles are of shape S, the others of the half as large S2
 // (2731 x 8192 x 2048: 92 us in 2 rounds of 256 x 256, 80 with the rest halved).
 //
-// EPI 1: W rows in groups of 64 gate | 64 up; stores the gated unit [M, N / 2].
+// EPI 1: W rows in groups of 64 gate | 64 up; stores the gated unit [M, N / 2] of
+// the results rounded to bf16: that is, to the bit, what the library's product and
+// the unit behind it give (sums over K go in the same order).
 // EPI 2: the result, rounded to bf16, as f32 (a vocabulary's scores).
 // EPI 3: squared ReLU. EPI 4: W rows in turns of 16 gate | 16 up, [M, N / 2].
 // Rows past M and N are read as zeros by the buffer descriptors' bounds, and so are
@@ -263,7 +265,8 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
                 for (int r = 0; r < 8; ++r) {
                     const float v = acc[a][b + (r >> 2)][r & 3];
                     f[r] = EPI == 1 ? glu_act(
-                        v, acc[a][b + (r >> 2) + B / 2][r & 3], p.glu)
+                        (float)(__bf16)v,
+                        (float)(__bf16)acc[a][b + (r >> 2) + B / 2][r & 3], p.glu)
                         : EPI == 3 ? fmaxf(v, 0.f) * fmaxf(v, 0.f) : v;
                 }
                 const bf16x8 v = to_bf16x8(f);

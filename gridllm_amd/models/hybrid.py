@@ -23,6 +23,7 @@ from __future__ import annotations
 import glob
 import os
 from dataclasses import dataclass
+from functools import partial
 from typing import Callable, Optional, Sequence
 
 import numpy as np
@@ -35,17 +36,23 @@ from gridllm_amd.models.registry import (AttentionMixer, DenseFF, GlaMixer,
                                          HybridSpec, LatentMixer,
                                          LightningMixer, ParallelMixer, PolyFF,
                                          Rotary, RoutedFF, TalkingMixer)
+from gridllm_amd.ops import autotune
 from gridllm_amd.ops import hybrid as hops
-from gridllm_amd.ops.autotune import linear as _linear
 from gridllm_amd.ops.autotune import linear_f32 as _linear_f32
-from gridllm_amd.ops.autotune import linear_gateup as _linear_gateup
-from gridllm_amd.ops.autotune import linear_parts as _linear_parts
 from gridllm_amd.ops.hybrid import (ChunkPortions, Choice, DepthAverage, Keys,
                                     StepMeta, Talk)
 from gridllm_amd.ops.reference import SWIGLU, Glu
 from gridllm_amd.parallel.tp import TPContext
 
 _DTYPES = {"bf16": torch.bfloat16, "fp32": torch.float32}
+
+# Recurrent and gated heads are normed whatever their size, so that at a sequence's
+# first token, which has one key, the sign of q . k is all that is left: a rounding
+# there is amplified to some percent of a short sequence. More than 256 rows'
+# products are therefore the library's to the bit, whatever runs them.
+_linear = partial(autotune.linear, whole=True)
+_linear_gateup = partial(autotune.linear_gateup, whole=True)
+_linear_parts = partial(autotune.linear_parts, whole=True)
 # portions of up to this many tokens run latent and talking-heads attention
 # token by token against the cached rows; for longer ones it pays to lay out
 # keys and values

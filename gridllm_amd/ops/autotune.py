@@ -125,7 +125,8 @@ def _fit(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple[int, int, int]]:
 
 
 @functools.lru_cache(maxsize=4096)
-def _rule(m: int, n: int, k: int, fuse: bool = False) -> tuple:
+def _rule(m: int, n: int, k: int, fuse: bool = False,
+          whole: bool = False) -> tuple:
     """The choice for sizes that were not timed. gemm_rows has no second kernel,
     but every block reads all of x, and takes all of K by itself: it is the faster
     one for w of up to 20 MB with up to 4 rows and up to 14 MB with 16 (against
@@ -134,7 +135,7 @@ def _rule(m: int, n: int, k: int, fuse: bool = False) -> tuple:
     21.7, 19.8), if K is 4096 or less (1024 x 6144, 16 rows 18.6 us, 10.3, the
     library 13.1; 1024 x 8192, 4 rows 15.5, 10.6, 13.6)."""
     if m > 256:
-        return hip_ops.gemm_plan(m, n, k, fuse) or ("blas",)
+        return hip_ops.gemm_plan(m, n, k, fuse, whole) or ("blas",)
     rows = hip_ops.gemm_rows_fits(m, n, k, fuse)
     if rows and k <= 4096 and n * k <= (10_000_000 if m <= 4 else 7_000_000):
         return ("rows",)
@@ -198,12 +199,14 @@ def tune_gateup(m: int, n: int, k: int, device) -> tuple:
     return _CHOICE_GU[key]
 
 
-def linear_gateup(x: torch.Tensor, w_il: torch.Tensor,
-                  glu: Glu = SWIGLU) -> torch.Tensor:
+def linear_gateup(x: torch.Tensor, w_il: torch.Tensor, glu: Glu = SWIGLU,
+                  whole: bool = False) -> torch.Tensor:
     """Fused gate/up projection + gated linear unit on an INTERLEAVED weight:
-    returns [M, F] activated, through the tuned table or by rule."""
+    returns [M, F] activated, through the tuned table or by rule. whole: as in
+    linear."""
     fit = _fit(x, w_il)
-    c = ("blas",) if fit is None else _CHOICE_GU.get(fit) or _rule(*fit, True)
+    c = ("blas",) if fit is None else _CHOICE_GU.get(fit) or \
+        _rule(*fit, True, whole)
     return _run(c, x, w_il, glu)
 
 
@@ -211,13 +214,15 @@ def choice(m: int, n: int, k: int) -> Optional[tuple[str, int]]:
     return _CHOICE.get((m, n, k))
 
 
-def _choose(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple]:
+def _choose(x: torch.Tensor, w: torch.Tensor, whole: bool = False
+            ) -> Optional[tuple]:
     """Choice for x @ w.T, None for what is not a GPU product of bf16 rows."""
     if not x.is_cuda or (torch.is_grad_enabled() and
                          (x.requires_grad or w.requires_grad)):
         return None
     fit = _fit(x, w)
-    return None if fit is None else _CHOICE.get(fit) or _rule(*fit)
+    return None if fit is None else _CHOICE.get(fit) or \
+        _rule(*fit, False, whole)
 
 
 def choice_of(m: int, w: torch.Tensor, fuse: bool = False) -> Optional[tuple]:
@@ -232,10 +237,12 @@ def choice_of(m: int, w: torch.Tensor, fuse: bool = False) -> Optional[tuple]:
     return c if c[0] in ("rows", "tile", "wide") else None
 
 
-def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+def linear(x: torch.Tensor, w: torch.Tensor, whole: bool = False
+           ) -> torch.Tensor:
     """Dispatch x @ w.T (GPU bf16 2-D x only) through the tuned table or by
-    rule."""
-    c = _choose(x, w)
+    rule. whole: more than 256 rows' products are the library's to the bit (see
+    gl_gemm_plan)."""
+    c = _choose(x, w, whole)
     return F.linear(x, w) if c is None else _run(c, x, w)
 
 
@@ -245,10 +252,11 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return F.linear(x, w).float() if c is None else _run_f32(c, x, w)
 
 
-def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+def linear_parts(x: torch.Tensor, w: torch.Tensor, whole: bool = False
+                 ) -> torch.Tensor:
     """linear(x, w), or its f32 partial sums [parts, M, N] if K is in parts, for
     post_norm, join_norm and rope_kv."""
-    c = _choose(x, w)
+    c = _choose(x, w, whole)
     if c is not None and c[0] == "tile" and c[3] > 1 and w.shape[1] > 64:
         return hip_ops.gemm_tile_parts(x, w, *c[1:])
     return F.linear(x, w) if c is None else _run(c, x, w)

@@ -75,7 +75,7 @@ def _load() -> ctypes.CDLL:
     lib.gl_gemm_tile.restype = c_i
     lib.gl_gemm_wide.argtypes = [c_vp] * 4 + [c_i] * 6 + [c_f] * 4
     lib.gl_gemm_wide.restype = c_i
-    lib.gl_gemm_plan.argtypes = [c_i] * 4 + [c_vp]
+    lib.gl_gemm_plan.argtypes = [c_i] * 5 + [c_vp]
     lib.gl_gemm_plan.restype = c_i
     lib.gl_attn_prefill.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_i, c_i,
                                     c_i, c_i, c_i, c_i, c_i, c_i, c_f]
@@ -647,15 +647,17 @@ def gemm_wide_tilings(m: int, n: int, k: int, fuse_swiglu: bool = False,
 
 
 @functools.lru_cache(maxsize=4096)
-def gemm_plan(m: int, n: int, k: int, fuse_swiglu: bool = False
-              ) -> Optional[tuple]:
+def gemm_plan(m: int, n: int, k: int, fuse_swiglu: bool = False,
+              whole: bool = False) -> Optional[tuple]:
     """("tile", rows, columns, parts) or ("wide", shape, whole tiles) for a
     product of more than 256 rows that was not timed, None if it is better left
-    to the library (see gl_gemm_plan)."""
+    to the library (see gl_gemm_plan). whole: one whose results are the library's
+    to the bit."""
     if not (0 < m < 1 << 24 and 0 < n < 1 << 24 and 0 < k < 1 << 20):
         return None
     plan = (ctypes.c_int * 4)()
-    _check(_load().gl_gemm_plan(m, n, k, fuse_swiglu, ctypes.addressof(plan)),
+    _check(_load().gl_gemm_plan(m, n, k, fuse_swiglu, whole,
+                                ctypes.addressof(plan)),
            "gemm_plan")
     if plan[0] == 1:
         return ("tile", *plan[1:4])

@@ -394,3 +394,15 @@ def test_rope_kv_refuses():
                  torch.zeros(128, dtype=bf16)[::2]):
         with pytest.raises(ValueError):
             call(rows, bias)
+
+
+def test_plans_of_whole_products():
+    """None is in parts of K, or by the kernel of which parts are."""
+    from gridllm_amd.ops import hip_ops
+    for m in (257, 300, 1200, 1201, 5000):
+        for n in (896, 3072, 16384):
+            for k in (896, 3072, 8192):
+                for fuse in (False, True):
+                    plan = hip_ops.gemm_plan(m, n, k, fuse, True)
+                    assert plan is None or plan[0] == "wide"
+                    assert plan is not None or not fuse
