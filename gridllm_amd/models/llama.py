@@ -524,31 +524,28 @@ class LlamaModel:
         for ln in lens:
             bounds.append(bounds[-1] + ln)
         tokens = torch.cat(token_lists)
-        # position/slot indices built host-side: TWO H2D copies instead of
-        # ~3k tiny device aranges per admission batch
-        pos_np = np.concatenate(
-            [np.arange(ln, dtype=np.int32) for ln in lens])
-        slot_np = np.concatenate(
-            [sl * self.cache.max_seq + np.arange(ln, dtype=np.int32)
-             for ln, sl in zip(lens, slots)])
-        idx = self.up.upload(np.stack([pos_np, slot_np]))
-        pos, slot_t = idx[0], idx[1]
-        # varlen batched attention (one meta-driven kernel launch per layer
-        # instead of a per-sequence Python loop of 36 ms per admission);
-        # meta rows: {q_off, len, slot, q0}
-        meta = None
+        # index arrays are built host-side, and go to the device in ONE copy
+        # (varlen batched attention: one meta-driven kernel launch per layer
+        # instead of a per-sequence Python loop of 36 ms per admission; meta rows:
+        # {q_off, len, slot, q0})
         trim = not return_hidden and min(lens) > 0 and \
             self._ends_suffice(bounds[-1], len(lens))
-        if trim:
-            ends = self.up.upload(np.asarray(
-                [[ln - 1 for ln in lens], lens, slots,
-                 [b - 1 for b in bounds[1:]]], dtype=np.int32))
-        if (tokens.is_cuda and self.dtype == torch.bfloat16
-                and s.head_dim in (64, 128)):
-            rows = [(bounds[i], ln, sl, q0)
-                    for i, (ln, sl) in enumerate(zip(lens, slots))
-                    for q0 in range(0, ln, 128)]
-            meta = self.up.upload(np.asarray(rows, dtype=np.int32))
+        batched = (tokens.is_cuda and self.dtype == torch.bfloat16
+                   and s.head_dim in (64, 128))
+        rows = [(bounds[i], ln, sl, q0)
+                for i, (ln, sl) in enumerate(zip(lens, slots))
+                for q0 in range(0, ln, 128)] if batched else []
+        ends = [lens, slots, [b - 1 for b in bounds[1:]], [ln - 1 for ln in lens]]
+        flat = self.up.upload(np.concatenate(
+            [np.asarray(rows, dtype=np.int32).reshape(-1)]
+            + [np.arange(ln, dtype=np.int32) for ln in lens]
+            + [sl * self.cache.max_seq + np.arange(ln, dtype=np.int32)
+               for ln, sl in zip(lens, slots)]
+            + [np.asarray(e, dtype=np.int32) for e in ends]))
+        at, total, n = 4 * len(rows), bounds[-1], len(lens)
+        meta = flat[:at].view(-1, 4) if batched else None
+        pos, slot_t = flat[at:at + total], flat[at + total:at + 2 * total]
+        len_t, of_slots, lasts, last_pos = flat[at + 2 * total:].view(4, n)
         resid, normed = ops.embed_norm(tokens, self.embed,
                                        self.layers[0].attn_norm, s.norm_eps)
         run = 0 if meta is None else self._layers_by_call(
@@ -558,8 +555,8 @@ class LlamaModel:
                 continue
             if trim and li + 1 == len(self.layers):
                 normed = self._last_layer(
-                    normed, pos, slot_t, normed[ends[3]], resid[ends[3]],
-                    ends[0], ends[1], ends[2])
+                    normed, pos, slot_t, normed[lasts], resid[lasts], last_pos,
+                    len_t, of_slots)
                 break
             q = ops.rope_kv(self._qkv(normed, lw), self.cache.k[li],
                             self.cache.v[li], self.cos, self.sin, pos, slot_t,
@@ -579,16 +576,10 @@ class LlamaModel:
             next_norm = (self.layers[li + 1].attn_norm
                          if li + 1 < len(self.layers) else self.final_norm)
             normed, resid = self._joined(act, lw.wdown, next_norm, resid)
-        # ONE scatter instead of k per-sequence device writes (each is a
-        # serialized H2D launch — 15 ms of host time per admission batch)
-        host = np.asarray([[sl for sl in slots], lens,
-                           [b - 1 for b in bounds[1:]]], dtype=np.int64)
-        dev3 = self.up.upload(host)
-        self.cache.seq_lens[dev3[0]] = dev3[1].to(torch.int32)
-        # fresh slots start unshifted (alloc no longer touches the device)
-        self.cache.rope_off.index_fill_(0, dev3[0], 0)
-        lasts = dev3[2]
-        logits = _linear_f32(normed if trim else normed[lasts], self.lm_head)
+        # (fresh slots start unshifted: alloc no longer touches the device)
+        x = ops.prompts_end(self.cache.seq_lens, self.cache.rope_off, of_slots,
+                            len_t, None if trim else normed, lasts)
+        logits = _linear_f32(normed if trim else x, self.lm_head)
         if return_hidden:
             hidden = torch.stack([
                 normed[bounds[i]:bounds[i + 1]].float().mean(dim=0)

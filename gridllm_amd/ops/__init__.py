@@ -77,6 +77,20 @@ def prompt_end(t: int, slot: int, start: int, seq_lens: torch.Tensor,
     reference.prompt_end(t, slot, start, seq_lens, rope_off)
 
 
+def prompts_end(seq_lens: torch.Tensor, rope_off: torch.Tensor,
+                slots: torch.Tensor, lens: torch.Tensor,
+                x: Optional[torch.Tensor], lasts: torch.Tensor
+                ) -> Optional[torch.Tensor]:
+    """End of a step of new sequences: lengths of their slots, whose rope_off is
+    0, and their last rows of x, if there is one. (int32 indices)"""
+    if _on_gpu(seq_lens) and (x is None or (
+            x.dtype == torch.bfloat16 and x.is_contiguous()
+            and x.shape[1] % 8 == 0 and x.data_ptr() % 16 == 0)):
+        from gridllm_amd.ops import hip_ops
+        return hip_ops.prompts_end(seq_lens, rope_off, slots, lens, x, lasts)
+    return reference.prompts_end(seq_lens, rope_off, slots, lens, x, lasts)
+
+
 def embed_norm(tokens: torch.Tensor, emb: torch.Tensor, weight: torch.Tensor,
                eps: float) -> Tuple[torch.Tensor, torch.Tensor]:
     """emb[tokens] and its rmsnorm. The fused kernel has token numbers on emb's

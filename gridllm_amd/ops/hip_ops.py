@@ -51,6 +51,9 @@ def _load() -> ctypes.CDLL:
     lib.gl_prompt_positions.restype = c_i
     lib.gl_prompt_end.argtypes = [c_vp] * 3 + [c_i] * 3
     lib.gl_prompt_end.restype = c_i
+    lib.gl_prompts_end.argtypes = [c_vp] * 5 + [c_i, c_i] + [c_vp] * 3 + [
+        c_i, c_i]
+    lib.gl_prompts_end.restype = c_i
     lib.gl_embed_norm.argtypes = [c_vp] * 6 + [c_l, c_i, c_i, c_f]
     lib.gl_embed_norm.restype = c_i
     lib.gl_rope.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i, c_i, c_i, c_i]
@@ -207,6 +210,30 @@ def prompt_end(t: int, slot: int, start: int, seq_lens: torch.Tensor,
         raise IndexError(f"slot {slot} of {seq_lens.shape[0]}")
     _check(_load().gl_prompt_end(_stream(), _ptr(seq_lens), _ptr(rope_off),
                                  slot, start, t), "prompt_end")
+
+
+def prompts_end(seq_lens: torch.Tensor, rope_off: torch.Tensor,
+                slots: torch.Tensor, lens: torch.Tensor,
+                x: Optional[torch.Tensor], lasts: torch.Tensor
+                ) -> Optional[torch.Tensor]:
+    """Sets the lengths of slots [B] int32 to lens, their rope_off to 0, and
+    returns x[lasts] (x [n, H] bf16), if there is an x."""
+    _check_ints("prompts_end", slots, seq_lens, rope_off)
+    _check_ints("prompts_end", slots, lens, lasts)
+    b = slots.shape[0]
+    if lens.shape != (b,) or (x is not None and not (
+            x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()
+            and x.device == slots.device and x.data_ptr() % 16 == 0)):
+        raise ValueError("prompts_end: lengths and rows [B], dense bf16 x")
+    _check_range("prompts_end.slots", slots, seq_lens.shape[0])
+    out = None if x is None else torch.empty(b, x.shape[1], dtype=x.dtype,
+                                             device=x.device)
+    _check(_load().gl_prompts_end(
+        _stream(), _ptr(seq_lens), _ptr(rope_off), _ptr(slots), _ptr(lens), b,
+        seq_lens.shape[0], _ptr(out), _ptr(x), _ptr(lasts),
+        0 if x is None else x.shape[0], 0 if x is None else x.shape[1]),
+        "prompts_end")
+    return out
 
 
 def decode_lengths(seq_lens: torch.Tensor,

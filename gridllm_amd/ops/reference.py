@@ -67,6 +67,16 @@ def prompt_end(t: int, slot: int, start: int, seq_lens: torch.Tensor,
         rope_off[slot] = 0
 
 
+def prompts_end(seq_lens: torch.Tensor, rope_off: torch.Tensor,
+                slots: torch.Tensor, lens: torch.Tensor,
+                x: Optional[torch.Tensor], lasts: torch.Tensor
+                ) -> Optional[torch.Tensor]:
+    """Sets the lengths of slots [B], their rope_off to 0; x[lasts]."""
+    seq_lens[slots.long()] = lens
+    rope_off.index_fill_(0, slots.long(), 0)
+    return None if x is None else x[lasts.long()]
+
+
 def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
                      rope_off: torch.Tensor, smax: int
                      ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:

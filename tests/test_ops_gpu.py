@@ -260,6 +260,30 @@ def test_rope_kv_fused_gpu(dev, n, hq, hk, d):
     assert _mx(vc.cpu(), vc_ref) < 1e-6
 
 
+@pytest.mark.parametrize("b,h", [(1, 8), (3, 896), (70, 3072)])
+def test_prompts_end_gpu(dev, b, h):
+    """Lengths, offsets and last rows, one of them counted from the end; lengths
+    alone."""
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator().manual_seed(b)
+    lens, off = (torch.randint(1, 99, (b + 2,), generator=g, dtype=torch.int32)
+                 for _ in range(2))
+    slots = torch.randperm(b + 2, generator=g)[:b].int()
+    new = torch.randint(0, 900, (b,), generator=g, dtype=torch.int32)
+    x = torch.randn(2 * b + 5, h, generator=g).bfloat16()
+    lasts = torch.randint(0, 2 * b + 5, (b,), generator=g, dtype=torch.int32)
+    lasts[0] = -1
+    args = [t.to(dev) for t in (lens, off, slots, new, x, lasts)]
+    got = hip_ops.prompts_end(*args)
+    want = R.prompts_end(lens, off, slots, new, x, lasts)
+    assert torch.equal(got.cpu(), want)
+    assert torch.equal(args[0].cpu(), lens) and torch.equal(args[1].cpu(), off)
+    args[1] += 3
+    assert hip_ops.prompts_end(*args[:3], args[3] + 1, None, args[5]) is None
+    assert torch.equal(args[0][args[2].long()], args[3] + 1)
+    assert not args[1][args[2].long()].any()
+
+
 @pytest.mark.parametrize("n,hq,hk,d,parts,bias", [
     (1, 3, 1, 16, 1, False), (45, 32, 8, 64, 4, True), (7, 24, 8, 128, 9, False)])
 def test_rope_kv_of_parts_gpu(dev, n, hq, hk, d, parts, bias):
