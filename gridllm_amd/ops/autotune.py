@@ -221,8 +221,8 @@ def _choose(x: torch.Tensor, w: torch.Tensor, whole: bool = False
                          (x.requires_grad or w.requires_grad)):
         return None
     fit = _fit(x, w)
-    return None if fit is None else _CHOICE.get(fit) or \
-        _rule(*fit, False, whole)
+    return None if fit is None else _CHOICE.get(fit) or (
+        _rule(*fit, False, True) if whole and fit[0] > 256 else _rule(*fit))
 
 
 def choice_of(m: int, w: torch.Tensor, fuse: bool = False) -> Optional[tuple]:
