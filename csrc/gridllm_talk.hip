@@ -136,6 +136,13 @@ DEV_INLINE int parts_of(int x, float c) {
 // smallest of some sizes that all rows' parts are `blocks` at most with, so that
 // all run at once; no row in parts if none is. N <= 256 rows; all lanes of a wave
 // find the same. Returns false for a block that is left over.
+// The longest part is what a launch takes as long as, 3 us a tile (8 value heads
+// of 128), whatever the other blocks do. So sizes lie close: among 16 from c0 to
+// 8 c0, 15 % apart, 160 rows of up to 1000 got 18 tiles, now 17: a step of 8
+// layers 1764 -> 1740 us; 200 rows of up to 1000 (26 tiles, 24) 1986 -> 1949, 150
+// of 600 1589 -> 1558. Shares that are all alike (12 tiles) would cut each row: a
+// cut's sums are 100 KB, written and read, and its queries another start: about
+// the 5 tiles that they spare.
 struct Part { int n, split, parts, block0; };
 DEV_INLINE bool find_part(int b, int blocks, const int* pos, int last, int N,
                           int chunk, Part* x) {
@@ -151,31 +158,45 @@ DEV_INLINE bool find_part(int b, int blocks, const int* pos, int last, int N,
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1)
         total += __shfl_xor(total, off, WAVE);
-    // sizes from all rows' share of a block on to 8 times that
-    const int c0 = max(2, (total + blocks - 1) / blocks);
-    auto size = [&](int k) {
-        return (float)(int)(c0 * fast_exp2(k * 0.2f) + 0.5f);
+    // the smallest of 8 sizes that asks for no more parts than blocks, by two a
+    // register; 8: none
+    auto first_of = [&](auto size) {
+        u32 sums[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            sums[k] = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                sums[k] += parts_of(len[i], (float)size(2 * k)) |
+                           parts_of(len[i], (float)size(2 * k + 1)) << 16;
+        }
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) sums[k] += __shfl_xor(sums[k], off, WAVE);
+        int best = 8;
+#pragma unroll
+        for (int k = 3; k >= 0; --k) {
+            if ((int)(sums[k] >> 16) <= blocks) best = 2 * k + 1;
+            if ((int)(sums[k] & 0xffff) <= blocks) best = 2 * k;
+        }
+        return best;
     };
-    u32 sums[8];                       // of two sizes each
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        sums[k] = 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            sums[k] += parts_of(len[i], size(2 * k)) |
-                       parts_of(len[i], size(2 * k + 1)) << 16;
+    // Sizes from all rows' share of a block on to 8 times that, then those up to
+    // the one that fits: the largest part is what the kernel takes as long as.
+    const int c0 = max(2, (total + blocks - 1) / blocks);
+    auto wide = [&](int k) {
+        return (int)(c0 * fast_exp2(k * (3.f / 7.f)) + 0.5f);
+    };
+    const int near = first_of(wide);
+    float c = 1e6f;
+    if (near == 0) {
+        c = c0;
+    } else if (near < 8) {
+        const int lo = wide(near - 1), gap = wide(near) - lo;
+        auto fine = [&](int k) { return lo + ((k + 1) * gap + 7) / 8; };
+        c = fine(first_of(fine));          // (the last one is wide(near))
     }
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1)
-#pragma unroll
-        for (int k = 0; k < 8; ++k) sums[k] += __shfl_xor(sums[k], off, WAVE);
-    int best = 16;
-#pragma unroll
-    for (int k = 7; k >= 0; --k) {
-        if ((int)(sums[k] >> 16) <= blocks) best = 2 * k + 1;
-        if ((int)(sums[k] & 0xffff) <= blocks) best = 2 * k;
-    }
-    const float c = best < 16 ? size(best) : 1e6f;
     int cnt[4], ahead = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) ahead += cnt[i] = parts_of(len[i], c);

@@ -367,6 +367,33 @@ def test_decode_in_parts(n, sizes, monkeypatch):
         0.05 + 0.01 * math.sqrt(heads)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,of", [(224, [700]), (224, [899] + [0] * 55),
+                                  (100, [880, 300]), (2, [5, 899]),
+                                  (150, list(range(100, 850, 5)))])
+def test_parts_by_lengths(n, of, monkeypatch):
+    """Sizes of parts that fit at once, far off, and in between: parts against
+    whole rows, which are the same products added up in another order."""
+    from gridllm_amd.ops import hip_hybrid
+    m = build(config((attn(16, 8, 128, 4096, 64, 1e4, 128 ** -0.5, 30.0), None)),
+              ("cuda", "bf16"), slots=1, max_seq=900)
+    c, tk = m.cache, m.layers[0].talk
+    c.extend([c.alloc(900)], [900])
+    g = torch.Generator().manual_seed(n)
+    c.v[0].copy_(torch.randn(c.v[0].shape, generator=g))
+    c.inv[0].copy_(torch.rand(c.inv[0].shape, generator=g) + 0.5)
+    st = hops.StepMeta(nd=n, pos=torch.tensor((of * n)[:n]).to(
+        "cuda", torch.int32), slot=torch.zeros(n, dtype=torch.int32,
+                                               device="cuda"),
+        table=c.table, max_len=900)
+    st.absorbed = n
+    q = torch.randn(n, 16, 128, generator=g).to("cuda", torch.bfloat16)
+    got = hops.talk_attn(q, c.v[0], c.inv[0], st, tk).float()
+    monkeypatch.setattr(hip_hybrid, "_talk_blocks", lambda *a: 0)
+    alone = hops.talk_attn(q, c.v[0], c.inv[0], st, tk).float()
+    assert bool(((got - alone).abs() <= 2 ** -7 * alone.abs() + 1e-4).all())
+
+
 # ----------------------------------------------- cuts, batches, pages, slots
 
 @pytest.mark.parametrize("run", RUNS)
