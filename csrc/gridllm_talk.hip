@@ -136,13 +136,12 @@ DEV_INLINE int parts_of(int x, float c) {
 // smallest of some sizes that all rows' parts are `blocks` at most with, so that
 // all run at once; no row in parts if none is. N <= 256 rows; all lanes of a wave
 // find the same. Returns false for a block that is left over.
-// The longest part is what a launch takes as long as, 3 us a tile (8 value heads
-// of 128), whatever the other blocks do. So sizes lie close: among 16 from c0 to
-// 8 c0, 15 % apart, 160 rows of up to 1000 got 18 tiles, now 17: a step of 8
-// layers 1764 -> 1740 us; 200 rows of up to 1000 (26 tiles, 24) 1986 -> 1949, 150
-// of 600 1589 -> 1558. Shares that are all alike (12 tiles) would cut each row: a
-// cut's sums are 100 KB, written and read, and its queries another start: about
-// the 5 tiles that they spare.
+// The longest part is what a launch takes as long as, whatever the other blocks
+// do. So sizes lie close: among 16 from c0 to 8 c0, 15 % apart, 160 rows of up to
+// 1000 got 18 tiles, now 17: a step of 8 layers 1764 -> 1740 us; 200 rows of up to
+// 1000 (26 tiles, 24) 1986 -> 1949, 150 of 600 1589 -> 1558. Shares that are all
+// alike (12 tiles) would cut each row: a cut's sums are 100 KB, written and read,
+// and its queries another start: about the 5 tiles that they spare.
 struct Part { int n, split, parts, block0; };
 DEV_INLINE bool find_part(int b, int blocks, const int* pos, int last, int N,
                           int chunk, Part* x) {
@@ -236,11 +235,12 @@ DEV_INLINE bool find_part(int b, int blocks, const int* pos, int last, int N,
 //   ws: sums [blocks][G][H][P], of each row the first block and the number of
 //   its parts, int [N][2] (at 8 bytes there), and the weights' sums [blocks][H]
 // Bound by the tiles' way to LDS: a block fits a CU once (24 heads, 8 values of
-// 128) and takes 3.4 us for a tile of 64 KB, 4.9 TB/s if all CUs have a block.
-// With a block per row, 160 rows of up to 1000 keys took 105 us, the longest
-// row's time, on 160 of 256 CUs; in parts they take 75 with the combining kernel,
-// and rows of 1000 keys all, which are left whole, 114 (112). (One behind the
-// other in a loop; among a step's other kernels 74 and 8.)
+// 128), and a tile is 64 KB. With a block per row, 160 rows of up to 1000 keys took
+// 105 us, the longest row's time, on 160 of 256 CUs; in parts 75 with the combining
+// kernel. All of that had the scores wait for the next tile: accesses to LDS that
+// do not say of what they are wait for every load into it (see load_lds16). With
+// plain vector types 160 rows among a step's other kernels take 61 us and 8 for 74
+// and 8 (200 rows of up to 1000, a step of 8 layers: 1949 -> 1830 us).
 // ===========================================================================
 template <int P, int GP, int HB, int R>
 struct DecodeShape {
@@ -365,7 +365,7 @@ k_talk_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
 
     for (int t = t0; t < t1; ++t) {
         const bf16_t* tile = smem + (t & 1) * Sh::TILE;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        WAIT_LOADS(0);
         lds_barrier();              // tile is there, the other one is free
         if (t + 1 < t1) issue(t + 1, page);
         page = tab[min(t + 2, t1 - 1) >> 1];
@@ -404,7 +404,7 @@ k_talk_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
         auto weigh = [&](f32x4 sc, int kb, int hk, float* sum) {
             float e[4], iv[4];
             const int key = t * 32 + kb * 16 + gq * 4;
-            ld4(ivs + (t & 1) * GP * 32 + kv * 32 + kb * 16 + gq * 4, iv);
+            lds_ld4(ivs + (t & 1) * GP * 32 + kv * 32 + kb * 16 + gq * 4, iv);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 e[r] = fast_exp2(capped(sc[r] * iv[r], cap,
@@ -413,8 +413,8 @@ k_talk_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
                 *sum += e[r];
             }
             if (hk < rep)
-                *(uint2*)(pb + (kv * rep + hk) * PLD + kb * 16 + gq * 4) =
-                    make_uint2(pack2(e[0], e[1]), pack2(e[2], e[3]));
+                lds_st2(pb + (kv * rep + hk) * PLD + kb * 16 + gq * 4,
+                        pack2(e[0], e[1]), pack2(e[2], e[3]));
         };
         if (mine == 2) {
             f32x4 a = score(0);

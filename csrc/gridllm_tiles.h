@@ -20,11 +20,19 @@ struct Rotation {
     int half, rows;
 };
 
+// 16 and 8 bytes of LDS by plain vector types (see load_lds16)
+DEV_INLINE void lds_ld4(const float* p, float* f) {
+    const f32x4 v = *(const f32x4*)p;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f[i] = v[i];
+}
+DEV_INLINE void lds_st2(bf16_t* p, u32 a, u32 b) { *(u32x2*)p = (u32x2){a, b}; }
+
 // Rotate the neighbouring pairs of 8 coordinates by 4 cosines and sines.
 DEV_INLINE void rotate_by(float* f, const float* cos_, const float* sin_) {
     float co[4], si[4];
-    ld4(cos_, co);
-    ld4(sin_, si);
+    lds_ld4(cos_, co);                     // (or of global memory)
+    lds_ld4(sin_, si);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const float u = f[2 * i], v = f[2 * i + 1];
@@ -70,15 +78,24 @@ DEV_INLINE float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 // 4 x 16 block of 16-bit elements in LDS, read transposed by 16 lanes: lane l
 // passes the address of row l / 4, columns 4 (l % 4) .. + 3, and gets column l,
 // rows 0 .. 3.
-DEV_INLINE bf16x4 read_transposed(const bf16_t* p) {
+DEV_INLINE bf16x4 read_transposed(const bf16_t* __restrict__ p) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)p);
 }
 
+// A load into LDS. The compiler has each later access to LDS wait for it, unless
+// that access says of what it is: plain vector types, not HIP's structs (float4,
+// uint2), and a __restrict__ pointer to a builtin. Kernels with a tile under way
+// while they work on another one wait by themselves (WAIT_LOADS).
 DEV_INLINE void load_lds16(const bf16_t* src, bf16_t* dst) {
     __builtin_amdgcn_global_load_lds(
         (const __attribute__((address_space(1))) unsigned int*)src,
         (__attribute__((address_space(3))) unsigned int*)dst, 16, 0, 0);
 }
+
+// Waits until no more than n loads or stores of the wave are under way.
+#define WAIT_LOADS(n) do { \
+        __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | 0xf70); \
+        asm volatile("" ::: "memory"); } while (0)
 
 // Barrier that orders LDS accesses alone: loads into LDS stay in flight.
 DEV_INLINE void lds_barrier() {

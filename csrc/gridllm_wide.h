@@ -39,11 +39,6 @@
 
 #include "gridllm_tiles.h"
 
-// Waits until no more than n loads or stores of the wave are under way.
-#define WAIT_LOADS(n) do { \
-        __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | 0xf70); \
-        asm volatile("" ::: "memory"); } while (0)
-
 #define WIDE_BYTES 0xe0000000L         // (so that offsets fit into 32 bits)
 
 struct WideArgs {
