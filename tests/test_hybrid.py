@@ -358,6 +358,28 @@ def test_wanted_rows_alone(run):
 
 
 @pytest.mark.parametrize("run", RUNS)
+@pytest.mark.parametrize("where", [("run", torch.int64), ("run", torch.int32),
+                                   ("run", None), ("cpu", torch.int64)])
+def test_prompts_tokens_from_anywhere(where, run):
+    """Several prompts' tokens of one type on the model's device (one copy), of
+    several types, and on the host: the same step, so the same results."""
+    m = build(FULL, run)
+    lists = [tokens(n, seed=n) for n in (40, 1, 70)]
+
+    def logits(tensors):
+        slots = [m.cache.alloc(0) for _ in tensors]
+        out = m.forward_prefill_batch(tensors, slots)
+        for slot in slots:
+            m.cache.free(slot)
+        return out
+    dev = run[0] if where[0] == "run" else "cpu"
+    kinds = [where[1] or kind for kind in (torch.int64, torch.int32, torch.int64)]
+    got = logits([torch.tensor(ids, dtype=kind, device=dev)
+                  for ids, kind in zip(lists, kinds)])
+    assert torch.equal(got, logits([torch.tensor(ids) for ids in lists]))
+
+
+@pytest.mark.parametrize("run", RUNS)
 def test_unequal_batch_against_each_alone(run):
     m = build(FULL, run)
     seqs = {s: tokens(n, seed=s) for s, n in ((1, 150), (2, 3), (3, 70),
