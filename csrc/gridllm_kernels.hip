@@ -1615,10 +1615,15 @@ int gl_gemm_wide(void* stream, void* out, const void* x, const void* w, int M,
 // library's to the bit. Where a model makes much of a rounding (a sequence's first
 // token has one key, and a head's norm behind it leaves the sign of q . k alone),
 // they then don't depend on what runs them.
-int gl_gemm_plan(int M, int N, int K, int fuse_glu, int whole, int* plan) {
+//   epi: as of gl_gemm_wide, which has not each shape for each. Scores in f32 (2) go
+// by the line of a plain product: the library's need another pass, so it is not a
+// worse one.
+int gl_gemm_plan(int M, int N, int K, int epi, int whole, int* plan) {
     plan[0] = plan[1] = plan[2] = plan[3] = 0;
+    if (epi < 0 || epi > 2) return -100;
+    const bool fuse_glu = epi == 1;
     int shape = 0, full = 0, way = 0;
-    float best = wide_best(M, N, K, fuse_glu ? 1 : 0, &shape, &full);
+    float best = wide_best(M, N, K, epi, &shape, &full);
     if (best < INFINITY) {
         way = 2;
         plan[1] = shape;

@@ -28,6 +28,8 @@ log = get_logger("autotune")
 # (m, n, k) -> ("blas",) | ("rows",) | ("ours", splitk) |
 # ("tile", rows, cols, splitk) | ("wide", shape, whole tiles)
 _CHOICE: dict[tuple[int, int, int], tuple] = {}
+# the same with f32 results (a vocabulary's scores), which not all shapes have
+_CHOICE_F32: dict[tuple[int, int, int], tuple] = {}
 # gate/up projection with fused SwiGLU (n = 2F interleaved rows):
 # (m, n, k) -> ("blas",) | ("rows",) | ("tile", rows, cols, splitk) |
 # ("wide", shape, whole tiles)
@@ -125,8 +127,8 @@ def _fit(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple[int, int, int]]:
 
 
 @functools.lru_cache(maxsize=4096)
-def _rule(m: int, n: int, k: int, fuse: bool = False,
-          whole: bool = False) -> tuple:
+def _rule(m: int, n: int, k: int, fuse: bool = False, whole: bool = False,
+          f32: bool = False) -> tuple:
     """The choice for sizes that were not timed. gemm_rows has no second kernel,
     but every block reads all of x, and takes all of K by itself: it is the faster
     one for w of up to 20 MB with up to 4 rows and up to 14 MB with 16 (against
@@ -135,7 +137,7 @@ def _rule(m: int, n: int, k: int, fuse: bool = False,
     21.7, 19.8), if K is 4096 or less (1024 x 6144, 16 rows 18.6 us, 10.3, the
     library 13.1; 1024 x 8192, 4 rows 15.5, 10.6, 13.6)."""
     if m > 256:
-        return hip_ops.gemm_plan(m, n, k, fuse, whole) or ("blas",)
+        return hip_ops.gemm_plan(m, n, k, fuse, whole, f32) or ("blas",)
     rows = hip_ops.gemm_rows_fits(m, n, k, fuse)
     if rows and k <= 4096 and n * k <= (10_000_000 if m <= 4 else 7_000_000):
         return ("rows",)
@@ -182,11 +184,11 @@ def _tune(x: torch.Tensor, n: int, glu: Optional[Glu] = None,
 
 
 def tune_shape(m: int, n: int, k: int, device, f32: bool = False) -> tuple:
-    key = (m, n, k)
-    if key not in _CHOICE:
+    key, table = (m, n, k), _CHOICE_F32 if f32 else _CHOICE
+    if key not in table:
         x = torch.randn(m, k, device=device).to(torch.bfloat16) * 0.1
-        _CHOICE[key] = _tune(x, n, f32=f32)
-    return _CHOICE[key]
+        table[key] = _tune(x, n, f32=f32)
+    return table[key]
 
 
 def tune_gateup(m: int, n: int, k: int, device) -> tuple:
@@ -214,14 +216,19 @@ def choice(m: int, n: int, k: int) -> Optional[tuple[str, int]]:
     return _CHOICE.get((m, n, k))
 
 
-def _choose(x: torch.Tensor, w: torch.Tensor, whole: bool = False
-            ) -> Optional[tuple]:
-    """Choice for x @ w.T, None for what is not a GPU product of bf16 rows."""
+def _choose(x: torch.Tensor, w: torch.Tensor, whole: bool = False,
+            f32: bool = False) -> Optional[tuple]:
+    """Choice for x @ w.T (f32: a result of that), None for what is not a GPU
+    product of bf16 rows."""
     if not x.is_cuda or (torch.is_grad_enabled() and
                          (x.requires_grad or w.requires_grad)):
         return None
     fit = _fit(x, w)
-    return None if fit is None else _CHOICE.get(fit) or (
+    if fit is None:
+        return None
+    if f32:
+        return _CHOICE_F32.get(fit) or _rule(*fit, f32=True)
+    return _CHOICE.get(fit) or (
         _rule(*fit, False, True) if whole and fit[0] > 256 else _rule(*fit))
 
 
@@ -248,7 +255,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, whole: bool = False
 
 def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """linear(x, w).float(): a vocabulary's scores."""
-    c = _choose(x, w)
+    c = _choose(x, w, f32=True)
     return F.linear(x, w).float() if c is None else _run_f32(c, x, w)
 
 
@@ -290,6 +297,7 @@ def tune_model_shapes(model, buckets) -> None:
                 tune_gateup(m, n, k, model.device)
             else:
                 tune_shape(m, n, k, model.device)
-    picked = sum(1 for v in _CHOICE.values() if v[0] != "blas")
-    log.performance("gemm autotune done", shapes=len(_CHOICE),
-                    ours=picked, ms=int((time.monotonic() - t0) * 1000))
+    picked = [*_CHOICE.values(), *_CHOICE_F32.values()]
+    log.performance("gemm autotune done", shapes=len(picked),
+                    ours=sum(1 for c in picked if c[0] != "blas"),
+                    ms=int((time.monotonic() - t0) * 1000))

@@ -675,16 +675,16 @@ def gemm_wide_tilings(m: int, n: int, k: int, fuse_swiglu: bool = False,
 
 @functools.lru_cache(maxsize=4096)
 def gemm_plan(m: int, n: int, k: int, fuse_swiglu: bool = False,
-              whole: bool = False) -> Optional[tuple]:
+              whole: bool = False, f32: bool = False) -> Optional[tuple]:
     """("tile", rows, columns, parts) or ("wide", shape, whole tiles) for a
     product of more than 256 rows that was not timed, None if it is better left
     to the library (see gl_gemm_plan). whole: one whose results are the library's
-    to the bit."""
+    to the bit. f32: for a result of that."""
     if not (0 < m < 1 << 24 and 0 < n < 1 << 24 and 0 < k < 1 << 20):
         return None
     plan = (ctypes.c_int * 4)()
-    _check(_load().gl_gemm_plan(m, n, k, fuse_swiglu, whole,
-                                ctypes.addressof(plan)),
+    _check(_load().gl_gemm_plan(m, n, k, 1 if fuse_swiglu else 2 if f32 else 0,
+                                whole, ctypes.addressof(plan)),
            "gemm_plan")
     if plan[0] == 1:
         return ("tile", *plan[1:4])

@@ -406,3 +406,44 @@ def test_plans_of_whole_products():
                     plan = hip_ops.gemm_plan(m, n, k, fuse, True)
                     assert plan is None or plan[0] == "wide"
                     assert plan is not None or not fuse
+
+
+def test_scores_of_many_rows_by_shapes_that_have_them(monkeypatch):
+    """A vocabulary's scores (f32) of more than 256 rows take no shape of tiles that
+    has bf16 results alone, nor does a product in bf16 take one of theirs; by rule,
+    and where the same sizes were timed as the other."""
+    from gridllm_amd.ops import autotune, hip_ops
+
+    class OnGpu(torch.Tensor):
+        is_cuda = True
+    ran = []
+
+    def wide(x, w, shape, whole, fuse_swiglu=False, glu=None, f32=False):
+        assert shape in ((0, 4) if f32 or fuse_swiglu else (0, 1, 2, 3))
+        ran.append(("wide", f32))
+
+    def others(c, x, w, glu=None):
+        ran.append(c[:1])
+        return wide(x, w, *c[1:]) if c[0] == "wide" else x
+    monkeypatch.setattr(hip_ops, "gemm_wide", wide)
+    monkeypatch.setattr(hip_ops, "gemm_tile_f32", lambda x, w, *c: ran.append("f32"))
+    monkeypatch.setattr(autotune, "_run", others)
+    for n, k in ((32000, 2048), (32064, 3072), (1024, 896), (128256, 2048)):
+        w = torch.empty(n, k, dtype=torch.bfloat16)
+        for m in (*range(257, 600, 9), 1201, 2000, 4096):
+            x = torch.empty(m, k, dtype=torch.bfloat16).as_subclass(OnGpu)
+            autotune.linear_f32(x, w)
+            autotune.linear(x, w)
+    assert ("wide", True) in ran and ("wide", False) in ran
+    m, n, k = 350, 32000, 2048
+    x = torch.empty(m, k, dtype=torch.bfloat16).as_subclass(OnGpu)
+    w = torch.empty(n, k, dtype=torch.bfloat16)
+    for f32, choice in ((True, ("wide", 4, 250)), (False, ("wide", 3, 500))):
+        monkeypatch.setattr(autotune, "_tune", lambda *a, **kw: choice)
+        assert autotune.tune_shape(m, n, k, "cpu", f32) == choice
+    try:
+        autotune.linear_f32(x, w)
+        autotune.linear(x, w)
+    finally:
+        for table in (autotune._CHOICE, autotune._CHOICE_F32):
+            table.pop((m, n, k), None)

@@ -957,6 +957,22 @@ def test_linear_of_many_rows(dev):
     assert took == {"blas", "tile", "wide"}
 
 
+@pytest.mark.parametrize("m,n,k", [(350, 32000, 2048), (2000, 1024, 896),
+                                   (257, 128256, 256), (300, 520, 64)])
+def test_scores_of_many_rows(dev, m, n, k):
+    """linear_f32 of more than 256 rows: by a kernel, and by the library."""
+    import torch.nn.functional as F
+    from gridllm_amd.ops import autotune
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(m, k, generator=g).to(dev, torch.bfloat16)
+    w = torch.randn(n, k, generator=g).to(dev, torch.bfloat16)
+    got, want = autotune.linear_f32(x, w), F.linear(x, w).float()
+    assert got.dtype == torch.float32 and got.shape == want.shape
+    # f32 sums in another order: some results round to bf16's neighbour
+    assert bool(((got - want).abs() <= 2 ** -7 * want.abs() +
+                 k * 2e-7 * k ** 0.5).all())
+
+
 def test_whole_products_are_the_librarys(dev):
     """Products of more than 256 rows that are not in parts of K give the library's
     results, and gated units those of the kernel behind it, to the bit."""
