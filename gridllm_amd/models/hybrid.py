@@ -48,11 +48,6 @@ from gridllm_amd.parallel.tp import TPContext
 
 _DTYPES = {"bf16": torch.bfloat16, "fp32": torch.float32}
 
-# Recurrent and gated heads are normed whatever their size, so that at a sequence's
-# first token, which has one key, the sign of q . k is all that is left: a rounding
-# there is amplified to some percent of a short sequence. More than 256 rows'
-# products are therefore the library's to the bit, whatever runs them.
-_WHOLE = True
 # portions of up to this many tokens run latent and talking-heads attention
 # token by token against the cached rows; for longer ones it pays to lay out
 # keys and values
@@ -616,19 +611,27 @@ class HybridModel:
 
     # -- layers ------------------------------------------------------------
 
-    def _joined(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    # Recurrent and gated heads are normed whatever their size, so that at a
+    # sequence's first token, which has one key, the sign of q . k is all that is
+    # left: a rounding there is amplified to some percent of a short sequence.
+    # Steps with prompts therefore keep the sums over K of more than 256 rows'
+    # products whole, as the library has them (st.whole); fewer rows' are in parts
+    # in every path, which few rows need (see hip_ops.gemm_tiling).
+
+    def _joined(self, x: torch.Tensor, w: torch.Tensor,
+                st: StepMeta) -> torch.Tensor:
         """A sublayer's last projection: its partial sums, where the norm behind
         it is a kernel that adds them up."""
         s = self.spec
         adds = s.pre_norms or (not s.streams and s.post_alpha is None)
-        return (_linear_parts if adds else _linear)(x, w, _WHOLE)
+        return (_linear_parts if adds else _linear)(x, w, st.whole)
 
     def _mix(self, i: int, w: BlockWeights, mx, xb: torch.Tensor,
              st: StepMeta, only: Optional[torch.Tensor] = None
              ) -> Optional[torch.Tensor]:
         """A mixer's output, or its rows `only` (None if there are none)."""
         c, eps = self.cache, self.spec.norm_eps
-        rows = _linear(xb, w.wmix, _WHOLE)
+        rows = _linear(xb, w.wmix, st.whole)
         if isinstance(mx, ParallelMixer):
             o = torch.empty(xb.shape[0], w.wo.shape[1], dtype=xb.dtype,
                             device=xb.device)
@@ -650,7 +653,7 @@ class HybridModel:
             cq = hops.latent_rows(rows, c.lat[i], st, self.rot[i], w.qnorm,
                                   w.kvnorm, mx.q_rank, mx.kv_rank, eps)
             at = w.qnorm.shape[0] + c.lat[i].shape[2]
-            o = hops.latent_attn(_linear(cq, w.wuq, _WHOLE), c.lat[i], st,
+            o = hops.latent_attn(_linear(cq, w.wuq, st.whole), c.lat[i], st,
                                  self.rot[i], w.wuk, w.wuv, w.wukv, mx.scale,
                                  rows[:, at:at + mx.heads])
         elif isinstance(mx, TalkingMixer):
@@ -669,7 +672,7 @@ class HybridModel:
             if not only.numel():
                 return None
             o = o[only]
-        return self._joined(o, w.wo)
+        return self._joined(o, w.wo, st)
 
     def _attend(self, i: int, w: BlockWeights, mx: AttentionMixer,
                 rows: torch.Tensor, st: StepMeta, out: torch.Tensor,
@@ -694,22 +697,23 @@ class HybridModel:
                         out[:, :h * p], scale)
         return end
 
-    def _gated(self, w: BlockWeights, ff: DenseFF,
-               xb: torch.Tensor) -> torch.Tensor:
+    def _gated(self, w: BlockWeights, ff: DenseFF, xb: torch.Tensor,
+               st: StepMeta) -> torch.Tensor:
         if self.gateup_il:
-            return _linear_gateup(xb, w.wgateup, _glu(ff), _WHOLE)
-        return hops.glu(_linear(xb, w.wgateup, _WHOLE), _glu(ff))
+            return _linear_gateup(xb, w.wgateup, _glu(ff), st.whole)
+        return hops.glu(_linear(xb, w.wgateup, st.whole), _glu(ff))
 
-    def _feed(self, w: BlockWeights, ff, xb: torch.Tensor):
+    def _feed(self, w: BlockWeights, ff, xb: torch.Tensor, st: StepMeta):
         """Feed-forward output, and, if it is still a row per (token, chosen
         expert), the pairs' weights and those of identity experts; with weighted
         inputs the rows just add up."""
         if isinstance(ff, DenseFF):
-            return self._joined(self._gated(w, ff, xb), w.down), None, None
+            return self._joined(self._gated(w, ff, xb, st), w.down,
+                                st), None, None
         if isinstance(ff, PolyFF):
-            z = hops.poly_norm(_linear(xb, w.up, _WHOLE), w.act, ff.ff,
+            z = hops.poly_norm(_linear(xb, w.up, st.whole), w.act, ff.ff,
                                self.spec.norm_eps)
-            return self._joined(z, w.down), None, None
+            return self._joined(z, w.down, st), None, None
         assert isinstance(ff, RoutedFF)
         return hops.moe(xb, hops.proj_f32(xb, w.router), w.up, w.down,
                         self._choice(w, ff))
@@ -769,7 +773,7 @@ class HybridModel:
                 hist, self.averages[i], i + 1, i + 1 < len(s.layers))
             join(y, w.norm1, avg if ly.ff is None else None)
             if ly.ff is not None:
-                y, pair_w, ident = self._feed(w, ly.ff, xb)
+                y, pair_w, ident = self._feed(w, ly.ff, xb, st)
                 join(y, w.norm2, avg, pair_w, ident)
             if trail is not None:
                 trail.append(x[:, :s.hidden].clone())
@@ -795,7 +799,7 @@ class HybridModel:
             h = hops.join_norm(x, y, w.norm1, ahead if ly.ff is None
                                else w.pre2, *how)
             if ly.ff is not None:
-                y = self._feed(w, ly.ff, h)[0]
+                y = self._feed(w, ly.ff, h, st)[0]
                 h = hops.join_norm(x, y, w.norm2, ahead, *how)
             if trail is not None:
                 trail.append(x[:, :s.hidden].clone())
@@ -822,18 +826,18 @@ class HybridModel:
             h = hops.streams_join(x, y, w.hc1, *(
                 ahead if ly.ff is None else (w.read2, w.norm2)), *size)
             if isinstance(ly.ff, RoutedFF):
-                y, extra = self._feed_pairs(w, ly.ff, h)
+                y, extra = self._feed_pairs(w, ly.ff, h, st)
                 h = hops.streams_join(x, y, w.hc2, *ahead, *size, ly.ff.top,
                                       extra)
             elif ly.ff is not None:
-                h = hops.streams_join(x, self._feed(w, ly.ff, h)[0], w.hc2,
-                                      *ahead, *size)
+                h = hops.streams_join(x, self._feed(w, ly.ff, h, st)[0],
+                                      w.hc2, *ahead, *size)
             if trail is not None:
                 trail.append(x[..., :s.hidden].sum(1))
         return x
 
-    def _feed_pairs(self, w: BlockWeights, ff: RoutedFF, h: torch.Tensor
-                    ) -> tuple[torch.Tensor, Optional[tuple]]:
+    def _feed_pairs(self, w: BlockWeights, ff: RoutedFF, h: torch.Tensor,
+                    st: StepMeta) -> tuple[torch.Tensor, Optional[tuple]]:
         """Experts' outputs by (token, chosen expert), which just add up; and
         the shared expert's with the logits of its gate."""
         z = hops.proj_f32(h, w.router)
@@ -841,8 +845,8 @@ class HybridModel:
                            self._choice(w, ff))
         if ff.shared is None:
             return y, None
-        return y, (_linear(self._gated(w, ff.shared, h), w.sdown, _WHOLE),
-                   z[:, ff.outputs:])
+        return y, (_linear(self._gated(w, ff.shared, h, st), w.sdown,
+                           st.whole), z[:, ff.outputs:])
 
     def _normed(self, x: torch.Tensor, rows: Optional[torch.Tensor],
                 w: torch.Tensor) -> torch.Tensor:
@@ -935,7 +939,8 @@ class HybridModel:
                       chunk_segs=dev[6].view(-1, 4) if mixed else None,
                       absorbed=absorbed, lat_rows=lrows,
                       lat_items=dev[7].view(-1, 4) if litems else None,
-                      lat_tiles=dev[8].view(-1, 8) if ltiles else None)
+                      lat_tiles=dev[8].view(-1, 8) if ltiles else None,
+                      whole=mixed or 0 in starts)
         for k, (c, t) in enumerate(zip(self.chunks, talks)):
             if t[0]:
                 items, t16, t128 = dev[9 + 3 * k:12 + 3 * k]

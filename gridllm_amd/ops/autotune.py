@@ -205,11 +205,20 @@ def linear_gateup(x: torch.Tensor, w_il: torch.Tensor, glu: Glu = SWIGLU,
                   whole: bool = False) -> torch.Tensor:
     """Fused gate/up projection + gated linear unit on an INTERLEAVED weight:
     returns [M, F] activated, through the tuned table or by rule. whole: as in
-    linear."""
+    linear, and the unit of more than 256 rows is that of the products rounded."""
     fit = _fit(x, w_il)
-    c = ("blas",) if fit is None else _CHOICE_GU.get(fit) or \
+    c = ("blas",) if fit is None else _timed(_CHOICE_GU, fit, whole) or \
         _rule(*fit, True, whole)
     return _run(c, x, w_il, glu)
+
+
+def _timed(table: dict, fit: tuple[int, int, int], whole: bool
+           ) -> Optional[tuple]:
+    """The choice that was timed for these sizes, if it is one for `whole`: decode
+    batches are timed, with K in parts too, and a prompt may have as many rows."""
+    c = table.get(fit)
+    return None if whole and c and fit[0] > 256 and c[0] not in (
+        "blas", "wide") else c
 
 
 def choice(m: int, n: int, k: int) -> Optional[tuple[str, int]]:
@@ -228,7 +237,7 @@ def _choose(x: torch.Tensor, w: torch.Tensor, whole: bool = False,
         return None
     if f32:
         return _CHOICE_F32.get(fit) or _rule(*fit, f32=True)
-    return _CHOICE.get(fit) or (
+    return _timed(_CHOICE, fit, whole) or (
         _rule(*fit, False, True) if whole and fit[0] > 256 else _rule(*fit))
 
 
@@ -247,7 +256,8 @@ def choice_of(m: int, w: torch.Tensor, fuse: bool = False) -> Optional[tuple]:
 def linear(x: torch.Tensor, w: torch.Tensor, whole: bool = False
            ) -> torch.Tensor:
     """Dispatch x @ w.T (GPU bf16 2-D x only) through the tuned table or by
-    rule. whole: more than 256 rows' products are the library's to the bit (see
+    rule. whole: more than 256 rows' products have their sums over K whole and in
+    order, as the library's are where it does not cut K itself (see
     gl_gemm_plan)."""
     c = _choose(x, w, whole)
     return F.linear(x, w) if c is None else _run(c, x, w)

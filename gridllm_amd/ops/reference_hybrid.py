@@ -53,6 +53,8 @@ class StepMeta:
                + 256 * rows to write} per page
     lat_tiles  [*, 8] {first token, length, first gathered row, first row,
                start} per 128 rows of a portion
+    whole      products of more than 256 rows keep their sums over K whole (of
+               steps with first tokens, or portions of prompts)
     """
     nd: int
     pos: torch.Tensor            # [n] int32
@@ -69,6 +71,7 @@ class StepMeta:
     lat_tiles: Optional[torch.Tensor] = None
     # by chunk size: the portions behind the absorbed tokens
     talk: dict[int, ChunkPortions] = field(default_factory=dict)
+    whole: bool = False
 
     def entries(self) -> list:
         """(first token, length, slot, start) of every entry, on the host."""

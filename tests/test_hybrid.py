@@ -890,3 +890,37 @@ def test_prompt_gates(kind):
     clear = ((mant % 1) - 0.5).abs() > 1.5e-6 * mant
     assert bool(clear.float().mean() > 0.99)
     assert torch.equal(got.cpu()[clear], want.to(torch.bfloat16)[clear])
+
+
+@pytest.mark.parametrize("name", ["tiny-birepel", "tiny-maferax", "tiny-vivepel",
+                                  "tiny-zinavik"])
+def test_prompts_products_are_whole(name, monkeypatch):
+    """All of a model's products know whether a step has prompts: portions, or
+    first tokens; decode batches take the choices that were timed for them."""
+    from gridllm_amd.models import hybrid
+    m = HybridModel(get_spec(name), dtype="fp32", kv_slots=3, max_seq=256)
+    seen = []
+
+    def spy(run):
+        def call(x, w, *rest):
+            seen.append(rest[-1])
+            return run(x, w, *rest)
+        return call
+    for f in ("_linear", "_linear_parts", "_linear_gateup"):
+        monkeypatch.setattr(hybrid, f, spy(getattr(hybrid, f)))
+
+    def flags():
+        got, seen[:] = set(seen), []
+        return got
+    a, b = m.cache.alloc(0), m.cache.alloc(0)
+    m.forward_prefill(torch.arange(20), a)
+    assert flags() == {True}
+    m.forward_step([(a, [3], [0]), (b, [5], [0])])      # b's first token
+    assert flags() == {True}
+    m.forward_step([(a, [3], [0]), (b, [5], [0])])
+    assert flags() == {False}
+    m.forward_step([(a, [3], [0]), (b, [5, 6], [0])])
+    assert flags() == {True}
+    m.cache.extend([a], [1])
+    m.forward_decode(torch.tensor([1]), torch.tensor([a], dtype=torch.int32))
+    assert flags() == {False}

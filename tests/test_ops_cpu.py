@@ -447,3 +447,32 @@ def test_scores_of_many_rows_by_shapes_that_have_them(monkeypatch):
     finally:
         for table in (autotune._CHOICE, autotune._CHOICE_F32):
             table.pop((m, n, k), None)
+
+
+def test_whole_products_of_sizes_that_were_timed(monkeypatch):
+    """More than 256 rows whose sums over K are to stay whole do not take a choice
+    with K in parts that a decode batch of as many rows was timed with."""
+    from gridllm_amd.ops import autotune, hip_ops
+
+    class OnGpu(torch.Tensor):
+        is_cuda = True
+    ran = []
+    monkeypatch.setattr(autotune, "_run", lambda c, x, *rest: ran.append(c))
+    monkeypatch.setattr(hip_ops, "gemm_tile_parts",
+                        lambda x, w, *c: ran.append(("tile", *c)))
+    n, k, cut = 3072, 8192, ("tile", 128, 128, 2)
+    w = torch.empty(n, k, dtype=torch.bfloat16)
+    for m, timed in ((512, cut), (512, ("ours", 2)), (512, ("blas",)),
+                     (512, ("wide", 1, 48)), (256, cut)):
+        x = torch.empty(m, k, dtype=torch.bfloat16).as_subclass(OnGpu)
+        monkeypatch.setitem(autotune._CHOICE, (m, n, k), timed)
+        monkeypatch.setitem(autotune._CHOICE_GU, (m, n, k), timed)
+        for run in (autotune.linear, autotune.linear_parts,
+                    lambda x, w, whole=False: autotune.linear_gateup(
+                        x, w, whole=whole)):
+            ran.clear()
+            run(x, w)
+            run(x, w, whole=True)
+            assert ran[0] == timed
+            assert ran[1] == timed if m == 256 or timed[0] in ("blas", "wide") \
+                else ran[1][0] in ("blas", "wide")
