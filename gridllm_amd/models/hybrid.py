@@ -119,6 +119,13 @@ def _pair_order(dim: int, rot_dims: int) -> torch.Tensor:
     return torch.cat([pairs, torch.arange(rot_dims, dim)])
 
 
+def _host_ids(tokens) -> Sequence[int]:
+    """Token ids on the host: a tensor's as an array (3500 as a list: 130 us more),
+    else what tolist() gives (numpy's and other arrays)."""
+    return tokens.long().cpu().numpy() if torch.is_tensor(tokens) else \
+        tokens.tolist()
+
+
 def _glu(ff: Optional[DenseFF]) -> Glu:
     return SWIGLU if ff is None else Glu(ff.alpha, ff.limit, ff.shift,
                                          ff.cubic)
@@ -1018,7 +1025,7 @@ class HybridModel:
         if start_pos != self.cache.lens[slot]:
             raise ValueError(f"slot {slot} holds {self.cache.lens[slot]} "
                              f"tokens, not {start_pos}")
-        ids = tokens.long().cpu().numpy()   # (a list: 130 us more for 3500)
+        ids = _host_ids(tokens)
         out = self.forward_step([(slot, ids, [len(ids) - 1])], return_hidden)
         return (out[0][0], out[1][0]) if return_hidden else out[0]
 
@@ -1027,14 +1034,14 @@ class HybridModel:
         """Several fresh sequences in one step; logits of each last token."""
         # (one copy from the device instead of one each, which waits every time: 24
         # prompts of 14 tokens, three layers of birepel:3b, 1257 -> 918 us)
-        n = [len(t) for t in token_lists]
-        if len(n) > 1 and all(t.is_cuda and t.dim() == 1 for t in token_lists) \
-                and len({(t.device, t.dtype) for t in token_lists}) == 1:
-            ids = torch.cat(list(token_lists)).long().cpu().numpy()
-            ends = accumulate(n)
-            lists = [ids[e - m:e] for e, m in zip(ends, n)]
+        lists = list(token_lists)
+        if len(lists) > 1 and all(torch.is_tensor(t) and t.is_cuda and t.dim() == 1
+                                  for t in lists) \
+                and len({(t.device, t.dtype) for t in lists}) == 1:
+            ids, n = _host_ids(torch.cat(lists)), [len(t) for t in lists]
+            lists = [ids[e - m:e] for e, m in zip(accumulate(n), n)]
         else:
-            lists = [t.long().cpu().numpy() for t in token_lists]
+            lists = [_host_ids(t) for t in lists]
         return self.forward_step(
             [(sl, ids, [len(ids) - 1]) for sl, ids in zip(slots, lists)],
             return_hidden)

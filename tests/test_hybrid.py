@@ -1,6 +1,7 @@
 """Layer-list models (Birepel) against the plain implementation in
 hybrid_oracle: on the CPU in f32, on the GPU in f32 and bf16."""
 
+import array
 import io
 import json
 import os
@@ -377,6 +378,21 @@ def test_prompts_tokens_from_anywhere(where, run):
     got = logits([torch.tensor(ids, dtype=kind, device=dev)
                   for ids, kind in zip(lists, kinds)])
     assert torch.equal(got, logits([torch.tensor(ids) for ids in lists]))
+    # arrays, beside tensors and alone, and an iterator over them
+    arrays = [np.array(lists[0], dtype=np.int32), torch.tensor(lists[1], device=dev),
+              array.array("q", lists[2])]
+    assert torch.equal(got, logits(arrays))
+    slots = [m.cache.alloc(0) for _ in lists]
+    assert torch.equal(got, m.forward_prefill_batch(
+        (np.array(ids) for ids in lists), slots))
+    for slot in slots:
+        m.cache.free(slot)
+    slot = m.cache.alloc(0)
+    alone = m.forward_prefill(np.array(lists[2]), slot)
+    m.cache.free(slot)
+    slot = m.cache.alloc(0)
+    assert torch.equal(alone, m.forward_prefill(torch.tensor(lists[2]), slot))
+    m.cache.free(slot)
 
 
 @pytest.mark.parametrize("run", RUNS)
