@@ -519,6 +519,10 @@ class LlamaModel:
         logits [k, vocab] f32; with return_hidden, (logits, mean-pooled
         final hidden [k, H] f32) — the embedding path."""
         s = self.spec
+        # (a slot that there is not is an IndexError here, ahead of the first layer,
+        # which would write its keys)
+        places = range(self.cache.seq_lens.shape[0])
+        slots = [places[sl] for sl in slots]
         lens = [int(t.shape[0]) for t in token_lists]
         bounds = [0]
         for ln in lens:

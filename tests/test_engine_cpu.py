@@ -633,3 +633,20 @@ def test_a_prompt_for_no_slot_writes_nothing(monkeypatch):
     for slot in (m.cache.seq_lens.shape[0], -1):
         with pytest.raises(IndexError):
             m.forward_prefill(torch.tensor([5, 6]), slot)
+
+
+def test_prompts_for_no_slot_write_nothing(monkeypatch):
+    """The same of several prompts; slots from the end are as for an index."""
+    from gridllm_amd import ops
+    from gridllm_amd.models.llama import LlamaModel
+    from gridllm_amd.models.registry import get_spec
+    m = LlamaModel(get_spec("tiny"), device="cpu", dtype="fp32", kv_slots=3,
+                   max_seq=64)
+    lists = [torch.tensor([5, 6]), torch.tensor([7])]
+    want = m.forward_prefill_batch(lists, [0, 2])
+    assert torch.equal(want, m.forward_prefill_batch(lists, [0, -1]))
+    assert m.cache.seq_lens.tolist() == [2, 0, 1]
+    monkeypatch.setattr(ops, "embed_norm", None)    # not reached
+    for slot in (3, -4):
+        with pytest.raises(IndexError):
+            m.forward_prefill_batch(lists, [0, slot])
