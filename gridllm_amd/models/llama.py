@@ -431,7 +431,8 @@ class LlamaModel:
                         w.data_ptr() & 15 or not w.is_contiguous():
                     return 0
             if not (lw.mlp_norm.is_contiguous() and lw.attn_norm.is_contiguous()
-                    and (lw.bqkv is None or lw.bqkv.is_contiguous())):
+                    and (lw.bqkv is None or (lw.bqkv.is_contiguous() and
+                                             not lw.bqkv.data_ptr() & 15))):
                 return 0
         # a layer's rows, one behind the other, from 16 bytes on each
         dev, parts = self.device, 0

@@ -122,6 +122,9 @@ def rope_kv(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
             bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     if _on_gpu(qkv):
         from gridllm_amd.ops import hip_ops
+        if bias is not None and (bias.data_ptr() & 15
+                                 or not bias.is_contiguous()):
+            bias = bias.clone(memory_format=torch.contiguous_format)
         return hip_ops.rope_kv(qkv, kcache, vcache, cos, sin, pos, slot,
                                hq, hk, d, bias)
     return reference.rope_kv(qkv, kcache, vcache, cos, sin, pos, slot,

@@ -396,6 +396,26 @@ def test_rope_kv_refuses():
             call(rows, bias)
 
 
+def test_rope_kv_takes_any_bias_of_its_size(monkeypatch):
+    """A bias that is a view at any place or stride reaches the kernel dense and
+    aligned."""
+    from gridllm_amd import ops
+    from gridllm_amd.ops import hip_ops
+    bf16, got = torch.bfloat16, []
+    monkeypatch.setattr(ops, "_on_gpu", lambda t: True)
+    monkeypatch.setattr(hip_ops, "rope_kv", lambda *a: got.append(a[-1]))
+    want = torch.arange(64).to(bf16)
+    flat, wide = torch.zeros(65, dtype=bf16), torch.zeros(64, 2, dtype=bf16)
+    flat[1:], wide[:, 0] = want, want
+    for bias in (want, flat[1:], wide[:, 0]):
+        ops.rope_kv(torch.zeros(2, 64, dtype=bf16), *(None,) * 6, 2, 1, 16, bias)
+        assert torch.equal(got[-1], want) and got[-1].is_contiguous()
+        assert got[-1].data_ptr() % 16 == 0
+    assert got[0] is want
+    ops.rope_kv(torch.zeros(2, 64, dtype=bf16), *(None,) * 6, 2, 1, 16)
+    assert got[-1] is None
+
+
 def test_plans_of_whole_products():
     """None is in parts of K, or by the kernel of which parts are."""
     from gridllm_amd.ops import hip_ops
