@@ -1611,10 +1611,11 @@ int gl_gemm_wide(void* stream, void* out, const void* x, const void* w, int M,
 //   K up to 4096 and 256 x 256 tiles that fill whole rounds and up to 0.6 of one,
 //   the library's worst sizes (0.93 over 40, 1.07 at most; 8000 x 5120 x 3072 284 ->
 //   196). Elsewhere it is 5 to 10 % faster than the kernel here.
-//   whole: not in parts of K, and gated units by k_gemm_wide, so that results are the
-// library's to the bit. Where a model makes much of a rounding (a sequence's first
-// token has one key, and a head's norm behind it leaves the sign of q . k alone),
-// they then don't depend on what runs them.
+//   whole: not in parts of K, and gated units by k_gemm_wide, whose sums and roundings
+// are the library's but where that cuts K itself (more than 99.9 % of results are the
+// same to the bit). Where a model makes much of a rounding (a sequence's first token
+// has one key, and a head's norm behind it leaves the sign of q . k alone), single
+// values then hardly depend on what runs them; against 64 bits both are alike.
 //   epi: as of gl_gemm_wide, which has not each shape for each. Scores in f32 (2) go
 // by the line of a plain product: the library's need another pass, so it is not a
 // worse one.

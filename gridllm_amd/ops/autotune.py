@@ -35,7 +35,7 @@ _CHOICE_F32: dict[tuple[int, int, int], tuple] = {}
 # ("wide", shape, whole tiles)
 _CHOICE_GU: dict[tuple[int, int, int], tuple] = {}
 _BF16, _transformed = torch.bfloat16, torch._C._are_functorch_transforms_active
-_most_rows = 1 << 24            # of a choice by rule or timing
+_most_rows = 1 << 24            # of a choice by rule; more ones' are timed alone
 _ITERS = 24                     # calls of a timing, at most
 _SPLITK_CANDIDATES = (0, 2, 4, 6, 8, 12, 16, 24, 32)
 

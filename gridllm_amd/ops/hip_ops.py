@@ -574,7 +574,8 @@ def _tile_us(m: int, n: int, k: int, rows: int, cols: int, tiles: int,
     """What a tiling takes of gemm_tile's time, in us, beside 6 that all have: a
     CU's loads of its share of K, one block after the other, and with K in parts
     the second kernel, which reads the partial sums. (Fitted to 18000 timings of 65
-    to 256 rows, 7 % off in the mean.)"""
+    to 256 rows, 7 % off in the mean. gl_gemm_plan has the same for more rows; a test
+    holds the two together.)"""
     kslice = -(-(-(-k // parts)) // 64) * 64
     parts = -(-k // kslice)
     us = -(-tiles * parts // 256) * kslice * (rows + cols - 37) * 3.9e-5
@@ -678,8 +679,8 @@ def gemm_plan(m: int, n: int, k: int, fuse_swiglu: bool = False,
               whole: bool = False, f32: bool = False) -> Optional[tuple]:
     """("tile", rows, columns, parts) or ("wide", shape, whole tiles) for a
     product of more than 256 rows that was not timed, None if it is better left
-    to the library (see gl_gemm_plan). whole: one whose results are the library's
-    to the bit. f32: for a result of that."""
+    to the library (see gl_gemm_plan). whole: K in one part, in order, and a gated
+    unit on rounded products. f32: for a result of that."""
     if not (0 < m < 1 << 24 and 0 < n < 1 << 24 and 0 < k < 1 << 20):
         return None
     plan = (ctypes.c_int * 4)()
@@ -811,8 +812,8 @@ def _sample(logits, keys, temps, slots=None, seeds=None, draws=None,
                          "length, dense and on one GPU")
     if slots is not None:
         _check_range("sample_gumbel.slots", slots, n[0])
-    # four blocks a CU, of 2048 elements or more: 64 rows of 128256 take 21 us
-    # in 16 segments, 190 in one (with exact logarithms)
+    # four blocks a CU, of 2048 elements or more: 64 rows of 128256 take 16.5 us
+    # in 16 segments (190 in one, with exact logarithms)
     segments = max(1, min(1024 // max(1, b), v // 2048, 64))
     out = torch.empty(b, dtype=torch.int32, device=logits.device)
     ws = torch.empty(b * segments, dtype=i64, device=logits.device)

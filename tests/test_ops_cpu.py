@@ -496,3 +496,33 @@ def test_whole_products_of_sizes_that_were_timed(monkeypatch):
             assert ran[0] == timed
             assert ran[1] == timed if m == 256 or timed[0] in ("blas", "wide") \
                 else ran[1][0] in ("blas", "wide")
+
+
+def test_plans_times_are_the_tilings():
+    """What gl_gemm_plan says of a tiling's time is what _tile_us says: of the
+    tilings that it looks at, the one it names takes the least by both."""
+    from gridllm_amd.ops import hip_ops
+    seen = 0
+    for m in (257, 300, 384, 512, 700, 1000, 1200):
+        for n in (64, 896, 1024, 1152, 2048, 3072):
+            for k in (4096, 4864, 6144, 8192, 12288):
+                plan = hip_ops.gemm_plan(m, n, k)
+                if plan is None or plan[0] != "tile":
+                    continue
+
+                def us(rows, cols, parts):
+                    return hip_ops._tile_us(m, n, k, rows, cols,
+                                            -(-m // rows) * (n // cols), parts)
+                least = float("inf")
+                for rows in (96, 128, 160, 192, 256):
+                    for cols in (64, 96, 128):
+                        tiles = -(-m // rows) * (n // cols)
+                        if n % cols or tiles > 512:
+                            continue
+                        most = max(1, min(256 // tiles, k // 384))
+                        for parts in (1, (most + 1) // 2, most):
+                            least = min(least, us(rows, cols, parts))
+                # (the plan's sums are of 24 bits)
+                assert abs(us(*plan[1:]) - least) < 1e-5 * least, (m, n, k)
+                seen += 1
+    assert seen > 50
