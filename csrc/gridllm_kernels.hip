@@ -1607,7 +1607,9 @@ int gl_gemm_wide(void* stream, void* out, const void* x, const void* w, int M,
 //   here does (four layers of 0.5b, 260 tokens, are bound by that).
 //   192 x 192 and 192 x 128 tiles, which it seems not to have, where they nearly
 //   fill one or two rounds of CUs (0.93 over 17, 1.0 at most; 2731 x 3072 x 3072 56.7
-//   -> 48.4).
+//   -> 48.4). With more rounds its larger tiles fill theirs well enough: three and four
+//   full ones of 192 x 192 take 1.01 to 1.16 of its time (4608 x 6144 x 3072 152 us,
+//   150; 6144 x 4608 x 2048 108, 95; 6144 x 6144 x 4096 246, 226).
 //   K up to 4096 and 256 x 256 tiles that fill whole rounds and up to 0.6 of one,
 //   the library's worst sizes (0.93 over 40, 1.07 at most; 8000 x 5120 x 3072 284 ->
 //   196). Elsewhere it is 5 to 10 % faster than the kernel here.
@@ -1617,14 +1619,15 @@ int gl_gemm_wide(void* stream, void* out, const void* x, const void* w, int M,
 // has one key, and a head's norm behind it leaves the sign of q . k alone), single
 // values then hardly depend on what runs them; against 64 bits both are alike.
 //   epi: as of gl_gemm_wide, which has not each shape for each. Scores in f32 (2) go
-// by the line of a plain product: the library's need another pass, so it is not a
-// worse one.
+// as a plain product does if its shape has them (0), else by the library and a pass
+// to f32: by shape 4 350 x 32000 x 2048 takes 58 us, 62 by the library, but 300 x
+// 32064 x 3072 81, 79, and 513 x 32000 x 4096 178, 156.
 int gl_gemm_plan(int M, int N, int K, int epi, int whole, int* plan) {
     plan[0] = plan[1] = plan[2] = plan[3] = 0;
     if (epi < 0 || epi > 2) return -100;
     const bool fuse_glu = epi == 1;
     int shape = 0, full = 0, way = 0;
-    float best = wide_best(M, N, K, epi, &shape, &full);
+    float best = wide_best(M, N, K, fuse_glu ? 1 : 0, &shape, &full);
     if (best < INFINITY) {
         way = 2;
         plan[1] = shape;
@@ -1664,6 +1667,7 @@ int gl_gemm_plan(int M, int N, int K, int epi, int whole, int* plan) {
             here |= K <= 4096 && tiles > 256 && some > 0 && some <= 154;
         else if (plan[1] != 2)
             here |= tiles <= 512 && (some == 0 || some >= 218);
+        if (epi == 2 && plan[1] != 0) here = false;
     }
     plan[0] = here ? way : 0;
     return 0;

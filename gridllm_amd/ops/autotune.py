@@ -237,8 +237,9 @@ def _choose(x: torch.Tensor, w: torch.Tensor, whole: bool = False,
         return None
     if f32:
         return _CHOICE_F32.get(fit) or _rule(*fit, f32=True)
-    return _timed(_CHOICE, fit, whole) or (
-        _rule(*fit, False, True) if whole and fit[0] > 256 else _rule(*fit))
+    if whole and fit[0] > 256:
+        return _timed(_CHOICE, fit, True) or _rule(*fit, False, True)
+    return _CHOICE.get(fit) or _rule(*fit)
 
 
 def choice_of(m: int, w: torch.Tensor, fuse: bool = False) -> Optional[tuple]:

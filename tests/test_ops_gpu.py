@@ -957,12 +957,15 @@ def test_linear_of_many_rows(dev):
     assert took == {"blas", "tile", "wide"}
 
 
-@pytest.mark.parametrize("m,n,k", [(350, 32000, 2048), (2000, 1024, 896),
-                                   (257, 128256, 256), (300, 520, 64)])
-def test_scores_of_many_rows(dev, m, n, k):
-    """linear_f32 of more than 256 rows: by a kernel, and by the library."""
+@pytest.mark.parametrize("m,n,k,way", [
+    (350, 32000, 2048, "blas"), (2000, 1024, 896, "blas"),
+    (700, 32064, 896, "wide"), (260, 512, 128, "tile"), (300, 520, 64, "blas")])
+def test_scores_of_many_rows(dev, m, n, k, way):
+    """linear_f32 of more than 256 rows: by the kernels that have such results, and
+    by the library where a product in bf16 goes by a shape that has none."""
     import torch.nn.functional as F
     from gridllm_amd.ops import autotune
+    assert autotune._rule(m, n, k, f32=True)[0] == way
     g = torch.Generator().manual_seed(5)
     x = torch.randn(m, k, generator=g).to(dev, torch.bfloat16)
     w = torch.randn(n, k, generator=g).to(dev, torch.bfloat16)
