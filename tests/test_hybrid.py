@@ -940,3 +940,36 @@ def test_prompts_products_are_whole(name, monkeypatch):
     m.cache.extend([a], [1])
     m.forward_decode(torch.tensor([1]), torch.tensor([a], dtype=torch.int32))
     assert flags() == {False}
+
+
+@pytest.mark.gpu
+def test_decode_of_many_rows_against_halves():
+    """More than 256 decode rows, whose products may have their K in parts, against
+    the same rows in two steps; sizes at which the rule cuts K."""
+    from dataclasses import replace
+    from gridllm_amd.ops import autotune
+    spec = get_spec("birepel:3b")
+    own = next(ly.ff for ly in spec.layers if not hasattr(ly.ff, "experts"))
+    spec = replace(spec, vocab=1024, layers=tuple(
+        replace(ly, ff=own) for ly in spec.layers[:2]))
+    n = 300
+    c = autotune._rule(n, spec.hidden, own.ff)
+    assert c[0] == "tile" and c[3] > 1
+    out = []
+    for sizes in ((n,), (n // 2, n // 2)):
+        m = HybridModel(spec, device="cuda:0", dtype="bf16", seed=5, kv_slots=n,
+                        max_seq=64)
+        slots = [m.cache.alloc(8) for _ in range(n)]
+        g = torch.Generator().manual_seed(1)
+        m.forward_prefill_batch(list(torch.randint(0, 1024, (n, 7), generator=g)),
+                                slots)
+        at, parts = 0, []
+        for size in sizes:
+            some = slots[at:at + size]
+            m.cache.prepare_decode(some)
+            parts.append(m.forward_decode(
+                torch.arange(at, at + size).cuda(),
+                torch.tensor(some, dtype=torch.int32).cuda()))
+            at += size
+        out.append(torch.cat(parts).cpu())
+    close(out[0], out[1], ("cuda:0", "bf16"))
