@@ -234,6 +234,10 @@ k_attn_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
         const int k0 = first_key(st);
         return kv.off(bc, hk, k0 & ~63) + (k0 & 63) * D;
     };
+    // K and V past the Infinity Cache (see load_lds16_once): with weights that go past
+    // it and K that does not, K's part of it is slower than memory (256 rows of up to
+    // 384 keys 56 us, 51; 64 of up to 2000 in pages 87, 63). A row's four loads follow
+    // each other, so that both halves of a line come at once.
     auto load_k = [&](int st, long at) {
         const int last = seq - 1 - first_key(st);
         const bf16_t* p = kv.k + at + kg;
@@ -242,7 +246,8 @@ k_attn_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
             const bf16_t* r = p + min(t * 16 + fr, last) * D;
 #pragma unroll
             for (int s = 0; s < ND; ++s)
-                kf[t][s] = *(const bf16x8*)(r + s * 32);
+                kf[t][s] = __builtin_nontemporal_load(
+                    (const bf16x8*)(r + s * 32));
         }
     };
     typedef __attribute__((ext_vector_type(4))) u32 u32x4;

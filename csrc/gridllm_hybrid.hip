@@ -2350,7 +2350,8 @@ DEV_INLINE bool moe_work(const int4* tiles, int max_tiles, int ntn, int4& tl,
 // that the lane-linear image reads back without bank conflicts), NB buffers.
 // With few rows per expert the same pipeline streams the weights, in tiles of 32
 // rows with 3 buffers: 48 rows in all, 64 experts, 160 -> 155 us; 12 rows gated 199 ->
-// 168 (a CU's loads queue up, and of 128 rows as many are x's as W's).
+// 168 (a CU's loads queue up, and of 128 rows as many are x's as W's). Weights go past
+// the Infinity Cache (see load_lds16_once): 48 rows over and over, 805 MB, 150 -> 131.
 // ACT != 0 (up projection): row r of the tile is token sorted[row0 + r] / top,
 // output in sorted order through squared ReLU (1) or, with weight rows in turns
 // of 16 gate | 16 up, the gated unit `glu` in N / 2 columns (2); pw (nullable):
@@ -2394,11 +2395,9 @@ k_moe_gemm(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
 #pragma unroll
         for (int i = 0; i < GL; ++i) {
             const int piece = i < A ? wid * A + i : 4 * A + wid * 4 + i - A;
-            __builtin_amdgcn_global_load_lds(
-                (const __attribute__((address_space(1))) unsigned int*)
-                    (src[i] + (long)kt * BK * 2),
-                (__attribute__((address_space(3))) unsigned int*)
-                    (lds + buf * TB + piece * 512), 16, 0, 0);
+            const bf16_t* from = (const bf16_t*)(src[i] + (long)kt * BK * 2);
+            if (i < A) load_lds16(from, lds + buf * TB + piece * 512);
+            else load_lds16_once(from, lds + buf * TB + piece * 512);
         }
     };
     f32x4 acc[A][4];

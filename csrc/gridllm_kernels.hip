@@ -710,11 +710,18 @@ k_gemm_rows(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
 // Where W's rows are a multiple of 4096 bytes long, what all blocks read at a time,
 // a piece of 128 bytes at the same place of each row, is in few of the memory's
 // channels (800 MB in rows of 16384 bytes 4.0 TB/s, of 6144 5.7). Blocks of
-// neighbouring columns then start one tile of K further on and wrap (6.05): 45 rows
-// of 128256 x 2048 134.7 -> 121.2 us, of 16384 x 2048 gated 20.1 -> 18.3. Parts of K
+// neighbouring columns then start some tiles of K further on and wrap (6.05): 45 rows
+// of 128256 x 2048 134.7 -> 121.2 us, of 16384 x 2048 gated 20.1 -> 18.3. One tile, and
+// ten for odd multiples of 2048 (in order: one row of 16384 x 2048 gated 14.0, 12.4, of
+// 16384 x 6144 34.4, 33.5, of 11008 x 4096 18.1, 18.7; 45 rows of 128256 x 4096 187,
+// 190). Parts of K
 // are at different places anyway (24 rows of 3072 x 8192 in 5 parts 16.2 either way,
 // 64 of 3072 x 12288 24.2, 23.1), and other rows are read as fast in order (24 rows
 // of 5120 x 3072 12.8 us, 13.1; 16384 x 3072 22.8, 23.0).
+//
+// W goes past the Infinity Cache (see load_lds16_once; us, 2 GB of weights in turn, parts
+// of K without what adds them up): 5120 x 3072, one row 7.5 -> 7.0, 64 rows 9.7 -> 9.5;
+// 16384 x 3072 gated 20.7 -> 18.6, 22.8 -> 21.4; 128256 x 3072 141 -> 132, 166 -> 162.
 //
 // Bound by a CU's loads: those of x, which hit in L2, and of W queue up behind
 // one another (12288 x 3072, 160 rows: x alone 9 us, W alone 13, both 27, with
@@ -765,7 +772,8 @@ k_gemm_tile(bf16_t* __restrict__ out, float* __restrict__ ws,
         const int c = (n0 >> 1) + r % (BN / 2);
         return (c >> 6) * 128 + (c & 63) + (r >= BN / 2 ? 64 : 0);
     };
-    const int turn = K % 2048 || splitk > 1 ? 0 : item / rblocks % cols % nt;
+    const int turn = K % 2048 || splitk > 1
+        ? 0 : item / rblocks % cols * (K % 4096 ? 10 : 1) % nt;
     int left = nt - turn;                      // tiles up to the end of K's part
     const bf16_t* src[G];
 #pragma unroll
@@ -779,7 +787,9 @@ k_gemm_tile(bf16_t* __restrict__ out, float* __restrict__ ws,
     auto issue = [&](int buf) {                // the next tile
 #pragma unroll
         for (int i = 0; i < G; ++i) {
-            load_lds16(src[i], lds + buf * BUF + (i * 4 + wid) * 512);
+            bf16_t* dst = lds + buf * BUF + (i * 4 + wid) * 512;
+            if ((i * 4 + wid) * 8 < R) load_lds16(src[i], dst);
+            else load_lds16_once(src[i], dst);
             src[i] += 64;
         }
         if (--left == 0)

@@ -92,6 +92,17 @@ DEV_INLINE void load_lds16(const bf16_t* src, bf16_t* dst) {
         (__attribute__((address_space(3))) unsigned int*)dst, 16, 0, 0);
 }
 
+// The same of what a pass reads once and there is much of (weights, caches): past the
+// Infinity Cache. Read through it, more than its 256 MB push each other out, the other
+// kernels' data with them, and a next pass finds nothing there; past it, it keeps what
+// it has (us, all read in turn: 1600 MB 322, 284; 2400 MB 466, 425; what it would hold
+// is 5 % slower: 200 MB 38.8, 40.8). Whole lines of 128 bytes are to be taken.
+DEV_INLINE void load_lds16_once(const bf16_t* src, bf16_t* dst) {
+    __builtin_amdgcn_global_load_lds(
+        (const __attribute__((address_space(1))) unsigned int*)src,
+        (__attribute__((address_space(3))) unsigned int*)dst, 16, 0, 2);
+}
+
 // Waits until no more than n loads or stores of the wave are under way.
 #define WAIT_LOADS(n) do { \
         __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | 0xf70); \

@@ -29,7 +29,10 @@
 // the results rounded to bf16, as a library product and the unit behind it have it.
 // Sums go over all of K in order, as the library's do but for those of its tiles
 // whose K it cuts, so that more than 99.9 % of results are the same to the bit.
-// EPI 2: the result, rounded to bf16, as f32 (a vocabulary's scores).
+// EPI 2: the result, rounded to bf16, as f32 (a vocabulary's scores); W, which such a
+// product's few rows read once, past the Infinity Cache (see load_lds16_once; 256 rows of
+// 128256 x 3072 in a step 207 -> 201 us, and the step's other kernels find theirs
+// there: 4 layers 880 -> 861).
 // EPI 3: squared ReLU. EPI 4: W rows in turns of 16 gate | 16 up, [M, N / 2].
 // Rows past M and N are read as zeros by the buffer descriptors' bounds, and so are
 // the stages past the last tile: a wave's offset is the end of the matrix at most,
@@ -137,14 +140,16 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
         }
     };
     auto issue = [&](int buf, int i) {
-        const bool of_x = i * 64 < R;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            of_x ? xr : wrs,
-            (__attribute__((address_space(3))) unsigned int*)(
-                lds + buf * BUF + (i * 8 + wid) * 512),
-            16, of_x ? vx[i % GX]
-                : !Rows::GATHER && B % 2 && tile_of(i) == B - 1 ? vx[0] : vw,
-            so[i], 0, 0);
+        const auto dst = (__attribute__((address_space(3))) unsigned int*)(
+            lds + buf * BUF + (i * 8 + wid) * 512);
+        const int v = !Rows::GATHER && B % 2 && tile_of(i) == B - 1 ? vx[0] : vw;
+        if (i * 64 < R)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, dst, 16, vx[i % GX],
+                                                     so[i], 0, 0);
+        else if (EPI == 2)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, dst, 16, v, so[i], 0, 2);
+        else
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, dst, 16, v, so[i], 0, 0);
         if (i + 1 == G) {
 #pragma unroll
             for (int k = 0; k < GX; ++k) vx[k] += 128;

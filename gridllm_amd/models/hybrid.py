@@ -592,6 +592,13 @@ class HybridModel:
                 plain |= {tuple(w.up.shape), tuple(w.down.shape)}
         return sorted(plain), sorted(gu)
 
+    def joined_shapes(self) -> set:
+        """Those of the projections whose parts of K the next kernel adds up."""
+        if not self._parts_added():
+            return set()
+        return {tuple(t.shape) for w in self.unique_layers()
+                for t in (w.wo, w.down) if t is not None and t.dim() == 2}
+
     def interleave_gateup(self) -> None:
         """Gate and up rows in groups of 64 | 64, the layout of the fused
         gate/up projection (as LlamaModel.interleave_gateup)."""
@@ -629,9 +636,11 @@ class HybridModel:
                 st: StepMeta) -> torch.Tensor:
         """A sublayer's last projection: its partial sums, where the norm behind
         it is a kernel that adds them up."""
+        return (_linear_parts if self._parts_added() else _linear)(x, w, st.whole)
+
+    def _parts_added(self) -> bool:
         s = self.spec
-        adds = s.pre_norms or (not s.streams and s.post_alpha is None)
-        return (_linear_parts if adds else _linear)(x, w, st.whole)
+        return s.pre_norms or (not s.streams and s.post_alpha is None)
 
     def _mix(self, i: int, w: BlockWeights, mx, xb: torch.Tensor,
              st: StepMeta, only: Optional[torch.Tensor] = None

@@ -202,6 +202,12 @@ class LlamaModel:
                  (s.vocab, s.hidden)],                           # lm_head
                 [(2 * self.f_l, s.hidden)])
 
+    def joined_shapes(self) -> set:
+        """Those of the projections whose parts of K the next kernel adds up."""
+        plain = self.gemm_shapes()[0]
+        return set() if self.tp.size > 1 else set(
+            plain[self.spec.head_dim % 16 > 0:3])
+
     def interleave_gateup(self) -> None:
         """Reorder each wgateup's rows into 128-row groups [64 gate |
         64 up] so that a block of a fused-SwiGLU product (gemm_tile,

@@ -285,6 +285,32 @@ def test_tuner_skips_what_cannot_run(monkeypatch):
     assert autotune._fit(big, w) == (300, 512, 256)
 
 
+def test_products_joined_by_the_next_kernel(monkeypatch):
+    """The tuner times those with the norm behind them: each is one of the plain
+    products, and not the vocabulary's; the others are timed alone."""
+    from types import SimpleNamespace
+    from gridllm_amd.models import model_class
+    from gridllm_amd.models.registry import get_spec
+    from gridllm_amd.ops import autotune
+    for name, some in (("tiny", True), ("tiny-birepel", True),
+                       ("tiny-vivepel", True), ("tiny-maferax", False)):
+        spec = get_spec(name)
+        model = model_class(spec)(spec, device="cpu", dtype="fp32", kv_slots=2,
+                                  max_seq=64)
+        plain, joined = model.gemm_shapes()[0], model.joined_shapes()
+        assert joined <= set(plain) and bool(joined) == some
+        timed = {}
+        monkeypatch.setattr(autotune, "tune_shape", lambda m, n, k, dev, f32, j:
+                            timed.update({(n, k): (f32, j)}))
+        model.gateup_il = False
+        autotune.tune_model_shapes(SimpleNamespace(
+            spec=spec, device="cpu", gemm_shapes=lambda: (plain, []),
+            joined_shapes=lambda: joined), [4])
+        assert {s for s, (_, j) in timed.items() if j} == {
+            s for s in joined if s[0] != spec.vocab}
+        assert not any(f32 and j for f32, j in timed.values())
+
+
 def test_scripts_call_what_there_is():
     """Every function that a script takes from the kernel layer is there."""
     import ast
