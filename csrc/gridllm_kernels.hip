@@ -11,8 +11,8 @@
 //    matmul-shaped kernels (prefill attention, projection GEMMs).
 //  * memory-bound ops target the HBM3E roofline (~6.3 TB/s achievable);
 //    decode projections are bound by streaming W, or a CU's loads of x and W:
-//    k_gemm_rows loads straight into MFMA operands, k_gemm_tile moves both
-//    through a ring of tiles in LDS.
+//    k_gemm_rows loads straight into MFMA operands, k_gemm_tile and k_gemm_fed
+//    move both through rings in LDS.
 //  * attention decode: 4-wave workgroup per (batch, kv_head, split), K and V
 //    streamed through registers; split-S partials where B*Hk is small.
 //  * exported as extern "C" with an explicit hipStream_t so launches are
@@ -22,6 +22,7 @@
 // Build: hipcc --offload-arch=gfx950 -O3 -shared -fPIC
 
 #include "gridllm_attention.h"
+#include "gridllm_batch.h"
 #include "gridllm_wide.h"
 
 // ===========================================================================
@@ -687,233 +688,6 @@ k_gemm_rows(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
     }
 }
 
-// ===========================================================================
-// Batch GEMM: out[M,N] = x[M,K] @ W[N,K]^T (bf16 I/O, f32 sums), for more rows
-// than k_gemm_rows takes.
-//
-// Block: 4 waves, RT * 16 rows by CT * 16 columns of one of `splitk` parts of K;
-// a wave has half of the rows by half of the columns, so that it reads each
-// operand piece from LDS for several products. Tiles of 64 k of x and W go into
-// a ring of NB buffers by loads into LDS (16-byte pieces XOR-swizzled by the row
-// through their addresses), NB - 1 ahead. In the middle of a tile the waves meet:
-// the next one is there, and this one's buffer is free, its second half being in
-// registers; so the products of one half run while the other half is read.
-// Blocks of the same K part and neighbouring columns share an XCD, hence x's
-// lines in its L2; those of other rows and the same columns follow each other.
-//   EPI 1: W rows in groups of 64 gate | 64 up; a block takes CT * 8 of each and
-//   stores the gated unit [M, N / 2].
-//   splitk > 1: f32 partials [splitk][M][N] in ws. out == null otherwise: the
-//   result, rounded to bf16, as f32 in ws (a vocabulary's scores: 256 rows of
-//   128256 took 30 us to be widened behind it).
-// Constraints: N % (16 CT) == 0 (128 for EPI 1), K % 64 == 0, kslice % 64 == 0.
-//
-// Where W's rows are a multiple of 4096 bytes long, what all blocks read at a time,
-// a piece of 128 bytes at the same place of each row, is in few of the memory's
-// channels (800 MB in rows of 16384 bytes 4.0 TB/s, of 6144 5.7). Blocks of
-// neighbouring columns then start some tiles of K further on and wrap (6.05): 45 rows
-// of 128256 x 2048 134.7 -> 121.2 us, of 16384 x 2048 gated 20.1 -> 18.3. One tile, and
-// ten for odd multiples of 2048 (in order: one row of 16384 x 2048 gated 14.0, 12.4, of
-// 16384 x 6144 34.4, 33.5, of 11008 x 4096 18.1, 18.7; 45 rows of 128256 x 4096 187,
-// 190). Parts of K
-// are at different places anyway (24 rows of 3072 x 8192 in 5 parts 16.2 either way,
-// 64 of 3072 x 12288 24.2, 23.1), and other rows are read as fast in order (24 rows
-// of 5120 x 3072 12.8 us, 13.1; 16384 x 3072 22.8, 23.0).
-//
-// W goes past the Infinity Cache (see load_lds16_once; us, 2 GB of weights in turn, parts
-// of K without what adds them up): 5120 x 3072, one row 7.5 -> 7.0, 64 rows 9.7 -> 9.5;
-// 16384 x 3072 gated 20.7 -> 18.6, 22.8 -> 21.4; 128256 x 3072 141 -> 132, 166 -> 162.
-//
-// Bound by a CU's loads: those of x, which hit in L2, and of W queue up behind
-// one another (12288 x 3072, 160 rows: x alone 9 us, W alone 13, both 27, with
-// rings of any depth), so the tile is as large as the accumulators allow and all
-// of the chip has one. Against the kernel before it (rows in steps of 128, x and
-// W read from LDS once per wave and product row, a stop between tiles) and the
-// one for up to 64 rows (W straight to registers), at their best split:
-//   rows        64            160           256
-//   4096x3072   16.6 -> 12.1  18.8 -> 16.1  20.3 -> 18.8 us
-//   3072x8192   23.3 -> 15.5  26.5 -> 22.1  28.8 -> 26.9
-//   12288x3072  33.8 -> 20.6  35.7 -> 30.5  37.3 -> 33.1
-//   3072x12288  34.3 -> 21.2  35.4 -> 29.1  37.6 -> 35.3
-// ===========================================================================
-template <int RT, int CT>
-struct GemmTile {
-    static constexpr int R = RT * 16, BN = CT * 16;
-    static constexpr int BYTES = (R + BN) * 128;       // of 64 k
-    static constexpr int FIT = 160 * 1024 / BYTES;
-    static constexpr int NB = FIT > 8 ? 8 : FIT;
-};
-
-template <int RT, int CT, int EPI>
-__global__ void __launch_bounds__(256, 2)
-k_gemm_tile(bf16_t* __restrict__ out, float* __restrict__ ws,
-            const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
-            int M, int N, int K, int splitk, int kslice, int rblocks,
-            const GluParams glu) {
-    typedef GemmTile<RT, CT> Sh;
-    constexpr int R = Sh::R, BN = Sh::BN, NB = Sh::NB, BUF = (R + BN) * 64;
-    constexpr int G = (R + BN) / 32;           // loads of a wave and tile
-    constexpr int A = RT / 2, B = CT / 2;      // a wave's 16 x 16 tiles
-    static_assert(RT % 2 == 0 && CT % (EPI ? 4 : 2) == 0, "halves");
-    static_assert(NB >= 3 && G * (NB - 1) < 64, "loads that can be counted");
-    extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
-    const int lane = threadIdx.x & 63;
-    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int fr = lane & 15, gq = lane >> 4, wr = wid >> 1, wc = wid & 1;
-    const int cols = N / BN, total = cols * splitk * rblocks;
-    const int each = (total + 7) >> 3;         // blocks of an XCD
-    const int item = (int)(blockIdx.x & 7) * each + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= each || item >= total) return;
-    const int m0 = item % rblocks * R, n0 = item / rblocks % cols * BN;
-    const int ks = item / rblocks / cols, k0 = ks * kslice;
-    const int nt = (min(K, k0 + kslice) - k0) >> 6;
-
-    auto w_row = [&](int r) {                  // of W, for row r of the tile
-        if (EPI == 0) return n0 + r;
-        const int c = (n0 >> 1) + r % (BN / 2);
-        return (c >> 6) * 128 + (c & 63) + (r >= BN / 2 ? 64 : 0);
-    };
-    const int turn = K % 2048 || splitk > 1
-        ? 0 : item / rblocks % cols * (K % 4096 ? 10 : 1) % nt;
-    int left = nt - turn;                      // tiles up to the end of K's part
-    const bf16_t* src[G];
-#pragma unroll
-    for (int i = 0; i < G; ++i) {
-        const int row = (i * 4 + wid) * 8 + (lane >> 3);
-        const int at = ((lane & 7) ^ (row & 7)) * 8 + k0 + turn * 64;
-        src[i] = (i * 4 + wid) * 8 < R
-                     ? x + (long)min(m0 + row, M - 1) * K + at
-                     : w + (long)w_row(row - R) * K + at;
-    }
-    auto issue = [&](int buf) {                // the next tile
-#pragma unroll
-        for (int i = 0; i < G; ++i) {
-            bf16_t* dst = lds + buf * BUF + (i * 4 + wid) * 512;
-            if ((i * 4 + wid) * 8 < R) load_lds16(src[i], dst);
-            else load_lds16_once(src[i], dst);
-            src[i] += 64;
-        }
-        if (--left == 0)
-#pragma unroll
-            for (int i = 0; i < G; ++i) src[i] -= nt * 64;
-    };
-    // a wave's columns; with gates, the second half of its tiles are the ups
-    auto col_tile = [&](int b) {
-        return !EPI ? wc * B + b
-                    : b % (B / 2) + wc * (B / 2) + (b < B / 2 ? 0 : CT / 2);
-    };
-    f32x4 acc[A][B];
-#pragma unroll
-    for (int a = 0; a < A; ++a)
-#pragma unroll
-        for (int b = 0; b < B; ++b) acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    bf16x8 xf[2][A], wf[2][B];
-    auto read = [&](int buf, int c) {          // half c of a tile
-        const bf16_t* t = lds + buf * BUF + ((c * 4 + gq) ^ (fr & 7)) * 8;
-#pragma unroll
-        for (int b = 0; b < B; ++b)
-            wf[c][b] =
-                *(const bf16x8*)(t + (R + col_tile(b) * 16 + fr) * 64);
-#pragma unroll
-        for (int a = 0; a < A; ++a)
-            xf[c][a] = *(const bf16x8*)(t + ((wr * A + a) * 16 + fr) * 64);
-    };
-    // W's rows are the products' rows, so that a lane has 4 columns of a row
-    auto multiply = [&](int c) {
-#pragma unroll
-        for (int a = 0; a < A; ++a)
-#pragma unroll
-            for (int b = 0; b < B; ++b)
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    wf[c][b], xf[c][a], acc[a][b], 0, 0, 0);
-    };
-    auto spread = [] {                         // reads between the products
-        constexpr int EACH = A * B / (A + B) > 0 ? A * B / (A + B) : 1;
-#pragma unroll
-        for (int i = 0; i < A + B; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, EACH, 0);
-        }
-    };
-
-#pragma unroll
-    for (int u = 0; u < NB; ++u)
-        if (u < nt) issue(u);
-    if (nt < NB) {                             // all of K is under way
-        WAIT_LOADS(0);
-        lds_barrier();
-        for (int kt = 0; kt < nt; ++kt) {
-            read(kt, 0);
-            read(kt, 1);
-            multiply(0);
-            multiply(1);
-        }
-    } else {
-        WAIT_LOADS(G * (NB - 1));
-        lds_barrier();
-        read(0, 0);
-        int buf = 0;
-        for (int kt = NB; kt < nt; ++kt) {
-            const int next = buf + 1 == NB ? 0 : buf + 1;
-            read(buf, 1);
-            multiply(0);
-            spread();
-            WAIT_LOADS(G * (NB - 2));
-            lds_barrier();
-            issue(buf);
-            read(next, 0);
-            multiply(1);
-            spread();
-            buf = next;
-        }
-        auto last = [&](auto behind, auto&& rest) {    // tiles behind this one
-            constexpr int L = behind.value;
-            const int next = buf + 1 == NB ? 0 : buf + 1;
-            read(buf, 1);
-            multiply(0);
-            spread();
-            if constexpr (L > 0) {
-                WAIT_LOADS(G * (L - 1));
-                lds_barrier();
-                read(next, 0);
-            }
-            multiply(1);
-            buf = next;
-            if constexpr (L > 0)
-                rest(std::integral_constant<int, L - 1>(), rest);
-        };
-        last(std::integral_constant<int, NB - 1>(), last);
-    }
-
-    // lane holds columns gq * 4 + r, row fr of a 16 x 16 tile
-#pragma unroll
-    for (int a = 0; a < A; ++a) {
-        const int m = m0 + (wr * A + a) * 16 + fr;
-        if (m >= M) continue;
-        if (EPI && splitk == 1) {
-#pragma unroll
-            for (int b = 0; b < B / 2; ++b) {
-                float f[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    f[r] = glu_act(acc[a][b][r], acc[a][b + B / 2][r], glu);
-                st4(out + (long)m * (N >> 1) + (n0 >> 1) +
-                        (wc * (B / 2) + b) * 16 + gq * 4, f);
-            }
-            continue;
-        }
-#pragma unroll
-        for (int b = 0; b < B; ++b) {
-            const int n = w_row(col_tile(b) * 16) + gq * 4;
-            float f[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                f[r] = splitk == 1 ? bf2f(f2bf(acc[a][b][r])) : acc[a][b][r];
-            if (splitk == 1 && out) st4(out + (long)m * N + n, f);
-            else st4(ws + ((long)ks * M + m) * N + n, f);
-        }
-    }
-}
-
 // A kernel with more LDS than the default limit asks for it, once.
 template <auto Kernel>
 static int allow_lds(int bytes) {
@@ -924,19 +698,17 @@ static int allow_lds(int bytes) {
 }
 
 template <int RT, int CT, int EPI>
-static int launch_gemm_tile(hipStream_t st, bf16_t* out, float* ws,
-                            const bf16_t* x, const bf16_t* w, int M, int N,
-                            int K, int splitk, int kslice,
-                            const GluParams glu) {
-    typedef GemmTile<RT, CT> Sh;
-    constexpr int bytes = Sh::NB * Sh::BYTES;
-    const int e = allow_lds<k_gemm_tile<RT, CT, EPI>>(bytes);
+static int launch_gemm_tile(hipStream_t st, BatchArgs p) {
+    typedef std::conditional_t<RT <= 4, GemmTile<RT, CT>, GemmFed<RT, CT>> Sh;
+    constexpr auto kernel = [] {
+        if constexpr (RT <= 4) return k_gemm_tile<RT, CT, EPI>;
+        else return k_gemm_fed<RT, CT, EPI>;
+    }();
+    const int e = allow_lds<kernel>(Sh::BYTES);
     if (e) return e;
-    const int rblocks = (M + Sh::R - 1) / Sh::R;
-    const long total = (long)(N / Sh::BN) * splitk * rblocks;
-    k_gemm_tile<RT, CT, EPI><<<(unsigned)((total + 7) / 8 * 8), 256, bytes,
-                               st>>>(out, ws, x, w, M, N, K, splitk, kslice,
-                                     rblocks, glu);
+    p.rblocks = (p.M + Sh::R - 1) / Sh::R;
+    const long total = (long)(p.N / Sh::C) * p.splitk * p.rblocks;
+    kernel<<<(unsigned)((total + 7) / 8 * 8), Sh::THREADS, Sh::BYTES, st>>>(p);
     LAUNCH_CHECK();
     return 0;
 }
@@ -1551,14 +1323,16 @@ int gl_gemm_tile(void* stream, void* out, void* ws, const void* x,
         cols < 1 || N % cols || (fuse_swiglu && N % 128) || splitk < 1 ||
         (long)(splitk - 1) * kslice >= K || (long)splitk * kslice < K ||
         (splitk > 1 && !ws) || (!out && (!ws || fuse_swiglu))) return -100;
+    const BatchArgs p{(bf16_t*)out, (float*)ws, (const bf16_t*)x,
+                      (const bf16_t*)w, M, N, K, splitk, kslice, 0, glu};
     hipStream_t st = (hipStream_t)stream;
     int e = -103;
 #define GO(RT, CT, EPI) \
     if (rows == RT * 16 && cols == CT * 16 && !fuse_swiglu == !EPI) \
-        e = launch_gemm_tile<RT, CT, EPI>(st, (bf16_t*)out, (float*)ws, \
-            (const bf16_t*)x, (const bf16_t*)w, M, N, K, splitk, kslice, glu)
+        e = launch_gemm_tile<RT, CT, EPI>(st, p)
 #define COLS(RT) GO(RT, 4, 0); GO(RT, 6, 0); GO(RT, 8, 0); GO(RT, 4, 1); \
     GO(RT, 8, 1)
+    GO(6, 3, 0); GO(8, 3, 0); GO(10, 3, 0); GO(12, 3, 0); GO(16, 3, 0);
     COLS(2); COLS(4); COLS(6); COLS(8); COLS(10); COLS(12); COLS(16);
 #undef COLS
 #undef GO
@@ -1607,12 +1381,16 @@ int gl_gemm_wide(void* stream, void* out, const void* x, const void* w, int M,
 // What to run a product of more than 256 rows by: plan[0] 0 the library, 1
 // gl_gemm_tile by rows plan[1], columns plan[2], parts plan[3], 2 gl_gemm_wide by
 // shape plan[1] and full plan[2]. The times are those of wide_best and of _tile_us
-// in hip_ops.py, which holds up to 1200 rows too (0.2 % off in the mean, 10 %
-// standard deviation, 600 timings).
-//   Gated units are always done here: the library's needs another pass (0.82 of
-//   its time over 100 sizes, 1.09 at most; 2731 x 16384 x 3072 338 -> 220 us).
-//   K from 4096 on with up to 1200 rows: tiles with K in parts (0.82, 0.98 at most;
-//   300 x 2048 x 8192 36.7 -> 25.9).
+// in hip_ops.py, which holds up to 1200 rows too (over 130 sizes what is picked here
+// takes 1.017 of the best choice's time in the mean, 1.13 at most, and .88 of the
+// library's).
+//   Gated units are always done here: the library's needs another pass (16384 x 3072,
+//   272 rows 48 -> 38 us by tiles; 2731 338 -> 220).
+//   K from 4096 on with up to 1200 rows: tiles with K in parts (300 x 2048 x 8192 34 ->
+//   25, 512 x 3072 x 12288 74 -> 47, 1200 x 3072 x 8192 75 -> 65). Shorter K: tiles
+//   where they are one round of CUs, three quarters of it or more (300 x 12288 x 3072
+//   43 -> 33, 800 x 3072 x 3072 30 -> 26, 1024 x 5120 x 3072 42 -> 40; two rounds, 640
+//   x 12288 x 3072, take 63 us, the library 54; 160 tiles, 1200 x 4096 x 3072, 45, 40).
 //   20 us and less: what a call to the library costs the host, and twice what one
 //   here does (four layers of 0.5b, 260 tokens, are bound by that).
 //   192 x 192 and 192 x 128 tiles, which it seems not to have, where they nearly
@@ -1637,6 +1415,7 @@ int gl_gemm_plan(int M, int N, int K, int epi, int whole, int* plan) {
     if (epi < 0 || epi > 2) return -100;
     const bool fuse_glu = epi == 1;
     int shape = 0, full = 0, way = 0;
+    bool fills = false;                        // blocks of tiles: one round of CUs
     float best = wide_best(M, N, K, fuse_glu ? 1 : 0, &shape, &full);
     if (best < INFINITY) {
         way = 2;
@@ -1655,19 +1434,23 @@ int gl_gemm_plan(int M, int N, int K, int epi, int whole, int* plan) {
             for (int parts : {1, (most + 1) / 2, most}) {
                 const int slice = ((K + parts - 1) / parts + 63) / 64 * 64;
                 const int n = (K + slice - 1) / slice;
-                float us = 6.f + (tiles * n + 255) / 256 * slice *
-                    (float)(rows + cols - 37) * 3.9e-5f;
-                if (n > 1) us += 1.2f + (float)n * M * N * 2.5e-6f;
+                const float area = (float)rows * cols;
+                float us = 3.9f + (tiles * n + 255) / 256 *
+                    (3.f + slice * (rows * 1.42e-5f + cols * 3.2e-5f +
+                                    area * 1.09e-7f) +
+                     (fuse_glu ? area * 5.8e-5f : 0.f));
+                if (n > 1) us += (float)n * M * N * 2.4e-6f;
                 if (us >= best) continue;
                 best = us;
                 way = 1;
+                fills = tiles * n >= 192 && tiles * n <= 256;
                 plan[1] = rows;
                 plan[2] = cols;
                 plan[3] = n;
             }
         }
     }
-    bool here = fuse_glu || best <= 20.f || (way == 1 && K >= 4096);
+    bool here = fuse_glu || best <= 20.f || (way == 1 && (K >= 4096 || fills));
     if (way == 2) {
         const WideTimes& t = kWide[plan[1]];
         const long tiles = (long)((M + t.rows - 1) / t.rows) *

@@ -126,15 +126,17 @@ def _rule(m: int, n: int, k: int, fuse: bool = False, whole: bool = False,
           f32: bool = False) -> tuple:
     """The choice for sizes that were not timed. gemm_rows has no second kernel,
     but every block reads all of x, and takes all of K by itself: it is the faster
-    one for w of up to 20 MB with up to 4 rows and up to 14 MB with 16 (against
-    gemm_tile: 3072 x 2048, 16 rows: 7.2 us, 7.4; 3072 x 3072: one row 7.2, 7.9, 16
-    rows 9.8, 8.0; 5120 x 3072, one row 10.8, 10.0; gate/up 16384 x 3072, one row:
-    21.7, 19.8), if K is 4096 or less (1024 x 6144, 16 rows 18.6 us, 10.3, the
-    library 13.1; 1024 x 8192, 4 rows 15.5, 10.6, 13.6)."""
+    one for w of up to 20 MB with up to 4 rows and up to 10 MB with 16, while K is
+    short (against gemm_tile, us: 2048 x 2048, one row 5.7, 7.0, 16 rows 7.2, 7.6; 3072 x
+    3072, one row 6.7, 7.9, 16 rows 9.9, 8.3; 5120 x 3072, one row 11.1, 9.7; 896 x
+    4864, one row 8.3, 7.0; 2048 x 8192 13.0, 10.7; of a second kernel that is there
+    anyway gemm_tile's have 1 us). It takes a gated unit's two columns at half the rate
+    (9728 x 896, one row 7.8, 6.3)."""
     if m > 256:
         return hip_ops.gemm_plan(m, n, k, fuse, whole, f32) or ("blas",)
     rows = hip_ops.gemm_rows_fits(m, n, k, fuse)
-    if rows and k <= 4096 and n * k <= (10_000_000 if m <= 4 else 7_000_000):
+    few, short = (10_000_000, 4096) if m <= 4 else (5_000_000, 3072)
+    if rows and not fuse and k <= short and n * k <= few:
         return ("rows",)
     tiling = hip_ops.gemm_tiling(m, n, k, fuse)
     if tiling is not None:

@@ -496,18 +496,19 @@ def gemm_rows(x: torch.Tensor, w: torch.Tensor,
 _TILE_ROWS = (32, 64, 96, 128, 160, 192, 256)
 
 
-def _tile_grid(m: int, n: int, k: int,
-               fuse_swiglu: bool) -> list[tuple[int, int, int]]:
+def _tile_grid(m: int, n: int, k: int, fuse_swiglu: bool,
+               narrow: bool = False) -> list[tuple[int, int, int]]:
     """(rows, columns, blocks of these) of gemm_tile that are worth a thought:
     rows in as few blocks as can be, or twice as many, or, with few columns, in
-    up to 4."""
+    up to 4. narrow: columns in 48 too, which more than 64 rows have."""
     if m < 1 or k % 64 or (fuse_swiglu and n % 128):
         return []
     out = []
     base = -(-m // 128)
     for blocks in sorted({-(-m // r) for r in _TILE_ROWS}):
         rows = next((r for r in _TILE_ROWS if r >= -(-m // blocks)), 0)
-        for cols in (64, 128) if fuse_swiglu else (64, 96, 128):
+        for cols in (64, 128) if fuse_swiglu else (
+                48, 64, 96, 128)[not narrow or rows <= 64:]:
             tiles = n // cols * blocks
             if n % cols == 0 and rows and (
                     blocks <= base or (blocks <= 4 and tiles <= 256)):
@@ -520,7 +521,7 @@ def gemm_tilings(m: int, n: int, k: int,
     """(rows, columns, K parts) worth trying for gemm_tile: K in as many parts,
     of 128 or more, as give each of the 256 CUs a block, or in half as many."""
     out = set()
-    for rows, cols, tiles in _tile_grid(m, n, k, fuse_swiglu):
+    for rows, cols, tiles in _tile_grid(m, n, k, fuse_swiglu, True):
         most = max(1, min(256 // tiles, k // 128))
         for parts in (most, (most + 1) // 2, 1 if k <= 4096 else most):
             out.add((rows, cols, parts))
@@ -533,19 +534,17 @@ def gemm_tiling(m: int, n: int, k: int,
     """The tiling of gemm_tile for sizes that were not timed, or None if they are
     better left to the library.
 
-    Up to 64 rows: one block of rows and 64 columns as long as that is a block a
-    CU or less, K in parts for the others unless it is short (45 rows, the
-    library's time behind it: 2048 x 8192 12.2 us, 14.5; 1536 x 8960 11.8, 22.0;
-    896 x 4864 9.2, 13.3; 128256 x 3072 144, 171).
+    Up to 64 rows: one block of rows, or two of 32 if the weights are few, and 64
+    columns as long as that is a block a CU or less, K in parts of 512 or more for
+    the others (us, the library's time behind it: 48 rows of 2048 x 8192 13.0, 15.6; 896
+    x 4864 8.3 in two blocks and 9 parts, 9.2 in one, 11 in 18 parts, 17.3; 2048 x 2048
+    8.0, in one block 8.8, 11.6; 5120 x 3072 12.6, in two 13.9, 17.6; 128256 x 2048 107,
+    141).
     Up to 256: what _tile_us says of a block a CU or less, with K whole, in the
-    parts that then fill the CUs, or in half as many (160 rows: 3072 x 3072 16.6
-    us, 18.4; 5120 x 3072 16.0, 23.5; 3072 x 8192 21.7, 28.0; 1024 x 4096 11.1,
-    13.9; 256 rows: 19.4, 19.9; 19.8, 32.1; 26.2, 33.8; 13.1, 13.8). Over 51 sizes
-    of 0.3 to 50 M weights and 10 numbers of rows it takes 0.73 of the library's
-    time, 1.06 at most (2048 x 4096, 256 rows), and 1.01 of the best tiling's.
-    More blocks than CUs are a library product's sizes (17920 x 1536, 256 rows:
-    22.9 us, 22.2), but for the gated unit that it would need a second kernel
-    for."""
+    parts that then fill the CUs, or in half as many. It takes 1.003 of the best
+    choice's time in the mean, 1.07 at most, .70 of the library's (246 sizes). More blocks than CUs are a library product's sizes (17920 x
+    1536, 256 rows: 22.9 us, 22.2), but for the gated unit that it would need a second
+    kernel for."""
     if not 0 < m <= 256 or n < 1 or k < 1 or k % 64 or (
             fuse_swiglu and n % 128):
         return None
@@ -553,15 +552,16 @@ def gemm_tiling(m: int, n: int, k: int,
         cols = 128 if n // 64 > 256 and n % 128 == 0 else 64
         if n % cols:
             return None
-        parts = max(1, min(256 // (n // cols), k // (128 if k > 2048 else 512)))
-        return 32 if m <= 32 else 64, cols, parts
+        rows = 32 if m <= 32 or n * k <= 8_000_000 else 64
+        tiles = n // cols * (-(-m // rows))
+        return rows, cols, max(1, min(256 // tiles, k // 512))
     best, least = None, float("inf")
     for rows, cols, tiles in _tile_grid(m, n, k, fuse_swiglu):
         if tiles > 256:
             continue
         most = max(1, min(256 // tiles, k // 384))
         for parts in sorted({1, (most + 1) // 2, most}):
-            us = _tile_us(m, n, k, rows, cols, tiles, parts)
+            us = _tile_us(m, n, k, rows, cols, tiles, parts, fuse_swiglu)
             if us < least:
                 best, least = (rows, cols, parts), us
     if best is None and fuse_swiglu:
@@ -570,16 +570,19 @@ def gemm_tiling(m: int, n: int, k: int,
 
 
 def _tile_us(m: int, n: int, k: int, rows: int, cols: int, tiles: int,
-             parts: int) -> float:
-    """What a tiling takes of gemm_tile's time, in us, beside 6 that all have: a
-    CU's loads of its share of K, one block after the other, and with K in parts
-    the second kernel, which reads the partial sums. (Fitted to 18000 timings of 65
-    to 256 rows, 7 % off in the mean. gl_gemm_plan has the same for more rows; a test
-    holds the two together.)"""
+             parts: int, fuse_swiglu: bool = False) -> float:
+    """What a tiling takes of gemm_tile's time, in us, beside 3.9 that all have: for
+    each round of CUs its start, a CU's loads of its share of K (a row of x half as
+    long as one of w, which comes from memory), its products and gated units, and
+    with K in parts the second kernel, which reads the partial sums. (Fitted to 5800
+    timings of 65 to 1200 rows, 6.4 % standard deviation. gl_gemm_plan has the same for
+    more rows; a test holds the two together.)"""
     kslice = -(-(-(-k // parts)) // 64) * 64
     parts = -(-k // kslice)
-    us = -(-tiles * parts // 256) * kslice * (rows + cols - 37) * 3.9e-5
-    return us if parts == 1 else us + 1.2 + parts * m * n * 2.5e-6
+    us = -(-tiles * parts // 256) * (
+        3 + kslice * (rows * 1.42e-5 + cols * 3.2e-5 + rows * cols * 1.09e-7) +
+        (rows * cols * 5.8e-5 if fuse_swiglu else 0))
+    return us if parts == 1 else us + parts * m * n * 2.4e-6
 
 
 def gemm_tile(x: torch.Tensor, w: torch.Tensor, rows: int, cols: int,

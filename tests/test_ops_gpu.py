@@ -874,6 +874,28 @@ def test_gemm_tilings():
                 assert not (rule and fuse and (n % 128 or rule[1] == 96))
 
 
+@pytest.mark.parametrize("stages", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 32])
+def test_gemm_fed_stages(dev, stages):
+    """Blocks that have fewer stages of K than their rings, as many, and some more,
+    odd and even; 48 columns too; rows behind the last one."""
+    from gridllm_amd.ops import hip_ops
+    k = 64 * stages
+    g = torch.Generator().manual_seed(stages)
+    x, w = (torch.randn(*s, generator=g).to(dev, torch.bfloat16)
+            for s in ((261, k), (384, k)))
+    ref = x.float() @ w.float().t()
+    tol = 2 ** -8 * ref.abs() + k * 2 ** -24 * (x.float().abs() @
+                                                w.float().abs().t()) + 1e-6
+    for rows in (96, 128, 160, 192, 256):
+        for cols in (48, 64, 96, 128):
+            out = hip_ops.gemm_tile(x, w, rows, cols, 1,
+                                    torch.full_like(ref, 9e9).bfloat16())
+            assert bool(((out.float() - ref).abs() <= tol).all()), (rows, cols)
+    for rows in (32, 64):                      # which have no 48
+        with pytest.raises(RuntimeError):
+            hip_ops.gemm_tile(x, w, rows, 48)
+
+
 @pytest.mark.parametrize("m,n,k", [
     (1, 8, 256),               # one row and 8 columns of a tile; 4 stages
     (255, 256, 256), (257, 264, 320), (384, 1032, 576),
