@@ -862,15 +862,18 @@ static void launch_gemm_skinny(hipStream_t st, bf16_t* out, float* ws,
 // Ties pick the lowest index (torch.argmax first-max rule).
 //
 // A row is cut into S segments of a block each, so that few rows fill the chip
-// too, and a second kernel picks among the segments. Bound by the vector unit: the
-// hash's second product (three of 32 bits: its upper half is what is used; the
-// first one is a sum, see noise_of) and two logarithms an element. These are taken
-// by the hardware's instruction first, and exactly only for elements that come
-// near the best so far of the wave: the picked element is among them. Rows of
-// 128256: 64 take 190 us with one block a row and exact logarithms throughout, 21
-// with seven 32-bit products and a branch an element and maxima through LDS, 16.5
-// now; 512 (with the pick) 115 and 82, 3.2 TB/s. The pick takes 4 us instead of 53
-// us of small kernels for the keys.
+// too; their picks meet in the slot's marks, or a second kernel picks among them.
+// Bound by the vector unit: the hash's second product (three of 32 bits: its upper
+// half is what is used; the first one is a sum, see hash_of), beside which all that
+// is done for each element is a bound of its noise, one logarithm by the hardware.
+// What a block then looks at are the batches of 8 whose largest bound is next to its
+// largest, and after these whatever is not below the best of them: exactly, but for
+// elements that the hardware's two logarithms put clearly behind. The picked one is
+// among them. Rows of 128256, us with two logarithms for each element, exact values
+// in each step of a wave and a second kernel, and now: 1 row 13.3, 10.0 (what a call
+// costs the host), 20 15.2, 12.4, 64 20.4, 17.6, 149 33.4, 25.7, 512 82.5, 58.4. Of 64
+// rows' 17.6 some 10 are a launch, the loads of a key, the exact values and the two
+// atomics of a block; slots' marks in one line had 20 rows take 17.3.
 // ===========================================================================
 struct Pick {
     float val;
@@ -913,41 +916,66 @@ struct SampleKeys {
     }
 };
 
-// u of candidate i from (i ^ key) * NOISE. With the bits of i in two parts that is
-// a sum of two products, one of which all of a wave's lanes have, and the other
-// one all chunks of 256.
+// The hash's upper half of candidate i from (i ^ key) * NOISE. With the bits of i in
+// two parts that is a sum of two products, one of which all of a wave's lanes have,
+// and the other one all chunks of 256.
 #define NOISE 0x9E3779B97F4A7C15ull
-DEV_INLINE float noise_of(unsigned long long z) {
+DEV_INLINE u32 hash_of(unsigned long long z) {
     z ^= (unsigned long long)((long long)z >> 29);  // arithmetic >>
     // z *= 0xBF58476D1CE4E5B9; z ^= z >> 32: their upper half
     const u32 lo = (u32)z, top = (u32)(z >> 32);
-    u32 h = __umulhi(lo, 0x1CE4E5B9u) + lo * 0xBF58476Du + top * 0x1CE4E5B9u;
-    h ^= (u32)((int)h >> 31);
+    const u32 h = __umulhi(lo, 0x1CE4E5B9u) + lo * 0xBF58476Du +
+                  top * 0x1CE4E5B9u;
+    return h ^ (u32)((int)h >> 31);
+}
+DEV_INLINE float noise_of(u32 h) {
     const float u = (float)(h >> 6 & 0xFFFFFFu) * (1.0f / 16777216.0f);
     return fminf(fmaxf(u, 1e-6f), (float)(1.0 - 1e-6));  // rounded like torch
+}
+// The noise and c, or more: -log(-log u) <= -log(1 - u), and 1 - u is w 2^-24 at
+// least (15 for where u is clamped). c has the 24 log 2.
+#define LN2 0.6931472f
+DEV_INLINE float bounded(u32 h, float c) {
+    const float w = fmaxf((float)(~h >> 6 & 0xFFFFFFu), 15.f);
+    return fmaf(__builtin_amdgcn_logf(w), -LN2, c);
+}
+
+// The picks of a row's blocks meet in two words of its slot's cache line, which are 0
+// between calls: the largest pick, as a number whose order is that of better(), and how many
+// there have been. The last block stores the row's token and counts its draw. All that
+// blocks tell each other goes through these atomics, a block's second one behind the
+// answer to its first, so that there is nothing to release.
+#define MARK 16
+DEV_INLINE void meet(const Pick p, int* token, unsigned long long* mark,
+                     long long* draws, int blocks) {
+    const u32 v = __float_as_uint(p.val + 0.f);          // (no -0)
+    unsigned long long best = p.at == 2147483647 ? 0 :
+        (unsigned long long)(v >> 31 ? ~v : v | 0x80000000u) << 32 | ~(u32)p.at;
+    if (blocks > 1) {
+        const unsigned long long was = atomicMax(mark, best);
+        asm volatile("s_waitcnt vmcnt(0)" :: "v"(was) : "memory");
+        if (atomicAdd(mark + 1, 1ull) != blocks - 1) return;
+        best = atomicExch(mark, 0ull);
+        atomicExch(mark + 1, 0ull);
+    }
+    *token = best ? ~(u32)best : 0;                      // all -inf -> 0
+    *draws += 1;
 }
 
 // Candidates of a lane: 4 that follow each other in each of two chunks of 256.
 __global__ void __launch_bounds__(256)
-k_sample_gumbel(Pick* __restrict__ ws, const float* __restrict__ logits,
-                const SampleKeys how, int v, int segments) {
+k_sample_gumbel(Pick* __restrict__ ws, int* __restrict__ out,
+                unsigned long long* __restrict__ marks,
+                const float* __restrict__ logits, const SampleKeys how, int v,
+                int segments) {
     constexpr int E = 8;
     const int row = blockIdx.x / segments, seg = blockIdx.x % segments;
-    if (how.slots && (unsigned long long)how.slots[row] >= how.count)
-        __builtin_trap();
     const float* x = logits + (long)row * v;
-    const unsigned long long key = how.key(row);
-    const float t = how.temp(row), rt = 1.f / t;
     const int per = ((v + segments - 1) / segments + 255) & ~255;
     const int i0 = seg * per, i1 = min(v, i0 + per);
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool wide = (v & 3) == 0;    // rows start at 16 bytes
-    unsigned long long low[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-        low[e] = ((lane * 4 + e) ^ (key & 255)) * NOISE;
-    Pick best{-INFINITY, 2147483647};
     auto load = [&](int base, float* f) {
 #pragma unroll
         for (int c = 0; c < E; c += 4) {
@@ -961,53 +989,126 @@ k_sample_gumbel(Pick* __restrict__ ws, const float* __restrict__ logits,
             }
         }
     };
+    const int first = i0 + wid * 512;
     float f[E], ahead[E];
-    load(i0 + wid * 512, ahead);
-    for (int base = i0 + wid * 512; base < i1; base += 2048) {
-        float u[E], a[E];
-        auto at = [&](int e) { return base + (e >> 2) * 256 + lane * 4 + (e & 3); };
+    load(first, ahead);                // (no later than the row's slot)
+    if (how.slots && (unsigned long long)how.slots[row] >= how.count)
+        __builtin_trap();
+    const unsigned long long key = how.key(row);
+    const float t = how.temp(row), rt = 1.f / t;
+    unsigned long long low[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        low[e] = ((lane * 4 + e) ^ (key & 255)) * NOISE;
+    auto hash = [&](int base, int e) {
+        const unsigned long long chunk = base + (e >> 2) * 256;
+        return hash_of((chunk ^ (key & ~255ull)) * NOISE + low[e & 3]);
+    };
+
+    // bounds of all: a lane's largest batch, and the largest of its other ones
+    float most = -INFINITY, next = -INFINITY;
+    int at_most = first;
+    for (int base = first; base < i1; base += 2048) {
 #pragma unroll
         for (int e = 0; e < E; ++e) f[e] = ahead[e];
         load(base + 2048, ahead);
-        float lim = best.val;
+        float m = -INFINITY;
         if (key != 0ull) {             // (around the elements: they overlap)
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const unsigned long long chunk = base + (e >> 2) * 256;
-                u[e] = noise_of((chunk ^ (key & ~255ull)) * NOISE + low[e & 3]);
-                // log2 by the hardware: good to 1e-3 here, below u = 0.999
-                a[e] = f[e] * rt - 0.6931472f * __builtin_amdgcn_logf(
-                    -0.6931472f * __builtin_amdgcn_logf(u[e]));
-                lim = fmaxf(lim, u[e] <= 0.999f ? a[e] : -INFINITY);
-            }
+            for (int e = 0; e < E; ++e)
+                m = fmaxf(m, bounded(hash(base, e), fmaf(f[e], rt, 24 * LN2)));
         } else {
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                u[e] = 0.f;
-                a[e] = f[e] * rt;
-                lim = fmaxf(lim, a[e]);
+            for (int e = 0; e < E; ++e) m = fmaxf(m, f[e] * rt);
+        }
+        next = fmaxf(next, fminf(m, most));
+        if (m > most) {
+            most = m;
+            at_most = base;
+        }
+    }
+    if (!(fabsf(rt) <= FLT_MAX)) most = next = INFINITY;    // no bounds
+
+    // Exact values of a batch's elements, but for those that the hardware's logarithms
+    // put behind the best of the wave.
+    Pick best{-INFINITY, 2147483647};
+    auto look = [&](int base, bool mine) {
+        float g[E], u[E], a[E], lim = best.val;
+        auto at = [&](int e) { return base + (e >> 2) * 256 + lane * 4 + (e & 3); };
+        load(mine ? base : i1, g);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            u[e] = 0.f;
+            a[e] = g[e] * rt;
+            if (key != 0ull) {
+                u[e] = noise_of(hash(base, e));     // (lanes' batches may differ)
+                // log2 by the hardware: good to 1e-3 here, below u = 0.999
+                a[e] -= LN2 * __builtin_amdgcn_logf(
+                    -LN2 * __builtin_amdgcn_logf(u[e]));
             }
+            if (mine && u[e] <= 0.999f) lim = fmaxf(lim, a[e]);
         }
         lim = max_across16(max_of16(lim));
         lim -= 0.05f + 1e-5f * fabsf(lim);
+        u32 left = 0;
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-            // (written so that NaN and infinities take the exact way)
-            if (at(e) < i1 && !(a[e] < lim && u[e] <= 0.999f)) {
-                float val = f[e] / t;
-                if (key != 0ull) val += -logf(-logf(u[e]));
-                if (better(val, at(e), best)) best = Pick{val, at(e)};
-            }
+        for (int e = 0; e < E; ++e)        // (so that NaN and infinities are)
+            if (mine && at(e) < i1 && !(a[e] < lim && u[e] <= 0.999f))
+                left |= 1u << e;
+#pragma unroll 1
+        while (__any(left != 0)) {
+            const int at_e = left ? __ffs((int)left) - 1 : 0;
+            float x_e = g[0], u_e = u[0];
+#pragma unroll
+            for (int e = 1; e < E; ++e)
+                if (e == at_e) {
+                    x_e = g[e];
+                    u_e = u[e];
+                }
+            float val = x_e / t;
+            if (key != 0ull) val += -logf(-logf(u_e));
+            if (left && better(val, at(at_e), best)) best = Pick{val, at(at_e)};
+            left &= left - 1;
         }
+    };
+    __shared__ float bound[4];
+    __shared__ Pick part[4];
+    float top = max_across16(max_of16(most));
+    if (lane == 0) bound[wid] = top;
+    __syncthreads();
+    top = fmaxf(fmaxf(bound[0], bound[1]), fmaxf(bound[2], bound[3]));
+    const bool near = !(most < top - 0.1f - 1e-5f * fabsf(top));
+    // first the batches next to the largest bound; the best of these says what else
+    // may be it: other lanes' largest batches, and all of lanes with another large one
+    bool mine = near, more = false;
+    for (int base = at_most, behind = -1; ; ) {
+        if (__any(mine)) look(base, mine);
+        if (behind < 0) {
+            const Pick w = wave_pick(best);
+            __syncthreads();
+            if (lane == 0) bound[wid] = w.val;
+            __syncthreads();
+            float lim = fmaxf(fmaxf(bound[0], bound[1]), fmaxf(bound[2], bound[3]));
+            lim -= 1e-4f + 1e-5f * fabsf(lim);
+            more = !(next < lim);
+            mine = !near && !(most < lim);
+            behind = first;
+            continue;
+        }
+        if (!__any(more) || behind >= i1) break;
+        mine = more;
+        base = behind;
+        behind += 2048;
     }
     best = wave_pick(best);
-    __shared__ Pick part[4];
     if (lane == 0) part[wid] = best;
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 1; w < 4; ++w)
-            if (better(part[w].val, part[w].at, best)) best = part[w];
-        ws[blockIdx.x] = best;
+        for (int k = 1; k < 4; ++k)
+            if (better(part[k].val, part[k].at, best)) best = part[k];
+        if (marks) meet(best, out + row, marks + MARK * how.slots[row],
+                        how.draws + how.slots[row], segments);
+        else ws[blockIdx.x] = best;
     }
 }
 
@@ -1482,10 +1583,29 @@ int gl_sample_gumbel(void* stream, void* out, void* ws, const void* logits,
                          (unsigned long long)count};
     hipStream_t st = (hipStream_t)stream;
     k_sample_gumbel<<<dim3((unsigned)(b * segments)), dim3(256), 0, st>>>(
-        (Pick*)ws, (const float*)logits, how, v, segments);
+        (Pick*)ws, nullptr, nullptr, (const float*)logits, how, v, segments);
     LAUNCH_CHECK();
     k_sample_pick<<<dim3((unsigned)b), dim3(64), 0, st>>>(
         (int*)out, (const Pick*)ws, how, segments);
+    LAUNCH_CHECK();
+    return 0;
+}
+
+// By slot, in one launch: marks 128 bytes per slot, 0 (and left so).
+int gl_sample_slots(void* stream, void* out, const void* logits,
+                    const void* temps, const void* slots, const void* seeds,
+                    void* draws, const void* nongreedy, void* marks, int b, int v,
+                    int segments, int count) {
+    if (segments < 1 || count < 1 || v < 1 || !slots || !seeds || !draws ||
+        !nongreedy || !marks) return -100;
+    if (b <= 0) return 0;
+    const SampleKeys how{nullptr, (const float*)temps, (const long long*)slots,
+                         (const long long*)seeds, (long long*)draws,
+                         (const long long*)nongreedy, (unsigned long long)count};
+    k_sample_gumbel<<<dim3((unsigned)(b * segments)), dim3(256), 0,
+                      (hipStream_t)stream>>>(
+        nullptr, (int*)out, (unsigned long long*)marks, (const float*)logits, how, v,
+        segments);
     LAUNCH_CHECK();
     return 0;
 }

@@ -376,6 +376,7 @@ class SlotSampler:
         self.tps = torch.ones(n_slots, device=device)
         self.seeds = torch.zeros(n_slots, dtype=torch.int64, device=device)
         self.draws = torch.zeros(n_slots, dtype=torch.int64, device=device)
+        self.marks = torch.zeros(n_slots, 16, dtype=torch.int64, device=device)
 
     def admit(self, rows, vocab: int) -> None:
         """Register newly admitted rows (objects with .slot and .state)."""
@@ -443,7 +444,7 @@ class SlotSampler:
                 slot_ids = slot_ids.to(logits.device, torch.int64)
             return hip_ops.sample_gumbel_slots(
                 logits.contiguous(), slot_ids.contiguous(), self.temps,
-                self.seeds, self.draws, self.nongreedy)
+                self.seeds, self.draws, self.nongreedy, self.marks)
         temps = self.temps[slot_ids].unsqueeze(1)
         x = logits / temps
         v = logits.shape[1]

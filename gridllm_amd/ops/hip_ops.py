@@ -90,6 +90,8 @@ def _load() -> ctypes.CDLL:
                                  c_f, c_f, c_f, c_f]
     lib.gl_sample_gumbel.argtypes = [c_vp] * 10 + [c_i] * 4
     lib.gl_sample_gumbel.restype = c_i
+    lib.gl_sample_slots.argtypes = [c_vp] * 9 + [c_i] * 4
+    lib.gl_sample_slots.restype = c_i
     lib.gl_swiglu_il.restype = c_i
     lib.gl_device_sync.argtypes = []
     lib.gl_device_sync.restype = c_i
@@ -780,17 +782,19 @@ def sample_gumbel(logits: torch.Tensor, keys: torch.Tensor,
 
 def sample_gumbel_slots(logits: torch.Tensor, slots: torch.Tensor,
                         temps: torch.Tensor, seeds: torch.Tensor,
-                        draws: torch.Tensor, nongreedy: torch.Tensor
-                        ) -> torch.Tensor:
+                        draws: torch.Tensor, nongreedy: torch.Tensor,
+                        marks: Optional[torch.Tensor] = None) -> torch.Tensor:
     """sample_gumbel with the rows' parameters by slot (slots [B] i64, all
     different; temps f32, seeds, draws, nongreedy i64): the keys are made in the
     kernel, and the slots' draws advance by one. A slot that there is not ends the
-    program, as an index out of bounds does in torch."""
-    return _sample(logits, None, temps, slots, seeds, draws, nongreedy)
+    program, as an index out of bounds does in torch. marks: i64 [slots, 16] of zeros,
+    which stay zeros between calls and belong to the slots as their draws do: one
+    launch instead of two."""
+    return _sample(logits, None, temps, slots, seeds, draws, nongreedy, marks)
 
 
 def _sample(logits, keys, temps, slots=None, seeds=None, draws=None,
-            nongreedy=None) -> torch.Tensor:
+            nongreedy=None, marks=None) -> torch.Tensor:
     lib = _load()
     b, v = logits.shape
     f32, i64, dev, n = torch.float32, torch.int64, logits.get_device(), \
@@ -806,7 +810,10 @@ def _sample(logits, keys, temps, slots=None, seeds=None, draws=None,
               == seeds.get_device() == draws.get_device()
               == nongreedy.get_device() and slots.is_contiguous()
               and seeds.is_contiguous() and draws.is_contiguous()
-              and nongreedy.is_contiguous())
+              and nongreedy.is_contiguous()
+              and (marks is None or (
+                  marks.dtype is i64 and marks.shape == (*n, 16)
+                  and dev == marks.get_device() and marks.is_contiguous())))
     if not (ok and logits.dtype is f32 and temps.dtype is f32 and dev >= 0
             and dev == temps.get_device() and logits.is_contiguous()
             and temps.is_contiguous()):
@@ -815,10 +822,16 @@ def _sample(logits, keys, temps, slots=None, seeds=None, draws=None,
                          "length, dense and on one GPU")
     if slots is not None:
         _check_range("sample_gumbel.slots", slots, n[0])
-    # four blocks a CU, of 2048 elements or more: 64 rows of 128256 take 16.5 us
-    # in 16 segments (190 in one, with exact logarithms)
+    # four blocks a CU, of 2048 elements or more
     segments = max(1, min(1024 // max(1, b), v // 2048, 64))
     out = torch.empty(b, dtype=torch.int32, device=logits.device)
+    if marks is not None and v:
+        _check(lib.gl_sample_slots(
+            _stream(), out.data_ptr(), logits.data_ptr(), temps.data_ptr(),
+            slots.data_ptr(), seeds.data_ptr(), draws.data_ptr(),
+            nongreedy.data_ptr(), marks.data_ptr(), b, v, segments, n[0]),
+            "sample_slots")
+        return out
     ws = torch.empty(b * segments, dtype=i64, device=logits.device)
     at = (keys.data_ptr(), temps.data_ptr(), None, None, None, None) \
         if slots is None else (

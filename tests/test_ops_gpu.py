@@ -573,6 +573,41 @@ def test_sample_gumbel_segments(dev, b, v):
             assert at >= best - 1e-5 * abs(best) - 1e-4
 
 
+@pytest.mark.parametrize("b,v", [(1, 1), (3, 2047), (2, 4096), (64, 8192), (1, 128256),
+                                 (20, 128256), (600, 4352), (1100, 515)])
+def test_sample_gumbel_marks(dev, b, v):
+    """Picks that meet in the slots' marks are those of the second kernel, call after
+    call, with ties in all segments, -inf, +inf, NaN, flat and peaked rows, and
+    rows without noise; the marks are zeros again."""
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator().manual_seed(b + v)
+    x = torch.randn(b, v, generator=g) * 2
+    x[::5] = x[::5].round()
+    x[::7, ::2] = float("-inf")
+    if b > 2:
+        x[1] = float("-inf")
+        x[2, ::3] = 0.0
+        x[2, 1::3] = -0.0
+    if b > 20:
+        x[20], x[19, v // 3], x[18, v // 2], x[17, ::9] = 1.0, 30.0, float(
+            "inf"), float("nan")
+    x = x.to(dev)
+    slots = torch.randperm(b + 3, generator=g)[:b].to(dev)
+    temps = (torch.rand(b + 3, generator=g) + 0.3).to(dev)
+    seeds = torch.randint(0, 2 ** 62, (b + 3,), generator=g).to(dev)
+    live = (torch.arange(b + 3) % 4 != 3).long().to(dev)
+    draws, marks = torch.zeros_like(seeds), torch.zeros(b + 3, 16, dtype=torch.int64,
+                                                        device=dev)
+    draws2 = draws.clone()
+    for _ in range(4):
+        got = hip_ops.sample_gumbel_slots(x, slots, temps, seeds, draws, live, marks)
+        want = hip_ops.sample_gumbel_slots(x, slots, temps, seeds, draws2, live)
+        assert torch.equal(got, want) and torch.equal(draws, draws2)
+        assert not marks.any()
+    with pytest.raises(ValueError):
+        hip_ops.sample_gumbel_slots(x, slots, temps, seeds, draws, live, marks[1:])
+
+
 @pytest.mark.parametrize("b,v", [(7, 256), (5, 257), (3, 511), (4, 512), (2, 2049),
                                  (3, 4096), (2, 6400), (1, 133000), (600, 4352)])
 def test_sample_gumbel_chunks(dev, b, v):
