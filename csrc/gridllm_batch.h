@@ -152,6 +152,10 @@ DEV_INLINE void batch_join(const BatchArgs& p, const BatchTile& t, int m0, int k
 //   16384x3072  20.7 -> 18.6     20.8 -> 19.4     22.8 -> 21.4 (gated)
 //   128256x3072  141 ->  132      150 ->  138      166 ->  162
 // Waves that load alone, as below, take .3 to .5 us more here: a block starts later.
+// 256 columns, for rows of x that are read once for all of them, where there are more
+// tiles than CUs anyway: a vocabulary's scores, with up to 160 rows (128256 x 3072, us
+// in 128 columns and in 256: 64 rows 159, 147, 96 178, 159, 160 198, 186; 128256 x 2048
+// 106, 100, 120, 107, 134, 128; 192 columns 160 at 64 rows).
 // ===========================================================================
 template <int RT, int CT>
 struct GemmTile {
@@ -163,7 +167,7 @@ struct GemmTile {
 };
 
 template <int RT, int CT, int EPI>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, CT == 16 ? 1 : 2)
 k_gemm_tile(const BatchArgs p) {
     typedef GemmTile<RT, CT> Sh;
     constexpr int R = Sh::R, C = Sh::C, NB = Sh::NB, BUF = (R + C) * 64;

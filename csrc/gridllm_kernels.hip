@@ -699,9 +699,10 @@ static int allow_lds(int bytes) {
 
 template <int RT, int CT, int EPI>
 static int launch_gemm_tile(hipStream_t st, BatchArgs p) {
-    typedef std::conditional_t<RT <= 4, GemmTile<RT, CT>, GemmFed<RT, CT>> Sh;
+    constexpr bool both = RT <= 4 || CT == 16;  // waves load and multiply
+    typedef std::conditional_t<both, GemmTile<RT, CT>, GemmFed<RT, CT>> Sh;
     constexpr auto kernel = [] {
-        if constexpr (RT <= 4) return k_gemm_tile<RT, CT, EPI>;
+        if constexpr (both) return k_gemm_tile<RT, CT, EPI>;
         else return k_gemm_fed<RT, CT, EPI>;
     }();
     const int e = allow_lds<kernel>(Sh::BYTES);
@@ -1434,6 +1435,7 @@ int gl_gemm_tile(void* stream, void* out, void* ws, const void* x,
 #define COLS(RT) GO(RT, 4, 0); GO(RT, 6, 0); GO(RT, 8, 0); GO(RT, 4, 1); \
     GO(RT, 8, 1)
     GO(6, 3, 0); GO(8, 3, 0); GO(10, 3, 0); GO(12, 3, 0); GO(16, 3, 0);
+    GO(2, 16, 0); GO(4, 16, 0); GO(6, 16, 0); GO(8, 16, 0); GO(10, 16, 0);
     COLS(2); COLS(4); COLS(6); COLS(8); COLS(10); COLS(12); COLS(16);
 #undef COLS
 #undef GO

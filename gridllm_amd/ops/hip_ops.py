@@ -521,8 +521,13 @@ def _tile_grid(m: int, n: int, k: int, fuse_swiglu: bool,
 def gemm_tilings(m: int, n: int, k: int,
                  fuse_swiglu: bool = False) -> list[tuple[int, int, int]]:
     """(rows, columns, K parts) worth trying for gemm_tile: K in as many parts,
-    of 128 or more, as give each of the 256 CUs a block, or in half as many."""
+    of 128 or more, as give each of the 256 CUs a block, or in half as many; and 256
+    columns, if these are still more tiles than CUs."""
     out = set()
+    rows = next((r for r in _TILE_ROWS if r >= m), 256)
+    if 0 < m <= 160 and n % 256 == 0 and n > 65536 and k % 64 == 0 and \
+            not fuse_swiglu:
+        out.add((rows, 256, 1))
     for rows, cols, tiles in _tile_grid(m, n, k, fuse_swiglu, True):
         most = max(1, min(256 // tiles, k // 128))
         for parts in (most, (most + 1) // 2, 1 if k <= 4096 else most):

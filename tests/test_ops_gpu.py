@@ -926,9 +926,12 @@ def test_gemm_fed_stages(dev, stages):
             out = hip_ops.gemm_tile(x, w, rows, cols, 1,
                                     torch.full_like(ref, 9e9).bfloat16())
             assert bool(((out.float() - ref).abs() <= tol).all()), (rows, cols)
-    for rows in (32, 64):                      # which have no 48
+    for rows in (32, 64, 96, 128, 160):        # 256 columns: up to 160 rows
+        out = hip_ops.gemm_tile_f32(x, w[:256], rows, 256)
+        assert bool(((out - ref[:, :256]).abs() <= tol[:, :256]).all()), rows
+    for rows, cols in ((32, 48), (64, 48), (192, 256), (256, 256)):
         with pytest.raises(RuntimeError):
-            hip_ops.gemm_tile(x, w, rows, 48)
+            hip_ops.gemm_tile(x, w[:256] if cols == 256 else w, rows, cols)
 
 
 @pytest.mark.parametrize("m,n,k", [
