@@ -854,7 +854,7 @@ DEV_INLINE void mlstm_gates(const float* gr, int h, int H, float cap,
                             float& i, float& f) {
     i = cap * tanhf(gr[h] / cap);
     const float z = cap * tanhf(gr[H + h] / cap);
-    f = fminf(z, 0.f) - log1pf(expf(-fabsf(z)));
+    f = log_sigmoid(z);
 }
 
 // seg (int4): {first token, length, slot, start position}; null: row r is a
@@ -1670,74 +1670,101 @@ k_mlstm_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
 // without the normaliser row.
 // ===========================================================================
 
-// b of one chunk for 64 channels: z = W2 u + bias with w = W2^T, f32 [R][C]. A
-// wave has U tokens, whose sums meet in LDS. The first items are 4 U each of the
-// first nd tokens, chunks of their own; then come the chunks ({first token,
-// length, ..}). Bound by the logarithms and their latency: with one thread for
-// a channel's 64 tokens (3050 tokens, 1536 channels: 1.2 waves a SIMD) it took 45
-// us, so 31.
-template <int U>
+// log a of 16 tokens for 16 NT channels: z = W2 u + bias with w = W2^T, f32 [R][C],
+// by the matrix cores' f32 products. A lane has 4 tokens, (lane / 16) * 4 on, of
+// channels c0 + n * 16 + lane % 16.
+template <int NT>
+DEV_INLINE void log_decays(f32x4 (&z)[NT], const float* u, const float* w,
+                           const float* bias, int last, int c0, int R, int C,
+                           float inv_tau) {
+    const int fr = threadIdx.x & 15, gq = (threadIdx.x & 63) >> 4;
+    const float* ur = u + (long)min(fr, last) * R;
+    int c[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        c[n] = min(c0 + n * 16 + fr, C - 1);
+        const float b0 = bias[c[n]];
+        z[n] = (f32x4){b0, b0, b0, b0};
+    }
+    for (int rb = 0; rb < R; rb += 16) {
+        float a[4], v[4][NT];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int k = rb + j * 4 + gq;
+            a[j] = k < R ? ur[k] : 0.f;
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                v[j][n] = k < R ? w[(long)k * C + c[n]] : 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                z[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], v[j][n], z[n],
+                                                            0, 0, 0);
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z[n][r] = log_sigmoid(z[n][r]) * inv_tau;
+}
+
+// b for 64 channels, of 16 of the first nd tokens, chunks of their own (a wave has
+// 16 channels), or of one chunk ({first token, length, ..}; a wave has 16 tokens,
+// whose sums meet in LDS). Bound by the logarithms: 2730 tokens, 1536 channels, rank
+// 16: 34 us with log1pf and u in scalar registers, which are too few for 16 tokens
+// (25 without log1pf), now 13.7.
 __global__ void __launch_bounds__(256)
 k_gla_decay(float* __restrict__ b, const float* __restrict__ u,
             const float* __restrict__ w, const float* __restrict__ bias,
             const int4* __restrict__ chunks, int nd, int R, int C,
             float inv_tau) {
     __shared__ float sums[4][64];
-    const int it = blockIdx.x, singles = (nd + 4 * U - 1) / (4 * U);
-    const bool single = it < singles;
-    int4 ch = make_int4(it * 4 * U, min(4 * U, nd - it * 4 * U), 0, 0);
-    if (!single) ch = chunks[it - singles];
-    const int lane = threadIdx.x & 63;
+    const int it = blockIdx.x, singles = (nd + 15) / 16;
+    const int fr = threadIdx.x & 15, gq = (threadIdx.x & 63) >> 4;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int c = min((int)blockIdx.y * 64 + lane, C - 1);
-    const bool own = (int)blockIdx.y * 64 + lane < C;
-    const float b0 = bias[c];
-    float ahead = 0.f;                 // of the steps of 4 U tokens before
-    for (int s0 = 0; s0 < ch.y; s0 += 4 * U) {
-        const int t0 = s0 + wid * U;
-        float z[U];
-        const float* ur[U];
+    const int c0 = blockIdx.y * 64;
+    if (it < singles) {
+        const int left = nd - it * 16, c = c0 + wid * 16 + fr;
+        f32x4 z[1];
+        log_decays(z, u + (long)it * 16 * R, w, bias, left - 1, c0 + wid * 16,
+                   R, C, inv_tau);
 #pragma unroll
-        for (int i = 0; i < U; ++i) {
-            z[i] = b0;
-            ur[i] = u + (long)(ch.x + min(t0 + i, ch.y - 1)) * R;
+        for (int r = 0; r < 4; ++r)
+            if (c < C && gq * 4 + r < left)
+                b[(it * 16l + gq * 4 + r) * C + c] = z[0][r];
+        return;
+    }
+    const int4 ch = chunks[it - singles];
+    const int t0 = min(wid * 16, ch.y - 1);
+    f32x4 z[4];
+    log_decays(z, u + (long)(ch.x + t0) * R, w, bias, ch.y - 1 - t0, c0, R, C,
+               inv_tau);
+    float ahead[4];                    // of the wave's tokens before the lane's
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+#pragma unroll
+        for (int r = 1; r < 4; ++r) z[n][r] += z[n][r - 1];
+        float sum = z[n][3];
+        float up = __shfl_up(sum, 16, WAVE);
+        if (gq >= 1) sum += up;
+        up = __shfl_up(sum, 32, WAVE);
+        if (gq >= 2) sum += up;
+        up = __shfl_up(sum, 16, WAVE);
+        ahead[n] = gq ? up : 0.f;
+        if (gq == 3) sums[wid][n * 16 + fr] = sum;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+        const int c = c0 + n * 16 + fr;
+        for (int v = 0; v < wid; ++v) ahead[n] += sums[v][n * 16 + fr];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int t = wid * 16 + gq * 4 + r;
+            if (c < C && t < ch.y)
+                b[(long)(ch.x + t) * C + c] = z[n][r] + ahead[n];
         }
-        for (int rb = 0; rb < R; rb += 8) {    // 8 loads in flight
-            float wv[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                wv[k] = rb + k < R ? w[(long)(rb + k) * C + c] : 0.f;
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (rb + k < R)
-#pragma unroll
-                    for (int i = 0; i < U; ++i) z[i] += ur[i][rb + k] * wv[k];
-        }
-        float sum = 0.f;
-#pragma unroll
-        for (int i = 0; i < U; ++i) {
-            const float la =
-                (fminf(z[i], 0.f) - log1pf(expf(-fabsf(z[i])))) * inv_tau;
-            sum = single || t0 + i >= ch.y ? la : sum + la;
-            z[i] = sum;
-        }
-        if (!single) {
-            sums[wid][lane] = sum;
-            __syncthreads();
-            float all = ahead;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                if (v == wid) ahead = all;
-                all += sums[v][lane];
-            }
-#pragma unroll
-            for (int i = 0; i < U; ++i) z[i] += ahead;
-            ahead = all;
-            __syncthreads();
-        }
-#pragma unroll
-        for (int i = 0; i < U; ++i)
-            if (own && t0 + i < ch.y) b[(long)(ch.x + t0 + i) * C + c] = z[i];
     }
 }
 
@@ -3089,12 +3116,10 @@ int gh_gla_decay(void* stream, void* b, const void* u, const void* w,
                  const void* bias, const void* chunks, int nd, int nchunks,
                  int R, int C, float inv_tau) {
     if (nd + nchunks < 1 || R < 1 || C < 1) return -100;
-#define GO(U) k_gla_decay<U><<<dim3((nd + 4 * U - 1) / (4 * U) + nchunks, \
-        (C + 63) / 64), 256, 0, (hipStream_t)stream>>>((float*)b, \
-        (const float*)u, (const float*)w, (const float*)bias, \
-        (const int4*)chunks, nd, R, C, inv_tau)
-    if (nchunks) GO(16); else GO(1);
-#undef GO
+    k_gla_decay<<<dim3((nd + 15) / 16 + nchunks, (C + 63) / 64), 256, 0,
+                  (hipStream_t)stream>>>((float*)b, (const float*)u,
+        (const float*)w, (const float*)bias, (const int4*)chunks, nd, R, C,
+        inv_tau);
     LAUNCH_CHECK();
     return 0;
 }
