@@ -1778,89 +1778,156 @@ DEV_INLINE void split_bf16(float x, bf16_t& hi, bf16_t& lo) {
     lo = f2bf(x - bf2f(hi));
 }
 
-// A chunk's own contribution to the state, in blocks as mLSTM's. (3050 tokens, 12
-// heads of 128 x 256: 33 us before, now 28.)
-__global__ void __launch_bounds__(256)
-k_gla_chunk_state(float* __restrict__ dS, const bf16_t* __restrict__ qkv,
-                  const float* __restrict__ b, const int4* __restrict__ chunks,
-                  int H, int DK, int DV, int ld_, int cols) {
-    __shared__ __attribute__((aligned(16))) bf16_t vs[64 * 256];
-    __shared__ __attribute__((aligned(16))) bf16_t kh[64 * 64];
-    __shared__ __attribute__((aligned(16))) bf16_t kl[64 * 64];
-    const int4 ch = chunks[blockIdx.x];
-    const int h = blockIdx.y, nd = DK / 64, last = ch.y - 1;
-    const int d0 = (blockIdx.z % nd) * 64, v0 = (blockIdx.z / nd) * cols;
-    const int nv = min(cols, DV - v0);
-    const int t = threadIdx.x >> 2, c16 = (threadIdx.x & 3) * 16;
-    const bf16_t* row = qkv + (long)ch.x * ld_;
-    const long n = min(t, last);
-    const float* bt = b + (ch.x + n) * H * DK + h * DK + d0 + c16;
-    const float* bT = bt + (last - n) * H * DK;
-    float e[16], w[16];
+// The state that enters each chunk, left in dS as (hi | lo << 16) bf16 pairs; the
+// slot's state is advanced. Block = (segment, head, 32 key channels and 64 value
+// NK * 64 value columns), and the state stays in registers from chunk to chunk: a
+// wave has NK * 16 by 16. A chunk's operands are loaded two chunks ahead.
+// Bound by a step's instructions and latencies (.8 us a chunk) where a segment is
+// long, by the stores where there are many. 45 chunks of 4 segments, 12 heads of 128
+// x 256: 58 us when the chunks' own contributions were written first, read and
+// added up by a second kernel; now 35. (256 threads, each with twice the keys: 34,
+// but 54 instead of 44 for one segment of 3500.)
+#define STATE_K 32
+template <int NK>
+__global__ void __launch_bounds__(512)
+k_gla_states(u32* __restrict__ dS, float* __restrict__ S,
+             const bf16_t* __restrict__ qkv, const float* __restrict__ b,
+             const int4* __restrict__ chunks, const int4* __restrict__ segs,
+             int nseg, int H, int DK, int DV, int ld_) {
+    constexpr int VW = 64 * NK;
+    __shared__ __attribute__((aligned(16))) bf16_t vs[64 * VW];
+    __shared__ __attribute__((aligned(16))) bf16_t kh[64 * STATE_K];
+    __shared__ __attribute__((aligned(16))) bf16_t kl[64 * STATE_K];
+    __shared__ __attribute__((aligned(16))) float keep[STATE_K];
+    // (the grid's x is a multiple of 8, so that an XCD has all of a head's blocks)
+    if ((int)blockIdx.x >= nseg * H) return;
+    const int h = blockIdx.x % H, nd = DK / STATE_K;
+    const int d0 = (int)blockIdx.y % nd * STATE_K;
+    const int v0 = (int)blockIdx.y / nd * VW;
+    const int lane = threadIdx.x & 63, fr = lane & 15, gq = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kcol = NK == 1 ? wid >> 2 << 4 : 0;
+    const int vcol = NK == 1 ? (wid & 3) << 4 : wid << 4;
+    const int4 sg = segs[blockIdx.x / H];
+    const int first = chunks[sg.z].x;
+    const int4 end = chunks[sg.z + sg.w - 1];
+    const int n = end.x + end.y - first;           // tokens
+    const int t = threadIdx.x >> 3, c = threadIdx.x & 7;   // token, piece of its row
+    const long C = (long)H * DK;
+    const bf16_t* kp = qkv + (long)first * ld_ + C + h * DK + d0 + c * 4;
+    const bf16_t* vp = qkv + (long)first * ld_ + 2 * C + h * DV + v0 + c * 8;
+    const float* bp = b + (long)first * C + h * DK + d0 + c * 4;
+    struct Piece { f32x2 k; f32x4 v[NK], b, bT; } pieces[2];
+    auto load = [&](Piece& p, int at) {
+        const long row = min(at * 64 + t, n - 1);
+        p.k = *(const f32x2*)(kp + row * ld_);
 #pragma unroll
-    for (int i = 0; i < 16; i += 8) {
-        ld8(bt + i, e + i);
-        ld8(bT + i, w + i);
-    }
-    const bf16_t* kp = row + n * ld_ + (H + h) * DK + d0 + c16;
-    const uint4 kv[2] = {((const uint4*)kp)[0], ((const uint4*)kp)[1]};
-    load_values(vs, row + 2l * H * DK + h * DV + v0, ld_, last, nv);
+        for (int i = 0; i < NK; ++i)
+            p.v[i] = *(const f32x4*)(vp + row * ld_ + i * 64);
+        p.b = *(const f32x4*)(bp + row * C);
+        p.bT = *(const f32x4*)(bp + min(at * 64 + 63, n - 1) * C);
+    };
+    // places of 16-byte pieces among 32 columns, for reads as value_piece's
+    auto at32 = [](int row, int c) {
+        return row * STATE_K + (c ^ (row >> 2 & 2)) * 8;
+    };
+    auto key_piece = [&](const bf16_t* keys, int ks, int i0) {
+        const int d = kcol + i0 * 16 + (fr & 3) * 4;
+        bf16x8 v;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) w[i] = t <= last ? __expf(w[i] - e[i]) : 0.f;
-    store_keys(kh, kl, (const bf16_t*)kv, w);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    lds_barrier();
-    store_state(dS + (((long)blockIdx.x * H + h) * DV + v0) * DK + d0, vs, kh,
-                kl, nv, DK);
-}
-
-// The state that enters each chunk, left in dS as (hi | lo << 16) bf16 pairs;
-// the slot's state is advanced.
-__global__ void __launch_bounds__(256)
-k_gla_chunk_scan(float* __restrict__ dS, float* __restrict__ S,
-                 const float* __restrict__ b, const int4* __restrict__ chunks,
-                 const int4* __restrict__ segs, int H, int DK, int DV) {
-    const int4 sg = segs[blockIdx.x];
-    const int h = blockIdx.y;
+        for (int j = 0; j < 2; ++j) {
+            const int row = ks * 32 + gq * 8 + (fr >> 2) + j * 4;
+            const bf16x4 x =
+                read_transposed(keys + at32(row, d >> 3) + (d & 7));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[j * 4 + i] = x[i];
+        }
+        return v;
+    };
+    const long own = (long)(v0 + vcol + fr) * DK + d0 + kcol + gq * 4;
     const long size = (long)DV * DK;
-    const long e = (blockIdx.z * 256L + threadIdx.x) * 4;
-    if (e >= size) return;
-    float* Sb = S + ((long)sg.x * H + h) * size + e;
-    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (sg.y != 0) s = *(const float4*)Sb;
-    const long cs = (long)H * size;
-    float* Db = dS + ((long)sg.z * H + h) * size + e;
-    const float* bc = b + h * DK + (int)(e % DK);
-    constexpr int U = 8;
-    for (int c = 0; c < sg.w; c += U) {
-        float4 d[U], k[U];
+    float* Sb = S + ((long)sg.x * H + h) * size + own;
+    u32* Db = dS + ((long)sg.z * H + h) * size + own;
+    f32x4 acc[NK];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (c + u < sg.w) {
-                const int4 ch = chunks[sg.z + c + u];
-                d[u] = *(const float4*)(Db + (c + u) * cs);
-                k[u] = *(const float4*)(bc + (long)(ch.x + ch.y - 1) * H * DK);
+    for (int d = 0; d < NK; ++d) {
+        acc[d] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        if (sg.y != 0) acc[d] = *(const f32x4*)(Sb + d * 16);
+    }
+    auto step = [&](Piece& p, int at) {
+        lds_barrier();                             // the last chunk's are read
+        // (nothing of these loads is waited for earlier)
+        asm volatile("" : "+v"(p.k), "+v"(p.v[0]), "+v"(p.v[NK - 1]),
+                     "+v"(p.b), "+v"(p.bT));
+        float f[4];
+        ld4((const bf16_t*)&p.k, f);
+        const bool in = at * 64 + t < n;
+        bf16x4 hi, lo;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float x = f[i] * (in ? __expf(p.bT[i] - p.b[i]) : 0.f);
+            hi[i] = (__bf16)x;
+            lo[i] = (__bf16)(x - (float)hi[i]);
+        }
+        const int to = at32(t, c >> 1) + (c & 1) * 4;
+        *(bf16x4*)(kh + to) = hi;
+        *(bf16x4*)(kl + to) = lo;
+#pragma unroll
+        for (int i = 0; i < NK; ++i)
+            *(f32x4*)(vs + at_cols(t, i * 8 + c, VW)) = p.v[i];
+        if (t == 0)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) keep[c * 4 + i] = __expf(p.bT[i]);
+        lds_barrier();
+        load(p, at + 2);
+        bf16x8 v[2], k[2][NK][2];
+        f32x4 kept[NK];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            v[ks] = value_piece(vs, ks, vcol, VW);
+#pragma unroll
+            for (int d = 0; d < NK; ++d) {
+                k[ks][d][0] = key_piece(kh, ks, d);
+                k[ks][d][1] = key_piece(kl, ks, d);
             }
+        }
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (c + u >= sg.w) break;
+        for (int d = 0; d < NK; ++d)
+            kept[d] = *(const f32x4*)(keep + kcol + d * 16 + gq * 4);
+        __builtin_amdgcn_sched_barrier(0);         // all on their way
+#pragma unroll
+        for (int d = 0; d < NK; ++d) {
             uint4 pk;
-            const float sv[4] = {s.x, s.y, s.z, s.w};
             u32* pp = (u32*)&pk;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                bf16_t hi, lo;
-                split_bf16(sv[i], hi, lo);
-                pp[i] = (u32)hi | ((u32)lo << 16);
+            for (int r = 0; r < 4; ++r) {
+                bf16_t sh, sl;
+                split_bf16(acc[d][r], sh, sl);
+                pp[r] = (u32)sh | ((u32)sl << 16);
             }
-            *(uint4*)(Db + (c + u) * cs) = pk;
-            s.x = __expf(k[u].x) * s.x + d[u].x;
-            s.y = __expf(k[u].y) * s.y + d[u].y;
-            s.z = __expf(k[u].z) * s.z + d[u].z;
-            s.w = __expf(k[u].w) * s.w + d[u].w;
+            *(uint4*)(Db + at * (H * size) + d * 16) = pk;
+            acc[d] *= kept[d];
         }
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int d = 0; d < NK; ++d)
+                    acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        k[ks][d][i], v[ks], acc[d], 0, 0, 0);
+    };
+    load(pieces[0], 0);
+    __builtin_amdgcn_sched_barrier(0);             // in this order
+    load(pieces[1], 1);
+    for (int at = 0;;) {
+        step(pieces[0], at);
+        if (++at >= sg.w) break;
+        step(pieces[1], at);
+        if (++at >= sg.w) break;
     }
-    *(float4*)Sb = s;
+#pragma unroll
+    for (int d = 0; d < NK; ++d) *(f32x4*)(Sb + d * 16) = acc[d];
 }
 
 // 8 values f[i] exp(e[i]) as the (hi, lo) pair of bf16 fragments
@@ -3132,15 +3199,17 @@ int gh_gla_chunks(void* stream, void* o, void* out, void* S, void* dS,
     if (nchunks < 1 || nseg < 1 || DK % 64 || DV % 64 || (out && DV > 256))
         return -100;
     hipStream_t st_ = (hipStream_t)stream;
-    const int cols = state_columns(nchunks * H);
-    k_gla_chunk_state<<<dim3(nchunks, H, DK / 64 * ((DV + cols - 1) / cols)),
-                        256, 0, st_>>>((float*)dS, (const bf16_t*)qkv,
-        (const float*)b, (const int4*)chunks, H, DK, DV, ld_, cols);
-    LAUNCH_CHECK();
-    const long quads = (long)DV * DK / 4;
-    k_gla_chunk_scan<<<dim3(nseg, H, (unsigned)((quads + 255) / 256)), 256, 0,
-                       st_>>>((float*)dS, (float*)S, (const float*)b,
-        (const int4*)chunks, (const int4*)segs, H, DK, DV);
+    // Blocks of 128 value columns weigh keys half as often, and are half as many.
+    // 128 / 64 columns, 12 heads of 128 x 256, us: segments of 1100, 800, 500 and 331
+    // tokens (384 blocks of 128) 35 / 41, 12 of 300 40 / 47; one of 3500 (96) 63 / 44.
+    const bool wide = DV % 128 == 0 &&
+                      nseg * H * (DK / STATE_K) * (DV / 128) >= 256;
+#define GO(NK) k_gla_states<NK><<<dim3((nseg * H + 7) / 8 * 8, \
+        DK / STATE_K * (DV / (64 * NK))), 512, 0, st_>>>((u32*)dS, (float*)S, \
+        (const bf16_t*)qkv, (const float*)b, (const int4*)chunks, \
+        (const int4*)segs, nseg, H, DK, DV, ld_)
+    if (wide) GO(2); else GO(1);
+#undef GO
     LAUNCH_CHECK();
     k_gla_chunk_out<<<dim3(nchunks, H, (DV + 255) / 256), 256, 0, st_>>>(
         (float*)o, (bf16_t*)out, (const float*)dS, (const bf16_t*)qkv,

@@ -838,6 +838,61 @@ def test_mlstm_chunk_sizes(dk, dv, entering):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads,dv", [(16, 256), (32, 192), (2, 256)])
+@pytest.mark.parametrize("kind", ["gla"])
+def test_states_of_many_chunks(kind, heads, dv):
+    """Portions of one to four chunks, more and fewer blocks of the states than
+    the chip has CUs, with columns that go into 128 and that do not."""
+    from gridllm_amd.ops import reference_hybrid
+    dk, lens = 128, (250, 192, 129, 65, 64, 63, 1, 100)
+    n, at = sum(lens), 0
+    entries, chunks, segs = [], [], []
+    for i, ln in enumerate(lens):
+        start = (i % 2) * 9
+        entries.append((at, ln, i, start))
+        segs.append((i, start, len(chunks), -(-ln // 64)))
+        chunks += [(at + c, min(64, ln - c), i, 0) for c in range(0, ln, 64)]
+        at += ln
+    g = torch.Generator().manual_seed(heads + dv)
+    pos = torch.cat([torch.arange(e[3], e[3] + e[1]) for e in entries])
+    slot = torch.cat([torch.full((e[1],), e[2]) for e in entries])
+
+    def step(dev):
+        def t(rows):
+            return torch.tensor(rows, dtype=torch.int32, device=dev)
+        own = dict(segs=t(entries)) if dev == "cpu" else \
+            dict(segs=t(entries), chunks=t(chunks), chunk_segs=t(segs))
+        return hops.StepMeta(nd=0, pos=pos.int().to(dev),
+                             slot=slot.int().to(dev), max_len=300,
+                             table=torch.zeros(8, 1, dtype=torch.int32,
+                                               device=dev), **own)
+    rows = torch.randn(n, heads * 2 * (dk + dv), generator=g)
+    rows = rows.to(torch.bfloat16)
+    S = torch.randn(8, heads, dv + (kind == "mlstm"), dk, generator=g)
+    m = torch.rand(8, heads, generator=g)
+    norm = torch.ones(heads * dv)
+    u, ba = torch.randn(n, 8, generator=g), torch.randn(heads * dk, generator=g)
+    wa = torch.randn(8, heads * dk, generator=g)
+    gates = torch.randn(n, 2 * heads, generator=g) * 3
+    got = []
+    for fn, dev, x in ((reference_hybrid, "cpu", rows.float()),
+                       (hops, "cuda", rows.cuda())):
+        s, mx = S.clone().to(dev), m.clone().to(dev)
+        if kind == "gla":
+            fn.gla(x, u.to(dev), wa.to(dev), ba.to(dev), s, norm.to(dev),
+                   step(dev), dk, dv, 16.0, 1e-5)
+        else:
+            fn.mlstm(x, gates.to(dev), s, mx, norm.to(dev), step(dev), dk, dv,
+                     15.0, 1e-5)
+        got.append((s.cpu(), mx.cpu()))
+    # keys as (hi, lo) pairs of bf16 are within 2^-17, a sum of 64 of a chunk's
+    # products with unequal signs within that of its largest terms
+    assert float((got[1][0] - got[0][0]).abs().max()) < \
+        2 ** -13 * float(got[0][0].abs().max())
+    assert float((got[1][1] - got[0][1]).abs().max()) < 1e-4
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,w,parts,size", [(1, 64, 2, 8), (24, 3072, 5, 384),
                                             (3, 1088, 9, 4)])
 def test_norms_add_parts(n, w, parts, size):
