@@ -1090,16 +1090,15 @@ k_rec_row_out(T* __restrict__ out, const float* __restrict__ o,
 // inside a chunk, a_s = i_s - F_s and M_t = max(m_in, max_{s<=t} a_s):
 //   m_t = F_t + M_t
 //   S_t = exp(m_in - M_t) S_in + sum_{s<=t} exp(a_s - M_t) v_s k_s^T
-// so a chunk's own contribution (state kernel), the state that enters each
-// chunk (scan kernel), and the outputs (out kernel) separate; the first and
-// the last run over all chunks at once on the matrix cores. Where a product
-// takes f32 factors (state, weighted keys) they are split into two bf16 parts.
+// so the state that enters each chunk (one chunk after the other, in registers)
+// and the outputs (all chunks at once) separate, both on the matrix cores. Where a
+// product takes f32 factors (state, weighted keys) they are split into two bf16
+// parts.
 //
 // chunk (int4): {first token, length, segment, -}
 // seg   (int4): {slot, start position, first chunk, chunks}
-// dS: f32 [chunks][H][DV + 1][DK]; the scan leaves the entering state there as
-// (hi | lo << 16) bf16 pairs. scal: f32 [chunks][H][4] = {max a, F total,
-// m of the slot before the step, m_in}.
+// dS: [chunks][H][DV + 1][DK], the entering states as (hi | lo << 16) bf16 pairs.
+// scal: f32 [chunks][H][4] = {max a, F total, m of the slot before the step, -}.
 // ---------------------------------------------------------------------------
 #define MCH 64
 
@@ -1174,179 +1173,253 @@ DEV_INLINE bf16x8 value_piece(const bf16_t* vs, int ks, int col, int cols) {
     return v;
 }
 
-// 16 weighted keys of a thread's token (tid / 4) as (hi, lo) pairs of bf16, in LDS
-// as load_values lays out 64 columns; w: their weights
-DEV_INLINE void store_keys(bf16_t* kh, bf16_t* kl, const bf16_t* k,
-                           const float* w) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        float f[8];
-        ld8(k + i * 8, f);
-        bf16x8 hi, lo;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float x = f[j] * w[i * 8 + j];
-            hi[j] = (__bf16)x;
-            lo[j] = (__bf16)(x - (float)hi[j]);
-        }
-        const int at = at_cols(threadIdx.x >> 2, (threadIdx.x & 3) * 2 + i, 64);
-        *(bf16x8*)(kh + at) = hi;
-        *(bf16x8*)(kl + at) = lo;
-    }
-}
-
-// Sum over 64 tokens of values times weighted keys, for 64 key channels and up
-// to 256 value columns, of which a wave has every fourth 16: D, f32 rows of DK.
-DEV_INLINE void store_state(float* D, const bf16_t* vs, const bf16_t* kh,
-                            const bf16_t* kl, int nv, int DK) {
-    const int lane = threadIdx.x & 63;
-    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    f32x4 acc[4][4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int d = 0; d < 4; ++d) acc[c][d] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-        bf16x8 hi[4], lo[4];
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            hi[d] = value_piece(kh, ks, d * 16, 64);
-            lo[d] = value_piece(kl, ks, d * 16, 64);
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            if (c * 64 >= nv) continue;
-            const bf16x8 v = value_piece(vs, ks, c * 64 + wid * 16, nv);
-#pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                acc[c][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    hi[d], v, acc[c][d], 0, 0, 0);
-                acc[c][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    lo[d], v, acc[c][d], 0, 0, 0);
-            }
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        if (c * 64 >= nv) continue;
-        float* row = D + (long)(c * 64 + wid * 16 + (lane & 15)) * DK +
-                     (lane >> 4) * 4;
-#pragma unroll
-        for (int d = 0; d < 4; ++d) *(f32x4*)(row + d * 16) = acc[c][d];
-    }
-}
-
-// A chunk's own contribution to the state. Block = (chunk, head, 64 key channels
-// and `cols` value columns, up to 256). Bound by writing it, 128 KB a head and
-// chunk of 128 x 256: 3500 tokens, 12 heads: 43 us with 64 columns a block,
-// operands transposed by 2-byte stores to LDS and results stored by 4 bytes,
-// now 35.
+// Of each chunk and head: the weights exp(a - max a) of its keys, f32 [64] at w, and
+// of scal max a, F total and m of the slot before the step. A wave has a head.
 template <bool CONST>
 __global__ void __launch_bounds__(256)
-k_mlstm_chunk_state(float* __restrict__ dS, float* __restrict__ scal,
-                    const float* __restrict__ mst,
-                    const bf16_t* __restrict__ qkv,
-                    const float* __restrict__ gr,
-                    const int4* __restrict__ chunks,
-                    const int4* __restrict__ segs, int H, int DK, int DV,
-                    int ld_, float cap, int cols) {
-    __shared__ __attribute__((aligned(16))) bf16_t vs[64 * 256];
-    __shared__ __attribute__((aligned(16))) bf16_t kh[64 * 64];
-    __shared__ __attribute__((aligned(16))) bf16_t kl[64 * 64];
-    __shared__ float wgt[MCH];
+k_mlstm_weights(float* __restrict__ w, float* __restrict__ scal,
+                const float* __restrict__ mst, const float* __restrict__ gr,
+                const int4* __restrict__ chunks, const int4* __restrict__ segs,
+                int H, float cap) {
     const int4 ch = chunks[blockIdx.x];
-    const int h = blockIdx.y;
-    const int nd = DK / 64;
-    const int d0 = (blockIdx.z % nd) * 64, v0 = (blockIdx.z / nd) * cols;
-    const int nv = min(cols, DV - v0), last = ch.y - 1;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int t = threadIdx.x >> 2, c16 = (threadIdx.x & 3) * 16;
-    const bf16_t* row = qkv + (long)ch.x * ld_;
-    load_values(vs, row + 2l * H * DK + h * DV + v0, ld_, last, nv);
-    const bf16_t* kp = row + (long)min(t, last) * ld_ + (H + h) * DK + d0 + c16;
-    const uint4 kv[2] = {((const uint4*)kp)[0], ((const uint4*)kp)[1]};
-    if (wid == 0) {
-        float F, a, amax;
-        chunk_scan<CONST>(gr, ch.x, ch.y, h, H, cap, F, a, amax);
-        const float A = __shfl(amax, 63, WAVE);
-        wgt[lane] = lane < ch.y ? expf(a - A) : 0.f;
-        if (blockIdx.z == 0 && lane == 63) {
-            const int4 sg = segs[ch.z];
-            float* sp = scal + ((long)blockIdx.x * H + h) * 4;
-            sp[0] = A;
-            sp[1] = F;
-            sp[2] = CONST || sg.y == 0 ? 0.f : mst[(long)sg.x * H + h];
-        }
-    }
-    __syncthreads();
-    float w[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) w[i] = wgt[t];
-    store_keys(kh, kl, (const bf16_t*)kv, w);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    lds_barrier();
-    const int R = CONST ? DV : DV + 1;
-    float* Db = dS + ((long)blockIdx.x * H + h) * R * DK + d0;
-    store_state(Db + (long)v0 * DK, vs, kh, kl, nv, DK);
-    if (!CONST && v0 == 0 && threadIdx.x < 64) {
-        float s = 0.f;
-        for (int i = 0; i < MCH; ++i) {
-            const int at = at_cols(i, lane >> 3, 64) + (lane & 7);
-            s += bf2f(kh[at]) + bf2f(kl[at]);
-        }
-        Db[(long)DV * DK + lane] = s;
+    const int h = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (h >= H) return;
+    float F, a, amax;
+    chunk_scan<CONST>(gr, ch.x, ch.y, h, H, cap, F, a, amax);
+    const float A = __shfl(amax, 63, WAVE);
+    const long at = (long)blockIdx.x * H + h;
+    w[at * 64 + lane] = lane < ch.y ? expf(a - A) : 0.f;
+    if (lane == 63) {
+        const int4 sg = segs[ch.z];
+        scal[at * 4] = A;
+        scal[at * 4 + 1] = F;
+        scal[at * 4 + 2] = CONST || sg.y == 0 ? 0.f : mst[(long)sg.x * H + h];
     }
 }
 
-template <bool CONST>
-__global__ void __launch_bounds__(256)
-k_mlstm_chunk_scan(float* __restrict__ dS, float* __restrict__ scal,
-                   float* __restrict__ S, float* __restrict__ mst,
-                   const int4* __restrict__ segs, int H, int DK, int DV) {
-    const int4 sg = segs[blockIdx.x];
-    const int h = blockIdx.y;
-    const long size = (long)(CONST ? DV : DV + 1) * DK;
-    const long e = (blockIdx.z * 256L + threadIdx.x) * 4;
-    if (e >= size) return;
-    float* Sb = S + ((long)sg.x * H + h) * size + e;
-    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (sg.y != 0) s = *(const float4*)Sb;
-    float m = scal[((long)sg.z * H + h) * 4 + 2];
-    const long cs = (long)H * size;
-    float* Db = dS + ((long)sg.z * H + h) * size + e;
-    constexpr int U = 8;
-    for (int c = 0; c < sg.w; c += U) {
-        float4 d[U];
+// The state that enters each chunk of a prompt portion, left in dS as (hi | lo << 16) bf16 pairs; the
+// slot's state is advanced. Block = (segment, head, 32 key channels and 64 value
+// NK * 64 value columns), and the state stays in registers from chunk to chunk: a
+// wave has NK * 16 by 16. A chunk's operands are loaded two chunks ahead.
+// Bound by a step's instructions and latencies (.8 us a chunk) where a segment is
+// long, by the stores where there are many. 45 chunks of 4 segments, 12 heads of 128
+// x 256: 58 us when the chunks' own contributions were written first, read and
+// added up by a second kernel; now 35. (256 threads, each with twice the keys: 34,
+// but 54 instead of 44 for one segment of 3500.) With what is ahead of it and the
+// outputs, mLSTM's 55 chunks of one segment: 127 us before, now 105.
+// KIND: gated linear attention's decays by channel (b), or weights and sums of
+// k_mlstm_weights, where the slot's m is advanced too; mLSTM's normaliser, the row
+// behind the value columns, is the product of the keys with ones.
+#define STATE_K 32
+enum { STATE_GLA, STATE_MLSTM, STATE_CONST };
+// a thread's token in a chunk: b and the last token's, or its weight, max a and F total
+template <bool GLA> struct TokenWeights { f32x4 b, bT; };
+template <> struct TokenWeights<false> { float w, A, F; };
+template <int KIND, int NK>
+__global__ void __launch_bounds__(512)
+k_chunk_states(u32* __restrict__ dS, float* __restrict__ S,
+               const float* __restrict__ scal, float* __restrict__ m_in,
+               float* __restrict__ mst, const bf16_t* __restrict__ qkv,
+               const float* __restrict__ b, const int4* __restrict__ chunks,
+               const int4* __restrict__ segs, int nseg, int H, int DK, int DV,
+               int ld_) {
+    constexpr bool GLA = KIND == STATE_GLA, NORM = KIND == STATE_MLSTM;
+    constexpr int VW = 64 * NK;
+    __shared__ __attribute__((aligned(16))) bf16_t vs[64 * VW];
+    __shared__ __attribute__((aligned(16))) bf16_t kh[64 * STATE_K];
+    __shared__ __attribute__((aligned(16))) bf16_t kl[64 * STATE_K];
+    __shared__ __attribute__((aligned(16))) float keep[STATE_K];
+    // (the grid's x is a multiple of 8, so that an XCD has all of a head's blocks)
+    if ((int)blockIdx.x >= nseg * H) return;
+    const int h = blockIdx.x % H, nd = DK / STATE_K;
+    const int d0 = (int)blockIdx.y % nd * STATE_K;
+    const int v0 = (int)blockIdx.y / nd * VW;
+    const int lane = threadIdx.x & 63, fr = lane & 15, gq = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kcol = NK == 1 ? wid >> 2 << 4 : 0;
+    const int vcol = NK == 1 ? (wid & 3) << 4 : wid << 4;
+    const int4 sg = segs[blockIdx.x / H];
+    const int first = chunks[sg.z].x;
+    const int4 end = chunks[sg.z + sg.w - 1];
+    const int n = end.x + end.y - first;           // tokens
+    const int t = threadIdx.x >> 3, c = threadIdx.x & 7;   // token, piece of its row
+    const long C = (long)H * DK;
+    const bf16_t* kp = qkv + (long)first * ld_ + C + h * DK + d0 + c * 4;
+    const bf16_t* vp = qkv + (long)first * ld_ + 2 * C + h * DV + v0 + c * 8;
+    const float* bp = GLA ? b + (long)first * C + h * DK + d0 + c * 4
+                          : b + ((long)sg.z * H + h) * 64 + t;
+    const float* const sp = scal + ((long)sg.z * H + h) * 4;
+    float m = GLA ? 0.f : sp[2];
+    const bool leads = blockIdx.y == 0 && threadIdx.x == 0;
+    struct Piece { f32x2 k; f32x4 v[NK]; TokenWeights<GLA> w; } pieces[2];
+    auto load = [&](Piece& p, int at) {
+        const long row = min(at * 64 + t, n - 1);
+        p.k = *(const f32x2*)(kp + row * ld_);
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (c + u < sg.w) d[u] = *(const float4*)(Db + (c + u) * cs);
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (c + u >= sg.w) break;
-            float* sp = scal + ((long)(sg.z + c + u) * H + h) * 4;
-            const float A = sp[0], Ft = sp[1];
-            if (e == 0) sp[3] = m;
-            uint4 pk;
-            const float sv[4] = {s.x, s.y, s.z, s.w};
-            u32* pp = (u32*)&pk;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const bf16_t hi = f2bf(sv[i]);
-                pp[i] = (u32)hi | ((u32)f2bf(sv[i] - bf2f(hi)) << 16);
-            }
-            *(uint4*)(Db + (c + u) * cs) = pk;
-            const float M = fmaxf(m, A);
-            const float keep = expf(m - M), put = expf(A - M);
-            s.x = keep * s.x + put * d[u].x;
-            s.y = keep * s.y + put * d[u].y;
-            s.z = keep * s.z + put * d[u].z;
-            s.w = keep * s.w + put * d[u].w;
-            m = Ft + M;
+        for (int i = 0; i < NK; ++i)
+            p.v[i] = *(const f32x4*)(vp + row * ld_ + i * 64);
+        if constexpr (GLA) {
+            p.w.b = *(const f32x4*)(bp + row * C);
+            p.w.bT = *(const f32x4*)(bp + min(at * 64 + 63, n - 1) * C);
+        } else {
+            const long to = min(at, sg.w - 1);
+            p.w.w = bp[to * H * 64];
+            p.w.A = sp[to * H * 4];
+            p.w.F = sp[to * H * 4 + 1];
         }
+    };
+    // (so that nothing of it is waited for earlier)
+    auto wait = [](Piece& p) {
+        asm volatile("" : "+v"(p.k), "+v"(p.v[0]), "+v"(p.v[NK - 1]));
+        if constexpr (GLA)
+            asm volatile("" : "+v"(p.w.b), "+v"(p.w.bT));
+        else
+            asm volatile("" : "+v"(p.w.w));
+    };
+    // places of 16-byte pieces among 32 columns, for reads as value_piece's
+    auto at32 = [](int row, int c) {
+        return row * STATE_K + (c ^ (row >> 2 & 2)) * 8;
+    };
+    auto key_piece = [&](const bf16_t* keys, int ks, int i0) {
+        const int d = kcol + i0 * 16 + (fr & 3) * 4;
+        bf16x8 v;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int row = ks * 32 + gq * 8 + (fr >> 2) + j * 4;
+            const bf16x4 x =
+                read_transposed(keys + at32(row, d >> 3) + (d & 7));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[j * 4 + i] = x[i];
+        }
+        return v;
+    };
+    const long own = (long)(v0 + vcol + fr) * DK + d0 + kcol + gq * 4;
+    const long size = (long)(NORM ? DV + 1 : DV) * DK;
+    float* Sb = S + ((long)sg.x * H + h) * size + own;
+    u32* Db = dS + ((long)sg.z * H + h) * size + own;
+    f32x4 acc[NK];
+#pragma unroll
+    for (int d = 0; d < NK; ++d) {
+        acc[d] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        if (sg.y != 0) acc[d] = *(const f32x4*)(Sb + d * 16);
     }
-    *(float4*)Sb = s;
-    if (!CONST && e == 0) mst[(long)sg.x * H + h] = m;
+    // The normaliser: the waves of the first 16 columns have it, lanes 0 of 16 store.
+    const long below = (long)(DV - fr) * DK;
+    const bool norms = NORM && v0 + vcol == 0;
+    f32x4 den[NK];
+    if (norms)
+#pragma unroll
+        for (int d = 0; d < NK; ++d) {
+            den[d] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            if (sg.y != 0) den[d] = *(const f32x4*)(Sb + below + d * 16);
+        }
+    bf16x8 ones;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.f;
+    auto packed = [](f32x4 x) {
+        uint4 pk;
+        u32* pp = (u32*)&pk;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const bf16_t hi = f2bf(x[r]);
+            pp[r] = (u32)hi | ((u32)f2bf(x[r] - bf2f(hi)) << 16);
+        }
+        return pk;
+    };
+    auto step = [&](Piece& p, int at) {
+        lds_barrier();                             // the last chunk's are read
+        wait(p);
+        float f[4], stay = 0.f, w[4];
+        const bool in = at * 64 + t < n;
+        if constexpr (GLA) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w[i] = __expf(p.w.bT[i] - p.w.b[i]);
+            if (t == 0)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) keep[c * 4 + i] = __expf(p.w.bT[i]);
+        } else {
+            const float M = fmaxf(m, p.w.A);
+            if (leads) m_in[(sg.z + at) * (long)H + h] = m;
+            stay = expf(m - M);
+            w[0] = w[1] = w[2] = w[3] = expf(p.w.A - M) * p.w.w;
+            m = p.w.F + M;
+        }
+        ld4((const bf16_t*)&p.k, f);
+        bf16x4 hi, lo;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float x = f[i] * (in ? w[i] : 0.f);
+            hi[i] = (__bf16)x;
+            lo[i] = (__bf16)(x - (float)hi[i]);
+        }
+        const int to = at32(t, c >> 1) + (c & 1) * 4;
+        *(bf16x4*)(kh + to) = hi;
+        *(bf16x4*)(kl + to) = lo;
+#pragma unroll
+        for (int i = 0; i < NK; ++i)
+            *(f32x4*)(vs + at_cols(t, i * 8 + c, VW)) = p.v[i];
+        lds_barrier();
+        load(p, at + 2);
+        bf16x8 v[2], k[2][NK][2];
+        f32x4 kept[NK];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            v[ks] = value_piece(vs, ks, vcol, VW);
+#pragma unroll
+            for (int d = 0; d < NK; ++d) {
+                k[ks][d][0] = key_piece(kh, ks, d);
+                k[ks][d][1] = key_piece(kl, ks, d);
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < NK; ++d)
+            kept[d] = GLA ? *(const f32x4*)(keep + kcol + d * 16 + gq * 4)
+                          : (f32x4){stay, stay, stay, stay};
+        __builtin_amdgcn_sched_barrier(0);         // all on their way
+#pragma unroll
+        for (int d = 0; d < NK; ++d) {
+            *(uint4*)(Db + at * (H * size) + d * 16) = packed(acc[d]);
+            acc[d] *= kept[d];
+        }
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int d = 0; d < NK; ++d)
+                    acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        k[ks][d][i], v[ks], acc[d], 0, 0, 0);
+        if (!norms) return;
+#pragma unroll
+        for (int d = 0; d < NK; ++d) {
+            if (fr == 0)
+                *(uint4*)(Db + at * (H * size) + below + d * 16) =
+                    packed(den[d]);
+            den[d] *= kept[d];
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    den[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        k[ks][d][i], ones, den[d], 0, 0, 0);
+        }
+    };
+    load(pieces[0], 0);
+    load(pieces[1], 1);
+    wait(pieces[0]);               // (else each turn waits as the first one must)
+    wait(pieces[1]);
+    for (int at = 0;;) {
+        step(pieces[0], at);
+        if (++at >= sg.w) break;
+        step(pieces[1], at);
+        if (++at >= sg.w) break;
+    }
+#pragma unroll
+    for (int d = 0; d < NK; ++d) {
+        *(f32x4*)(Sb + d * 16) = acc[d];
+        if (norms && fr == 0) *(f32x4*)(Sb + below + d * 16) = den[d];
+    }
+    if (NORM && leads) mst[(long)sg.x * H + h] = m;
 }
 
 // 8 (hi | lo << 16) pairs -> the two bf16 fragments
@@ -1435,7 +1508,7 @@ template <bool CONST>
 __global__ void __launch_bounds__(256, 2)
 k_mlstm_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
                   const float* __restrict__ dS,
-                  const float* __restrict__ scal,
+                  const float* __restrict__ ms,
                   const bf16_t* __restrict__ qkv,
                   const float* __restrict__ gr,
                   const int4* __restrict__ chunks,
@@ -1494,7 +1567,7 @@ k_mlstm_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
     if (wid == 0) {
         float F, a, amax;
         chunk_scan<CONST>(gr, ch.x, ch.y, h, H, cap, F, a, amax);
-        const float m_in = scal[((long)blockIdx.x * H + h) * 4 + 3];
+        const float m_in = ms[(long)blockIdx.x * H + h];
         const float M = fmaxf(m_in, amax);
         sa[lane] = a;
         sM[lane] = M;
@@ -1776,158 +1849,6 @@ k_gla_decay(float* __restrict__ b, const float* __restrict__ u,
 DEV_INLINE void split_bf16(float x, bf16_t& hi, bf16_t& lo) {
     hi = f2bf(x);
     lo = f2bf(x - bf2f(hi));
-}
-
-// The state that enters each chunk, left in dS as (hi | lo << 16) bf16 pairs; the
-// slot's state is advanced. Block = (segment, head, 32 key channels and 64 value
-// NK * 64 value columns), and the state stays in registers from chunk to chunk: a
-// wave has NK * 16 by 16. A chunk's operands are loaded two chunks ahead.
-// Bound by a step's instructions and latencies (.8 us a chunk) where a segment is
-// long, by the stores where there are many. 45 chunks of 4 segments, 12 heads of 128
-// x 256: 58 us when the chunks' own contributions were written first, read and
-// added up by a second kernel; now 35. (256 threads, each with twice the keys: 34,
-// but 54 instead of 44 for one segment of 3500.)
-#define STATE_K 32
-template <int NK>
-__global__ void __launch_bounds__(512)
-k_gla_states(u32* __restrict__ dS, float* __restrict__ S,
-             const bf16_t* __restrict__ qkv, const float* __restrict__ b,
-             const int4* __restrict__ chunks, const int4* __restrict__ segs,
-             int nseg, int H, int DK, int DV, int ld_) {
-    constexpr int VW = 64 * NK;
-    __shared__ __attribute__((aligned(16))) bf16_t vs[64 * VW];
-    __shared__ __attribute__((aligned(16))) bf16_t kh[64 * STATE_K];
-    __shared__ __attribute__((aligned(16))) bf16_t kl[64 * STATE_K];
-    __shared__ __attribute__((aligned(16))) float keep[STATE_K];
-    // (the grid's x is a multiple of 8, so that an XCD has all of a head's blocks)
-    if ((int)blockIdx.x >= nseg * H) return;
-    const int h = blockIdx.x % H, nd = DK / STATE_K;
-    const int d0 = (int)blockIdx.y % nd * STATE_K;
-    const int v0 = (int)blockIdx.y / nd * VW;
-    const int lane = threadIdx.x & 63, fr = lane & 15, gq = lane >> 4;
-    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int kcol = NK == 1 ? wid >> 2 << 4 : 0;
-    const int vcol = NK == 1 ? (wid & 3) << 4 : wid << 4;
-    const int4 sg = segs[blockIdx.x / H];
-    const int first = chunks[sg.z].x;
-    const int4 end = chunks[sg.z + sg.w - 1];
-    const int n = end.x + end.y - first;           // tokens
-    const int t = threadIdx.x >> 3, c = threadIdx.x & 7;   // token, piece of its row
-    const long C = (long)H * DK;
-    const bf16_t* kp = qkv + (long)first * ld_ + C + h * DK + d0 + c * 4;
-    const bf16_t* vp = qkv + (long)first * ld_ + 2 * C + h * DV + v0 + c * 8;
-    const float* bp = b + (long)first * C + h * DK + d0 + c * 4;
-    struct Piece { f32x2 k; f32x4 v[NK], b, bT; } pieces[2];
-    auto load = [&](Piece& p, int at) {
-        const long row = min(at * 64 + t, n - 1);
-        p.k = *(const f32x2*)(kp + row * ld_);
-#pragma unroll
-        for (int i = 0; i < NK; ++i)
-            p.v[i] = *(const f32x4*)(vp + row * ld_ + i * 64);
-        p.b = *(const f32x4*)(bp + row * C);
-        p.bT = *(const f32x4*)(bp + min(at * 64 + 63, n - 1) * C);
-    };
-    // places of 16-byte pieces among 32 columns, for reads as value_piece's
-    auto at32 = [](int row, int c) {
-        return row * STATE_K + (c ^ (row >> 2 & 2)) * 8;
-    };
-    auto key_piece = [&](const bf16_t* keys, int ks, int i0) {
-        const int d = kcol + i0 * 16 + (fr & 3) * 4;
-        bf16x8 v;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int row = ks * 32 + gq * 8 + (fr >> 2) + j * 4;
-            const bf16x4 x =
-                read_transposed(keys + at32(row, d >> 3) + (d & 7));
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[j * 4 + i] = x[i];
-        }
-        return v;
-    };
-    const long own = (long)(v0 + vcol + fr) * DK + d0 + kcol + gq * 4;
-    const long size = (long)DV * DK;
-    float* Sb = S + ((long)sg.x * H + h) * size + own;
-    u32* Db = dS + ((long)sg.z * H + h) * size + own;
-    f32x4 acc[NK];
-#pragma unroll
-    for (int d = 0; d < NK; ++d) {
-        acc[d] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        if (sg.y != 0) acc[d] = *(const f32x4*)(Sb + d * 16);
-    }
-    auto step = [&](Piece& p, int at) {
-        lds_barrier();                             // the last chunk's are read
-        // (nothing of these loads is waited for earlier)
-        asm volatile("" : "+v"(p.k), "+v"(p.v[0]), "+v"(p.v[NK - 1]),
-                     "+v"(p.b), "+v"(p.bT));
-        float f[4];
-        ld4((const bf16_t*)&p.k, f);
-        const bool in = at * 64 + t < n;
-        bf16x4 hi, lo;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float x = f[i] * (in ? __expf(p.bT[i] - p.b[i]) : 0.f);
-            hi[i] = (__bf16)x;
-            lo[i] = (__bf16)(x - (float)hi[i]);
-        }
-        const int to = at32(t, c >> 1) + (c & 1) * 4;
-        *(bf16x4*)(kh + to) = hi;
-        *(bf16x4*)(kl + to) = lo;
-#pragma unroll
-        for (int i = 0; i < NK; ++i)
-            *(f32x4*)(vs + at_cols(t, i * 8 + c, VW)) = p.v[i];
-        if (t == 0)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) keep[c * 4 + i] = __expf(p.bT[i]);
-        lds_barrier();
-        load(p, at + 2);
-        bf16x8 v[2], k[2][NK][2];
-        f32x4 kept[NK];
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            v[ks] = value_piece(vs, ks, vcol, VW);
-#pragma unroll
-            for (int d = 0; d < NK; ++d) {
-                k[ks][d][0] = key_piece(kh, ks, d);
-                k[ks][d][1] = key_piece(kl, ks, d);
-            }
-        }
-#pragma unroll
-        for (int d = 0; d < NK; ++d)
-            kept[d] = *(const f32x4*)(keep + kcol + d * 16 + gq * 4);
-        __builtin_amdgcn_sched_barrier(0);         // all on their way
-#pragma unroll
-        for (int d = 0; d < NK; ++d) {
-            uint4 pk;
-            u32* pp = (u32*)&pk;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                bf16_t sh, sl;
-                split_bf16(acc[d][r], sh, sl);
-                pp[r] = (u32)sh | ((u32)sl << 16);
-            }
-            *(uint4*)(Db + at * (H * size) + d * 16) = pk;
-            acc[d] *= kept[d];
-        }
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int d = 0; d < NK; ++d)
-                    acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        k[ks][d][i], v[ks], acc[d], 0, 0, 0);
-    };
-    load(pieces[0], 0);
-    __builtin_amdgcn_sched_barrier(0);             // in this order
-    load(pieces[1], 1);
-    for (int at = 0;;) {
-        step(pieces[0], at);
-        if (++at >= sg.w) break;
-        step(pieces[1], at);
-        if (++at >= sg.w) break;
-    }
-#pragma unroll
-    for (int d = 0; d < NK; ++d) *(f32x4*)(Sb + d * 16) = acc[d];
 }
 
 // 8 values f[i] exp(e[i]) as the (hi, lo) pair of bf16 fragments
@@ -2769,6 +2690,25 @@ static int paged_decode(hipStream_t st, void* out, const void* q,
     return 0;
 }
 
+// Blocks of 128 value columns weigh keys half as often, and are half as many.
+// 128 / 64 columns, 12 heads of 128 x 256, us: segments of 1100, 800, 500 and 331
+// tokens (384 blocks of 128) 35 / 41, 12 of 300 40 / 47; one of 3500 (96) 63 / 44.
+template <int KIND>
+static void chunk_states(hipStream_t st, void* dS, void* S, const void* scal,
+                         float* m_in, void* mst, const void* qkv, const void* b, const void* chunks,
+                         const void* segs, int nseg, int H, int DK, int DV,
+                         int ld_) {
+    const bool wide = DV % 128 == 0 &&
+                      nseg * H * (DK / STATE_K) * (DV / 128) >= 256;
+#define GO(NK) k_chunk_states<KIND, NK><<<dim3((nseg * H + 7) / 8 * 8, \
+        DK / STATE_K * (DV / (64 * NK))), 512, 0, st>>>((u32*)dS, (float*)S, \
+        (const float*)scal, m_in, (float*)mst, (const bf16_t*)qkv, \
+        (const float*)b, (const int4*)chunks, (const int4*)segs, nseg, H, DK, \
+        DV, ld_)
+    if (wide) GO(2); else GO(1);
+#undef GO
+}
+
 extern "C" {
 
 int gh_embed(void* stream, int f32, void* x, void* xb, const void* emb,
@@ -3140,11 +3080,8 @@ int gh_rec_row_out(void* stream, int f32, void* out, const void* o,
     return 0;
 }
 
-// Value columns of a block of a chunk's state. Few chunks: 64, so that there are
-// more blocks, though each takes the keys' weights again.
-static int state_columns(int items) { return items >= 256 ? 256 : 64; }
-
-// constant: lightning attention (gr: log decay by head; mst unused)
+// constant: lightning attention (gr: log decay by head; mst unused). scal: f32
+// [nchunks][H][4], [nchunks][H] and [nchunks][H][64] one behind the other
 int gh_mlstm_chunks(void* stream, int constant, void* o, void* out, void* S,
                     void* mst, void* dS, void* scal, const void* qkv,
                     const void* gr, const void* chunks, const void* segs,
@@ -3155,22 +3092,19 @@ int gh_mlstm_chunks(void* stream, int constant, void* o, void* out, void* S,
         (out && (constant || DV > 256)))
         return -100;
     hipStream_t st_ = (hipStream_t)stream;
-    const long quads = (long)(DV + !constant) * DK / 4;
-    const int cols = state_columns(nchunks * H);
+    float* const m_in = (float*)scal + (long)nchunks * H * 4;
+    float* const w = m_in + (long)nchunks * H;
 #define GO(C) do { \
-    k_mlstm_chunk_state<C><<<dim3(nchunks, H, \
-        DK / 64 * ((DV + cols - 1) / cols)), 256, 0, st_>>>((float*)dS, \
-        (float*)scal, (const float*)mst, \
-        (const bf16_t*)qkv, (const float*)gr, (const int4*)chunks, \
-        (const int4*)segs, H, DK, DV, ld_, cap, cols); \
+    k_mlstm_weights<C><<<dim3(nchunks, (H + 3) / 4), 256, 0, st_>>>(w, \
+        (float*)scal, (const float*)mst, (const float*)gr, \
+        (const int4*)chunks, (const int4*)segs, H, cap); \
     LAUNCH_CHECK(); \
-    k_mlstm_chunk_scan<C><<<dim3(nseg, H, (unsigned)((quads + 255) / 256)), \
-        256, 0, st_>>>((float*)dS, (float*)scal, (float*)S, (float*)mst, \
-        (const int4*)segs, H, DK, DV); \
+    chunk_states<C ? STATE_CONST : STATE_MLSTM>(st_, dS, S, scal, m_in, mst, \
+        qkv, w, chunks, segs, nseg, H, DK, DV, ld_); \
     LAUNCH_CHECK(); \
     k_mlstm_chunk_out<C><<<dim3(nchunks, H, (DV + 255) / 256), 256, 0, \
-        st_>>>((float*)o, (bf16_t*)out, (const float*)dS, \
-        (const float*)scal, (const bf16_t*)qkv, (const float*)gr, \
+        st_>>>((float*)o, (bf16_t*)out, (const float*)dS, m_in, \
+        (const bf16_t*)qkv, (const float*)gr, \
         (const int4*)chunks, (const float*)norm, H, DK, DV, ld_, qscale, cap, \
         dvtrue, eps); \
     LAUNCH_CHECK(); } while (0)
@@ -3199,17 +3133,8 @@ int gh_gla_chunks(void* stream, void* o, void* out, void* S, void* dS,
     if (nchunks < 1 || nseg < 1 || DK % 64 || DV % 64 || (out && DV > 256))
         return -100;
     hipStream_t st_ = (hipStream_t)stream;
-    // Blocks of 128 value columns weigh keys half as often, and are half as many.
-    // 128 / 64 columns, 12 heads of 128 x 256, us: segments of 1100, 800, 500 and 331
-    // tokens (384 blocks of 128) 35 / 41, 12 of 300 40 / 47; one of 3500 (96) 63 / 44.
-    const bool wide = DV % 128 == 0 &&
-                      nseg * H * (DK / STATE_K) * (DV / 128) >= 256;
-#define GO(NK) k_gla_states<NK><<<dim3((nseg * H + 7) / 8 * 8, \
-        DK / STATE_K * (DV / (64 * NK))), 512, 0, st_>>>((u32*)dS, (float*)S, \
-        (const bf16_t*)qkv, (const float*)b, (const int4*)chunks, \
-        (const int4*)segs, nseg, H, DK, DV, ld_)
-    if (wide) GO(2); else GO(1);
-#undef GO
+    chunk_states<STATE_GLA>(st_, dS, S, nullptr, nullptr, nullptr, qkv, b,
+                            chunks, segs, nseg, H, DK, DV, ld_);
     LAUNCH_CHECK();
     k_gla_chunk_out<<<dim3(nchunks, H, (DV + 255) / 256), 256, 0, st_>>>(
         (float*)o, (bf16_t*)out, (const float*)dS, (const bf16_t*)qkv,

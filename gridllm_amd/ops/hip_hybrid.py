@@ -441,7 +441,7 @@ def mlstm(qkv: torch.Tensor, gates: torch.Tensor, S: torch.Tensor,
         nch = st.chunks.shape[0]
         ds = torch.empty(nch, h, dv + 1, dk, dtype=torch.float32,
                          device=qkv.device)
-        scal = torch.empty(nch, h, 4, dtype=torch.float32, device=qkv.device)
+        scal = torch.empty(nch, h, 69, dtype=torch.float32, device=qkv.device)
         _call("gh_mlstm_chunks", 0, o, out if whole else None, S, m, ds, scal,
               qkv, gates, st.chunks, st.chunk_segs, norm, nch,
               st.chunk_segs.shape[0], h, dk, dv, ld, qscale, cap, vdim, eps)
@@ -478,7 +478,7 @@ def lightning(rows: torch.Tensor, S: torch.Tensor, decay: torch.Tensor,
     if not f and st.chunks is not None:
         nch = st.chunks.shape[0]
         ds = torch.empty(nch, h, dv, dk, dtype=torch.float32, device=dev)
-        scal = torch.empty(nch, h, 4, dtype=torch.float32, device=dev)
+        scal = torch.empty(nch, h, 69, dtype=torch.float32, device=dev)
         _call("gh_mlstm_chunks", 1, o, None, S, None, ds, scal, rows, decay[1],
               st.chunks, st.chunk_segs, None, nch, st.chunk_segs.shape[0], h,
               dk, dv, ld, 1.0, 0.0, 0, 0.0)

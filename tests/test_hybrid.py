@@ -839,7 +839,7 @@ def test_mlstm_chunk_sizes(dk, dv, entering):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads,dv", [(16, 256), (32, 192), (2, 256)])
-@pytest.mark.parametrize("kind", ["gla"])
+@pytest.mark.parametrize("kind", ["gla", "mlstm"])
 def test_states_of_many_chunks(kind, heads, dv):
     """Portions of one to four chunks, more and fewer blocks of the states than
     the chip has CUs, with columns that go into 128 and that do not."""
