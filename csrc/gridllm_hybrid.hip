@@ -1880,10 +1880,12 @@ DEV_INLINE f32x4 mfma_split(bf16x8 ah, bf16x8 al, bf16x8 bh, bf16x8 bl,
 // pair by pair. Outputs: a wave owns every fourth 16 columns for all 64 tokens,
 // so that the state is read once; decayed queries and scores meet in LDS. With
 // all of a head's columns here (out), the head's norm and gate follow at once.
-// Bound by reading the state (128 KB a head and chunk of 128 x 256) and the
-// latencies between its few steps. 590 blocks of it: 78 us with tokens split
-// over the waves, each reading the whole state, and 22 of the norm behind it;
-// now 64, of which the gates take 21 and the scores' decays 11.
+// Bound by its instructions: a block alone takes 17 us, a CU with two 35, and 540
+// blocks as many rounds as 720 do. 590 blocks of it: 78 us with tokens split over
+// the waves, each reading the whole state, and 22 of the norm behind it; then 64, of
+// which the gates take 21 and the scores' decays 11. With queries through LDS, and
+// places in LDS that are one register and a constant, 540 blocks 58 -> 54 us. Eight
+// waves a block with half the columns each: 70; registers for 3 blocks a CU: 54 to 67.
 #define GLA_SPAN 60.f
 __global__ void __launch_bounds__(256, 2)
 k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
@@ -1891,10 +1893,12 @@ k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
                 const float* __restrict__ b, const int4* __restrict__ chunks,
                 const float* __restrict__ norm, int H, int DK, int DV,
                 int ld_, float qscale, int dvtrue, float eps) {
+    // keys, queries and decayed queries, then values
     __shared__ __attribute__((aligned(16))) bf16_t vs[64 * 256];
     __shared__ __attribute__((aligned(16))) float bs[64 * 64];
-    __shared__ __attribute__((aligned(16))) bf16_t ks_[64 * 64];
-    __shared__ __attribute__((aligned(16))) bf16_t qs[2][64 * 64];
+    bf16_t* const ks_ = vs;
+    bf16_t* const qr = vs + 64 * 64;
+    bf16_t* const qs[2] = {vs + 2 * 64 * 64, vs + 3 * 64 * 64};
     const int4 ch = chunks[blockIdx.x];
     const int h = blockIdx.y, v0 = blockIdx.z * 256, nv = min(256, DV - v0);
     const int lane = threadIdx.x & 63;
@@ -1905,12 +1909,11 @@ k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
     const float* bh = b + (long)ch.x * C + h * DK;     // row t at t * C
     const bf16_t* qh = qkv + (long)ch.x * ld_ + h * DK;
     const bf16_t* kh = qh + C;
-    const int tq = min(r0 + fr, last), tr = min(r0 - 1, last);
-    const float* ref = r0 ? bh + tr * C : nullptr;
+    const float* ref = r0 ? bh + min(r0 - 1, last) * C : nullptr;
     const u32* Sb = (const u32*)dS + ((long)blockIdx.x * H + h) * DV * DK +
                     (long)(v0 + wid * 16 + fr) * DK + kg;
 
-    auto issue = [&](int k0) {         // b and keys of 64 channels
+    auto issue = [&](int k0) {         // b, queries and keys of 64 channels
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int pc = i * 256 + threadIdx.x, row = pc >> 4;
@@ -1921,37 +1924,21 @@ k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int pc = i * 256 + threadIdx.x, row = pc >> 3;
-            load_lds16(kh + (long)min(row, last) * ld_ + k0 +
-                           ((pc & 7) ^ (row & 7)) * 8,
-                       ks_ + (i * 256 + wid * 64) * 8);
+            const bf16_t* src = qh + (long)min(row, last) * ld_ + k0 +
+                                ((pc & 7) ^ (row & 7)) * 8;
+            load_lds16(src, qr + (i * 256 + wid * 64) * 8);
+            load_lds16(src + C, ks_ + (i * 256 + wid * 64) * 8);
         }
     };
-    uint4 st[2][4][2], qown[2], qall[2];
+    uint4 st[4][2];
     const int tall = threadIdx.x >> 2;
     auto load_state = [&](int k0, int ks, int c) {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-            st[ks][c][i] = *(const uint4*)(Sb + (long)c * 64 * DK + k0 +
+            st[c][i] = *(const uint4*)(Sb + (long)c * 64 * DK + k0 +
                                            ks * 32 + i * 4);
     };
-    auto load_queries = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            qown[i] = *(const uint4*)(qh + (long)tq * ld_ + k0 + i * 32 + kg);
-            qall[i] = *(const uint4*)(qh + (long)min(tall, last) * ld_ + k0 +
-                                      (threadIdx.x & 3) * 16 + i * 8);
-        }
-    };
     issue(0);
-    load_queries(0);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (c * 64 < nv) load_state(0, ks, c);
-    load_values(vs, qkv + (long)ch.x * ld_ + 2 * C + h * DV + v0, ld_, last,
-                nv);
-
     // ---- does a channel lose too much within these 16 tokens?
     float span = 0.f;
     for (int c = lane; c < DK; c += 64)
@@ -1978,44 +1965,45 @@ k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
             ld4(bs + at_f32(tall, c * 2), e);
             ld4(bs + at_f32(tall, c * 2 + 1), e + 4);
             bf16x8 hi, lo;
-            decayed8((const bf16_t*)&qall[i], e, hi, lo);
+            decayed8(qr + at_bf16(tall, c), e, hi, lo);
             *(bf16x8*)(qs[0] + at_bf16(tall, c)) = hi;
             *(bf16x8*)(qs[1] + at_bf16(tall, c)) = lo;
         }
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
             const int c = ks * 4 + gq;
+            // (rows behind the last hold its b; places in tiles of 16 rows)
+            const int b0 = at_f32(fr, c * 2), b1 = at_f32(fr, c * 2 + 1);
             float rf[8], e[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) rf[i] = 0.f;
             if (r0) {
-                ld4(bs + at_f32(tr, c * 2), rf);
-                ld4(bs + at_f32(tr, c * 2 + 1), rf + 4);
+                ld4(bs + at_f32(r0 - 1, c * 2), rf);
+                ld4(bs + at_f32(r0 - 1, c * 2 + 1), rf + 4);
             }
-            ld4(bs + at_f32(tq, c * 2), e);
-            ld4(bs + at_f32(tq, c * 2 + 1), e + 4);
+            ld4(bs + r0 * 64 + b0, e);
+            ld4(bs + r0 * 64 + b1, e + 4);
 #pragma unroll
             for (int i = 0; i < 8; ++i) e[i] -= rf[i];
             bf16x8 ah, al;
-            decayed8((const bf16_t*)&qown[ks], e, ah, al);
+            decayed8(qr + r0 * 64 + at_bf16(fr, c), e, ah, al);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 if (j > jmax) continue;
-                const int s = j * 16 + fr;
-                ld4(bs + at_f32(s, c * 2), e);
-                ld4(bs + at_f32(s, c * 2 + 1), e + 4);
+                ld4(bs + j * 1024 + b0, e);
+                ld4(bs + j * 1024 + b1, e + 4);
 #pragma unroll
                 for (int i = 0; i < 8; ++i) e[i] = rf[i] - e[i];
                 bf16x8 th, tl;
-                decayed8(ks_ + at_bf16(s, c), e, th, tl);
+                decayed8(ks_ + j * 1024 + at_bf16(fr, c), e, th, tl);
                 sc[j] = mfma_split(ah, al, th, tl, sc[j]);
             }
         }
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (c * 64 < nv) load_state(k0, 0, c);
         lds_barrier();
-        if (k0 + 64 < DK) {
-            issue(k0 + 64);
-            load_queries(k0 + 64);
-        }
+        if (k0 + 64 < DK) issue(k0 + 64);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
             bf16x8 hi[4], lo[4];
@@ -2030,8 +2018,8 @@ k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
             for (int c = 0; c < 4; ++c) {
                 if (c * 64 >= nv) continue;
                 bf16x8 sh, sl;
-                split8((const u32*)st[ks][c], sh, sl);
-                if (k0 + 64 < DK) load_state(k0 + 64, ks, c);
+                split8((const u32*)st[c], sh, sl);
+                if (ks == 0) load_state(k0, 1, c);
 #pragma unroll
                 for (int rt = 0; rt < 4; ++rt)
                     acc[c][rt] = mfma_split(sh, sl, hi[rt], lo[rt],
@@ -2067,7 +2055,9 @@ k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
     if (out)
         load_gates(gates, qkv + (long)ch.x * ld_ + 2 * C + (long)H * DV + h * DV,
                    ld_, last, DV);
-    // (the b of all waves' scores is no longer needed)
+    lds_barrier();                     // keys, queries and b have been read
+    load_values(vs, qkv + (long)ch.x * ld_ + 2 * C + h * DV + v0, ld_, last,
+                nv);
     bf16_t* const ph = (bf16_t*)bs;
     bf16_t* const pl = ph + 64 * 64;
 #pragma unroll
@@ -2088,7 +2078,8 @@ k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
         for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[c][rt][r] *= qscale;
-    __syncthreads();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
     // the chunk's own values
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
@@ -2114,8 +2105,9 @@ k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
         }
     }
     if (out) {
+        lds_barrier();                 // scores have been read
         store_normed<true>(
-            out + ((long)ch.x * H + h) * DV, acc, (float*)qs, gates,
+            out + ((long)ch.x * H + h) * DV, acc, bs, gates,
             (long)H * DV, norm + h * DV, ch.y, DV, dvtrue, eps);
         return;
     }
