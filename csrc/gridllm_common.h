@@ -85,6 +85,24 @@ DEV_INLINE void st4(bf16_t* p, const float* f) {
                             (u32)f2bf(f[2]) | ((u32)f2bf(f[3]) << 16));
 }
 DEV_INLINE void st4(float* p, const float* f) { *(float4*)p = *(const float4*)f; }
+// 8 columns of a product's output that is still f32 partial sums [parts][N][W] (K
+// in parts): added up, and rounded as the product's result would be. Spares that
+// product's second launch.
+DEV_INLINE void summed8(const float* y, int parts, long n, long N, int W, int c,
+                        float* v) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = 0.f;
+#pragma unroll 4
+    for (int k = 0; k < parts; ++k) {
+        float f[8];
+        ld8(y + (k * N + n) * W + c, f);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] += f[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = bf2f(f2bf(v[i]));
+}
+
 // The hardware's reciprocal (1 ulp) and a Newton step, which came out as an exact
 // division does for 12 M arguments, in 0.82 of its time. (An infinite sum would
 // leave NaN; a NaN has to come through.)

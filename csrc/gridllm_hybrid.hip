@@ -102,24 +102,6 @@ DEV_INLINE void sublayer8(const T* y, const float* wt, int top, long n, int W,
     }
 }
 
-// 8 columns of a sublayer's output that is still f32 partial sums [parts][N][W]
-// of its last product (K in parts): added up, and rounded as the product's result
-// would be. Spares that product's second launch.
-DEV_INLINE void summed8(const float* y, int parts, long n, long N, int W, int c,
-                        float* v) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = 0.f;
-#pragma unroll 4
-    for (int k = 0; k < parts; ++k) {
-        float f[8];
-        ld8(y + (k * N + n) * W + c, f);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] += f[i];
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = bf2f(f2bf(v[i]));
-}
-
 // What y is: a sublayer's output, a row per (token, expert), or partial sums
 enum { PLAIN, PAIRS, PARTS };
 

@@ -63,10 +63,13 @@ DEV_INLINE void key8(float* f, const T* v, float r, const float* w, int c,
 // ===========================================================================
 // From a projection row [H*P q | G*P k | ...], stride ld, without its bias:
 // normed and rotated q [N][H][P], and the cached rows. P / 8 lanes per head.
+// PARTS: rows are f32 partial sums of the projection [parts][N][ld]. Bound by its
+// launch: 160 rows of 4096 with 2 parts 4.9 us, and 4.7 for a kernel ahead of it
+// that adds them up; both in one are 4.9.
 // ===========================================================================
-template <class T>
+template <class T, bool PARTS>
 __global__ void __launch_bounds__(256)
-k_talk_rows(const T* __restrict__ rows, T* __restrict__ q,
+k_talk_rows(const void* __restrict__ rows, int parts, T* __restrict__ q,
             T* __restrict__ vc, float* __restrict__ inv,
             const int* __restrict__ table, int per_slot,
             const int* __restrict__ pos, const int* __restrict__ slot,
@@ -79,7 +82,10 @@ k_talk_rows(const T* __restrict__ rows, T* __restrict__ q,
     const int hd = (int)(item % (H + G));
     const int c = (int)(threadIdx.x % sub) * 8;
     float f[8], g[8];
-    ld8(rows + (long)n * ld_ + hd * P + c, f);
+    if (PARTS)
+        summed8((const float*)rows, parts, n, N, ld_, hd * P + c, f);
+    else
+        ld8((const T*)rows + (long)n * ld_ + hd * P + c, f);
     ld8(bias + hd * P + c, g);
     float ss = 0.f;
 #pragma unroll
@@ -1120,20 +1126,23 @@ static int go_decode(hipStream_t st, bf16_t* out, const bf16_t* q,
 
 extern "C" {
 
-int gt_talk_rows(void* stream, int f32, const void* rows, void* q, void* vc,
-                 void* inv, const void* table, int per_slot, const void* pos,
+// parts > 0: rows are f32 partial sums [parts][N][ld_], q and vc bf16
+int gt_talk_rows(void* stream, int f32, const void* rows, int parts, void* q,
+                 void* vc, void* inv, const void* table, int per_slot, const void* pos,
                  const void* slot, const void* bias, const void* qw,
                  const void* cos_, const void* sin_, int nrot, int N, int H,
                  int G, int P, int R, int ld_, int dim, float eps) {
     if (N < 1 || !sizes_ok(H, G, P, R, nrot, 1) || dim < 1 || dim > P ||
-        ld_ < (H + G) * P || ld_ % 8) return -100;
+        ld_ < (H + G) * P || ld_ % 8 || parts < 0 || (f32 && parts)) return -100;
     const Rotation rot = rotation(cos_, sin_, R, nrot);
     const long threads = (long)N * (H + G) * (P / 8);
-#define GO(T) k_talk_rows<T><<<(unsigned)((threads + 255) / 256), 256, 0, \
-        (hipStream_t)stream>>>((const T*)rows, (T*)q, (T*)vc, (float*)inv, \
+#define GO(T, PARTS) k_talk_rows<T, PARTS><<<(unsigned)((threads + 255) / 256), \
+        256, 0, (hipStream_t)stream>>>(rows, parts, (T*)q, (T*)vc, (float*)inv, \
         (const int*)table, per_slot, (const int*)pos, (const int*)slot, \
         (const float*)bias, (const float*)qw, rot, N, H, G, P, ld_, dim, eps)
-    if (f32) GO(float); else GO(bf16_t);
+    if (f32) GO(float, false);
+    else if (parts) GO(bf16_t, true);
+    else GO(bf16_t, false);
 #undef GO
     LAUNCH_CHECK();
     return 0;

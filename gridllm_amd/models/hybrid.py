@@ -594,10 +594,10 @@ class HybridModel:
 
     def joined_shapes(self) -> set:
         """Those of the projections whose parts of K the next kernel adds up."""
-        if not self._parts_added():
-            return set()
         return {tuple(t.shape) for w in self.unique_layers()
-                for t in (w.wo, w.down) if t is not None and t.dim() == 2}
+                for t in ((w.wo, w.down) if self._parts_added() else ()) +
+                ((w.wmix,) if w.talk is not None else ())
+                if t is not None and t.dim() == 2}
 
     def interleave_gateup(self) -> None:
         """Gate and up rows in groups of 64 | 64, the layout of the fused
@@ -647,7 +647,8 @@ class HybridModel:
              ) -> Optional[torch.Tensor]:
         """A mixer's output, or its rows `only` (None if there are none)."""
         c, eps = self.cache, self.spec.norm_eps
-        rows = _linear(xb, w.wmix, st.whole)
+        rows = (_linear_parts if isinstance(mx, TalkingMixer) else _linear)(
+            xb, w.wmix, st.whole)
         if isinstance(mx, ParallelMixer):
             o = torch.empty(xb.shape[0], w.wo.shape[1], dtype=xb.dtype,
                             device=xb.device)

@@ -65,7 +65,7 @@ _SIGS = {
     "gn_latent_attn_f32": "pppppippppiiiiiif",
     "gn_latent_gather": "pppipii",
     "gn_latent_prefill": "ppppipippiiiifpi",
-    "gt_talk_rows": "ipppppippppppiiiiiiiif",
+    "gt_talk_rows": "ipippppippppppiiiiiiiif",
     "gt_talk_decode": "pppppippppppp" + "iiiiiiiifff",
     "gt_talk_gather": "pppppipppipiiii",
     "gt_talk_lse": "ppppiiiiifff",
@@ -701,18 +701,22 @@ def gla(rows: torch.Tensor, u: torch.Tensor, wa2: torch.Tensor,
 
 def talk_rows(rows: torch.Tensor, vc: torch.Tensor, inv: torch.Tensor,
               st: StepMeta, tk: Talk, eps: float) -> torch.Tensor:
-    """From projection rows [q H*P | k G*P | ...] without their bias: normed and
-    rotated queries [n, H, P]; k goes to the pages of vc [pages, G, 64, P], and
-    1 / rms(k) to inv f32 [pages, G, 64]."""
-    n, ld = rows.shape
+    """From projection rows [q H*P | k G*P | ...] without their bias, or f32
+    partial sums of bf16 ones [parts, n, ..]: normed and rotated queries [n, H, P];
+    k goes to the pages of vc [pages, G, 64, P], and 1 / rms(k) to inv f32
+    [pages, G, 64]."""
+    n, ld = rows.shape[-2:]
+    parts = rows.shape[0] if rows.dim() == 3 else 0
+    assert not parts or (rows.dtype, vc.dtype) == (torch.float32, torch.bfloat16)
     h, (g, _, p) = tk.heads, vc.shape[1:]
     _dense(rows, vc, inv, st.table, tk.bias, tk.qnorm, *tk.rot)
     assert ld >= (h + g) * p and tk.bias.shape == ((h + g) * p,)
     assert inv.shape == vc.shape[:3] and tk.qnorm.shape == (p,)
     _check_range("talk_rows.slot", st.slot, st.table.shape[0])
-    q = torch.empty(n, h, p, dtype=rows.dtype, device=rows.device)
-    _call("gt_talk_rows", _f32(rows), rows, q, vc, inv, st.table,
-          st.table.shape[1], st.pos, st.slot, tk.bias, tk.qnorm, *tk.rot,
+    q = torch.empty(n, h, p, dtype=vc.dtype if parts else rows.dtype,
+                    device=rows.device)
+    _call("gt_talk_rows", not parts and _f32(rows), rows, parts, q, vc, inv,
+          st.table, st.table.shape[1], st.pos, st.slot, tk.bias, tk.qnorm, *tk.rot,
           tk.rot[0].shape[0], n, h, g, p, 2 * tk.rot[0].shape[1], ld, tk.dim,
           eps)
     return q

@@ -328,6 +328,32 @@ def test_rotation_far_out(run):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,parts", [(1, 2), (5, 3), (33, 8)])
+def test_rows_in_parts(n, parts):
+    """Partial sums of a projection against the sums that it would have stored."""
+    m = build(config((attn(9, 3, 20, 70, 6, 1e4), None)), ("cuda", "bf16"),
+              max_seq=200)
+    c, tk = m.cache, m.layers[0].talk
+    g = torch.Generator().manual_seed(n)
+    ps = torch.randn(parts, n, m.layers[0].wmix.shape[0], generator=g).cuda()
+    rows = torch.zeros_like(ps[0])
+    for part in ps:                    # in the kernels' order
+        rows = rows + part
+    slot = c.alloc(n)
+    c.extend([slot], [n])
+    st = hops.StepMeta(nd=n, pos=torch.arange(n, dtype=torch.int32).cuda(),
+                       slot=torch.full((n,), slot, dtype=torch.int32).cuda(),
+                       table=c.table, max_len=n)
+    got = []
+    for r in (rows.to(torch.bfloat16), ps):
+        c.v[0].zero_(), c.inv[0].zero_()
+        got.append([hops.talk_rows(r, c.v[0], c.inv[0], st, tk, 1e-5),
+                    c.v[0].clone(), c.inv[0].clone()])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    assert bool(got[0][1].any())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 7, 60, 224])
 @pytest.mark.parametrize("sizes", [(24, 8, 128, 4096, 64), (9, 3, 20, 70, 6),
                                    (9, 3, 20, 130, 6), (40, 1, 64, 333, 64)])
