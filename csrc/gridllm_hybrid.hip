@@ -253,14 +253,15 @@ struct Groups {
     int count, size;
 };
 
-// v holds columns c .. c + 7 of j = 0 .. 3; factors 1 / rms by group into rs
-template <int GR>
-DEV_INLINE void group_factors(const float v[4][8], float* part, float* rs,
+// v holds a thread's columns, 8 from (j * threads + its number) * 8 on for each j;
+// factors 1 / rms by group into rs
+template <int NV, int GR>
+DEV_INLINE void group_factors(const float (&v)[NV][8], float* part, float* rs,
                               int W, const Groups gp, float eps) {
     __syncthreads();                       // part and rs are free
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int c = (j * 256 + threadIdx.x) * 8;
+    for (int j = 0; j < NV; ++j) {
+        const int c = (j * blockDim.x + threadIdx.x) * 8;
         if (c < W)
 #pragma unroll
             for (int i = 0; i < 8; i += GR) {
@@ -272,7 +273,7 @@ DEV_INLINE void group_factors(const float v[4][8], float* part, float* rs,
     }
     __syncthreads();
     const int lane = threadIdx.x & 63, n = gp.size / GR;
-    for (int g = threadIdx.x >> 6; g < gp.count; g += 4) {
+    for (int g = threadIdx.x >> 6; g < gp.count; g += blockDim.x >> 6) {
         float s = 0.f;
         for (int i = lane; i < n; i += 64) s += part[g * n + i];
         s = wave_reduce_sum(s);
@@ -283,7 +284,7 @@ DEV_INLINE void group_factors(const float v[4][8], float* part, float* rs,
 
 // f *= rs of each column's group
 template <int GR>
-DEV_INLINE void scale_groups(float* f, const float* rs, int c,
+DEV_INLINE void scale_groups(float (&f)[8], const float* rs, int c,
                              const Groups gp) {
 #pragma unroll
     for (int i = 0; i < 8; i += GR) {
@@ -293,9 +294,12 @@ DEV_INLINE void scale_groups(float* f, const float* rs, int c,
     }
 }
 
-// parts > 0: y is f32 partial sums
-template <class T, bool ADD, int GR>
-__global__ void __launch_bounds__(256)
+// parts > 0: y is f32 partial sums. A thread has 8 NV columns, and all its loads are
+// on their way at once. Bound by these and by the sums' steps: 160 rows of 3072 with 2
+// and 8 parts 7.6 us with 256 threads a row and weights read after the sums, now
+// 5.7.
+template <class T, bool ADD, int GR, int NV>
+__global__ void __launch_bounds__(512)
 k_group_norm(T* __restrict__ out, float* __restrict__ x,
              const void* __restrict__ y, int parts,
              const int* __restrict__ rows,
@@ -304,48 +308,41 @@ k_group_norm(T* __restrict__ out, float* __restrict__ x,
     extern __shared__ float part[];        // W / GR, then a factor per group
     float* const rs = part + W / GR;
     const long n = !ADD && rows ? rows[blockIdx.x] : blockIdx.x;
-    float v[4][8], a[4][8];
+    float v[NV][8], a[NV][8], gy[NV][8], g[NV][8];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int c = (j * 256 + threadIdx.x) * 8;
-        if (c < W) {
-            ld8(x + n * W + c, a[j]);
-            if (ADD) {
-                if (parts)
-                    summed8((const float*)y, parts, n, gridDim.x, W, c, v[j]);
-                else
-                    ld8((const T*)y + n * W + c, v[j]);
-            }
-        }
+    for (int j = 0; j < NV; ++j) {
+        const int c = (j * blockDim.x + threadIdx.x) * 8;
+        if (c >= W) continue;
+        ld8(x + n * W + c, a[j]);
+        if (ADD) ld8(wy + c, gy[j]);
+        if (out) ld8(w + c, g[j]);
+        if (ADD && parts)
+            summed8((const float*)y, parts, n, gridDim.x, W, c, v[j]);
+        else if (ADD)
+            ld8((const T*)y + n * W + c, v[j]);
     }
     if (ADD) {
-        group_factors<GR>(v, part, rs, W, gp, eps);
+        group_factors<NV, GR>(v, part, rs, W, gp, eps);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int c = (j * 256 + threadIdx.x) * 8;
-            if (c < W) {
-                float g[8];
-                ld8(wy + c, g);
-                scale_groups<GR>(v[j], rs, c, gp);
+        for (int j = 0; j < NV; ++j) {
+            const int c = (j * blockDim.x + threadIdx.x) * 8;
+            if (c >= W) continue;
+            scale_groups<GR>(v[j], rs, c, gp);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) a[j][i] += v[j][i] * g[i];
-                st8(x + n * W + c, a[j]);
-            }
+            for (int i = 0; i < 8; ++i) a[j][i] += v[j][i] * gy[j][i];
+            st8(x + n * W + c, a[j]);
         }
         if (!out) return;
     }
-    group_factors<GR>(a, part, rs, W, gp, eps);
+    group_factors<NV, GR>(a, part, rs, W, gp, eps);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int c = (j * 256 + threadIdx.x) * 8;
-        if (c < W) {
-            float g[8];
-            ld8(w + c, g);
-            scale_groups<GR>(a[j], rs, c, gp);
+    for (int j = 0; j < NV; ++j) {
+        const int c = (j * blockDim.x + threadIdx.x) * 8;
+        if (c >= W) continue;
+        scale_groups<GR>(a[j], rs, c, gp);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) a[j][i] *= g[i];
-            st8(out + (long)blockIdx.x * W + c, a[j]);
-        }
+        for (int i = 0; i < 8; ++i) a[j][i] *= g[j][i];
+        st8(out + (long)blockIdx.x * W + c, a[j]);
     }
 }
 
@@ -2769,7 +2766,12 @@ int gh_group_norm(void* stream, int f32, void* out, void* x, const void* y,
     const int lds = (W / gr + groups) * 4;
     if (lds > 64 * 1024) return -100;
     const Groups gp{groups, size};
-#define GO(T, A, B) k_group_norm<T, A, B><<<N, 256, lds, \
+    // (1024 threads for a row of 6144: 160 rows 5.8 and not 6.1 us, 4096 rows 70 and
+    // not 53; before 7.8 and 52)
+    const int threads = W <= 2048 ? 256 : 512;
+#define GO(T, A, B) do { if (W <= 4096) GON(T, A, B, 1); else GON(T, A, B, 2); \
+        } while (0)
+#define GON(T, A, B, NV) k_group_norm<T, A, B, NV><<<N, threads, lds, \
         (hipStream_t)stream>>>((T*)out, (float*)x, y, parts, \
         (const int*)rows, (const float*)wy, (const float*)w, W, gp, eps)
 #define PICK(T, A) do { if (gr == 8) GO(T, A, 8); else if (gr == 4) \
@@ -2778,6 +2780,7 @@ int gh_group_norm(void* stream, int f32, void* out, void* x, const void* y,
     if (f32) { if (y) PICK(float, true); else PICK(float, false); }
     else { if (y) PICK(bf16_t, true); else PICK(bf16_t, false); }
 #undef PICK
+#undef GON
 #undef GO
     LAUNCH_CHECK();
     return 0;
