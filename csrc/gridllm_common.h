@@ -133,12 +133,16 @@ DEV_INLINE float log_sigmoid(float z) {
     return (z > 0.f ? 0.f : z) - 2.f * (q + fmaf(q * q2, p, rest));
 }
 
-// sum over a block of 256 threads; every thread gets it
+// sum over a block of THREADS threads; every thread gets it
+template <int THREADS = 256>
 DEV_INLINE float block_sum(float v, float* red) {
     v = wave_reduce_sum(v);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    return red[0] + red[1] + red[2] + red[3];
+    v = red[0];
+#pragma unroll
+    for (int i = 1; i < THREADS / 64; ++i) v += red[i];
+    return v;
 }
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
