@@ -2463,8 +2463,12 @@ k_moe_gemm(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
 // columns, blocks of one a CU that take them in turn. 4096 tokens, 64 experts of 3072
 // x 1024, 8 of them chosen 621 -> 493 us for both products (840 TFLOP/s; the tile
 // lists' last tiles are half empty), gated, 7 762 -> 575; bound as k_gemm_wide.
+// ONCE: tiles of 128 rows are for experts that mostly have one. 150, 256, 512 and 700
+// tokens of 64 experts, 8 of them chosen, us: 162, 169, 184 and 192 with weights that
+// stay in the Infinity Cache, 147, 152, 165 and 167 with such that go past it.
+template <bool O>
 struct ExpertRows {
-    static constexpr bool GATHER = true;
+    static constexpr bool GATHER = true, ONCE = O;
     const int* sorted;
     const float* pw;
     int top;                       // up: x's rows are tokens'; 0: down
@@ -2487,7 +2491,7 @@ k_moe_wide(const WideArgs p, const int4* __restrict__ tiles,
         (int)(gridDim.x >> 3), [&](int it) {
             const int4 tl = tiles[it / cb];
             return WideTile{tl.y, tl.y + tl.z, it % cb * S::C, tl.x * p.N};
-        }, experts * p.N, ExpertRows{sorted, pw, ACT ? top : 0});
+        }, experts * p.N, ExpertRows<S::R == 128>{sorted, pw, ACT ? top : 0});
 }
 
 // A few rows: up to 16 against 16 columns per block, K split over the 4 waves,

@@ -58,9 +58,10 @@ struct WideTile {
     int m0, end, n0, w0;
 };
 
-// Where rows come from and go to. GATHER: x's rows are looked up one by one.
+// Where rows come from and go to. GATHER: x's rows are looked up one by one. ONCE: W's
+// are read once, and past the Infinity Cache.
 struct DenseRows {
-    static constexpr bool GATHER = false;
+    static constexpr bool GATHER = false, ONCE = false;
     DEV_INLINE int from(int m) const { return m; }
     DEV_INLINE long to(int m) const { return m; }
     DEV_INLINE float weight(int m) const { return 1.f; }
@@ -146,7 +147,7 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
         if (i * 64 < R)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, dst, 16, vx[i % GX],
                                                      so[i], 0, 0);
-        else if (EPI == 2)
+        else if (EPI == 2 || Rows::ONCE)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, dst, 16, v, so[i], 0, 2);
         else
             __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, dst, 16, v, so[i], 0, 0);
