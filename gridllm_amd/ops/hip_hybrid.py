@@ -494,10 +494,11 @@ def _expert_rows(pairs: int, experts: int, wide: tuple = ()) -> int:
     waves, while the pairs are mostly of different experts; 32 while most experts
     have no more, whose blocks load less beside the weights; else 128. In us with
     16, 32 and 128, 64 experts, of which 8 are chosen: 1 row 35, 42, 60; 8 111, 115,
-    119; 16 142, 140, 147; 48 183, 155, 160; 128 275, 158, 167; 192 -, 180, 170;
-    and gated, of which 7 are: 2 65, 60, 78; 6 137, 145, 173; 12 178, 168, 199; 24
-    223, 204, 216; 128 340, 223, 233; 192 -, 228, 237; 256 -, 248, 244. (64 rows are
-    at best 2 % faster than the better of 32 and 128.)
+    119; 16 142, 140, 147; and gated, of which 7 are: 2 65, 60, 78; 6 137, 145, 173;
+    12 178, 168, 199; with weights past the Infinity Cache 32 and 128: 48 rows 130,
+    138; 128 135, 143; 160 138, 144; 192 161, 148; gated 128 193, 201; 192 199, 205; 256
+    236, 212 (so 32 would be 3 to 5 % faster up to 22 pairs an expert; before, both
+    read at one rate there). 64 rows are at best 2 % faster than the better of the two.
     wide: ((N, K), ..) of the products if k_moe_wide takes them. Its tiles are of 256
     columns, and of the rows that the rounds of CUs take least with, times a tile's
     time (kWide's), were the pairs spread by chance: a few experts with a tile more
