@@ -1187,9 +1187,9 @@ k_mlstm_weights(float* __restrict__ w, float* __restrict__ scal,
     }
 }
 
-// The state that enters each chunk of a prompt portion, left in dS as (hi | lo << 16) bf16 pairs; the
-// slot's state is advanced. Block = (segment, head, 32 key channels and 64 value
-// NK * 64 value columns), and the state stays in registers from chunk to chunk: a
+// The state that enters each chunk of a prompt portion, left in dS as (hi | lo << 16)
+// bf16 pairs; the slot's state is advanced. Block = (segment, head, 32 key channels
+// and NK * 64 value columns), and the state stays in registers from chunk to chunk: a
 // wave has NK * 16 by 16. A chunk's operands are loaded two chunks ahead.
 // Bound by a step's instructions and latencies (.8 us a chunk) where a segment is
 // long, by the stores where there are many. 45 chunks of 4 segments, 12 heads of 128
