@@ -954,7 +954,8 @@ DEV_INLINE float bounded(u32 h, float c) {
 // between calls: the largest pick, as a number whose order is that of better(), and how many
 // there have been. The last block stores the row's token and counts its draw. All that
 // blocks tell each other goes through these atomics, a block's second one behind the
-// answer to its first, so that there is nothing to release.
+// answer to its first, so that there is nothing to release. A slot is in one call at a
+// time, as its draws are.
 #define MARK 16
 DEV_INLINE void meet(const Pick p, int* token, unsigned long long* mark,
                      long long* draws, int blocks) {
@@ -970,6 +971,39 @@ DEV_INLINE void meet(const Pick p, int* token, unsigned long long* mark,
     }
     *token = best ? ~(u32)best : 0;                      // all -inf -> 0
     *draws += 1;
+}
+
+// Rows that name one slot can neither meet in its mark nor count its draw before the
+// others have read it: a block takes all of them, one after the other, each element by
+// its exact value. Others leave them.
+DEV_INLINE void sample_same(int* out, const float* logits, const SampleKeys& how,
+                            int row, int rows, int v, Pick* part) {
+    const long long slot = how.slots[row];
+    for (int r = 0; r < row; ++r)
+        if (how.slots[r] == slot) return;
+    const unsigned long long key = how.key(row);
+    const float t = how.temp(row);
+    for (int r = row; r < rows; ++r) {
+        if (how.slots[r] != slot) continue;
+        Pick best{-INFINITY, 2147483647};
+        for (int i = threadIdx.x; i < v; i += 256) {
+            float val = logits[(long)r * v + i] / t;
+            if (key != 0ull)
+                val += -logf(-logf(noise_of(
+                    hash_of(((unsigned long long)i ^ key) * NOISE))));
+            if (better(val, i, best)) best = Pick{val, i};
+        }
+        best = wave_pick(best);
+        if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = best;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int k = 1; k < 4; ++k)
+                if (better(part[k].val, part[k].at, best)) best = part[k];
+            out[r] = best.at == 2147483647 ? 0 : best.at;
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) how.draws[slot] += 1;
 }
 
 // Candidates of a lane: 4 that follow each other in each of two chunks of 256.
@@ -1004,6 +1038,11 @@ k_sample_gumbel(Pick* __restrict__ ws, int* __restrict__ out,
     load(first, ahead);                // (no later than the row's slot)
     if (how.slots && (unsigned long long)how.slots[row] >= how.count)
         __builtin_trap();
+    const int rows = (int)gridDim.x / segments;
+    bool same = false;                 // another row has the slot
+    if (marks)
+        for (int r = threadIdx.x; r < rows; r += 256)
+            same |= r != row && how.slots[r] == how.slots[row];
     const unsigned long long key = how.key(row);
     const float t = how.temp(row), rt = 1.f / t;
     unsigned long long low[4];
@@ -1083,9 +1122,18 @@ k_sample_gumbel(Pick* __restrict__ ws, int* __restrict__ out,
     };
     __shared__ float bound[4];
     __shared__ Pick part[4];
+    __shared__ int twice[4];
     float top = max_across16(max_of16(most));
-    if (lane == 0) bound[wid] = top;
+    same = __any(same);
+    if (lane == 0) {
+        bound[wid] = top;
+        twice[wid] = same;
+    }
     __syncthreads();
+    if (twice[0] | twice[1] | twice[2] | twice[3]) {
+        if (seg == 0) sample_same(out, logits, how, row, rows, v, part);
+        return;
+    }
     top = fmaxf(fmaxf(bound[0], bound[1]), fmaxf(bound[2], bound[3]));
     const bool near = !(most < top - 0.1f - 1e-5f * fabsf(top));
     // first the batches next to the largest bound; the best of these says what else

@@ -793,8 +793,9 @@ def sample_gumbel_slots(logits: torch.Tensor, slots: torch.Tensor,
     different; temps f32, seeds, draws, nongreedy i64): the keys are made in the
     kernel, and the slots' draws advance by one. A slot that there is not ends the
     program, as an index out of bounds does in torch. marks: i64 [slots, 16] of zeros,
-    which stay zeros between calls and belong to the slots as their draws do: one
-    launch instead of two."""
+    which stay zeros between calls and belong to the slots as their draws do (a slot is
+    in one call at a time): one launch instead of two. (Rows with one slot get that
+    slot's key, too, but slowly.)"""
     return _sample(logits, None, temps, slots, seeds, draws, nongreedy, marks)
 
 

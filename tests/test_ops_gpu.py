@@ -608,6 +608,31 @@ def test_sample_gumbel_marks(dev, b, v):
         hip_ops.sample_gumbel_slots(x, slots, temps, seeds, draws, live, marks[1:])
 
 
+@pytest.mark.parametrize("b,v", [(2, 1), (3, 2047), (5, 128256), (40, 8195),
+                                 (600, 4352)])
+def test_sample_gumbel_slots_twice(dev, b, v):
+    """Rows that name one slot get its key each, as without marks, and the marks and
+    the other rows' tokens are what they are without such rows."""
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator().manual_seed(b + v)
+    x = (torch.randn(b, v, generator=g) * 2).to(dev)
+    temps = (torch.rand(b, generator=g) + 0.3).to(dev)
+    seeds = torch.randint(0, 2 ** 62, (b,), generator=g).to(dev)
+    live = (torch.arange(b) % 4 != 3).long().to(dev)
+    slots = torch.randperm(b, generator=g)
+    slots[b // 2], slots[-1] = slots[0], slots[b // 3]
+    count = torch.zeros(b, dtype=torch.int64)
+    count[slots] = 1
+    keys = (seeds * 6364136223846793005 + 1442695040888963407) & ((1 << 63) - 1)
+    slots = slots.to(dev)
+    want = hip_ops.sample_gumbel(x, (keys * live)[slots], temps[slots])
+    draws, marks = torch.zeros_like(seeds), torch.zeros(b, 16, dtype=torch.int64,
+                                                        device=dev)
+    got = hip_ops.sample_gumbel_slots(x, slots, temps, seeds, draws, live, marks)
+    assert torch.equal(got, want)
+    assert torch.equal(draws.cpu(), count) and not marks.any()
+
+
 @pytest.mark.parametrize("b,v", [(7, 256), (5, 257), (3, 511), (4, 512), (2, 2049),
                                  (3, 4096), (2, 6400), (1, 133000), (600, 4352)])
 def test_sample_gumbel_chunks(dev, b, v):
