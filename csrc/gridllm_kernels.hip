@@ -875,15 +875,21 @@ static void launch_gemm_skinny(hipStream_t st, bf16_t* out, float* ws,
 // too; their picks meet in the slot's marks, or a second kernel picks among them.
 // Bound by the vector unit: the hash's second product (three of 32 bits: its upper
 // half is what is used; the first one is a sum, see hash_of), beside which all that
-// is done for each element is a bound of its noise, one logarithm by the hardware.
-// What a block then looks at are the batches of 8 whose largest bound is next to its
-// largest, and after these whatever is not below the best of them: exactly, but for
-// elements that the hardware's two logarithms put clearly behind. The picked one is
-// among them. Rows of 128256, us with two logarithms for each element, exact values
-// in each step of a wave and a second kernel, and now: 1 row 13.3, 10.0 (what a call
-// costs the host), 20 15.2, 12.4, 64 20.4, 17.6, 149 33.4, 25.7, 512 82.5, 58.4. Of 64
-// rows' 17.6 some 10 are a launch, the loads of a key, the exact values and the two
-// atomics of a block; slots' marks in one line had 20 rows take 17.3.
+// is done for each element of a long segment is a bound of its noise, one logarithm by
+// the hardware. What a block then looks at are the batches of 8 whose largest bound is
+// next to its largest, and after these whatever is not below the best of them: exactly,
+// but for elements that the hardware's two logarithms put clearly behind. The picked one
+// is among them. A segment of three batches a lane or less is looked at right away:
+// bounds are two meetings of the block more (in a graph, us, looked at and with bounds:
+// 1 row 7.2, 9.3, 20 11.1, 13.3, 34 13.7, 14.5, 40 15.3, 15.3; two kernels that look at
+// all 8.3, 11.2, 13.3, 14.5). Rows of 128256, us, with two logarithms for each element,
+// exact values in each step of a wave and a second kernel, and now: 64 rows 18.3, 17.8,
+// 149 33.9, 26.9, 512 80.6, 57.6; called one by one, 1 row 13.3, 10.0 (the host's time).
+// Masked candidates cost no logarithm: 20, 64 and 512 rows of one candidate 10.7, 15.8
+// and 56 (13.8, 25.4 and 142 with exact values of all; bounds alone, behind which all of
+// a masked segment was looked at, 26.6, 45 and 257). Of 64 rows' 17.8 some 10 are a
+// launch, the loads of a key, the exact values and the two atomics of a block, and .3 the
+// look for rows of the same slot; slots' marks in one line had 20 rows take 5 more.
 // ===========================================================================
 struct Pick {
     float val;
@@ -973,6 +979,12 @@ DEV_INLINE void meet(const Pick p, int* token, unsigned long long* mark,
     *draws += 1;
 }
 
+// What is clearly less than x, which may be infinite.
+DEV_INLINE float below(float x, float by) {
+    x = fminf(x, 3e38f);
+    return x - by - 1e-5f * fabsf(x);
+}
+
 // Rows that name one slot can neither meet in its mark nor count its draw before the
 // others have read it: a block takes all of them, one after the other, each element by
 // its exact value. Others leave them.
@@ -999,7 +1011,7 @@ DEV_INLINE void sample_same(int* out, const float* logits, const SampleKeys& how
         if (threadIdx.x == 0) {
             for (int k = 1; k < 4; ++k)
                 if (better(part[k].val, part[k].at, best)) best = part[k];
-            out[r] = best.at == 2147483647 ? 0 : best.at;
+            out[r] = best.val == -INFINITY ? 0 : best.at;
         }
         __syncthreads();
     }
@@ -1036,13 +1048,10 @@ k_sample_gumbel(Pick* __restrict__ ws, int* __restrict__ out,
     const int first = i0 + wid * 512;
     float f[E], ahead[E];
     load(first, ahead);                // (no later than the row's slot)
-    if (how.slots && (unsigned long long)how.slots[row] >= how.count)
-        __builtin_trap();
-    const int rows = (int)gridDim.x / segments;
-    bool same = false;                 // another row has the slot
-    if (marks)
-        for (int r = threadIdx.x; r < rows; r += 256)
-            same |= r != row && how.slots[r] == how.slots[row];
+    const long long slot = how.slots ? how.slots[row] : 0;
+    if (how.slots && (unsigned long long)slot >= how.count) __builtin_trap();
+    const int rows = (int)gridDim.x / segments, r0 = min((int)threadIdx.x, rows - 1);
+    const long long other = marks ? how.slots[r0] : 0;  // (looked at later)
     const unsigned long long key = how.key(row);
     const float t = how.temp(row), rt = 1.f / t;
     unsigned long long low[4];
@@ -1057,7 +1066,10 @@ k_sample_gumbel(Pick* __restrict__ ws, int* __restrict__ out,
     // bounds of all: a lane's largest batch, and the largest of its other ones
     float most = -INFINITY, next = -INFINITY;
     int at_most = first;
-    for (int base = first; base < i1; base += 2048) {
+    const bool fair = __builtin_amdgcn_readfirstlane(fabsf(rt) <= FLT_MAX);
+    const bool bounds = fair && per > 6144;
+    const float least = fair ? -FLT_MAX : -INFINITY;    // behind it masked ones alone
+    for (int base = first; bounds && base < i1; base += 2048) {
 #pragma unroll
         for (int e = 0; e < E; ++e) f[e] = ahead[e];
         load(base + 2048, ahead);
@@ -1076,17 +1088,23 @@ k_sample_gumbel(Pick* __restrict__ ws, int* __restrict__ out,
             at_most = base;
         }
     }
-    if (!(fabsf(rt) <= FLT_MAX)) most = next = INFINITY;    // no bounds
+
+    bool same = marks && other == slot && r0 != row;    // another row has the slot
+    if (marks)
+        for (int r = threadIdx.x + 256; r < rows; r += 256)
+            same |= how.slots[r] == slot && r != row;
+    same = __any(same);
 
     // Exact values of a batch's elements, but for those that the hardware's logarithms
-    // put behind the best of the wave.
+    // put behind the best of the wave, and for masked ones.
     Pick best{-INFINITY, 2147483647};
     auto look = [&](int base, bool mine) {
         float g[E], u[E], a[E], lim = best.val;
         auto at = [&](int e) { return base + (e >> 2) * 256 + lane * 4 + (e & 3); };
-        load(mine ? base : i1, g);
+        if (bounds || base != first) load(mine ? base : i1, ahead);
 #pragma unroll
         for (int e = 0; e < E; ++e) {
+            g[e] = ahead[e];
             u[e] = 0.f;
             a[e] = g[e] * rt;
             if (key != 0ull) {
@@ -1097,11 +1115,10 @@ k_sample_gumbel(Pick* __restrict__ ws, int* __restrict__ out,
             }
             if (mine && u[e] <= 0.999f) lim = fmaxf(lim, a[e]);
         }
-        lim = max_across16(max_of16(lim));
-        lim -= 0.05f + 1e-5f * fabsf(lim);
+        lim = fmaxf(below(max_across16(max_of16(lim)), 0.05f), least);
         u32 left = 0;
 #pragma unroll
-        for (int e = 0; e < E; ++e)        // (so that NaN and infinities are)
+        for (int e = 0; e < E; ++e)        // (so that NaN and +inf are)
             if (mine && at(e) < i1 && !(a[e] < lim && u[e] <= 0.999f))
                 left |= 1u << e;
 #pragma unroll 1
@@ -1123,32 +1140,30 @@ k_sample_gumbel(Pick* __restrict__ ws, int* __restrict__ out,
     __shared__ float bound[4];
     __shared__ Pick part[4];
     __shared__ int twice[4];
-    float top = max_across16(max_of16(most));
-    same = __any(same);
-    if (lane == 0) {
-        bound[wid] = top;
-        twice[wid] = same;
-    }
-    __syncthreads();
-    if (twice[0] | twice[1] | twice[2] | twice[3]) {
-        if (seg == 0) sample_same(out, logits, how, row, rows, v, part);
-        return;
-    }
-    top = fmaxf(fmaxf(bound[0], bound[1]), fmaxf(bound[2], bound[3]));
-    const bool near = !(most < top - 0.1f - 1e-5f * fabsf(top));
     // first the batches next to the largest bound; the best of these says what else
     // may be it: other lanes' largest batches, and all of lanes with another large one
-    bool mine = near, more = false;
-    for (int base = at_most, behind = -1; ; ) {
+    bool near = true, mine = true, more = !bounds;
+    bool masked = false;               // all of the segment
+    int base = at_most, behind = bounds ? -1 : first + 2048;
+    if (bounds) {
+        float top = max_across16(max_of16(most));
+        if (lane == 0) bound[wid] = top;
+        __syncthreads();
+        top = fmaxf(fmaxf(bound[0], bound[1]), fmaxf(bound[2], bound[3]));
+        near = !(most < below(top, 0.1f));
+        masked = !(top > -INFINITY);
+        mine = near && !masked;
+    }
+    for (;;) {
         if (__any(mine)) look(base, mine);
         if (behind < 0) {
             const Pick w = wave_pick(best);
             __syncthreads();
             if (lane == 0) bound[wid] = w.val;
             __syncthreads();
-            float lim = fmaxf(fmaxf(bound[0], bound[1]), fmaxf(bound[2], bound[3]));
-            lim -= 1e-4f + 1e-5f * fabsf(lim);
-            more = !(next < lim);
+            const float lim = below(
+                fmaxf(fmaxf(bound[0], bound[1]), fmaxf(bound[2], bound[3])), 1e-4f);
+            more = !masked && !(next < lim);
             mine = !near && !(most < lim);
             behind = first;
             continue;
@@ -1159,13 +1174,21 @@ k_sample_gumbel(Pick* __restrict__ ws, int* __restrict__ out,
         behind += 2048;
     }
     best = wave_pick(best);
-    if (lane == 0) part[wid] = best;
+    if (lane == 0) {
+        part[wid] = best;
+        twice[wid] = same;
+    }
     __syncthreads();
+    if (twice[0] | twice[1] | twice[2] | twice[3]) {
+        if (seg == 0) sample_same(out, logits, how, row, rows, v, part);
+        return;
+    }
     if (threadIdx.x == 0) {
         for (int k = 1; k < 4; ++k)
             if (better(part[k].val, part[k].at, best)) best = part[k];
-        if (marks) meet(best, out + row, marks + MARK * how.slots[row],
-                        how.draws + how.slots[row], segments);
+        if (best.val == -INFINITY) best.at = 2147483647;    // (not all were looked at)
+        if (marks) meet(best, out + row, marks + MARK * slot, how.draws + slot,
+                        segments);
         else ws[blockIdx.x] = best;
     }
 }

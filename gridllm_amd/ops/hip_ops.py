@@ -828,8 +828,8 @@ def _sample(logits, keys, temps, slots=None, seeds=None, draws=None,
                          "length, dense and on one GPU")
     if slots is not None:
         _check_range("sample_gumbel.slots", slots, n[0])
-    # four blocks a CU, of 2048 elements or more
-    segments = max(1, min(1024 // max(1, b), v // 2048, 64))
+    # four blocks a CU, of 2048 elements (what its waves have at a time) or more
+    segments = max(1, min(1024 // max(1, b), -(-v // 2048), 64))
     out = torch.empty(b, dtype=torch.int32, device=logits.device)
     if marks is not None and v:
         _check(lib.gl_sample_slots(

@@ -633,6 +633,32 @@ def test_sample_gumbel_slots_twice(dev, b, v):
     assert torch.equal(draws.cpu(), count) and not marks.any()
 
 
+@pytest.mark.parametrize("b,v", [(1, 128256), (6, 2048), (6, 2049), (40, 128256),
+                                 (600, 9000)])
+def test_sample_gumbel_masked(dev, b, v):
+    """Rows of which a mask leaves one candidate, some, or none, by -inf or by the
+    least number, and rows with +inf: segments of one batch a wave and of several."""
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator().manual_seed(b + v)
+    x = torch.full((b, v), float("-inf"))
+    left = torch.randint(0, v, (b, 9), generator=g)
+    x[1::6] = torch.finfo(torch.float32).min
+    x.scatter_(1, left, torch.randn(b, 9, generator=g))
+    x[2::6] = float("-inf")
+    x[3::6].scatter_(1, left[3::6, :2], float("inf"))
+    x[4::6].scatter_(1, left[4::6, 1:], float("-inf"))
+    temps = torch.rand(b, generator=g) + 0.3
+    keys = torch.randint(1, 2 ** 62, (b,), generator=g)
+    z = (torch.arange(v).unsqueeze(0) ^ keys.unsqueeze(1)) * -7046029254386353131
+    z = (z ^ (z >> 29)) * -4658895280553007687
+    z = z ^ (z >> 32)
+    u = (((z >> 38) & 0xFFFFFF).float() / (1 << 24)).clamp(1e-6, 1 - 1e-6).double()
+    val = x.double() / temps.double().unsqueeze(1) - torch.log(-torch.log(u))
+    got = hip_ops.sample_gumbel(x.to(dev), keys.to(dev), temps.to(dev)).cpu()
+    # (the first of equal ones; no two of these others are next to each other)
+    assert torch.equal(got.long(), val.argmax(1))
+
+
 @pytest.mark.parametrize("b,v", [(7, 256), (5, 257), (3, 511), (4, 512), (2, 2049),
                                  (3, 4096), (2, 6400), (1, 133000), (600, 4352)])
 def test_sample_gumbel_chunks(dev, b, v):
