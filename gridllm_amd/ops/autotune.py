@@ -30,6 +30,9 @@ log = get_logger("autotune")
 _CHOICE: dict[tuple[int, int, int], tuple] = {}
 # the same with f32 results (a vocabulary's scores), which not all shapes have
 _CHOICE_F32: dict[tuple[int, int, int], tuple] = {}
+# of products whose parts of K the next kernel adds up (linear_parts,
+# linear_rmsnorm): timed with one behind them, so not what linear does best
+_CHOICE_JOINED: dict[tuple[int, int, int], tuple] = {}
 # gate/up projection with fused SwiGLU (n = 2F interleaved rows):
 # (m, n, k) -> ("blas",) | ("rows",) | ("tile", rows, cols, splitk) |
 # ("wide", shape, whole tiles)
@@ -147,7 +150,8 @@ def _rule(m: int, n: int, k: int, fuse: bool = False, whole: bool = False,
 def _tune(x: torch.Tensor, n: int, glu: Optional[Glu] = None,
           f32: bool = False, joined: bool = False) -> tuple:
     """The fastest for x and a weight of n rows; f32: with a result of that; joined:
-    with the norm behind it, which adds up the parts of K that there are.
+    with a norm behind it, which adds up the parts of K that there are (and stands for
+    the other kernels that do).
 
     The library's is taken if it is 5 % faster: its loads go through the Infinity
     Cache and push out what other kernels find there (decode of 256 rows, 4 layers of
@@ -194,7 +198,8 @@ def _tune(x: torch.Tensor, n: int, glu: Optional[Glu] = None,
 
 def tune_shape(m: int, n: int, k: int, device, f32: bool = False,
                joined: bool = False) -> tuple:
-    key, table = (m, n, k), _CHOICE_F32 if f32 else _CHOICE
+    key, table = (m, n, k), _CHOICE_F32 if f32 else \
+        _CHOICE_JOINED if joined else _CHOICE
     if key not in table:
         x = torch.randn(m, k, device=device).to(torch.bfloat16) * 0.1
         table[key] = _tune(x, n, f32=f32, joined=joined)
@@ -232,13 +237,14 @@ def _timed(table: dict, fit: tuple[int, int, int], whole: bool
 
 
 def choice(m: int, n: int, k: int) -> Optional[tuple[str, int]]:
-    return _CHOICE.get((m, n, k))
+    key = (m, n, k)
+    return _CHOICE.get(key) or _CHOICE_JOINED.get(key)
 
 
 def _choose(x: torch.Tensor, w: torch.Tensor, whole: bool = False,
-            f32: bool = False) -> Optional[tuple]:
-    """Choice for x @ w.T (f32: a result of that), None for what is not a GPU
-    product of bf16 rows."""
+            f32: bool = False, joined: bool = False) -> Optional[tuple]:
+    """Choice for x @ w.T (f32: a result of that; joined: if the next kernel adds up
+    its parts), None for what is not a GPU product of bf16 rows."""
     if not x.is_cuda or (torch.is_grad_enabled() and
                          (x.requires_grad or w.requires_grad)):
         return None
@@ -247,20 +253,21 @@ def _choose(x: torch.Tensor, w: torch.Tensor, whole: bool = False,
         return None
     if f32:
         return _CHOICE_F32.get(fit) or _rule(*fit, f32=True)
-    if whole and fit[0] > 256:
-        return _timed(_CHOICE, fit, True) or _rule(*fit, False, True)
-    return _CHOICE.get(fit) or _rule(*fit)
+    whole = whole and fit[0] > 256
+    return (joined and _timed(_CHOICE_JOINED, fit, whole)) or \
+        _timed(_CHOICE, fit, whole) or _rule(*fit, False, whole)
 
 
 def choice_of(m: int, w: torch.Tensor, fuse: bool = False) -> Optional[tuple]:
-    """What linear (fuse: linear_gateup) runs dense aligned bf16 rows [m, K] and w
-    by, if that is one of the kernels here."""
+    """What linear_parts and linear_rmsnorm (fuse: linear_gateup) run dense aligned
+    bf16 rows [m, K] and w by, if that is one of the kernels here."""
     if m > _most_rows or w.dtype is not _BF16 or _transformed() or \
             forward_ad._current_level >= 0 or w.dim() != 2 or \
             not w.is_contiguous() or w.data_ptr() & 15 or not w.numel():
         return None
     key = (m, *w.shape)
-    c = (_CHOICE_GU if fuse else _CHOICE).get(key) or _rule(*key, fuse)
+    c = (_CHOICE_GU.get(key) if fuse else _CHOICE_JOINED.get(key) or _CHOICE.get(key)
+         ) or _rule(*key, fuse)
     return c if c[0] in ("rows", "tile", "wide") else None
 
 
@@ -284,7 +291,7 @@ def linear_parts(x: torch.Tensor, w: torch.Tensor, whole: bool = False
                  ) -> torch.Tensor:
     """linear(x, w), or its f32 partial sums [parts, M, N] if K is in parts, for
     post_norm, join_norm and rope_kv."""
-    c = _choose(x, w, whole)
+    c = _choose(x, w, whole, joined=True)
     if c is not None and c[0] == "tile" and c[3] > 1 and w.shape[1] > 64:
         return hip_ops.gemm_tile_parts(x, w, *c[1:])
     return F.linear(x, w) if c is None else _run(c, x, w)
@@ -295,7 +302,7 @@ def linear_rmsnorm(x: torch.Tensor, w: torch.Tensor, weight: torch.Tensor,
                    ) -> tuple[torch.Tensor, torch.Tensor]:
     """(rmsnorm(y) * weight, y) of y = x @ w.T + residual. A product with its K
     in parts leaves adding them up to the norm."""
-    c = _choose(x, w)
+    c = _choose(x, w, joined=True)
     if c is None:
         return ops.rmsnorm(F.linear(x, w), weight, eps, residual=residual)
     return _run_joined(c, x, w, weight, eps, residual)
@@ -328,7 +335,7 @@ def tune_model_shapes(model, buckets) -> None:
                 tune_gateup(m, n, k, model.device)
             else:
                 tune_shape(m, n, k, model.device)
-    picked = [*_CHOICE.values(), *_CHOICE_F32.values()]
+    picked = [*_CHOICE.values(), *_CHOICE_F32.values(), *_CHOICE_JOINED.values()]
     log.performance("gemm autotune done", shapes=len(picked),
                     ours=sum(1 for c in picked if c[0] != "blas"),
                     ms=int((time.monotonic() - t0) * 1000))

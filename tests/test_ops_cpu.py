@@ -524,6 +524,47 @@ def test_whole_products_of_sizes_that_were_timed(monkeypatch):
                 else ran[1][0] in ("blas", "wide")
 
 
+def test_joined_choices_are_their_own(monkeypatch):
+    """What was timed with the norm behind it, which adds up parts of K, is not what
+    a product alone runs by, nor the other way round."""
+    from gridllm_amd import ops
+    from gridllm_amd.ops import autotune, hip_ops
+
+    class OnGpu(torch.Tensor):
+        is_cuda = True
+    ran = []
+    monkeypatch.setattr(autotune, "_run", lambda c, x, *rest: ran.append(c))
+    monkeypatch.setattr(hip_ops, "gemm_tile_parts",
+                        lambda x, w, *c: ran.append(("tile", *c)))
+    monkeypatch.setattr(hip_ops, "gemm_tile_rmsnorm",
+                        lambda x, w, *c: ran.append(("tile", *c[:3])))
+    monkeypatch.setattr(ops, "rmsnorm", lambda *a, **kw: None)
+    m, n, k = 24, 3072, 8192
+    x = torch.empty(m, k, dtype=torch.bfloat16).as_subclass(OnGpu)
+    w = torch.empty(n, k, dtype=torch.bfloat16)
+    norm, resid = (torch.zeros(*s, dtype=torch.bfloat16) for s in ((n,), (m, n)))
+    cut, alone = ("tile", 32, 64, 16), ("tile", 32, 64, 2)
+
+    def both():
+        ran.clear()
+        autotune.linear(x, w)
+        autotune.linear_parts(x, w)
+        autotune.linear_rmsnorm(x, w, norm, 1e-5, resid)
+        return [*ran, autotune.choice_of(m, w)]
+    rule = both()[0]
+    for order in ((True, False), (False, True)):
+        with monkeypatch.context() as mp:
+            for table in ("_CHOICE", "_CHOICE_JOINED"):
+                mp.setattr(autotune, table, {}, raising=False)
+            mp.setattr(autotune, "_tune", lambda x, n, f32, joined:
+                       cut if joined else alone)
+            autotune.tune_shape(m, n, k, "cpu", False, order[0])
+            # of one kind alone: joined ones still take what was timed alone
+            assert both() == ([rule, cut, cut, cut] if order[0] else [alone] * 4)
+            autotune.tune_shape(m, n, k, "cpu", False, order[1])
+            assert both() == [alone, cut, cut, cut]
+
+
 def test_plans_times_are_the_tilings():
     """What gl_gemm_plan says of a tiling's time is what _tile_us says: of the
     tilings that it looks at, the one it names takes the least by both."""
