@@ -43,14 +43,24 @@ _CALLS = 128                    # of a timing, at most
 _SPLITK_CANDIDATES = (0, 2, 4, 6, 8, 12, 16, 24, 32)
 
 
+def _copies(size: int, room: float) -> int:
+    """Copies of a weight of `size` bytes, 2 GB of them if that is 128 or less: each
+    call of a timing reads its own, and as little of it is in the Infinity Cache (256
+    MB) as of a model's. (Loads past the caches leave there what is in it: of 640 MB
+    that they read in turn two fifths, and the other kernels' loads nothing.) With less
+    than 4 GB left, behind the KV cache, 24 and 640 MB: not to fail for want of
+    memory."""
+    most, total = (_CALLS, 2 << 30) if room >= 4 << 30 else (24, 640 << 20)
+    return min(most, max(2, total // max(1, size)))
+
+
 def _weights(n: int, k: int, device) -> list[torch.Tensor]:
-    """Copies of a weight, 2 GB of them if that is 128 or less: each call of a timing
-    reads its own, and as little of it is in the Infinity Cache (256 MB) as of a
-    model's. (Loads past the caches leave there what is in it: of 640 MB that they read
-    in turn two fifths, and the other kernels' loads nothing.)"""
-    copies = min(_CALLS, max(2, (2 << 30) // max(1, n * k * 2)))
+    room = float("inf")
+    if device.type == "cuda":
+        room = torch.cuda.mem_get_info(device)[0] + torch.cuda.memory_reserved(
+            device) - torch.cuda.memory_allocated(device)
     w = torch.randn(n, k, device=device).to(torch.bfloat16) * 0.1
-    return [w] + [w.clone() for _ in range(copies - 1)]
+    return [w] + [w.clone() for _ in range(_copies(n * k * 2, room) - 1)]
 
 
 def _time_fn(fn, ws, limit: float = float("inf")) -> float:

@@ -565,6 +565,20 @@ def test_joined_choices_are_their_own(monkeypatch):
             assert both() == [alone, cut, cut, cut]
 
 
+@pytest.mark.parametrize("n,k", [(64, 64), (3072, 3072), (128256, 3072)])
+def test_timings_fit_beside_a_full_cache(n, k):
+    """An engine whose KV cache leaves little memory starts: the tuner takes no more
+    than 24 copies of a weight, in 640 MB, or the two that it cannot do without."""
+    from gridllm_amd.ops import autotune
+    size = n * k * 2
+    for room in (0, 1 << 30, (4 << 30) - 1):
+        few = autotune._copies(size, room)
+        assert few >= 2 and few <= 24 and (few == 2 or few * size <= 640 << 20)
+    for room in (4 << 30, float("inf")):
+        copies = autotune._copies(size, room)
+        assert copies >= few and (copies == 2 or copies * size <= 2 << 30)
+
+
 def test_plans_times_are_the_tilings():
     """What gl_gemm_plan says of a tiling's time is what _tile_us says: of the
     tilings that it looks at, the one it names takes the least by both."""
