@@ -723,16 +723,18 @@ static int launch_gemm_tile(hipStream_t st, BatchArgs p) {
     return 0;
 }
 
-template <class S, class S2, int EPI>
+template <class S, class S2, int EPI, bool ONCE = false>
 static int launch_gemm_wide(hipStream_t st, const WideArgs& p, int full) {
+    if constexpr (EPI == 2 && !ONCE)
+        if (p.M <= S::R) return launch_gemm_wide<S, S2, EPI, true>(st, p, full);
     constexpr int bytes = S::BYTES > S2::BYTES ? S::BYTES : S2::BYTES;
-    const int e = allow_lds<k_gemm_wide<S, S2, EPI>>(bytes);
+    constexpr auto kernel = k_gemm_wide<S, S2, EPI, ONCE>;
+    const int e = allow_lds<kernel>(bytes);
     if (e) return e;
     const int total = (p.M + S::R - 1) / S::R * ((p.N + S::C - 1) / S::C);
     full = S2::R ? min(full, total) : total;
     const int most = max(full, (total - full) * 2);     // blocks' tiles
-    k_gemm_wide<S, S2, EPI><<<8 * min((most + 7) / 8, 32), 512, bytes, st>>>(
-        p, full);
+    kernel<<<8 * min((most + 7) / 8, 32), 512, bytes, st>>>(p, full);
     LAUNCH_CHECK();
     return 0;
 }

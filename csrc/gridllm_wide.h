@@ -29,10 +29,12 @@
 // the results rounded to bf16, as a library product and the unit behind it have it.
 // Sums go over all of K in order, as the library's do but for those of its tiles
 // whose K it cuts, so that more than 99.9 % of results are the same to the bit.
-// EPI 2: the result, rounded to bf16, as f32 (a vocabulary's scores); W, which such a
-// product's few rows read once, past the Infinity Cache (see load_lds16_once; 256 rows of
+// EPI 2: the result, rounded to bf16, as f32 (a vocabulary's scores); with one tile of
+// rows, which reads W once, past the Infinity Cache (see load_lds16_once; 256 rows of
 // 128256 x 3072 in a step 207 -> 201 us, and the step's other kernels find theirs
-// there: 4 layers 880 -> 861).
+// there: 4 layers 880 -> 861). More tiles of rows read W again, and would wait for memory
+// where the Infinity Cache has it (us, through it and past it, 128256 x 3072: 257 rows 300,
+// 361, 512 444, 481, 1024 886, 936; 300 of 151936 x 896 131, 155).
 // EPI 3: squared ReLU. EPI 4: W rows in turns of 16 gate | 16 up, [M, N / 2].
 // Rows past M and N are read as zeros by the buffer descriptors' bounds, and so are
 // the stages past the last tile: a wave's offset is the end of the matrix at most,
@@ -60,8 +62,9 @@ struct WideTile {
 
 // Where rows come from and go to. GATHER: x's rows are looked up one by one. ONCE: W's
 // are read once, and past the Infinity Cache.
+template <bool O>
 struct DenseRows {
-    static constexpr bool GATHER = false, ONCE = false;
+    static constexpr bool GATHER = false, ONCE = O;
     DEV_INLINE int from(int m) const { return m; }
     DEV_INLINE long to(int m) const { return m; }
     DEV_INLINE float weight(int m) const { return 1.f; }
@@ -77,10 +80,10 @@ struct NoShape {
 };
 
 // Tiles item, item + stride, ... < last, as place says; wrows: of W.
-template <class S, int EPI, class Place, class Rows = DenseRows>
+template <class S, int EPI, class Place, class Rows>
 DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
                            int stride, Place place, int wrows,
-                           const Rows rows = Rows()) {
+                           const Rows rows) {
 #ifdef __HIP_DEVICE_COMPILE__          // (the host has no buffer descriptors)
     constexpr int A = S::A, B = S::B, NB = S::NB, R = S::R, C = S::C;
     constexpr int BUF = (R + C) * 64, G = (R + C) / 64;  // loads of a wave, stage
@@ -147,7 +150,7 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
         if (i * 64 < R)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, dst, 16, vx[i % GX],
                                                      so[i], 0, 0);
-        else if (EPI == 2 || Rows::ONCE)
+        else if (Rows::ONCE)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, dst, 16, v, so[i], 0, 2);
         else
             __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, dst, 16, v, so[i], 0, 0);
@@ -295,7 +298,7 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
 #endif
 }
 
-template <class S, class S2, int EPI>
+template <class S, class S2, int EPI, bool ONCE>
 __global__ void __launch_bounds__(512, 2)
 k_gemm_wide(const WideArgs p, int full) {
     extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
@@ -309,7 +312,7 @@ k_gemm_wide(const WideArgs p, int full) {
     };
     const int each = (full + 7) >> 3;           // tiles of an XCD
     wide_tiles<S, EPI>(p, lds, xcd * each + at, min(full, (xcd + 1) * each),
-                       stride, place, p.N);
+                       stride, place, p.N, DenseRows<ONCE>());
     if constexpr (S2::R > 0) {
         static_assert(S2::R * 2 == S::R && S2::C == S::C, "halves");
         const int rest = (rb * cb - full) * 2, each = (rest + 7) >> 3;
@@ -319,7 +322,7 @@ k_gemm_wide(const WideArgs p, int full) {
                 WideTile t = place(full + (it >> 1));
                 t.m0 += (it & 1) * S2::R;
                 return t;
-            }, p.N);
+            }, p.N, DenseRows<ONCE>());
     }
 }
 
