@@ -1,5 +1,6 @@
 // Batch GEMM: out[M,N] = x[M,K] @ W[N,K]^T (bf16 I/O, f32 sums), for more rows
-// than k_gemm_rows takes: k_gemm_tile up to 64 rows a block, k_gemm_fed above.
+// than k_gemm_rows takes: k_gemm_tile up to 64 rows a block, or 256 columns, k_gemm_fed
+// above.
 //
 // A block has RT * 16 rows by CT * 16 columns of one of `splitk` parts of K. Pieces
 // of 64 k of x and W come into rings in LDS by direct loads, 8 rows of 128 bytes
@@ -18,7 +19,12 @@
 // where x hits in L2 and 950 where W comes from memory, hence 51 KB a us (12288 x 3072,
 // 192 rows, loads alone in tiles of 96 x 96: x 7.4 us, W 16.4, both 25.7; with W in the
 // Infinity Cache both 16.2). So the tile is as large as the accumulators allow and all
-// of the chip has one. W goes past the Infinity Cache (see load_lds16_once).
+// of the chip has one. ONCE: one block of rows, which reads W once, and past the Infinity
+// Cache (see load_lds16_once). Several blocks of rows do not quite read it at one time,
+// and what is past that cache has left L2, too: mean of its time through the cache, with
+// 2, 3, 4 and more blocks of rows, over 178 tilings of up to 256 rows a block .98, .99,
+// .99 and .97, of up to 64 .94, .91, .94 and .93 (200 rows of 5120 x 3072, 96 by 64, 21.2
+// us past it, 17.1; 48 of 2048 x 2048, 32 by 64, in 4 parts, 7.5 and 8.1).
 //
 // Where W's rows are a multiple of 4096 bytes long, what all blocks read at a time, a
 // piece of 128 bytes at the same place of each row, is in few of the memory's
@@ -145,7 +151,8 @@ DEV_INLINE void batch_join(const BatchArgs& p, const BatchTile& t, int m0, int k
 // buffers, NB - 1 ahead. In the middle of a stage the waves meet: the next one is
 // there, and this one's buffer is free, its second half being in registers; so the
 // products of one half run while the other half is read.
-// W past the caches (us, 2 GB of weights in turn; parts of K without what adds them up):
+// W through and past that cache (us, 2 GB of weights in turn, parts of K without what
+// adds them up):
 //   rows        1                24               64
 //   5120x3072    7.5 ->  7.0      8.0 ->  7.6      9.7 ->  9.5
 //   3072x8192   11.2 -> 10.4     11.5 -> 10.7     13.1 -> 12.4
@@ -166,7 +173,7 @@ struct GemmTile {
     static constexpr int BYTES = NB * STAGE;
 };
 
-template <int RT, int CT, int EPI>
+template <int RT, int CT, int EPI, bool ONCE>
 __global__ void __launch_bounds__(256, CT == 16 ? 1 : 2)
 k_gemm_tile(const BatchArgs p) {
     typedef GemmTile<RT, CT> Sh;
@@ -196,7 +203,7 @@ k_gemm_tile(const BatchArgs p) {
 #pragma unroll
         for (int i = 0; i < G; ++i) {
             bf16_t* dst = lds + buf * BUF + (i * 4 + wid) * 512;
-            if ((i * 4 + wid) * 8 < R) load_lds16(src[i], dst);
+            if (!ONCE || (i * 4 + wid) * 8 < R) load_lds16(src[i], dst);
             else load_lds16_once(src[i], dst);
             src[i] += 64;
         }
@@ -339,7 +346,7 @@ struct GemmFed {
     static constexpr bool BY_K = RT / 2 * CT <= 36;
 };
 
-template <int RT, int CT, int EPI>
+template <int RT, int CT, int EPI, bool ONCE>
 __global__ void __launch_bounds__(512, 2)
 k_gemm_fed(const BatchArgs p) {
     typedef GemmFed<RT, CT> Sh;
@@ -387,9 +394,11 @@ k_gemm_fed(const BatchArgs p) {
             const int half = v & 1;            // (behind the last stage: it again)
             const int s = min(iw + turn - (iw + turn >= nt ? nt : 0) + half, nt - 1);
 #pragma unroll
-            for (int i = 0; i < GW; ++i)
-                load_lds16_once(sw[i] + s * 64, ldw + ((bw + half) * C +
-                                                (i * 2 + (v >> 1)) * 8) * 64);
+            for (int i = 0; i < GW; ++i) {
+                bf16_t* dst = ldw + ((bw + half) * C + (i * 2 + (v >> 1)) * 8) * 64;
+                if (ONCE) load_lds16_once(sw[i] + s * 64, dst);
+                else load_lds16(sw[i] + s * 64, dst);
+            }
             bw = bw + 2 == NW ? 0 : bw + 2;
             iw += 2;
         };

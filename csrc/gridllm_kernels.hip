@@ -706,17 +706,19 @@ static int allow_lds(int bytes) {
     return (int)e;
 }
 
-template <int RT, int CT, int EPI>
+template <int RT, int CT, int EPI, bool ONCE = false>
 static int launch_gemm_tile(hipStream_t st, BatchArgs p) {
     constexpr bool both = RT <= 4 || CT == 16;  // waves load and multiply
     typedef std::conditional_t<both, GemmTile<RT, CT>, GemmFed<RT, CT>> Sh;
+    p.rblocks = (p.M + Sh::R - 1) / Sh::R;
+    if constexpr (!ONCE)
+        if (p.rblocks == 1) return launch_gemm_tile<RT, CT, EPI, true>(st, p);
     constexpr auto kernel = [] {
-        if constexpr (both) return k_gemm_tile<RT, CT, EPI>;
-        else return k_gemm_fed<RT, CT, EPI>;
+        if constexpr (both) return k_gemm_tile<RT, CT, EPI, ONCE>;
+        else return k_gemm_fed<RT, CT, EPI, ONCE>;
     }();
     const int e = allow_lds<kernel>(Sh::BYTES);
     if (e) return e;
-    p.rblocks = (p.M + Sh::R - 1) / Sh::R;
     const long total = (long)(p.N / Sh::C) * p.splitk * p.rblocks;
     kernel<<<(unsigned)((total + 7) / 8 * 8), Sh::THREADS, Sh::BYTES, st>>>(p);
     LAUNCH_CHECK();
