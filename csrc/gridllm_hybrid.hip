@@ -300,9 +300,11 @@ DEV_INLINE void scale_groups(float (&f)[8], const float* rs, int c,
 }
 
 // parts > 0: y is f32 partial sums. A thread has 8 NV columns, and all its loads are
-// on their way at once. Bound by these and by the sums' steps: 160 rows of 3072 with 2
-// and 8 parts 7.6 us with 256 threads a row and weights read after the sums, now
-// 5.7.
+// on their way at once, but for the weights of two turns, whose registers would have a
+// SIMD hold fewer waves (8192 rows of 5120 in groups of 128: 157 us with them ahead, 116
+// behind the sums; 1024 20.8, 19.9; one 7.6 either way). Bound by the loads and the
+// sums' steps: 160 rows of 3072 with 2 and 8 parts 7.6 us with 256 threads a row and
+// weights read after the sums, now 5.7.
 template <class T, bool ADD, int GR, int NV>
 __global__ void __launch_bounds__(512)
 k_group_norm(T* __restrict__ out, float* __restrict__ x,
@@ -319,8 +321,8 @@ k_group_norm(T* __restrict__ out, float* __restrict__ x,
         const int c = (j * blockDim.x + threadIdx.x) * 8;
         if (c >= W) continue;
         ld8(x + n * W + c, a[j]);
-        if (ADD) ld8(wy + c, gy[j]);
-        if (out) ld8(w + c, g[j]);
+        if (NV == 1 && ADD) ld8(wy + c, gy[j]);
+        if (NV == 1 && out) ld8(w + c, g[j]);
         if (ADD && parts)
             summed8((const float*)y, parts, n, gridDim.x, W, c, v[j]);
         else if (ADD)
@@ -332,6 +334,7 @@ k_group_norm(T* __restrict__ out, float* __restrict__ x,
         for (int j = 0; j < NV; ++j) {
             const int c = (j * blockDim.x + threadIdx.x) * 8;
             if (c >= W) continue;
+            if (NV > 1) ld8(wy + c, gy[j]);
             scale_groups<GR>(v[j], rs, c, gp);
 #pragma unroll
             for (int i = 0; i < 8; ++i) a[j][i] += v[j][i] * gy[j][i];
@@ -344,6 +347,7 @@ k_group_norm(T* __restrict__ out, float* __restrict__ x,
     for (int j = 0; j < NV; ++j) {
         const int c = (j * blockDim.x + threadIdx.x) * 8;
         if (c >= W) continue;
+        if (NV > 1) ld8(w + c, g[j]);
         scale_groups<GR>(a[j], rs, c, gp);
 #pragma unroll
         for (int i = 0; i < 8; ++i) a[j][i] *= g[j][i];
@@ -2786,8 +2790,8 @@ int gh_group_norm(void* stream, int f32, void* out, void* x, const void* y,
     const int lds = (W / gr + groups) * 4;
     if (lds > 64 * 1024) return -100;
     const Groups gp{groups, size};
-    // (1024 threads for a row of 6144: 160 rows 5.8 and not 6.1 us, 4096 rows 70 and
-    // not 53; before 7.8 and 52)
+    // (256 threads for a row of 6144 in groups of 128: 160 rows 15.5 and not 9.7 us,
+    // 4096 rows 73.5 and not 64.7)
     const int threads = W <= 2048 ? 256 : 512;
 #define GO(T, A, B) do { if (W <= 4096) GON(T, A, B, 1); else GON(T, A, B, 2); \
         } while (0)

@@ -894,7 +894,8 @@ def test_states_of_many_chunks(kind, heads, dv):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,w,parts,size", [(1, 64, 2, 8), (24, 3072, 5, 384),
-                                            (3, 1088, 9, 4)])
+                                            (3, 1088, 9, 4), (5, 4160, 3, 8),
+                                            (2, 8192, 2, 128)])
 def test_norms_add_parts(n, w, parts, size):
     """Partial sums against the sum that a product would have stored."""
     g = torch.Generator().manual_seed(w)
