@@ -528,7 +528,8 @@ k_streams_norm(T* __restrict__ out, const float* __restrict__ x,
 // them are zero). NV > 0: a row of up to NV * THREADS * 8 columns stays in registers.
 // Bound by its loads and steps. With 256 and 512 threads, in a graph, us: 160 rows of
 // 12288 5.7 and 4.6, 4096 rows 35.4 and 34.1; of 4096 columns 3.8 and 3.4, but 16.0 and
-// 18.0.
+// 18.0. Between 4096 and 6144 columns two turns of 512 threads are mostly empty, which
+// many rows show: 5120 columns, 160 rows 3.8 and 3.5, 512 4.4 and 4.7, 8192 34.0 and 41.3.
 // ===========================================================================
 template <class T, int NV, int THREADS>
 __global__ void __launch_bounds__(THREADS)
@@ -2817,6 +2818,7 @@ int gh_poly_norm(void* stream, int f32, void* out, const void* z,
         (hipStream_t)stream>>>((T*)out, (const T*)z, (const float*)coef, F, \
         Ftrue, eps)
 #define PICK(T) do { if (F <= 4096) GO(T, 2, 256); \
+        else if (F <= 6144 && N >= 512) GO(T, 3, 256); \
         else if (F <= 8192) GO(T, 2, 512); else if (F <= 16384) GO(T, 4, 512); \
         else GO(T, 0, 512); } while (0)
     if (f32) PICK(float); else PICK(bf16_t);

@@ -196,6 +196,19 @@ def test_poly_norm(ff, run):
         (1e-5 if run[1] == "fp32" else 0.005)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("ff", [4104, 5000, 6144])
+@pytest.mark.parametrize("rows", [511, 512])
+def test_poly_norm_of_many_rows(rows, ff):
+    """Both sides of the number of rows from which on 256 threads have one of these."""
+    g = torch.Generator().manual_seed(ff)
+    z = torch.randn(rows, ff, generator=g)
+    coef = torch.tensor([0.7, -0.4, 0.3, 0.2])
+    want = oracle.poly_norm(z.double(), coef.double(), 1e-3)
+    got = hops.poly_norm(z.cuda(), coef.cuda(), ff, 1e-3)
+    assert float(errors(got, want).max()) < 1e-5
+
+
 # ------------------------------------------------------ keys that stand out
 
 CUTS = {"whole": [330], "decode-tail": [185, 1], "pairs": [250, 2],
