@@ -893,6 +893,93 @@ def test_states_of_many_chunks(kind, heads, dv):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads,dv", [(12, 256), (2, 192)])
+@pytest.mark.parametrize("kind", ["gla", "mlstm", "lightning"])
+def test_outputs_of_many_chunks(kind, heads, dv):
+    """Each token's output, behind the state that enters its chunk, and the state
+    behind the last one: with 128 value columns a block, and with 64. Queries and keys
+    are not negative, and the norm's eps is so large that it is a factor: results are
+    sums of values, and the sums of their sizes bound the errors."""
+    from gridllm_amd.ops import reference_hybrid
+    dk, lens, eps = 128, (250, 192, 129, 65, 64, 63, 1, 100), 1e18
+    n, at = sum(lens), 0
+    entries, chunks, segs = [], [], []
+    for i, ln in enumerate(lens):
+        start = (i % 2) * 9
+        entries.append((at, ln, i, start))
+        segs.append((i, start, len(chunks), -(-ln // 64)))
+        chunks += [(at + c, min(64, ln - c), i, 0) for c in range(0, ln, 64)]
+        at += ln
+    g = torch.Generator().manual_seed(heads + dv)
+    pos = torch.cat([torch.arange(e[3], e[3] + e[1]) for e in entries])
+    slot = torch.cat([torch.full((e[1],), e[2]) for e in entries])
+
+    def step(dev):
+        def t(rows):
+            return torch.tensor(rows, dtype=torch.int32, device=dev)
+        own = dict(segs=t(entries)) if dev == "cpu" else \
+            dict(segs=t(entries), chunks=t(chunks), chunk_segs=t(segs))
+        return hops.StepMeta(nd=0, pos=pos.int().to(dev),
+                             slot=slot.int().to(dev), max_len=300,
+                             table=torch.zeros(8, 1, dtype=torch.int32,
+                                               device=dev), **own)
+    rows = torch.randn(n, heads * 2 * (dk + dv), generator=g).to(torch.bfloat16)
+    rows[:, :2 * heads * dk] = rows[:, :2 * heads * dk].abs()
+    S = torch.randn(8, heads, dv + (kind == "mlstm"), dk, generator=g)
+    S[:, :, dv:] = S[:, :, dv:].abs()
+    m, norm = torch.rand(8, heads, generator=g), torch.full((heads * dv,), 1e9)
+    u, ba = torch.randn(n, 8, generator=g), torch.randn(heads * dk, generator=g)
+    wa = torch.randn(8, heads * dk, generator=g)
+    gates = torch.randn(n, 2 * heads, generator=g) * 3
+    decay = torch.rand(heads, generator=g) * 0.2 + 0.8
+    decay = torch.stack([decay, decay.log()])
+
+    def run(fn, dev, x, s):
+        x, s, mx, w, st = x.to(dev), s.clone().to(dev), m.clone().to(dev), \
+            norm.to(dev), step(dev)
+        if kind == "gla":
+            o = fn.gla(x, u.to(dev), wa.to(dev), ba.to(dev), s, w, st, dk, dv, 16.0,
+                       eps)
+        elif kind == "mlstm":
+            o = fn.mlstm(x, gates.to(dev), s, mx, w, st, dk, dv, 15.0, eps)
+        else:
+            o = fn.lightning(x, s, decay.to(dev), w, st, dv, eps)
+        return o.cpu().float(), s.cpu(), mx.cpu()
+    sizes = rows.float()
+    at = 2 * heads * dk
+    sizes[:, at:at + heads * dv] = sizes[:, at:at + heads * dv].abs()
+    want, S1, m1 = run(reference_hybrid, "cpu", rows.float(), S)
+    room = run(reference_hybrid, "cpu", sizes, S.abs())[0].abs()
+    got, S2, m2 = run(hops, "cuda", rows, S)
+    # bf16: the result, and the weight of each of a chunk's own values
+    assert bool(((got - want).abs() <= 2 ** -8 * (want.abs() + room)).all())
+    assert float((S2 - S1).abs().max()) < 2 ** -13 * float(S1.abs().max())
+    assert float((m2 - m1).abs().max()) < 1e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,w,top", [(3, 2048, 2), (5, 3072, 8), (2, 4160, 3),
+                                     (4, 8192, 2)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_post_norm_of_pairs(dtype, n, w, top):
+    """A row per (token, expert) by its weight: one turn and two, 256 threads and
+    512."""
+    from gridllm_amd.ops import reference_hybrid
+    g = torch.Generator().manual_seed(w)
+    x, a = torch.randn(n, w, generator=g), torch.rand(w, generator=g)
+    y = torch.randn(n * top, w, generator=g).to(dtype)
+    wt = torch.rand(n, top, generator=g)
+    x1, b1 = x.cuda(), torch.empty(n, w, dtype=dtype, device="cuda")
+    hops.post_norm(x1, b1, y.cuda(), a.cuda(), 1.0, w, 1e-5, wt.cuda())
+    x2, b2 = x.double(), torch.empty(n, w, dtype=torch.float64)
+    reference_hybrid.post_norm(x2, b2, y.double(), a.double(), 1.0, w, 1e-5,
+                               wt.double())
+    # f32: a sum of `top` and one of w squares
+    assert float((x1.cpu() - x2).abs().max()) < 1e-5 * float(x2.abs().max())
+    assert torch.equal(b1, x1.to(dtype))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,w,parts,size", [(1, 64, 2, 8), (24, 3072, 5, 384),
                                             (3, 1088, 9, 4), (5, 4160, 3, 8),
                                             (2, 8192, 2, 128)])

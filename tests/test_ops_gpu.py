@@ -985,6 +985,43 @@ def test_gemm_fed_stages(dev, stages):
             hip_ops.gemm_tile(x, w[:256] if cols == 256 else w, rows, cols)
 
 
+@pytest.mark.parametrize("m,n,k,sk", [(1, 192, 576, 2), (100, 960, 1088, 4),
+                                      (257, 1536, 2048, 5), (300, 6144, 320, 2)])
+def test_gemm_fed_parts(dev, m, n, k, sk):
+    """Parts of K, the last one shorter, in 48 columns, too; results as f32; and the
+    norm that adds the parts up, of one turn of threads and two."""
+    from gridllm_amd import ops
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator().manual_seed(m + k)
+    x, w, r = (torch.randn(*s, generator=g).to(dev, torch.bfloat16)
+               for s in ((m, k), (n, k), (m, n)))
+    weight = (torch.rand(n, generator=g) + 0.5).to(dev, torch.bfloat16)
+    ref = x.float() @ w.float().t()
+    tol = 2 ** -8 * ref.abs() + k * 2 ** -24 * (x.float().abs() @
+                                                w.float().abs().t()) + 1e-6
+    for rows in (96, 128, 160, 192, 256):
+        for cols in (48, 64, 96, 128):
+            if n % cols:
+                continue
+            out = hip_ops.gemm_tile(x, w, rows, cols, sk,
+                                    torch.full_like(ref, 9e9).bfloat16())
+            assert bool(((out.float() - ref).abs() <= tol).all()), (rows, cols)
+            whole = hip_ops.gemm_tile(x, w, rows, cols, 1)
+            assert torch.equal(hip_ops.gemm_tile_f32(x, w, rows, cols),
+                               whole.float()), (rows, cols)
+            parts = hip_ops.gemm_tile_parts(x, w, rows, cols, sk)
+            assert bool(((parts.sum(0) - ref).abs() <= tol).all()), (rows, cols)
+    # the norm adds up in the order of the parts, and rounds as the product does
+    for rows, cols in ((96, 48), (256, 64)):
+        parts = hip_ops.gemm_tile_parts(x, w, rows, cols, sk)
+        total = torch.zeros_like(parts[0])
+        for part in parts:
+            total = total + part
+        y, res = hip_ops.gemm_tile_rmsnorm(x, w, rows, cols, sk, weight, 1e-5, r)
+        want, res2 = ops.rmsnorm(total.bfloat16(), weight, 1e-5, residual=r)
+        assert torch.equal(res, res2) and torch.equal(y, want)
+
+
 @pytest.mark.parametrize("m,n,k", [
     (1, 8, 256),               # one row and 8 columns of a tile; 4 stages
     (255, 256, 256), (257, 264, 320), (384, 1032, 576),
