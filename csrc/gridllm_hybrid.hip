@@ -1199,9 +1199,11 @@ k_mlstm_weights(float* __restrict__ w, float* __restrict__ scal,
 // Bound by a step's instructions and latencies (.8 us a chunk) where a segment is
 // long, by the stores where there are many. 45 chunks of 4 segments, 12 heads of 128
 // x 256: 58 us when the chunks' own contributions were written first, read and
-// added up by a second kernel; now 35. (256 threads, each with twice the keys: 34,
-// but 54 instead of 44 for one segment of 3500.) With what is ahead of it and the
-// outputs, mLSTM's 55 chunks of one segment: 127 us before, now 105.
+// added up by a second kernel; now 35, with operands that the Infinity Cache has. In a
+// step it has some of them, and they take 44; with all from memory, 51. (256 threads,
+// each with twice the keys: 34, but 54 instead of 44 for one segment of 3500.) With what
+// is ahead of it and the outputs, mLSTM's 55 chunks of one segment: 127 us before, now
+// 105; of 4 heads, whose blocks are 64, 76 and 78.
 // KIND: gated linear attention's decays by channel (b), or weights and sums of
 // k_mlstm_weights, where the slot's m is advanced too; mLSTM's normaliser, the row
 // behind the value columns, is the product of the keys with ones.
@@ -1494,11 +1496,10 @@ DEV_INLINE void store_normed(bf16_t* out, const f32x4 (&acc)[4][4],
 // outputs: every fourth 16 columns for all 64, so that the state is read once.
 // Queries and keys come through LDS, 64 channels ahead of their use. With all of a
 // head's columns here (out), the head's norm and gate follow at once; out and
-// CONST exclude each other. Bound by reading the state and the few steps'
-// latencies: 3500 tokens, 12 heads of 128 x 256: 92 us with tokens split over
-// the waves and 128 columns a block, and 28 of the norm behind it, now 66 (8 of
-// it the gates' exponentials and divisions, which are not the hardware's: those
-// are off by 6e-8 |z|).
+// CONST exclude each other. Bound by its instructions, as k_gla_chunk_out: 3500
+// tokens, 12 heads of 128 x 256: 92 us with tokens split over the waves and 128 columns
+// a block, and 28 of the norm behind it, now 66 (some 8 of it the gates' exponentials,
+// which are not the hardware's: those are off by 6e-8 |z|).
 template <bool CONST>
 __global__ void __launch_bounds__(256, 2)
 k_mlstm_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
@@ -2353,7 +2354,9 @@ DEV_INLINE bool moe_work(const int4* tiles, int max_tiles, int ntn, int4& tl,
 // With few rows per expert the same pipeline streams the weights, in tiles of 32
 // rows with 3 buffers: 48 rows in all, 64 experts, 160 -> 155 us; 12 rows gated 199 ->
 // 168 (a CU's loads queue up, and of 128 rows as many are x's as W's). Weights go past
-// the Infinity Cache (see load_lds16_once): 48 rows over and over, 805 MB, 150 -> 131.
+// the Infinity Cache (see load_lds16_once): 48 rows with the same 805 MB call after call,
+// of which part then stays there, 150 -> 131; three sets of them in turn 151 -> 131. (8
+// experts of 320 x 512, all of which would: 150 rows 27.0 -> 28.3.)
 // ACT != 0 (up projection): row r of the tile is token sorted[row0 + r] / top,
 // output in sorted order through squared ReLU (1) or, with weight rows in turns
 // of 16 gate | 16 up, the gated unit `glu` in N / 2 columns (2); pw (nullable):
@@ -2686,9 +2689,9 @@ static int paged_decode(hipStream_t st, void* out, const void* q,
 // tokens (384 blocks of 128) 35 / 41, 12 of 300 40 / 47; one of 3500 (96) 63 / 44.
 template <int KIND>
 static void chunk_states(hipStream_t st, void* dS, void* S, const void* scal,
-                         float* m_in, void* mst, const void* qkv, const void* b, const void* chunks,
-                         const void* segs, int nseg, int H, int DK, int DV,
-                         int ld_) {
+                         float* m_in, void* mst, const void* qkv, const void* b,
+                         const void* chunks, const void* segs, int nseg, int H,
+                         int DK, int DV, int ld_) {
     const bool wide = DV % 128 == 0 &&
                       nseg * H * (DK / STATE_K) * (DV / 128) >= 256;
 #define GO(NK) k_chunk_states<KIND, NK><<<dim3((nseg * H + 7) / 8 * 8, \

@@ -585,11 +585,12 @@ k_gemm_skinny(bf16_t* __restrict__ out, float* __restrict__ ws,
 // each, whose loads start a batch of U chunks ahead, straight into MFMA
 // operands. The waves' sums meet in LDS, so there is no second kernel and no
 // workspace, which is what makes it the fastest for up to 20 MB of W with up to 4
-// rows and 14 MB with 16, while K is 4096 or less (one row, k_gemm_tile's best
-// split behind it: 2048 x 2048 4.7 us, 6.2; 3072 x 3072 7.2, 7.9; larger W streams
-// faster there: 5120 x 3072 10.8, 10.0; 3072 x 8192 15.0, 13.2; longer K keeps a
-// block at it: 1024 x 8192, 4 rows 15.5, 10.6). Every block reads all of x, which
-// for 16 rows costs as much as W. W's loads are plain: each takes half a cache
+// rows while K is 4096 or less, and 10 MB with 16 while it is 3072 or less (one row,
+// k_gemm_tile's best split behind it: 2048 x 2048 5.7 us, 7.0; 3072 x 3072 6.7, 7.9;
+// larger W streams faster there: 5120 x 3072 11.1, 9.7; longer K keeps a block at it:
+// 2048 x 8192 13.0, 10.7; 16 rows of 2048 x 2048 7.2, 7.6, of 3072 x 3072 9.9, 8.3).
+// Every block reads all of x, which for 16 rows costs as much as W. A gated unit's two
+// columns halve its rate: it has those that no tiling fits. W's loads are plain: each takes half a cache
 // line of a row, and past the caches (nontemporal) both halves fetch it: 8.0, 11.1, 16.6
 // and 24.3 us.
 // mfma_f32_16x16x32_bf16: A = x rows, B = W rows (k-contiguous both).

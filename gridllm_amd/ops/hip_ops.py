@@ -549,9 +549,9 @@ def gemm_tiling(m: int, n: int, k: int,
     141).
     Up to 256: what _tile_us says of a block a CU or less, with K whole, in the
     parts that then fill the CUs, or in half as many. It takes 1.003 of the best
-    choice's time in the mean, 1.07 at most, .70 of the library's (246 sizes). More blocks than CUs are a library product's sizes (17920 x
-    1536, 256 rows: 22.9 us, 22.2), but for the gated unit that it would need a second
-    kernel for."""
+    choice's time in the mean, 1.07 at most, .70 of the library's (246 sizes). More
+    blocks than CUs are a library product's sizes (17920 x 1536, 256 rows: 22.9 us,
+    22.2), but for the gated unit that it would need a second kernel for."""
     if not 0 < m <= 256 or n < 1 or k < 1 or k % 64 or (
             fuse_swiglu and n % 128):
         return None
