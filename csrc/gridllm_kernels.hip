@@ -62,7 +62,7 @@ struct SummedRow {
 // turns of THREADS threads have the row, and all loads are on their way at once,
 // the weights', too. In a graph, rows of 3072 with a residual, us: 1 row 3.3 with 256
 // threads and the weights loaded after the sum, now 2.6; 256 rows 3.8 and 3.2; 8000
-// rows 30.1 and 29.6.
+// rows 30.1 and 29.6. None of 2304 to 8192 columns and 1 to 8192 rows got slower.
 template <int NV, int THREADS, class Row>
 DEV_INLINE void rmsnorm_row(bf16_t* yr, const Row x, const bf16_t* w,
                             const bf16_t* rr, bf16_t* ro, int H, float eps,
