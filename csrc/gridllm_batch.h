@@ -19,14 +19,13 @@
 // where x hits in L2 and 950 where W comes from memory, hence 51 KB a us (12288 x 3072,
 // 192 rows, loads alone in tiles of 96 x 96: x 7.4 us, W 16.4, both 25.7; with W in the
 // Infinity Cache both 16.2). So the tile is as large as the accumulators allow and all
-// of the chip has one. ONCE: one block of rows, which reads W once, and past the Infinity
-// Cache (see load_lds16_once). Several blocks of rows do not quite read it at one time,
-// and what is past that cache has left L2, too: mean of its time through the cache, with
-// 2, 3, 4 and more blocks of rows, over 178 tilings of up to 256 rows a block .98, .99,
-// .99 and .97, of up to 64 .94, .91, .94 and .93 (200 rows of 5120 x 3072, 96 by 64, 21.2
-// us past it, 17.1; 48 of 2048 x 2048, 32 by 64, in 4 parts, 7.5 and 8.1). Prompts of
-// 300, 400 and 700 tokens by 0.5b, 1.5b and 3b 1443 -> 1405, 2915 -> 2824, 5640 -> 5590;
-// 400 by 4 layers of 1.5b, of which what is past the cache leaves much there, 427 -> 441.
+// of the chip has one. ONCE: W is read past the Infinity Cache (see load_lds16_once), as one
+// block of rows does. Several blocks of rows do not quite read it at one time, and what
+// is past that cache has left L2, too (200 rows of 5120 x 3072, 96 by 64, 21.2 us past it,
+// 17.1; but 48 of 2048 x 2048, 32 by 64, in 4 parts, 7.5 and 8.1). In all layers, prompts
+// of 300, 400 and 700 tokens by 0.5b, 1.5b and 3b 1443 -> 1405, 2915 -> 2824, 5640 ->
+// 5590; 400 by 4 layers of 1.5b, of which what is past the cache leaves much there, 427
+// -> 441.
 //
 // Where W's rows are a multiple of 4096 bytes long, what all blocks read at a time, a
 // piece of 128 bytes at the same place of each row, is in few of the memory's

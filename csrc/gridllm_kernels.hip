@@ -707,13 +707,25 @@ static int allow_lds(int bytes) {
     return (int)e;
 }
 
+// Whether W, in parts of kslice of K, is read past the Infinity Cache: with one block of
+// rows, or with two or three if it is little, in parts so short that these read it
+// nearly at one time. (Time through the cache of that past it, mean of 28 such tilings
+// 1.02, of 20 with longer parts 1.00, of 43 with more blocks of rows .97, of 148 with
+// larger W .96. See gridllm_batch.h.)
+static bool tile_once(int M, int N, int K, int rows, int kslice) {
+    const int blocks = (M + rows - 1) / rows;
+    return blocks == 1 ||
+           (blocks < 4 && (long)N * K <= 8000000 && kslice < 1536);
+}
+
 template <int RT, int CT, int EPI, bool ONCE = false>
 static int launch_gemm_tile(hipStream_t st, BatchArgs p) {
     constexpr bool both = RT <= 4 || CT == 16;  // waves load and multiply
     typedef std::conditional_t<both, GemmTile<RT, CT>, GemmFed<RT, CT>> Sh;
     p.rblocks = (p.M + Sh::R - 1) / Sh::R;
     if constexpr (!ONCE)
-        if (p.rblocks == 1) return launch_gemm_tile<RT, CT, EPI, true>(st, p);
+        if (tile_once(p.M, p.N, p.K, Sh::R, p.kslice))
+            return launch_gemm_tile<RT, CT, EPI, true>(st, p);
     constexpr auto kernel = [] {
         if constexpr (both) return k_gemm_tile<RT, CT, EPI, ONCE>;
         else return k_gemm_fed<RT, CT, EPI, ONCE>;
@@ -1535,6 +1547,10 @@ int gl_gemm_tile(void* stream, void* out, void* ws, const void* x,
             (bf16_t*)out, (const float*)ws, (long)M * N, splitk);
     LAUNCH_CHECK();
     return 0;
+}
+
+int gl_gemm_tile_once(int M, int N, int K, int rows, int kslice) {
+    return rows < 1 ? -100 : tile_once(M, N, K, rows, kslice);
 }
 
 // shape: one of kWide; full: of its tiles, the others are halved (shape 0). epi: as

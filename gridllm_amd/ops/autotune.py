@@ -163,9 +163,11 @@ def _tune(x: torch.Tensor, n: int, glu: Optional[Glu] = None,
     with a norm behind it, which adds up the parts of K that there are (and stands for
     the other kernels that do).
 
-    The library's is taken if it is 5 % faster: its loads go through the Infinity
-    Cache and push out what other kernels find there (decode of 256 rows, 4 layers of
-    llama3.2:3b, 3072 x 3072 by the library, 1 us faster alone: 861 -> 915 us)."""
+    What reads w through the Infinity Cache, the library or tiles of several blocks of
+    rows, is taken if it is 5 % faster: it pushes out what other kernels find there
+    (decode of 256 rows, 4 layers of llama3.2:3b, 3072 x 3072 by the library, 1 us faster
+    alone: 861 -> 915 us; of 82 rows, qwen2.5:1.5b, 1536 x 8960 by two blocks of 64 rows
+    instead of one of 96: 2103 -> 2142)."""
     global _most_rows
     m, k = x.shape
     _most_rows = max(_most_rows, m)
@@ -194,8 +196,10 @@ def _tune(x: torch.Tensor, n: int, glu: Optional[Glu] = None,
         tried = [("ours", sk) for sk in _SPLITK_CANDIDATES
                  if sk <= max(1, k // 256)]
     for c in tried:
+        through = c[0] == "tile" and not hip_ops.gemm_tile_once(
+            m, n, k, c[1], c[3])
         try:
-            t = time_of(c, 1.3 * t_best)
+            t = time_of(c, 1.3 * t_best) * (1.05 if through else 1)
         except RuntimeError as e:           # one that cannot run is no choice
             log.logger.warning("gemm choice %s of %s failed: %s", c,
                                (m, n, k), e)

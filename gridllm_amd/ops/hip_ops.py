@@ -80,6 +80,8 @@ def _load() -> ctypes.CDLL:
     lib.gl_gemm_wide.restype = c_i
     lib.gl_gemm_plan.argtypes = [c_i] * 5 + [c_vp]
     lib.gl_gemm_plan.restype = c_i
+    lib.gl_gemm_tile_once.argtypes = [c_i] * 5
+    lib.gl_gemm_tile_once.restype = c_i
     lib.gl_attn_prefill.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_i, c_i,
                                     c_i, c_i, c_i, c_i, c_i, c_i, c_f]
     lib.gl_attn_prefill.restype = c_i
@@ -614,6 +616,12 @@ def gemm_tile(x: torch.Tensor, w: torch.Tensor, rows: int, cols: int,
                             m, n, k, splitk, kslice, rows, cols,
                             1 if fuse_swiglu else 0, *glu), "gemm_tile")
     return out
+
+
+def gemm_tile_once(m: int, n: int, k: int, rows: int, splitk: int) -> bool:
+    """Whether gemm_tile reads w past the Infinity Cache."""
+    kslice = ((k + splitk - 1) // splitk + 63) // 64 * 64
+    return _load().gl_gemm_tile_once(m, n, k, rows, kslice) == 1
 
 
 def gemm_tile_f32(x: torch.Tensor, w: torch.Tensor, rows: int,

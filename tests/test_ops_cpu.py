@@ -579,6 +579,32 @@ def test_timings_fit_beside_a_full_cache(n, k):
         assert copies >= few and (copies == 2 or copies * size <= 2 << 30)
 
 
+def test_tuner_asks_more_of_what_goes_through_the_cache(monkeypatch):
+    """Tiles of several blocks of rows read weights through the Infinity Cache, but for
+    few weights in short parts, and are taken if they are 5 % faster than one block's."""
+    from gridllm_amd.ops import autotune, hip_ops
+    once = hip_ops.gemm_tile_once
+    assert once(96, 3072, 8192, 96, 1) and once(256, 128256, 3072, 256, 1)
+    assert not once(97, 3072, 8192, 96, 1) and not once(90, 5120, 3072, 32, 4)
+    assert once(48, 2048, 2048, 32, 4) and once(90, 1536, 1536, 32, 3)
+    assert not once(48, 896, 4864, 32, 1) and not once(128, 2048, 2048, 32, 4)
+    rows, ran = 96, []
+    monkeypatch.setattr(hip_ops, "gemm_tilings", lambda *a: [(96, 64, 5), (64, 64, 5)])
+    monkeypatch.setattr(hip_ops, "gemm_rows_supported", lambda *a: False)
+    monkeypatch.setattr(autotune, "_weights", lambda *a: [None, None])
+    monkeypatch.setattr(autotune, "_run", lambda c, *rest: ran.append(c))
+    monkeypatch.setattr(autotune, "_most_rows", autotune._most_rows)
+
+    def timed(fn, ws, *rest):
+        fn(ws[0])
+        return {"blas": 20.0, 96: 10.0, 64: cut}[ran[-1][1] if len(ran[-1]) > 1
+                                                 else "blas"]
+    monkeypatch.setattr(autotune, "_time_fn", timed)
+    x = _mat(rows, 8960)
+    for cut, best in ((9.6, 96), (9.2, 64)):
+        assert autotune._tune(x, 1536)[1] == best
+
+
 def test_plans_times_are_the_tilings():
     """What gl_gemm_plan says of a tiling's time is what _tile_us says: of the
     tilings that it looks at, the one it names takes the least by both."""

@@ -905,6 +905,17 @@ def test_gemm_tile_long_rows(dev, m, n, k, sk, fuse):
     test_gemm_tile(dev, m, n, k, sk, fuse)
 
 
+@pytest.mark.parametrize("fuse", [False, True])
+@pytest.mark.parametrize("m,n,k,sk", [(257, 1152, 1600, 1), (257, 1152, 3136, 2)])
+def test_gemm_tile_several_blocks(dev, m, n, k, sk, fuse):
+    """The same where several blocks of rows read weights through the cache: K in one
+    part, and in two of unequal length."""
+    from gridllm_amd.ops import hip_ops
+    for rows in (32, 64, 96, 128, 160, 192, 256):
+        assert not hip_ops.gemm_tile_once(m, n, k, rows, sk)
+    test_gemm_tile(dev, m, n, k, sk, fuse)
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 64, 64), (33, 192, 576),
                                    (257, 8256, 128)])
 def test_gemm_tile_f32(dev, m, n, k):
