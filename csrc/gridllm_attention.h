@@ -16,6 +16,11 @@ struct SlotKV {
     DEV_INLINE long off(int slot, int hk, int key) const {
         return (((long)slot * Hk + hk) * Smax + key) * D;
     }
+    struct Walk {
+        DEV_INLINE long operator()(const SlotKV& kv, int slot, int hk, int key) {
+            return kv.off(slot, hk, key);
+        }
+    };
 };
 
 // Caches of pages of 64 keys: [pages, Hk, 64, D]; table[slot][i] is the page
@@ -31,6 +36,22 @@ struct PagedKV {
         const int page = table[(long)slot * per_slot + (key / KV_PAGE)];
         return (((long)page * Hk + hk) * KV_PAGE + key % KV_PAGE) * D;
     }
+    // The same for keys in order: lanes hold the numbers of 64 pages, since a load for
+    // each would be waited for, and all loads of keys that are under way with it
+    struct Walk {
+        int pages = 0, first = -1;
+        DEV_INLINE long operator()(const PagedKV& kv, int slot, int hk, int key) {
+            const int page = key / KV_PAGE;
+            if (page >> 6 != first) {
+                first = page >> 6;
+                pages = kv.table[(long)slot * kv.per_slot +
+                                 min(first * 64 + (int)(threadIdx.x & 63),
+                                     kv.per_slot - 1)];
+            }
+            const int at = __builtin_amdgcn_readlane(pages, page & 63);
+            return (((long)at * kv.Hk + hk) * KV_PAGE + key % KV_PAGE) * D;
+        }
+    };
 };
 
 // Which keys up to its own a query sees. Kernels walk blocks of keys by number
@@ -455,12 +476,15 @@ k_attn_combine(bf16_t* __restrict__ out, const float* __restrict__ ws,
 // transposing reads. The softmax's reference moves only when a row's maximum
 // grows by more than 2^MAX_LAG (weights are at most that, sums are f32).
 //
-// 8000 tokens, 24 heads of 128 over 8: 481 us, 817 TFLOP/s of the pairs that
-// are seen (1889 us with one 32-key tile at a time, V transposed by stores into
-// LDS and K read from L2 by every wave). Matrix cores, vector unit (half of it
-// the exponentials) and LDS are each 40 % busy, one wave's phases after each
-// other; two waves share a SIMD. Tiles of 32 keys with three waves a SIMD take
-// 512 us; working on three tiles at once by software, 526 (registers).
+// 8000 tokens, 24 heads of 128 over 8: 383 us, 1026 TFLOP/s of the pairs that are
+// seen (1889 us with one 32-key tile at a time, V transposed by stores into LDS and K
+// read from L2 by every wave; 432 with waits for all reads of LDS, and heads one after
+// the other); 8 prompts of up to 1300 79 -> 62, 3500 in pages 116 -> 94. Matrix cores
+// are busy half of the time, at a clock of 1.94 GHz (2.05 when they were 44 %: power),
+// vector unit (half of it the exponentials) and LDS some 40 %, one wave's phases after
+// each other; two waves share a SIMD. Tiles of 32 keys with three waves a SIMD,
+// working on three tiles at once by software, and two groups of four waves that take
+// turns at products and at the softmax, were slower (the last 412 us).
 // mfma_f32_32x32x16_bf16:
 //   A[i][k]: lane l holds i = l&31, k = (l>>5)*8 + 0..7
 //   B[k][j]: lane l holds j = l&31, same k chunk
@@ -485,16 +509,8 @@ DEV_INLINE void reads_ahead() {
     __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
 }
 
-// Work item of a prefill block: tiles of one head lie on one XCD (blocks go
-// round the 8 XCDs), later tiles, which see more keys, first. False: none.
 DEV_INLINE bool prefill_item(int ntiles, int Hq, int* tile, int* head) {
-    const int total = ntiles * Hq, per = (total + 7) >> 3;
-    const int at = (int)(blockIdx.x >> 3);
-    const int i = (int)(blockIdx.x & 7) * per + at;
-    if (at >= per || i >= total) return false;
-    *head = i / ntiles;
-    *tile = ntiles - 1 - i % ntiles;
-    return true;
+    return prefill_place(blockIdx.x, ntiles, Hq, tile, head);
 }
 static inline unsigned prefill_grid(long ntiles, long Hq) {
     return (unsigned)((ntiles * Hq + 7) / 8 * 8);
@@ -547,26 +563,17 @@ attn_prefill_tile(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
     const int trow = threadIdx.x / CPR, tcol = threadIdx.x % CPR;
     const int kcol = (tcol ^ (trow & 7)) * 8;
     const int vcol = (tcol ^ (CPR > 8 ? (trow & 3) << 2 : (trow & 2) << 1)) * 8;
-    // keys from k0 on, which lie together; rows behind the last key repeat it
-    auto issue = [&](int k0, bf16_t* to) {
-        const long at = kv.off(slot, hk, k0);
-        const bf16_t *ks = kv.k + at, *vs = kv.v + at;
-        const int last = s_total - 1 - k0;
+    // keys from k0 on, which lie together; rows behind the last key are zeros
+    const u32 ko = (trow * D + kcol) * 2, vo = (trow * D + vcol) * 2;
+    auto issue = [&](int k0, long at, bf16_t* to) {
+        const u32 bytes = min(s_total - k0, 64) * D * 2;
+        const LdsSource ks = lds_source(kv.k + at, bytes);
+        const LdsSource vs = lds_source(kv.v + at, bytes);
         bf16_t* tw = to + wid * 512;
-        if (last >= 63) {
-            const u32 ko = trow * D + kcol, vo = trow * D + vcol;
 #pragma unroll
-            for (int i = 0; i < LOADS; ++i) {
-                load_lds16(ks + i * 2048 + ko, tw + i * 2048);
-                load_lds16(vs + i * 2048 + vo, tw + TILE / 2 + i * 2048);
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < LOADS; ++i) {
-                const u32 r = min(trow + i * (256 / CPR), last) * D;
-                load_lds16(ks + r + kcol, tw + i * 2048);
-                load_lds16(vs + r + vcol, tw + TILE / 2 + i * 2048);
-            }
+        for (int i = 0; i < LOADS; ++i) {
+            load_lds16(ks, ko, i * 4096, tw + i * 2048);
+            load_lds16(vs, vo, i * 4096, tw + TILE / 2 + i * 2048);
         }
     };
 
@@ -689,7 +696,11 @@ attn_prefill_tile(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
     const int kmax = min(s_total, causal_off + q0 + 128);
     const int qfirst = causal_off + q0;
     int k0 = keys.skip(0, qfirst), buf = 0;
-    if (k0 < kmax) issue(k0, lds);
+    typename KV::Walk place;
+    if (k0 < kmax) issue(k0, place(kv, slot, hk, k0), lds);
+    // (or the compiler waits for q in each step, and for the next tile with it)
+#pragma unroll
+    for (int s = 0; s < NS; ++s) asm volatile("" : "+v"(qf[s]));
     // all rows of the block see the whole tile
     auto whole = [&] {
         return k0 + 63 <= qfirst && k0 + 63 < s_total &&
@@ -702,7 +713,7 @@ attn_prefill_tile(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
         lds_barrier();              // tile is there, the other one is free
         buf ^= 1;
         k0 = keys.skip(k0 + 64, qfirst);
-        if (k0 < kmax) issue(k0, lds + buf * TILE);
+        if (k0 < kmax) issue(k0, place(kv, slot, hk, k0), lds + buf * TILE);
         if (!decltype(MASK)::value || kc <= causal_off + qw + 31)
             step(kt, kc, MASK);     // else ahead of all of the wave's rows
     };

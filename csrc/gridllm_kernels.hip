@@ -1726,6 +1726,11 @@ int gl_swiglu_il(void* stream, void* out, const void* gu, long n, int f,
     return 0;
 }
 
+// The tile and head of a prefill block: place[0], place[1] (1 if it has none).
+int gl_prefill_place(int block, int ntiles, int Hq, int* place) {
+    return !prefill_place(block, ntiles, Hq, place, place + 1);
+}
+
 int gl_attn_prefill(void* stream, void* out, const void* q, const void* kc,
                     const void* vc, int T, int Hq, int Hk, int D, int Smax,
                     int slot, int s_total, int causal_off, float scale) {

@@ -479,16 +479,11 @@ k_latent_prefill(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
                  int lat_ld, const int* __restrict__ meta, int ntiles,
                  const Rotation rot, int H, float scale,
                  const bf16_t* __restrict__ gate, int gate_ld) {
-    constexpr int KD = P + R, KC = KD / 8, VC = P / 8;
-    constexpr int LOADS = 32 * (KC + VC) / 256;
-    constexpr int NS = KD / 16, NT = P / 32;
+    constexpr int KD = P + R, NS = KD / 16, NT = P / 32;
     __shared__ __attribute__((aligned(16))) bf16_t tile[2][32 * (KD + P)];
-    // neighbouring work (tiles of one head) on the same XCD, longest first
-    const int total = ntiles * H, per = (total + 7) >> 3;
-    const int i0 = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per || i0 >= total) return;
-    const int h = i0 / ntiles;
-    const int* mt = meta + (ntiles - 1 - i0 % ntiles) * 8;
+    int at_tile, h;
+    if (!prefill_place(blockIdx.x, ntiles, H, &at_tile, &h)) return;
+    const int* mt = meta + at_tile * 8;
     const int q_off = mt[0], len = mt[1], key_off = mt[2], q0 = mt[3];
     const int start = mt[4];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -514,30 +509,25 @@ k_latent_prefill(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
         }
     }
 
-    const bf16_t* src[LOADS];
-    int step[LOADS];
+    // 32 keys: [32][P], their rotated parts [32][R], values [32][P], whose 16-byte
+    // pieces are XORed with the row's low bits; 256 pieces a load, all of one part
+    auto part = [&](LdsSource from, u32 row_bytes, int width, bf16_t* to) {
+        const int chunks = width / 8;
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-        const int pc = i * 256 + threadIdx.x;
-        const bool is_k = pc < 32 * KC;
-        const int pr = is_k ? pc : pc - 32 * KC;
-        const int row = is_k ? pr / KC : pr / VC;
-        const int c = ((is_k ? pr % KC : pr % VC) ^ (row & 7)) * 8;
-        if (is_k && c >= P) {
-            src[i] = lat + (long)(key_off + row) * lat_ld + lat_ld - R + c - P;
-            step[i] = 32 * lat_ld;
-        } else {
-            src[i] = e + ((long)(key_off + row) * H + h) * 2 * P +
-                     (is_k ? c : P + c);
-            step[i] = 64 * H * P;
+        for (int i = 0; i < 32 * chunks / 256; ++i) {
+            const int pc = i * 256 + threadIdx.x, row = pc / chunks;
+            load_lds16(from, row * row_bytes + ((pc % chunks) ^ (row & 7)) * 16, 0,
+                       to + (i * 256 + wid * 64) * 8);
         }
-    }
-    auto issue = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < LOADS; ++i) {
-            load_lds16(src[i], tile[buf] + (i * 256 + wid * 64) * 8);
-            src[i] += step[i];
-        }
+    };
+    const u32 e_row = H * P * 4, lat_row = lat_ld * 2;
+    auto issue = [&](int k0, bf16_t* to) {
+        const long row = key_off + k0;
+        const bf16_t* er = e + (row * H + h) * 2 * P;
+            part(lds_source(er, 31 * e_row + P * 2), e_row, P, to);
+        part(lds_source(lat + row * lat_ld + lat_ld - R, 31 * lat_row + R * 2),
+             lat_row, R, to + 32 * P);
+        part(lds_source(er + P, 31 * e_row + P * 2), e_row, P, to + 32 * KD);
     };
 
     float m = -INFINITY, l = 0.f;
@@ -547,13 +537,13 @@ k_latent_prefill(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
     const float scale2 = scale * LOG2E;
-    issue(0);
+    issue(0, tile[0]);
     for (int k0 = 0; k0 < kmax; k0 += 32) {
         const bf16_t* kt = tile[(k0 >> 5) & 1];
         const bf16_t* vt = kt + 32 * KD;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         lds_barrier();              // tile is there, the other one is free
-        if (k0 + 32 < kmax) issue(((k0 >> 5) + 1) & 1);
+        if (k0 + 32 < kmax) issue(k0 + 32, tile[((k0 >> 5) + 1) & 1]);
         if (k0 > start + qw + 31) continue;     // ahead of all of this wave
         f32x16 sv;
 #pragma unroll
@@ -561,8 +551,9 @@ k_latent_prefill(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
 #pragma unroll
         for (int s = 0; s < NS; ++s)
             sv = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                *(const bf16x8*)(kt + ln * KD +
-                                 ((s * 2 + hi) ^ (ln & 7)) * 8),
+                *(const bf16x8*)(s * 16 < P
+                    ? kt + ln * P + ((s * 2 + hi) ^ (ln & 7)) * 8
+                    : kt + 32 * P + ln * R + ((s * 2 + hi - P / 8) ^ (ln & 7)) * 8),
                 qf[s], sv, 0, 0, 0);
         float mx = -INFINITY;
         if (k0 + 31 <= start + qw) {

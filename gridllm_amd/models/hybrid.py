@@ -935,6 +935,8 @@ class HybridModel:
                            for q0 in range(0, ln, 128)]
                 lrows += -(-total // 32) * 32
             off += ln
+        for t in (tiles, ltiles):          # blocks start with the last one
+            t.sort(key=lambda r: r[3] + r[4])
         talks = [self._chunk_portions(segs, c) for c in self.chunks]
         ids_np = np.concatenate(toks)
         if ids_np.min() < 0 or ids_np.max() >= self.spec.vocab:

@@ -543,9 +543,10 @@ class LlamaModel:
             self._ends_suffice(bounds[-1], len(lens))
         batched = (tokens.is_cuda and self.dtype == torch.bfloat16
                    and s.head_dim in (64, 128))
-        rows = [(bounds[i], ln, sl, q0)
-                for i, (ln, sl) in enumerate(zip(lens, slots))
-                for q0 in range(0, ln, 128)] if batched else []
+        rows = sorted(((bounds[i], ln, sl, q0)
+                       for i, (ln, sl) in enumerate(zip(lens, slots))
+                       for q0 in range(0, ln, 128)),  # blocks start with the last
+                      key=lambda r: r[3]) if batched else []
         ends = [lens, slots, [b - 1 for b in bounds[1:]], [ln - 1 for ln in lens]]
         flat = self.up.upload(np.concatenate(
             [np.asarray(rows, dtype=np.int32).reshape(-1)]

@@ -82,6 +82,8 @@ def _load() -> ctypes.CDLL:
     lib.gl_gemm_plan.restype = c_i
     lib.gl_gemm_tile_once.argtypes = [c_i] * 5
     lib.gl_gemm_tile_once.restype = c_i
+    lib.gl_prefill_place.argtypes = [c_i] * 3 + [c_vp]
+    lib.gl_prefill_place.restype = c_i
     lib.gl_attn_prefill.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_i, c_i,
                                     c_i, c_i, c_i, c_i, c_i, c_i, c_f]
     lib.gl_attn_prefill.restype = c_i

@@ -1116,3 +1116,42 @@ def test_decode_of_many_rows_against_halves():
             at += size
         out.append(torch.cat(parts).cpu())
     close(out[0], out[1], ("cuda:0", "bf16"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("window", [0, 300])
+@pytest.mark.parametrize("start,ln", [(3967, 257), (4033, 70), (4100, 130)])
+def test_prompt_attention_past_64_pages(start, ln, window):
+    """A prompt block has the numbers of 64 pages at a time. Pages in any order give
+    to the bit what a cache of contiguous slots gives (a window is compared with f64:
+    outputs of up to 3.3, of which bf16 rounds 2^-9, and the weights 2^-9 of each
+    value)."""
+    from gridllm_amd.ops import hip_ops
+    dev, H, G, d, room = torch.device("cuda"), 6, 2, 64, 8192
+    g = torch.Generator(device=dev).manual_seed(start)
+    n = start + ln
+    k, v = (torch.randn(1, G, room, d, generator=g, device=dev).bfloat16()
+            for _ in range(2))
+    q = torch.randn(ln, H, d, generator=g, device=dev).bfloat16()
+    pages = torch.randperm(room // 64, generator=g, device=dev)
+    pool_k, pool_v = (torch.zeros(room // 64, G, 64, d, dtype=t.dtype, device=dev)
+                      .index_copy_(0, pages, t[0].view(G, -1, 64, d).transpose(0, 1)
+                                   .contiguous()) for t in (k, v))
+
+    class Cache:
+        table, max_seq = pages.int().view(1, -1).contiguous(), room
+    st = meta_for(Cache, 0, start, ln, dev)
+    st.tiles = st.tiles.flip(0).contiguous()          # (tiles in any order, too)
+    got = hops.paged_attn(q, pool_k, pool_v, st, 0.11, None, None,
+                          hops.Keys(window, 64 if window else 0))
+    if not window:
+        want = hip_ops.attn_prefill_cache(q, k, v, 0, n, start, 0.11)
+        assert torch.equal(got.view_as(want), want)
+        return
+    kd, vd = (t[0, :, :n].double().repeat_interleave(H // G, 0) for t in (k, v))
+    sc = torch.einsum("nhd,hkd->hnk", q.double(), kd) * 0.11
+    at, key = torch.arange(start, n, device=dev).view(-1, 1), torch.arange(
+        n, device=dev)
+    sc.masked_fill_((key > at) | ((at - key >= window) & (key >= 64)), -1e30)
+    want = (torch.softmax(sc, -1) @ vd).transpose(0, 1)
+    assert float((got.view_as(want).double() - want).abs().max()) < 0.02

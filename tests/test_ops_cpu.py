@@ -633,3 +633,27 @@ def test_plans_times_are_the_tilings():
                 assert abs(us(*plan[1:]) - least) < 1e-5 * least, (m, n, k)
                 seen += 1
     assert seen > 50
+
+
+@pytest.mark.parametrize("heads", [1, 3, 7, 8, 9, 14, 24, 33])
+def test_prefill_blocks_have_each_tile_once(heads):
+    """Blocks of prompt attention, by XCD: an eighth of the heads' tiles each, that of
+    heads which follow each other, later tiles first."""
+    import ctypes
+    from gridllm_amd.ops import hip_ops
+    call, place = hip_ops._load().gl_prefill_place, (ctypes.c_int * 2)()
+    for tiles in (1, 2, 3, 5, 8, 31, 63):
+        per = -(-tiles * heads // 8)
+        seen = set()
+        for xcd in range(8):
+            last = tiles
+            for at in range(per):
+                if call(at * 8 + xcd, tiles, heads, place):
+                    break
+                tile, head = place
+                assert 0 <= tile <= last
+                last = tile
+                # (head by head, later tiles first, it would be the same eighth)
+                assert (head * tiles + tiles - 1 - tile) // per == xcd
+                seen.add((tile, head))
+        assert len(seen) == tiles * heads
