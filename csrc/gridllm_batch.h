@@ -12,7 +12,8 @@
 //   splitk > 1: f32 partials [splitk][M][N] in ws. out == null otherwise: the
 //   result, rounded to bf16, as f32 in ws (a vocabulary's scores: 256 rows of
 //   128256 took 30 us to be widened behind it).
-// Constraints: N % (16 CT) == 0 (128 for EPI 1), K % 64 == 0, kslice % 64 == 0.
+// Constraints: N % (16 CT) == 0 (128 for EPI 1), K % 64 == 0, K <= BATCH_K (a tile's
+// offsets fit into 32 bits), kslice % 64 == 0.
 //
 // Bound by a CU's loads: it has some 128 lines of 128 bytes on their way (counted:
 // TCP_TCC_READ_REQ_LATENCY over time, with rings of 2 stages as of 6), for 500 cycles
@@ -42,6 +43,8 @@
 #include <type_traits>
 
 #include "gridllm_tiles.h"
+
+#define BATCH_K (1 << 20)
 
 struct BatchArgs {
     bf16_t* out;
@@ -160,6 +163,11 @@ DEV_INLINE void batch_join(const BatchArgs& p, const BatchTile& t, int m0, int k
 //   16384x3072  20.7 -> 18.6     20.8 -> 19.4     22.8 -> 21.4 (gated)
 //   128256x3072  141 ->  132      150 ->  138      166 ->  162
 // Waves that load alone, as below, take .3 to .5 us more here: a block starts later.
+// Loads by buffer descriptors, behind which waits for LDS are for what is needed (see
+// tiles.h), without 64-bit addresses for each (x not in L2 either): 45 rows of 2048 x
+// 2048 in 4 parts 4.7 -> 4.5, 3072 x 2048 7.9 -> 7.6, 64 of 3072 x 3072 in 5 7.3 -> 7.0,
+// 128 of 128256 x 3072 173.5 -> 170, what W's way from memory bounds 0 to 2 %. The
+// waves below, which only load, gain nothing by it.
 // 256 columns, for rows of x that are read once for all of them, where there are more
 // tiles than CUs anyway: a vocabulary's scores, with up to 160 rows (128256 x 3072, us
 // in 128 columns and in 256: 64 rows 159, 147, 96 178, 159, 160 198, 186; 128256 x 2048
@@ -190,27 +198,31 @@ k_gemm_tile(const BatchArgs p) {
     BatchTile t;
     if (!batch_tile<R, C>(p, &t)) return;
     const int K = p.K, nt = t.stages, turn = batch_turn(p, t);
-    int left = nt - turn;                      // tiles up to the end of K's part
-    const bf16_t* src[G];
+    // rows behind the last one come as zeros; a load takes 8 rows, a stage's start and
+    // a load's rows are scalars
+    const int w0 = batch_row<C, EPI>(t.n0, 0), at = ((lane & 7) ^ (lane >> 3)) * 16;
+    const LdsSource xs = lds_source(p.x + (long)t.m0 * K,
+                                    (u32)min(p.M - t.m0, R) * K * 2);
+    const LdsSource ws = lds_source(p.w + (long)w0 * K,
+                                    min((long)(p.N - w0) * K * 2, 0xffffffffl));
+    const u32 lane_at = (u32)(lane >> 3) * K * 2 + at;
+    u32 rows[G];
 #pragma unroll
     for (int i = 0; i < G; ++i) {
-        const int row = (i * 4 + wid) * 8 + (lane >> 3);
-        const int at = ((lane & 7) ^ (row & 7)) * 8 + t.k0 + turn * 64;
-        src[i] = (i * 4 + wid) * 8 < R
-                     ? p.x + (long)min(t.m0 + row, p.M - 1) * K + at
-                     : p.w + (long)batch_row<C, EPI>(t.n0, row - R) * K + at;
+        const int row = (i * 4 + wid) * 8;
+        rows[i] = (u32)(row < R ? row : batch_row<C, EPI>(t.n0, row - R) - w0) * K * 2;
     }
+    const u32 first = t.k0 * 2, behind = first + nt * 128;
+    u32 stage = first + turn * 128;
     auto issue = [&](int buf) {                // the next tile
 #pragma unroll
         for (int i = 0; i < G; ++i) {
             bf16_t* dst = lds + buf * BUF + (i * 4 + wid) * 512;
-            if (!ONCE || (i * 4 + wid) * 8 < R) load_lds16(src[i], dst);
-            else load_lds16_once(src[i], dst);
-            src[i] += 64;
+            if ((i * 4 + wid) * 8 < R) load_lds16(xs, lane_at, rows[i] + stage, dst);
+            else load_lds16<ONCE>(ws, lane_at, rows[i] + stage, dst);
         }
-        if (--left == 0)
-#pragma unroll
-            for (int i = 0; i < G; ++i) src[i] -= nt * 64;
+        stage += 128;
+        if (stage == behind) stage = first;
     };
     // a wave's columns; with gates, the second half of its tiles are the ups
     auto col_tile = [&](int b) {
