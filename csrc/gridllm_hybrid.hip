@@ -2646,13 +2646,13 @@ static int go_moe_wide(hipStream_t st, const WideArgs& p, const void* tiles,
 template <int D, int G>
 static void launch_paged_decode(hipStream_t st, void* out, const void* q,
                                 const PagedKV<D>& kv, const int* pos,
-                                const int* slot, float* ws, int B, int ngrp,
-                                int nsplit, float scale,
+                                const int* slot, const int4* rows, float* ws,
+                                int B, int ngrp, int nsplit, float scale,
                                 const HeadEpilogue& epi,
                                 const WindowKeys& keys) {
     const dim3 grid((unsigned)(B * kv.Hk * ngrp * nsplit));
     k_attn_decode<D, G><<<grid, dim3(256), 0, st>>>(
-        (bf16_t*)out, (const bf16_t*)q, kv, pos, 1, slot, ws, ngrp, nsplit,
+        (bf16_t*)out, (const bf16_t*)q, kv, pos, 1, slot, rows, ws, ngrp, nsplit,
         scale, epi, keys);
 }
 
@@ -2660,8 +2660,8 @@ template <int D>
 static int paged_decode(hipStream_t st, void* out, const void* q,
                         const void* kc, const void* vc, const int* table,
                         int per_slot, const int* pos, const int* slot,
-                        float* ws, int B, int Hq, int Hk, int nsplit,
-                        float scale, const HeadEpilogue& epi,
+                        const int4* rows, float* ws, int B, int Hq, int Hk,
+                        int nsplit, float scale, const HeadEpilogue& epi,
                         const WindowKeys& keys) {
     const PagedKV<D> kv{(const bf16_t*)kc, (const bf16_t*)vc, table, Hk,
                         per_slot};
@@ -2670,7 +2670,7 @@ static int paged_decode(hipStream_t st, void* out, const void* q,
     if (g > MAXG) for (g = MAXG; per % g; --g) {}
     switch (g) {
 #define CASE_G(GG) case GG: launch_paged_decode<D, GG>(st, out, q, kv, pos, \
-        slot, ws, B, per / GG, nsplit, scale, epi, keys); break;
+        slot, rows, ws, B, per / GG, nsplit, scale, epi, keys); break;
         CASE_G(1) CASE_G(2) CASE_G(3) CASE_G(4)
         CASE_G(5) CASE_G(6) CASE_G(7) CASE_G(8)
 #undef CASE_G
@@ -2947,12 +2947,12 @@ int gh_qknorm_kv(void* stream, int f32, void* qkv, void* q_out,
 // HeadEpilogue
 int gh_paged_decode(void* stream, void* out, const void* q, const void* kc,
                     const void* vc, const void* table, int per_slot,
-                    const void* pos, const void* slot, void* ws, int B,
-                    int Hq, int Hk, int D, int nsplit, float scale,
+                    const void* pos, const void* slot, const void* rows,
+                    void* ws, int B, int Hq, int Hk, int D, int nsplit, float scale,
                     int window, int keep, const void* sink, const void* gate,
                     int gate_ld, int gate_el, float oscale, int out_ld) {
     if (B < 1 || Hq % Hk || nsplit < 1 || nsplit > MAX_SPLIT || window < 0 ||
-        keep < 0)
+        keep < 0 || (unsigned long)rows % 16)
         return -100;
     const HeadEpilogue epi{(const float*)sink, (const bf16_t*)gate, gate_ld,
                            gate && gate_el, oscale, out_ld};
@@ -2960,7 +2960,7 @@ int gh_paged_decode(void* stream, void* out, const void* q, const void* kc,
     hipStream_t st_ = (hipStream_t)stream;
 #define GO(DD) return paged_decode<DD>(st_, out, q, kc, vc, \
         (const int*)table, per_slot, (const int*)pos, (const int*)slot, \
-        (float*)ws, B, Hq, Hk, nsplit, scale, epi, keys)
+        (const int4*)rows, (float*)ws, B, Hq, Hk, nsplit, scale, epi, keys)
     if (D == 64) GO(64);
     if (D == 128) GO(128);
     if (D == 256) GO(256);

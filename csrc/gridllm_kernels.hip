@@ -153,22 +153,47 @@ k_rmsnorm_parts(bf16_t* __restrict__ y, const float* __restrict__ ws, int parts,
 // a step had. A slot that there is not ends the program, as an index does that
 // torch finds out of bounds, before anything is read or counted by it.
 // ===========================================================================
+// rows (B <= ROWS_ORDERED): {row, keys, slot, -}, the longest first and equal ones in
+// the batch's order, as attention's blocks start. Four lanes count the rows that are
+// ahead of one, by LDS: in the launch that there is anyway, 5.8 us for 256 rows (4.7
+// without; 12.7 by a lane a row).
+#define ROWS_ORDERED 1024
 __global__ void __launch_bounds__(256)
 k_decode_positions(int* __restrict__ pos, int* __restrict__ slot_t,
                    int* __restrict__ pos_rope, int* __restrict__ attn_seq,
-                   const int* __restrict__ seq_lens,
+                   int4* __restrict__ rows, const int* __restrict__ seq_lens,
                    const int* __restrict__ rope_off,
                    const int* __restrict__ slot_map, int B, int slots,
                    int Smax) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= B) return;
-    const int s = slot_map[i];
+    typedef __attribute__((ext_vector_type(4))) int i32x4;
+    __shared__ __attribute__((aligned(16))) int lens[ROWS_ORDERED];
+    const int i = blockIdx.x * 64 + (threadIdx.x >> 2), part = threadIdx.x & 3;
+    const int s = i < B ? slot_map[i] : 0;
     if ((unsigned)s >= (unsigned)slots) __builtin_trap();
-    const int p = seq_lens[s];
-    pos[i] = p;
-    if (slot_t) slot_t[i] = s * Smax + p;
-    if (attn_seq) attn_seq[i] = p + 1;
-    if (pos_rope) pos_rope[i] = p + rope_off[s];
+    const int p = seq_lens[s], all = (B + 15) & ~15;
+    if (rows)
+        for (int j = threadIdx.x; j < all; j += 256) {
+            const int t = j < B ? slot_map[j] : -1;
+            lens[j] = (unsigned)t < (unsigned)slots ? seq_lens[t] : INT_MIN;
+        }
+    if (i < B && part == 0) {
+        pos[i] = p;
+        if (slot_t) slot_t[i] = s * Smax + p;
+        if (attn_seq) attn_seq[i] = p + 1;
+        if (pos_rope) pos_rope[i] = p + rope_off[s];
+    }
+    if (!rows) return;
+    __syncthreads();
+    int ahead = 0;
+#pragma unroll 4
+    for (int j = part * 4; j < all; j += 16) {
+        const i32x4 m = *(const i32x4*)(lens + j);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) ahead += m[k] > p || (m[k] == p && j + k < i);
+    }
+    ahead += __shfl_xor(ahead, 1, WAVE);
+    ahead += __shfl_xor(ahead, 2, WAVE);
+    if (i < B && part == 0) rows[ahead] = make_int4(i, p + 1, s, 0);
 }
 
 __global__ void __launch_bounds__(256)
@@ -1235,16 +1260,16 @@ template <int D>
 static int launch_attn_decode(hipStream_t st, bf16_t* out, const bf16_t* q,
                               const bf16_t* kc, const bf16_t* vc,
                               const int* seqlen, const int* slot_map,
-                              float* ws, int B, int Hk, int G, int Smax,
-                              int nsplit, float scale) {
+                              const int4* rows, float* ws, int B, int Hk, int G,
+                              int Smax, int nsplit, float scale) {
     dim3 grid((unsigned)(B * Hk * nsplit));
     const SlotKV<D> kv{kc, vc, Hk, Smax};
     const HeadEpilogue epi{nullptr, nullptr, 0};
     switch (G) {   // compile-time G keeps softmax state in registers
 #define CASE_G(GG) \
         case GG: k_attn_decode<D, GG><<<grid, dim3(256), 0, st>>>( \
-                out, q, kv, seqlen, 0, slot_map, ws, 1, nsplit, scale, epi, \
-                AllKeys()); \
+                out, q, kv, seqlen, 0, slot_map, rows, ws, 1, nsplit, scale, \
+                epi, AllKeys()); \
             break;
         CASE_G(1) CASE_G(2) CASE_G(3) CASE_G(4)
         CASE_G(5) CASE_G(6) CASE_G(7) CASE_G(8)
@@ -1298,19 +1323,29 @@ int gl_rmsnorm_parts(void* stream, void* y, const void* ws, int parts,
 // What a decode step starts with. Per batch row: position, place in the cache,
 // rotary position and number of keys of its slot. slots: of seq_lens and
 // rope_off. slot_t, pos_rope, attn_seq and rope_off may be null.
-int gl_decode_positions(void* stream, void* pos, void* slot_t, void* pos_rope,
-                        void* attn_seq, const void* seq_lens,
-                        const void* rope_off, const void* slot_map, int B,
-                        int slots, int Smax) {
-    if (slots < 1 || (pos_rope && !rope_off)) return -100;
+// rows (nullable): see k_decode_positions
+int gl_decode_start(void* stream, void* pos, void* slot_t, void* pos_rope,
+                    void* attn_seq, void* rows, const void* seq_lens,
+                    const void* rope_off, const void* slot_map, int B, int slots,
+                    int Smax) {
+    if (slots < 1 || (pos_rope && !rope_off) ||
+        (rows && (B > ROWS_ORDERED || (unsigned long)rows % 16))) return -100;
     if (B < 1) return 0;
-    k_decode_positions<<<dim3((B + 255) / 256), dim3(256), 0,
+    k_decode_positions<<<dim3((B + 63) / 64), dim3(256), 0,
                          (hipStream_t)stream>>>(
-        (int*)pos, (int*)slot_t, (int*)pos_rope, (int*)attn_seq,
+        (int*)pos, (int*)slot_t, (int*)pos_rope, (int*)attn_seq, (int4*)rows,
         (const int*)seq_lens, (const int*)rope_off, (const int*)slot_map, B,
         slots, Smax);
     LAUNCH_CHECK();
     return 0;
+}
+
+int gl_decode_positions(void* stream, void* pos, void* slot_t, void* pos_rope,
+                        void* attn_seq, const void* seq_lens,
+                        const void* rope_off, const void* slot_map, int B,
+                        int slots, int Smax) {
+    return gl_decode_start(stream, pos, slot_t, pos_rope, attn_seq, nullptr, seq_lens,
+                           rope_off, slot_map, B, slots, Smax);
 }
 
 // What it ends with: the rows' slots are one longer (rows may share a slot).
@@ -1447,10 +1482,10 @@ int gl_rope_kv(void* stream, const void* qkv, int parts, void* q_out, void* kc,
 
 int gl_attn_decode(void* stream, void* out, const void* q, const void* kc,
                    const void* vc, const void* seqlen, const void* slot_map,
-                   void* ws, int B, int Hq,
+                   const void* rows, void* ws, int B, int Hq,
                    int Hk, int D, int Smax, int nsplit, float scale) {
     const int G = Hq / Hk;
-    if (Hq % Hk != 0 || G > MAXG || nsplit < 1 || nsplit > MAX_SPLIT)
+    if ((unsigned long)rows % 16 || Hq % Hk != 0 || G > MAXG || nsplit < 1 || nsplit > MAX_SPLIT)
         return -100;
     hipStream_t st = (hipStream_t)stream;
     int rc;
@@ -1458,12 +1493,14 @@ int gl_attn_decode(void* stream, void* out, const void* q, const void* kc,
         rc = launch_attn_decode<128>(st, (bf16_t*)out, (const bf16_t*)q,
                                      (const bf16_t*)kc, (const bf16_t*)vc,
                                      (const int*)seqlen, (const int*)slot_map,
-                                     (float*)ws, B, Hk, G, Smax, nsplit, scale);
+                                     (const int4*)rows, (float*)ws, B, Hk, G,
+                                     Smax, nsplit, scale);
     } else if (D == 64) {
         rc = launch_attn_decode<64>(st, (bf16_t*)out, (const bf16_t*)q,
                                     (const bf16_t*)kc, (const bf16_t*)vc,
                                     (const int*)seqlen, (const int*)slot_map,
-                                    (float*)ws, B, Hk, G, Smax, nsplit, scale);
+                                    (const int4*)rows, (float*)ws, B, Hk, G,
+                                    Smax, nsplit, scale);
     } else {
         return -101;
     }

@@ -148,6 +148,7 @@ k_head_gemm_f32(float* __restrict__ out, const float* __restrict__ x,
 // ===========================================================================
 // Absorbed attention. Row n of a step sees the keys 0 .. pos[n] of slot[n].
 //   ql: [N][H][KR] absorbed queries; q: [N][H][P + R] for the rotated part
+//   rows: [N] {row, ..} in the order in which their blocks start, or null
 //   out: [N][H][KR] weighted sums of latents, or partial ones and their
 //   log2-domain maxima and sums, f32 [N][H][nsplit][KR + 2], if nsplit > 1
 // Block: a row, HG times 16 heads, a split of the keys. Tiles of 32 cached rows
@@ -164,8 +165,9 @@ k_latent_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ ql,
                 const bf16_t* __restrict__ q, const bf16_t* __restrict__ lat,
                 const int* __restrict__ table, int per_slot,
                 const int* __restrict__ pos, const int* __restrict__ slot,
-                float* __restrict__ ws, const Rotation rot, int N, int H,
-                int P, int nsplit, float scale) {
+                const int4* __restrict__ rows, float* __restrict__ ws,
+                const Rotation rot, int N, int H, int P, int nsplit,
+                float scale) {
     constexpr int D = KR + R, CH = D / 8;         // 16-byte pieces of a row
     constexpr int WAVES = 4 * HG;
     constexpr int LOADS = (CH / 2 + WAVES - 1) / WAVES;   // of a wave, 64 each
@@ -181,7 +183,8 @@ k_latent_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ ql,
     const int hgs = (H + 16 * HG - 1) / (16 * HG);
     const int item = (int)(blockIdx.x >> 3) / hgs * 8 + (blockIdx.x & 7);
     if (item >= N * nsplit) return;
-    const int n = item / nsplit, split = item % nsplit;
+    const int split = item % nsplit, turn = item / nsplit;
+    const int n = rows ? rows[turn].x : turn;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int g = wv >> 2, wid = wv & 3;
     const int h0 = ((int)(blockIdx.x >> 3) % hgs * HG + g) * 16;
@@ -687,10 +690,11 @@ int gn_head_gemm(void* stream, int f32, void* out, const void* x,
 
 int gn_latent_decode(void* stream, void* out, const void* ql, const void* q,
                      const void* lat, const void* table, int per_slot,
-                     const void* pos, const void* slot, void* ws,
-                     const void* cos_, const void* sin_, int nrot, int N,
-                     int H, int P, int KR, int R, int nsplit, float scale) {
-    if (N < 1 || H < 1 || nsplit < 1 || nsplit > 64 || !sizes_ok(KR, R))
+                     const void* pos, const void* slot, const void* rows,
+                     void* ws, const void* cos_, const void* sin_, int nrot,
+                     int N, int H, int P, int KR, int R, int nsplit,
+                     float scale) {
+    if (N < 1 || H < 1 || (unsigned long)rows % 16 || nsplit < 1 || nsplit > 64 || !sizes_ok(KR, R))
         return -100;
     hipStream_t st_ = (hipStream_t)stream;
     const Rotation rot{(const float*)cos_, (const float*)sin_, R / 2, nrot};
@@ -701,7 +705,7 @@ int gn_latent_decode(void* stream, void* out, const void* ql, const void* q,
 #define GO1(A, B, C) k_latent_decode<A, B, C><<<grid, 256 * C, 0, st_>>>( \
         (bf16_t*)out, (const bf16_t*)ql, (const bf16_t*)q, (const bf16_t*)lat, \
         (const int*)table, per_slot, (const int*)pos, (const int*)slot, \
-        (float*)ws, rot, N, H, P, nsplit, scale)
+        (const int4*)rows, (float*)ws, rot, N, H, P, nsplit, scale)
 #define PICK(B) do { if (KR == 64) { GO(64, B); } \
         else if (KR == 128) { GO(128, B); } \
         else if (KR == 256) { GO(256, B); } else { GO(512, B); } } while (0)

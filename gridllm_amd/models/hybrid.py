@@ -172,6 +172,10 @@ class HybridModel:
         # sizes laid out
         self.expands = dtype == "bf16" and any(
             isinstance(m, LatentMixer) for m in mixers)
+        # decode attention takes rows by their length
+        self.orders = dtype == "bf16" and any(
+            isinstance(m, (AttentionMixer, LatentMixer, ParallelMixer))
+            for m in mixers)
         self.chunks = sorted({m.chunk for m in mixers
                               if isinstance(m, TalkingMixer)}) \
             if dtype == "bf16" else []
@@ -1064,10 +1068,13 @@ class HybridModel:
         """One decode step of a batch, from device tensors alone (capturable):
         tokens [B] int64, slot_map [B] int32 -> logits f32 [B, vocab]. The
         cache must have been prepared for the slots (prepare_decode)."""
-        pos = hops.decode_lengths(self.cache.seq_lens, slot_map)
+        # (talking heads' blocks have their own places, recurrences no lengths)
+        pos, rows = hops.decode_ordered(self.cache.seq_lens, slot_map) \
+            if self.orders else (hops.decode_lengths(self.cache.seq_lens, slot_map),
+                                 None)
         st = StepMeta(nd=tokens.shape[0], pos=pos, slot=slot_map,
                       table=self.cache.table, max_len=self.max_seq,
-                      absorbed=tokens.shape[0])
+                      absorbed=tokens.shape[0], rows=rows)
         x = self._run(tokens, st)
         ops.advance_lengths(self.cache.seq_lens, slot_map)
         return self._head(x, None)

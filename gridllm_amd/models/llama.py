@@ -608,7 +608,7 @@ class LlamaModel:
         s = self.spec
         b = tokens.shape[0]
         # rope at the ABSOLUTE position (shifted slots have rope_off > 0)
-        slot_t, pos_rope, attn_seq = ops.decode_positions(
+        slot_t, pos_rope, attn_seq, rows = ops.decode_start(
             self.cache.seq_lens, slot_map, self.cache.rope_off,
             self.cache.max_seq)
         resid, normed = ops.embed_norm(tokens, self.embed,
@@ -619,7 +619,8 @@ class LlamaModel:
                             slot_t, self.hq_l, self.hkv_l, self.spec.head_dim,
                             lw.bqkv)
             attn = ops.attn_decode(q, self.cache.k[li], self.cache.v[li],
-                                   attn_seq, self.scale, slot_map=slot_map)
+                                   attn_seq, self.scale, slot_map=slot_map,
+                                   rows=rows)
             normed, resid = self._joined(attn.reshape(b, -1), lw.wo,
                                          lw.mlp_norm, resid)
             act = self._mlp_act(normed, lw)

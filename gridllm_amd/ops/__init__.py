@@ -50,6 +50,17 @@ def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
     return reference.decode_positions(seq_lens, slot_map, rope_off, smax)
 
 
+def decode_start(seq_lens: torch.Tensor, slot_map: torch.Tensor,
+                 rope_off: torch.Tensor, smax: int) -> tuple:
+    """decode_positions, and the order in which attn_decode takes the rows (or
+    None)."""
+    if _on_gpu(seq_lens):
+        from gridllm_amd.ops import hip_ops
+        return hip_ops.decode_start(
+            seq_lens, slot_map.int().contiguous(), rope_off, smax)
+    return (*reference.decode_positions(seq_lens, slot_map, rope_off, smax), None)
+
+
 def advance_lengths(seq_lens: torch.Tensor, slot_map: torch.Tensor) -> None:
     """End of a decode step: slots slot_map [B] are one longer, by each row."""
     if _on_gpu(seq_lens):
@@ -149,11 +160,12 @@ def kv_append(kcache: torch.Tensor, vcache: torch.Tensor, k_new: torch.Tensor,
 
 def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
                 seqlen: torch.Tensor, scale: float,
-                slot_map: Optional[torch.Tensor] = None) -> torch.Tensor:
+                slot_map: Optional[torch.Tensor] = None,
+                rows: Optional[torch.Tensor] = None) -> torch.Tensor:
     if _on_gpu(q):
         from gridllm_amd.ops import hip_ops
         return hip_ops.attn_decode(q, kcache, vcache, seqlen, scale,
-                                   slot_map=slot_map)
+                                   slot_map=slot_map, rows=rows)
     return reference.attn_decode(q, kcache, vcache, seqlen, scale,
                                  slot_map=slot_map)
 

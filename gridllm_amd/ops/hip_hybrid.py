@@ -48,7 +48,7 @@ _SIGS = {
     "gh_streams_join": "iipppippipppiiiif",
     "gh_streams_norm": "ippppiiiif",
     "gh_qknorm_kv": "ipppppippiiiiiiffippiiii",
-    "gh_paged_decode": "pppppipppiiiiifiippiifi",
+    "gh_paged_decode": "pppppippppiiiiifiippiifi",
     "gh_paged_prefill": "pppppipiiiifiippiifi",
     "gh_attn_rows_f32": "pppppippiiiifiippiifi",
     "gh_rec_step": "iippppppppiiiiiffi",
@@ -61,7 +61,7 @@ _SIGS = {
     "gh_moe_gemm": "iipppppiiiiiiiiffffp",
     "gn_latent_rows": "ippppippppppiiiiiiiif",
     "gn_head_gemm": "ippppiiiiili",
-    "gn_latent_decode": "pppppipppppiiiiiiif",
+    "gn_latent_decode": "pppppippppppiiiiiiif",
     "gn_latent_attn_f32": "pppppippppiiiiiif",
     "gn_latent_gather": "pppipii",
     "gn_latent_prefill": "ppppipippiiiifpi",
@@ -130,6 +130,11 @@ def decode_lengths(seq_lens: torch.Tensor,
                    slot_map: torch.Tensor) -> torch.Tensor:
     """The lengths of slots slot_map [B] int32."""
     return hip_ops.decode_lengths(seq_lens, slot_map.int().contiguous())
+
+
+def decode_ordered(seq_lens: torch.Tensor, slot_map: torch.Tensor) -> tuple:
+    """decode_lengths, and StepMeta.rows."""
+    return hip_ops.decode_ordered(seq_lens, slot_map.int().contiguous())
 
 
 def embed(tok: torch.Tensor, pos: torch.Tensor, emb: torch.Tensor,
@@ -405,7 +410,7 @@ def paged_attn(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor,
         ws = torch.empty(st.nd * h * nsplit * (p + 2), dtype=torch.float32,
                          device=q.device) if nsplit > 1 else None
         _call("gh_paged_decode", out, q, kc, vc, st.table, per, st.pos,
-              st.slot, ws, st.nd, h, g, p, nsplit, *how)
+              st.slot, st.rows, ws, st.nd, h, g, p, nsplit, *how)
     if st.tiles is not None:
         _call("gh_paged_prefill", out, q, kc, vc, st.table, per, st.tiles,
               st.tiles.shape[0], h, g, p, *how)
@@ -646,7 +651,8 @@ def latent_attn(q: torch.Tensor, lat: torch.Tensor, st: StepMeta, rot: tuple,
             ws = torch.empty(na * h * nsplit * (kr + 2), dtype=torch.float32,
                              device=q.device) if nsplit > 1 else None
             _call("gn_latent_decode", ol, ql, q, lat, st.table, per, st.pos,
-                  st.slot, ws, *rot, nrot, na, h, p, kr, r, nsplit, scale)
+                  st.slot, st.rows, ws, *rot, nrot, na, h, p, kr, r, nsplit,
+                  scale)
         _head_gemm(out, ol.view(na, h * kr), wuv, gate, na, kr)
     if na < n:
         rows = torch.empty(st.lat_rows, kr + r, dtype=q.dtype,

@@ -45,6 +45,8 @@ def _load() -> ctypes.CDLL:
     lib.gl_rmsnorm_parts.restype = c_i
     lib.gl_decode_positions.argtypes = [c_vp] * 8 + [c_i] * 3
     lib.gl_decode_positions.restype = c_i
+    lib.gl_decode_start.argtypes = [c_vp] * 9 + [c_i] * 3
+    lib.gl_decode_start.restype = c_i
     lib.gl_advance_lengths.argtypes = [c_vp] * 3 + [c_i] * 2
     lib.gl_advance_lengths.restype = c_i
     lib.gl_prompt_positions.argtypes = [c_vp] * 3 + [c_i] * 4
@@ -67,7 +69,7 @@ def _load() -> ctypes.CDLL:
     lib.gl_kv_append.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i, c_i, c_i, c_i]
     lib.gl_kv_append.restype = c_i
     lib.gl_attn_decode.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp,
-                                   c_vp, c_i, c_i, c_i, c_i, c_i, c_i, c_f]
+                                   c_vp, c_vp, c_i, c_i, c_i, c_i, c_i, c_i, c_f]
     lib.gl_attn_decode.restype = c_i
     lib.gl_gemm_skinny.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp,
                                    c_i, c_i, c_i, c_i, c_i]
@@ -168,21 +170,46 @@ def _check_ints(op: str, slot_map: torch.Tensor, *by_slot: torch.Tensor
         raise ValueError(f"{op}: lengths by slot differ")
 
 
+_ROWS_ORDERED = 1024           # rows that decode_start puts in order
+
+
+def _decode_start(seq_lens: torch.Tensor, slot_map: torch.Tensor,
+                  rope_off: Optional[torch.Tensor], smax: int, ordered: bool,
+                  what: str) -> tuple[torch.Tensor, Optional[torch.Tensor]]:
+    """[lengths | cache places | rotary positions | key counts] (without rope_off the
+    lengths alone), and the rows in order."""
+    b = slot_map.shape[0]
+    _check_ints(what, slot_map, seq_lens, *(() if rope_off is None else (rope_off,)))
+    _check_range(what + ".slot_map", slot_map, seq_lens.shape[0])
+    out = torch.empty(1 if rope_off is None else 4, b, dtype=torch.int32,
+                      device=seq_lens.device)
+    rows = torch.empty(b, 4, dtype=torch.int32, device=seq_lens.device) \
+        if ordered and 1 < b <= _ROWS_ORDERED else None
+    _check(_load().gl_decode_start(
+        _stream(), _ptr(out[0]), *((None,) * 3 if rope_off is None else map(
+            _ptr, out[1:])), _ptr(rows), _ptr(seq_lens), _ptr(rope_off),
+        _ptr(slot_map), b, seq_lens.shape[0], smax), what)
+    return out, rows
+
+
 def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
                      rope_off: torch.Tensor, smax: int
                      ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Start of a decode step over slots slot_map [B] int32 of seq_lens: cache
     places slot * smax + length, rotary positions length + rope_off[slot], and
     key counts length + 1, all int32 [B]."""
-    b = slot_map.shape[0]
-    _check_ints("decode_positions", slot_map, seq_lens, rope_off)
-    _check_range("decode_positions.slot_map", slot_map, seq_lens.shape[0])
-    out = torch.empty(4, b, dtype=torch.int32, device=seq_lens.device)
-    _check(_load().gl_decode_positions(
-        _stream(), _ptr(out[0]), _ptr(out[1]), _ptr(out[2]), _ptr(out[3]),
-        _ptr(seq_lens), _ptr(rope_off), _ptr(slot_map), b, seq_lens.shape[0],
-        smax), "decode_positions")
+    out, _ = _decode_start(seq_lens, slot_map, rope_off, smax, False,
+                           "decode_positions")
     return out[1], out[2], out[3]
+
+
+def decode_start(seq_lens: torch.Tensor, slot_map: torch.Tensor,
+                 rope_off: torch.Tensor, smax: int) -> tuple:
+    """decode_positions, and rows [B, 4] {row, keys, slot, -}, the longest first, for
+    attn_decode (None for a single row, or more than are put in order)."""
+    out, rows = _decode_start(seq_lens, slot_map, rope_off, smax, True,
+                              "decode_start")
+    return out[1], out[2], out[3], rows
 
 
 def advance_lengths(seq_lens: torch.Tensor, slot_map: torch.Tensor) -> None:
@@ -245,14 +272,13 @@ def prompts_end(seq_lens: torch.Tensor, rope_off: torch.Tensor,
 def decode_lengths(seq_lens: torch.Tensor,
                    slot_map: torch.Tensor) -> torch.Tensor:
     """The lengths of slots slot_map [B] int32."""
-    b = slot_map.shape[0]
-    _check_ints("decode_lengths", slot_map, seq_lens)
-    _check_range("decode_lengths.slot_map", slot_map, seq_lens.shape[0])
-    pos = torch.empty(b, dtype=torch.int32, device=seq_lens.device)
-    _check(_load().gl_decode_positions(
-        _stream(), _ptr(pos), None, None, None, _ptr(seq_lens), None,
-        _ptr(slot_map), b, seq_lens.shape[0], 0), "decode_lengths")
-    return pos
+    return _decode_start(seq_lens, slot_map, None, 0, False, "decode_lengths")[0][0]
+
+
+def decode_ordered(seq_lens: torch.Tensor, slot_map: torch.Tensor) -> tuple:
+    """decode_lengths, and decode_start's rows."""
+    out, rows = _decode_start(seq_lens, slot_map, None, 0, True, "decode_ordered")
+    return out[0], rows
 
 
 def embed_norm(tokens: torch.Tensor, emb: torch.Tensor, weight: torch.Tensor,
@@ -365,10 +391,12 @@ def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
                 seqlen: torch.Tensor, scale: float, nsplit: int = 0,
                 slot_map: Optional[torch.Tensor] = None,
                 ws: Optional[torch.Tensor] = None,
-                out: Optional[torch.Tensor] = None) -> torch.Tensor:
+                out: Optional[torch.Tensor] = None,
+                rows: Optional[torch.Tensor] = None) -> torch.Tensor:
     """GQA decode attention. q/out: [B,Hq,D]; caches [Slots,Hk,Smax,D];
     seqlen [B] int32; slot_map [B] int32 maps batch row -> cache slot
-    (None -> identity). nsplit=0 -> auto."""
+    (None -> identity). nsplit=0 -> auto. rows: decode_start's, which say the
+    same as seqlen and slot_map."""
     lib = _load()
     b, hq, d = q.shape
     hk, smax = kcache.shape[1], kcache.shape[2]
@@ -378,6 +406,8 @@ def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
     _check_range("attn_decode.seqlen", seqlen, smax + 1)
     if slot_map is not None:
         _check_range("attn_decode.slot_map", slot_map, kcache.shape[0])
+    assert rows is None or (rows.shape == (b, 4) and rows.dtype == torch.int32 and
+                            rows.is_contiguous())
     if out is None:
         out = torch.empty_like(q)
     if nsplit > 1 and ws is None:
@@ -386,7 +416,7 @@ def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
                          device=q.device)
     _check(lib.gl_attn_decode(_stream(), _ptr(out), _ptr(q), _ptr(kcache),
                               _ptr(vcache), _ptr(seqlen), _ptr(slot_map),
-                              _ptr(ws), b, hq, hk, d, smax, nsplit,
+                              _ptr(rows), _ptr(ws), b, hq, hk, d, smax, nsplit,
                               scale), "attn_decode")
     return out
 

@@ -22,6 +22,7 @@ def _dispatch(name: str):
 
 
 decode_lengths = _dispatch("decode_lengths")
+decode_ordered = _dispatch("decode_ordered")
 embed = _dispatch("embed")
 post_norm = _dispatch("post_norm")
 sum_norm = _dispatch("sum_norm")

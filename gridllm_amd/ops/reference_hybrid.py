@@ -55,6 +55,9 @@ class StepMeta:
                start} per 128 rows of a portion
     whole      products of more than 256 rows keep their sums over K whole (of
                steps with first tokens, or portions of prompts)
+    rows       [n, 4] {row, keys, slot, -} of a step of decode rows alone, the
+               longest first: the order in which attention takes them. None:
+               that of the step
     """
     nd: int
     pos: torch.Tensor            # [n] int32
@@ -72,6 +75,7 @@ class StepMeta:
     # by chunk size: the portions behind the absorbed tokens
     talk: dict[int, ChunkPortions] = field(default_factory=dict)
     whole: bool = False
+    rows: Optional[torch.Tensor] = None
 
     def entries(self) -> list:
         """(first token, length, slot, start) of every entry, on the host."""
@@ -151,6 +155,10 @@ class DepthAverage:
 
 def decode_lengths(seq_lens, slot_map):
     return seq_lens[slot_map.long()]
+
+
+def decode_ordered(seq_lens, slot_map):
+    return decode_lengths(seq_lens, slot_map), None
 
 
 def embed(tok, pos, emb, ptab, w=None, w_off=0.0, width=0, eps=0.0, out=None):

@@ -1256,3 +1256,44 @@ def test_attn_prefill_without_keys(dev, d):
     q, kc, vc = (torch.randn(*s, device=dev).to(torch.bfloat16)
                  for s in ((130, 4, d), (2, 2, 64, d), (2, 2, 64, d)))
     assert not hip_ops.attn_prefill_cache(q, kc, vc, 1, 0, 0, 0.1).any()
+
+
+@pytest.mark.parametrize("b", [2, 3, 16, 63, 64, 65, 255, 257, 1024])
+def test_decode_rows_in_order_gpu(dev, b):
+    """Rows by their keys, the longest first and equal ones in the batch's order; no
+    order for one row, or for more than are put in one."""
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator().manual_seed(b)
+    slots = torch.randperm(1500, generator=g)[:b].int()
+    slots[b // 2] = slots[0]                  # (a slot may have several rows)
+    lens = torch.randint(0, 9 if b % 2 else 4000, (1500,), generator=g).int()
+    off = torch.zeros_like(lens)
+    got = hip_ops.decode_start(lens.to(dev), slots.to(dev), off.to(dev), 4096)
+    for a, w in zip(got, R.decode_positions(lens, slots, off, 4096)):
+        assert torch.equal(a.cpu(), w)
+    n = lens[slots.long()]
+    order = torch.sort(n, descending=True, stable=True).indices
+    want = torch.stack([order.int(), n[order] + 1, slots[order],
+                        torch.zeros_like(slots)], 1)
+    assert torch.equal(got[3].cpu(), want)
+    assert torch.equal(hip_ops.decode_ordered(lens.to(dev), slots.to(dev))[1], got[3])
+    many = torch.zeros(1025, dtype=torch.int32, device=dev)
+    for few in (many[:1], many):
+        assert hip_ops.decode_ordered(lens.to(dev), few)[1] is None
+
+
+@pytest.mark.parametrize("nsplit", [0, 1, 3])
+@pytest.mark.parametrize("hq,hk,d", [(6, 2, 64), (24, 8, 128)])
+def test_attn_decode_in_order_gpu(dev, hq, hk, d, nsplit):
+    """The order in which rows' blocks start changes no result."""
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator(device=dev).manual_seed(hq)
+    b, smax = 37, 640
+    q, kc, vc = (torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)
+                 for s in ((b, hq, d), (b + 3, hk, smax, d), (b + 3, hk, smax, d)))
+    slots = torch.randperm(b + 3, generator=g, device=dev)[:b].int()
+    lens = torch.randint(0, smax, (b + 3,), generator=g, device=dev).int()
+    _, _, seq, rows = hip_ops.decode_start(lens, slots, torch.zeros_like(lens), smax)
+    want = hip_ops.attn_decode(q, kc, vc, seq, d ** -0.5, nsplit, slots)
+    assert torch.equal(hip_ops.attn_decode(q, kc, vc, seq, d ** -0.5, nsplit, slots,
+                                           rows=rows), want)
