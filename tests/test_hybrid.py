@@ -1155,3 +1155,29 @@ def test_prompt_attention_past_64_pages(start, ln, window):
     sc.masked_fill_((key > at) | ((at - key >= window) & (key >= 64)), -1e30)
     want = (torch.softmax(sc, -1) @ vd).transpose(0, 1)
     assert float((got.view_as(want).double() - want).abs().max()) < 0.02
+
+
+@pytest.mark.gpu
+def test_prompts_on_the_device():
+    """Token ids that a step reads from the device behind its preparation give what
+    those of the host give: 64-bit, 32-bit and strided, prompts that a step puts in
+    another order. Ones that the vocabulary has not are refused as there."""
+    lists = [tokens(40), tokens(1, seed=1), tokens(5, seed=2), tokens(130, seed=3)]
+    m = build(FULL, ("cuda", "bf16"), slots=32)
+    want = m.forward_prefill_batch([np.array(t) for t in lists],
+                                   [m.cache.alloc(0) for _ in lists])
+    kinds = (lambda t: torch.tensor(t, device="cuda"),
+             lambda t: torch.tensor(t, dtype=torch.int32, device="cuda"),
+             lambda t: torch.tensor(t, device="cuda").repeat_interleave(2)[::2])
+    for dev in kinds:
+        got = m.forward_prefill_batch([dev(t) for t in lists],
+                                      [m.cache.alloc(0) for _ in lists])
+        assert torch.equal(got, want)
+    alone = m.forward_prefill(np.array(lists[0]), m.cache.alloc(0))
+    for dev in kinds:
+        assert torch.equal(m.forward_prefill(dev(lists[0]), m.cache.alloc(0)), alone)
+        with pytest.raises(ValueError):
+            m.forward_prefill(dev([3, FULL["vocab"]]), m.cache.alloc(0))
+        with pytest.raises(ValueError):
+            m.forward_prefill_batch([dev([1]), dev([2, -1])],
+                                    [m.cache.alloc(0), m.cache.alloc(0)])
