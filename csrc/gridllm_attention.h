@@ -160,7 +160,14 @@ struct HeadEpilogue {
 //   B[k][j]: lane l holds j = l&15, same k chunk
 //   D[i][j]: lane l holds j = l&15, i = (l>>4)*4 + reg
 // Constraints: D in {64, 128, 256}; G <= 8.
+// Own: where a row's queries, new key and value come from. StoredQueries: q, and the
+// cache has the other two. Else the block makes them (own(row, head, turned, column,
+// position, lo, hi) gives 8 columns and those D / 2 further on), keeps them in LDS, and
+// one of the row's blocks of a kv head writes them to the cache.
 // ===========================================================================
+struct StoredQueries {
+    static constexpr bool MADE = false;
+};
 
 #define MAXG 8
 #define MAX_SPLIT 64
@@ -194,7 +201,7 @@ DEV_INLINE int split_steps(int steps, int nsplit) {
 
 // A kv head with more than MAXG query heads is served by `ngrp` blocks of G
 // query heads each. Sequence lengths are given as seqlen + seq_add.
-template <int D, int G, class KV, class Keys>
+template <int D, int G, class KV, class Keys, class Own = StoredQueries>
 __global__ void __launch_bounds__(256, 2)
 k_attn_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
               const KV kv,
@@ -202,7 +209,7 @@ k_attn_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
               const int* __restrict__ slot_map,
               const int4* __restrict__ rows, float* __restrict__ ws,
               int ngrp, int nsplit, float scale, const HeadEpilogue epi,
-              const Keys keys) {
+              const Keys keys, const Own own = Own()) {
     constexpr int KS = 4096 / D;           // keys of a step
     constexpr int SPB = 64 / KS;           // steps of a block of 64 keys
     constexpr int KT = KS / 16, ND = D / 32;
@@ -213,14 +220,17 @@ k_attn_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
     const int hg = (blockIdx.x / nsplit) % Hg;
     const int hk = hg / ngrp;
     int b = blockIdx.x / (nsplit * Hg), bc = b, seq;  // row, its slot, its keys
+    int place = 0;                                    // and (own) rotary position
     if (rows) {
         const int4 r = rows[b];
         b = r.x;
         seq = r.y;
         bc = r.z;
+        place = r.w;
     } else {
         if (slot_map) bc = slot_map[b];
         seq = seqlen[b] + seq_add;
+        if constexpr (Own::MADE) place = own.pos[b];
     }
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -229,6 +239,8 @@ k_attn_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
     __shared__ __attribute__((aligned(16))) float p_lds[4][G][KS];
     __shared__ float red[4][G * D];
     __shared__ float wml[4][G][2];         // per-wave m, l
+    // the row's queries, key and value
+    __shared__ __attribute__((aligned(16))) bf16_t made[Own::MADE ? (G + 2) * D : 8];
 
     const int blocks = keys.blocks(seq);
     const int steps = blocks <= 0 ? 0 : (blocks - 1) * SPB +
@@ -248,12 +260,12 @@ k_attn_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
 
     const int fr = lane & 15, kg = (lane >> 4) * 8;
     bf16x8 qf[ND];                         // head fr (or the last one)
-    {
-        const bf16_t* qr = q + ((long)b * Hq + hg * G + min(fr, G - 1)) * D +
-                           kg;
+    auto load_q = [&](const bf16_t* heads) {
+        const bf16_t* qr = heads + min(fr, G - 1) * D + kg;
 #pragma unroll
         for (int s = 0; s < ND; ++s) qf[s] = *(const bf16x8*)(qr + s * 32);
-    }
+    };
+    if constexpr (!Own::MADE) load_q(q + ((long)b * Hq + hg * G) * D);
     const float scale2 = scale * LOG2E;    // log2-domain softmax
 
     const int rg = lane / LV, d8 = (lane % LV) * 8;
@@ -310,6 +322,22 @@ k_attn_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
     auto step = [&](int st, auto MORE) {
         long next = 0;
         if constexpr (decltype(MORE)::value) next = start_of(st + 4);
+        if constexpr (Own::MADE && !decltype(MORE)::value) {
+            if (st + 1 == steps) {         // the new key, which the cache may not have
+                const int last = seq - 1 - first_key(st);
+#pragma unroll
+                for (int c = 0; c < ND; ++c) {
+                    const bf16x8 k = *(const bf16x8*)(made + G * D + kg + c * 32);
+#pragma unroll
+                    for (int t = 0; t < KT; ++t)
+                        if (t * 16 + fr >= last) kf[t][c] = k;
+                }
+                const bf16x8 v = *(const bf16x8*)(made + (G + 1) * D + d8);
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (rg * 8 + j >= last) vf[j] = __builtin_bit_cast(uint4, v);
+            }
+        }
         f32x4 s[KT];
 #pragma unroll
         for (int t = 0; t < KT; ++t) {
@@ -381,10 +409,34 @@ k_attn_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
         if constexpr (decltype(MORE)::value) load_v(st + 4, next);
         asm volatile("" ::: "memory");     // weights are read
     };
+    // the last wave makes the row ahead of its own loads, under the others'
+    if constexpr (Own::MADE) {
+        constexpr int L = D / 16;          // lanes of a head
+        for (int at = lane; wid == 3 && at < (G + 2) * L; at += 64) {
+            const int i = at / L, c = at % L * 8;
+            const int head = i < G ? hg * G + i : Hq + (i - G) * kv.Hk + hk;
+            uint4 lo, hi;
+            own(b, head, i <= G, c, place, lo, hi);
+            *(uint4*)(made + i * D + c) = lo;
+            *(uint4*)(made + i * D + c + D / 2) = hi;
+            if (i >= G && end == steps && hg % ngrp == 0) {
+                bf16_t* to = (bf16_t*)(i == G ? kv.k : kv.v) +
+                             kv.off(bc, hk, seq - 1) + c;
+                *(uint4*)to = lo;
+                *(uint4*)(to + D / 2) = hi;
+            }
+        }
+    }
     if (cur < end) {
         const long at = start_of(cur);
         load_k(cur, at);
         load_v(cur, at);
+    }
+    if constexpr (Own::MADE) {
+        lds_barrier();                     // (K and V stay under way)
+        load_q(made);
+    }
+    if (cur < end) {
         for (; cur + 4 < end; cur += 4) step(cur, std::true_type());
         step(cur, std::false_type());
     }

@@ -40,6 +40,10 @@
 struct StoredRow {
     const bf16_t* x;
     DEV_INLINE uint4 operator()(long c) const { return ((const uint4*)x)[c]; }
+    DEV_INLINE void two(long c, long d, uint4& lo, uint4& hi) const {
+        lo = (*this)(c);
+        hi = (*this)(d);
+    }
 };
 struct SummedRow {
     const float* ws;
@@ -55,6 +59,32 @@ struct SummedRow {
             for (int i = 0; i < 8; ++i) f[i] += a[i];
         }
         return pack8(f);
+    }
+    // (up to eight parts of two places at a time: one after the other they would wait
+    // two to four times)
+    DEV_INLINE void two(long c, long d, uint4& lo, uint4& hi) const {
+        float f[8] = {}, g[8] = {};
+#pragma unroll 1
+        for (int k0 = 0; k0 < parts; k0 += 8) {
+            float a[8][8], b[8][8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                if (k0 + k >= parts) break;
+                ld8(ws + (k0 + k) * stride + c * 8, a[k]);
+                ld8(ws + (k0 + k) * stride + d * 8, b[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                if (k0 + k >= parts) break;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    f[i] += a[k][i];
+                    g[i] += b[k][i];
+                }
+            }
+        }
+        lo = pack8(f);
+        hi = pack8(g);
     }
 };
 
@@ -153,7 +183,7 @@ k_rmsnorm_parts(bf16_t* __restrict__ y, const float* __restrict__ ws, int parts,
 // a step had. A slot that there is not ends the program, as an index does that
 // torch finds out of bounds, before anything is read or counted by it.
 // ===========================================================================
-// rows (B <= ROWS_ORDERED): {row, keys, slot, -}, the longest first and equal ones in
+// rows (B <= ROWS_ORDERED): {row, keys, slot, rotary position}, the longest first and equal ones in
 // the batch's order, as attention's blocks start. Four lanes count the rows that are
 // ahead of one, by LDS: in the launch that there is anyway, 5.8 us for 256 rows (4.7
 // without; 12.7 by a lane a row).
@@ -193,7 +223,8 @@ k_decode_positions(int* __restrict__ pos, int* __restrict__ slot_t,
     }
     ahead += __shfl_xor(ahead, 1, WAVE);
     ahead += __shfl_xor(ahead, 2, WAVE);
-    if (i < B && part == 0) rows[ahead] = make_int4(i, p + 1, s, 0);
+    if (i < B && part == 0)
+        rows[ahead] = make_int4(i, p + 1, s, rope_off ? p + rope_off[s] : p);
 }
 
 __global__ void __launch_bounds__(256)
@@ -399,6 +430,41 @@ k_rope_kv(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ q_out,
 // which spares the kernel that adds them up (four layers of llama3.2:1b, 45
 // tokens 323 -> 316 us).
 template <class Row>
+DEV_INLINE void turned8(const Row& rows, long src, int half, const bf16_t* bias,
+                        bool turn, const float* cos_, const float* sin_, uint4& lo,
+                        uint4& hi) {
+    rows.two(src, src + (half >> 3), lo, hi);
+    if (bias) {
+        float a[8], b[8];
+        unpack8(lo, a);
+        ld8(bias, b);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) a[k] += b[k];
+        lo = pack8(a);
+        unpack8(hi, a);
+        ld8(bias + half, b);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) a[k] += b[k];
+        hi = pack8(a);
+    }
+    if (turn) {
+        float a[8], b[8], co[8], si[8];
+        ld8(cos_, co);
+        ld8(sin_, si);
+        unpack8(lo, a);
+        unpack8(hi, b);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const float u = a[k], v = b[k];
+            a[k] = u * co[k] - v * si[k];
+            b[k] = u * si[k] + v * co[k];
+        }
+        lo = pack8(a);
+        hi = pack8(b);
+    }
+}
+
+template <class Row>
 __global__ void __launch_bounds__(256)
 k_rope_kv8(const Row rows, bf16_t* __restrict__ q_out,
            bf16_t* __restrict__ kc, bf16_t* __restrict__ vc,
@@ -412,37 +478,10 @@ k_rope_kv8(const Row rows, bf16_t* __restrict__ q_out,
     if (item >= (long)N * heads) return;
     const int c = (int)(i % lanes) * 8;
     const int n = (int)(item / heads), h = (int)(item % heads);
-    const long src = (item * D + c) >> 3;
-    uint4 lo = rows(src), hi = rows(src + (half >> 3));
-    if (bias) {
-        float a[8], b[8];
-        unpack8(lo, a);
-        ld8(bias + h * D + c, b);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) a[k] += b[k];
-        lo = pack8(a);
-        unpack8(hi, a);
-        ld8(bias + h * D + c + half, b);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) a[k] += b[k];
-        hi = pack8(a);
-    }
-    if (h < Hq + Hk) {
-        const long at = (long)pos[n] * half + c;
-        float a[8], b[8], co[8], si[8];
-        ld8(cost + at, co);
-        ld8(sint + at, si);
-        unpack8(lo, a);
-        unpack8(hi, b);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const float u = a[k], v = b[k];
-            a[k] = u * co[k] - v * si[k];
-            b[k] = u * si[k] + v * co[k];
-        }
-        lo = pack8(a);
-        hi = pack8(b);
-    }
+    const long at = h < Hq + Hk ? (long)pos[n] * half + c : 0;
+    uint4 lo, hi;
+    turned8(rows, (item * D + c) >> 3, half, bias ? bias + h * D + c : nullptr,
+            h < Hq + Hk, cost + at, sint + at, lo, hi);
     bf16_t* dst;
     if (h < Hq) {
         dst = q_out + ((long)n * Hq + h) * D + c;
@@ -455,6 +494,27 @@ k_rope_kv8(const Row rows, bf16_t* __restrict__ q_out,
     *(uint4*)dst = lo;
     *(uint4*)(dst + half) = hi;
 }
+
+// A decode row's queries, key and value for k_attn_decode (see Own there), in place of
+// that kernel ahead of it: a launch less a layer. The last wave makes them under the
+// others' loads of keys (all of them behind their own: 256 rows of up to 384 keys 54, now
+// 48; 53 with the kernel ahead). A decode step of 256 rows, 4 layers, 840 -> 805 us.
+template <int D, class Row>
+struct TurnedHeads {
+    static constexpr bool MADE = true;
+    Row rows;
+    const float *cos_, *sin_;
+    const int* pos;
+    const bf16_t* bias;
+    int heads;                         // queries', keys' and values'
+    DEV_INLINE void operator()(int row, int head, bool turn, int c, int place,
+                               uint4& lo, uint4& hi) const {
+        const long at = (long)place * (D / 2) + c;
+        turned8(rows, (((long)row * heads + head) * D + c) >> 3, D / 2,
+                bias ? bias + head * D + c : nullptr, turn, cos_ + at, sin_ + at, lo,
+                hi);
+    }
+};
 
 // ===========================================================================
 // KV-cache append.
@@ -1256,12 +1316,12 @@ k_sample_pick(int* __restrict__ out, const Pick* __restrict__ ws,
 // All return hipError_t as int (0 == success); callers must check.
 // ===========================================================================
 
-template <int D>
+template <int D, class Own>
 static int launch_attn_decode(hipStream_t st, bf16_t* out, const bf16_t* q,
                               const bf16_t* kc, const bf16_t* vc,
                               const int* seqlen, const int* slot_map,
                               const int4* rows, float* ws, int B, int Hk, int G,
-                              int Smax, int nsplit, float scale) {
+                              int Smax, int nsplit, float scale, const Own own) {
     dim3 grid((unsigned)(B * Hk * nsplit));
     const SlotKV<D> kv{kc, vc, Hk, Smax};
     const HeadEpilogue epi{nullptr, nullptr, 0};
@@ -1269,7 +1329,7 @@ static int launch_attn_decode(hipStream_t st, bf16_t* out, const bf16_t* q,
 #define CASE_G(GG) \
         case GG: k_attn_decode<D, GG><<<grid, dim3(256), 0, st>>>( \
                 out, q, kv, seqlen, 0, slot_map, rows, ws, 1, nsplit, scale, \
-                epi, AllKeys()); \
+                epi, AllKeys(), own); \
             break;
         CASE_G(1) CASE_G(2) CASE_G(3) CASE_G(4)
         CASE_G(5) CASE_G(6) CASE_G(7) CASE_G(8)
@@ -1488,23 +1548,46 @@ int gl_attn_decode(void* stream, void* out, const void* q, const void* kc,
     if ((unsigned long)rows % 16 || Hq % Hk != 0 || G > MAXG || nsplit < 1 || nsplit > MAX_SPLIT)
         return -100;
     hipStream_t st = (hipStream_t)stream;
-    int rc;
-    if (D == 128) {
-        rc = launch_attn_decode<128>(st, (bf16_t*)out, (const bf16_t*)q,
-                                     (const bf16_t*)kc, (const bf16_t*)vc,
-                                     (const int*)seqlen, (const int*)slot_map,
-                                     (const int4*)rows, (float*)ws, B, Hk, G,
-                                     Smax, nsplit, scale);
-    } else if (D == 64) {
-        rc = launch_attn_decode<64>(st, (bf16_t*)out, (const bf16_t*)q,
-                                    (const bf16_t*)kc, (const bf16_t*)vc,
-                                    (const int*)seqlen, (const int*)slot_map,
-                                    (const int4*)rows, (float*)ws, B, Hk, G,
-                                    Smax, nsplit, scale);
-    } else {
-        return -101;
-    }
-    return rc;
+#define GO(DD) return launch_attn_decode<DD>( \
+        st, (bf16_t*)out, (const bf16_t*)q, (const bf16_t*)kc, (const bf16_t*)vc, \
+        (const int*)seqlen, (const int*)slot_map, (const int4*)rows, (float*)ws, B, \
+        Hk, G, Smax, nsplit, scale, StoredQueries())
+    if (D == 128) GO(128);
+    if (D == 64) GO(64);
+#undef GO
+    return -101;
+}
+
+// The same of rows of a product [B][(Hq + 2 Hk) D], or its f32 sums in parts (> 0): q and
+// k are turned by cost and sint at pos (rows' own, if there are rows), k and v written
+// to the cache as key seqlen - 1.
+int gl_rope_attn_decode(void* stream, void* out, const void* qkv, int parts,
+                        void* kc, void* vc, const void* cost, const void* sint,
+                        const void* pos, const void* bias, const void* seqlen,
+                        const void* slot_map, const void* rows, void* ws, int B,
+                        int Hq, int Hk, int D, int Smax, int nsplit, float scale) {
+    const int G = Hq / Hk;
+    const unsigned long ptrs = (unsigned long)qkv | (unsigned long)kc |
+        (unsigned long)vc | (unsigned long)cost | (unsigned long)sint |
+        (unsigned long)bias | (unsigned long)rows;
+    if (ptrs % 16 || B < 1 || Hq % Hk != 0 || G > MAXG || nsplit < 1 ||
+        nsplit > MAX_SPLIT || parts < 0) return -100;
+    const int heads = Hq + 2 * Hk;
+#define GO(DD, Row, ...) return launch_attn_decode<DD>( \
+        (hipStream_t)stream, (bf16_t*)out, (const bf16_t*)nullptr, \
+        (const bf16_t*)kc, (const bf16_t*)vc, (const int*)seqlen, \
+        (const int*)slot_map, (const int4*)rows, (float*)ws, B, Hk, G, Smax, nsplit, \
+        scale, TurnedHeads<DD, Row>{__VA_ARGS__, (const float*)cost, \
+        (const float*)sint, (const int*)pos, (const bf16_t*)bias, heads})
+#define PICK(DD) do { \
+        if (parts) GO(DD, SummedRow, SummedRow{(const float*)qkv, \
+                                               (long)B * heads * DD, parts}); \
+        else GO(DD, StoredRow, StoredRow{(const bf16_t*)qkv}); } while (0)
+    if (D == 128) PICK(128);
+    if (D == 64) PICK(64);
+#undef PICK
+#undef GO
+    return -101;
 }
 
 int gl_gemm_skinny(void* stream, void* out, void* ws, const void* x,

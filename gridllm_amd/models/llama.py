@@ -614,13 +614,10 @@ class LlamaModel:
         resid, normed = ops.embed_norm(tokens, self.embed,
                                        self.layers[0].attn_norm, s.norm_eps)
         for li, lw in enumerate(self.layers):
-            q = ops.rope_kv(self._qkv(normed, lw), self.cache.k[li],
-                            self.cache.v[li], self.cos, self.sin, pos_rope,
-                            slot_t, self.hq_l, self.hkv_l, self.spec.head_dim,
-                            lw.bqkv)
-            attn = ops.attn_decode(q, self.cache.k[li], self.cache.v[li],
-                                   attn_seq, self.scale, slot_map=slot_map,
-                                   rows=rows)
+            attn = ops.rope_attn_decode(
+                self._qkv(normed, lw), self.cache.k[li], self.cache.v[li],
+                self.cos, self.sin, pos_rope, slot_t, attn_seq, self.hq_l,
+                self.scale, slot_map, lw.bqkv, rows)
             normed, resid = self._joined(attn.reshape(b, -1), lw.wo,
                                          lw.mlp_norm, resid)
             act = self._mlp_act(normed, lw)

@@ -170,6 +170,22 @@ def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
                                  slot_map=slot_map)
 
 
+def rope_attn_decode(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
+                     cos: torch.Tensor, sin: torch.Tensor, pos: torch.Tensor,
+                     slot: torch.Tensor, seqlen: torch.Tensor, hq: int, scale: float,
+                     slot_map: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                     rows: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """rope_kv and attn_decode of a decode step."""
+    if _on_gpu(qkv):
+        from gridllm_amd.ops import hip_ops
+        return hip_ops.rope_attn_decode(
+            qkv, kcache, vcache, cos, sin, pos, slot, seqlen, hq, scale,
+            slot_map.int().contiguous(), bias, rows)
+    q = rope_kv(qkv, kcache, vcache, cos, sin, pos, slot, hq, kcache.shape[1],
+                kcache.shape[3], bias)
+    return attn_decode(q, kcache, vcache, seqlen, scale, slot_map=slot_map)
+
+
 def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                  scale: float, causal_offset: int = 0) -> torch.Tensor:
     # view-based fallback (CPU reference path / odd head dims); the GPU

@@ -71,6 +71,9 @@ def _load() -> ctypes.CDLL:
     lib.gl_attn_decode.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp,
                                    c_vp, c_vp, c_i, c_i, c_i, c_i, c_i, c_i, c_f]
     lib.gl_attn_decode.restype = c_i
+    lib.gl_rope_attn_decode.argtypes = [c_vp] * 3 + [c_i] + [c_vp] * 10 + [
+        c_i] * 6 + [c_f]
+    lib.gl_rope_attn_decode.restype = c_i
     lib.gl_gemm_skinny.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp,
                                    c_i, c_i, c_i, c_i, c_i]
     lib.gl_gemm_skinny.restype = c_i
@@ -205,8 +208,8 @@ def decode_positions(seq_lens: torch.Tensor, slot_map: torch.Tensor,
 
 def decode_start(seq_lens: torch.Tensor, slot_map: torch.Tensor,
                  rope_off: torch.Tensor, smax: int) -> tuple:
-    """decode_positions, and rows [B, 4] {row, keys, slot, -}, the longest first, for
-    attn_decode (None for a single row, or more than are put in order)."""
+    """decode_positions, and rows [B, 4] {row, keys, slot, rotary position}, the
+    longest first, for attn_decode (None for a single row, or more than are put in order)."""
     out, rows = _decode_start(seq_lens, slot_map, rope_off, smax, True,
                               "decode_start")
     return out[1], out[2], out[3], rows
@@ -418,6 +421,59 @@ def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
                               _ptr(vcache), _ptr(seqlen), _ptr(slot_map),
                               _ptr(rows), _ptr(ws), b, hq, hk, d, smax, nsplit,
                               scale), "attn_decode")
+    return out
+
+
+def rope_attn_decode(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
+                     cos: torch.Tensor, sin: torch.Tensor, pos: torch.Tensor,
+                     slot: torch.Tensor, seqlen: torch.Tensor, hq: int, scale: float,
+                     slot_map: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                     rows: Optional[torch.Tensor] = None, nsplit: int = 0
+                     ) -> torch.Tensor:
+    """rope_kv and attn_decode of a decode step in one kernel, which makes a row's
+    queries, key and value where they are read (sizes and addresses that it does not
+    take: in two). slot: place slot_map * Smax + seqlen - 1 of each row's key.
+
+    In us, two kernels and one, rows of a product, and its sums in 5 parts: 24 heads
+    of 128 over 8, one row of 900 keys 12.5 and 9.9, 13.5 and 11.3; 24 of up to 6000
+    71.1 and 67.3, 70.7 and 69.6; 256 of up to 384 52.9 and 48.0, 56.8 and 52.9. Each
+    part of a row makes the queries anew: sums of 4 heads or more of a kv head are left
+    to two kernels if there are more than two blocks a CU (16 rows of up to 3000, 32
+    heads of 64 over 8, 1664 blocks: 27.9, 28.5; 64 of up to 2000, 12 of 128 over 2, 37.9,
+    40.0; 8 of up to 3000, 496 blocks, 20.1, 19.3)."""
+    b, d = qkv.shape[-2], kcache.shape[3]
+    hk, smax = kcache.shape[1:3]
+    parts = qkv.shape[0] if qkv.dim() == 3 else 0
+    nsplit = min(nsplit if nsplit > 0 else decode_splits(b * hk, smax), _MAX_SPLIT)
+    many = parts and nsplit > 1 and hq // hk >= 4 and b * hk * nsplit > 512
+    dense = [qkv, kcache, vcache, cos, sin] + ([] if bias is None else [bias])
+    if many or not (b and d in (64, 128) and hq and hq % hk == 0 and hq // hk <= 8 and
+            qkv.dtype == (torch.float32 if parts else torch.bfloat16) and
+            kcache.dtype == vcache.dtype == torch.bfloat16 and
+            cos.dtype == sin.dtype == torch.float32 and
+            cos.shape[1] * 2 == d == sin.shape[1] * 2 and
+            qkv.shape[-1] == (hq + 2 * hk) * d and
+            (bias is None or (bias.dtype == torch.bfloat16 and
+                              bias.shape == qkv.shape[-1:])) and
+            all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in dense) and
+            all(t.dtype == torch.int32 and t.is_contiguous()
+                for t in (pos, seqlen, slot_map))):
+        q = rope_kv(qkv, kcache, vcache, cos, sin, pos, slot, hq, hk, d, bias)
+        return attn_decode(q, kcache, vcache, seqlen, scale, nsplit, slot_map,
+                           rows=rows)
+    _check_range("rope_attn_decode.seqlen", seqlen, smax + 1)
+    _check_range("rope_attn_decode.slot_map", slot_map, kcache.shape[0])
+    _check_range("rope_attn_decode.pos", pos, cos.shape[0])
+    assert rows is None or (rows.shape == (b, 4) and rows.dtype == torch.int32 and
+                            rows.is_contiguous())
+    out = torch.empty(b, hq, d, dtype=torch.bfloat16, device=qkv.device)
+    ws = torch.empty(b * hq * nsplit * (d + 2), dtype=torch.float32,
+                     device=qkv.device) if nsplit > 1 else None
+    _check(_load().gl_rope_attn_decode(
+        _stream(), _ptr(out), _ptr(qkv), parts, _ptr(kcache), _ptr(vcache),
+        _ptr(cos), _ptr(sin), _ptr(pos), _ptr(bias), _ptr(seqlen), _ptr(slot_map),
+        _ptr(rows), _ptr(ws), b, hq, hk, d, smax, nsplit, scale),
+        "rope_attn_decode")
     return out
 
 

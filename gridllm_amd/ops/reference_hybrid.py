@@ -55,7 +55,7 @@ class StepMeta:
                start} per 128 rows of a portion
     whole      products of more than 256 rows keep their sums over K whole (of
                steps with first tokens, or portions of prompts)
-    rows       [n, 4] {row, keys, slot, -} of a step of decode rows alone, the
+    rows       [n, 4] {row, keys, slot, ..} of a step of decode rows alone, the
                longest first: the order in which attention takes them. None:
                that of the step
     """

@@ -1267,16 +1267,18 @@ def test_decode_rows_in_order_gpu(dev, b):
     slots = torch.randperm(1500, generator=g)[:b].int()
     slots[b // 2] = slots[0]                  # (a slot may have several rows)
     lens = torch.randint(0, 9 if b % 2 else 4000, (1500,), generator=g).int()
-    off = torch.zeros_like(lens)
+    off = torch.randint(0, 50, (1500,), generator=g).int()
     got = hip_ops.decode_start(lens.to(dev), slots.to(dev), off.to(dev), 4096)
     for a, w in zip(got, R.decode_positions(lens, slots, off, 4096)):
         assert torch.equal(a.cpu(), w)
     n = lens[slots.long()]
     order = torch.sort(n, descending=True, stable=True).indices
     want = torch.stack([order.int(), n[order] + 1, slots[order],
-                        torch.zeros_like(slots)], 1)
+                        n[order] + off[slots[order].long()]], 1)
     assert torch.equal(got[3].cpu(), want)
-    assert torch.equal(hip_ops.decode_ordered(lens.to(dev), slots.to(dev))[1], got[3])
+    want[:, 3] = n[order]
+    assert torch.equal(hip_ops.decode_ordered(lens.to(dev), slots.to(dev))[1].cpu(),
+                       want)
     many = torch.zeros(1025, dtype=torch.int32, device=dev)
     for few in (many[:1], many):
         assert hip_ops.decode_ordered(lens.to(dev), few)[1] is None
@@ -1297,3 +1299,41 @@ def test_attn_decode_in_order_gpu(dev, hq, hk, d, nsplit):
     want = hip_ops.attn_decode(q, kc, vc, seq, d ** -0.5, nsplit, slots)
     assert torch.equal(hip_ops.attn_decode(q, kc, vc, seq, d ** -0.5, nsplit, slots,
                                            rows=rows), want)
+
+
+@pytest.mark.parametrize("nsplit", [0, 1, 5])
+@pytest.mark.parametrize("hq,hk,d", [(6, 2, 64), (8, 1, 128), (24, 8, 128)])
+@pytest.mark.parametrize("parts,biased,ordered", [
+    (0, False, False), (3, False, True), (0, True, True), (3, True, False)])
+def test_rope_attn_decode_gpu(dev, hq, hk, d, nsplit, parts, biased, ordered):
+    """To the bit what rope_kv and attn_decode give, outputs and caches: one key, the
+    edges of steps and splits, shifted positions, and a cache whose place for the new
+    key is NaN."""
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator(device=dev).manual_seed(hq + parts)
+    keys = [1, 2, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 257, 640]
+    b, smax, width = len(keys), 640, (hq + 2 * hk) * d
+
+    def rand(*shape):
+        return torch.randn(*shape, generator=g, device=dev)
+    kc, vc = (rand(b + 2, hk, smax, d).to(torch.bfloat16) for _ in range(2))
+    slots = torch.randperm(b + 2, generator=g, device=dev)[:b].int()
+    lens = torch.zeros(b + 2, dtype=torch.int32, device=dev)
+    lens[slots.long()] = torch.tensor(keys, dtype=torch.int32, device=dev) - 1
+    for s, n in zip(slots.tolist(), keys):
+        kc[s, :, n - 1:], vc[s, :, n - 1:] = float("nan"), float("nan")
+    off = torch.randint(0, 90, (b + 2,), generator=g, device=dev).int()
+    cos, sin = R.rope_tables(d, 800)
+    cos, sin = cos.to(dev), sin.to(dev)
+    place, pos, seq, rows = hip_ops.decode_start(lens, slots, off, smax)
+    qkv = rand(parts, b, width) if parts else rand(b, width).to(torch.bfloat16)
+    bias = rand(width).to(torch.bfloat16) if biased else None
+    k2, v2 = kc.clone(), vc.clone()
+    q = hip_ops.rope_kv(qkv, k2, v2, cos, sin, pos, place, hq, hk, d, bias)
+    want = hip_ops.attn_decode(q, k2, v2, seq, d ** -0.5, nsplit, slots)
+    got = hip_ops.rope_attn_decode(qkv, kc, vc, cos, sin, pos, place, seq, hq,
+                                   d ** -0.5, slots, bias, rows if ordered else None,
+                                   nsplit)
+    assert want.isfinite().all() and torch.equal(got, want)
+    for a, w in ((kc, k2), (vc, v2)):
+        assert torch.equal(a.view(torch.int16), w.view(torch.int16))
