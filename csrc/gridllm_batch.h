@@ -1,6 +1,6 @@
 // Batch GEMM: out[M,N] = x[M,K] @ W[N,K]^T (bf16 I/O, f32 sums), for more rows
-// than k_gemm_rows takes: k_gemm_tile up to 64 rows a block, or 256 columns, k_gemm_fed
-// above.
+// than k_gemm_rows takes: k_gemm_tile up to 64 rows a block, k_gemm_fed above, and
+// k_gemm_cols in 256 columns.
 //
 // A block has RT * 16 rows by CT * 16 columns of one of `splitk` parts of K. Pieces
 // of 64 k of x and W come into rings in LDS by direct loads, 8 rows of 128 bytes
@@ -60,18 +60,26 @@ struct BatchTile {
 };
 
 template <int R, int C>
+DEV_INLINE BatchTile batch_place(const BatchArgs& p, int item) {
+    BatchTile t;
+    const int cols = p.N / C;
+    t.m0 = item % p.rblocks * R;
+    t.col = item / p.rblocks % cols;
+    t.n0 = t.col * C;
+    t.ks = item / p.rblocks / cols;
+    t.k0 = t.ks * p.kslice;
+    t.stages = (min(p.K, t.k0 + p.kslice) - t.k0) >> 6;
+    return t;
+}
+
+template <int R, int C>
 DEV_INLINE bool batch_tile(const BatchArgs& p, BatchTile* t) {
-    const int cols = p.N / C, total = cols * p.splitk * p.rblocks;
+    const int total = p.N / C * p.splitk * p.rblocks;
     const int each = (total + 7) >> 3;         // blocks of an XCD
     const int at = (int)(blockIdx.x >> 3);
     const int item = (int)(blockIdx.x & 7) * each + at;
     if (at >= each || item >= total) return false;
-    t->m0 = item % p.rblocks * R;
-    t->col = item / p.rblocks % cols;
-    t->n0 = t->col * C;
-    t->ks = item / p.rblocks / cols;
-    t->k0 = t->ks * p.kslice;
-    t->stages = (min(p.K, t->k0 + p.kslice) - t->k0) >> 6;
+    *t = batch_place<R, C>(p, item);
     return true;
 }
 
@@ -168,10 +176,6 @@ DEV_INLINE void batch_join(const BatchArgs& p, const BatchTile& t, int m0, int k
 // 2048 in 4 parts 4.7 -> 4.5, 3072 x 2048 7.9 -> 7.6, 64 of 3072 x 3072 in 5 7.3 -> 7.0,
 // 128 of 128256 x 3072 173.5 -> 170, what W's way from memory bounds 0 to 2 %. The
 // waves below, which only load, gain nothing by it.
-// 256 columns, for rows of x that are read once for all of them, where there are more
-// tiles than CUs anyway: a vocabulary's scores, with up to 160 rows (128256 x 3072, us
-// in 128 columns and in 256: 64 rows 159, 147, 96 178, 159, 160 198, 186; 128256 x 2048
-// 106, 100, 120, 107, 134, 128; 192 columns 160 at 64 rows).
 // ===========================================================================
 template <int RT, int CT>
 struct GemmTile {
@@ -183,7 +187,7 @@ struct GemmTile {
 };
 
 template <int RT, int CT, int EPI, bool ONCE>
-__global__ void __launch_bounds__(256, CT == 16 ? 1 : 2)
+__global__ void __launch_bounds__(256, 2)
 k_gemm_tile(const BatchArgs p) {
     typedef GemmTile<RT, CT> Sh;
     constexpr int R = Sh::R, C = Sh::C, NB = Sh::NB, BUF = (R + C) * 64;
@@ -320,6 +324,156 @@ k_gemm_tile(const BatchArgs p) {
             p, t.ks, m, acc[a],
             [&](int b) { return batch_row<C, EPI>(t.n0, col_tile(b) * 16); },
             [&](int b) { return (t.n0 >> 1) + col_tile(b) * 16; });
+    }
+}
+
+// ===========================================================================
+// 256 columns: a vocabulary's scores of up to 160 rows.
+//
+// 4 waves load, and 8 multiply, 2 by 4: with a wave a SIMD that does both, as above, the
+// products wait while the CU's queue of loads is full, a stage's time is the sum of the
+// two (1.9 us for 160 rows, .6 of them products), and a round's stores and first loads are
+// on top. Here the ring runs on from one tile to the next under the stores, a block
+// stays for its tiles, and the waves meet once a stage: the next one is there, the one
+// before is free. What is left to gain was in the stores: 160 rows without them 129 us,
+// with stores of half lines 166, of whole ones (turn_tiles) 164, of these past the
+// caches, as W goes, 152 (half ones past them 160). W's way from memory bounds it; the
+// products take 105 us alone. 128256 columns, us, k_gemm_tile in 256 columns and this:
+//   rows   24           64           96           128          160
+//   K 3072 130 -> 122   143 -> 129   158 -> 135   173 -> 142   184 -> 152
+//   K 2048                           106 -> 96                 129 -> 104
+// ===========================================================================
+template <int RT>
+struct GemmCols {
+    static constexpr int R = RT * 16, C = 256, THREADS = 768;
+    static constexpr int STAGE = (R + C) * 128;         // bytes
+    static constexpr int NB = 160 * 1024 / STAGE, BYTES = NB * STAGE;
+};
+
+template <int RT, bool ONCE>
+__global__ void __launch_bounds__(768, 3)
+k_gemm_cols(const BatchArgs p) {
+    typedef GemmCols<RT> Sh;
+    constexpr int R = Sh::R, C = Sh::C, NB = Sh::NB, BUF = (R + C) * 64;
+    constexpr int G = (R + C) / 32;            // loads of a wave and stage
+    constexpr int A = RT / 2, B = 4;           // a wave's 16 x 16 tiles
+    static_assert(RT % 2 == 0 && NB >= 3 && NB <= 4 && G * (NB - 1) < 64,
+                  "loads that can be counted");
+    extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
+    const int lane = threadIdx.x & 63, K = p.K;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // an XCD's tiles follow each other, a block's are `stride` apart
+    const int total = p.N / C * p.splitk * p.rblocks, each = (total + 7) >> 3;
+    const int first = (int)(blockIdx.x & 7) * each + (int)(blockIdx.x >> 3);
+    const int last = min(total, ((int)(blockIdx.x & 7) + 1) * each);
+    const int stride = (int)(gridDim.x >> 3);
+    if (first >= last) return;
+
+    if (wid >= 8) {                            // the loads
+        const int v = wid - 8, lr = lane >> 3;
+        const u32 lane_at = (u32)lr * K * 2 + ((lane & 7) ^ lr) * 16;
+        int item = first, left = 0;            // the tile to load, its stages
+        u32 stage = 0, begin = 0, behind = 0;
+        LdsSource xs, ws;
+        auto aim = [&] {
+            const BatchTile t = batch_place<R, C>(p, item);
+            xs = lds_source(p.x + (long)t.m0 * K, (u32)min(p.M - t.m0, R) * K * 2);
+            ws = lds_source(p.w + (long)t.n0 * K, (u32)C * K * 2);
+            begin = t.k0 * 2;
+            behind = begin + t.stages * 128;
+            stage = begin + batch_turn(p, t) * 128;
+            left = t.stages;
+        };
+        auto issue = [&](int buf) {
+#pragma unroll
+            for (int i = 0; i < G; ++i) {
+                const int row = (i * 4 + v) * 8;
+                bf16_t* dst = lds + buf * BUF + (i * 4 + v) * 512;
+                if (row < R) load_lds16(xs, lane_at, (u32)row * K * 2 + stage, dst);
+                else load_lds16<ONCE>(ws, lane_at, (u32)(row - R) * K * 2 + stage, dst);
+            }
+            stage += 128;
+            if (stage == behind) stage = begin;
+            if (--left == 0) {
+                item += stride;
+                if (item < last) aim();
+            }
+        };
+        aim();
+        int ahead = 0, buf = 0;                // stages under way, next buffer
+        for (; ahead < NB - 1 && item < last; ++ahead) {
+            issue(buf);
+            buf = buf + 1 == NB ? 0 : buf + 1;
+        }
+        while (ahead) {                        // the oldest one is there
+            if (ahead == NB - 1) WAIT_LOADS(G * (NB - 2));
+            else if (NB > 3 && ahead == 2) WAIT_LOADS(G);
+            else WAIT_LOADS(0);
+            lds_barrier();
+            --ahead;
+            if (item < last) {
+                issue(buf);
+                buf = buf + 1 == NB ? 0 : buf + 1;
+                ++ahead;
+            }
+        }
+        return;
+    }
+
+    const int fr = lane & 15, gq = lane >> 4, wr = wid >> 2, wc = wid & 3;
+    int buf = 0;
+    for (int item = first; item < last; item += stride) {
+        const BatchTile t = batch_place<R, C>(p, item);
+        f32x4 acc[A][B];
+#pragma unroll
+        for (int a = 0; a < A; ++a)
+#pragma unroll
+            for (int b = 0; b < B; ++b) acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int kt = 0; kt < t.stages; ++kt) {
+            lds_barrier();
+            bf16x8 xf[2][A], wf[2][B];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const bf16_t* s = lds + buf * BUF + ((c * 4 + gq) ^ (fr & 7)) * 8 +
+                                  fr * 64;
+#pragma unroll
+                for (int b = 0; b < B; ++b)
+                    wf[c][b] = *(const bf16x8*)(s + (R + (wc * B + b) * 16) * 64);
+#pragma unroll
+                for (int a = 0; a < A; ++a)
+                    xf[c][a] = *(const bf16x8*)(s + (wr * A + a) * 1024);
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+#pragma unroll
+                for (int a = 0; a < A; ++a)
+#pragma unroll
+                    for (int b = 0; b < B; ++b)
+                        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            wf[c][b], xf[c][a], acc[a][b], 0, 0, 0);
+            buf = buf + 1 == NB ? 0 : buf + 1;
+        }
+#pragma unroll
+        for (int a = 0; a < A; ++a) {
+            turn_tiles(acc[a]);
+            const int n = t.n0 + (wc * B + (fr >> 2)) * 16 + gq * 4;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int m = t.m0 + (wr * A + a) * 16 + j * 4 + (fr & 3);
+                if (m >= p.M) continue;
+                f32x4 v = acc[a][j];
+                if (p.splitk == 1)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] = bf2f(f2bf(v[r]));
+                if (p.splitk == 1 && p.out)
+                    *(u32x2*)(p.out + (long)m * p.N + n) =
+                        (u32x2){pack2(v[0], v[1]), pack2(v[2], v[3])};
+                else
+                    __builtin_nontemporal_store(
+                        v, (f32x4*)(p.ws + ((long)t.ks * p.M + m) * p.N + n));
+            }
+        }
     }
 }
 

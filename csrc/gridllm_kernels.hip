@@ -805,20 +805,24 @@ static bool tile_once(int M, int N, int K, int rows, int kslice) {
 
 template <int RT, int CT, int EPI, bool ONCE = false>
 static int launch_gemm_tile(hipStream_t st, BatchArgs p) {
-    constexpr bool both = RT <= 4 || CT == 16;  // waves load and multiply
-    typedef std::conditional_t<both, GemmTile<RT, CT>, GemmFed<RT, CT>> Sh;
+    constexpr bool both = RT <= 4;              // waves load and multiply
+    typedef std::conditional_t<CT == 16, GemmCols<RT>, std::conditional_t<
+        both, GemmTile<RT, CT>, GemmFed<RT, CT>>> Sh;
     p.rblocks = (p.M + Sh::R - 1) / Sh::R;
     if constexpr (!ONCE)
         if (tile_once(p.M, p.N, p.K, Sh::R, p.kslice))
             return launch_gemm_tile<RT, CT, EPI, true>(st, p);
     constexpr auto kernel = [] {
-        if constexpr (both) return k_gemm_tile<RT, CT, EPI, ONCE>;
+        if constexpr (CT == 16) return k_gemm_cols<RT, ONCE>;
+        else if constexpr (both) return k_gemm_tile<RT, CT, EPI, ONCE>;
         else return k_gemm_fed<RT, CT, EPI, ONCE>;
     }();
     const int e = allow_lds<kernel>(Sh::BYTES);
     if (e) return e;
     const long total = (long)(p.N / Sh::C) * p.splitk * p.rblocks;
-    kernel<<<(unsigned)((total + 7) / 8 * 8), Sh::THREADS, Sh::BYTES, st>>>(p);
+    const long each = (total + 7) / 8;         // (256 columns: blocks stay)
+    kernel<<<(unsigned)(8 * (CT == 16 ? min(each, 32l) : each)), Sh::THREADS,
+             Sh::BYTES, st>>>(p);
     LAUNCH_CHECK();
     return 0;
 }

@@ -75,6 +75,33 @@ DEV_INLINE float max_across16(float x) {
 // 2^x by the hardware instruction (tiny results become 0)
 DEV_INLINE float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// Products' results as they are stored: a lane has 4 columns of row l % 16 in each of 4
+// tiles v[j]. Turned, it has those of rows 4 j + l % 4 in tile l / 4 % 4: a store of 16
+// bytes a lane fills whole lines of 4 rows, 256 bytes each, and not half lines of 16.
+// (Group k of 4 lanes gets as v[j] what group j had as v[k].)
+template <int ROTATE, int GROUPS>
+DEV_INLINE float of_group(float mine, float other) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(
+        __float_as_uint(mine), __float_as_uint(other), 0x120 + ROTATE, 0xf, GROUPS,
+        false));
+}
+DEV_INLINE void turn_tiles(f32x4 (&v)[4]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        float a[4];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {          // groups 0 and 2, 1 and 3
+            a[j] = of_group<8, 0xc>(v[j][r], v[j + 2][r]);
+            a[j + 2] = of_group<8, 0x3>(v[j + 2][r], v[j][r]);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j += 2) {       // 0 and 1, 2 and 3
+            v[j][r] = of_group<4, 0xa>(a[j], a[j + 1]);
+            v[j + 1][r] = of_group<12, 0x5>(a[j + 1], a[j]);
+        }
+    }
+}
+
 // 4 x 16 block of 16-bit elements in LDS, read transposed by 16 lanes: lane l
 // passes the address of row l / 4, columns 4 (l % 4) .. + 3, and gets column l,
 // rows 0 .. 3.

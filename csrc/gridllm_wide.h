@@ -32,7 +32,8 @@
 // EPI 2: the result, rounded to bf16, as f32 (a vocabulary's scores); with one tile of
 // rows, which reads W once, past the Infinity Cache (see load_lds16_once; 256 rows of
 // 128256 x 3072 in a step 207 -> 201 us, and the step's other kernels find theirs
-// there: 4 layers 880 -> 861). More tiles of rows read W again, and would wait for memory
+// there: 4 layers 880 -> 861), and stores go past the caches, too, in whole lines (256
+// rows 200 -> 194, 192 198 -> 181). More tiles of rows read W again, and would wait for memory
 // where the Infinity Cache has it (us, through it and past it, 128256 x 3072: 257 rows 300,
 // 361, 512 444, 481, 1024 886, 936; 300 of 151936 x 896 131, 155).
 // EPI 3: squared ReLU. EPI 4: W rows in turns of 16 gate | 16 up, [M, N / 2].
@@ -240,6 +241,26 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
         // lane holds row fr and columns gq * 4 + 0 .. 3 of each tile
 #pragma unroll
         for (int a = 0; a < A; ++a) {
+            if constexpr (EPI == 2) {          // (tile b: 4 of each 8 of its pair's)
+                static_assert(B == 4, "tiles to turn");
+                f32x4 v[4];
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[b][r] = (float)(__bf16)acc[a][b][r];
+                turn_tiles(v);
+                const int n = n0 + wc * 64 + (fr >> 3) * 32 + gq * 8 +
+                              (fr >> 2 & 1) * 4;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int m = m0 + (wr * A + a) * 16 + j * 4 + (fr & 3);
+                    if (m >= t.end || n >= N) continue;
+                    f32x4* to = (f32x4*)((float*)p.out + rows.to(m) * N + n);
+                    if (Rows::ONCE) __builtin_nontemporal_store(v[j], to);
+                    else *to = v[j];
+                }
+                continue;
+            }
             const int m = m0 + (wr * A + a) * 16 + fr;
             if (m >= t.end) continue;
             const int ld = EPI == 1 || EPI == 4 ? N >> 1 : N;
@@ -274,13 +295,7 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
                         (float)(__bf16)acc[a][b + (r >> 2) + B / 2][r & 3], p.glu)
                         : EPI == 3 ? fmaxf(v, 0.f) * fmaxf(v, 0.f) : v;
                 }
-                const bf16x8 v = to_bf16x8(f);
-                if (EPI == 2) {
-                    unpack8(__builtin_bit_cast(uint4, v), f);
-                    st8((float*)p.out + at + n, f);
-                } else {
-                    *(bf16x8*)((bf16_t*)p.out + at + n) = v;
-                }
+                *(bf16x8*)((bf16_t*)p.out + at + n) = to_bf16x8(f);
             }
             if constexpr (B % 2 && EPI == 0) {
                 const int n = nw + (B - 1) * 16 + gq * 4;

@@ -1337,3 +1337,32 @@ def test_rope_attn_decode_gpu(dev, hq, hk, d, nsplit, parts, biased, ordered):
     assert want.isfinite().all() and torch.equal(got, want)
     for a, w in ((kc, k2), (vc, v2)):
         assert torch.equal(a.view(torch.int16), w.view(torch.int16))
+
+
+@pytest.mark.parametrize("rows", [32, 64, 96, 128, 160])
+@pytest.mark.parametrize("m,n,k,sk", [
+    (1, 256, 64, 1),           # a stage, of four or three that are loaded ahead
+    (33, 768, 192, 1), (160, 512, 256, 1),
+    (95, 1280, 896, 4),        # the last part of K shorter, of fewer stages
+    (161, 2304, 4096, 1),      # several blocks of rows, blocks that start further on
+    (31, 69888, 128, 1),       # two tiles a block for some, one for others
+    (200, 66048, 192, 2),      # up to eight, of unlike parts
+])
+def test_gemm_in_256_columns(dev, rows, m, n, k, sk):
+    """Results as bf16, as f32 and in parts, at edges of rows, of K's parts and of the
+    ring of stages, which runs on from one tile of a block to its next."""
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator(device=dev).manual_seed(m + k)
+    x = torch.randn(m, k, generator=g, device=dev).to(torch.bfloat16)
+    w = torch.randn(n, k, generator=g, device=dev).to(torch.bfloat16)
+    ref = x.float() @ w.float().t()
+    # bf16 result: 2^-9 of its size; K products' sums: k eps of their sizes' sum
+    small = k * 2 ** -24 * (x.float().abs() @ w.float().abs().t()) + 1e-6
+    out = torch.full((m, n), 9e9, dtype=torch.bfloat16, device=dev)
+    hip_ops.gemm_tile(x, w, rows, 256, sk, out)
+    assert bool(((out.float() - ref).abs() <= 2 ** -8 * ref.abs() + small).all())
+    if sk == 1:
+        assert torch.equal(hip_ops.gemm_tile_f32(x, w, rows, 256), out.float())
+    else:
+        parts = hip_ops.gemm_tile_parts(x, w, rows, 256, sk)
+        assert bool(((parts.sum(0) - ref).abs() <= small).all())
