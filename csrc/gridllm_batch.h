@@ -107,10 +107,13 @@ DEV_INLINE void batch_store(const BatchArgs& p, int ks, int m, const f32x4* acc,
     if (EPI && p.splitk == 1) {
 #pragma unroll
         for (int b = 0; b < B / 2; ++b) {
-            float f[4];
+            float f[4], u[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                f[r] = glu_act(acc[b][r], acc[b + B / 2][r], p.glu);
+            for (int r = 0; r < 4; ++r) {
+                f[r] = acc[b][r];
+                u[r] = acc[b + B / 2][r];
+            }
+            glu_units(f, f, u, p.glu);
             st4(p.out + (long)m * (p.N >> 1) + g(b) + gq * 4, f);
         }
         return;

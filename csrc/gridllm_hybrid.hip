@@ -2457,12 +2457,14 @@ k_moe_gemm(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
         for (int c = 0; c < 4; c += ACT == 2 ? 2 : 1) {
             const int n = (ACT == 2 ? (n0 + wc + c * 16) / 2
                                     : n0 + wc + c * 16) + (lane >> 4) * 4;
-            float f[4];
+            float f[4], u[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                f[r] = ACT == 2 ? glu_act(wi * acc[a][c][r],
-                                          wi * acc[a][(c + 1) & 3][r], glu)
+            for (int r = 0; r < 4; ++r) {
+                f[r] = ACT == 2 ? wi * acc[a][c][r]
                      : ACT == 1 ? sq_relu(acc[a][c][r]) : acc[a][c][r];
+                u[r] = wi * acc[a][(c + 1) & 3][r];
+            }
+            if (ACT == 2) glu_units(f, f, u, glu);
             if (n < NO) st4(orow + n, f);
         }
     }
@@ -2561,9 +2563,11 @@ k_moe_gemm_few(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
         v[t] = red[t][0][m][c] + red[t][1][m][c] + red[t][2][m][c] +
                red[t][3][m][c];
     const float wi = ACT == 2 && pw ? pw[sorted[tl.y + m]] : 1.f;
+    float y[1] = {ACT == 2 ? wi * v[0] : ACT == 1 ? sq_relu(v[0]) : v[0]};
+    const float u[1] = {wi * v[NW - 1]};
+    if (ACT == 2) glu_units(y, y, u, glu);
     out[(UP ? (long)tl.y + m : sorted[tl.y + m]) * (long)(N / NW) + nti * 16 +
-        c] = f2bf(ACT == 2 ? glu_act(wi * v[0], wi * v[NW - 1], glu)
-                           : ACT == 1 ? sq_relu(v[0]) : v[0]);
+        c] = f2bf(y[0]);
 }
 
 // Exact mode: 16 rows x 64 weight rows per block, f32 products.

@@ -360,10 +360,7 @@ k_swiglu(bf16_t* __restrict__ out, const bf16_t* __restrict__ gateup,
         float g[8], u[8];
         unpack8(gv, g);
         unpack8(uv, u);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            g[i] = glu_act(g[i], u[i], glu);
-        }
+        glu_units(g, g, u, glu);
         ((uint4*)(out + r * (long)F))[c] = pack8(g);
     }
 }
@@ -774,12 +771,17 @@ k_gemm_rows(bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
     }
     const int col = GLU ? (blockIdx.x >> 2) * 64 + (blockIdx.x & 3) * 16 + fr
                         : n0 + fr;
+    float y[4], u[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        y[r] = s[0][r];
+        u[r] = s[NC - 1][r];
+    }
+    if (GLU) glu_units(y, y, u, glu);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int m = (lane >> 4) * 4 + r;
-        if (m < M)
-            out[(long)m * (GLU ? N >> 1 : N) + col] =
-                f2bf(GLU ? glu_act(s[0][r], s[NC - 1][r], glu) : s[0][r]);
+        if (m < M) out[(long)m * (GLU ? N >> 1 : N) + col] = f2bf(y[r]);
     }
 }
 
@@ -867,8 +869,7 @@ k_gemm_combine_swiglu(bf16_t* __restrict__ out, const float* __restrict__ ws,
                 u[e] += b[e];
             }
         }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) g[e] = glu_act(g[e], u[e], glu);
+        glu_units(g, g, u, glu);
         st4(out + m * (long)no + j, g);
     }
 }
@@ -892,8 +893,7 @@ k_swiglu_il(bf16_t* __restrict__ out, const bf16_t* __restrict__ gu,
         float g[8], u[8];
         unpack8(gv, g);
         unpack8(uv, u);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) g[i] = glu_act(g[i], u[i], glu);
+        glu_units(g, g, u, glu);
         ((uint4*)(out + r * (long)F))[j >> 3] = pack8(g);
     }
 }

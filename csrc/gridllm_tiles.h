@@ -54,6 +54,12 @@ DEV_INLINE bf16x8 to_bf16x8(const float* f) {
     return o;
 }
 
+// to bf16's values, by two (the compiler converts one at a time)
+DEV_INLINE void round8(float (&f)[8]) {
+    const bf16x8 b = to_bf16x8(f);
+    unpack8(*(const uint4*)&b, f);
+}
+
 DEV_INLINE u32 pack2(float a, float b) {
     typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
     bf16x2 v = {(__bf16)a, (__bf16)b};

@@ -273,11 +273,13 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
                 for (int b = 0; b < B; b += 2) {
                     const int n = nw + b * 8 + gq * 4;
                     if (n >= ld) continue;
-                    float f[4];
+                    float f[4], u[4];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        f[r] = glu_act(wi * acc[a][b][r],
-                                       wi * acc[a][(b + 1) % B][r], p.glu);
+                    for (int r = 0; r < 4; ++r) {
+                        f[r] = wi * acc[a][b][r];
+                        u[r] = wi * acc[a][(b + 1) % B][r];
+                    }
+                    glu_units(f, f, u, p.glu);
                     st4((bf16_t*)p.out + at + n, f);
                 }
                 continue;
@@ -286,14 +288,17 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
             for (int b = 0; b + 1 < (EPI == 1 ? B / 2 : B); b += 2) {
                 const int n = nw + b * 16 + gq * 8;
                 if (n >= ld) continue;
-                float f[8];
+                float f[8], u[8];
 #pragma unroll
                 for (int r = 0; r < 8; ++r) {
-                    const float v = acc[a][b + (r >> 2)][r & 3];
-                    f[r] = EPI == 1 ? glu_act(
-                        (float)(__bf16)v,
-                        (float)(__bf16)acc[a][b + (r >> 2) + B / 2][r & 3], p.glu)
-                        : EPI == 3 ? fmaxf(v, 0.f) * fmaxf(v, 0.f) : v;
+                    f[r] = acc[a][b + (r >> 2)][r & 3];
+                    if (EPI == 1) u[r] = acc[a][b + (r >> 2) + B / 2][r & 3];
+                    if (EPI == 3) f[r] = fmaxf(f[r], 0.f) * fmaxf(f[r], 0.f);
+                }
+                if constexpr (EPI == 1) {
+                    round8(f);
+                    round8(u);
+                    glu_units(f, f, u, p.glu);
                 }
                 *(bf16x8*)((bf16_t*)p.out + at + n) = to_bf16x8(f);
             }

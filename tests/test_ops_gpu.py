@@ -1366,3 +1366,34 @@ def test_gemm_in_256_columns(dev, rows, m, n, k, sk):
     else:
         parts = hip_ops.gemm_tile_parts(x, w, rows, 256, sk)
         assert bool(((parts.sum(0) - ref).abs() <= small).all())
+
+
+@pytest.mark.parametrize("glu", [
+    (1.0, float("inf"), 0.0, 0.0), (1.702, float("inf"), 0.0, 0.0),
+    (1.702, 7.0, 1.0, 0.0),        # each constant alone leaves the short form
+    (1.0, 7.0, 0.0, 0.0), (1.0, float("inf"), 1.0, 0.0),
+    (1.6, float("inf"), 0.0, 0.044715)])
+def test_gated_units_of_all_sizes(dev, glu):
+    """Units of gates from 2^-20 to 2^10, both signs: where the exponential
+    overflows, where it is nothing, and where an argument is not finite."""
+    from gridllm_amd.ops import hip_ops
+    from gridllm_amd.ops.reference import Glu
+    alpha, limit, shift, cubic = glu
+    a = torch.cat([s * 2.0 ** (torch.arange(-80, 40, device=dev) / 4)
+                   for s in (1, -1)]).to(torch.bfloat16)
+    b = torch.tensor([3.0, -0.37, 0.0, 60.0], device=dev, dtype=torch.bfloat16)
+    gates, ups = (x.reshape(1, -1) for x in torch.meshgrid(a, b, indexing="ij"))
+    out = hip_ops.swiglu(torch.cat([gates, ups], 1), glu=Glu(*glu)).double()
+    g = gates.double().clamp(max=limit)
+    u = ups.double().clamp(-limit, limit)
+    z = alpha * g * (1 + cubic * g * g)
+    ref = g * torch.sigmoid(z) * (u + shift)
+    # bf16's half step; z and its multiple of log2 e, rounded, in the exponential;
+    # and what f32 keeps of the smallest (2^-126, 1024 * 61 times)
+    room = 2 ** -8 + 4 * 2 ** -24 * z.abs().clamp(max=128)
+    assert bool(((out - ref).abs() <= room * ref.abs() + 2.0 ** -110).all())
+    # a gate that is no number
+    odd = torch.ones(1, 16, device=dev, dtype=torch.bfloat16)
+    odd[0, 0] = float("nan")
+    assert bool(hip_ops.swiglu(odd, glu=Glu(1.702, float("inf"), 0.0, 0.0))[
+        0, 0].isnan())
