@@ -17,7 +17,14 @@
 //
 // Blocks stay for several tiles: the ring runs on from one to the next, under the
 // stores (16 bytes a lane: W's rows are laid into LDS in an order that gives a lane
-// 8 columns that follow each other). Tiles of an XCD are neighbours, in groups of 4
+// 8 columns that follow each other). A tile's last stage reads the next one's first
+// pieces, as every stage does, and a tile's first products add to nothing, in a copy of
+// the stage (4096 x 16384 x 3072 309 -> 302 us, 3072 x 6144 x 3072 in 192 x 192 105 ->
+// 103, 2048 x 3072 x 3072 in 192 x 128 66 -> 62.5; gated units of 192 x 256 261 -> 253).
+// What is left of a tile's end is its stores: all CUs' at once, they take 15 of 302 us
+// (measured with stores that stay in L2), and starting CUs or XCDs 1 to 6 us apart
+// changes nothing.
+// Tiles of an XCD are neighbours, in groups of 4
 // rows of tiles, so that what its 32 CUs read at a time fits in its L2: 8000 x 16384
 // x 3072 617 us in groups of 8, 600 of 4.
 //
@@ -174,9 +181,9 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
     };
     // Products of half c and half of its rows of tiles, from a0 on, between them
     // the pieces of half rc of rbuf (ahead of the last products) and loads l0 ..
-    // l1 - 1 into lbuf.
-    auto quarter = [&](int c, int a0, int rbuf, int rc, bool reads, int lbuf,
-                       int l0, int l1) {
+    // l1 - 1 into lbuf. first: the first products of a tile.
+    auto quarter = [&](auto first, int c, int a0, int rbuf, int rc, bool reads,
+                       int lbuf, int l0, int l1) {
         constexpr int Q = A / 2, PER = (A + B + Q - 2) / (Q - 1);
         const int each = (l1 - l0 + Q - 1) / Q;
 #pragma unroll
@@ -190,22 +197,25 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
 #pragma unroll
             for (int b = 0; b < B; ++b)
                 acc[a0 + j][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    wf[c][b], xf[c][a0 + j], acc[a0 + j][b], 0, 0, 0);
+                    wf[c][b], xf[c][a0 + j],
+                    decltype(first)::value ? (f32x4){0.f, 0.f, 0.f, 0.f}
+                                           : acc[a0 + j][b], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
     int buf = 0;
     // fresh: the next stage's loads are older than the stores of the tile before
-    auto stage = [&](bool fresh, auto reads) {
+    auto stage = [&](bool fresh, auto first) {
+        const std::false_type no;
         const int next = buf + 1 == NB ? 0 : buf + 1;
-        quarter(0, 0, buf, 1, true, 0, 0, 0);
+        quarter(first, 0, 0, buf, 1, true, 0, 0, 0);
         lds_barrier();                          // all have this stage
-        quarter(0, A / 2, 0, 0, false, buf, 0, L1);
-        quarter(1, 0, 0, 0, false, buf, L1, L2);
+        quarter(first, 0, A / 2, 0, 0, false, buf, 0, L1);
+        quarter(no, 1, 0, 0, 0, false, buf, L1, L2);
         if (fresh) WAIT_LOADS((NB - 2) * G + L2 + STORES);
         else WAIT_LOADS((NB - 2) * G + L2);
         lds_barrier();                          // the next one is there
-        quarter(1, A / 2, next, 0, decltype(reads)::value, buf, L2, G);
+        quarter(no, 1, A / 2, next, 0, true, buf, L2, G);
         buf = next;
     };
 
@@ -217,27 +227,26 @@ DEV_INLINE void wide_tiles(const WideArgs& p, bf16_t* lds, int item, int last,
     WAIT_LOADS(G * (NB - 1));
     lds_barrier();
     bool stored = false;                        // all of the tile before
+#pragma unroll
+    for (int i = 0; i < A + B; ++i) read(buf, 0, i);
     for (; item < last; item += stride) {
         const WideTile t = place(item);
         const int m0 = t.m0, n0 = t.n0;
+        auto ahead = [&](int kt) {
+            if (kt != nt - NB) return;          // loads go on to the next tile
+            if (item + stride < last) aim(item + stride);
+            else
 #pragma unroll
-        for (int i = 0; i < A + B; ++i) read(buf, 0, i);
-#pragma unroll
-        for (int a = 0; a < A; ++a)
-#pragma unroll
-            for (int b = 0; b < B; ++b) acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                for (int i = 0; i < G; ++i)
+                    so[i] = (u32)(i * 64 < R ? M : wrows) * K * 2;
+        };
+        ahead(0);
+        stage(stored, std::true_type());
 #pragma unroll 1
-        for (int kt = 0; kt < nt - 1; ++kt) {
-            if (kt == nt - NB) {                // loads go on to the next tile
-                if (item + stride < last) aim(item + stride);
-                else
-#pragma unroll
-                    for (int i = 0; i < G; ++i)
-                        so[i] = (u32)(i * 64 < R ? M : wrows) * K * 2;
-            }
-            stage(kt < NB - 1 && stored, std::true_type());
+        for (int kt = 1; kt < nt; ++kt) {
+            ahead(kt);
+            stage(kt < NB - 1 && stored, std::false_type());
         }
-        stage(false, std::false_type());
         // lane holds row fr and columns gq * 4 + 0 .. 3 of each tile
 #pragma unroll
         for (int a = 0; a < A; ++a) {
