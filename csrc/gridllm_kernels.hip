@@ -1721,14 +1721,15 @@ int gl_gemm_wide(void* stream, void* out, const void* x, const void* w, int M,
 //   x 12288 x 3072, take 63 us, the library 54; 160 tiles, 1200 x 4096 x 3072, 45, 40).
 //   20 us and less: what a call to the library costs the host, and twice what one
 //   here does (four layers of 0.5b, 260 tokens, are bound by that).
-//   192 x 192 and 192 x 128 tiles, which it seems not to have, where they nearly
-//   fill one or two rounds of CUs (0.93 over 17, 1.0 at most; 2731 x 3072 x 3072 56.7
-//   -> 48.4). With more rounds its larger tiles fill theirs well enough: three and four
-//   full ones of 192 x 192 take 1.01 to 1.16 of its time (4608 x 6144 x 3072 152 us,
-//   150; 6144 x 4608 x 2048 108, 95; 6144 x 6144 x 4096 246, 226).
-//   K up to 4096 and 256 x 256 tiles that fill whole rounds and up to 0.6 of one,
-//   the library's worst sizes (0.93 over 40, 1.07 at most; 8000 x 5120 x 3072 284 ->
-//   196). Elsewhere it is 5 to 10 % faster than the kernel here.
+//   Longer ones go here where the tiles fill their last round of CUs as the library's
+// do not (its time over 610 random products of 257 to 8192 rows, N 2048 to 12288, K
+// 1024 to 8192, in the mean, and at most, and that of the others of the shape):
+//   256 x 256 whose last round is .6 full at most, so that its halves fill one: .95 of
+// it, 1.13 (1.06). With one round before and K above 4096 from a quarter on: 1.09
+// below. 256 x 192 from the third round on, that one .6 full at least: .91, 1.05 (1.05).
+// 192 x 192 in rounds nearly full, or more than one: .95, 1.08 (no others). 192 x 128
+// likewise: .97, 1.12 (1.26). Some sizes the library takes 1.3 to 1.8 times as long for
+// (8000 x 5120 x 3072, 2800 x 8192 x 4096).
 //   whole: not in parts of K, and gated units by k_gemm_wide, whose sums and roundings
 // are the library's but where that cuts K itself (more than 99.9 % of results are the
 // same to the bit). Where a model makes much of a rounding (a sequence's first token
@@ -1786,9 +1787,12 @@ int gl_gemm_plan(int M, int N, int K, int epi, int whole, int* plan) {
                            ((N + t.cols - 1) / t.cols);
         const long some = tiles % 256;
         if (plan[1] == 0)
-            here |= K <= 4096 && tiles > 256 && some > 0 && some <= 154;
-        else if (plan[1] != 2)
-            here |= tiles <= 512 && (some == 0 || some >= 218);
+            here |= some > 0 && some <= 160 &&
+                    (tiles > 512 || (tiles > 256 && (K <= 4096 || some >= 64)));
+        else if (plan[1] == 2)
+            here |= tiles > 512 && some >= 160;
+        else
+            here |= tiles >= 256 || some >= (plan[1] == 1 ? 218 : 208);
         if (epi == 2 && plan[1] != 0) here = false;
     }
     plan[0] = here ? way : 0;

@@ -357,21 +357,21 @@ k_gemm_wide(const WideArgs p, int full) {
 
 // Shapes by number, their sizes, and what they take, in us: a stage (`idle` of it
 // with one tile on the chip, as a whole round takes), a tile beside it (`glu` more
-// for the unit), a launch. Fitted to 270 to 590 timings each over the products of
-// the models here and 257 to 8000 rows, 3 to 6 % off in the mean.
+// for the unit), a launch. Fitted to 330 to 1550 timings each over the products of
+// the models here and 257 to 8192 rows, 3 to 4 % off in the mean.
 struct WideTimes {
     int rows, cols;
     float stage, idle, tile, glu, launch;
 };
 static constexpr WideTimes kWide[] = {
-    {256, 256, 1.367f, .724f, 5.34f, 2.74f, 2.3f},      // rest in halves
-    {192, 192, .846f, .772f, 3.99f, 0.f, 2.5f},
-    {256, 192, 1.108f, .786f, 3.86f, 0.f, 2.8f},
-    {192, 128, .639f, .817f, 1.79f, 0.f, 3.1f},
-    {192, 256, 1.167f, .777f, 1.14f, 3.33f, 3.4f},      // gated units, f32
+    {256, 256, 1.350f, .660f, 3.82f, .15f, 4.7f},       // rest in halves
+    {192, 192, .885f, .720f, 2.23f, 0.f, 5.4f},
+    {256, 192, 1.090f, .716f, 2.91f, 0.f, 5.2f},
+    {192, 128, .648f, .713f, .77f, 0.f, 5.0f},
+    {192, 256, 1.117f, .697f, .05f, 2.24f, 4.2f},       // gated units, f32
 };
-static constexpr WideTimes kWideHalf = {128, 256, .841f, .768f, 1.07f, 2.14f,
-                                        1.f};
+static constexpr WideTimes kWideHalf = {128, 256, .801f, .712f, 1.67f, .34f,
+                                        0.f};
 static constexpr int kWideShapes = 5;
 typedef WideShape<8, 4, 2> Wide256;
 typedef WideShape<4, 4, 3> WideHalf;
