@@ -1140,11 +1140,12 @@ DEV_INLINE int at_cols(int row, int c, int cols) {
     return row * cols + (c ^ ((row & 3) << 1 | (row >> 2 & 1))) * 8;
 }
 
-// 64 tokens' values, up to 256 columns of them, on their way to LDS
+// The tokens' values, up to 256 columns of them, on their way to LDS
+template <int TOKENS = 64>
 DEV_INLINE void load_values(bf16_t* vs, const bf16_t* v, long ld_, int last,
                             int cols) {
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    for (int i = 0; i < cols / 32; ++i) {
+    for (int i = 0; i < cols / 32 * TOKENS / 64; ++i) {
         const int pc = i * 256 + threadIdx.x, row = pc / (cols / 8);
         const int c = at_cols(row, pc % (cols / 8), cols) / 8 -
                       row * (cols / 8);
@@ -1434,11 +1435,12 @@ DEV_INLINE void split8(const u32* p, bf16x8& hi, bf16x8& lo) {
 
 // Output gates of a chunk, for lane = 4 columns c * 64 + wid * 16 + gq * 4 + r of
 // tokens rt * 16 + fr: on their way ahead of the last products.
-DEV_INLINE void load_gates(uint2 (&z)[4][4], const bf16_t* gate, long ld_,
+template <int RT>
+DEV_INLINE void load_gates(uint2 (&z)[4][RT], const bf16_t* gate, long ld_,
                            int last, int DV) {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int c = 0; c < 4; ++c)
             if (c * 64 < DV)
@@ -1449,16 +1451,16 @@ DEV_INLINE void load_gates(uint2 (&z)[4][4], const bf16_t* gate, long ld_,
 
 // A chunk's outputs, laid out as its gates, with all of the head's columns in the
 // block: unit RMS, times norm, times the gate's sigmoid (SILU: and the gate).
-// red: f32 [4][64] in LDS.
-template <bool SILU>
-DEV_INLINE void store_normed(bf16_t* out, const f32x4 (&acc)[4][4],
-                             float* red, const uint2 (&gates)[4][4],
+// red: f32 [4][RT * 16] in LDS.
+template <bool SILU, int RT>
+DEV_INLINE void store_normed(bf16_t* out, const f32x4 (&acc)[4][RT],
+                             float* red, const uint2 (&gates)[4][RT],
                              long out_ld, const float* norm, int len, int DV,
                              int dvtrue, float eps) {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const int fr = lane & 15, gq = lane >> 4, col0 = wid * 16 + gq * 4;
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
+    for (int rt = 0; rt < RT; ++rt) {
         float ss = 0.f;
 #pragma unroll
         for (int c = 0; c < 4; ++c)
@@ -1467,7 +1469,7 @@ DEV_INLINE void store_normed(bf16_t* out, const f32x4 (&acc)[4][4],
                 for (int r = 0; r < 4; ++r) ss += acc[c][rt][r] * acc[c][rt][r];
         ss += __shfl_xor(ss, 16, WAVE);
         ss += __shfl_xor(ss, 32, WAVE);
-        if (gq == 0) red[wid * 64 + rt * 16 + fr] = ss;
+        if (gq == 0) red[(wid * RT + rt) * 16 + fr] = ss;
     }
     float w[4][4];
 #pragma unroll
@@ -1475,9 +1477,10 @@ DEV_INLINE void store_normed(bf16_t* out, const f32x4 (&acc)[4][4],
         if (c * 64 < DV) ld4(norm + c * 64 + col0, w[c]);
     __syncthreads();
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
+    for (int rt = 0; rt < RT; ++rt) {
         const int t = rt * 16 + fr;
-        const float ss = red[t] + red[64 + t] + red[128 + t] + red[192 + t];
+        const float ss = red[t] + red[RT * 16 + t] + red[RT * 32 + t] +
+                         red[RT * 48 + t];
         const float rs = 1.f / sqrtf(ss / (float)dvtrue + eps);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
@@ -1869,106 +1872,116 @@ DEV_INLINE f32x4 mfma_split(bf16x8 ah, bf16x8 al, bf16x8 bh, bf16x8 bl,
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, c, 0, 0, 0);
 }
 
-// Block = (chunk, head, 256 value columns). Scores: wave w owns tokens 16 w ..
-// 16 w + 15. They refer to b at the end of the 16 tokens before: queries then
-// decay by exp(b_t - ref) and older keys by exp(ref - b_s), both at most 1. Keys
-// of the same 16 tokens grow by exp(ref - b_s) instead, unless a channel loses
-// so much in 16 tokens that this could overflow; then these scores are taken
-// pair by pair. Outputs: a wave owns every fourth 16 columns for all 64 tokens,
-// so that the state is read once; decayed queries and scores meet in LDS. With
-// all of a head's columns here (out), the head's norm and gate follow at once.
-// Bound by its instructions: a block alone takes 17 us, a CU with two 35, and 540
-// blocks as many rounds as 720 do. 590 blocks of it: 78 us with tokens split over
-// the waves, each reading the whole state, and 22 of the norm behind it; then 64, of
-// which the gates take 21 and the scores' decays 11. With queries through LDS, and
-// places in LDS that are one register and a constant, 540 blocks 58 -> 54 us. Eight
-// waves a block with half the columns each: 70; registers for 3 blocks a CU: 54 to 67.
+// Block = (chunk, head, 256 value columns, half): 32 of the chunk's tokens, against
+// its keys up to them (HALF 1: the later ones and all 64 keys). Scores: a wave has 16
+// tokens and every other 32 channels; two waves' sums meet in LDS. They refer to b at
+// the end of the 16 tokens before: queries then decay by exp(b_t - ref) and older keys
+// by exp(ref - b_s), both at most 1. Keys of the same 16 tokens grow by exp(ref - b_s)
+// instead, unless a channel loses so much in 16 tokens that this could overflow; then
+// these scores are taken pair by pair. Outputs: a wave owns every fourth 16 columns for
+// all 32 tokens; decayed queries and scores meet in LDS. With all of a head's columns
+// here (out), the head's norm and gate follow at once.
+// Bound by waiting (53 % of a wave's time) and its instructions (35 % of a SIMD's). With
+// all 64 tokens in a block, two a CU, a wave having one to four tiles of keys: 540 of
+// them, 12 heads of 128 x 256, took three turns of 17 us, 59 in all. 1080 of 32 tokens,
+// three a CU, their waves with 3 or 4 tiles (1 or 2): 49, and with the two of a chunk on
+// one XCD 48. Four a CU with 112 bytes spilled: 56; the state loaded earlier, into
+// registers that spill: 53.
 #define GLA_SPAN 60.f
-__global__ void __launch_bounds__(256, 2)
-k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
-                const float* __restrict__ dS, const bf16_t* __restrict__ qkv,
-                const float* __restrict__ b, const int4* __restrict__ chunks,
-                const float* __restrict__ norm, int H, int DK, int DV,
-                int ld_, float qscale, int dvtrue, float eps) {
+template <int HALF, bool FULL>
+DEV_INLINE void gla_out(float* lds, float* o, bf16_t* out,
+                        const float* dS, const bf16_t* qkv, const float* b,
+                        const int4 ch, const float* norm, int at, int v0, int H, int DK,
+                        int DV, int ld_, float qscale, int dvtrue, float eps) {
+    constexpr int T0 = HALF * 32, KT = 2 + HALF * 2;   // first token, tiles of keys
     // keys, queries and decayed queries, then values
-    __shared__ __attribute__((aligned(16))) bf16_t vs[64 * 256];
-    __shared__ __attribute__((aligned(16))) float bs[64 * 64];
+    bf16_t* const vs = (bf16_t*)lds;
+    float* const bs = lds + 24 * 256;
     bf16_t* const ks_ = vs;
     bf16_t* const qr = vs + 64 * 64;
-    bf16_t* const qs[2] = {vs + 2 * 64 * 64, vs + 3 * 64 * 64};
-    const int4 ch = chunks[blockIdx.x];
-    const int h = blockIdx.y, v0 = blockIdx.z * 256, nv = min(256, DV - v0);
+    bf16_t* const qs[2] = {vs + 96 * 64, vs + 128 * 64};
+    const int h = blockIdx.y, nv = FULL ? 256 : min(256, DV - v0);
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int fr = lane & 15, gq = lane >> 4, kg = gq * 8, r0 = wid * 16;
+    const int fr = lane & 15, gq = lane >> 4;
+    const int rt0 = wid & 1, half = wid >> 1, r0 = T0 + rt0 * 16;
     const long C = (long)H * DK;
     const int last = ch.y - 1;
     const float* bh = b + (long)ch.x * C + h * DK;     // row t at t * C
     const bf16_t* qh = qkv + (long)ch.x * ld_ + h * DK;
     const bf16_t* kh = qh + C;
     const float* ref = r0 ? bh + min(r0 - 1, last) * C : nullptr;
-    const u32* Sb = (const u32*)dS + ((long)blockIdx.x * H + h) * DV * DK +
-                    (long)(v0 + wid * 16 + fr) * DK + kg;
+    const LdsSource states =
+        lds_source(dS + ((long)at * H + h) * DV * DK, (u32)DV * DK * 4);
+    const u32 state_at = (u32)(v0 + wid * 16 + fr) * DK * 4 + gq * 32;
 
-    auto issue = [&](int k0) {         // b, queries and keys of 64 channels
+    // b, queries and keys of 64 channels; behind the last ones nothing is read
+    const u32 bbytes = (u32)(last * C + DK) * 4;
+    const u32 qbytes = (u32)(last * (long)ld_ + C + DK) * 2;
+    const LdsSource bsrc = lds_source(bh, bbytes), qsrc = lds_source(qh, qbytes);
+    u32 bat[KT], qat, kat[KT / 2];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int pc = i * 256 + threadIdx.x, row = pc >> 4;
-            load_lds16((const bf16_t*)(bh + min(row, last) * C + k0 +
-                                       ((pc & 15) ^ (row & 15)) * 4),
-                       (bf16_t*)(bs + (i * 256 + wid * 64) * 4));
-        }
+    for (int i = 0; i < KT; ++i) {
+        const int pc = i * 256 + threadIdx.x, row = pc >> 4;
+        bat[i] = (u32)(min(row, last) * C) * 4 + ((pc & 15) ^ (row & 15)) * 16;
+    }
+    {
+        const int row = threadIdx.x >> 3, c = ((threadIdx.x & 7) ^ (row & 7)) * 16;
+        qat = (u32)min(T0 + row, last) * ld_ * 2 + c;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int pc = i * 256 + threadIdx.x, row = pc >> 3;
-            const bf16_t* src = qh + (long)min(row, last) * ld_ + k0 +
-                                ((pc & 7) ^ (row & 7)) * 8;
-            load_lds16(src, qr + (i * 256 + wid * 64) * 8);
-            load_lds16(src + C, ks_ + (i * 256 + wid * 64) * 8);
-        }
+        for (int i = 0; i < KT / 2; ++i)
+            kat[i] = (u32)min(i * 32 + row, last) * ld_ * 2 + c;
+    }
+    auto issue = [&](int k0) {
+        const bool any = k0 < DK;
+        const u32 at = any ? k0 * 4 : bbytes, qa = any ? k0 * 2 : qbytes;
+#pragma unroll
+        for (int i = 0; i < KT; ++i)
+            load_lds16(bsrc, bat[i], at, (bf16_t*)(bs + (i * 256 + wid * 64) * 4));
+        load_lds16(qsrc, qat, qa, qr + wid * 64 * 8);
+#pragma unroll
+        for (int i = 0; i < KT / 2; ++i)
+            load_lds16(qsrc, kat[i], qa + (u32)C * 2, ks_ + (i * 256 + wid * 64) * 8);
     };
-    uint4 st[4][2];
-    const int tall = threadIdx.x >> 2;
+    u32x4 st[4][2];
     auto load_state = [&](int k0, int ks, int c) {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-            st[c][i] = *(const uint4*)(Sb + (long)c * 64 * DK + k0 +
-                                           ks * 32 + i * 4);
+            st[c][i] = load16(states, state_at,
+                                  (c * 64 * DK + k0 + ks * 32 + i * 4) * 4);
     };
-    issue(0);
     // ---- does a channel lose too much within these 16 tokens?
     float span = 0.f;
     for (int c = lane; c < DK; c += 64)
         span = fmaxf(span, (ref ? ref[c] : 0.f) -
                                bh[min(r0 + 15, last) * C + c]);
+    issue(0);
     const bool pairwise = wave_reduce_max(span) > GLA_SPAN;
 
     // scores, and what the entering state gives
-    const int jmax = pairwise ? wid - 1 : wid;
-    f32x4 sc[4], acc[4][4];
+    const int own = T0 / 16 + rt0, jmax = pairwise ? own - 1 : own;
+    f32x4 sc[KT], acc[4][2];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        sc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < KT; ++j) sc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc[j][c] = sc[j];
-    }
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) acc[c][rt] = (f32x4){0.f, 0.f, 0.f, 0.f};
     for (int k0 = 0; k0 < DK; k0 += 64) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         lds_barrier();
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {              // queries for the state
-            const int c = (threadIdx.x & 3) * 2 + i;
+        {                                          // queries for the state
+            const int t = threadIdx.x >> 3, c = threadIdx.x & 7;
             float e[8];
-            ld4(bs + at_f32(tall, c * 2), e);
-            ld4(bs + at_f32(tall, c * 2 + 1), e + 4);
+            ld4(bs + at_f32(T0 + t, c * 2), e);
+            ld4(bs + at_f32(T0 + t, c * 2 + 1), e + 4);
             bf16x8 hi, lo;
-            decayed8(qr + at_bf16(tall, c), e, hi, lo);
-            *(bf16x8*)(qs[0] + at_bf16(tall, c)) = hi;
-            *(bf16x8*)(qs[1] + at_bf16(tall, c)) = lo;
+            decayed8(qr + at_bf16(t, c), e, hi, lo);
+            *(bf16x8*)(qs[0] + at_bf16(t, c)) = hi;
+            *(bf16x8*)(qs[1] + at_bf16(t, c)) = lo;
         }
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const int c = ks * 4 + gq;
+        {
+            const int c = half * 4 + gq;
             // (rows behind the last hold its b; places in tiles of 16 rows)
             const int b0 = at_f32(fr, c * 2), b1 = at_f32(fr, c * 2 + 1);
             float rf[8], e[8];
@@ -1983,9 +1996,9 @@ k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
 #pragma unroll
             for (int i = 0; i < 8; ++i) e[i] -= rf[i];
             bf16x8 ah, al;
-            decayed8(qr + r0 * 64 + at_bf16(fr, c), e, ah, al);
+            decayed8(qr + rt0 * 1024 + at_bf16(fr, c), e, ah, al);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
+            for (int j = 0; j < KT; ++j) {
                 if (j > jmax) continue;
                 ld4(bs + j * 1024 + b0, e);
                 ld4(bs + j * 1024 + b1, e + 4);
@@ -1998,44 +2011,44 @@ k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
         }
 #pragma unroll
         for (int c = 0; c < 4; ++c)
-            if (c * 64 < nv) load_state(k0, 0, c);
+            if (FULL || c * 64 < nv) load_state(k0, 0, c);
         lds_barrier();
-        if (k0 + 64 < DK) issue(k0 + 64);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            bf16x8 hi[4], lo[4];
+            bf16x8 hi[2], lo[2];
 #pragma unroll
-            for (int rt = 0; rt < 4; ++rt) {
-                hi[rt] = *(const bf16x8*)(
-                    qs[0] + at_bf16(rt * 16 + fr, ks * 4 + gq));
-                lo[rt] = *(const bf16x8*)(
-                    qs[1] + at_bf16(rt * 16 + fr, ks * 4 + gq));
+            for (int rt = 0; rt < 2; ++rt) {
+                const int at = at_bf16(rt * 16 + fr, ks * 4 + gq);
+                hi[rt] = *(const bf16x8*)(qs[0] + at);
+                lo[rt] = *(const bf16x8*)(qs[1] + at);
             }
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                if (c * 64 >= nv) continue;
+                if (!FULL && c * 64 >= nv) continue;
                 bf16x8 sh, sl;
                 split8((const u32*)st[c], sh, sl);
                 if (ks == 0) load_state(k0, 1, c);
 #pragma unroll
-                for (int rt = 0; rt < 4; ++rt)
+                for (int rt = 0; rt < 2; ++rt)
                     acc[c][rt] = mfma_split(sh, sl, hi[rt], lo[rt],
                                             acc[c][rt]);
             }
+            if (ks == 0) issue(k0 + 64);
         }
     }
-    if (pairwise) {
+    WAIT_LOADS(0);                     // (zeros, of the last turn)
+    if (pairwise && half == 0) {
         const int s = min(r0 + fr, last);
         const bf16_t* kr = kh + (long)s * ld_;
-        const float* bs = bh + s * C;
+        const float* bk = bh + s * C;
         f32x4 d = {0.f, 0.f, 0.f, 0.f};
         for (int c = 0; c < DK; c += 4) {
             float kf[4], e[4];
             ld4(kr + c, kf);
-            ld4(bs + c, e);
+            ld4(bk + c, e);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int t = min(r0 + (lane >> 4) * 4 + r, last);
+                const int t = min(r0 + gq * 4 + r, last);
                 float qf[4], f[4];
                 ld4(qh + (long)t * ld_ + c, qf);
                 ld4(bh + t * C + c, f);
@@ -2045,26 +2058,36 @@ k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
             }
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (j == wid) sc[j] = d;
+        for (int j = 0; j < KT; ++j)
+            if (j == own) sc[j] = d;
     }
-    uint2 gates[4][4];
+    uint2 gates[4][2];
     if (out)
-        load_gates(gates, qkv + (long)ch.x * ld_ + 2 * C + (long)H * DV + h * DV,
-                   ld_, last, DV);
+        load_gates(gates, qkv + (long)(ch.x + T0) * ld_ + 2 * C + (long)H * DV +
+                              h * DV, ld_, last - T0, DV);
     lds_barrier();                     // keys, queries and b have been read
-    load_values(vs, qkv + (long)ch.x * ld_ + 2 * C + h * DV + v0, ld_, last,
-                nv);
-    bf16_t* const ph = (bf16_t*)bs;
-    bf16_t* const pl = ph + 64 * 64;
+    load_values<KT * 16>(vs, qkv + (long)ch.x * ld_ + 2 * C + h * DV + v0, ld_,
+                         last, nv);
+    f32x4* const meet = (f32x4*)(lds + 32 * 256) + rt0 * 256 + lane;
+    bf16_t* const ph = vs + 256 * 64;
+    bf16_t* const pl = ph + 32 * 64;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        if (j > (wid | 1)) continue;
+    for (int j = 0; j < KT; ++j)       // the other one's tiles
+        if ((j & 1) != half) meet[j * 64] = sc[j];
+    lds_barrier();
+#pragma unroll
+    for (int j = 0; j < KT; ++j)
+        if ((j & 1) == half) sc[j] += meet[j * 64];
+    lds_barrier();
+#pragma unroll
+    for (int j = 0; j < KT; ++j) {
+        if ((j & 1) != half) continue;
         const int key = j * 16 + fr;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int row = r0 + gq * 4 + r;
-            const float p = key <= row && key <= last ? sc[j][r] * qscale : 0.f;
+            const int row = rt0 * 16 + gq * 4 + r;
+            const float p =
+                key <= T0 + row && key <= last ? sc[j][r] * qscale : 0.f;
             const int at = at_bf16(row, key >> 3) + (key & 7);
             split_bf16(p, ph[at], pl[at]);
         }
@@ -2072,28 +2095,27 @@ k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
+        for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[c][rt][r] *= qscale;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lds_barrier();
     // the chunk's own values
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-        bf16x8 hi[4], lo[4];
+    for (int ks = 0; ks < KT / 2; ++ks) {
+        bf16x8 hi[2], lo[2];
 #pragma unroll
-        for (int rt = ks * 2; rt < 4; ++rt) {
-            hi[rt] =
-                *(const bf16x8*)(ph + at_bf16(rt * 16 + fr, ks * 4 + gq));
-            lo[rt] =
-                *(const bf16x8*)(pl + at_bf16(rt * 16 + fr, ks * 4 + gq));
+        for (int rt = 0; rt < 2; ++rt) {
+            const int at = at_bf16(rt * 16 + fr, ks * 4 + gq);
+            hi[rt] = *(const bf16x8*)(ph + at);
+            lo[rt] = *(const bf16x8*)(pl + at);
         }
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            if (c * 64 >= nv) continue;
+            if (!FULL && c * 64 >= nv) continue;
             const bf16x8 v = value_piece(vs, ks, c * 64 + wid * 16, nv);
 #pragma unroll
-            for (int rt = ks * 2; rt < 4; ++rt) {
+            for (int rt = 0; rt < 2; ++rt) {
                 acc[c][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                     v, hi[rt], acc[c][rt], 0, 0, 0);
                 acc[c][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
@@ -2102,23 +2124,44 @@ k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
         }
     }
     if (out) {
-        lds_barrier();                 // scores have been read
+        lds_barrier();                 // values have been read
         store_normed<true>(
-            out + ((long)ch.x * H + h) * DV, acc, bs, gates,
-            (long)H * DV, norm + h * DV, ch.y, DV, dvtrue, eps);
+            out + ((long)(ch.x + T0) * H + h) * DV, acc, lds, gates,
+            (long)H * DV, norm + h * DV, ch.y - T0, DV, dvtrue, eps);
         return;
     }
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-        const int t = rt * 16 + fr;
+    for (int rt = 0; rt < 2; ++rt) {
+        const int t = T0 + rt * 16 + fr;
         if (t > last) continue;
-        float* ob = o + ((long)(ch.x + t) * H + h) * (DV + 4) + v0 + r0 +
+        float* ob = o + ((long)(ch.x + t) * H + h) * (DV + 4) + v0 + wid * 16 +
                     gq * 4;
 #pragma unroll
         for (int c = 0; c < 4; ++c)
             if (c * 64 < nv)
                 *(f32x4*)(ob + c * 64) = acc[c][rt];
     }
+}
+
+__global__ void __launch_bounds__(256, 3)
+k_gla_chunk_out(float* __restrict__ o, bf16_t* __restrict__ out,
+                const float* __restrict__ dS, const bf16_t* __restrict__ qkv,
+                const float* __restrict__ b, const int4* __restrict__ chunks,
+                const float* __restrict__ norm, int nchunks, int H, int DK, int DV,
+                int ld_, float qscale, int dvtrue, float eps) {
+    __shared__ __attribute__((aligned(16))) float lds[40 * 256];
+    // (the two halves 8 blocks apart: on one XCD, whose L2 has the state)
+    const int x = blockIdx.x, at = (x >> 4) * 8 + (x & 7);
+    if (at >= nchunks) return;
+    const int4 ch = chunks[at];
+    const bool late = !(x & 8);
+    const int v0 = blockIdx.z * 256;
+#define GO(...) gla_out<__VA_ARGS__>(lds, o, out, dS, qkv, b, ch, norm, at, v0, H, DK, \
+                                     DV, ld_, qscale, dvtrue, eps)
+    if (late && ch.y <= 32) return;
+    if (DV - v0 >= 256) { if (late) GO(1, true); else GO(0, true); }
+    else { if (late) GO(1, false); else GO(0, false); }
+#undef GO
 }
 
 // ===========================================================================
@@ -3149,10 +3192,10 @@ int gh_gla_chunks(void* stream, void* o, void* out, void* S, void* dS,
     chunk_states<STATE_GLA>(st_, dS, S, nullptr, nullptr, nullptr, qkv, b,
                             chunks, segs, nseg, H, DK, DV, ld_);
     LAUNCH_CHECK();
-    k_gla_chunk_out<<<dim3(nchunks, H, (DV + 255) / 256), 256, 0, st_>>>(
+    k_gla_chunk_out<<<dim3((nchunks + 7) / 8 * 16, H, (DV + 255) / 256), 256, 0, st_>>>(
         (float*)o, (bf16_t*)out, (const float*)dS, (const bf16_t*)qkv,
-        (const float*)b, (const int4*)chunks, (const float*)norm, H, DK, DV,
-        ld_, qscale, dvtrue, eps);
+        (const float*)b, (const int4*)chunks, (const float*)norm, nchunks, H, DK,
+        DV, ld_, qscale, dvtrue, eps);
     LAUNCH_CHECK();
     return 0;
 }

@@ -163,6 +163,16 @@ DEV_INLINE void load_lds16(LdsSource src, u32 lane_at, u32 at, bf16_t* dst) {
 #endif
 }
 
+// 16 bytes of it into registers
+typedef __attribute__((ext_vector_type(4))) u32 u32x4;
+DEV_INLINE u32x4 load16(LdsSource src, u32 lane_at, u32 at) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_raw_buffer_load_b128(src, lane_at, at, 0);
+#else
+    return {};
+#endif
+}
+
 // Waits until no more than n loads or stores of the wave are under way.
 #define WAIT_LOADS(n) do { \
         __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | 0xf70); \

@@ -843,3 +843,48 @@ def test_gla_chunk_sizes(dk, dv):
     used = [e[2] for e in entries]
     assert float((S1.cpu()[used] - S0[used]).abs().max()) < \
         2 ** -11 * float(S0.abs().max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dk,dv", [(128, 256), (64, 128), (64, 512)])
+@pytest.mark.parametrize("tau", [16.0, 0.3])       # (.3: scores pair by pair)
+def test_gla_chunk_halves(dk, dv, tau):
+    """Chunks that end within either half of their tokens, more of them than 8.
+    (With tau .05 a token sees itself alone; where its q . k of 128 terms, 81 in
+    absolute sum, cancels to .2, 2^-16 of 81 / .2 is 2^-7.5 of its result, which is more
+    than the room here: one of 513 rows is off by 1.6 of it, as it was by 64 tokens.)"""
+    from gridllm_amd.ops import reference_hybrid
+    h, lens = 3, (1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 97)
+    g = torch.Generator().manual_seed(dk + dv)
+    n = sum(lens)
+    entries, chunks, segs, at = [], [], [], 0
+    for i, ln in enumerate(lens):
+        entries.append((at, ln, i, i % 2))
+        segs.append((i, i % 2, len(chunks), -(-ln // 64)))
+        chunks += [(at + c, min(64, ln - c), i, 0) for c in range(0, ln, 64)]
+        at += ln
+    pos = torch.cat([torch.arange(e[3], e[3] + e[1]) for e in entries])
+    slot = torch.cat([torch.full((e[1],), e[2]) for e in entries])
+
+    def t(rows):
+        return torch.tensor(rows, dtype=torch.int32, device="cuda")
+    meta = dict(nd=0, pos=pos.int(), slot=slot.int(), max_len=200,
+                table=torch.zeros(len(lens), 1, dtype=torch.int32))
+    rows = torch.randn(n, h * 2 * (dk + dv), generator=g).to(torch.bfloat16)
+    u = torch.randn(n, 8, generator=g)
+    wa, ba = torch.randn(8, h * dk, generator=g), torch.randn(h * dk,
+                                                              generator=g)
+    S = torch.randn(len(lens), h, dv, dk, generator=g)
+    norm = torch.rand(h * dv, generator=g) + 0.5
+    want = reference_hybrid.gla(rows.float(), u, wa, ba, S.clone(), norm,
+                                hops.StepMeta(segs=t(entries).cpu(), **meta), dk,
+                                dv, tau, 1e-5)
+    st = hops.StepMeta(chunks=t(chunks), chunk_segs=t(segs), segs=t(entries),
+                       **{k: v.to("cuda") if torch.is_tensor(v) else v
+                          for k, v in meta.items()})
+    got = hops.gla(rows.cuda(), u.cuda(), wa.cuda(), ba.cuda(), S.cuda(),
+                   norm.cuda(), st, dk, dv, tau, 1e-5).cpu().float()
+    # as in test_gla_chunk_sizes
+    gate = torch.nn.functional.silu(rows[:, -h * dv:].float()).abs() * norm
+    assert bool(((got - want).abs() <= 2 ** -8 * want.abs() +
+                 2 ** -11 * gate + 1e-6).all())
