@@ -838,6 +838,35 @@ def test_mlstm_chunk_sizes(dk, dv, entering):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,h", [(57, 12), (58, 12), (90, 16)])
+def test_states_past_the_caches(n, h):
+    """Decode rows whose states are just less than 90 MB, just more, and of several
+    rounds of a block: the same as the rows one by one."""
+    dk, dv = 128, 256
+    g = torch.Generator(device="cuda").manual_seed(n)
+
+    def r(*s):
+        return torch.randn(*s, generator=g, device="cuda")
+    rows = r(n, h * 2 * (dk + dv)).to(torch.bfloat16)
+    gates, norm = r(n, 2 * h), r(h * dv).abs() + 0.5
+    S, m = r(n, h, dv + 1, dk), r(n, h).abs()
+    pos = torch.arange(n, device="cuda", dtype=torch.int32) % 3    # (0: fresh)
+    slot = torch.randperm(n, generator=g, device="cuda").int()
+
+    def step(at, S, m):
+        st = hops.StepMeta(nd=at.stop - at.start, pos=pos[at], slot=slot[at],
+                           table=torch.zeros(n, 1, dtype=torch.int32,
+                                             device="cuda"), max_len=4)
+        return hops.mlstm(rows[at].contiguous(), gates[at].contiguous(), S, m,
+                          norm, st, dk, dv, 15.0, 1e-5)
+    S1, m1 = S.clone(), m.clone()
+    got = step(slice(0, n), S1, m1)
+    want = torch.cat([step(slice(i, i + 1), S, m) for i in range(n)])
+    assert torch.equal(got, want)
+    assert torch.equal(S1, S) and torch.equal(m1, m)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("heads,dv", [(16, 256), (32, 192), (2, 256)])
 @pytest.mark.parametrize("kind", ["gla", "mlstm"])
 def test_states_of_many_chunks(kind, heads, dv):
