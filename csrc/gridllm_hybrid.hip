@@ -1221,7 +1221,7 @@ k_mlstm_weights(float* __restrict__ w, float* __restrict__ scal,
 // long, by the stores where there are many. 45 chunks of 4 segments, 12 heads of 128
 // x 256: 58 us when the chunks' own contributions were written first, read and
 // added up by a second kernel; now 35, with operands that the Infinity Cache has. In a
-// step it has some of them, and they take 44; with all from memory, 51. (256 threads,
+// step it has most of them, and they take 34; with all from memory, 51. (256 threads,
 // each with twice the keys: 34, but 54 instead of 44 for one segment of 3500.) With what
 // is ahead of it and the outputs, mLSTM's 55 chunks of one segment: 127 us before, now
 // 105; of 4 heads, whose blocks are 64, 76 and 78.
