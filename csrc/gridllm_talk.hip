@@ -303,22 +303,26 @@ k_talk_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
     if (t0 >= t1) return;
     const int* tab = table + (long)slot[n] * per_slot;
 
+    // loads by descriptors: addresses are a scalar and a register kept (8 fewer, and a
+    // step of 160 rows, 8 layers, 1459 -> 1451 us)
+    u32 value_at[LOADS];                           // a lane's, in a page's half
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int pc = (i * WAVES + wv) * 64 + lane;
+        const int kv = pc / (32 * CH), row = pc / CH % 32, c = pc % CH;
+        value_at[i] = ((u32)(kv * PAGE + row) * P + (c ^ twist(row)) * 8) * 2;
+    }
+    const u32 inv_at = ((u32)(wv * 8 + (lane >> 3)) * PAGE + (lane & 7) * 4) * 4;
     auto issue = [&](int t, long page) {
-        const bf16_t* src = vc + page * G * PAGE * P + (t & 1) * 32 * P;
+        const LdsSource vsrc = lds_source(vc + page * G * PAGE * P, (u32)G * PAGE * P * 2);
+        const LdsSource isrc = lds_source(inv + page * G * PAGE, (u32)G * PAGE * 4);
         bf16_t* dst = smem + (t & 1) * Sh::TILE;
 #pragma unroll
-        for (int i = 0; i < LOADS; ++i) {
-            const int pc = (i * WAVES + wv) * 64 + lane;
-            const int kv = pc / (32 * CH), row = pc / CH % 32, c = pc % CH;
-            if (kv < G)                            // the same for a wave
-                load_lds16_once(src + ((long)kv * PAGE + row) * P +
-                                    (c ^ twist(row)) * 8,
-                                dst + (i * WAVES + wv) * 512);
-        }
-        const int kv = wv * 8 + (lane >> 3);       // 8 value heads a wave
-        if (wv * 8 < GP && kv < G)
-            load_lds16((const bf16_t*)(inv + (page * G + kv) * PAGE +
-                                       (t & 1) * 32 + (lane & 7) * 4),
+        for (int i = 0; i < LOADS; ++i)            // (behind the last head: zeros)
+            load_lds16<true>(vsrc, value_at[i], (t & 1) * 32 * P * 2,
+                             dst + (i * WAVES + wv) * 512);
+        if (wv * 8 < GP && wv * 8 + (lane >> 3) < G)   // 8 value heads a wave
+            load_lds16(isrc, inv_at, (t & 1) * 32 * 4,
                        (bf16_t*)(ivs + (t & 1) * GP * 32 + wv * 256));
     };
     // rotation of a tile's positions; 16-byte pieces swizzled by the row
