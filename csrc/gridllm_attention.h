@@ -163,7 +163,8 @@ struct HeadEpilogue {
 // Own: where a row's queries, new key and value come from. StoredQueries: q, and the
 // cache has the other two. Else the block makes them (own(row, head, turned, column,
 // position, lo, hi) gives 8 columns and those D / 2 further on), keeps them in LDS, and
-// one of the row's blocks of a kv head writes them to the cache.
+// one of the row's blocks of a kv head writes them to the cache (a row without keys has
+// no place there).
 // ===========================================================================
 struct StoredQueries {
     static constexpr bool MADE = false;
@@ -419,7 +420,7 @@ k_attn_decode(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
             own(b, head, i <= G, c, place, lo, hi);
             *(uint4*)(made + i * D + c) = lo;
             *(uint4*)(made + i * D + c + D / 2) = hi;
-            if (i >= G && end == steps && hg % ngrp == 0) {
+            if (i >= G && steps && end == steps && hg % ngrp == 0) {
                 bf16_t* to = (bf16_t*)(i == G ? kv.k : kv.v) +
                              kv.off(bc, hk, seq - 1) + c;
                 *(uint4*)to = lo;

@@ -432,7 +432,8 @@ def rope_attn_decode(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tens
                      ) -> torch.Tensor:
     """rope_kv and attn_decode of a decode step in one kernel, which makes a row's
     queries, key and value where they are read (sizes and addresses that it does not
-    take: in two). slot: place slot_map * Smax + seqlen - 1 of each row's key.
+    take: in two). slot: place slot_map * Smax + seqlen - 1 of each row's key; a row
+    of no keys gives zeros and writes none.
 
     In us, two kernels and one, rows of a product, and its sums in 5 parts: 24 heads
     of 128 over 8, one row of 900 keys 12.5 and 9.9, 13.5 and 11.3; 24 of up to 6000

@@ -1339,6 +1339,37 @@ def test_rope_attn_decode_gpu(dev, hq, hk, d, nsplit, parts, biased, ordered):
         assert torch.equal(a.view(torch.int16), w.view(torch.int16))
 
 
+@pytest.mark.parametrize("nsplit", [1, 5])
+@pytest.mark.parametrize("ordered", [False, True])
+def test_rope_attn_decode_without_keys_gpu(dev, ordered, nsplit):
+    """A row of no keys gives zeros and writes nothing, into its own slot or ahead of
+    it; the other rows are as without it."""
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator(device=dev).manual_seed(nsplit)
+    hq, hk, d, smax, slots = 6, 2, 64, 256, 5
+
+    def rand(*shape):
+        return torch.randn(*shape, generator=g, device=dev)
+    # (slot 0 is not taken by a row of no keys: there is memory ahead of each)
+    kc, vc = (rand(slots, hk, smax, d).to(torch.bfloat16) for _ in range(2))
+    slot = torch.tensor([3, 1, 4], dtype=torch.int32, device=dev)
+    seq = torch.tensor([70, 0, 1], dtype=torch.int32, device=dev)
+    pos = torch.tensor([69, 0, 0], dtype=torch.int32, device=dev)
+    rows = torch.stack([torch.arange(3, device=dev, dtype=torch.int32), seq, slot,
+                        pos], 1)[[0, 2, 1]].contiguous() if ordered else None
+    cos, sin = (t.to(dev) for t in R.rope_tables(d, 128))
+    qkv = rand(3, (hq + 2 * hk) * d).to(torch.bfloat16)
+    k2, v2 = kc.clone(), vc.clone()
+    some = [0, 2]
+    place = (slot * smax + seq - 1)[some].contiguous()
+    q = hip_ops.rope_kv(qkv[some], k2, v2, cos, sin, pos[some], place, hq, hk, d)
+    want = hip_ops.attn_decode(q, k2, v2, seq[some], d ** -0.5, nsplit, slot[some])
+    got = hip_ops.rope_attn_decode(qkv, kc, vc, cos, sin, pos, slot * smax + seq - 1,
+                                   seq, hq, d ** -0.5, slot, None, rows, nsplit)
+    assert torch.equal(got[some], want) and not got[1].any()
+    assert torch.equal(kc, k2) and torch.equal(vc, v2)
+
+
 @pytest.mark.parametrize("rows", [32, 64, 96, 128, 160])
 @pytest.mark.parametrize("m,n,k,sk", [
     (1, 256, 64, 1),           # a stage, of four or three that are loaded ahead
