@@ -1548,9 +1548,10 @@ int gl_attn_decode(void* stream, void* out, const void* q, const void* kc,
                    const void* vc, const void* seqlen, const void* slot_map,
                    const void* rows, void* ws, int B, int Hq,
                    int Hk, int D, int Smax, int nsplit, float scale) {
-    const int G = Hq / Hk;
-    if ((unsigned long)rows % 16 || Hq % Hk != 0 || G > MAXG || nsplit < 1 || nsplit > MAX_SPLIT)
+    if ((unsigned long)rows % 16 || Hq < 1 || Hk < 1 || Hq % Hk != 0 ||
+        Hq / Hk > MAXG || nsplit < 1 || nsplit > MAX_SPLIT || (nsplit > 1 && !ws))
         return -100;
+    const int G = Hq / Hk;
     hipStream_t st = (hipStream_t)stream;
 #define GO(DD) return launch_attn_decode<DD>( \
         st, (bf16_t*)out, (const bf16_t*)q, (const bf16_t*)kc, (const bf16_t*)vc, \
@@ -1570,12 +1571,13 @@ int gl_rope_attn_decode(void* stream, void* out, const void* qkv, int parts,
                         const void* pos, const void* bias, const void* seqlen,
                         const void* slot_map, const void* rows, void* ws, int B,
                         int Hq, int Hk, int D, int Smax, int nsplit, float scale) {
-    const int G = Hq / Hk;
     const unsigned long ptrs = (unsigned long)qkv | (unsigned long)kc |
         (unsigned long)vc | (unsigned long)cost | (unsigned long)sint |
         (unsigned long)bias | (unsigned long)rows;
-    if (ptrs % 16 || B < 1 || Hq % Hk != 0 || G > MAXG || nsplit < 1 ||
-        nsplit > MAX_SPLIT || parts < 0) return -100;
+    if (ptrs % 16 || B < 1 || Hq < 1 || Hk < 1 || Hq % Hk != 0 || Hq / Hk > MAXG ||
+        nsplit < 1 || nsplit > MAX_SPLIT || (nsplit > 1 && !ws) || parts < 0)
+        return -100;
+    const int G = Hq / Hk;
     const int heads = Hq + 2 * Hk;
 #define GO(DD, Row, ...) return launch_attn_decode<DD>( \
         (hipStream_t)stream, (bf16_t*)out, (const bf16_t*)nullptr, \

@@ -1102,6 +1102,8 @@ class HybridModel:
         pos, rows = hops.decode_ordered(self.cache.seq_lens, slot_map) \
             if self.orders else (hops.decode_lengths(self.cache.seq_lens, slot_map),
                                  None)
+        if rows is not None and rows.shape[0] != tokens.shape[0]:
+            rows = None                            # (more slots than tokens)
         st = StepMeta(nd=tokens.shape[0], pos=pos, slot=slot_map,
                       table=self.cache.table, max_len=self.max_seq,
                       absorbed=tokens.shape[0], rows=rows)

@@ -611,6 +611,8 @@ class LlamaModel:
         slot_t, pos_rope, attn_seq, rows = ops.decode_start(
             self.cache.seq_lens, slot_map, self.cache.rope_off,
             self.cache.max_seq)
+        if rows is not None and rows.shape[0] != b:    # more slots than tokens
+            rows = None
         resid, normed = ops.embed_norm(tokens, self.embed,
                                        self.layers[0].attn_norm, s.norm_eps)
         for li, lw in enumerate(self.layers):

@@ -22,7 +22,7 @@ import torch.nn.functional as F
 from gridllm_amd.ops import hip_ops
 from gridllm_amd.ops.build import lib_path
 from gridllm_amd.ops.hip_ops import (HipExtensionMissing, _check,
-                                     _check_range, decode_splits)
+                                     _check_range, _check_rows, decode_splits)
 from gridllm_amd.ops.reference import Glu
 from gridllm_amd.ops.reference_hybrid import (ALL_KEYS, Choice, Keys, StepMeta,
                                               Talk)
@@ -405,6 +405,7 @@ def paged_attn(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor,
               st.slot, n, h, g, p, *how)
         return out
     if st.nd:
+        _check_rows("paged_attn", st.rows, st.nd)
         groups = h // max(d for d in range(1, 9) if (h // g) % d == 0)
         nsplit = decode_splits(st.nd * groups, keys.most(st.max_len))
         ws = torch.empty(st.nd * h * nsplit * (p + 2), dtype=torch.float32,
@@ -645,6 +646,7 @@ def latent_attn(q: torch.Tensor, lat: torch.Tensor, st: StepMeta, rot: tuple,
             _call("gn_latent_attn_f32", ol, ql, q, lat, st.table, per, st.pos,
                   st.slot, *rot, nrot, na, h, p, kr, r, scale)
         else:
+            _check_rows("latent_attn", st.rows, na)
             # a CU takes one block of 32 heads, or two of 16
             blocks, fill = (na * -(-h // 32), 256) if h > 16 else (na, 512)
             nsplit = max(1, min(fill // blocks, -(-st.max_len // 128), 32))

@@ -390,6 +390,13 @@ def decode_splits(blocks: int, keys: int) -> int:
     return max(1, parts - 1 | 1)
 
 
+def _check_rows(op: str, rows: Optional[torch.Tensor], b: int) -> None:
+    """decode_start's order is of a step's b rows, by which kernels find them."""
+    if rows is not None and not (rows.shape == (b, 4) and rows.dtype == torch.int32
+                                 and rows.is_contiguous()):
+        raise ValueError(f"{op}: rows [{b}, 4], dense int32")
+
+
 def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
                 seqlen: torch.Tensor, scale: float, nsplit: int = 0,
                 slot_map: Optional[torch.Tensor] = None,
@@ -409,8 +416,7 @@ def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
     _check_range("attn_decode.seqlen", seqlen, smax + 1)
     if slot_map is not None:
         _check_range("attn_decode.slot_map", slot_map, kcache.shape[0])
-    assert rows is None or (rows.shape == (b, 4) and rows.dtype == torch.int32 and
-                            rows.is_contiguous())
+    _check_rows("attn_decode", rows, b)
     if out is None:
         out = torch.empty_like(q)
     if nsplit > 1 and ws is None:
@@ -444,6 +450,11 @@ def rope_attn_decode(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tens
     40.0; 8 of up to 3000, 496 blocks, 20.1, 19.3)."""
     b, d = qkv.shape[-2], kcache.shape[3]
     hk, smax = kcache.shape[1:3]
+    _check_rows("rope_attn_decode", rows, b)
+    if vcache.shape != kcache.shape or any(
+            t.dim() != 1 or t.shape[0] < b for t in (pos, seqlen, slot_map)):
+        raise ValueError("rope_attn_decode: caches of one shape, and a position, a "
+                         "length and a slot of each row")
     parts = qkv.shape[0] if qkv.dim() == 3 else 0
     nsplit = min(nsplit if nsplit > 0 else decode_splits(b * hk, smax), _MAX_SPLIT)
     many = parts and nsplit > 1 and hq // hk >= 4 and b * hk * nsplit > 512
@@ -465,8 +476,6 @@ def rope_attn_decode(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tens
     _check_range("rope_attn_decode.seqlen", seqlen, smax + 1)
     _check_range("rope_attn_decode.slot_map", slot_map, kcache.shape[0])
     _check_range("rope_attn_decode.pos", pos, cos.shape[0])
-    assert rows is None or (rows.shape == (b, 4) and rows.dtype == torch.int32 and
-                            rows.is_contiguous())
     out = torch.empty(b, hq, d, dtype=torch.bfloat16, device=qkv.device)
     ws = torch.empty(b * hq * nsplit * (d + 2), dtype=torch.float32,
                      device=qkv.device) if nsplit > 1 else None

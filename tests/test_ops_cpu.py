@@ -228,6 +228,35 @@ def test_decode_positions_refuse():
             *(None,) * 8, 1, 0, 64) == -100
 
 
+def test_rope_attn_decode_refuses():
+    """Operands by which the kernel would read or write behind others: caches of two
+    shapes, fewer lengths, positions or slots than rows, and an order of other rows."""
+    from gridllm_amd.ops import hip_ops
+    hq, hk, d, b = 4, 2, 64, 3
+    qkv, cos = _mat(b, (hq + 2 * hk) * d), torch.zeros(64, d // 2)
+    kc, ids = _mat(5, hk, 64, d), torch.zeros(b, dtype=torch.int32)
+
+    def call(vc=kc, pos=ids, seq=ids, slots=ids, rows=None):
+        hip_ops.rope_attn_decode(qkv, kc, vc, cos, cos, pos, ids, seq, hq, 1.0, slots,
+                                 None, rows)
+    order = torch.zeros(b, 4, dtype=torch.int32)
+    for bad in (dict(vc=kc[:4]), dict(vc=kc[:, :, :32]), dict(pos=ids[:2]),
+                dict(seq=ids[:2]), dict(slots=ids[:2]), dict(seq=ids[0]),
+                dict(rows=order[:2]), dict(rows=order[:, :3]),
+                dict(rows=order.long()), dict(rows=order.t().contiguous().t())):
+        with pytest.raises(ValueError):
+            call(**bad)
+    with pytest.raises(ValueError):
+        hip_ops.attn_decode(_mat(b, hq, d), kc, kc, ids, 1.0, rows=order[:2])
+    if hip_ops.available():
+        lib = hip_ops._load()
+        for tail in ((b, hq, 0, d, 64, 1, 1.0), (b, 0, hk, d, 64, 1, 1.0),
+                     (b, hq, hk, d, 64, 3, 1.0)):   # (parts without a workspace)
+            assert lib.gl_attn_decode(*(None,) * 9, *tail) == -100
+            assert lib.gl_rope_attn_decode(*(None,) * 3, 0, *(None,) * 10,
+                                           *tail) == -100
+
+
 def test_decode_splits():
     """Odd numbers, which spread the first parts of all rows over the chip's
     engines; none of less than 128 keys; no more than the combining kernel has."""

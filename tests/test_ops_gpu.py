@@ -1370,6 +1370,34 @@ def test_rope_attn_decode_without_keys_gpu(dev, ordered, nsplit):
     assert torch.equal(kc, k2) and torch.equal(vc, v2)
 
 
+@pytest.mark.parametrize("name", ["llama3.2:1b", "birepel:3b", "maferax:5b"])
+def test_decode_of_fewer_tokens_than_slots_gpu(dev, name):
+    """A slot without a token is as if it were not there (but for its length)."""
+    from dataclasses import replace
+    from gridllm_amd.models import model_class
+    from gridllm_amd.models.registry import DenseFF, get_spec
+    spec = get_spec(name)
+    spec = replace(spec, layers=1 if isinstance(spec.layers, int) else tuple(
+        replace(ly, ff=DenseFF(256, 7.0)) for ly in spec.layers[:2]))
+    m = model_class(spec)(spec, device=dev, dtype="bf16", kv_slots=6, max_seq=256)
+    slots = [m.cache.alloc(0) for _ in range(4)]
+    for i, s in enumerate(slots):
+        m.forward_prefill(torch.arange(5 + 40 * i, device=dev), s)
+    toks = torch.tensor([3, 5, 7], device=dev)
+    slot_map = torch.tensor(slots, dtype=torch.int32, device=dev)
+    out = []
+    kept = [m.cache.seq_lens] + [
+        t for name in ("S", "m") for t in getattr(m.cache, name, []) if t is not None]
+    were = [t.clone() for t in kept]
+    for at in (slot_map[:3].contiguous(), slot_map):
+        for t, was in zip(kept, were):
+            t.copy_(was)
+        if hasattr(m.cache, "prepare_decode"):
+            m.cache.prepare_decode(slots)
+        out.append(m.forward_decode(toks, at))
+    assert torch.equal(*out)
+
+
 @pytest.mark.parametrize("rows", [32, 64, 96, 128, 160])
 @pytest.mark.parametrize("m,n,k,sk", [
     (1, 256, 64, 1),           # a stage, of four or three that are loaded ahead
