@@ -144,6 +144,14 @@ class _DeviceIds:
         return torch.is_tensor(t) and t.is_cuda and t.dim() == 1 and \
             t.device == like.device and t.dtype in (torch.int64, torch.int32)
 
+    @classmethod
+    def of(cls, lists: Sequence[torch.Tensor]) -> list["_DeviceIds"]:
+        """Of a copy, never the caller's memory: a step's kernels read the ids behind
+        the call, when a caller on another stream may have changed or freed theirs, and
+        what they read has to be what was checked. (read waits for the copy.)"""
+        ids, ends = torch.cat(lists).long(), accumulate(len(t) for t in lists)
+        return [cls(ids, e - len(t), len(t)) for e, t in zip(ends, lists)]
+
     @staticmethod
     def read(parts: Sequence["_DeviceIds"]) -> tuple[torch.Tensor, np.ndarray]:
         """The parts one behind the other, on the device and on the host."""
@@ -1071,8 +1079,8 @@ class HybridModel:
         if start_pos != self.cache.lens[slot]:
             raise ValueError(f"slot {slot} holds {self.cache.lens[slot]} "
                              f"tokens, not {start_pos}")
-        ids = _DeviceIds(tokens.long().contiguous(), 0, len(tokens)) \
-            if _DeviceIds.can(tokens, self.embed) else _host_ids(tokens)
+        ids = _DeviceIds.of([tokens])[0] if _DeviceIds.can(tokens, self.embed) \
+            else _host_ids(tokens)
         out = self.forward_step([(slot, ids, [len(ids) - 1])], return_hidden)
         return (out[0][0], out[1][0]) if return_hidden else out[0]
 
@@ -1083,9 +1091,7 @@ class HybridModel:
         # prompts of 14 tokens, three layers of birepel:3b, 1257 -> 918 us)
         lists = list(token_lists)
         if lists and all(_DeviceIds.can(t, self.embed) for t in lists):
-            ids, ends = torch.cat(lists).long(), accumulate(len(t) for t in lists)
-            lists = [_DeviceIds(ids, e - len(t), len(t))
-                     for e, t in zip(ends, lists)]
+            lists = _DeviceIds.of(lists)
         else:
             lists = [_host_ids(t) for t in lists]
         return self.forward_step(

@@ -1186,6 +1186,26 @@ def test_prompt_attention_past_64_pages(start, ln, window):
     assert float((got.view_as(want).double() - want).abs().max()) < 0.02
 
 
+def test_prompts_on_the_device_are_copies(monkeypatch):
+    """A step has its own copy of token ids on the device, of one prompt and of several:
+    the caller may change or free theirs on another stream as soon as the call is back."""
+    from gridllm_amd.models import hybrid
+    m = build(FULL, ("cpu", "fp32"))
+    seen = []
+    monkeypatch.setattr(hybrid._DeviceIds, "can", staticmethod(
+        lambda t, like: torch.is_tensor(t)))
+    run = m._run
+    monkeypatch.setattr(m, "_run", lambda t, *a: seen.append(t) or run(t, *a))
+    a, b = (torch.tensor(tokens(n, seed=n)) for n in (6, 9))
+    want = m.forward_prefill(np.array(a), m.cache.alloc(0))
+    assert torch.equal(m.forward_prefill(a, m.cache.alloc(0)), want)
+    m.forward_prefill_batch([b], [m.cache.alloc(0)])
+    m.forward_prefill_batch([a, b], [m.cache.alloc(0) for _ in "ab"])
+    theirs = {t.untyped_storage().data_ptr() for t in (a, b)}
+    assert len(seen) == 4 and not any(
+        t.untyped_storage().data_ptr() in theirs for t in seen)
+
+
 @pytest.mark.gpu
 def test_prompts_on_the_device():
     """Token ids that a step reads from the device behind its preparation give what
