@@ -12,8 +12,9 @@
 //   splitk > 1: f32 partials [splitk][M][N] in ws. out == null otherwise: the
 //   result, rounded to bf16, as f32 in ws (a vocabulary's scores: 256 rows of
 //   128256 took 30 us to be widened behind it).
-// Constraints: N % (16 CT) == 0 (128 for EPI 1), K % 64 == 0, K <= BATCH_K (a tile's
-// offsets fit into 32 bits), kslice % 64 == 0.
+// Constraints: N % (16 CT) == 0 (128 for EPI 1), K % 64 == 0, kslice % 64 == 0; for
+// k_gemm_tile and k_gemm_cols K <= BATCH_K, by which a tile's offsets fit into 32 bits
+// (longer rows go to k_gemm_fed, whose loads have 64-bit addresses).
 //
 // Bound by a CU's loads: it has some 128 lines of 128 bytes on their way (counted:
 // TCP_TCC_READ_REQ_LATENCY over time, with rings of 2 stages as of 6), for 500 cycles

@@ -810,6 +810,9 @@ static int launch_gemm_tile(hipStream_t st, BatchArgs p) {
     constexpr bool both = RT <= 4;              // waves load and multiply
     typedef std::conditional_t<CT == 16, GemmCols<RT>, std::conditional_t<
         both, GemmTile<RT, CT>, GemmFed<RT, CT>>> Sh;
+    if constexpr (both || CT == 16)
+        if (p.K > BATCH_K)                      // (see there)
+            return launch_gemm_tile<RT < 6 ? 6 : RT, CT == 16 ? 8 : CT, EPI>(st, p);
     p.rblocks = (p.M + Sh::R - 1) / Sh::R;
     if constexpr (!ONCE)
         if (tile_once(p.M, p.N, p.K, Sh::R, p.kslice))
@@ -1644,7 +1647,7 @@ int gl_gemm_tile(void* stream, void* out, void* ws, const void* x,
                  int rows, int cols, int fuse_swiglu, float alpha,
                  float limit, float shift, float cubic) {
     const GluParams glu{alpha, limit, shift, cubic};
-    if (M < 1 || K < 1 || K % 64 || K > BATCH_K || kslice < 64 || kslice % 64 || N < 1 ||
+    if (M < 1 || K < 1 || K % 64 || kslice < 64 || kslice % 64 || N < 1 ||
         cols < 1 || N % cols || (fuse_swiglu && N % 128) || splitk < 1 ||
         (long)(splitk - 1) * kslice >= K || (long)splitk * kslice < K ||
         (splitk > 1 && !ws) || (!out && (!ws || fuse_swiglu))) return -100;
@@ -1756,7 +1759,6 @@ int gl_gemm_plan(int M, int N, int K, int epi, int whole, int* plan) {
     const int heights[] = {96, 128, 160, 192, 256};
     const int widths[] = {64, 96, 128};
     if (!whole && M > 0 && M <= 1200 && N > 0 && K > 0 && K % 64 == 0 &&
-        K <= BATCH_K &&
         !(fuse_glu && N % 128)) {
         for (int rows : heights) for (int cols : widths) {
             if (N % cols || (fuse_glu && cols == 96)) continue;

@@ -618,17 +618,12 @@ def _tile_grid(m: int, n: int, k: int, fuse_swiglu: bool,
     return out
 
 
-_TILE_K = 1 << 20              # the longest rows that gemm_tile takes
-
-
 def gemm_tilings(m: int, n: int, k: int,
                  fuse_swiglu: bool = False) -> list[tuple[int, int, int]]:
     """(rows, columns, K parts) worth trying for gemm_tile: K in as many parts,
     of 128 or more, as give each of the 256 CUs a block, or in half as many; and 256
     columns, if these are still more tiles than CUs."""
     out = set()
-    if k > _TILE_K:
-        return []
     rows = next((r for r in _TILE_ROWS if r >= m), 256)
     if 0 < m <= 160 and n % 256 == 0 and n > 65536 and k % 64 == 0 and \
             not fuse_swiglu:
@@ -657,7 +652,7 @@ def gemm_tiling(m: int, n: int, k: int,
     choice's time in the mean, 1.07 at most, .70 of the library's (246 sizes). More
     blocks than CUs are a library product's sizes (17920 x 1536, 256 rows: 22.9 us,
     22.2), but for the gated unit that it would need a second kernel for."""
-    if not 0 < m <= 256 or n < 1 or not 0 < k <= _TILE_K or k % 64 or (
+    if not 0 < m <= 256 or n < 1 or k < 1 or k % 64 or (
             fuse_swiglu and n % 128):
         return None
     if m <= 64:

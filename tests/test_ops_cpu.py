@@ -257,6 +257,19 @@ def test_rope_attn_decode_refuses():
                                            *tail) == -100
 
 
+def test_tilings_of_long_rows():
+    """Tilings are offered and picked for rows of any length, and the entry takes them
+    (as far as it can be asked on the host: a wrong tile is refused ahead of a launch)."""
+    from gridllm_amd.ops import hip_ops
+    for k in (1 << 20, (1 << 20) + 64, 1 << 24):
+        assert hip_ops.gemm_tilings(48, 1024, k) and hip_ops.gemm_tiling(48, 1024, k)
+        assert hip_ops.gemm_tiling(200, 1024, k, True)
+        if hip_ops.available():
+            call = hip_ops._load().gl_gemm_tile
+            tail = (32, 48, 0, 1.0, float("inf"), 0.0, 0.0)      # (no such tile)
+            assert call(None, 64, None, None, None, 8, 96, k, 1, k, *tail) == -103
+
+
 def test_decode_splits():
     """Odd numbers, which spread the first parts of all rows over the chip's
     engines; none of less than 128 keys; no more than the combining kernel has."""

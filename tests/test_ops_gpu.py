@@ -1427,6 +1427,34 @@ def test_gemm_in_256_columns(dev, rows, m, n, k, sk):
         assert bool(((parts.sum(0) - ref).abs() <= small).all())
 
 
+@pytest.mark.parametrize("k", [1 << 20, (1 << 20) + 64])
+def test_gemm_tile_of_long_rows(dev, k):
+    """The longest rows of 32-bit offsets, and longer ones, which other kernels take for
+    the same tilings. Products of -1, 0 and 1: sums of up to 2^24 are exact in any
+    order."""
+    from gridllm_amd.ops import hip_ops
+    g = torch.Generator(device=dev).manual_seed(k)
+    m, n = 70, 768
+    x, w = (torch.randint(-1, 2, (r, k), generator=g, device=dev,
+                          dtype=torch.int8).to(torch.bfloat16) for r in (m, n))
+    want = sum(x[:, a:a + 65536].float() @ w[:, a:a + 65536].float().t()
+               for a in range(0, k, 65536))
+    assert float(want.abs().max()) < 2 ** 24
+    for rows, cols, parts in ((32, 64, 1), (32, 96, 5), (64, 128, 3), (32, 256, 1),
+                              (96, 256, 2), (96, 64, 1)):
+        got = hip_ops.gemm_tile(x, w, rows, cols, parts)
+        assert torch.equal(got, want.to(torch.bfloat16)), (rows, cols, parts)
+        if parts > 1:
+            assert torch.equal(hip_ops.gemm_tile_parts(x, w, rows, cols, parts).sum(0),
+                               want)
+        else:
+            assert torch.equal(hip_ops.gemm_tile_f32(x, w, rows, cols), got.float())
+    got = hip_ops.gemm_tile(x, w, 64, 64, 2, fuse_swiglu=True).double()
+    gate, up = want.double().view(m, -1, 2, 64).unbind(2)
+    ref = (torch.nn.functional.silu(gate) * up).reshape(m, -1)
+    assert bool(((got - ref).abs() <= 2 ** -8 * ref.abs() + 1e-6).all())
+
+
 @pytest.mark.parametrize("glu", [
     (1.0, float("inf"), 0.0, 0.0), (1.702, float("inf"), 0.0, 0.0),
     (1.702, 7.0, 1.0, 0.0),        # each constant alone leaves the short form
