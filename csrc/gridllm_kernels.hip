@@ -1714,9 +1714,11 @@ int gl_gemm_wide(void* stream, void* out, const void* x, const void* w, int M,
 // What to run a product of more than 256 rows by: plan[0] 0 the library, 1
 // gl_gemm_tile by rows plan[1], columns plan[2], parts plan[3], 2 gl_gemm_wide by
 // shape plan[1] and full plan[2]. The times are those of wide_best and of _tile_us
-// in hip_ops.py, which holds up to 1200 rows too (over 130 sizes what is picked here
-// takes 1.017 of the best choice's time in the mean, 1.13 at most, and .88 of the
-// library's).
+// in hip_ops.py, which holds up to 1200 rows too. Over 2712 random sizes of the models
+// here, of 257 to 8192 rows and more than 21 us, what is picked takes .973 of the
+// library's time in the mean; what is run here, in the mean and at most: tiles .90 and
+// 1.24 of it, 256 x 256 .95, 1.12, 192 x 192 .93, 1.29, 256 x 192 .91, 1.05, 192 x 128
+// .97, 1.51.
 //   Gated units are always done here: the library's needs another pass (16384 x 3072,
 //   272 rows 48 -> 38 us by tiles; 2731 338 -> 220).
 //   K from 4096 on with up to 1200 rows: tiles with K in parts (300 x 2048 x 8192 34 ->
@@ -1724,17 +1726,14 @@ int gl_gemm_wide(void* stream, void* out, const void* x, const void* w, int M,
 //   where they are one round of CUs, three quarters of it or more (300 x 12288 x 3072
 //   43 -> 33, 800 x 3072 x 3072 30 -> 26, 1024 x 5120 x 3072 42 -> 40; two rounds, 640
 //   x 12288 x 3072, take 63 us, the library 54; 160 tiles, 1200 x 4096 x 3072, 45, 40).
-//   20 us and less: what a call to the library costs the host, and twice what one
+//   21 us and less: what a call to the library costs the host, and twice what one
 //   here does (four layers of 0.5b, 260 tokens, are bound by that).
-//   Longer ones go here where the tiles fill their last round of CUs as the library's
-// do not (its time over 610 random products of 257 to 8192 rows, N 2048 to 12288, K
-// 1024 to 8192, in the mean, and at most, and that of the others of the shape):
-//   256 x 256 whose last round is .6 full at most, so that its halves fill one: .95 of
-// it, 1.13 (1.06). With one round before and K above 4096 from a quarter on: 1.09
-// below. 256 x 192 from the third round on, that one .6 full at least: .91, 1.05 (1.05).
-// 192 x 192 in rounds nearly full, or more than one: .95, 1.08 (no others). 192 x 128
-// likewise: .97, 1.12 (1.26). Some sizes the library takes 1.3 to 1.8 times as long for
-// (8000 x 5120 x 3072, 2800 x 8192 x 4096).
+//   Longer ones go here where a shape's tiles fill their last round of CUs as the
+// library's do not: 256 x 256 one that is .6 full at most, as its halves fill one (rows
+// of more than 4096 with one or two rounds before, and that one .37 to .5 full: outside
+// of that 1.0 to 1.1 of the library's time in the mean); 192 x 192 none or .8 of one
+// behind full rounds, .85 alone; 256 x 192 .6 behind two or more; 192 x 128 .85 alone,
+// .75 behind two, none behind one or three (.75 and more behind one or three: 1.07 to 1.28).
 //   whole: not in parts of K, and gated units by k_gemm_wide, whose sums and roundings
 // are the library's but where that cuts K itself (more than 99.9 % of results are the
 // same to the bit). Where a model makes much of a rounding (a sequence's first token
@@ -1784,19 +1783,23 @@ int gl_gemm_plan(int M, int N, int K, int epi, int whole, int* plan) {
             }
         }
     }
-    bool here = fuse_glu || best <= 20.f || (way == 1 && (K >= 4096 || fills));
+    bool here = fuse_glu || best <= 21.f || (way == 1 && (K >= 4096 || fills));
     if (way == 2) {
         const WideTimes& t = kWide[plan[1]];
         const long tiles = (long)((M + t.rows - 1) / t.rows) *
                            ((N + t.cols - 1) / t.cols);
-        const long some = tiles % 256;
+        const long some = tiles % 256, rounds = tiles / 256;   // full ones
         if (plan[1] == 0)
-            here |= some > 0 && some <= 160 &&
-                    (tiles > 512 || (tiles > 256 && (K <= 4096 || some >= 64)));
+            here |= rounds > 0 && some > 0 &&
+                    (K <= 4096 ? some <= 154
+                               : rounds < 3 && some >= 96 && some <= 128);
+        else if (plan[1] == 1)
+            here |= rounds > 0 ? some == 0 || some >= 204 : some >= 218;
         else if (plan[1] == 2)
-            here |= tiles > 512 && some >= 160;
+            here |= rounds > 1 && some >= 160;
         else
-            here |= tiles >= 256 || some >= (plan[1] == 1 ? 218 : 208);
+            here |= rounds % 2 ? rounds < 4 && some == 0
+                    : rounds == 0 ? some >= 218 : rounds == 2 && some >= 192;
         if (epi == 2 && plan[1] != 0) here = false;
     }
     plan[0] = here ? way : 0;

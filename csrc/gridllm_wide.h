@@ -358,19 +358,22 @@ k_gemm_wide(const WideArgs p, int full) {
 // Shapes by number, their sizes, and what they take, in us: a stage (`idle` of it
 // with one tile on the chip, as a whole round takes), a tile beside it (`glu` more
 // for the unit), a launch. Fitted to 330 to 1550 timings each over the products of
-// the models here and 257 to 8192 rows, 3 to 4 % off in the mean.
+// the models here and 257 to 8192 rows; later ones, of more products, are 3 to 4 %
+// longer, with a standard deviation of 4 to 6 %. Gated units, both shapes, to 435 of
+// these others: the faster shape in all but 1.7 % of sizes, where the other one is 2 to 4 %
+// faster (before, in 6.1 %, and up to 17).
 struct WideTimes {
     int rows, cols;
     float stage, idle, tile, glu, launch;
 };
 static constexpr WideTimes kWide[] = {
-    {256, 256, 1.350f, .660f, 3.82f, .15f, 4.7f},       // rest in halves
+    {256, 256, 1.350f, .660f, 3.82f, 1.49f, 4.7f},      // rest in halves
     {192, 192, .885f, .720f, 2.23f, 0.f, 5.4f},
     {256, 192, 1.090f, .716f, 2.91f, 0.f, 5.2f},
     {192, 128, .648f, .713f, .77f, 0.f, 5.0f},
-    {192, 256, 1.117f, .697f, .05f, 2.24f, 4.2f},       // gated units, f32
+    {192, 256, 1.190f, .755f, 0.f, 1.33f, 5.5f},        // gated units, f32
 };
-static constexpr WideTimes kWideHalf = {128, 256, .801f, .712f, 1.67f, .34f,
+static constexpr WideTimes kWideHalf = {128, 256, .801f, .712f, 1.67f, 1.75f,
                                         0.f};
 static constexpr int kWideShapes = 5;
 typedef WideShape<8, 4, 2> Wide256;

@@ -434,6 +434,28 @@ def test_plans_of_many_rows():
         assert hip_ops.gemm_plan(*bad) is None
 
 
+@pytest.mark.parametrize("m,n,k,fuse,whole,plan", [
+    # gated units of 256 x 256 with halves, 112 us, by 192 x 256 122; 125, 144
+    (1053, 16384, 3072, True, False, ("wide", 0, 256)),
+    (346, 37888, 3584, True, True, ("wide", 0, 256)),
+    # 20.7 us, by the library 23.2
+    (2159, 2048, 1536, False, False, ("wide", 3, 192)),
+    # by the library 61 us, 192 x 128 73; 123, 142; 256 x 256 920, 1034; 414, 424
+    # and of 192 x 192 whose last round is three quarters full 99, 91
+    (2640, 6144, 3072, False, True, None),
+    (1306, 8192, 3072, False, True, None), (2613, 9216, 3072, False, False, None),
+    (2405, 8192, 28672, False, False, None), (7440, 12288, 3072, False, True, None),
+    # by the library 491 us, 287; 212, 183; 78, by 192 x 128 94
+    (2768, 8192, 8192, False, True, ("wide", 0, 256)),
+    (4276, 8192, 3072, False, True, ("wide", 2, 731)),
+    (2944, 4096, 4096, False, True, None)])
+def test_plans_that_were_measured(m, n, k, fuse, whole, plan):
+    """One of each kind of size on which the kernels here and the library are on
+    different sides."""
+    from gridllm_amd.ops import hip_ops
+    assert hip_ops.gemm_plan(m, n, k, fuse, whole) == plan
+
+
 def test_rmsnorm_of_a_residual_needs_a_place_for_the_sum():
     """(refused on the host: the kernel would store to address 0)"""
     from gridllm_amd.ops import hip_ops
