@@ -868,12 +868,18 @@ DEV_INLINE int4 segment(const int4* seg, const int* pos, const int* slot,
 // being the logarithm of the decay, f32 [n][H*DK] (gated linear attention), or
 // by a constant per head, gr f32 [H] (lightning attention).
 // Bound by reading and writing the states: past the caches both ways, and ahead of the
-// gates, queries and keys (ONCE), where a call has 90 MB of them or more, so that two
-// layers' with what lies between are more than the Infinity Cache holds. 64 sequences, 12
-// heads of 128 x 257, 101 MB each way: 48.9 -> 47.0 us (4.3 TB/s), and a step of 3 layers,
-// two of them such, finds more of its other data there, 548 -> 529 (without the loads
-// ahead 533). With 48 sequences, 75 MB, it would go from 474 to 490, with 24 from 403 to
-// 406; loads ahead of the rest through the caches: 474 to 483. 32 rows a block; 64: 49.9.
+// gates, queries and keys (ONCE), where all of a step's recurrent layers have REC_ONCE of
+// them or more (the Infinity Cache is 256 MB): a layer then finds nothing of what it wrote
+// a step before, and the step's other data stays. Below, with one sequence's states from
+// step to step, it does. A step with and without ONCE, us, by MB of states:
+//   two layers of 12 x 128 x 257 (101 MB a call at 64 rows) 152 482, 463, 202 526, 504,
+//   227 524, 522, 253 547, 550, 303 605, 617, 404 653, 669, 808 932, 963
+//   birepel:3b, five such layers  126 1480, 1492, 189 1538, 1527, 253 1577, 1612, 505 1772, 1801
+//   maferax:5b, six of 12 x 128 x 256  151 1936, 1945, 226 2064, 2090, 302 2144, 2211
+//   zinavik:4b, eight  151 2114, 2126, 201 2370, 2395, 302 2484, 2530, 805 2975, 3026
+// (Steps of several models in turn, whose states push each other out, gain from less on.)
+// 32 rows a block; 64: 49.9 us a call of 64 sequences, not 47.0.
+#define REC_ONCE 225000000l
 enum Rec { MLSTM = 0, CHANNELS = 1, CONSTANT = 2 };
 
 template <class T, int LPR, int NJ, int KIND, bool ONCE>
@@ -3086,18 +3092,18 @@ int gh_attn_rows_f32(void* stream, void* out, const void* q, const void* kc,
     return 0;
 }
 
-// kind: Rec
+// kind: Rec. step: bytes of states of all the step's recurrent layers (see k_rec_step)
 int gh_rec_step(void* stream, int f32, int kind, void* o, void* S, const void* mst,
                 const void* qkv, const void* gr, const void* segs,
                 const void* pos, const void* slot, int nseg, int H, int DK,
-                int DV, int ld_, float qscale, float cap, int rpb) {
+                int DV, int ld_, float qscale, float cap, int rpb, long step) {
     if (nseg < 1 || DK % 64 || DV % 64 || DK > 1024 || rpb < 1 || kind < 0 ||
         kind > CONSTANT || (kind == MLSTM && !mst))
         return -100;
     hipStream_t st_ = (hipStream_t)stream;
     const dim3 grid((unsigned)nseg, (unsigned)H,
                     (unsigned)((DV + (kind == MLSTM) + rpb - 1) / rpb));
-    const bool once = !f32 && (long)nseg * H * DV * DK * 4 >= 90000000;
+    const bool once = !f32 && step >= REC_ONCE;
 #define GO1(T, L, J, C, O) k_rec_step<T, L, J, C, O><<<grid, 256, 0, st_>>>( \
         (float*)o, (float*)S, (const float*)mst, (const T*)qkv, \
         (const float*)gr, (const int4*)segs, (const int*)pos, \

@@ -995,7 +995,8 @@ class HybridModel:
                       absorbed=absorbed, lat_rows=lrows,
                       lat_items=dev[7].view(-1, 4) if litems else None,
                       lat_tiles=dev[8].view(-1, 8) if ltiles else None,
-                      whole=mixed or 0 in starts)
+                      whole=mixed or 0 in starts,
+                      state_bytes=self.cache.state_bytes)
         for k, (c, t) in enumerate(zip(self.chunks, talks)):
             if t[0]:
                 items, t16, t128 = dev[9 + 3 * k:12 + 3 * k]
@@ -1112,7 +1113,8 @@ class HybridModel:
             rows = None                            # (more slots than tokens)
         st = StepMeta(nd=tokens.shape[0], pos=pos, slot=slot_map,
                       table=self.cache.table, max_len=self.max_seq,
-                      absorbed=tokens.shape[0], rows=rows)
+                      absorbed=tokens.shape[0], rows=rows,
+                      state_bytes=self.cache.state_bytes)
         x = self._run(tokens, st)
         ops.advance_lengths(self.cache.seq_lens, slot_map)
         return self._head(x, None)

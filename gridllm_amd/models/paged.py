@@ -117,6 +117,8 @@ class PagedCache:
             self.inv.append(inv)
             self.S.append(s)
             self.m.append(m)
+        # of a sequence, in all layers
+        self.state_bytes = sum(4 * s[0].numel() for s in self.S if s is not None)
         self.table = torch.zeros(slots, self.per_slot, dtype=torch.int32,
                                  device=device)
         self.seq_lens = torch.zeros(slots, dtype=torch.int32, device=device)

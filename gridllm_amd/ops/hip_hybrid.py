@@ -51,7 +51,7 @@ _SIGS = {
     "gh_paged_decode": "pppppippppiiiiifiippiifi",
     "gh_paged_prefill": "pppppipiiiifiippiifi",
     "gh_attn_rows_f32": "pppppippiiiifiippiifi",
-    "gh_rec_step": "iippppppppiiiiiffi",
+    "gh_rec_step": "iippppppppiiiiiffil",
     "gh_rec_row_out": "ippppiiiiiif",
     "gh_rec_out": "iipppppppppiiiiiiiiff",
     "gh_mlstm_chunks": "ipppppppppppiiiiiiffif",
@@ -438,7 +438,8 @@ def mlstm(qkv: torch.Tensor, gates: torch.Tensor, S: torch.Tensor,
         # is full anyway and a block amortises its loads of q and k
         rpb = 128 if nseg * h * (dv + 1) >= 128 * 2048 else 32
         _call("gh_rec_step", f, _MLSTM, o, S, m, qkv, gates, segs, st.pos,
-              st.slot, nseg, h, dk, dv, ld, qscale, cap, rpb)
+              st.slot, nseg, h, dk, dv, ld, qscale, cap, rpb,
+              _state_bytes(st, S, nseg))
     out = torch.empty(n, h * dv, dtype=qkv.dtype, device=qkv.device)
     nplain = 0
     if not f and st.chunks is not None:
@@ -455,6 +456,12 @@ def mlstm(qkv: torch.Tensor, gates: torch.Tensor, S: torch.Tensor,
         _call("gh_rec_out", f, 0, out, o, m, qkv, gates, segs, st.pos, st.slot,
               norm, nseg, st.nd, nplain, h, dk, dv, ld, vdim, cap, eps)
     return out
+
+
+def _state_bytes(st: StepMeta, S: torch.Tensor, rows: int) -> int:
+    """What a step's recurrent layers hold for its rows, this one alone if the step does
+    not say."""
+    return rows * (st.state_bytes or 4 * S[0].numel())
 
 
 def lightning(rows: torch.Tensor, S: torch.Tensor, decay: torch.Tensor,
@@ -480,7 +487,8 @@ def lightning(rows: torch.Tensor, S: torch.Tensor, decay: torch.Tensor,
     if nseg:
         rpb = 128 if nseg * h * dv >= 128 * 2048 else 32
         _call("gh_rec_step", f, _CONSTANT, o, S, None, rows, decay[0], segs,
-              st.pos, st.slot, nseg, h, dk, dv, ld, 1.0, 0.0, rpb)
+              st.pos, st.slot, nseg, h, dk, dv, ld, 1.0, 0.0, rpb,
+              _state_bytes(st, S, nseg))
     if not f and st.chunks is not None:
         nch = st.chunks.shape[0]
         ds = torch.empty(nch, h, dv, dk, dtype=torch.float32, device=dev)
@@ -694,7 +702,8 @@ def gla(rows: torch.Tensor, u: torch.Tensor, wa2: torch.Tensor,
     if nseg:
         rpb = 128 if nseg * h * dv >= 128 * 2048 else 32
         _call("gh_rec_step", f, _CHANNELS, o, S, None, rows, b, segs, st.pos,
-              st.slot, nseg, h, dk, dv, ld, qscale, 0.0, rpb)
+              st.slot, nseg, h, dk, dv, ld, qscale, 0.0, rpb,
+              _state_bytes(st, S, nseg))
     whole = nch and dv <= 256          # chunks' blocks have all of a head
     if nch:
         ds = torch.empty(nch, h, dv, dk, dtype=torch.float32, device=dev)

@@ -58,6 +58,8 @@ class StepMeta:
     rows       [n, 4] {row, keys, slot, ..} of a step of decode rows alone, the
                longest first: the order in which attention takes them. None:
                that of the step
+    state_bytes  what all of the model's recurrent layers hold for a sequence, 0
+               if that is not known
     """
     nd: int
     pos: torch.Tensor            # [n] int32
@@ -76,6 +78,7 @@ class StepMeta:
     talk: dict[int, ChunkPortions] = field(default_factory=dict)
     whole: bool = False
     rows: Optional[torch.Tensor] = None
+    state_bytes: int = 0
 
     def entries(self) -> list:
         """(first token, length, slot, start) of every entry, on the host."""

@@ -837,11 +837,36 @@ def test_mlstm_chunk_sizes(dk, dv, entering):
     assert float((m1.cpu()[used] - m0[used]).abs().max()) < 1e-4
 
 
+def test_a_step_says_what_its_states_take(monkeypatch):
+    """Whether states go past the caches is decided by all recurrent layers' of a step,
+    decoded or mixed, and by a call's own where there is no step."""
+    from gridllm_amd.models import hybrid
+    from gridllm_amd.ops import hip_hybrid
+    m = build(FULL, ("cpu", "fp32"))
+    states = [t for t in m.cache.S if t is not None]
+    each = sum(t[0].numel() * t.element_size() for t in states)
+    assert len(states) > 1 and m.cache.state_bytes == each
+    seen = []
+    real = hybrid.hops.mlstm
+
+    def spy(rows, gates, S, mm, norm, st, *rest):
+        seen.append(hip_hybrid._state_bytes(st, S, 3))
+        return real(rows, gates, S, mm, norm, st, *rest)
+    monkeypatch.setattr(hybrid.hops, "mlstm", spy)
+    slot = m.cache.alloc(0)
+    m.forward_prefill(np.array(tokens(5)), slot)
+    m.cache.prepare_decode([slot])
+    m.forward_decode(torch.tensor([3]), torch.tensor([slot], dtype=torch.int32))
+    assert seen == [3 * each] * (2 * len(states))
+    st = hops.StepMeta(nd=1, pos=None, slot=None, table=None, max_len=4)
+    assert hip_hybrid._state_bytes(st, states[0], 3) == 12 * states[0][0].numel()
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,h", [(57, 12), (58, 12), (90, 16)])
-def test_states_past_the_caches(n, h):
-    """Decode rows whose states are just less than 90 MB, just more, and of several
-    rounds of a block: the same as the rows one by one."""
+@pytest.mark.parametrize("n,h,more", [(57, 12, -1), (57, 12, 1), (90, 16, 1)])
+def test_states_past_the_caches(n, h, more):
+    """Decode rows of a step whose states are just less than what goes past the caches,
+    or just more, and of several rounds of a block: the same as the rows one by one."""
     dk, dv = 128, 256
     g = torch.Generator(device="cuda").manual_seed(n)
 
@@ -856,7 +881,8 @@ def test_states_past_the_caches(n, h):
     def step(at, S, m):
         st = hops.StepMeta(nd=at.stop - at.start, pos=pos[at], slot=slot[at],
                            table=torch.zeros(n, 1, dtype=torch.int32,
-                                             device="cuda"), max_len=4)
+                                             device="cuda"), max_len=4,
+                           state_bytes=225_000_000 // n + more)
         return hops.mlstm(rows[at].contiguous(), gates[at].contiguous(), S, m,
                           norm, st, dk, dv, 15.0, 1e-5)
     S1, m1 = S.clone(), m.clone()
@@ -864,6 +890,42 @@ def test_states_past_the_caches(n, h):
     want = torch.cat([step(slice(i, i + 1), S, m) for i in range(n)])
     assert torch.equal(got, want)
     assert torch.equal(S1, S) and torch.equal(m1, m)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dk", [64, 128, 192, 512, 576])
+@pytest.mark.parametrize("kind", [0, 1, 2])     # mLSTM, decays by channel, by head
+def test_states_past_the_caches_of_all_kinds(kind, dk):
+    """To the bit what goes through them: each width of a row's lanes, one round of a
+    block and several, rows alone and segments of several tokens, whose states are read
+    behind the stores of the token before."""
+    from gridllm_amd.ops import hip_hybrid
+    g = torch.Generator(device="cuda").manual_seed(dk)
+    h, dv, lens = 2, 192, (1, 5, 2, 7)
+    n, r = sum(lens), 192 + (kind == 0)
+
+    def rand(*s):
+        return torch.randn(*s, generator=g, device="cuda")
+
+    def ints(rows):
+        return torch.tensor(rows, dtype=torch.int32, device="cuda")
+    rows, m = rand(n, h * 2 * (dk + dv)).to(torch.bfloat16), rand(n, h).abs()
+    gates = (rand(n, 2 * h), -rand(n, h * dk).abs(), rand(h).abs() / 4)[kind]
+    S, slot = rand(n, h, r, dk), torch.randperm(n, generator=g, device="cuda").int()
+    segs = ints([(sum(lens[:i]), ln, i, 3 * (i % 2)) for i, ln in enumerate(lens)])
+    pos = ints([i % 3 for i in range(n)])
+    for of, count in ((segs, len(lens)), (None, n)):
+        for rpb in (32, 128):
+            out = []
+            for step in (0, 1 << 40):
+                o, s = torch.zeros(n, h, dv + 4, device="cuda"), S.clone()
+                hip_hybrid._call("gh_rec_step", 0, kind, o, s, m, rows, gates, of, pos,
+                                 slot, count, h, dk, dv, rows.shape[1], dk ** -0.5,
+                                 15.0, rpb, step)
+                out.append((o, s))
+            assert not torch.equal(out[0][1], S)
+            for a, w in zip(*out):
+                assert a.isfinite().all() and torch.equal(a, w)
 
 
 @pytest.mark.gpu
