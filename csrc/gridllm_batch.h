@@ -342,11 +342,18 @@ k_gemm_tile(const BatchArgs p) {
 // before is free. What is left to gain was in the stores: 160 rows without them 129 us,
 // with stores of half lines 166, of whole ones (turn_tiles) 164, of these past the
 // caches, as W goes, 152 (half ones past them 160). W's way from memory bounds it; the
-// products take 105 us alone. 128256 columns, us, k_gemm_tile in 256 columns and this:
+// products take 105 us alone. The token pick behind it then reads from memory: from
+// COLS_PAST bytes of scores on a step and its pick are faster so by 1 to 2 % where tokens
+// are drawn, and where the highest are taken at most 2 % slower (128256 x 3072, a step of
+// 4 layers with the pick, us, through the caches and past them, drawn; highest: 16 rows
+// 410, 407; 439, 447, 24 488, 485; 516, 523, 48 509, 499; 531, 533, 128 673, 659; 689,
+// 686), with fewer rows by less, and slower by more. Parts of K are read next. 128256 columns, us, k_gemm_tile in 256 columns and this:
 //   rows   24           64           96           128          160
 //   K 3072 130 -> 122   143 -> 129   158 -> 135   173 -> 142   184 -> 152
 //   K 2048                           106 -> 96                 129 -> 104
 // ===========================================================================
+#define COLS_PAST 20000000l
+
 template <int RT>
 struct GemmCols {
     static constexpr int R = RT * 16, C = 256, THREADS = 768;
@@ -354,7 +361,9 @@ struct GemmCols {
     static constexpr int NB = 160 * 1024 / STAGE, BYTES = NB * STAGE;
 };
 
-template <int RT, bool ONCE>
+// PAST: scores past the caches. (Not by a branch: the compiler makes one store of two
+// that differ in that alone.)
+template <int RT, bool ONCE, bool PAST>
 __global__ void __launch_bounds__(768, 3)
 k_gemm_cols(const BatchArgs p) {
     typedef GemmCols<RT> Sh;
@@ -473,9 +482,11 @@ k_gemm_cols(const BatchArgs p) {
                 if (p.splitk == 1 && p.out)
                     *(u32x2*)(p.out + (long)m * p.N + n) =
                         (u32x2){pack2(v[0], v[1]), pack2(v[2], v[3])};
-                else
-                    __builtin_nontemporal_store(
-                        v, (f32x4*)(p.ws + ((long)t.ks * p.M + m) * p.N + n));
+                else {
+                    f32x4* to = (f32x4*)(p.ws + ((long)t.ks * p.M + m) * p.N + n);
+                    if constexpr (PAST) __builtin_nontemporal_store(v, to);
+                    else *to = v;
+                }
             }
         }
     }

@@ -805,7 +805,7 @@ static bool tile_once(int M, int N, int K, int rows, int kslice) {
            (blocks < 4 && (long)N * K <= 8000000 && kslice < 1536);
 }
 
-template <int RT, int CT, int EPI, bool ONCE = false>
+template <int RT, int CT, int EPI, bool ONCE = false, bool PAST = false>
 static int launch_gemm_tile(hipStream_t st, BatchArgs p) {
     constexpr bool both = RT <= 4;              // waves load and multiply
     typedef std::conditional_t<CT == 16, GemmCols<RT>, std::conditional_t<
@@ -817,8 +817,11 @@ static int launch_gemm_tile(hipStream_t st, BatchArgs p) {
     if constexpr (!ONCE)
         if (tile_once(p.M, p.N, p.K, Sh::R, p.kslice))
             return launch_gemm_tile<RT, CT, EPI, true>(st, p);
+    if constexpr (CT == 16 && ONCE && !PAST)
+        if (p.splitk == 1 && (long)p.M * p.N * 4 >= COLS_PAST)
+            return launch_gemm_tile<RT, CT, EPI, ONCE, true>(st, p);
     constexpr auto kernel = [] {
-        if constexpr (CT == 16) return k_gemm_cols<RT, ONCE>;
+        if constexpr (CT == 16) return k_gemm_cols<RT, ONCE, PAST>;
         else if constexpr (both) return k_gemm_tile<RT, CT, EPI, ONCE>;
         else return k_gemm_fed<RT, CT, EPI, ONCE>;
     }();

@@ -1406,6 +1406,7 @@ def test_decode_of_fewer_tokens_than_slots_gpu(dev, name):
     (161, 2304, 4096, 1),      # several blocks of rows, blocks that start further on
     (31, 69888, 128, 1),       # two tiles a block for some, one for others
     (200, 66048, 192, 2),      # up to eight, of unlike parts
+    (75, 66048, 64, 1), (76, 66048, 64, 1),    # scores through the caches, and past them
 ])
 def test_gemm_in_256_columns(dev, rows, m, n, k, sk):
     """Results as bf16, as f32 and in parts, at edges of rows, of K's parts and of the
