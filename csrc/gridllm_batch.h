@@ -344,10 +344,11 @@ k_gemm_tile(const BatchArgs p) {
 // caches, as W goes, 152 (half ones past them 160). W's way from memory bounds it; the
 // products take 105 us alone. The token pick behind it then reads from memory: from
 // COLS_PAST bytes of scores on a step and its pick are faster so by 1 to 2 % where tokens
-// are drawn, and where the highest are taken at most 2 % slower (128256 x 3072, a step of
-// 4 layers with the pick, us, through the caches and past them, drawn; highest: 16 rows
-// 410, 407; 439, 447, 24 488, 485; 516, 523, 48 509, 499; 531, 533, 128 673, 659; 689,
-// 686), with fewer rows by less, and slower by more. Parts of K are read next. 128256 columns, us, k_gemm_tile in 256 columns and this:
+// are drawn, and where the highest are taken at most 2 % slower; with fewer rows by
+// less, and slower by more (128256 x 3072, a step of 4 layers with the pick, us, through
+// the caches and past them, drawn; highest: 16 rows 410, 407; 439, 447, 24 488, 485; 516,
+// 523, 48 509, 499; 531, 533, 128 673, 659; 689, 686). Parts of K are read next. 128256
+// columns, us, k_gemm_tile in 256 columns and this:
 //   rows   24           64           96           128          160
 //   K 3072 130 -> 122   143 -> 129   158 -> 135   173 -> 142   184 -> 152
 //   K 2048                           106 -> 96                 129 -> 104

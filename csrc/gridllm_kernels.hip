@@ -178,15 +178,15 @@ k_rmsnorm_parts(bf16_t* __restrict__ y, const float* __restrict__ ws, int parts,
 }
 
 // ===========================================================================
-// Start and end of a decode step: see gl_decode_positions and
+// Start and end of a decode step: see gl_decode_start and
 // gl_advance_lengths, which stand for the dozen index kernels of 4 us each that
 // a step had. A slot that there is not ends the program, as an index does that
 // torch finds out of bounds, before anything is read or counted by it.
 // ===========================================================================
-// rows (B <= ROWS_ORDERED): {row, keys, slot, rotary position}, the longest first and equal ones in
-// the batch's order, as attention's blocks start. Four lanes count the rows that are
-// ahead of one, by LDS: in the launch that there is anyway, 5.8 us for 256 rows (4.7
-// without; 12.7 by a lane a row).
+// rows (B <= ROWS_ORDERED): {row, keys, slot, rotary position}, the longest first and
+// equal ones in the batch's order, as attention's blocks start. Four lanes count the
+// rows that are ahead of one, by LDS: in the launch that there is anyway, 5.8 us for 256
+// rows (4.7 without; 12.7 by a lane a row).
 #define ROWS_ORDERED 1024
 __global__ void __launch_bounds__(256)
 k_decode_positions(int* __restrict__ pos, int* __restrict__ slot_t,
@@ -1410,14 +1410,6 @@ int gl_decode_start(void* stream, void* pos, void* slot_t, void* pos_rope,
     return 0;
 }
 
-int gl_decode_positions(void* stream, void* pos, void* slot_t, void* pos_rope,
-                        void* attn_seq, const void* seq_lens,
-                        const void* rope_off, const void* slot_map, int B,
-                        int slots, int Smax) {
-    return gl_decode_start(stream, pos, slot_t, pos_rope, attn_seq, nullptr, seq_lens,
-                           rope_off, slot_map, B, slots, Smax);
-}
-
 // What it ends with: the rows' slots are one longer (rows may share a slot).
 int gl_advance_lengths(void* stream, void* seq_lens, const void* slot_map,
                        int B, int slots) {
@@ -1736,7 +1728,8 @@ int gl_gemm_wide(void* stream, void* out, const void* x, const void* w, int M,
 // of more than 4096 with one or two rounds before, and that one .37 to .5 full: outside
 // of that 1.0 to 1.1 of the library's time in the mean); 192 x 192 none or .8 of one
 // behind full rounds, .85 alone; 256 x 192 .6 behind two or more; 192 x 128 .85 alone,
-// .75 behind two, none behind one or three (.75 and more behind one or three: 1.07 to 1.28).
+// .75 behind two, none behind one or three (.75 and more behind one or three: 1.07 to
+// 1.28).
 //   whole: not in parts of K, and gated units by k_gemm_wide, whose sums and roundings
 // are the library's but where that cuts K itself (more than 99.9 % of results are the
 // same to the bit). Where a model makes much of a rounding (a sequence's first token

@@ -527,7 +527,7 @@ k_latent_prefill(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
     auto issue = [&](int k0, bf16_t* to) {
         const long row = key_off + k0;
         const bf16_t* er = e + (row * H + h) * 2 * P;
-            part(lds_source(er, 31 * e_row + P * 2), e_row, P, to);
+        part(lds_source(er, 31 * e_row + P * 2), e_row, P, to);
         part(lds_source(lat + row * lat_ld + lat_ld - R, 31 * lat_row + R * 2),
              lat_row, R, to + 32 * P);
         part(lds_source(er + P, 31 * e_row + P * 2), e_row, P, to + 32 * KD);
@@ -694,7 +694,8 @@ int gn_latent_decode(void* stream, void* out, const void* ql, const void* q,
                      void* ws, const void* cos_, const void* sin_, int nrot,
                      int N, int H, int P, int KR, int R, int nsplit,
                      float scale) {
-    if (N < 1 || H < 1 || (unsigned long)rows % 16 || nsplit < 1 || nsplit > 64 || !sizes_ok(KR, R))
+    if (N < 1 || H < 1 || (unsigned long)rows % 16 || nsplit < 1 || nsplit > 64 ||
+        !sizes_ok(KR, R))
         return -100;
     hipStream_t st_ = (hipStream_t)stream;
     const Rotation rot{(const float*)cos_, (const float*)sin_, R / 2, nrot};

@@ -41,9 +41,10 @@
 // 128256 x 3072 in a step 207 -> 201 us, and the step's other kernels find theirs
 // there: 4 layers 880 -> 861), and stores go past the caches, too, in whole lines (256
 // rows 200 -> 194, 192 198 -> 181; a step of 256 rows with the token pick behind it, which
-// then reads them from memory: drawn tokens 852 -> 840, the highest 860 -> 858). More tiles of rows read W again, and would wait for memory
-// where the Infinity Cache has it (us, through it and past it, 128256 x 3072: 257 rows 300,
-// 361, 512 444, 481, 1024 886, 936; 300 of 151936 x 896 131, 155).
+// then reads them from memory: drawn tokens 852 -> 840, the highest 860 -> 858). More
+// tiles of rows read W again, and would wait for memory where the Infinity Cache has it
+// (us, through it and past it, 128256 x 3072: 257 rows 300, 361, 512 444, 481, 1024 886,
+// 936; 300 of 151936 x 896 131, 155).
 // EPI 3: squared ReLU. EPI 4: W rows in turns of 16 gate | 16 up, [M, N / 2].
 // Rows past M and N are read as zeros by the buffer descriptors' bounds, and so are
 // the stages past the last tile: a wave's offset is the end of the matrix at most,

@@ -43,8 +43,6 @@ def _load() -> ctypes.CDLL:
     lib.gl_rmsnorm_parts.argtypes = [c_vp] * 3 + [c_i] + [c_vp] * 3 + [
         c_i, c_i, c_f]
     lib.gl_rmsnorm_parts.restype = c_i
-    lib.gl_decode_positions.argtypes = [c_vp] * 8 + [c_i] * 3
-    lib.gl_decode_positions.restype = c_i
     lib.gl_decode_start.argtypes = [c_vp] * 9 + [c_i] * 3
     lib.gl_decode_start.restype = c_i
     lib.gl_advance_lengths.argtypes = [c_vp] * 3 + [c_i] * 2

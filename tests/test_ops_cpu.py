@@ -212,7 +212,8 @@ def test_embed_norm_refuses():
 
 def test_decode_positions_refuse():
     """Host tensors, other types and tables of other lengths are an error ahead of
-    the launch; so is a step over no slots."""
+    the launch; so is a step over no slots, rotary positions without their shifts, and
+    an order of more rows than are put in one or at an address that is no int4's."""
     from gridllm_amd.ops import hip_ops
     i32 = torch.zeros(4, dtype=torch.int32)
     with pytest.raises(ValueError):
@@ -224,8 +225,11 @@ def test_decode_positions_refuse():
         with pytest.raises(ValueError):
             hip_ops.decode_lengths(meta, bad)
     if hip_ops.available():
-        assert hip_ops._load().gl_decode_positions(
-            *(None,) * 8, 1, 0, 64) == -100
+        call, at = hip_ops._load().gl_decode_start, 1 << 20
+        assert call(*(None,) * 9, 1, 0, 64) == -100
+        assert call(None, at, at, at, at, None, at, None, at, 1, 4, 64) == -100
+        for rows, b in ((at, hip_ops._ROWS_ORDERED + 1), (at + 4, 8)):
+            assert call(None, at, None, None, None, rows, at, None, at, b, 4, 64) == -100
 
 
 def test_rope_attn_decode_refuses():
