@@ -127,17 +127,21 @@ def rope(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor,
     return reference.rope(q, k, cos, sin, pos)
 
 
+def _dense_bias(bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """As kernels read it; a view at any place or stride is copied."""
+    if bias is None or (bias.is_contiguous() and not bias.data_ptr() & 15):
+        return bias
+    return bias.clone(memory_format=torch.contiguous_format)
+
+
 def rope_kv(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
             cos: torch.Tensor, sin: torch.Tensor, pos: torch.Tensor,
             slot: torch.Tensor, hq: int, hk: int, d: int,
             bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     if _on_gpu(qkv):
         from gridllm_amd.ops import hip_ops
-        if bias is not None and (bias.data_ptr() & 15
-                                 or not bias.is_contiguous()):
-            bias = bias.clone(memory_format=torch.contiguous_format)
         return hip_ops.rope_kv(qkv, kcache, vcache, cos, sin, pos, slot,
-                               hq, hk, d, bias)
+                               hq, hk, d, _dense_bias(bias))
     return reference.rope_kv(qkv, kcache, vcache, cos, sin, pos, slot,
                              hq, hk, d, bias)
 
@@ -180,7 +184,7 @@ def rope_attn_decode(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tens
         from gridllm_amd.ops import hip_ops
         return hip_ops.rope_attn_decode(
             qkv, kcache, vcache, cos, sin, pos, slot, seqlen, hq, scale,
-            slot_map.int().contiguous(), bias, rows)
+            slot_map.int().contiguous(), _dense_bias(bias), rows)
     q = rope_kv(qkv, kcache, vcache, cos, sin, pos, slot, hq, kcache.shape[1],
                 kcache.shape[3], bias)
     return attn_decode(q, kcache, vcache, seqlen, scale, slot_map=slot_map)

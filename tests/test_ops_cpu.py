@@ -510,6 +510,24 @@ def test_rope_kv_takes_any_bias_of_its_size(monkeypatch):
     assert got[-1] is None
 
 
+def test_rope_attn_decode_takes_any_bias_of_its_size(monkeypatch):
+    """As rope_kv does, in whose place it stands in a decode step."""
+    from gridllm_amd import ops
+    from gridllm_amd.ops import hip_ops
+    bf16, got = torch.bfloat16, []
+    monkeypatch.setattr(ops, "_on_gpu", lambda t: True)
+    monkeypatch.setattr(hip_ops, "rope_attn_decode", lambda *a: got.append(a[-2]))
+    want, rows = torch.arange(64).to(bf16), torch.zeros(2, 64, dtype=bf16)
+    flat, wide = torch.zeros(65, dtype=bf16), torch.zeros(64, 2, dtype=bf16)
+    flat[1:], wide[:, 0] = want, want
+    slots = torch.zeros(2, dtype=torch.int32)
+    for bias in (want, flat[1:], wide[:, 0], None):
+        ops.rope_attn_decode(rows, *(None,) * 7, 2, 1.0, slots, bias)
+    assert got[0] is want and got.pop() is None
+    for b in got:
+        assert torch.equal(b, want) and b.is_contiguous() and b.data_ptr() % 16 == 0
+
+
 def test_plans_of_whole_products():
     """None is in parts of K, or by the kernel of which parts are."""
     from gridllm_amd.ops import hip_ops
