@@ -869,17 +869,18 @@ DEV_INLINE int4 segment(const int4* seg, const int* pos, const int* slot,
 // by a constant per head, gr f32 [H] (lightning attention).
 // Bound by reading and writing the states: past the caches both ways, and ahead of the
 // gates, queries and keys (ONCE), where all of a step's recurrent layers have REC_ONCE of
-// them or more (the Infinity Cache is 256 MB): a layer then finds nothing of what it wrote
-// a step before, and the step's other data stays. Below, with one sequence's states from
-// step to step, it does. A step with and without ONCE, us, by MB of states:
-//   two layers of 12 x 128 x 257 (101 MB a call at 64 rows) 152 482, 463, 202 526, 504,
-//   227 524, 522, 253 547, 550, 303 605, 617, 404 653, 669, 808 932, 963
-//   birepel:3b, five such layers  126 1480, 1492, 189 1538, 1527, 253 1577, 1612, 505 1772, 1801
-//   maferax:5b, six of 12 x 128 x 256  151 1936, 1945, 226 2064, 2090, 302 2144, 2211
+// them or more (the Infinity Cache is 256 MB): a layer then finds little of what it wrote
+// a step before, and the step's other data stays. Below, states stay from step to step.
+// The line is where whole models change sides; a step with and without ONCE, us, by MB:
+//   birepel:3b, five layers of 12 x 128 x 257  126 1480, 1492, 189 1538, 1527, 253 1577,
+//     1612, 505 1772, 1801
+//   maferax:5b, six of 12 x 128 x 256  151 1936, 1945, 189 2004, 1999, 226 2064, 2090,
+//     302 2144, 2211
 //   zinavik:4b, eight  151 2114, 2126, 201 2370, 2395, 302 2484, 2530, 805 2975, 3026
-// (Steps of several models in turn, whose states push each other out, gain from less on.)
+//   two of birepel's five, in three layers  152 482, 463, 202 526, 504, 227 524, 522, 253
+//     547, 550, 404 653, 669, 808 932, 963; 202 MB of several batches in turn 530, 548
 // 32 rows a block; 64: 49.9 us a call of 64 sequences, not 47.0.
-#define REC_ONCE 225000000l
+#define REC_ONCE 200000000l
 enum Rec { MLSTM = 0, CHANNELS = 1, CONSTANT = 2 };
 
 template <class T, int LPR, int NJ, int KIND, bool ONCE>

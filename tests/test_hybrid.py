@@ -882,7 +882,7 @@ def test_states_past_the_caches(n, h, more):
         st = hops.StepMeta(nd=at.stop - at.start, pos=pos[at], slot=slot[at],
                            table=torch.zeros(n, 1, dtype=torch.int32,
                                              device="cuda"), max_len=4,
-                           state_bytes=225_000_000 // n + more)
+                           state_bytes=200_000_000 // n + more)
         return hops.mlstm(rows[at].contiguous(), gates[at].contiguous(), S, m,
                           norm, st, dk, dv, 15.0, 1e-5)
     S1, m1 = S.clone(), m.clone()
