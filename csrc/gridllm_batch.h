@@ -350,7 +350,7 @@ k_gemm_tile(const BatchArgs p) {
 // 523, 48 509, 499; 531, 533, 128 673, 659; 689, 686). Parts of K are read next. 128256
 // columns, us, k_gemm_tile in 256 columns and this:
 //   rows   24           64           96           128          160
-//   K 3072 130 -> 122   143 -> 129   158 -> 135   173 -> 142   184 -> 152
+//   K 3072 130 -> 126   143 -> 129   158 -> 135   173 -> 142   184 -> 152
 //   K 2048                           106 -> 96                 129 -> 104
 // ===========================================================================
 #define COLS_PAST 20000000l
